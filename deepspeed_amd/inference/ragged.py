@@ -442,7 +442,8 @@ class PagedKVCache:
         self.lens = torch.zeros(num_slots, dtype=torch.long)
         self.max_seq = max_seq
         self.device = device
-        self.last_mask: Optional[torch.Tensor] = None
+        self._slots: Optional[List[int]] = None
+        self._plans = {}     # of the current step, by (heads, key heads)
 
     def free(self, slot: int):
         self.free_blocks.extend(reversed(self.block_table[slot]))
@@ -468,23 +469,39 @@ class PagedKVCache:
         L = int((starts + q_len).max())
         for s, st in zip(self._slots, starts.tolist()):
             self._ensure_blocks(s, st + q_len)
-        pos = torch.arange(L, device=self.device)
-        qpos = (starts.to(self.device)[:, None, None] +
-                torch.arange(q_len, device=self.device)[None, :, None])
-        self.last_mask = (pos[None, None, :] <= qpos).unsqueeze(1)
         self._L = L
         self._starts = starts
+        self._plans = {}
+
+    @property
+    def last_mask(self) -> Optional[torch.Tensor]:
+        """[n, 1, q_len, L] validity of the padded views of ``update``; None
+        outside a step."""
+        if self._slots is None:
+            return None
+        pos = torch.arange(self._L, device=self.device)
+        qpos = (self._starts.to(self.device)[:, None, None] +
+                torch.arange(self._q_len, device=self.device)[None, :, None])
+        return (pos[None, None, :] <= qpos).unsqueeze(1)
+
+    def _row_places(self):
+        """Slot and position of every row of the step, in order."""
+        n = self._q_len
+        pos = (self._starts[:, None] + torch.arange(n)).reshape(-1).numpy()
+        slots = self._slots if n == 1 else \
+            [s for s in self._slots for _ in range(n)]
+        return slots, pos
 
     def update(self, layer_idx: int, k: torch.Tensor, v: torch.Tensor):
         n, Hkv, q_len, D = k.shape
         bs = self.block_size
-        for i, s in enumerate(self._slots):
-            st = int(self._starts[i])
-            for j in range(q_len):
-                p = st + j
-                blk = self.block_table[s][p // bs]
-                self.k[layer_idx][blk, :, p % bs] = k[i, :, j]
-                self.v[layer_idx][blk, :, p % bs] = v[i, :, j]
+        from ..ops.paged_attention import StepPlan
+        dst, _, _ = StepPlan.rows(*self._row_places(), self.block_table, bs)
+        dst = torch.from_numpy(dst).to(self.device)
+        blk, at = dst // bs, dst % bs
+        for pool, x in ((self.k[layer_idx], k), (self.v[layer_idx], v)):
+            pool[blk, :, at] = x.transpose(1, 2).reshape(
+                n * q_len, Hkv, D).to(pool.dtype)
         # materialize padded views: gather each slot's blocks
         nblk = (self._L + bs - 1) // bs
         idx = torch.tensor([ (self.block_table[s] + [0] * nblk)[:nblk]
@@ -496,35 +513,60 @@ class PagedKVCache:
         vb = vb.permute(0, 2, 1, 3, 4).reshape(n, Hkv, nblk * bs, D)
         return kb[:, :, :self._L], vb[:, :, :self._L]
 
+    def _eligible(self, layer_idx: int, q, k, v) -> bool:
+        from ..ops.paged_attention import paged_decode_available
+        kp = self.k[layer_idx]
+        return (q.is_cuda and kp.is_cuda and kp.dtype == torch.bfloat16
+                and k.dtype == v.dtype == torch.bfloat16
+                and paged_decode_available(
+                    q.reshape(-1, q.size(-2), q.size(-1)), kp))
+
+    def _attend(self, layer_idx: int, q, k, v, cos=None, sin=None,
+                positions=None, scale=None):
+        """New rows into the pool, then attention over it: three launches (two
+        where no history is split) for the whole step."""
+        from ..ops.paged_attention import (StepPlan, paged_append,
+                                           paged_attention)
+        kp, vp = self.k[layer_idx], self.v[layer_idx]
+        n, S, H, D = q.shape
+        plan = self._plans.get((H, kp.size(1)))
+        if plan is None:
+            plan = self._plans[H, kp.size(1)] = StepPlan.build(
+                *self._row_places(), self.block_table, self.block_size, H,
+                kp.size(1), kp.device)
+        q, k, v = (x.reshape(n * S, -1, D).contiguous() for x in (q, k, v))
+        q = paged_append(plan, q, k, v, kp, vp, cos, sin, positions, S)
+        o = paged_attention(plan, q, kp, vp, scale)
+        return o.view(n, S, H, D)
+
+    def rope_attention(self, layer_idx: int, q, k, v, cos, sin,
+                       positions=None, scale=None):
+        """A step's attention from the unrotated projections q [n, S, H, D]
+        and k, v [n, S, Hkv, D]: rotary embedding (tables [max_pos, D/2];
+        positions int32 [n, S] or each row's index in S), cache write and
+        causal attention over the paged pool. None when ineligible (the caller
+        rotates and takes ``decode_attention`` or ``update``)."""
+        if not self._eligible(layer_idx, q, k, v) or (
+                torch.is_grad_enabled() and q.requires_grad):
+            return None
+        if positions is not None and (
+                positions.dtype != torch.int32 or not positions.is_cuda
+                or positions.numel() != q.size(0) * q.size(1)):
+            return None
+        if positions is not None:
+            positions = positions.contiguous()
+        return self._attend(layer_idx, q, k, v, cos, sin, positions, scale)
+
     def decode_attention(self, layer_idx: int, q, k, v, scale=None):
         """Single-token decode THROUGH the paged pool: writes the new
-        token's k/v into its block and runs the split-S flash-decode HIP
-        kernel over the block table — the padded [n, Hkv, L, D] views are
-        never materialized (reference blocked_flash path). q/k/v are
-        [n, 1, H(kv), D] (BSHD step slices); returns [n, 1, H, D] or None
-        when ineligible (caller falls back to update() + SDPA)."""
-        from ..ops.paged_attention import (paged_decode_attention,
-                                           paged_decode_available)
-        if self._q_len != 1 or not q.is_cuda or q.dtype != torch.bfloat16:
+        token's k/v into its block and attends over the block lists — the
+        padded [n, Hkv, L, D] views are never materialized (reference
+        blocked_flash path). q/k/v are [n, 1, H(kv), D] (BSHD step slices);
+        returns [n, 1, H, D] or None when ineligible (caller falls back to
+        update() + SDPA)."""
+        if self._q_len != 1 or not self._eligible(layer_idx, q, k, v):
             return None
-        kp = self.k[layer_idx]
-        if not paged_decode_available(q.reshape(q.size(0), -1, q.size(-1)),
-                                      kp):
-            return None
-        bs = self.block_size
-        for i, s_ in enumerate(self._slots):
-            p = int(self._starts[i])
-            blk = self.block_table[s_][p // bs]
-            self.k[layer_idx][blk, :, p % bs] = k[i, 0]
-            self.v[layer_idx][blk, :, p % bs] = v[i, 0]
-        nblk = (int(self._starts.max()) + 1 + bs - 1) // bs
-        table = torch.tensor(
-            [(self.block_table[s_] + [0] * nblk)[:nblk]
-             for s_ in self._slots], dtype=torch.int32, device=q.device)
-        lens = (self._starts + 1).to(q.device, torch.int32)
-        o = paged_decode_attention(q[:, 0], kp, self.v[layer_idx], table,
-                                   lens, scale=scale)
-        return o.unsqueeze(1)
+        return self._attend(layer_idx, q, k, v, scale=scale)
 
     def end_step(self):
         idx = torch.as_tensor(self._slots, device=self.lens.device)
@@ -533,4 +575,4 @@ class PagedKVCache:
         else:
             self.lens[idx] += self._q_len
         self._slots = None
-        self.last_mask = None
+        self._plans = {}

@@ -130,6 +130,14 @@ class LlamaAttention(nn.Module):
         q = self.q_proj(x).view(B, S, self.num_heads, self.head_dim)
         k = self.k_proj(x).view(B, S, self.num_kv_heads, self.head_dim)
         v = self.v_proj(x).view(B, S, self.num_kv_heads, self.head_dim)
+        if attention_fn is None and hasattr(kv_cache, "rope_attention"):
+            # paged pool: rotation, cache write and attention over the block
+            # lists in three launches; None -> ineligible, paths below
+            o = kv_cache.rope_attention(self.layer_idx, q, k, v, cos, sin,
+                                        positions)
+            if o is not None:
+                kv_cache.last_decoded = S == 1
+                return self.o_proj(o.reshape(B, S, -1))
         q = apply_rope(q, cos, sin, positions)
         k = apply_rope(k, cos, sin, positions)
 

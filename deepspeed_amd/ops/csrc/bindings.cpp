@@ -66,12 +66,19 @@ extern "C" void ds_flash_bwd_dkdv_dbg(const void* q, const void* k,
                                       void* dk, void* dv, int B, int S,
                                       int H, int Hkv, float scale,
                                       int variant, void* stream);
-extern "C" void ds_paged_decode(const void* q, const void* kpool,
-                                const void* vpool, const int* block_table,
-                                const int* lens, float* part, float* part_ml,
-                                void* o, int n, int H, int Hkv, int BS,
-                                int max_blocks, int splits, float scale,
-                                void* stream);
+extern "C" void ds_paged_append(const void* q, const void* k, const void* v,
+                                void* qout, void* kpool, void* vpool,
+                                const int* dst, const float* cs,
+                                const float* sn, const int* positions, int T,
+                                int S, int H, int Hkv, int BS, void* stream);
+extern "C" void ds_paged_rows(const void* q, const void* kpool,
+                              const void* vpool, const int* table,
+                              const int* runs, const int* items,
+                              const int* merges, const int* lens, void* out,
+                              float* part, float* part_ml, int n_items,
+                              int n_merges, int any_merge, int nq, int H,
+                              int Hkv, int BS, int max_blocks, int splits,
+                              float scale, void* stream);
 extern "C" void ds_transpose_bf16(const void* src, void* dst, int n_batch,
                                   int R, int C, long long row_stride,
                                   int inner, long long inner_stride,
@@ -289,31 +296,120 @@ at::Tensor dropout_bwd(at::Tensor dy, at::Tensor mask, double ratio) {
   return dx;
 }
 
+static void check_pool(const at::Tensor& q, const at::Tensor& kpool,
+                       const at::Tensor& vpool, const char* what) {
+  TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kBFloat16 &&
+              q.is_contiguous() && q.dim() == 3 &&
+              kpool.scalar_type() == at::kBFloat16 && kpool.is_cuda() &&
+              kpool.is_contiguous() && kpool.dim() == 4 &&
+              vpool.scalar_type() == at::kBFloat16 && vpool.is_cuda() &&
+              vpool.is_contiguous() && kpool.sizes() == vpool.sizes(),
+              what, ": bf16 cuda contiguous");
+  TORCH_CHECK(q.size(2) == 128 && kpool.size(3) == 128, what,
+              ": D must be 128");
+  TORCH_CHECK(kpool.size(1) > 0 && q.size(1) % kpool.size(1) == 0, what,
+              ": H must be a multiple of Hkv");
+}
+
 at::Tensor paged_decode(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
                         at::Tensor block_table, at::Tensor lens,
                         int64_t splits, double scale) {
-  TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kBFloat16 &&
-              q.is_contiguous() && kpool.is_contiguous() &&
-              vpool.is_contiguous(), "paged_decode: bf16 cuda contiguous");
-  TORCH_CHECK(block_table.scalar_type() == at::kInt &&
-              lens.scalar_type() == at::kInt, "table/lens must be int32");
+  check_pool(q, kpool, vpool, "paged_decode");
   const int n = q.size(0), H = q.size(1);
   const int Hkv = kpool.size(1), BS = kpool.size(2);
-  TORCH_CHECK(q.size(2) == 128 && kpool.size(3) == 128, "D must be 128");
-  const int G = H / Hkv;
-  TORCH_CHECK(G == 1 || G == 2 || G == 4 || G == 8, "H/Hkv must be 1/2/4/8");
-  const int mb = block_table.size(1);
-  auto part = at::empty({(long)n, (long)Hkv, splits, (long)G, 128L},
-                        q.options().dtype(at::kFloat));
-  auto part_ml = at::empty({(long)n, (long)Hkv, splits, (long)G, 2L},
-                           q.options().dtype(at::kFloat));
+  TORCH_CHECK(H / Hkv <= 16, "paged_decode: at most 16 heads a key head");
+  TORCH_CHECK(block_table.scalar_type() == at::kInt &&
+              block_table.is_cuda() && block_table.is_contiguous() &&
+              block_table.dim() == 2 && block_table.size(0) == n &&
+              lens.scalar_type() == at::kInt && lens.is_cuda() &&
+              lens.is_contiguous() && lens.numel() == n,
+              "table/lens must be int32, one row each");
+  TORCH_CHECK(splits >= 1, "paged_decode: at least one split");
+  const long items = (long)n * splits;
+  auto f32 = q.options().dtype(at::kFloat);
+  auto part = at::empty({splits > 1 ? items * Hkv * 16 * 128 : 0}, f32);
+  auto part_ml = at::empty({splits > 1 ? items * Hkv * 16 * 2 : 0}, f32);
   auto o = at::empty_like(q);
-  ds_paged_decode(q.data_ptr(), kpool.data_ptr(), vpool.data_ptr(),
-                  block_table.data_ptr<int>(), lens.data_ptr<int>(),
-                  part.data_ptr<float>(), part_ml.data_ptr<float>(),
-                  o.data_ptr(), n, H, Hkv, BS, mb, (int)splits, (float)scale,
-                  cur_stream());
+  if (n == 0) return o;
+  ds_paged_rows(q.data_ptr(), kpool.data_ptr(), vpool.data_ptr(),
+                block_table.data_ptr<int>(), nullptr, nullptr, nullptr,
+                lens.data_ptr<int>(), o.data_ptr(), part.data_ptr<float>(),
+                part_ml.data_ptr<float>(), (int)items, n, splits > 1, 1, H,
+                Hkv, BS, (int)block_table.size(1), (int)splits, (float)scale,
+                cur_stream());
   return o;
+}
+
+// meta: int32 [items 4 each | runs 4 each | merges 2 each | table ...], the
+// plan of one serving step (built on the host from the cache's block lists).
+at::Tensor paged_rows(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
+                      at::Tensor meta, int64_t n_items, int64_t n_runs,
+                      int64_t n_merges, bool any_merge, int64_t nq,
+                      double scale) {
+  check_pool(q, kpool, vpool, "paged_rows");
+  TORCH_CHECK(meta.scalar_type() == at::kInt && meta.is_cuda() &&
+              meta.is_contiguous() &&
+              meta.numel() >= 4 * n_items + 4 * n_runs + 2 * n_merges &&
+              (nq == 1 || nq == 2), "paged_rows: plan");
+  const int H = q.size(1), Hkv = kpool.size(1);
+  const int* p = meta.data_ptr<int>();
+  auto f32 = q.options().dtype(at::kFloat);
+  const long cols = any_merge ? n_items * Hkv * 16 * nq : 0;
+  auto part = at::empty({cols * 128}, f32);
+  auto part_ml = at::empty({cols * 2}, f32);
+  auto o = at::empty_like(q);
+  if (n_items == 0) return o;
+  ds_paged_rows(q.data_ptr(), kpool.data_ptr(), vpool.data_ptr(),
+                p + 4 * (n_items + n_runs) + 2 * n_merges, p + 4 * n_items, p,
+                p + 4 * (n_items + n_runs), nullptr, o.data_ptr(),
+                part.data_ptr<float>(), part_ml.data_ptr<float>(),
+                (int)n_items, (int)n_merges, any_merge, (int)nq, H, Hkv,
+                (int)kpool.size(2), 0, 0, (float)scale, cur_stream());
+  return o;
+}
+
+// New rows k, v [T, Hkv, 128] into the pool rows dst [T]; with tables also
+// the rotary embedding of k on its way there and of q [T, H, 128], returned.
+at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
+                        at::Tensor kpool, at::Tensor vpool, at::Tensor dst,
+                        c10::optional<at::Tensor> cos_table,
+                        c10::optional<at::Tensor> sin_table,
+                        c10::optional<at::Tensor> positions, int64_t S) {
+  check_pool(q, kpool, vpool, "paged_append");
+  const int T = q.size(0), H = q.size(1), Hkv = kpool.size(1);
+  for (auto& x : {k, v})
+    TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
+                x.is_contiguous() && x.dim() == 3 && x.size(0) == T &&
+                x.size(1) == Hkv && x.size(2) == 128, "paged_append: k/v");
+  TORCH_CHECK(dst.scalar_type() == at::kInt && dst.is_cuda() &&
+              dst.is_contiguous() && dst.numel() == T, "paged_append: dst");
+  TORCH_CHECK(S >= 1 && T % S == 0, "paged_append: S");
+  const float *cs = nullptr, *sn = nullptr;
+  const int* pos = nullptr;
+  at::Tensor out = q;
+  if (cos_table.has_value()) {
+    for (auto& t : {*cos_table, *sin_table})
+      TORCH_CHECK(t.scalar_type() == at::kFloat && t.is_cuda() &&
+                  t.is_contiguous() && t.dim() == 2 && t.size(1) == 64,
+                  "paged_append: tables must be fp32 [positions, 64]");
+    cs = cos_table->data_ptr<float>();
+    sn = sin_table->data_ptr<float>();
+    if (positions.has_value()) {
+      TORCH_CHECK(positions->scalar_type() == at::kInt &&
+                  positions->is_cuda() && positions->is_contiguous() &&
+                  positions->numel() == T, "paged_append: positions");
+      pos = positions->data_ptr<int>();
+    } else {
+      TORCH_CHECK(cos_table->size(0) >= S, "table shorter than sequence");
+    }
+    out = at::empty_like(q);
+  }
+  if (T == 0) return out;
+  ds_paged_append(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+                  kpool.data_ptr(), vpool.data_ptr(), dst.data_ptr<int>(), cs,
+                  sn, pos, T, (int)S, H, Hkv, (int)kpool.size(2),
+                  cur_stream());
+  return out;
 }
 
 class ShmComm {
@@ -630,7 +726,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def(pybind11::init<const std::string&, int64_t, int64_t, int64_t>())
       .def("all_reduce", &ShmComm::all_reduce);
   m.def("paged_decode", &paged_decode,
-        "split-S flash-decode over a paged KV block table");
+        "split-KV decode attention over a paged KV block table");
+  m.def("paged_rows", &paged_rows,
+        "attention of a serving step's runs of tokens over the paged pool");
+  m.def("paged_append", &paged_append,
+        "rotary embedding and cache write of a serving step's new rows");
   m.def("fused_softmax", &fused_softmax,
         "fused masked/alibi/causal softmax");
   m.def("fused_dropout", &fused_dropout, "fused bias+dropout(+residual)");

@@ -1,21 +1,31 @@
-"""Paged flash-decode attention wrapper (reference:
-inference/v2/kernels/ragged_ops/blocked_flash). Consumes the PagedKVCache
-pool + block tables directly — single-token decode never materializes the
-padded [n, Hkv, L, D] views."""
+"""Attention over the paged KV pool (reference:
+inference/v2/kernels/ragged_ops/blocked_flash). The kernels read the
+PagedKVCache pool through its block lists: the padded [n, Hkv, L, D] views are
+never materialized, be the step single-token decoding, a portion of a prompt or
+both (csrc/paged_attention.hip)."""
 
+import itertools
 import math
-from typing import Optional
+from dataclasses import dataclass
+from typing import List, Optional
 
+import numpy as np
 import torch
 
 from ._loader import get_ext
 
+# Workgroups wanted in flight: four waves each, two to three to a CU of 256.
+# More splits than that only add partial results to write and merge.
+WORKGROUPS = 1024
+# Keys of the shortest split: one tile of 32 for each of a workgroup's waves.
+MIN_SPLIT = 128
+
 
 def paged_decode_available(q: torch.Tensor, kpool: torch.Tensor) -> bool:
-    G = q.size(1) // kpool.size(1)
     return (get_ext() is not None and q.is_cuda
             and q.dtype == torch.bfloat16 and q.size(-1) == 128
-            and G in (1, 2, 4, 8))
+            and q.size(1) % kpool.size(1) == 0
+            and 1 <= q.size(1) // kpool.size(1) <= 16)
 
 
 def paged_decode_attention(q: torch.Tensor, kpool: torch.Tensor,
@@ -23,13 +33,112 @@ def paged_decode_attention(q: torch.Tensor, kpool: torch.Tensor,
                            lens: torch.Tensor, splits: Optional[int] = None,
                            scale: Optional[float] = None) -> torch.Tensor:
     """q [n, H, 128] bf16; kpool/vpool [nb, Hkv, BS, 128] bf16;
-    block_table [n, max_blocks] int32; lens [n] int32 -> o [n, H, 128]."""
+    block_table [n, max_blocks] int32; lens [n] int32 -> o [n, H, 128].
+    The lengths stay on the device, so every request is cut into the same
+    number of splits; ``StepPlan`` cuts by length."""
     ext = get_ext()
     scale = scale if scale is not None else 1.0 / math.sqrt(q.size(-1))
     if splits is None:
-        # fill the chip: ~2048 workgroups wanted; grid = n * Hkv * splits
         nw = max(1, q.size(0) * kpool.size(1))
-        splits = max(1, min(32, 2048 // nw))
+        splits = max(1, min(32, WORKGROUPS // nw))
     return ext.paged_decode(q.contiguous(), kpool, vpool,
                             block_table.contiguous().int(),
                             lens.contiguous().int(), splits, scale)
+
+
+@dataclass
+class StepPlan:
+    """One serving step for the kernels: where each new row goes (``dst``) and
+    the work items of its attention (``meta``), both on the device."""
+
+    dst: torch.Tensor
+    meta: torch.Tensor
+    items: int
+    runs: int
+    merges: int
+    any_merge: bool
+    nq: int
+
+    @staticmethod
+    def rows(slots: List[int], pos: np.ndarray, tables, block_size: int):
+        """Pool row (block * block_size + offset) of every new token, and the
+        block lists of the step's slots, one after another."""
+        used = list(dict.fromkeys(slots))
+        lists = [tables[s] for s in used]
+        flat = np.fromiter(itertools.chain.from_iterable(lists), np.int32,
+                           sum(map(len, lists)))
+        first, at = {}, 0
+        for s, blocks in zip(used, lists):
+            first[s] = at
+            at += len(blocks)
+        offs = np.array([first[s] for s in slots], np.int64)
+        dst = flat[offs + pos // block_size].astype(np.int64) * block_size \
+            + pos % block_size
+        return dst, flat, offs
+
+    @classmethod
+    def build(cls, slots: List[int], pos: np.ndarray, tables, block_size: int,
+              heads: int, kv_heads: int, device) -> "StepPlan":
+        """``slots[i]`` and ``pos[i]``: request slot and position of row i.
+        Neighbouring rows of one slot at following positions form a run and
+        share the reads of its keys and values."""
+        T = len(slots)
+        dst, flat, offs = cls.rows(slots, pos, tables, block_size)
+        sl = np.asarray(slots)
+        cut = np.flatnonzero((sl[1:] != sl[:-1]) | (pos[1:] != pos[:-1] + 1))
+        row0 = np.concatenate(([0], cut + 1))
+        m = np.diff(np.append(row0, T))
+        kv_len = pos[row0] + m
+        runs = np.stack([row0, m, kv_len, offs[row0]], 1)
+        G = heads // kv_heads
+        # columns (rows times heads a key head) go in tiles of 16; two tiles
+        # share the loads of a key tile where runs are long enough
+        nq = 2 if int(m.max()) * G > 16 else 1
+        width = 16 * nq
+        tiles = -(-m * G // width)
+        run_of = np.repeat(np.arange(len(m)), tiles)
+        tile = np.arange(len(run_of)) - np.repeat(np.cumsum(tiles) - tiles,
+                                                  tiles)
+        tok = np.minimum((tile + 1) * width, m[run_of] * G) - 1
+        end = kv_len[run_of] - m[run_of] + tok // G + 1
+        # split long histories until the chip is full
+        if len(end) * kv_heads >= WORKGROUPS:
+            n = np.ones_like(end)
+        else:
+            per = max(MIN_SPLIT, int(end.sum()) * kv_heads // WORKGROUPS)
+            n = -(-end // per)
+        step = -(-(-(-end // n)) // 32) * 32
+        n = -(-end // step)
+        of = np.repeat(np.arange(len(end)), n)
+        first = np.cumsum(n) - n
+        part = np.arange(len(of)) - first[of]
+        lo = part * step[of]
+        hi = np.minimum(lo + step[of], end[of])
+        hi = np.where(n[of] == 1, -hi, hi)
+        items = np.stack([run_of[of], tile[of], lo, hi], 1)
+        merges = np.stack([first, n], 1)
+        head = 4 * len(items) + 4 * len(runs) + 2 * len(merges) + len(flat)
+        both = torch.from_numpy(np.concatenate(
+            [items.ravel(), runs.ravel(), merges.ravel(), flat, dst]).astype(
+                np.int32)).to(device)
+        return cls(dst=both[head:], meta=both, items=len(items),
+                   runs=len(runs), merges=len(merges),
+                   any_merge=bool((n > 1).any()), nq=nq)
+
+
+def paged_append(plan: StepPlan, q, k, v, kpool, vpool, cos=None, sin=None,
+                 positions=None, seq: int = 1):
+    """Write the step's new rows k, v [T, Hkv, 128] into the pool; with cos and
+    sin tables, after the rotary embedding of k, and return that of q [T, H,
+    128] (positions [T] int32, or row t at t % seq)."""
+    return get_ext().paged_append(q, k, v, kpool, vpool, plan.dst, cos, sin,
+                                  positions, seq)
+
+
+def paged_attention(plan: StepPlan, q, kpool, vpool,
+                    scale: Optional[float] = None):
+    """q [T, H, 128] over the pool, each row up to its own position."""
+    scale = scale if scale is not None else 1.0 / math.sqrt(q.size(-1))
+    return get_ext().paged_rows(q, kpool, vpool, plan.meta, plan.items,
+                                plan.runs, plan.merges, plan.any_merge,
+                                plan.nq, scale)

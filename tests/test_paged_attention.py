@@ -1,0 +1,171 @@
+"""Attention over the paged pool: the step plan (CPU) and the kernels against
+a plain fp32 attention over the gathered rows (GPU)."""
+
+import numpy as np
+import pytest
+import torch
+
+from deepspeed_amd.inference.ragged import PagedKVCache
+from deepspeed_amd.ops.paged_attention import StepPlan
+
+# (slots with the new rows of each, kept tokens by slot)
+STEPS = {
+    "decode": ([(0, 1), (1, 1), (2, 1)], [0, 31, 700]),
+    "portion": ([(0, 70)], [33]),
+    "first": ([(0, 129), (1, 129)], [0, 0]),
+    "packed": ([(0, 1), (2, 45), (1, 1), (2, 3)], [64, 1, 500]),
+    "long": ([(0, 1)], [5000]),
+}
+
+
+def _rows(step, lens):
+    """Slots and positions of the rows; a slot's later runs go on behind its
+    earlier ones."""
+    slots, pos, at = [], [], list(lens)
+    for s, m in step:
+        slots += [s] * m
+        pos += range(at[s], at[s] + m)
+        at[s] += m
+    return slots, np.array(pos), at
+
+
+@pytest.mark.parametrize("name", list(STEPS))
+@pytest.mark.parametrize("bs", [16, 24, 64])
+@pytest.mark.parametrize("heads", [(8, 8), (14, 2), (32, 8)])
+def test_step_plan_covers_every_key_once(name, bs, heads):
+    step, lens = STEPS[name]
+    slots, pos, end = _rows(step, lens)
+    rng = np.random.default_rng(0)
+    free = list(rng.permutation(1000))
+    tables = {s: [int(free.pop()) for _ in range(-(-n // bs))]
+              for s, n in enumerate(end)}
+    plan = StepPlan.build(slots, pos, tables, bs, *heads, "cpu")
+    meta = plan.meta.numpy()
+    items = meta[:4 * plan.items].reshape(-1, 4)
+    runs = meta[4 * plan.items:][:4 * plan.runs].reshape(-1, 4)
+    merges = meta[4 * (plan.items + plan.runs):][:2 * plan.merges]
+    merges = merges.reshape(-1, 2)
+    table = meta[4 * (plan.items + plan.runs) + 2 * plan.merges:]
+    G = heads[0] // heads[1]
+    for i, (s, p) in enumerate(zip(slots, pos)):
+        assert plan.dst[i] == tables[s][p // bs] * bs + p % bs
+        r = next(r for r in runs if r[0] <= i < r[0] + r[1])
+        assert r[2] - r[1] + i - r[0] == p
+        assert list(table[r[3]:r[3] + p // bs + 1]) == \
+            tables[s][:p // bs + 1]
+    for first, n in merges:
+        run, tile = items[first][:2]
+        ncols = runs[run][1] * G
+        last = (min((tile + 1) * 16 * plan.nq, ncols) - 1) // G
+        want = runs[run][2] - runs[run][1] + last + 1
+        at = 0
+        for it in items[first:first + n]:
+            assert tuple(it[:2]) == (run, tile) and it[2] == at
+            assert it[2] % 32 == 0 and (it[3] < 0) == (n == 1)
+            at = abs(it[3])
+            assert at > it[2]
+        assert at == want
+    tiles = sorted((int(items[f][0]), int(items[f][1])) for f, _ in merges)
+    assert tiles == [(r, t) for r in range(len(runs))
+                     for t in range(-(-runs[r][1] * G // (16 * plan.nq)))]
+    assert plan.items == merges[:, 1].sum()
+
+
+def _reference(q, k, v, pos, scale):
+    """q [m, H, D] at positions ``pos`` over k, v [L, Hkv, D], in fp64."""
+    G = q.shape[1] // k.shape[1]
+    k, v = (t.double().repeat_interleave(G, 1).transpose(0, 1)
+            for t in (k, v))
+    s = torch.matmul(q.double().transpose(0, 1),
+                     k.transpose(1, 2).contiguous()) * scale
+    hidden = torch.arange(k.shape[1], device=q.device)[None] > pos[:, None]
+    return torch.matmul(torch.softmax(s.masked_fill(hidden, -np.inf), -1),
+                        v).transpose(0, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(STEPS))
+@pytest.mark.parametrize("bs", [16, 24, 64])
+@pytest.mark.parametrize("heads", [(1, 1), (8, 8), (14, 2), (32, 8), (16, 1)])
+def test_paged_attention_gpu(name, bs, heads):
+    """Rotation, cache write and attention of every kind of step. The pool's
+    other rows hold NaN: nothing outside a request's own rows is used."""
+    H, Hkv = heads
+    step, lens = STEPS[name]
+    slots, pos, end = _rows(step, lens)
+    g = torch.Generator().manual_seed(H * 100 + bs)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=g).to(torch.bfloat16).cuda()
+
+    cache = PagedKVCache(1, 3, Hkv, 8192, 128, dtype=torch.bfloat16,
+                         device="cuda", block_size=bs,
+                         num_blocks=sum(-(-n // bs) for n in end) + 5)
+    cache.free_blocks = torch.randperm(cache.num_blocks, generator=g).tolist()
+    for t in (cache.k[0], cache.v[0]):
+        t.fill_(float("nan"))
+    kept = []
+    for s, n in enumerate(lens):
+        cache._ensure_blocks(s, n)
+        rows = rand(n, Hkv, 128), rand(n, Hkv, 128)
+        p = torch.arange(n, device="cuda")
+        blk = torch.tensor(cache.block_table[s], dtype=torch.long,
+                           device="cuda")
+        for pool, x in zip((cache.k[0], cache.v[0]), rows):
+            pool[blk[p // bs], :, p % bs] = x
+        kept.append(rows)
+    cache.lens[:] = torch.tensor(lens + [0] * (3 - len(lens)))
+    T = len(slots)
+    q, k, v = rand(T, 1, H, 128), rand(T, 1, Hkv, 128), rand(T, 1, Hkv, 128)
+    ang = torch.rand(8192, 64, generator=g) * 6.28
+    cos, sin = ang.cos().cuda(), ang.sin().cuda()
+    positions = torch.tensor(pos, dtype=torch.int32, device="cuda")[:, None]
+    cache.begin_step(slots, 1, offsets=[int(p) - lens[s] for s, p in
+                                        zip(slots, pos)])
+    got = cache.rope_attention(0, q, k, v, cos, sin, positions)
+    from deepspeed_amd.ops.rope import apply_rope
+    q2, k2 = (apply_rope(x, cos, sin, positions) for x in (q, k))
+    cache.end_step()
+    for s, n in enumerate(lens):
+        mine = [i for i, t in enumerate(slots) if t == s]
+        if not mine:
+            continue
+        kk = torch.cat([kept[s][0], k2[mine, 0]])
+        vv = torch.cat([kept[s][1], v[mine, 0]])
+        at = torch.tensor(pos[mine], device="cuda")
+        want = _reference(q2[mine, 0], kk, vv, at, 128 ** -0.5)
+        # one rounding to bf16 (2^-9 of the value) of sums whose terms carry
+        # 2^-18 (split probabilities) and fp32 rounding
+        err = (got[mine, 0].double() - want).abs()
+        # 2^-13 a unit of the values; rotations rounded another way move the
+        # result by some 2^-9 of the new rows' share, a value's 2^-8 at most
+        assert (err <= 2.0 ** -7 * want.abs() + 2.0 ** -10).all(), err.max()
+        blk = torch.tensor(cache.block_table[s], device="cuda")
+        # fp32 rounding of the rotation may turn one rounding to bf16
+        torch.testing.assert_close(cache.k[0][blk[at // bs], :, at % bs],
+                                   k2[mine, 0], rtol=2.0 ** -7,
+                                   atol=2.0 ** -20)
+        assert torch.equal(cache.v[0][blk[at // bs], :, at % bs], v[mine, 0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [0.05, -0.05, 0.0])
+@pytest.mark.parametrize("splits", [None, 1, 5])
+def test_paged_decode_scales_and_splits(scale, splits):
+    from deepspeed_amd.ops.paged_attention import paged_decode_attention
+    torch.manual_seed(1)
+    lens = torch.tensor([0, 1, 33, 200], dtype=torch.int32, device="cuda")
+    table = torch.randperm(16)[:16].view(4, 4).int().cuda()
+    kp, vp = (torch.randn(16, 2, 64, 128, device="cuda").bfloat16()
+              for _ in range(2))
+    q = (4 * torch.randn(4, 14, 128, device="cuda")).bfloat16()
+    got = paged_decode_attention(q, kp, vp, table, lens, splits, scale)
+    assert not got[0].any()
+    for i in range(1, 4):
+        n = int(lens[i])
+        kk, vv = (p[table[i].long()].transpose(1, 2).reshape(-1, 2, 128)[:n]
+                  for p in (kp, vp))
+        want = _reference(q[i:i + 1], kk, vv,
+                          torch.tensor([n - 1], device="cuda"), scale)
+        err = (got[i:i + 1].double() - want).abs()
+        assert (err <= 2.0 ** -8 * want.abs() + 2.0 ** -13).all(), err.max()
