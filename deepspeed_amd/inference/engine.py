@@ -115,25 +115,14 @@ class InferenceEngine(nn.Module):
         self.module.eval()
 
     def _quantize_linear_weights(self, group_size: int = 2048) -> int:
-        from ..linear.optimized_linear import (QuantizationConfig,
-                                               QuantizedParameter)
+        from ..linear.optimized_linear import QuantizationConfig, WOQLinear
         qcfg = QuantizationConfig(group_size=group_size)
-
-        class WOQLinear(nn.Module):
-            def __init__(self, lin: nn.Linear):
-                super().__init__()
-                self.qweight = QuantizedParameter(lin.weight.data, qcfg)
-                self.bias = lin.bias
-
-            def forward(self, x):
-                w = self.qweight.dequantized().to(x.dtype)
-                return torch.nn.functional.linear(x, w, self.bias)
 
         n = 0
         for parent in list(self.module.modules()):
             for name, child in list(parent.named_children()):
                 if type(child) is nn.Linear:
-                    setattr(parent, name, WOQLinear(child))
+                    setattr(parent, name, WOQLinear(child, qcfg))
                     n += 1
         return n
 

@@ -43,9 +43,27 @@ class QuantizedParameter(nn.Module):
         self.register_buffer("scales", s)
 
     def dequantized(self) -> torch.Tensor:
-        return dequantize(self.q, self.scales, int(torch.tensor(self.shape)
-                          .prod()), self.cfg.group_size, self.cfg.q_bits,
+        return dequantize(self.q, self.scales, self.shape.numel(),
+                          self.cfg.group_size, self.cfg.q_bits,
                           self.dtype).view(self.shape)
+
+
+class WOQLinear(nn.Module):
+    """Inference linear on a quantized weight (weight-only quantization): few
+    rows read the int8 weight as it is, many have it dequantized first."""
+
+    def __init__(self, lin: nn.Linear, cfg: QuantizationConfig):
+        super().__init__()
+        self.qweight = QuantizedParameter(lin.weight.data, cfg)
+        self.bias = lin.bias
+
+    def forward(self, x):
+        from ..ops.linear import rows_linear
+        y = rows_linear(x, (self,), hooks_ran=True)
+        if y is not None:
+            return y[0]
+        w = self.qweight.dequantized().to(x.dtype)
+        return nn.functional.linear(x, w, self.bias)
 
 
 class OptimizedLinear(nn.Module):

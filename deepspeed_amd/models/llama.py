@@ -16,6 +16,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from ..ops.linear import SWIGLU, rows_linear, unhooked
 from ..ops.norms import RMSNorm
 from ..ops.rope import apply_rope, rope_tables
 from ..ops.swiglu import swiglu
@@ -124,12 +125,22 @@ class LlamaAttention(nn.Module):
         self.v_proj = nn.Linear(h, cfg.num_kv_heads * self.head_dim, bias=ab)
         self.o_proj = nn.Linear(cfg.num_heads * self.head_dim, h, bias=False)
 
+    def _out(self, o, residual):
+        """Output projection, with the layer's residual if it was handed in."""
+        if residual is not None:
+            y = rows_linear(o, (self.o_proj,), residual=residual)
+            return residual + self.o_proj(o) if y is None else y[0]
+        return self.o_proj(o)
+
     def forward(self, x, cos, sin, positions=None, kv_cache=None,
-                attention_fn=None):
+                attention_fn=None, residual=None):
         B, S, _ = x.shape
-        q = self.q_proj(x).view(B, S, self.num_heads, self.head_dim)
-        k = self.k_proj(x).view(B, S, self.num_kv_heads, self.head_dim)
-        v = self.v_proj(x).view(B, S, self.num_kv_heads, self.head_dim)
+        qkv = rows_linear(x, (self.q_proj, self.k_proj, self.v_proj))
+        if qkv is None:
+            qkv = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        q = qkv[0].view(B, S, self.num_heads, self.head_dim)
+        k = qkv[1].view(B, S, self.num_kv_heads, self.head_dim)
+        v = qkv[2].view(B, S, self.num_kv_heads, self.head_dim)
         if attention_fn is None and hasattr(kv_cache, "rope_attention"):
             # paged pool: rotation, cache write and attention over the block
             # lists in three launches; None -> ineligible, paths below
@@ -137,7 +148,7 @@ class LlamaAttention(nn.Module):
                                         positions)
             if o is not None:
                 kv_cache.last_decoded = S == 1
-                return self.o_proj(o.reshape(B, S, -1))
+                return self._out(o.reshape(B, S, -1), residual)
         q = apply_rope(q, cos, sin, positions)
         k = apply_rope(k, cos, sin, positions)
 
@@ -145,7 +156,7 @@ class LlamaAttention(nn.Module):
             # Ulysses: all-to-all scatters heads / gathers the sequence so
             # each rank runs full-sequence causal attention on H/P heads
             o = self._ulysses_attn(q, k, v)
-            return self.o_proj(o.reshape(B, S, -1))
+            return self._out(o.reshape(B, S, -1), residual)
 
         if kv_cache is None and attention_fn is None:
             from ..ops.attention import (flash_attn_available, flash_attn_fwd,
@@ -155,11 +166,11 @@ class LlamaAttention(nn.Module):
                 # hand-written CDNA4 MFMA flash kernel, BSHD layout — skips
                 # the transpose entirely (inference/no-grad prefill path)
                 o = flash_attn_fwd(q, k, v, causal=True)
-                return self.o_proj(o.reshape(B, S, -1))
+                return self._out(o.reshape(B, S, -1), residual)
             if torch.is_grad_enabled() and flash_train_available(q, k):
                 # differentiable hand-written path (fwd + dk/dv/dq kernels)
                 o = flash_attn_func(q, k, v, causal=True)
-                return self.o_proj(o.reshape(B, S, -1))
+                return self._out(o.reshape(B, S, -1), residual)
 
         if (S == 1 and kv_cache is not None
                 and hasattr(kv_cache, "decode_attention")
@@ -169,7 +180,7 @@ class LlamaAttention(nn.Module):
             o = kv_cache.decode_attention(self.layer_idx, q, k, v)
             if o is not None:
                 kv_cache.last_decoded = True
-                return self.o_proj(o.reshape(B, S, -1))
+                return self._out(o.reshape(B, S, -1), residual)
 
         # [B, H, S, D] for SDPA
         q = q.transpose(1, 2)
@@ -189,8 +200,7 @@ class LlamaAttention(nn.Module):
             o = sdpa_gqa(q, k, v,
                          causal=attn_mask is None and q.size(2) == k.size(2),
                          attn_mask=attn_mask)
-        o = o.transpose(1, 2).reshape(B, S, -1)
-        return self.o_proj(o)
+        return self._out(o.transpose(1, 2).reshape(B, S, -1), residual)
 
 
 def _bshd_causal_attention(q, k, v):
@@ -242,8 +252,13 @@ class LlamaMLP(nn.Module):
         self.up_proj = nn.Linear(h, i, bias=False)
         self.down_proj = nn.Linear(i, h, bias=False)
 
-    def forward(self, x):
-        return self.down_proj(swiglu(self.gate_proj(x), self.up_proj(x)))
+    def forward(self, x, residual=None):
+        h = rows_linear(x, (self.gate_proj, self.up_proj), SWIGLU)
+        h = swiglu(self.gate_proj(x), self.up_proj(x)) if h is None else h[0]
+        if residual is not None:
+            y = rows_linear(h, (self.down_proj,), residual=residual)
+            return residual + self.down_proj(h) if y is None else y[0]
+        return self.down_proj(h)
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -256,10 +271,20 @@ class LlamaDecoderLayer(nn.Module):
         self.mlp = LlamaMLP(cfg)
 
     def forward(self, x, cos, sin, positions=None, kv_cache=None):
-        x = x + self.self_attn(self.input_layernorm(x), cos, sin, positions,
-                               kv_cache)
-        x = x + self.mlp(self.post_attention_layernorm(x))
-        return x
+        # serving: the residual goes along and is added where the sublayer's
+        # last product is written
+        if torch.is_grad_enabled() or type(self.self_attn) is not \
+                LlamaAttention or not unhooked(self.self_attn):
+            x = x + self.self_attn(self.input_layernorm(x), cos, sin,
+                                   positions, kv_cache)
+        else:
+            x = self.self_attn(self.input_layernorm(x), cos, sin, positions,
+                               kv_cache, residual=x)
+        h = self.post_attention_layernorm(x)
+        if torch.is_grad_enabled() or type(self.mlp) is not LlamaMLP or \
+                not unhooked(self.mlp):
+            return x + self.mlp(h)
+        return self.mlp(h, residual=x)
 
 
 class LlamaModel(nn.Module):
@@ -319,7 +344,8 @@ class LlamaForCausalLM(nn.Module):
             # [B*S, vocab] fp32 logits (vocab=128256 -> ~2 GB per 4k tokens).
             # Routed through the lm_head MODULE so ZeRO-3 fetch hooks fire.
             return chunked_cross_entropy(hidden, self.lm_head, labels)
-        return self.lm_head(hidden)
+        logits = rows_linear(hidden, (self.lm_head,))
+        return self.lm_head(hidden) if logits is None else logits[0]
 
     def num_parameters(self):
         return sum(p.numel() for p in self.parameters())

@@ -79,6 +79,11 @@ extern "C" void ds_paged_rows(const void* q, const void* kpool,
                               int n_merges, int any_merge, int nq, int H,
                               int Hkv, int BS, int max_blocks, int splits,
                               float scale, void* stream);
+extern "C" void ds_rows_linear(const void* x, int layers, const void* const* w,
+                               const float* const* scales,
+                               const void* const* bias, void* const* out,
+                               const int* n, const void* residual, int M,
+                               int K, int group, int mode, void* stream);
 extern "C" void ds_transpose_bf16(const void* src, void* dst, int n_batch,
                                   int R, int C, long long row_stride,
                                   int inner, long long inner_stride,
@@ -412,6 +417,69 @@ at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
   return out;
 }
 
+// Linear layers on one input of a few rows (rows_linear.hip). weights: bf16
+// [N, K], or int8 (any shape, N * K long) with their groupwise scales.
+// mode 1 returns silu(layer 0) * layer 1. residual is added to the first.
+std::vector<at::Tensor> rows_linear(
+    at::Tensor x, std::vector<at::Tensor> weights,
+    std::vector<at::Tensor> scales,
+    std::vector<c10::optional<at::Tensor>> biases,
+    c10::optional<at::Tensor> residual, int64_t group, int64_t mode) {
+  const int L = weights.size();
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
+              x.is_contiguous() && x.dim() == 2, "rows_linear: x");
+  const int64_t M = x.size(0), K = x.size(1);
+  TORCH_CHECK(M >= 1 && M <= (scales.empty() ? 32 : 64) && K > 0 && K % 256 == 0 && L >= 1 &&
+              L <= 3 && (mode == 0 || L == 2) &&
+              (scales.empty() || (int)scales.size() == L) &&
+              (int)biases.size() == L, "rows_linear: shape");
+  const bool i8 = !scales.empty();
+  const void *w[3], *b[3];
+  const float* sc[3];
+  void* o[3];
+  int n[3];
+  std::vector<at::Tensor> out;
+  for (int i = 0; i < L; ++i) {
+    const auto& t = weights[i];
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
+                t.scalar_type() == (i8 ? at::kChar : at::kBFloat16) &&
+                t.numel() % K == 0 && t.numel() > 0 &&
+                ((uintptr_t)t.data_ptr() & 15) == 0, "rows_linear: weight");
+    n[i] = t.numel() / K;
+    w[i] = t.data_ptr();
+    b[i] = nullptr;
+    if (biases[i].has_value()) {
+      TORCH_CHECK(biases[i]->is_cuda() && biases[i]->is_contiguous() &&
+                  biases[i]->scalar_type() == at::kBFloat16 &&
+                  biases[i]->numel() == n[i], "rows_linear: bias");
+      b[i] = biases[i]->data_ptr();
+    }
+    if (i8) {
+      TORCH_CHECK(scales[i].is_cuda() && scales[i].is_contiguous() &&
+                  scales[i].scalar_type() == at::kFloat && group > 0 &&
+                  group % 256 == 0 &&
+                  scales[i].numel() == (t.numel() + group - 1) / group,
+                  "rows_linear: scales");
+      sc[i] = scales[i].data_ptr<float>();
+    }
+    if (mode == 0 || i == 0)
+      out.push_back(at::empty({M, n[i]}, x.options()));
+    o[i] = out.back().data_ptr();
+  }
+  TORCH_CHECK(mode == 0 || n[0] == n[1], "rows_linear: gate and up");
+  TORCH_CHECK(((uintptr_t)x.data_ptr() & 15) == 0, "rows_linear: alignment");
+  const void* res = nullptr;
+  if (residual.has_value()) {
+    TORCH_CHECK(residual->is_cuda() && residual->is_contiguous() &&
+                residual->scalar_type() == at::kBFloat16 &&
+                residual->numel() == M * n[0], "rows_linear: residual");
+    res = residual->data_ptr();
+  }
+  ds_rows_linear(x.data_ptr(), L, w, i8 ? sc : nullptr, b, o, n, res, (int)M,
+                 (int)K, (int)group, (int)mode, cur_stream());
+  return out;
+}
+
 class ShmComm {
  public:
   ShmComm(const std::string& name, int64_t rank, int64_t world,
@@ -727,6 +795,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def("all_reduce", &ShmComm::all_reduce);
   m.def("paged_decode", &paged_decode,
         "split-KV decode attention over a paged KV block table");
+  m.def("rows_linear", &rows_linear,
+        "linear layers of a few rows, bf16 or groupwise int8 weights");
   m.def("paged_rows", &paged_rows,
         "attention of a serving step's runs of tokens over the paged pool");
   m.def("paged_append", &paged_append,

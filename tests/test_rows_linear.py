@@ -1,0 +1,118 @@
+"""Linear layers of a few rows: which calls take the kernel (CPU) and the kernel
+against fp64 products of the same weights (GPU)."""
+
+import pytest
+import torch
+import torch.nn as nn
+
+from deepspeed_amd.linear.optimized_linear import (QuantizationConfig,
+                                                   WOQLinear)
+from deepspeed_amd.ops.linear import SWIGLU, rows_linear, unhooked
+
+
+def test_unhooked():
+    lin = nn.Linear(8, 8)
+    assert unhooked(lin)
+    for register in (lin.register_forward_hook,
+                     lin.register_forward_pre_hook,
+                     lin.register_full_backward_hook,
+                     lin.register_full_backward_pre_hook):
+        h = register(lambda *a: None)
+        assert not unhooked(lin)
+        h.remove()
+    h = nn.modules.module.register_module_forward_hook(lambda *a: None)
+    assert not unhooked(lin)
+    h.remove()
+    assert unhooked(lin)
+
+
+def test_cpu_and_grad_calls_are_left_alone():
+    lin = nn.Linear(256, 16).bfloat16()
+    x = torch.randn(2, 256).bfloat16()
+    with torch.no_grad():
+        assert rows_linear(x, (lin,)) is None
+    assert rows_linear(x, (lin,)) is None
+
+
+def _layer(n, k, bias, int8, g):
+    lin = nn.Linear(k, n, bias=bias).bfloat16().cuda()
+    with torch.no_grad():
+        lin.weight.copy_(0.05 * torch.randn(n, k, generator=g))
+        if bias:
+            lin.bias.copy_(torch.randn(n, generator=g))
+    w = lin.weight.double()
+    if int8:
+        lin = WOQLinear(lin, QuantizationConfig())
+        q, s = lin.qweight.q, lin.qweight.scales
+        w = (q.double() * s.double().repeat_interleave(2048)[:n * k]).view(n,
+                                                                          k)
+    b = lin.bias.double() if bias else 0.0
+    return lin, lambda x: x.double() @ w.t() + b
+
+
+def _close(got, want):
+    # fp32 sums rounded to bf16 once
+    err = (got.double() - want).abs()
+    lim = 2.0 ** -8 * want.abs() + 2.0 ** -16 * want.abs().max()
+    assert (err <= lim).all(), (err / lim).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 32, 33, 64, 65])
+@pytest.mark.parametrize("sizes", [((37,), 256), ((6144,), 512),
+                                   ((14336,), 256), ((256, 24, 40), 3072)])
+@torch.no_grad()
+def test_rows_linear_gpu(int8, m, sizes):
+    ns, k = sizes
+    g = torch.Generator().manual_seed(m)
+    both = [_layer(n, k, i % 2 == 0, int8, g) for i, n in enumerate(ns)]
+    x = torch.randn(1, m, k, generator=g).bfloat16().cuda()
+    got = rows_linear(x, [b[0] for b in both])
+    if m > (64 if int8 else 32):
+        assert got is None
+        return
+    for (lin, want), y in zip(both, got):
+        assert y.shape == (1, m, y.shape[-1])
+        _close(y, want(x))
+    res = torch.randn(1, m, ns[0], generator=g).bfloat16().cuda()
+    y, = rows_linear(x, (both[0][0],), residual=res)
+    _close(y, both[0][1](x) + res.double())
+    if int8:
+        _close(both[0][0](x), both[0][1](x))
+    h = both[0][0].register_forward_hook(lambda *a: None)
+    assert rows_linear(x, (both[0][0],)) is None
+    h.remove()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 50])
+@torch.no_grad()
+def test_rows_swiglu_gpu(int8, m):
+    if m > 32 and not int8:
+        return
+    g = torch.Generator().manual_seed(m)
+    (gate, fg), (up, fu) = (_layer(1000, 512, False, int8, g)
+                            for _ in range(2))
+    x = torch.randn(m, 512, generator=g).bfloat16().cuda()
+    y, = rows_linear(x, (gate, up), SWIGLU)
+    _close(y, torch.nn.functional.silu(fg(x)) * fu(x))
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+def test_model_with_and_without_rows_linear(monkeypatch):
+    """A decoding step's logits by either way, through a whole model."""
+    from deepspeed_amd.models import llama
+    torch.manual_seed(0)
+    cfg = llama.LlamaConfig(vocab_size=1000, hidden_size=512,
+                            intermediate_size=768, num_layers=2, num_heads=4,
+                            num_kv_heads=2, max_seq_len=64,
+                            attention_bias=True)
+    model = llama.LlamaForCausalLM(cfg).bfloat16().cuda().eval()
+    ids = torch.randint(0, 1000, (3, 7), device="cuda")
+    a = model(ids).float()
+    monkeypatch.setattr(llama, "rows_linear", lambda *a, **k: None)
+    b = model(ids).float()
+    assert (a - b).norm() < 0.02 * b.norm()
