@@ -18,6 +18,7 @@ import torch.nn as nn
 from .. import accel
 from .. import comm as dist
 from ..parallel import groups
+from ..ops.linear import Linear
 from ..utils.logging import log_dist
 from .auto_tp import shard_attention_heads, shard_model
 from .kv_cache import StaticKVCache
@@ -121,7 +122,7 @@ class InferenceEngine(nn.Module):
         n = 0
         for parent in list(self.module.modules()):
             for name, child in list(parent.named_children()):
-                if type(child) is nn.Linear:
+                if type(child) in (nn.Linear, Linear):
                     setattr(parent, name, WOQLinear(child, qcfg))
                     n += 1
         return n
@@ -165,7 +166,7 @@ class InferenceEngine(nn.Module):
         n = 0
         for parent in list(self.module.modules()):
             for name, child in list(parent.named_children()):
-                if type(child) is nn.Linear:
+                if type(child) in (nn.Linear, Linear):
                     setattr(parent, name, FPWOQLinear(child))
                     n += 1
         return n

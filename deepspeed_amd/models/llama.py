@@ -16,7 +16,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from ..ops.linear import SWIGLU, rows_linear, unhooked
+from ..ops.linear import SWIGLU, Linear, rows_linear, unhooked
 from ..ops.norms import RMSNorm
 from ..ops.rope import apply_rope, rope_tables
 from ..ops.swiglu import swiglu
@@ -120,10 +120,10 @@ class LlamaAttention(nn.Module):
         self.head_dim = cfg.head_dim
         h = cfg.hidden_size
         ab = cfg.attention_bias
-        self.q_proj = nn.Linear(h, cfg.num_heads * self.head_dim, bias=ab)
-        self.k_proj = nn.Linear(h, cfg.num_kv_heads * self.head_dim, bias=ab)
-        self.v_proj = nn.Linear(h, cfg.num_kv_heads * self.head_dim, bias=ab)
-        self.o_proj = nn.Linear(cfg.num_heads * self.head_dim, h, bias=False)
+        self.q_proj = Linear(h, cfg.num_heads * self.head_dim, bias=ab)
+        self.k_proj = Linear(h, cfg.num_kv_heads * self.head_dim, bias=ab)
+        self.v_proj = Linear(h, cfg.num_kv_heads * self.head_dim, bias=ab)
+        self.o_proj = Linear(cfg.num_heads * self.head_dim, h, bias=False)
 
     def _out(self, o, residual):
         """Output projection, with the layer's residual if it was handed in."""
@@ -248,9 +248,9 @@ class LlamaMLP(nn.Module):
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
         h, i = cfg.hidden_size, cfg.intermediate_size
-        self.gate_proj = nn.Linear(h, i, bias=False)
-        self.up_proj = nn.Linear(h, i, bias=False)
-        self.down_proj = nn.Linear(i, h, bias=False)
+        self.gate_proj = Linear(h, i, bias=False)
+        self.up_proj = Linear(h, i, bias=False)
+        self.down_proj = Linear(i, h, bias=False)
 
     def forward(self, x, residual=None):
         h = rows_linear(x, (self.gate_proj, self.up_proj), SWIGLU)
@@ -323,7 +323,7 @@ class LlamaForCausalLM(nn.Module):
         super().__init__()
         self.cfg = cfg
         self.model = LlamaModel(cfg)
-        self.lm_head = nn.Linear(cfg.hidden_size, cfg.vocab_size, bias=False)
+        self.lm_head = Linear(cfg.hidden_size, cfg.vocab_size, bias=False)
         if cfg.tie_embeddings:
             self.lm_head.weight = self.model.embed_tokens.weight
         self.apply(self._init_weights)

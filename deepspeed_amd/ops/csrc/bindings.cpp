@@ -88,6 +88,8 @@ extern "C" void ds_transpose_bf16(const void* src, void* dst, int n_batch,
                                   int R, int C, long long row_stride,
                                   int inner, long long inner_stride,
                                   long long outer_stride, void* stream);
+extern "C" void ds_transpose_2d(const void* src, void* dst, int R, int C,
+                                int ld, void* stream);
 extern "C" void ds_fused_softmax(const void* x, const void* mask, void* y,
                                  const float* alibi_slopes, long long rows,
                                  int n, int heads, int sq, int mask_stride,
@@ -250,6 +252,21 @@ at::Tensor transpose_bf16(at::Tensor src, int64_t n_batch, int64_t R,
                     (int)C, row_stride, (int)inner, inner_stride,
                     outer_stride, cur_stream());
   return dst;
+}
+
+// x [R, C] bf16 -> its transpose [C, R], whose rows start on 16 bytes (their
+// stride is R rounded up to 8).
+at::Tensor transpose_2d(at::Tensor x) {
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
+              x.dim() == 2 && x.is_contiguous(), "transpose_2d: bf16 matrix");
+  const int64_t R = x.size(0), C = x.size(1), ld = (R + 7) / 8 * 8;
+  TORCH_CHECK(R < (1ll << 31) && C < (1ll << 31) && (C + 255) / 256 <= 65535,
+              "transpose_2d: size");
+  auto dst = at::empty({C, ld}, x.options());
+  if (R && C)
+    ds_transpose_2d(x.data_ptr(), dst.data_ptr(), (int)R, (int)C, (int)ld,
+                    cur_stream());
+  return dst.narrow(1, 0, R);
 }
 
 at::Tensor fused_softmax(at::Tensor x, c10::optional<at::Tensor> mask,
@@ -805,6 +822,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fused masked/alibi/causal softmax");
   m.def("fused_dropout", &fused_dropout, "fused bias+dropout(+residual)");
   m.def("dropout_bwd", &dropout_bwd, "dropout backward from saved mask");
+  m.def("transpose_2d", &transpose_2d, "bf16 matrix transpose");
   m.def("transpose_bf16", &transpose_bf16, "tiled bf16 batched transpose");
   m.def("fp_quantize", &fp_quantize, "groupwise FP4/6/8/12 quantize");
   m.def("fp_dequantize", &fp_dequantize, "groupwise FP dequantize");

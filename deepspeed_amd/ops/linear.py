@@ -1,9 +1,14 @@
-"""Linear layers of a few rows (decoding): the weight-streaming kernel of
+"""Linear layers.
+
+``Linear`` is torch's, with a backward whose products read their operands along
+the contiguous axis (see ``_Linear``).
+
+``rows_linear``, for a few rows (decoding): the weight-streaming kernel of
 csrc/rows_linear.hip in place of a library GEMM, with several layers of one
 input in one launch and the gate's activation or the residual in its epilogue.
 
-``rows_linear`` takes the modules themselves and returns None wherever calling
-them is the thing to do: with gradients, hooks, autocast, other types, sharded
+It takes the modules themselves and returns None wherever calling them is the
+thing to do: with gradients, hooks, autocast, other types, sharded
 or replaced modules, or more rows than the kernel is the faster one for."""
 
 import torch
@@ -17,6 +22,98 @@ from ._loader import get_ext
 ROWS, ROWS_INT8 = 32, 64
 
 PLAIN, SWIGLU = 0, 1
+
+# What the library's bf16 products reach for the input's gradient, with the
+# weight as stored and transposed (FLOP/s: 1140 to 1425 and 1500 to 1660 over
+# 8192 rows), and the transposing kernel (bytes/s, seconds a launch).
+DGRAD, DGRAD_T = 1220e12, 1530e12
+STREAM, LAUNCH = 5e12, 5e-6
+
+
+def backward_plan(T: int, N: int, K: int):
+    """Which operands to transpose in the backward of a layer [N, K] over T
+    rows: (weight, for the input's gradient; gradient, input, for the
+    weight's). A product reads an operand along the contracted axis faster than
+    across it, and transposing costs a read and a write.
+
+    Weight: pays from some 3000 rows (N 14336, K 4096, us as stored and
+    transposed: 2048 rows 211 / 257, 4000 340 / 344, 8192 708 / 647).
+    Gradient of the weight: both operands lie across. Transposing the narrower
+    is within 7% of the best choice over all sizes measured (8192 rows: 14336 x
+    4096 993 / 756, both 741; 4096 x 14336 994 / 785, both 734; 128256 x 4096
+    7178 / 6247, both 6364). Outputs under 256 tiles of 256 x 256 and fewer
+    rows stay: there the library splits the contraction over more of the chip
+    in its own layout (3072 x 3072 over 32768 rows 598 / 994, 14336 x 4096 over
+    1000 rows 160 / 161)."""
+    flops = 2.0 * T * N * K
+    w = flops / DGRAD_T + 4.0 * N * K / STREAM + LAUNCH < flops / DGRAD
+    big = N * K >= 1 << 24 and T >= 2048
+    return w, big and N < K, big and N >= K
+
+
+class _Linear(torch.autograd.Function):
+    """x W^T + b whose backward lays operands out for the matrix product:
+    dx = dy W reads W across its rows, and dW = dy^T x reads both across
+    theirs, at two thirds of the forward product's rate. Transposing costs a
+    read and a write of an operand and pays where ``backward_plan`` says."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias):
+        ctx.save_for_backward(x, weight)
+        return nn.functional.linear(x, weight, bias)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        need_x, need_w, need_b = ctx.needs_input_grad
+        N, K = weight.shape
+        dy2, x2 = dy.reshape(-1, N), x.reshape(-1, K)
+        T = x2.shape[0]
+        w_t = dy_t = x_t = False
+        # differentiable products where the gradient itself is differentiated
+        if not torch.is_grad_enabled() and dy.dtype is torch.bfloat16:
+            w_t, dy_t, x_t = backward_plan(T, N, K)
+        dx = dw = db = None
+        if need_x:
+            dx = nn.functional.linear(dy2, _transposed(weight)) if w_t \
+                else dy2 @ weight
+            dx = dx.view(x.shape)
+        if need_w:
+            a = _transposed(dy2) if dy_t else dy2.t()
+            b = _transposed(x2).t() if x_t else x2
+            dw = a @ b
+        if need_b:
+            db = dy2.sum(0)
+        return dx, dw, db
+
+
+def _transposed(a: torch.Tensor) -> torch.Tensor:
+    return get_ext().transpose_2d(a.contiguous())
+
+
+def _plain_autograd() -> bool:
+    """No transform or tangent is about that an autograd function without
+    rules of its own would stop."""
+    return (torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0
+            and not torch.compiler.is_compiling()
+            and not torch.is_autocast_enabled()
+            and not torch.jit.is_tracing())
+
+
+class Linear(nn.Linear):
+    """nn.Linear with the backward of ``_Linear`` on a GPU."""
+
+    def forward(self, x):
+        w = self.weight
+        if (torch.is_grad_enabled() and x.is_cuda and x.dim() > 1
+                and type(x) is torch.Tensor and type(w) is nn.Parameter
+                and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16
+                and w.is_contiguous() and w.dim() == 2
+                and get_ext() is not None and _plain_autograd()
+                and x.numel() and x.shape[-1] == w.shape[1]):
+            return _Linear.apply(x, w, self.bias)
+        return nn.functional.linear(x, w, self.bias)
 
 
 def unhooked(mod: nn.Module) -> bool:
@@ -49,7 +146,7 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN, residual=None,
     for m in mods:
         if type(m) is not kind or not (hooks_ran or unhooked(m)):
             return None
-        if kind is nn.Linear:
+        if kind is Linear or kind is nn.Linear:
             w = m.weight
             if M > ROWS or w.dtype is not torch.bfloat16 or \
                     type(w) is not nn.Parameter or w.shape[1:] != (K,):
