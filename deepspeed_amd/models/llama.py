@@ -125,15 +125,12 @@ class LlamaAttention(nn.Module):
         self.v_proj = Linear(h, cfg.num_kv_heads * self.head_dim, bias=ab)
         self.o_proj = Linear(cfg.num_heads * self.head_dim, h, bias=False)
 
-    def _out(self, o, residual):
-        """Output projection, with the layer's residual if it was handed in."""
-        if residual is not None:
-            y = rows_linear(o, (self.o_proj,), residual=residual)
-            return residual + self.o_proj(o) if y is None else y[0]
-        return self.o_proj(o)
+    def _out(self, o):
+        y = rows_linear(o, (self.o_proj,))
+        return self.o_proj(o) if y is None else y[0]
 
     def forward(self, x, cos, sin, positions=None, kv_cache=None,
-                attention_fn=None, residual=None):
+                attention_fn=None):
         B, S, _ = x.shape
         qkv = rows_linear(x, (self.q_proj, self.k_proj, self.v_proj))
         if qkv is None:
@@ -148,7 +145,7 @@ class LlamaAttention(nn.Module):
                                         positions)
             if o is not None:
                 kv_cache.last_decoded = S == 1
-                return self._out(o.reshape(B, S, -1), residual)
+                return self._out(o.reshape(B, S, -1))
         q = apply_rope(q, cos, sin, positions)
         k = apply_rope(k, cos, sin, positions)
 
@@ -156,7 +153,7 @@ class LlamaAttention(nn.Module):
             # Ulysses: all-to-all scatters heads / gathers the sequence so
             # each rank runs full-sequence causal attention on H/P heads
             o = self._ulysses_attn(q, k, v)
-            return self._out(o.reshape(B, S, -1), residual)
+            return self._out(o.reshape(B, S, -1))
 
         if kv_cache is None and attention_fn is None:
             from ..ops.attention import (flash_attn_available, flash_attn_fwd,
@@ -166,11 +163,11 @@ class LlamaAttention(nn.Module):
                 # hand-written CDNA4 MFMA flash kernel, BSHD layout — skips
                 # the transpose entirely (inference/no-grad prefill path)
                 o = flash_attn_fwd(q, k, v, causal=True)
-                return self._out(o.reshape(B, S, -1), residual)
+                return self._out(o.reshape(B, S, -1))
             if torch.is_grad_enabled() and flash_train_available(q, k):
                 # differentiable hand-written path (fwd + dk/dv/dq kernels)
                 o = flash_attn_func(q, k, v, causal=True)
-                return self._out(o.reshape(B, S, -1), residual)
+                return self._out(o.reshape(B, S, -1))
 
         if (S == 1 and kv_cache is not None
                 and hasattr(kv_cache, "decode_attention")
@@ -180,7 +177,7 @@ class LlamaAttention(nn.Module):
             o = kv_cache.decode_attention(self.layer_idx, q, k, v)
             if o is not None:
                 kv_cache.last_decoded = True
-                return self._out(o.reshape(B, S, -1), residual)
+                return self._out(o.reshape(B, S, -1))
 
         # [B, H, S, D] for SDPA
         q = q.transpose(1, 2)
@@ -200,7 +197,7 @@ class LlamaAttention(nn.Module):
             o = sdpa_gqa(q, k, v,
                          causal=attn_mask is None and q.size(2) == k.size(2),
                          attn_mask=attn_mask)
-        return self._out(o.transpose(1, 2).reshape(B, S, -1), residual)
+        return self._out(o.transpose(1, 2).reshape(B, S, -1))
 
 
 def _bshd_causal_attention(q, k, v):
@@ -252,13 +249,22 @@ class LlamaMLP(nn.Module):
         self.up_proj = Linear(h, i, bias=False)
         self.down_proj = Linear(i, h, bias=False)
 
-    def forward(self, x, residual=None):
+    def forward(self, x):
         h = rows_linear(x, (self.gate_proj, self.up_proj), SWIGLU)
         h = swiglu(self.gate_proj(x), self.up_proj(x)) if h is None else h[0]
-        if residual is not None:
-            y = rows_linear(h, (self.down_proj,), residual=residual)
-            return residual + self.down_proj(h) if y is None else y[0]
-        return self.down_proj(h)
+        y = rows_linear(h, (self.down_proj,))
+        return self.down_proj(h) if y is None else y[0]
+
+
+def add_norm(norm, x, delta):
+    """(norm of the residual stream x with a sublayer's output added, the new
+    stream); one kernel where nothing watches or replaces the norm."""
+    if delta is None:
+        return norm(x), x
+    if type(norm) is RMSNorm and unhooked(norm, internal_ok=True):
+        return norm(delta, residual=x)
+    x = x + delta
+    return norm(x), x
 
 
 class LlamaDecoderLayer(nn.Module):
@@ -270,21 +276,18 @@ class LlamaDecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, eps=cfg.rms_eps)
         self.mlp = LlamaMLP(cfg)
 
+    def chain(self, x, delta, cos, sin, positions=None, kv_cache=None):
+        """The layer on a residual stream x that still lacks the last
+        sublayer's output ``delta`` (or None); returns it the same way, so that
+        every add happens inside the norm behind it."""
+        h, x = add_norm(self.input_layernorm, x, delta)
+        h, x = add_norm(self.post_attention_layernorm, x,
+                        self.self_attn(h, cos, sin, positions, kv_cache))
+        return x, self.mlp(h)
+
     def forward(self, x, cos, sin, positions=None, kv_cache=None):
-        # serving: the residual goes along and is added where the sublayer's
-        # last product is written
-        if torch.is_grad_enabled() or type(self.self_attn) is not \
-                LlamaAttention or not unhooked(self.self_attn):
-            x = x + self.self_attn(self.input_layernorm(x), cos, sin,
-                                   positions, kv_cache)
-        else:
-            x = self.self_attn(self.input_layernorm(x), cos, sin, positions,
-                               kv_cache, residual=x)
-        h = self.post_attention_layernorm(x)
-        if torch.is_grad_enabled() or type(self.mlp) is not LlamaMLP or \
-                not unhooked(self.mlp):
-            return x + self.mlp(h)
-        return self.mlp(h, residual=x)
+        x, delta = self.chain(x, None, cos, sin, positions, kv_cache)
+        return x + delta
 
 
 class LlamaModel(nn.Module):
@@ -306,13 +309,18 @@ class LlamaModel(nn.Module):
                      and torch.is_grad_enabled())
         if recompute:
             from ..runtime.activation_checkpointing import checkpoint
+        delta = None
         for layer in self.layers:
             if recompute:
                 x = checkpoint(lambda x_, l=layer: l(x_, cos, sin, positions,
                                                      kv_cache), x)
+            elif type(layer) is LlamaDecoderLayer and unhooked(layer):
+                x, delta = layer.chain(x, delta, cos, sin, positions,
+                                       kv_cache)
             else:
-                x = layer(x, cos, sin, positions, kv_cache)
-        return self.norm(x)
+                x = x if delta is None else x + delta
+                x, delta = layer(x, cos, sin, positions, kv_cache), None
+        return add_norm(self.norm, x, delta)[0]
 
     def gradient_checkpointing_enable(self):
         self.gradient_checkpointing = True

@@ -25,10 +25,17 @@ extern "C" void ds_fused_lamb(float* p, const void* g, int grad_dtype,
 extern "C" void ds_norm_fwd(const void* x, const void* w, const void* b,
                             void* y, float* invrms, float* mean, int rows,
                             int H, float eps, int ln, int dtype, void* stream);
+extern "C" void ds_add_norm_fwd(const void* x, const void* res, const void* w,
+                                void* sum, void* y, float* invrms, int rows,
+                                int H, float eps, int dtype, void* stream);
+extern "C" long long ds_norm_bwd_parts(const void* dy, const void* x,
+                                       const void* dres, const void* dx,
+                                       int rows, int H, int ln, int dtype);
 extern "C" void ds_norm_bwd(const void* dy, const void* x, const void* w,
-                            const float* invrms, const float* mean, void* dx,
-                            float* dw, float* db, int rows, int H, int ln,
-                            int dtype, void* stream);
+                            const float* invrms, const float* mean,
+                            const void* dres, void* dx, float* dwb,
+                            float* part, int rows, int H, int ln, int dtype,
+                            void* stream);
 extern "C" void ds_rope(void* x, const float* cos_table, const float* sin_table,
                         const int* positions, long long batch, long long seq,
                         long long heads, long long dim, int bwd, int dtype,
@@ -82,7 +89,7 @@ extern "C" void ds_paged_rows(const void* q, const void* kpool,
 extern "C" void ds_rows_linear(const void* x, int layers, const void* const* w,
                                const float* const* scales,
                                const void* const* bias, void* const* out,
-                               const int* n, const void* residual, int M,
+                               const int* n, int M,
                                int K, int group, int mode, void* stream);
 extern "C" void ds_transpose_bf16(const void* src, void* dst, int n_batch,
                                   int R, int C, long long row_stride,
@@ -436,12 +443,12 @@ at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
 
 // Linear layers on one input of a few rows (rows_linear.hip). weights: bf16
 // [N, K], or int8 (any shape, N * K long) with their groupwise scales.
-// mode 1 returns silu(layer 0) * layer 1. residual is added to the first.
+// mode 1 returns silu(layer 0) * layer 1.
 std::vector<at::Tensor> rows_linear(
     at::Tensor x, std::vector<at::Tensor> weights,
     std::vector<at::Tensor> scales,
-    std::vector<c10::optional<at::Tensor>> biases,
-    c10::optional<at::Tensor> residual, int64_t group, int64_t mode) {
+    std::vector<c10::optional<at::Tensor>> biases, int64_t group,
+    int64_t mode) {
   const int L = weights.size();
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
               x.is_contiguous() && x.dim() == 2, "rows_linear: x");
@@ -485,14 +492,7 @@ std::vector<at::Tensor> rows_linear(
   }
   TORCH_CHECK(mode == 0 || n[0] == n[1], "rows_linear: gate and up");
   TORCH_CHECK(((uintptr_t)x.data_ptr() & 15) == 0, "rows_linear: alignment");
-  const void* res = nullptr;
-  if (residual.has_value()) {
-    TORCH_CHECK(residual->is_cuda() && residual->is_contiguous() &&
-                residual->scalar_type() == at::kBFloat16 &&
-                residual->numel() == M * n[0], "rows_linear: residual");
-    res = residual->data_ptr();
-  }
-  ds_rows_linear(x.data_ptr(), L, w, i8 ? sc : nullptr, b, o, n, res, (int)M,
+  ds_rows_linear(x.data_ptr(), L, w, i8 ? sc : nullptr, b, o, n, (int)M,
                  (int)K, (int)group, (int)mode, cur_stream());
   return out;
 }
@@ -566,24 +566,66 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_fwd(
   return {y, invrms, mean};
 }
 
+// dres (RMS only): a further gradient of x, added to dx.
 std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_bwd(
     at::Tensor dy, at::Tensor x, at::Tensor w, at::Tensor invrms,
-    c10::optional<at::Tensor> mean, bool layernorm) {
+    c10::optional<at::Tensor> mean, bool layernorm,
+    c10::optional<at::Tensor> dres) {
   TORCH_CHECK(dy.is_contiguous() && x.is_contiguous() && w.is_contiguous(),
               "must be contiguous");
   const int64_t H = x.size(-1);
   const int64_t rows = x.numel() / H;
   auto dx = at::empty_like(x);
   auto f32opts = x.options().dtype(at::kFloat);
-  auto dw = at::zeros({H}, f32opts);
-  auto db = layernorm ? at::zeros({H}, f32opts) : at::empty({0}, f32opts);
-  ds_norm_bwd(dy.data_ptr(), x.data_ptr(), w.data_ptr(),
-              invrms.data_ptr<float>(),
-              layernorm ? mean->data_ptr<float>() : nullptr, dx.data_ptr(),
-              dw.data_ptr<float>(), layernorm ? db.data_ptr<float>() : nullptr,
-              (int)rows, (int)H, layernorm ? 1 : 0, dtype_code(x),
-              cur_stream());
-  return {dx, dw, db};
+  const void* rp = nullptr;
+  if (dres.has_value()) {
+    TORCH_CHECK(!layernorm && dres->is_contiguous() &&
+                dres->scalar_type() == x.scalar_type() &&
+                dres->numel() == x.numel(), "norm_bwd: dres");
+    rp = dres->data_ptr();
+  }
+  const int code = dtype_code(x), ln = layernorm ? 1 : 0;
+  const long long n = rows ? ds_norm_bwd_parts(
+      dy.data_ptr(), x.data_ptr(), rp, dx.data_ptr(), (int)rows, (int)H, ln,
+      code) : 0;
+  auto part = at::empty({n}, f32opts);
+  const int64_t width = layernorm ? 2 * H : H;
+  auto dwb = n ? at::empty({width}, f32opts) : at::zeros({width}, f32opts);
+  if (rows)
+    ds_norm_bwd(dy.data_ptr(), x.data_ptr(), w.data_ptr(),
+                invrms.data_ptr<float>(),
+                layernorm ? mean->data_ptr<float>() : nullptr, n ? rp : nullptr,
+                dx.data_ptr(), dwb.data_ptr<float>(),
+                n ? part.data_ptr<float>() : nullptr, (int)rows, (int)H, ln,
+                code, cur_stream());
+  if (rp != nullptr && !n) dx.add_(*dres);
+  return {dx, dwb.narrow(0, 0, H),
+          layernorm ? dwb.narrow(0, H, H) : at::empty({0}, f32opts)};
+}
+
+// RMS norm of x + res -> (norm, sum, 1/rms). The caller sees to the sizes
+// (ops/norms.py, add_norm_eligible).
+std::tuple<at::Tensor, at::Tensor, at::Tensor> add_norm_fwd(
+    at::Tensor x, at::Tensor res, at::Tensor w, double eps) {
+  const int64_t H = x.size(-1);
+  for (auto& t : {x, res})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
+                t.scalar_type() == w.scalar_type() &&
+                t.sizes() == x.sizes() &&
+                (t.scalar_type() == at::kBFloat16 ||
+                 t.scalar_type() == at::kHalf) &&
+                ((uintptr_t)t.data_ptr() & 15) == 0, "add_norm_fwd");
+  TORCH_CHECK(H % 8 == 0 && H > 0 && H <= 16384 && w.numel() == H &&
+              w.is_cuda() && w.is_contiguous(), "add_norm_fwd: size");
+  const int64_t rows = x.numel() / H;
+  auto y = at::empty_like(x), sum = at::empty_like(x);
+  auto inv = at::empty({rows}, x.options().dtype(at::kFloat));
+  if (rows)
+    ds_add_norm_fwd(x.data_ptr(), res.data_ptr(), w.data_ptr(),
+                    sum.data_ptr(), y.data_ptr(), inv.data_ptr<float>(),
+                    (int)rows, (int)H, (float)eps, dtype_code(x),
+                    cur_stream());
+  return {y, sum, inv};
 }
 
 at::Tensor token_gather(at::Tensor x, at::Tensor idx) {
@@ -849,7 +891,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         },
         "Host Lion on flat fp32 master");
   m.def("norm_fwd", &norm_fwd, "RMSNorm/LayerNorm forward");
-  m.def("norm_bwd", &norm_bwd, "RMSNorm/LayerNorm backward");
+  m.def("norm_bwd", &norm_bwd, "RMSNorm/LayerNorm backward",
+        pybind11::arg("dy"), pybind11::arg("x"), pybind11::arg("w"),
+        pybind11::arg("invrms"), pybind11::arg("mean"),
+        pybind11::arg("layernorm"), pybind11::arg("dres") = c10::nullopt);
+  m.def("add_norm_fwd", &add_norm_fwd, "RMS norm of a sum, and the sum");
   m.def("rope", &rope, "Rotary position embedding (in-place)");
   m.def("token_gather", &token_gather,
         "row-coalesced token gather [B,S,D] x [B,K] -> [B,K,D]");

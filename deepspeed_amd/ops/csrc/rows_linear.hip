@@ -25,8 +25,8 @@
 //     the weight is not written out as bf16 and read again. N 14336, K 4096, M
 //     8: 21.8 us; dequantizing took 85 us and the product 28.
 //   * Several layers on one input (q, k, v; gate and up) are one launch, and
-//     the epilogue takes the gate's activation, the bias and the residual with
-//     it: a decoder layer has 9 launches instead of 16.
+//     the epilogue takes the gate's activation and the bias with it: four
+//     launches a decoder layer instead of eight.
 
 #include "ds_kernels.h"
 
@@ -49,7 +49,6 @@ struct Args {
   short* out[MAXL];
   int n[MAXL], tile_end[MAXL];
   const short* x;
-  const short* residual;    // added to layer 0's output, or null
   int M, K, group;
 };
 
@@ -221,7 +220,6 @@ __global__ __launch_bounds__(NW * 64) void rows_linear_kernel(const Args a) {
       float o = y[0];
       if (MODE == SWIGLU) o = y[0] / (1.f + expf(-y[0])) * y[L - 1];
       const long long to = (long long)r * N + n;
-      if (a.residual && layer == 0) o += value(a.residual[to]);
       a.out[layer][to] = bits(o);
     }
   }
@@ -272,7 +270,7 @@ void launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
 extern "C" void ds_rows_linear(const void* x, int layers, const void* const* w,
                                const float* const* scales,
                                const void* const* bias, void* const* out,
-                               const int* n, const void* residual, int M,
+                               const int* n, int M,
                                int K, int group, int mode,
                                void* stream) {
   Args a = {};
@@ -284,7 +282,6 @@ extern "C" void ds_rows_linear(const void* x, int layers, const void* const* w,
     a.n[i] = n[i];
   }
   a.x = (const short*)x;
-  a.residual = (const short*)residual;
   a.M = M; a.K = K; a.group = group;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (scales) launch_rows<true>(a, layers, mode, st);

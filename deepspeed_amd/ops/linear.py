@@ -5,7 +5,7 @@ the contiguous axis (see ``_Linear``).
 
 ``rows_linear``, for a few rows (decoding): the weight-streaming kernel of
 csrc/rows_linear.hip in place of a library GEMM, with several layers of one
-input in one launch and the gate's activation or the residual in its epilogue.
+input in one launch and the gate's activation in its epilogue.
 
 It takes the modules themselves and returns None wherever calling them is the
 thing to do: with gradients, hooks, autocast, other types, sharded
@@ -110,28 +110,32 @@ class Linear(nn.Linear):
                 and type(x) is torch.Tensor and type(w) is nn.Parameter
                 and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16
                 and w.is_contiguous() and w.dim() == 2
-                and get_ext() is not None and _plain_autograd()
-                and x.numel() and x.shape[-1] == w.shape[1]):
+                and x.numel() and x.shape[-1] == w.shape[1]
+                and any(backward_plan(x.numel() // w.shape[1], *w.shape))
+                and get_ext() is not None and _plain_autograd()):
             return _Linear.apply(x, w, self.bias)
         return nn.functional.linear(x, w, self.bias)
 
 
-def unhooked(mod: nn.Module) -> bool:
-    """No hook sees the module's call: its work may move elsewhere."""
-    return not (mod._forward_hooks or mod._forward_pre_hooks
-                or mod._backward_hooks or mod._backward_pre_hooks
+def unhooked(mod: nn.Module, internal_ok: bool = False) -> bool:
+    """No hook sees the module's call: its work may move elsewhere. With
+    ``internal_ok`` the call itself stays, in another form that the
+    framework's own hooks (marked ``_ds_internal``) take as well."""
+    own = (mod._forward_hooks, mod._forward_pre_hooks, mod._backward_hooks,
+           mod._backward_pre_hooks)
+    return not (any(not (internal_ok and getattr(h, "_ds_internal", False))
+                    for hooks in own if hooks for h in hooks.values())
                 or _module._global_forward_hooks
                 or _module._global_forward_pre_hooks
                 or _module._global_backward_hooks
                 or _module._global_backward_pre_hooks)
 
 
-def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN, residual=None,
+def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
                 hooks_ran: bool = False):
     """Outputs of the linear modules ``mods`` on x [..., K], a list: one each,
-    or with ``SWIGLU`` silu(first) * second. ``residual`` is added to the first
-    output. ``hooks_ran``: called from inside the module's own call. None when
-    ineligible."""
+    or with ``SWIGLU`` silu(first) * second. ``hooks_ran``: called from inside
+    the module's own call. None when ineligible."""
     if torch.is_grad_enabled() or not x.is_cuda or \
             x.dtype is not torch.bfloat16 or type(x) is not torch.Tensor:
         return None
@@ -169,12 +173,8 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN, residual=None,
             return None
         weights.append(w)
         biases.append(b)
-    if residual is not None and (residual.dtype is not torch.bfloat16 or
-                                 not residual.is_contiguous()):
-        return None
     x2 = x.reshape(M, K).contiguous()
     if x2.data_ptr() % 16:
         return None
-    out = get_ext().rows_linear(x2, weights, scales, biases, residual, group,
-                                mode)
+    out = get_ext().rows_linear(x2, weights, scales, biases, group, mode)
     return [o.view(*x.shape[:-1], o.shape[-1]) for o in out]

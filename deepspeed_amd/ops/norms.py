@@ -94,6 +94,44 @@ class _LayerNormFn(torch.autograd.Function):
         return dx, dw.to(weight.dtype), grad_bias, None
 
 
+class _AddNormFn(torch.autograd.Function):
+    """RMS norm of x + residual, and the sum itself (GPU, 16-bit)."""
+
+    @staticmethod
+    def forward(ctx, x, residual, weight, eps):
+        y, total, invrms = get_ext().add_norm_fwd(x, residual, weight, eps)
+        ctx.save_for_backward(total, weight, invrms)
+        ctx.set_materialize_grads(False)
+        return y, total
+
+    @staticmethod
+    def backward(ctx, dy, dtotal):
+        total, weight, invrms = ctx.saved_tensors
+        if dy is None:
+            return dtotal, dtotal, None, None
+        if dtotal is not None:
+            dtotal = dtotal.contiguous()
+        dx, dw, _ = get_ext().norm_bwd(dy.contiguous(), total,
+                                       weight.contiguous(), invrms, None,
+                                       False, dtotal)
+        return dx, dx, dw.to(weight.dtype), None
+
+
+def add_rms_norm(x, residual, weight, eps=1e-6):
+    """(RMS norm of ``residual + x``, ``residual + x``). One kernel each way
+    where the types and sizes allow, which takes the norm from the fp32 sum."""
+    if (x.is_cuda and get_ext() is not None and x.shape == residual.shape
+            and x.dtype in (torch.bfloat16, torch.float16)
+            and x.dtype == residual.dtype == weight.dtype
+            and x.shape[-1] % 8 == 0 and 0 < x.shape[-1] <= 16384):
+        x, residual = x.contiguous(), residual.contiguous()
+        weight = weight.contiguous()
+        if x.data_ptr() % 16 == 0 and residual.data_ptr() % 16 == 0:
+            return _AddNormFn.apply(x, residual, weight, eps)
+    total = residual + x
+    return _RMSNormFn.apply(total, weight, eps), total
+
+
 def rms_norm(x, weight, eps=1e-6):
     return _RMSNormFn.apply(x, weight, eps)
 
@@ -112,8 +150,12 @@ class RMSNorm(torch.nn.Module):
     def reset_parameters(self):
         torch.nn.init.ones_(self.weight)
 
-    def forward(self, x):
-        return _RMSNormFn.apply(x, self.weight, self.eps)
+    def forward(self, x, residual=None):
+        """The norm of x; with ``residual`` that of residual + x, and the
+        sum."""
+        if residual is None:
+            return _RMSNormFn.apply(x, self.weight, self.eps)
+        return add_rms_norm(x, residual, self.weight, self.eps)
 
     def extra_repr(self):
         return f"{self.weight.numel()}, eps={self.eps}"

@@ -657,6 +657,11 @@ class ZeroStage3Optimizer:
             self._ensure_grad_buffer(u)
         self._drain_inflight_rs(limit=self._max_inflight_rs)
 
+    # these see to the module's parameters only, whatever it is called with
+    for _hook in (_pre_forward_hook, _post_forward_hook, _pre_backward_hook):
+        _hook._ds_internal = True
+    del _hook
+
     def _ensure_grad_buffer(self, u: _Unit):
         """Allocate the unit's flat grad landing buffer UNZEROED. Grads are
         copied in by the post-accumulate hook (first arrival = copy, later

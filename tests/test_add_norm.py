@@ -1,0 +1,99 @@
+"""RMS norm of a residual stream with a sublayer's output added: which calls
+take the fused kernel, and both ways against fp64."""
+
+import pytest
+import torch
+
+from deepspeed_amd.models import llama
+from deepspeed_amd.ops.linear import unhooked
+from deepspeed_amd.ops.norms import RMSNorm, add_rms_norm, rms_norm
+
+
+def test_cpu_is_add_then_norm():
+    torch.manual_seed(0)
+    x, r, w = torch.randn(3, 5, 16), torch.randn(3, 5, 16), torch.randn(16)
+    y, s = add_rms_norm(x, r, w, 1e-5)
+    assert torch.equal(s, r + x) and torch.equal(y, rms_norm(r + x, w, 1e-5))
+
+
+def test_hooked_or_replaced_layers_see_their_calls():
+    """A hook on a norm or a layer, or another module in its place, gets what
+    it got: one tensor in, one out, and the same loss."""
+    torch.manual_seed(0)
+    model = llama.LlamaForCausalLM(llama.llama_tiny())
+    ids = torch.randint(0, 512, (2, 9))
+    want = model(ids, labels=ids)
+    seen = []
+    norm = model.model.layers[1].post_attention_layernorm
+    assert unhooked(norm)
+    h1 = norm.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    h2 = model.model.layers[0].register_forward_hook(
+        lambda m, i, o: seen.append(o.shape))
+    assert torch.equal(model(ids, labels=ids), want)
+    assert len(seen) == 2
+    h1.remove(), h2.remove()
+
+    class Other(torch.nn.Module):
+        def forward(self, x):
+            return norm(x)
+
+    model.model.layers[1].post_attention_layernorm = Other()
+    assert torch.equal(model(ids, labels=ids), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,h", [(1, 8), (3, 2040), (7, 2048), (1030, 4096),
+                                    (5000, 1024), (9, 8192), (4, 8200),
+                                    (3, 16384), (5, 20), (2, 16392)])
+@pytest.mark.parametrize("used", ["both", "norm", "sum"])
+def test_add_norm_gpu(dtype, rows, h, used):
+    g = torch.Generator().manual_seed(rows + h)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=g).to(dtype).cuda()
+
+    x, r, w = rand(rows, h).requires_grad_(), rand(rows, h), rand(h)
+    r.requires_grad_(), w.requires_grad_()
+    dy, ds = rand(rows, h), rand(rows, h)
+    norm = RMSNorm(h, eps=1e-5)
+    norm.weight = torch.nn.Parameter(w.detach().clone())
+    y, s = norm(x, residual=r)
+    eps = torch.finfo(dtype).eps
+    xd, rd, wd = (t.detach().double().requires_grad_() for t in (x, r, w))
+    sd = xd + rd
+    yd = sd * torch.rsqrt(sd.square().mean(-1, keepdim=True) + 1e-5) * wd
+    # a rounding or two of values that are sums of two
+    lim = 2 * eps * (1 + yd.abs())
+    assert ((y.double() - yd).abs() <= lim).all()
+    assert ((s.double() - sd).abs() <= eps * (1 + sd.abs())).all()
+    loss = sum((a * b).sum() for a, b, n in ((y, dy, "norm"), (s, ds, "sum"))
+               if used in ("both", n))
+    want = sum((a * b.double()).sum() for a, b, n in ((yd, dy, "norm"),
+                                                      (sd, ds, "sum"))
+               if used in ("both", n))
+    loss.backward()
+    want.backward()
+    if used == "sum":
+        assert torch.equal(x.grad, ds) and torch.equal(r.grad, ds)
+        return
+    assert torch.equal(x.grad, r.grad)
+    top = xd.grad.abs().amax(-1, keepdim=True) + 1
+    assert ((x.grad.double() - xd.grad).abs() <= 4 * eps * top).all()
+    got = norm.weight.grad.double()
+    # the sum is rounded to 16 bits before the backward reads it again
+    assert (got - wd.grad).norm() <= 2 * eps * (wd.grad.norm() + 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 4, 1029])
+def test_norm_weight_gradient_repeats(rows):
+    torch.manual_seed(0)
+    x = torch.randn(rows, 1024, device="cuda").bfloat16()
+    dy = torch.randn_like(x)
+    grads = []
+    for _ in range(3):
+        w = torch.ones(1024, device="cuda").bfloat16().requires_grad_()
+        rms_norm(x, w).backward(dy)
+        grads.append(w.grad)
+    assert torch.equal(grads[0], grads[1]) and torch.equal(grads[0], grads[2])

@@ -75,9 +75,6 @@ def test_rows_linear_gpu(int8, m, sizes):
     for (lin, want), y in zip(both, got):
         assert y.shape == (1, m, y.shape[-1])
         _close(y, want(x))
-    res = torch.randn(1, m, ns[0], generator=g).bfloat16().cuda()
-    y, = rows_linear(x, (both[0][0],), residual=res)
-    _close(y, both[0][1](x) + res.double())
     if int8:
         _close(both[0][0](x), both[0][1](x))
     h = both[0][0].register_forward_hook(lambda *a: None)
