@@ -1,13 +1,9 @@
-"""Flash-attention forward (hand-written CDNA4 MFMA kernel).
-
-See csrc/attention.hip for the kernel design (probe-verified MFMA
-layouts, swapped-QK^T online softmax). This wrapper owns the V transpose
-(the kernel consumes vt[B,Hkv,D,S] so its PV fragments are contiguous
-16-byte loads) and the eligibility check, falling back to torch SDPA where
-the kernel does not apply (training backward, D!=128, ragged seq, CPU).
-"""
+"""Flash attention on the matrix cores (csrc/attention.hip), forward and
+backward: heads of 64, 96 and 128, any sequence length, grouped key heads, bf16.
+Elsewhere callers take torch's scaled_dot_product_attention."""
 
 import math
+import os
 from typing import Optional
 
 import torch
@@ -17,28 +13,45 @@ from ._loader import get_ext
 
 def _eligible(q: torch.Tensor, k: torch.Tensor) -> bool:
     return (get_ext() is not None and q.is_cuda
-            and q.dtype == torch.bfloat16
-            and q.size(-1) == 128 and q.size(1) % 32 == 0
-            and q.size(1) == k.size(1))
+            and q.dtype == k.dtype == torch.bfloat16
+            and q.dim() == 4 and k.dim() == 4
+            and q.size(-1) == k.size(-1) and q.size(-1) in (64, 96, 128)
+            and q.size(1) == k.size(1) and q.size(2) % k.size(2) == 0
+            and q.numel() > 0)
 
 
 def flash_attn_available(q: torch.Tensor, k: torch.Tensor) -> bool:
-    """Inference/prefill forward: ON by default (v3 kernel beats aotriton
-    SDPA on the bench shape, 417 vs <=402 TF). DS_AMD_FLASH=0 opts out."""
-    import os
+    """Inference/prefill forward; DS_AMD_FLASH=0 opts out."""
     if os.environ.get("DS_AMD_FLASH", "1") == "0":
         return False
     return _eligible(q, k) and not torch.is_grad_enabled()
 
 
 def flash_train_available(q: torch.Tensor, k: torch.Tensor) -> bool:
-    """Training fwd+bwd path (FlashAttnFunc). Gated by DS_AMD_FLASH_TRAIN
-    until the v2 backward beats the aotriton backward on the bench shape
-    (flip the default then)."""
-    import os
-    if os.environ.get("DS_AMD_FLASH_TRAIN", "0") != "1":
+    """Training forward and backward (FlashAttnFunc); DS_AMD_FLASH_TRAIN=0
+    opts out."""
+    if os.environ.get("DS_AMD_FLASH_TRAIN", "1") == "0":
         return False
-    return _eligible(q, k)
+    from .linear import _plain_autograd
+    return _eligible(q, k) and _plain_autograd()
+
+
+def _rows(x: torch.Tensor) -> torch.Tensor:
+    """x as the kernels read it: unit stride inside a head, 16-byte rows."""
+    if x.stride(3) == 1 and x.data_ptr() % 16 == 0 and all(
+            x.stride(d) % 8 == 0 and x.stride(d) >= 0 for d in range(3)) and \
+            x.stride(1) < 1 << 24:
+        return x
+    return x.clone(memory_format=torch.contiguous_format)
+
+
+def _scaled(q, scale):
+    """(q, scale, factor of dq) with a positive scale: the kernels take maxima
+    of unscaled scores."""
+    scale = scale if scale is not None else 1.0 / math.sqrt(q.size(-1))
+    if scale > 0:
+        return q, scale, 1
+    return (-q, -scale, -1) if scale < 0 else (torch.zeros_like(q), 1.0, 0)
 
 
 def _vt_from_bshd(v):
@@ -67,11 +80,9 @@ def flash_attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                    scale: Optional[float] = None) -> torch.Tensor:
     """q,k,v: [B, S, H(kv), D] bf16 -> o [B, S, H, D]. Inference/prefill
     only (no autograd)."""
-    ext = get_ext()
-    scale = scale if scale is not None else 1.0 / math.sqrt(q.size(-1))
-    vt = _vt_from_bshd(v)  # [B, Hkv, D, S]
-    return ext.flash_attn_fwd(q.contiguous(), k.contiguous(), vt, scale,
-                              causal)
+    q, scale, _ = _scaled(q, scale)
+    return get_ext().flash_attn_fwd(_rows(q), _rows(k), _rows(v), scale,
+                                    causal, False)[0]
 
 
 def sdpa_reference(q, k, v, causal=True, scale=None):
@@ -88,45 +99,34 @@ def sdpa_reference(q, k, v, causal=True, scale=None):
 
 def flash_attn_bwd(q, k, v, o, do, lse, causal=True, scale=None):
     """Backward pass in BHSD ([B,H(kv),S,D] bf16; lse [B,H,S] fp32).
-    Returns (dq, dk, dv). GPU-validation pending (round-2 item) — the
-    tile algebra is CPU-verified in ops/flash_bwd_ref.py."""
-    ext = get_ext()
-    scale = scale if scale is not None else 1.0 / math.sqrt(q.size(-1))
-    delta = (do.float() * o.float()).sum(-1)              # [B,H,S]
-    qt = _t_last2_bhsd(q)
-    kt = _t_last2_bhsd(k)
-    dot = _t_last2_bhsd(do)
-    return ext.flash_attn_bwd(q.contiguous(), k.contiguous(), v.contiguous(),
-                              do.contiguous(), qt, kt, dot,
-                              lse.contiguous().float(), delta.contiguous(),
-                              scale, causal)
+    Returns (dq, dk, dv)."""
+    q, scale, factor = _scaled(q, scale)
+    dq, dk, dv = get_ext().flash_attn_bwd(
+        *(_rows(t.transpose(1, 2)) for t in (q, k, v, o, do)),
+        lse.contiguous().float(), scale, causal)
+    dq = dq if factor == 1 else dq * factor
+    return tuple(g.transpose(1, 2).contiguous() for g in (dq, dk, dv))
 
 
 class FlashAttnFunc(torch.autograd.Function):
-    """Training-path flash attention (BSHD in/out). GPU-validation of the
-    backward kernels is a round-2 gate; until then the model keeps SDPA."""
+    """Training-path flash attention (BSHD in/out)."""
 
     @staticmethod
     def forward(ctx, q, k, v, causal, scale):
-        ext = get_ext()
-        scale = scale if scale is not None else 1.0 / math.sqrt(q.size(-1))
-        vt = _vt_from_bshd(v)
-        o, lse = ext.flash_attn_fwd_lse(q.contiguous(), k.contiguous(), vt,
-                                        scale, causal)
+        q, scale, ctx.factor = _scaled(q, scale)
+        q, k, v = _rows(q), _rows(k), _rows(v)
+        o, lse = get_ext().flash_attn_fwd(q, k, v, scale, causal, True)
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.causal, ctx.scale = causal, scale
         return o
 
     @staticmethod
+    @torch.autograd.function.once_differentiable
     def backward(ctx, do):
         q, k, v, o, lse = ctx.saved_tensors
-        # kernels run in BHSD
-        qh, kh, vh, oh, doh = (t.transpose(1, 2).contiguous()
-                               for t in (q, k, v, o, do))
-        dq, dk, dv = flash_attn_bwd(qh, kh, vh, oh, doh, lse,
-                                    causal=ctx.causal, scale=ctx.scale)
-        return (dq.transpose(1, 2), dk.transpose(1, 2),
-                dv.transpose(1, 2), None, None)
+        dq, dk, dv = get_ext().flash_attn_bwd(q, k, v, o, _rows(do), lse,
+                                              ctx.scale, ctx.causal)
+        return (dq if ctx.factor == 1 else dq * ctx.factor), dk, dv, None, None
 
 
 def flash_attn_func(q, k, v, causal=True, scale=None):

@@ -1,340 +1,717 @@
-// Flash-attention forward for MI355X (gfx950 / CDNA4) — hand-written MFMA.
+// Flash attention, forward and backward, for MI355X (gfx950) on the matrix
+// cores: any sequence length, heads of 64, 96 and 128, grouped key heads,
+// causal or full. q, o, do [B, S, H, D], k, v [B, S, Hkv, D] bf16 (any strides
+// between tokens and heads, unit stride inside a head), lse fp32 [B, H, S].
 //
-// Replaces the aotriton SDPA forward on the training/prefill hot path
-// (reference analogue: csrc/transformer/inference softmax+GEMM chain and
-// inference/v2 blocked flash). v3 follows the CDNA4 guide's verified
-// 8-wave/QB32/KVBLK64 attention ladder (cdna_hip_programming.md §B).
+// Reference analogue: the softmax and GEMM chain of csrc/transformer and the
+// blocked flash attention of inference/v2.
 //
-// v3 structure (fixes v2's 144 B/lane scratch spill and 2-barrier stalls):
-// * 512-thread workgroup = 8 waves x 32 query rows (Q tile = 256 rows);
-//   grid (ceil(S/256), H, B). KVBLK = 64 rows per step.
-// * K and V^T tiles double-buffered in LDS (64 KB total): ONE
-//   __syncthreads per 64-row kv step instead of two per 32-row step.
-// * async-STAGE split: next tile's global loads are issued into registers
-//   BEFORE the current tile's compute (HBM latency hides under MFMA),
-//   ds_writes land after the compute, before the barrier.
-// * XOR swizzle on both LDS tiles (`chunk ^= row&7`) — bank-conflict-free
-//   row-strided ds_read_b128 fragment reads.
-// * mfma_f32_32x32x16_bf16 with probe-verified layouts
-//   (scripts/mfma_probe.hip, run on gfx950 2026-08-20):
-//     A: row = lane&31, k = reg + 8*(lane>>5)
-//     B: col = lane&31, k = reg + 8*(lane>>5)
-//     C/D: col = lane&31, row = (reg&3) + 8*(reg>>2) + 4*(lane>>5)
-// * swapped S^T = mfma(A=K, B=Q): each lane owns 32 score entries of ONE
-//   query column -> row max/sum is ~31 VALU ops + one shfl_xor(32).
-// * P re-layout for PV (C/D -> B fragment) with COMPILE-TIME register
-//   indices (v2 used half-dependent runtime indices -> scratch): for
-//   pf[ks][reg], the owner half is ho=(reg>>2)&1 and both candidate
-//   source registers rp = (reg&3)+8*(ks&1)+4*{ho,1-ho} are constants;
-//   the cross-half value moves with one shfl_xor(32).
-// * defer-max (RESCALE_THRESHOLD=8): skip the O(64-VALU) rescale pass
-//   when the tile max doesn't raise the running max by >8 (exp stays
-//   bounded by e^8, fp32 accumulators don't care).
-// * s_setprio(1) around the MFMA clusters.
+// mfma_f32_32x32x16_bf16 lane maps (col = lane & 31, half = lane >> 5):
+//   A: row = col, k = 8 half + j    B: col, k = 8 half + j   (j = 0..7)
+//   C/D: col, row = (r & 3) + 8 (r >> 2) + 4 half            (r = 0..15)
 //
-// Layouts: q,k [B,S,H(kv),128] bf16; vt [B,Hkv,128,S] bf16; o [B,S,H,128].
-// Requires D=128, S % 32 == 0 (wrapper falls back to SDPA otherwise).
+// One idea runs through all kernels: the order of the contracted index is
+// free. A product's result holds, for its column, the rows 16 s + 8 (j >> 2) +
+// 4 half + (j & 3) in the registers 8 s + j; taken as the contracted index of
+// the next product in just that order, those registers ARE its B operand. The
+// other operand has to bring the same rows, transposed: ds_read_b64_tr_b16
+// reads four consecutive rows of one column, which is a run of j & 3. So
+// neither probabilities nor their gradients move between lanes or through
+// LDS, and no operand is transposed in memory beforehand (the transposed
+// copies of V, K, Q and dO that the earlier kernels took cost a pass each).
+//
+// LDS tiles are rows of 16-byte chunks, chunk c of row r stored at c ^ f(r),
+// which spreads both the row-wise (b128) and the transposing reads over the
+// banks. Heads of 96 use the layout of 128.
 
 #include "ds_kernels.h"
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) short bf16x8s;
-typedef __attribute__((ext_vector_type(8))) short lds_chunk;  // 16 B
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __attribute__((ext_vector_type(2))) int i32x2;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int QB = 32;    // query rows per wave
-constexpr int NWAVE = 8;  // waves per workgroup
-constexpr int QTILE = QB * NWAVE;
-constexpr int TPB = NWAVE * 64;  // 8 waves x 64 lanes
-constexpr int D = 128;           // head dim
-constexpr int KB = 64;           // kv rows per step
+constexpr float LOG2E = 1.4426950408889634f;
 
-__device__ __forceinline__ short f2bf(float f) {
-  union {
-    float f;
-    unsigned u;
-  } c;
-  c.f = f;
-  unsigned r = c.u + 0x7FFF + ((c.u >> 16) & 1);
-  return (short)(r >> 16);
-}
-
-// Swizzled chunk index inside a tile: row-major rows of NC 16-byte chunks,
-// chunk XOR'd with row&7 so row-strided fragment reads spread the banks.
-__device__ __forceinline__ int k_sw(int row, int chunk) {
-  return row * 16 + (chunk ^ (row & 7));
-}
-__device__ __forceinline__ int v_sw(int row, int chunk) {
-  return row * 8 + (chunk ^ (row & 7));
-}
-
-struct StageRegs {
-  bf16x8s k0, k1, v0, v1;
+struct View {             // element strides of [B, S, H, D]
+  long long b, s, h;
 };
 
-// Issue the global loads for one kv tile (2 K chunks + 2 V^T chunks per
-// thread). Called EARLY so the HBM latency hides under the MFMA phase.
-__device__ __forceinline__ StageRegs stage_load(
-    const short* __restrict__ k, const short* __restrict__ vtp,
-    long long k_base, int HkvD, int kv0, int S, int tid) {
-  StageRegs r;
-  const int krow = tid >> 4, kc = tid & 15;
-  const long long kr0 = min(kv0 + krow, S - 1);
-  const long long kr1 = min(kv0 + krow + 32, S - 1);
-  r.k0 = *(const bf16x8s*)(k + k_base + kr0 * HkvD + kc * 8);
-  r.k1 = *(const bf16x8s*)(k + k_base + kr1 * HkvD + kc * 8);
-  const int vrow = tid >> 3, vc = tid & 7;
-  const int kvc = min(kv0 + vc * 8, S - 8);
-  r.v0 = *(const bf16x8s*)(vtp + (long long)vrow * S + kvc);
-  r.v1 = *(const bf16x8s*)(vtp + (long long)(vrow + 64) * S + kvc);
-  return r;
+__device__ __forceinline__ f32x16 mfma(s16x8 a, s16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+      __builtin_bit_cast(b16x8, a), __builtin_bit_cast(b16x8, b), c, 0, 0, 0);
 }
 
-__device__ __forceinline__ void stage_write(const StageRegs& r,
-                                            lds_chunk* kbuf, lds_chunk* vbuf,
-                                            int tid) {
-  const int krow = tid >> 4, kc = tid & 15;
-  kbuf[k_sw(krow, kc)] = r.k0;
-  kbuf[k_sw(krow + 32, kc)] = r.k1;
-  const int vrow = tid >> 3, vc = tid & 7;
-  vbuf[v_sw(vrow, vc)] = r.v0;
-  vbuf[v_sw(vrow + 64, vc)] = r.v1;
+__device__ __forceinline__ s16x4 tr_read(const short* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s16x4*)p);
 }
 
-template <bool CAUSAL, bool DEFER = true>
-__global__ __launch_bounds__(TPB) void flash_fwd_kernel(
-    const short* __restrict__ q,   // [B, S, H, D]
-    const short* __restrict__ k,   // [B, S, Hkv, D]
-    const short* __restrict__ vt,  // [B, Hkv, D, S]
-    short* __restrict__ o,         // [B, S, H, D]
-    float* __restrict__ lse,       // optional [B, H, S] log-sum-exp
-    const int B, const int S, const int H, const int Hkv,
-    const float scale) {
-  __shared__ lds_chunk kbuf[2][KB * 16];  // K: [64 rows][16 chunks]
-  __shared__ lds_chunk vbuf[2][D * 8];    // V^T: [128 rows][8 chunks]
+__device__ __forceinline__ int pack2(float a, float b) {
+  return __builtin_bit_cast(
+      int, __builtin_convertvector((f32x2{a, b}), b16x2));
+}
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int q0b = blockIdx.x * QTILE;  // block's first q row
-  const int h = blockIdx.y;
-  const int b = blockIdx.z;
-  const int hkv = h / (H / Hkv);
+// Registers 8 s .. 8 s + 7 of a result as the next product's B operand.
+__device__ __forceinline__ s16x8 operand(const f32x16& p, int s) {
+  typedef int i32x4 __attribute__((ext_vector_type(4)));
+  const i32x4 v = {pack2(p[8 * s], p[8 * s + 1]),
+                   pack2(p[8 * s + 2], p[8 * s + 3]),
+                   pack2(p[8 * s + 4], p[8 * s + 5]),
+                   pack2(p[8 * s + 6], p[8 * s + 7])};
+  return __builtin_bit_cast(s16x8, v);
+}
 
-  const int col = lane & 31;  // my query row within the wave / kv row in A
-  const int half = lane >> 5;
-  const int q0w = q0b + wid * QB;
-  const int qrow = q0w + col;
-  const bool q_ok = qrow < S;
-  const int qload = q_ok ? qrow : S - 1;
-
-  // ---- preload Q as B-fragments: qf[kk] holds d = kk*16 + 8*half + [0,8)
-  bf16x8s qf[8];
-  {
-    const short* qp = q + (((long long)b * S + qload) * H + h) * D;
+// Tile of rows of D bf16 in LDS. Within a row the swizzle is an exclusive or,
+// so the addresses of one lane's reads differ by one from a first one.
+template <int D>
+struct Tile {
+  static constexpr int CH = D / 8;                  // chunks of a row
+  static constexpr int SC = D == 64 ? 8 : 16;       // places of a row
+  static constexpr int RB = SC * 16;                // bytes of a row
+  static __device__ __forceinline__ int turn(int row) {
+    return D == 64 ? (row >> 1) & 7 : row & 15;
+  }
+  // A operand: rows row0 + col, contracted k = 16 kk + 8 half + j
+  static __device__ __forceinline__ int rows_at(int lane) {
+    const int col = lane & 31;
+    return col * RB + (((lane >> 5) ^ turn(col)) << 4);
+  }
+  static __device__ __forceinline__ s16x8 rows(const short* t, int row0,
+                                               int kk, int at) {
+    return *(const s16x8*)((const char*)t + row0 * RB + (at ^ (kk * 32)));
+  }
+  // A operand of the transpose: rows are the coordinates 32 db + col,
+  // contracted the tile's rows row0 + 8 (j >> 2) + 4 half + (j & 3), row0 a
+  // multiple of 16
+  static __device__ __forceinline__ int cols_at(int lane) {
+    const int sub = lane & 15, r = 4 * (lane >> 5) + (sub >> 2);
+    const int c = 2 * ((lane >> 4) & 1) + ((sub & 3) >> 1);
+    return r * RB + ((c ^ turn(r)) << 4) + (sub & 1) * 8;
+  }
+  static __device__ __forceinline__ s16x8 cols(const short* t, int row0,
+                                               int db, int at) {
+    const char* p = (const char*)t + row0 * RB;
+    const int lo = at ^ (db * 64), hi = lo ^ (RB / 2);   // row + 8
+    const s16x4 a = tr_read((const short*)(p + lo));
+    const s16x4 b = tr_read((const short*)(p + 8 * RB + hi));
+    return s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  }
+  // N rows of src (of which `left` are there: the last is repeated) straight
+  // into LDS: the destination of a direct load is linear, so the swizzle goes
+  // into the source. TPB threads; places past a row's chunks (D = 96) repeat.
+  template <int N, int TPB>
+  static __device__ __forceinline__ void fetch(const short* src, int stride,
+                                               int left, short* t, int tid) {
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk)
-      qf[kk] = *(const bf16x8s*)(qp + kk * 16 + 8 * half);
+    for (int i = 0; i < N * SC / TPB; ++i) {
+      const int j = tid + i * TPB;
+      const int row = j / SC;
+      int c = (j % SC) ^ turn(row);
+      if (CH < SC) c = min(c, CH - 1);
+      const int off = min(row, left - 1) * stride + c * 8;
+      __builtin_amdgcn_global_load_lds((const unsigned int*)(src + off),
+                                       (unsigned int*)(t + j * 8), 16, 0, 0);
+    }
   }
+};
 
-  float m_run = -1e30f;
-  float l_run = 0.f;
-  f32x16 oacc[4] = {};  // O^T accumulators, one per 32-wide d block
+// Workgroup -> (block of rows, batch * head): workgroups go round the eight
+// XCDs, so each XCD takes an eighth of the heads (its L2 then holds their K
+// and V, or Q and dO), and the blocks that see the most come first.
+__device__ __forceinline__ void place(int id, int blocks, int heads, int& blk,
+                                      int& bh) {
+  if (heads % 8 == 0) {
+    const int per = heads / 8, k = id >> 3;
+    blk = k / per;
+    bh = (id & 7) * per + k % per;
+  } else {
+    blk = id / heads;
+    bh = id % heads;
+  }
+}
 
-  const int kv_end_blk = CAUSAL ? min(S, q0b + QTILE) : S;
-  const int kv_end_wave = CAUSAL ? min(S, q0w + QB) : S;
-  const int HkvD = Hkv * D;
-  const long long k_base = (((long long)b * S) * Hkv + hkv) * D;
-  const short* vtp = vt + (((long long)b * Hkv + hkv) * D) * S;
-  const int nt = (kv_end_blk + KB - 1) / KB;
+// ------------------------------------------------------------------ forward
+//
+// 8 waves of 32 query rows; 64 keys a step, K and V double-buffered, the next
+// tile's direct loads in flight behind this one's products. Per key and row
+// the vector unit does one multiply-add, one exp2, half a maximum, one add and
+// half a conversion; the maximum is raised only where it grows by more than
+// 2^8, so that most steps rescale nothing. Bound by the vector unit beside the
+// matrix cores. 32 on 8 heads of 128, causal: 1 x 4096 173 us (793 TFLOP/s), 8
+// x 4096 1340 us (820); with V transposed beforehand, fp32 scaling and
+// conversions bit by bit it took 350 us, torch's attention 389 and 2716.
 
-  // ---- prologue: stage tile 0 into buffer 0
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(512) void fwd_kernel(
+    const short* __restrict__ q, const short* __restrict__ k,
+    const short* __restrict__ v, short* __restrict__ o,
+    float* __restrict__ lse, const View vq, const View vk, const View vv,
+    const View vo, const int S, const int H, const int Hkv, const float c,
+    const int blocks, const int heads) {
+  constexpr int KB = 64, DB = D / 32, KK = D / 16;
+  using T = Tile<D>;
+  __shared__ __attribute__((aligned(16))) short kt[2][KB * T::SC * 8];
+  __shared__ __attribute__((aligned(16))) short vt[2][KB * T::SC * 8];
+
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int col = lane & 31, half = lane >> 5;
+  const int ra = T::rows_at(lane), ca = T::cols_at(lane);
+  int blk, bh;
+  place(blockIdx.x, blocks, heads, blk, bh);
+  blk = blocks - 1 - blk;
+  const int b = bh / H, h = bh % H, hkv = h / (H / Hkv);
+  const int q0b = blk * 256, q0 = q0b + wid * 32, row = q0 + col;
+
+  const short* kp = k + b * vk.b + hkv * vk.h;
+  const short* vp = v + b * vv.b + hkv * vv.h;
+
+  s16x8 qf[KK];
   {
-    StageRegs sr = stage_load(k, vtp, k_base, HkvD, 0, S, tid);
-    stage_write(sr, kbuf[0], vbuf[0], tid);
+    const short* qp = q + b * vq.b + h * vq.h + min(row, S - 1) * vq.s;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk)
+      qf[kk] = *(const s16x8*)(qp + 16 * kk + 8 * half);
   }
+
+  float m = -1e30f, l = 0.f;
+  f32x16 acc[DB] = {};
+  const int end_b = CAUSAL ? min(S, q0b + 256) : S;
+  const int end_w = CAUSAL ? min(S, q0 + 32) : S;
+  const int steps = (end_b + KB - 1) / KB;
+
+  T::template fetch<KB, 512>(kp, (int)vk.s, S, kt[0], tid);
+  T::template fetch<KB, 512>(vp, (int)vv.s, S, vt[0], tid);
   __syncthreads();
 
-  for (int it = 0; it < nt; ++it) {
-    const int kv0 = it * KB;
-    const int cur = it & 1;
-
-    // ---- async stage: issue next tile's loads before compute
-    StageRegs sr;
-    const bool have_next = (it + 1 < nt);
-    if (have_next)
-      sr = stage_load(k, vtp, k_base, HkvD, kv0 + KB, S, tid);
-
-    if (kv0 < kv_end_wave) {
-      const lds_chunk* kt_lds = kbuf[cur];
-      const lds_chunk* vt_lds = vbuf[cur];
-
-      // ---- S^T = K · Q^T for both 32-row kv subtiles
-      f32x16 p2[2];
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub) {
-        f32x16 st = {};
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-          bf16x8s kf = kt_lds[k_sw(sub * 32 + col, kk * 2 + half)];
-          st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], st,
-                                                       0, 0, 0);
-        }
-        __builtin_amdgcn_s_setprio(0);
-        p2[sub] = st;
-      }
-
-      // ---- masked scale + tile max (lane owns 32 kv entries of one q).
-      // Interior tiles (fully below the causal diagonal for every q row
-      // of this wave, fully inside S) skip the 64 mask compares.
-      float mt = -1e30f;
-      const bool interior = kv0 + KB <= (CAUSAL ? q0w + 1 : S) &&
-                            kv0 + KB <= S;
-      if (interior) {
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float s = p2[sub][r] * scale;
-            p2[sub][r] = s;
-            mt = fmaxf(mt, s);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int kvl = kv0 + sub * 32 + (r & 3) + 8 * (r >> 2) + 4 * half;
-            float s = p2[sub][r] * scale;
-            if ((CAUSAL && kvl > qrow) || kvl >= S) s = -1e30f;
-            p2[sub][r] = s;
-            mt = fmaxf(mt, s);
-          }
-        }
-      }
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-
-      // ---- online softmax with defer-max
-      bool rescale = true;
-      float m_new;
-      if (DEFER) {
-        rescale = !__all(mt <= m_run + 8.f);
-        m_new = rescale ? fmaxf(m_run, mt) : m_run;
-      } else {
-        m_new = fmaxf(m_run, mt);
-      }
-      float lt = 0.f;
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          p2[sub][r] = __expf(p2[sub][r] - m_new);
-          lt += p2[sub][r];
-        }
-      }
-      lt += __shfl_xor(lt, 32, 64);
-      const float alpha = __expf(m_run - m_new);
-      l_run = (rescale ? l_run * alpha : l_run) + lt;
-      m_run = m_new;
-
-      // ---- build P B-fragments with compile-time register indices.
-      // pf[ks] covers kv = ks*16 + reg + 8*half; the owner half of that
-      // score is ho=(reg>>2)&1 (independent of the requester's half), at
-      // register rp = (reg&3)+8*(ks&1)+4*h of p2[ks>>1]. One
-      // permlane32_swap(a=low-half need, b=high-half need) delivers BOTH
-      // fragment slots (reg=rr at r0, reg=rr+4 at r1) — 16 VALU-pipe
-      // permlanes per tile instead of 32 LDS-pipe ds_bpermutes.
-      bf16x8s pf[4];
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int s_ = ks >> 1;                   // compile-time
-          const int rpA = rr + 8 * (ks & 1);        // h=0 requester's need
-          const int rpB = rpA + 4;                  // h=1 requester's need
-          // inline asm: the __builtin_amdgcn_permlane32_swap intrinsic is
-          // wrongly CSE'd across calls with different args by this LLVM
-          // (16 calls collapse to 2 — see /tmp repro pl3/pl6, 2026-08-20)
-          float a = p2[s_][rpA], b = p2[s_][rpB];
-          asm("v_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-          pf[ks][rr] = f2bf(a);
-          pf[ks][rr + 4] = f2bf(b);
-        }
-      }
-
-      // ---- O^T += V^T · P : A = V^T rows (d), k = kv; B = P cols (q)
-#pragma unroll
-      for (int dblk = 0; dblk < 4; ++dblk) {
-        if (rescale) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) oacc[dblk][r] *= alpha;
-        }
-        __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          bf16x8s vf = vt_lds[v_sw(dblk * 32 + col, ks * 2 + half)];
-          oacc[dblk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              vf, pf[ks], oacc[dblk], 0, 0, 0);
-        }
-        __builtin_amdgcn_s_setprio(0);
-      }
+  for (int it = 0; it < steps; ++it) {
+    const int k0 = it * KB, cur = it & 1;
+    if (it + 1 < steps) {
+      T::template fetch<KB, 512>(kp + (k0 + KB) * vk.s, (int)vk.s, S - k0 - KB,
+                                kt[cur ^ 1], tid);
+      T::template fetch<KB, 512>(vp + (k0 + KB) * vv.s, (int)vv.s, S - k0 - KB,
+                                vt[cur ^ 1], tid);
     }
+    if (k0 < end_w) {
+      f32x16 p[2] = {};
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk)
+          p[t] = mfma(T::rows(kt[cur], 32 * t, kk, ra), qf[kk], p[t]);
+      __builtin_amdgcn_s_setprio(0);
 
-    // ---- write next tile into the other buffer; barrier flips it live
-    if (have_next)
-      stage_write(sr, kbuf[cur ^ 1], vbuf[cur ^ 1], tid);
+      if (k0 + KB > (CAUSAL ? min(S, q0 + 1) : S)) {
+        const int last = (CAUSAL ? min(row, S - 1) : S - 1) - k0 - 4 * half;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (32 * t + (r & 3) + 8 * (r >> 2) > last) p[t][r] = -1e30f;
+      }
+      float mt = -1e30f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mt = fmaxf(mt, p[t][r]);
+      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      if (!__all((mt - m) * c <= 8.f)) {
+        const float mn = fmaxf(m, mt);
+        const float alpha = __builtin_amdgcn_exp2f((m - mn) * c);
+        m = mn;
+        l *= alpha;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+      }
+      const float mc = m * c;
+      float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+          p[t][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[t][r], c, -mc));
+          p[t][r + 1] =
+              __builtin_amdgcn_exp2f(__builtin_fmaf(p[t][r + 1], c, -mc));
+          l0 += p[t][r];
+          l1 += p[t][r + 1];
+        }
+      l += l0 + l1;
+
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const s16x8 pb = operand(p[t], s);
+#pragma unroll
+          for (int db = 0; db < DB; ++db)
+            acc[db] = mfma(T::cols(vt[cur], 32 * t + 16 * s, db, ca), pb, acc[db]);
+        }
+      __builtin_amdgcn_s_setprio(0);
+    }
     __syncthreads();
   }
 
-  // ---- epilogue: O[q][d] = O^T / l
-  if (!q_ok) return;
-  const float inv_l = l_run > 0.f ? 1.f / l_run : 0.f;
-  if (lse != nullptr && half == 0)  // one lane half owns the q row
-    lse[((long long)b * H + h) * S + qrow] = m_run + __logf(l_run);
-  short* op = o + (((long long)b * S + qrow) * H + h) * D;
+  l += __shfl_xor(l, 32, 64);
+  if (row >= S) return;
+  const float inv = l > 0.f ? 1.f / l : (l != l ? l : 0.f);
+  if (lse != nullptr && half == 0)
+    lse[((long long)b * H + h) * S + row] =
+        m * c * (1.f / LOG2E) + __logf(l);
+  short* op = o + b * vo.b + h * vo.h + row * vo.s + 4 * half;
 #pragma unroll
-  for (int dblk = 0; dblk < 4; ++dblk) {
+  for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int d = dblk * 32 + (r & 3) + 8 * (r >> 2) + 4 * half;
-      op[d] = f2bf(oacc[dblk][r] * inv_l);
+    for (int g = 0; g < 4; ++g) {
+      typedef int i32x2 __attribute__((ext_vector_type(2)));
+      *(i32x2*)(op + 32 * db + 8 * g) =
+          i32x2{pack2(acc[db][4 * g] * inv, acc[db][4 * g + 1] * inv),
+                pack2(acc[db][4 * g + 2] * inv, acc[db][4 * g + 3] * inv)};
     }
+}
+
+// ----------------------------------------------------------------- backward
+//
+// stat[0][b, h, s] = lse * log2(e), stat[1][b, h, s] = sum(do * o): one wave
+// four rows of a head; both passes below start from these two numbers a row.
+
+template <int D>
+__global__ __launch_bounds__(256) void stat_kernel(
+    const short* __restrict__ dout, const short* __restrict__ o,
+    const float* __restrict__ lse, float* __restrict__ stat, const View vd,
+    const View vo, const int S, const int H, const long long rows) {
+  const int sub = threadIdx.x & 15;
+  const long long u = (long long)blockIdx.x * 16 + (threadIdx.x >> 4);
+  if (u >= rows) return;               // u = (b S + s) H + h
+  const int h = (int)(u % H);
+  const long long bs = u / H;
+  const int s = (int)(bs % S);
+  const long long b = bs / S;
+  float sum = 0.f;
+  if (8 * sub < D) {
+    const s16x8 x = *(const s16x8*)(dout + b * vd.b + s * vd.s + h * vd.h +
+                                    8 * sub);
+    const s16x8 y = *(const s16x8*)(o + b * vo.b + s * vo.s + h * vo.h +
+                                    8 * sub);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      sum += __builtin_bit_cast(float, (unsigned)(unsigned short)x[e] << 16) *
+             __builtin_bit_cast(float, (unsigned)(unsigned short)y[e] << 16);
+  }
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  if (sub == 0) {
+    const long long at = (b * H + h) * S + s;
+    stat[at] = lse[at] * LOG2E;
+    stat[rows + at] = sum;
+  }
+}
+
+// Both passes recompute S and dP: seven products where one pass with atomic
+// sums of dQ would have five, but every sum is made in registers, in one order.
+// Backward in all, 32 on 8 heads of 128, causal: 2 x 4096 1100 us (620
+// TFLOP/s of the five), 8 x 4096 4205 us (654); torch's attention 3324 and
+// 12151, the earlier kernels over transposed copies 15800 at 8 x 4096.
+//
+// dK and dV: a wave owns 32 key rows of one key head (K and V as B operands in
+// registers) and walks the queries of the group's heads, 64 rows of Q and dO a
+// step, double-buffered in LDS by direct loads. S = Q K^T and dP = dO V^T come
+// out with a key a column; P and dS are then B operands of dV^T += dO^T P and
+// dK^T += Q^T dS, and the same LDS tiles give dO^T and Q^T by transposing
+// reads. 4 waves a workgroup, two workgroups a CU. Where that leaves CUs idle,
+// the group's heads are split over more workgroups, whose fp32 sums add_kernel
+// adds up.
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(256, 2) void dkdv_kernel(
+    const short* __restrict__ q, const short* __restrict__ k,
+    const short* __restrict__ v, const short* __restrict__ dout,
+    const float* __restrict__ stat, short* __restrict__ dk,
+    short* __restrict__ dv, const View vq, const View vk, const View vv,
+    const View vd, const View vdk, const View vdv, const int S, const int H,
+    const int Hkv, const float scale, const int blocks, const int heads,
+    const long long rows, float* __restrict__ part) {
+  constexpr int QB = 64, DB = D / 32, KK = D / 16;
+  using T = Tile<D>;
+  __shared__ __attribute__((aligned(16))) short qt[2][QB * T::SC * 8];
+  __shared__ __attribute__((aligned(16))) short dt[2][QB * T::SC * 8];
+  __shared__ __attribute__((aligned(16))) float st[2][2][QB];
+
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int col = lane & 31, half = lane >> 5;
+  const int ra0 = T::rows_at(lane), ca0 = T::cols_at(lane);
+  int blk, bh;
+  place(blockIdx.x, blocks, heads, blk, bh);
+  const int b = bh / Hkv, hkv = bh % Hkv, G = H / Hkv;
+  const int k0b = blk * 128, k0 = k0b + wid * 32, key = k0 + col;
+  const float c = scale * LOG2E;
+
+  s16x8 kf[KK], vf[KK];
+  {
+    const short* kp = k + b * vk.b + hkv * vk.h + min(key, S - 1) * vk.s;
+    const short* vp = v + b * vv.b + hkv * vv.h + min(key, S - 1) * vv.s;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      kf[kk] = *(const s16x8*)(kp + 16 * kk + 8 * half);
+      vf[kk] = *(const s16x8*)(vp + 16 * kk + 8 * half);
+    }
+  }
+  f32x16 dka[DB] = {}, dva[DB] = {};
+
+  const int first = CAUSAL ? k0b : 0;       // a multiple of 64
+  const int per = (S - first + QB - 1) / QB;
+  // the group's heads of this split
+  const int g0 = blockIdx.y * G / gridDim.y;
+  const int steps = ((blockIdx.y + 1) * G / gridDim.y - g0) * per;
+
+  auto fetch = [&](int h, int s0, int buf, int tid) {
+    T::template fetch<QB, 256>(q + b * vq.b + h * vq.h + s0 * vq.s,
+                               (int)vq.s, S - s0, qt[buf], tid);
+    T::template fetch<QB, 256>(dout + b * vd.b + h * vd.h + s0 * vd.s,
+                               (int)vd.s, S - s0, dt[buf], tid);
+    if (wid < 2) {
+      const float* p = stat + wid * rows + ((long long)b * H + h) * S + s0;
+      __builtin_amdgcn_global_load_lds(
+          (const unsigned int*)(p + min(lane, S - s0 - 1)),
+          (unsigned int*)(&st[buf][wid][lane]), 4, 0, 0);
+    }
+  };
+
+  int h = hkv * G + g0, s0 = first;
+  fetch(h, s0, 0, tid);
+  __syncthreads();
+  for (int it = 0; it < steps; ++it) {
+    const int cur = it & 1;
+    int s1 = s0 + QB;
+    if (s1 >= S) {
+      s1 = first;
+      ++h;
+    }
+    if (it + 1 < steps) {
+      int tid_ = tid;
+      asm("" : "+v"(tid_));
+      fetch(h, s1, cur ^ 1, tid_);
+    }
+#pragma unroll 1
+    for (int t = 0; t < 2; ++t) {
+      const int r0 = s0 + 32 * t;
+      if ((CAUSAL && r0 + 31 < k0) || r0 >= S) continue;
+      // recomputed here: kept out of the loop they would take registers that
+      // the loop needs
+      int ra = ra0, ca = ca0;
+      asm("" : "+v"(ra), "+v"(ca));
+      f32x16 p = {}, dp = {};
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk)
+        p = mfma(T::rows(qt[cur], 32 * t, kk, ra), kf[kk], p);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk)
+        dp = mfma(T::rows(dt[cur], 32 * t, kk, ra), vf[kk], dp);
+      __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 ls = *(const f32x4*)&st[cur][0][32 * t + 8 * g + 4 * half];
+        const f32x4 dl = *(const f32x4*)&st[cur][1][32 * t + 8 * g + 4 * half];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = 4 * g + e;
+          p[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[r], c, -ls[e]));
+          dp[r] -= dl[e];
+        }
+      }
+      if ((CAUSAL && r0 < k0 + 31) || r0 + 32 > S) {
+        const int from = (CAUSAL ? key : 0) - r0 - 4 * half;
+        const int to = S - r0 - 4 * half;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int at = (r & 3) + 8 * (r >> 2);
+          if (at < from || at >= to) p[r] = 0.f;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dp[r] *= p[r];
+      if ((CAUSAL && r0 < k0 + 31) || r0 + 32 > S) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (p[r] == 0.f) dp[r] = 0.f;      // also where dP overflowed
+      }
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const s16x8 pb = operand(p, s), sb = operand(dp, s);
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+          dva[db] = mfma(T::cols(dt[cur], 32 * t + 16 * s, db, ca), pb, dva[db]);
+          dka[db] = mfma(T::cols(qt[cur], 32 * t + 16 * s, db, ca), sb, dka[db]);
+        }
+      }
+      __builtin_amdgcn_s_setprio(0);
+    }
+    __syncthreads();
+    s0 = s1;
+  }
+
+  if (key >= S) return;
+  if (part != nullptr) {     // added up by add_kernel
+    const long long n = rows / H * Hkv * D;
+    float* pp = part + 2 * n * blockIdx.y +
+                (((long long)b * S + key) * Hkv + hkv) * D + 4 * half;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        *(f32x4*)(pp + 32 * db + 8 * g) =
+            f32x4{dka[db][4 * g], dka[db][4 * g + 1], dka[db][4 * g + 2],
+                  dka[db][4 * g + 3]};
+        *(f32x4*)(pp + n + 32 * db + 8 * g) =
+            f32x4{dva[db][4 * g], dva[db][4 * g + 1], dva[db][4 * g + 2],
+                  dva[db][4 * g + 3]};
+      }
+    return;
+  }
+  typedef int i32x2 __attribute__((ext_vector_type(2)));
+  short* kp = dk + b * vdk.b + hkv * vdk.h + key * vdk.s + 4 * half;
+  short* vp = dv + b * vdv.b + hkv * vdv.h + key * vdv.s + 4 * half;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      *(i32x2*)(kp + 32 * db + 8 * g) = i32x2{
+          pack2(dka[db][4 * g] * scale, dka[db][4 * g + 1] * scale),
+          pack2(dka[db][4 * g + 2] * scale, dka[db][4 * g + 3] * scale)};
+      *(i32x2*)(vp + 32 * db + 8 * g) =
+          i32x2{pack2(dva[db][4 * g], dva[db][4 * g + 1]),
+                pack2(dva[db][4 * g + 2], dva[db][4 * g + 3])};
+    }
+}
+
+// dK and dV from the partial sums of the splits: part [splits][dk, dv][n].
+__global__ __launch_bounds__(256) void add_kernel(
+    const float* __restrict__ part, short* __restrict__ dk,
+    short* __restrict__ dv, const long long n, const int splits,
+    const float scale) {
+  const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= 2 * n) return;
+  f32x4 t = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < splits; ++s) t += *(const f32x4*)(part + 2 * n * s + i);
+  const bool is_k = i < n;
+  if (is_k) t *= scale;
+  typedef int i32x2 __attribute__((ext_vector_type(2)));
+  *(i32x2*)((is_k ? dk : dv - n) + i) =
+      i32x2{pack2(t[0], t[1]), pack2(t[2], t[3])};
+}
+
+// dQ: a wave owns 32 query rows (Q and dO as B operands) and walks the keys, 64
+// rows of K and V a step. S^T = K Q^T, dP^T = V dO^T, dQ^T += K^T dS^T.
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(256, 2) void dq_kernel(
+    const short* __restrict__ q, const short* __restrict__ k,
+    const short* __restrict__ v, const short* __restrict__ dout,
+    const float* __restrict__ stat, short* __restrict__ dq, const View vq,
+    const View vk, const View vv, const View vd, const View vdq, const int S,
+    const int H, const int Hkv, const float scale, const int blocks,
+    const int heads, const long long rows) {
+  constexpr int KB = 64, DB = D / 32, KK = D / 16;
+  using T = Tile<D>;
+  __shared__ __attribute__((aligned(16))) short kt[2][KB * T::SC * 8];
+  __shared__ __attribute__((aligned(16))) short vt[2][KB * T::SC * 8];
+
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int col = lane & 31, half = lane >> 5;
+  const int ra = T::rows_at(lane), ca = T::cols_at(lane);
+  int blk, bh;
+  place(blockIdx.x, blocks, heads, blk, bh);
+  blk = blocks - 1 - blk;
+  const int b = bh / H, h = bh % H, hkv = h / (H / Hkv);
+  const int q0b = blk * 128, q0 = q0b + wid * 32, row = q0 + col;
+  const int at = min(row, S - 1);
+  const float c = scale * LOG2E;
+  const short* kp = k + b * vk.b + hkv * vk.h;
+  const short* vp = v + b * vv.b + hkv * vv.h;
+
+  s16x8 qf[KK], df[KK];
+  {
+    const short* qp = q + b * vq.b + h * vq.h + at * vq.s;
+    const short* dp = dout + b * vd.b + h * vd.h + at * vd.s;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      qf[kk] = *(const s16x8*)(qp + 16 * kk + 8 * half);
+      df[kk] = *(const s16x8*)(dp + 16 * kk + 8 * half);
+    }
+  }
+  const long long sat = ((long long)b * H + h) * S + at;
+  const float ls = stat[sat], dl = stat[rows + sat];
+  f32x16 acc[DB] = {};
+
+  const int end_b = CAUSAL ? min(S, q0b + 128) : S;
+  const int end_w = CAUSAL ? min(S, q0 + 32) : S;
+  const int steps = (end_b + KB - 1) / KB;
+  T::template fetch<KB, 256>(kp, (int)vk.s, S, kt[0], tid);
+  T::template fetch<KB, 256>(vp, (int)vv.s, S, vt[0], tid);
+  __syncthreads();
+  for (int it = 0; it < steps; ++it) {
+    const int k0 = it * KB, cur = it & 1;
+    if (it + 1 < steps) {
+      T::template fetch<KB, 256>(kp + (k0 + KB) * vk.s, (int)vk.s, S - k0 - KB,
+                                kt[cur ^ 1], tid);
+      T::template fetch<KB, 256>(vp + (k0 + KB) * vv.s, (int)vv.s, S - k0 - KB,
+                                vt[cur ^ 1], tid);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int key0 = k0 + 32 * t;
+      if (key0 >= end_w) continue;
+      f32x16 p = {}, dp = {};
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk)
+        p = mfma(T::rows(kt[cur], 32 * t, kk, ra), qf[kk], p);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk)
+        dp = mfma(T::rows(vt[cur], 32 * t, kk, ra), df[kk], dp);
+      __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        dp[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[r], c, -ls)) *
+                (dp[r] - dl);
+      if (key0 + 32 > (CAUSAL ? min(S, q0 + 1) : S)) {
+        const int last = (CAUSAL ? at : S - 1) - key0 - 4 * half;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if ((r & 3) + 8 * (r >> 2) > last) dp[r] = 0.f;
+      }
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const s16x8 sb = operand(dp, s);
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+          acc[db] = mfma(T::cols(kt[cur], 32 * t + 16 * s, db, ca), sb, acc[db]);
+      }
+      __builtin_amdgcn_s_setprio(0);
+    }
+    __syncthreads();
+  }
+  if (row >= S) return;
+  typedef int i32x2 __attribute__((ext_vector_type(2)));
+  short* qp = dq + b * vdq.b + h * vdq.h + row * vdq.s + 4 * half;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *(i32x2*)(qp + 32 * db + 8 * g) = i32x2{
+          pack2(acc[db][4 * g] * scale, acc[db][4 * g + 1] * scale),
+          pack2(acc[db][4 * g + 2] * scale, acc[db][4 * g + 3] * scale)};
+}
+
+View view(const long long* s) { return View{s[0], s[1], s[2]}; }
+
+template <int D>
+void launch_fwd(const void* q, const void* k, const void* v, void* o,
+                float* lse, const long long* st, int B, int S, int H, int Hkv,
+                float scale, bool causal, hipStream_t s) {
+  const int blocks = (S + 255) / 256, heads = B * H;
+#define GO(C)                                                                \
+  hipLaunchKernelGGL((fwd_kernel<D, C>), dim3((unsigned)blocks * heads),     \
+                     dim3(512), 0, s, (const short*)q, (const short*)k,      \
+                     (const short*)v, (short*)o, lse, view(st), view(st + 3),\
+                     view(st + 6), view(st + 9), S, H, Hkv, scale * LOG2E,   \
+                     blocks, heads)
+  if (causal) GO(true);
+  else GO(false);
+#undef GO
+}
+
+template <int D>
+void launch_bwd(const void* q, const void* k, const void* v, const void* o,
+                const void* dout, const float* lse, float* stat, float* part,
+                int splits, void* dq, void* dk, void* dv, const long long* st,
+                int B, int S, int H, int Hkv, float scale, bool causal,
+                hipStream_t s) {
+  const long long rows = (long long)B * S * H;
+  hipLaunchKernelGGL((stat_kernel<D>), dim3((unsigned)((rows + 15) / 16)),
+                     dim3(256), 0, s, (const short*)dout, (const short*)o, lse,
+                     stat, view(st + 12), view(st + 9), S, H, rows);
+  const int blocks = (S + 127) / 128;
+#define GO(C)                                                                 \
+  hipLaunchKernelGGL((dkdv_kernel<D, C>),                                     \
+                     dim3((unsigned)blocks * B * Hkv, splits), dim3(256), 0,  \
+                     s, (const short*)q, (const short*)k, (const short*)v,    \
+                     (const short*)dout, stat, (short*)dk, (short*)dv,        \
+                     view(st), view(st + 3), view(st + 6), view(st + 12),     \
+                     view(st + 18), view(st + 21), S, H, Hkv, scale, blocks,  \
+                     B * Hkv, rows, splits > 1 ? part : nullptr);             \
+  hipLaunchKernelGGL((dq_kernel<D, C>), dim3((unsigned)blocks * B * H),       \
+                     dim3(256), 0, s, (const short*)q, (const short*)k,       \
+                     (const short*)v, (const short*)dout, stat, (short*)dq,   \
+                     view(st), view(st + 3), view(st + 6), view(st + 12),     \
+                     view(st + 15), S, H, Hkv, scale, blocks, B * H, rows)
+  if (causal) { GO(true); }
+  else { GO(false); }
+#undef GO
+  if (splits > 1) {
+    const long long n = (long long)B * S * Hkv * D;
+    hipLaunchKernelGGL(add_kernel, dim3((unsigned)((2 * n / 4 + 255) / 256)),
+                       dim3(256), 0, s, part, (short*)dk, (short*)dv, n,
+                       splits, scale);
   }
 }
 
 }  // namespace
 
-extern "C" void ds_flash_fwd(const void* q, const void* k, const void* vt,
-                             void* o, void* lse, int B, int S, int H,
-                             int Hkv, float scale, int causal, void* stream) {
-  dim3 grid((S + QTILE - 1) / QTILE, H, B);
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (causal)
-    hipLaunchKernelGGL((flash_fwd_kernel<true>), grid, dim3(TPB), 0, st,
-                       (const short*)q, (const short*)k, (const short*)vt,
-                       (short*)o, (float*)lse, B, S, H, Hkv, scale);
-  else
-    hipLaunchKernelGGL((flash_fwd_kernel<false>), grid, dim3(TPB), 0, st,
-                       (const short*)q, (const short*)k, (const short*)vt,
-                       (short*)o, (float*)lse, B, S, H, Hkv, scale);
+// strides: (batch, token, head) of q, k, v, o. scale > 0; lse may be null.
+extern "C" void ds_flash_fwd(const void* q, const void* k, const void* v,
+                             void* o, float* lse, const long long* strides,
+                             int B, int S, int H, int Hkv, int D, float scale,
+                             int causal, void* stream) {
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+#define GO(N) \
+  launch_fwd<N>(q, k, v, o, lse, strides, B, S, H, Hkv, scale, causal, s)
+  if (D == 64) GO(64);
+  else if (D == 96) GO(96);
+  else GO(128);
+#undef GO
 }
 
-// dbg variants: 0 = defer-max OFF (numerics A/B), everything else = full v3
-extern "C" void ds_flash_fwd_dbg(const void* q, const void* k, const void* vt,
-                                 void* o, int B, int S, int H, int Hkv,
-                                 float scale, int variant, void* stream) {
-  dim3 grid((S + QTILE - 1) / QTILE, H, B);
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (variant == 0)
-    hipLaunchKernelGGL((flash_fwd_kernel<true, false>), grid, dim3(TPB), 0,
-                       st, (const short*)q, (const short*)k, (const short*)vt,
-                       (short*)o, nullptr, B, S, H, Hkv, scale);
-  else
-    hipLaunchKernelGGL((flash_fwd_kernel<true, true>), grid, dim3(TPB), 0, st,
-                       (const short*)q, (const short*)k, (const short*)vt,
-                       (short*)o, nullptr, B, S, H, Hkv, scale);
+// Splits of a key head's group for dK and dV. 512 workgroups are resident and
+// a causal one's work goes from nothing to the whole sequence: under 1024 some
+// CUs are idle for a good part, and a divisor of the group (an uneven split
+// leaves the longest as long) that makes 2048 of them pays. Backward, us, by
+// splits 1 / 2 / 4: B 1 x 4096, 32 on 8 heads of 128 (256 workgroups) 995 /
+// 723 / 647; B 2 1362 / 1129 / 1100; B 8 x 2048 (1024) 1236 / 1239 / 1317; 3 x
+// 777, 28 on 4 heads (84), splits 1 / 7: 327 / 126.
+extern "C" int ds_flash_bwd_splits(int B, int S, int H, int Hkv) {
+  const long long wgs = (long long)((S + 127) / 128) * B * Hkv;
+  const int G = H / Hkv;
+  if (wgs >= 1024) return 1;
+  int n = 1;
+  while (n < G && (G % n || wgs * n < 2048)) ++n;
+  return n;
+}
+
+// strides: (batch, token, head) of q, k, v, o, do, dq, dk, dv; dk and dv are
+// contiguous. stat: 2 B H S floats of workspace, part: splits 2 B S Hkv D
+// (splits > 1).
+extern "C" void ds_flash_bwd(const void* q, const void* k, const void* v,
+                             const void* o, const void* dout, const float* lse,
+                             float* stat, float* part, int splits, void* dq,
+                             void* dk, void* dv, const long long* strides,
+                             int B, int S, int H, int Hkv, int D, float scale,
+                             int causal, void* stream) {
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+#define GO(N)                                                              \
+  launch_bwd<N>(q, k, v, o, dout, lse, stat, part, splits, dq, dk, dv,     \
+                strides, B, S, H, Hkv, scale, causal, s)
+  if (D == 64) GO(64);
+  else if (D == 96) GO(96);
+  else GO(128);
+#undef GO
 }

@@ -66,13 +66,17 @@ extern "C" void ds_groupwise_dequant(const void* q, const float* scales,
 extern "C" void ds_fp_quantize(const void* x, int dtype, void* out,
                                float* scales, long long n, int group_size,
                                int bits, int dequant, void* stream);
-extern "C" void ds_flash_bwd_dkdv_dbg(const void* q, const void* k,
-                                      const void* v, const void* dout,
-                                      const void* qt, const void* dot,
-                                      const float* lse, const float* delta,
-                                      void* dk, void* dv, int B, int S,
-                                      int H, int Hkv, float scale,
-                                      int variant, void* stream);
+extern "C" void ds_flash_fwd(const void* q, const void* k, const void* v,
+                             void* o, float* lse, const long long* strides,
+                             int B, int S, int H, int Hkv, int D, float scale,
+                             int causal, void* stream);
+extern "C" int ds_flash_bwd_splits(int B, int S, int H, int Hkv);
+extern "C" void ds_flash_bwd(const void* q, const void* k, const void* v,
+                             const void* o, const void* dout, const float* lse,
+                             float* stat, float* part, int splits, void* dq,
+                             void* dk, void* dv, const long long* strides,
+                             int B, int S, int H, int Hkv, int D, float scale,
+                             int causal, void* stream);
 extern "C" void ds_paged_append(const void* q, const void* k, const void* v,
                                 void* qout, void* kpool, void* vpool,
                                 const int* dst, const float* cs,
@@ -122,19 +126,10 @@ extern "C" int ds_aio_pwrite(void* h, const void* data, long long nbytes,
 extern "C" int ds_aio_pread(void* h, void* data, long long nbytes,
                             const char* path);
 extern "C" int ds_aio_wait(void* h);
-extern "C" void ds_flash_fwd(const void* q, const void* k, const void* vt,
-                             void* o, void* lse, int B, int S, int H,
-                             int Hkv, float scale, int causal, void* stream);
 extern "C" void ds_cpu_lion_flat(float* p, const void* g, int grad_dtype,
                                  float* m, void* p16, long long n, float lr,
                                  float beta1, float beta2, float weight_decay,
                                  float inv_scale);
-extern "C" void ds_flash_bwd(const void* q, const void* k, const void* v,
-                             const void* dout, const void* qt,
-                             const void* kt, const void* dot,
-                             const float* lse, const float* delta, void* dq,
-                             void* dk, void* dv, int B, int S, int H,
-                             int Hkv, float scale, int causal, void* stream);
 extern "C" void ds_ce_fwd(const void* logits, const long long* labels,
                           float* loss, float* lse, int N, long long V,
                           long long ignore_index, void* stream);
@@ -142,9 +137,6 @@ extern "C" void ds_ce_bwd(const void* logits, const long long* labels,
                           const float* lse, const float* gscale,
                           void* dlogits, int N, long long V,
                           long long ignore_index, void* stream);
-extern "C" void ds_flash_fwd_dbg(const void* q, const void* k, const void* vt,
-                                 void* o, int B, int S, int H, int Hkv,
-                                 float scale, int variant, void* stream);
 
 namespace {
 
@@ -765,35 +757,76 @@ at::Tensor groupwise_dequant(at::Tensor q, at::Tensor scales, int64_t numel,
   return out;
 }
 
-at::Tensor flash_attn_fwd(at::Tensor q, at::Tensor k, at::Tensor vt,
-                          double scale, bool causal) {
-  TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kBFloat16,
-              "flash_fwd: bf16 GPU tensors only");
-  TORCH_CHECK(q.is_contiguous() && k.is_contiguous() && vt.is_contiguous(),
-              "flash_fwd: contiguous tensors required");
-  const int B = q.size(0), S = q.size(1), H = q.size(2), D = q.size(3);
-  const int Hkv = k.size(2);
-  TORCH_CHECK(D == 128, "flash_fwd: head_dim must be 128");
-  TORCH_CHECK(S % 32 == 0, "flash_fwd: seq must be a multiple of 32");
-  TORCH_CHECK(k.size(1) == S && vt.size(3) == S && vt.size(2) == D &&
-              vt.size(1) == Hkv && H % Hkv == 0, "flash_fwd: shape mismatch");
-  auto o = at::empty_like(q);
-  ds_flash_fwd(q.data_ptr(), k.data_ptr(), vt.data_ptr(), o.data_ptr(),
-               nullptr, B, S, H, Hkv, (float)scale, causal ? 1 : 0,
-               cur_stream());
-  return o;
+// q, o, do [B, S, H, D], k, v [B, S, Hkv, D] with any strides between tokens
+// and heads that keep 16-byte rows: (batch, token, head) strides, in order.
+struct FlashArgs {
+  int B, S, H, Hkv, D;
+  std::vector<long long> strides;
+  FlashArgs(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+            double scale) {
+    TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && k.sizes() == v.sizes() &&
+                q.size(0) == k.size(0) && q.size(1) == k.size(1) &&
+                q.size(3) == k.size(3), "flash: q [B,S,H,D], k/v [B,S,Hkv,D]");
+    B = q.size(0); S = q.size(1); H = q.size(2); D = q.size(3);
+    Hkv = k.size(2);
+    TORCH_CHECK(D == 64 || D == 96 || D == 128, "flash: D of 64, 96 or 128");
+    TORCH_CHECK(Hkv > 0 && H % Hkv == 0, "flash: H a multiple of Hkv");
+    TORCH_CHECK(scale > 0, "flash: scale must be positive");
+    TORCH_CHECK(q.size(1) < (1 << 30) && q.size(0) * (int64_t)H *
+                ((S + 127) / 128) < (1ll << 31), "flash: size");
+  }
+  void add(const at::Tensor& t, const at::Tensor& like) {
+    TORCH_CHECK(t.is_cuda() && t.scalar_type() == at::kBFloat16 &&
+                t.sizes() == like.sizes() && t.stride(3) == 1 &&
+                ((uintptr_t)t.data_ptr() & 15) == 0 &&
+                t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 &&
+                t.stride(2) % 8 == 0 && t.stride(1) >= 0 &&
+                t.stride(1) < (1 << 24), "flash: bf16 GPU, 16-byte rows");
+    for (int d = 0; d < 3; ++d) strides.push_back(t.stride(d));
+  }
+};
+
+std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
+    at::Tensor q, at::Tensor k, at::Tensor v, double scale, bool causal,
+    bool with_lse) {
+  FlashArgs a(q, k, v, scale);
+  auto o = at::empty({a.B, a.S, a.H, a.D}, q.options());
+  auto lse = at::empty({with_lse ? a.B : 0, a.H, a.S},
+                       q.options().dtype(at::kFloat));
+  a.add(q, q); a.add(k, k); a.add(v, k); a.add(o, q);
+  if (q.numel())
+    ds_flash_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+                 with_lse ? lse.data_ptr<float>() : nullptr, a.strides.data(),
+                 a.B, a.S, a.H, a.Hkv, a.D, (float)scale, causal ? 1 : 0,
+                 cur_stream());
+  return {o, lse};
 }
 
-std::tuple<at::Tensor, at::Tensor> flash_attn_fwd_lse(
-    at::Tensor q, at::Tensor k, at::Tensor vt, double scale, bool causal) {
-  const int B = q.size(0), S = q.size(1), H = q.size(2);
-  const int Hkv = k.size(2);
-  auto o = at::empty_like(q);
-  auto lse = at::empty({B, H, S}, q.options().dtype(at::kFloat));
-  ds_flash_fwd(q.data_ptr(), k.data_ptr(), vt.data_ptr(), o.data_ptr(),
-               lse.data_ptr<float>(), B, S, H, Hkv, (float)scale,
-               causal ? 1 : 0, cur_stream());
-  return {o, lse};
+std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
+    at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor o, at::Tensor dout,
+    at::Tensor lse, double scale, bool causal, int64_t splits) {
+  FlashArgs a(q, k, v, scale);
+  if (splits == 0) splits = ds_flash_bwd_splits(a.B, a.S, a.H, a.Hkv);
+  TORCH_CHECK(splits >= 1 && splits <= a.H / a.Hkv, "flash_bwd: splits");
+  TORCH_CHECK(lse.is_cuda() && lse.scalar_type() == at::kFloat &&
+              lse.is_contiguous() &&
+              lse.numel() == (int64_t)a.B * a.H * a.S, "flash_bwd: lse");
+  auto dq = at::empty({a.B, a.S, a.H, a.D}, q.options());
+  auto dk = at::empty({a.B, a.S, a.Hkv, a.D}, q.options());
+  auto dv = at::empty({a.B, a.S, a.Hkv, a.D}, q.options());
+  auto stat = at::empty({2, lse.numel()}, lse.options());
+  auto part = at::empty({splits > 1 ? 2 * splits * dk.numel() : 0},
+                        lse.options());
+  a.add(q, q); a.add(k, k); a.add(v, k); a.add(o, q); a.add(dout, q);
+  a.add(dq, q); a.add(dk, k); a.add(dv, k);
+  if (q.numel())
+    ds_flash_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+                 dout.data_ptr(), lse.data_ptr<float>(),
+                 stat.data_ptr<float>(), part.data_ptr<float>(), (int)splits,
+                 dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                 a.strides.data(), a.B, a.S, a.H, a.Hkv, a.D, (float)scale,
+                 causal ? 1 : 0, cur_stream());
+  return {dq, dk, dv};
 }
 
 class AioHandle {
@@ -835,23 +868,6 @@ class AioHandle {
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("flash_bwd_dkdv_dbg",
-        [](at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor dout,
-           at::Tensor qt, at::Tensor dot, at::Tensor lse, at::Tensor delta,
-           at::Tensor dk, at::Tensor dv, double scale, int64_t variant) {
-          const int B = q.size(0), H = q.size(1), S = q.size(2);
-          const int Hkv = k.size(1);
-          ds_flash_bwd_dkdv_dbg(q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                dout.data_ptr(), qt.data_ptr(),
-                                dot.data_ptr(), lse.data_ptr<float>(),
-                                delta.data_ptr<float>(), dk.data_ptr(),
-                                dv.data_ptr(), B, S, H, Hkv, (float)scale,
-                                (int)variant, cur_stream());
-        },
-        "dkdv-only launcher (perf diagnosis)");
-  pybind11::class_<ShmComm>(m, "ShmComm")
-      .def(pybind11::init<const std::string&, int64_t, int64_t, int64_t>())
-      .def("all_reduce", &ShmComm::all_reduce);
   m.def("paged_decode", &paged_decode,
         "split-KV decode attention over a paged KV block table");
   m.def("rows_linear", &rows_linear,
@@ -939,48 +955,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           return d;
         },
         "fused CE backward: dlogits in bf16");
-  m.def("flash_attn_fwd_lse", &flash_attn_fwd_lse,
-        "flash fwd returning (o, logsumexp) for training");
-  m.def("flash_attn_bwd",
-        [](at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor dout,
-           at::Tensor qt, at::Tensor kt, at::Tensor dot, at::Tensor lse,
-           at::Tensor delta, double scale, bool causal) {
-          TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kBFloat16 &&
-                      q.is_contiguous() && k.is_contiguous() &&
-                      v.is_contiguous() && dout.is_contiguous() &&
-                      qt.is_contiguous() && kt.is_contiguous() &&
-                      dot.is_contiguous(), "flash_bwd: bf16 contiguous GPU");
-          TORCH_CHECK(lse.scalar_type() == at::kFloat &&
-                      delta.scalar_type() == at::kFloat, "lse/delta fp32");
-          const int B = q.size(0), H = q.size(1), S = q.size(2);
-          const int Hkv = k.size(1);
-          TORCH_CHECK(q.size(3) == 128 && S % 32 == 0,
-                      "flash_bwd: D=128, S%32==0");
-          auto dq = at::empty_like(q);
-          auto dk = at::empty_like(k);
-          auto dv = at::empty_like(v);
-          ds_flash_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                       dout.data_ptr(), qt.data_ptr(), kt.data_ptr(),
-                       dot.data_ptr(), lse.data_ptr<float>(),
-                       delta.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(),
-                       dv.data_ptr(), B, S, H, Hkv, (float)scale,
-                       causal ? 1 : 0, cur_stream());
-          return std::make_tuple(dq, dk, dv);
-        },
-        "MFMA flash-attention backward (BHSD; GPU-validation pending)");
-  m.def("flash_attn_fwd_dbg",
-        [](at::Tensor q, at::Tensor k, at::Tensor vt, double scale,
-           int64_t variant) {
-          auto o = at::empty_like(q);
-          ds_flash_fwd_dbg(q.data_ptr(), k.data_ptr(), vt.data_ptr(),
-                           o.data_ptr(), q.size(0), q.size(1), q.size(2),
-                           k.size(2), (float)scale, (int)variant,
-                           cur_stream());
-          return o;
-        },
-        "flash fwd ablation (bit0 K-LDS, bit1 V-LDS)");
   m.def("flash_attn_fwd", &flash_attn_fwd,
-        "MFMA flash-attention forward (bf16, D=128, GQA, causal)");
+        "flash attention forward (bf16, MFMA): (o, logsumexp)");
+  m.def("flash_attn_bwd", &flash_attn_bwd,
+        "flash attention backward (bf16, MFMA): (dq, dk, dv)",
+        pybind11::arg("q"), pybind11::arg("k"), pybind11::arg("v"),
+        pybind11::arg("o"), pybind11::arg("dout"), pybind11::arg("lse"),
+        pybind11::arg("scale"), pybind11::arg("causal"),
+        pybind11::arg("splits") = 0);
   pybind11::class_<AioHandle>(m, "AioHandle")
       .def(pybind11::init<int64_t, int>(),
            pybind11::arg("block_size") = 1 << 20,

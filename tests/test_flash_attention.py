@@ -1,0 +1,108 @@
+"""Flash attention kernels against fp64 attention, head by head."""
+
+import math
+
+import pytest
+import torch
+
+from deepspeed_amd.ops import attention
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(q, k, v, do, causal, scale):
+    B, S, H, D = q.shape
+    G = H // k.shape[2]
+    q, k, v = (x.detach().double().requires_grad_() for x in (q, k, v))
+    hidden = torch.ones(S, S, dtype=torch.bool, device=q.device).triu(1)
+    out = []
+    for b in range(B):
+        for h in range(H):
+            s = q[b, :, h] @ k[b, :, h // G].t() * scale
+            if causal:
+                s = s.masked_fill(hidden, -math.inf)
+            out.append(torch.softmax(s, -1) @ v[b, :, h // G])
+    o = torch.stack(out).view(B, H, S, D).transpose(1, 2)
+    o.backward(do.double())
+    return o.detach(), q.grad, k.grad, v.grad
+
+
+def _close(got, want, what):
+    # operands, probabilities and the result are bf16: 2^-9 each, a handful of
+    # them in a row; sums of few terms, or that cancel, count by their size
+    d = (got.double() - want).norm()
+    assert d <= 0.01 * want.norm() + 1e-3 * want.numel() ** 0.5 * 0.05, \
+        (what, (d / want.norm()).item())
+
+
+SHAPES = [(1, 1, 2, 1), (1, 31, 1, 1), (2, 64, 4, 2), (1, 65, 7, 1),
+          (1, 127, 3, 3), (1, 128, 14, 2), (2, 129, 4, 1), (1, 255, 8, 8),
+          (1, 257, 16, 2), (1, 777, 28, 4)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("d", [64, 96, 128])
+@pytest.mark.parametrize("causal", [True, False])
+def test_flash_attention(shape, d, causal):
+    B, S, H, Hkv = shape
+    torch.manual_seed(S + d)
+    q = torch.randn(B, S, H, d, device="cuda").bfloat16().requires_grad_()
+    k, v = (torch.randn(B, S, Hkv, d, device="cuda").bfloat16()
+            .requires_grad_() for _ in range(2))
+    do = torch.randn(B, S, H, d, device="cuda").bfloat16()
+    o = attention.flash_attn_func(q, k, v, causal=causal)
+    o.backward(do)
+    want = _reference(q, k, v, do, causal, d ** -0.5)
+    for got, w, n in zip((o, q.grad, k.grad, v.grad), want,
+                         ("o", "dq", "dk", "dv")):
+        assert got.isfinite().all()
+        _close(got, w, n)
+    with torch.no_grad():
+        assert torch.equal(attention.flash_attn_fwd(q, k, v, causal), o)
+
+
+@pytest.mark.parametrize("splits", [1, 2, 3, 4])
+def test_splits_agree(splits):
+    from deepspeed_amd.ops import _C
+    torch.manual_seed(0)
+    q, do = (torch.randn(2, 300, 8, 128, device="cuda").bfloat16()
+             for _ in range(2))
+    k, v = (torch.randn(2, 300, 2, 128, device="cuda").bfloat16()
+            for _ in range(2))
+    o, lse = _C.flash_attn_fwd(q, k, v, 0.09, True, True)
+    got = _C.flash_attn_bwd(q, k, v, o, do, lse, 0.09, True, splits)
+    for g, w, n in zip(got, _reference(q, k, v, do, True, 0.09)[1:],
+                       ("dq", "dk", "dv")):
+        _close(g, w, n)
+
+
+@pytest.mark.parametrize("scale", [0.3, -0.2, 0.0])
+def test_scales_and_strides(scale):
+    """Slices of one buffer, as a joint projection leaves them, BHSD views and
+    an odd offset; any sign of the scale."""
+    torch.manual_seed(0)
+    joint = torch.randn(2, 100, 8, 64, device="cuda").bfloat16()
+    q, k, v = joint[:, :, :4], joint[:, :, 4:6], joint[:, :, 6:]
+    do = torch.randn(2, 4, 100, 64, device="cuda").bfloat16().transpose(1, 2)
+    odd = torch.empty(k.numel() + 1, device="cuda").bfloat16()[1:]
+    k2 = odd.view(k.shape).copy_(k)
+    for kk in (k, k2):
+        a, b, c = (t.detach().requires_grad_() for t in (q, kk, v))
+        o = attention.flash_attn_func(a, b, c, True, scale)
+        o.backward(do)
+        want = _reference(q, kk, v, do, True, scale)
+        for got, w, n in zip((o, a.grad, b.grad, c.grad), want,
+                             ("o", "dq", "dk", "dv")):
+            _close(got, w, n)
+
+
+def test_backward_repeats():
+    torch.manual_seed(0)
+    q = torch.randn(1, 500, 8, 128, device="cuda").bfloat16().requires_grad_()
+    k, v = (torch.randn(1, 500, 2, 128, device="cuda").bfloat16()
+            .requires_grad_() for _ in range(2))
+    do = torch.randn_like(q)
+    o = attention.flash_attn_func(q, k, v)
+    a = torch.autograd.grad(o, (q, k, v), do, retain_graph=True)
+    b = torch.autograd.grad(o, (q, k, v), do)
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
