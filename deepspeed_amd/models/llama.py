@@ -6,8 +6,9 @@ synthetic data; architecture matches Llama-3 (GQA attention, RoPE
 theta=500000, SwiGLU MLP, RMSNorm, tied-off lm_head).
 
 Hot ops: RMSNorm / RoPE / SwiGLU are the hand-written HIP kernels in
-``deepspeed_amd.ops``; GEMMs go through torch (hipBLASLt); attention uses
-torch SDPA (flash backend on ROCm) with an explicit-math fallback.
+``deepspeed_amd.ops``, and so is attention (flash forward and backward, paged
+serving) wherever its kernels apply, else torch SDPA; GEMMs go through torch
+(hipBLASLt).
 """
 
 from dataclasses import dataclass
@@ -16,6 +17,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from ..ops.attention import rope_flash_attention
 from ..ops.linear import SWIGLU, Linear, rows_linear, unhooked
 from ..ops.norms import RMSNorm
 from ..ops.rope import apply_rope, rope_tables
@@ -146,28 +148,20 @@ class LlamaAttention(nn.Module):
             if o is not None:
                 kv_cache.last_decoded = S == 1
                 return self._out(o.reshape(B, S, -1))
+        sp = getattr(self, "sp_group", None)
+        if kv_cache is None and attention_fn is None and sp is None:
+            # hand-written CDNA4 kernels, [B, S, H, D] throughout
+            o = rope_flash_attention(q, k, v, cos, sin, positions)
+            if o is not None:
+                return self._out(o.reshape(B, S, -1))
         q = apply_rope(q, cos, sin, positions)
         k = apply_rope(k, cos, sin, positions)
 
-        if getattr(self, "sp_group", None) is not None and kv_cache is None:
+        if sp is not None and kv_cache is None:
             # Ulysses: all-to-all scatters heads / gathers the sequence so
             # each rank runs full-sequence causal attention on H/P heads
             o = self._ulysses_attn(q, k, v)
             return self._out(o.reshape(B, S, -1))
-
-        if kv_cache is None and attention_fn is None:
-            from ..ops.attention import (flash_attn_available, flash_attn_fwd,
-                                         flash_attn_func,
-                                         flash_train_available)
-            if flash_attn_available(q, k):
-                # hand-written CDNA4 MFMA flash kernel, BSHD layout — skips
-                # the transpose entirely (inference/no-grad prefill path)
-                o = flash_attn_fwd(q, k, v, causal=True)
-                return self._out(o.reshape(B, S, -1))
-            if torch.is_grad_enabled() and flash_train_available(q, k):
-                # differentiable hand-written path (fwd + dk/dv/dq kernels)
-                o = flash_attn_func(q, k, v, causal=True)
-                return self._out(o.reshape(B, S, -1))
 
         if (S == 1 and kv_cache is not None
                 and hasattr(kv_cache, "decode_attention")

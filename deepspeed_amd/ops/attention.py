@@ -13,7 +13,7 @@ from ._loader import get_ext
 
 def _eligible(q: torch.Tensor, k: torch.Tensor) -> bool:
     return (get_ext() is not None and q.is_cuda
-            and q.dtype == k.dtype == torch.bfloat16
+            and q.dtype is torch.bfloat16 and k.dtype is torch.bfloat16
             and q.dim() == 4 and k.dim() == 4
             and q.size(-1) == k.size(-1) and q.size(-1) in (64, 96, 128)
             and q.size(1) == k.size(1) and q.size(2) % k.size(2) == 0
@@ -127,6 +127,50 @@ class FlashAttnFunc(torch.autograd.Function):
         dq, dk, dv = get_ext().flash_attn_bwd(q, k, v, o, _rows(do), lse,
                                               ctx.scale, ctx.causal)
         return (dq if ctx.factor == 1 else dq * ctx.factor), dk, dv, None, None
+
+
+class RopeFlashFunc(torch.autograd.Function):
+    """Causal attention of unrotated q, k [B, S, H(kv), D]: one launch rotates
+    both, and the gradients on their way back in place."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, cos, sin, positions):
+        ext = get_ext()
+        q, k = ext.rope(q.contiguous(), k.contiguous(), cos, sin, positions,
+                        False)
+        v = _rows(v)
+        ctx.scale = 1.0 / math.sqrt(q.size(-1))
+        o, lse = ext.flash_attn_fwd(q, k, v, ctx.scale, True, True)
+        ctx.save_for_backward(q, k, v, o, lse, cos, sin, positions)
+        return o
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, do):
+        q, k, v, o, lse, cos, sin, positions = ctx.saved_tensors
+        ext = get_ext()
+        dq, dk, dv = ext.flash_attn_bwd(q, k, v, o, _rows(do), lse, ctx.scale,
+                                        True)
+        ext.rope(dq, dk, cos, sin, positions, True, True)
+        return dq, dk, dv, None, None, None
+
+
+def rope_flash_attention(q, k, v, cos, sin, positions=None):
+    """Rotary embedding and causal attention, [B, S, H(kv), D] bf16; None where
+    the kernels do not apply."""
+    grad = torch.is_grad_enabled()
+    if not (flash_train_available(q, k) if grad else
+            flash_attn_available(q, k)) or (
+            positions is None and cos.size(0) < q.size(1)) or (
+            positions is not None and positions.dtype != torch.int32):
+        return None
+    if positions is not None:
+        positions = positions.contiguous()
+    if grad:
+        return RopeFlashFunc.apply(q, k, v, cos, sin, positions)
+    q, k = get_ext().rope(q.contiguous(), k.contiguous(), cos, sin, positions,
+                          False)
+    return flash_attn_fwd(q, k, v)
 
 
 def flash_attn_func(q, k, v, causal=True, scale=None):

@@ -36,10 +36,11 @@ extern "C" void ds_norm_bwd(const void* dy, const void* x, const void* w,
                             const void* dres, void* dx, float* dwb,
                             float* part, int rows, int H, int ln, int dtype,
                             void* stream);
-extern "C" void ds_rope(void* x, const float* cos_table, const float* sin_table,
-                        const int* positions, long long batch, long long seq,
-                        long long heads, long long dim, int bwd, int dtype,
-                        void* stream);
+extern "C" void ds_rope(const void* x1, void* y1, int heads1, const void* x2,
+                        void* y2, int heads2, const float* cos_table,
+                        const float* sin_table, const int* positions,
+                        long long batch, long long seq, long long dim, int bwd,
+                        int dtype, void* stream);
 extern "C" void ds_gated_act_fwd(const void* gate, const void* up, void* out,
                                  long long n, int act, int dtype, void* stream);
 extern "C" void ds_gated_act_bwd(const void* dout, const void* gate,
@@ -685,12 +686,18 @@ at::Tensor nhwc_bias_add(at::Tensor act, at::Tensor bias,
   return out;
 }
 
-void rope(at::Tensor x, at::Tensor cos_table, at::Tensor sin_table,
-          c10::optional<at::Tensor> positions, bool backward) {
-  TORCH_CHECK(x.dim() == 4 && x.is_contiguous(), "rope expects [B,S,H,D]");
-  TORCH_CHECK(cos_table.scalar_type() == at::kFloat &&
-              sin_table.scalar_type() == at::kFloat, "tables must be fp32");
-  const int64_t B = x.size(0), S = x.size(1), Hh = x.size(2), D = x.size(3);
+// Rotates x [B, S, H, D] (and x2, of other heads) into new tensors, or in
+// place.
+std::vector<at::Tensor> rope(at::Tensor x, c10::optional<at::Tensor> x2,
+                             at::Tensor cos_table, at::Tensor sin_table,
+                             c10::optional<at::Tensor> positions,
+                             bool backward, bool inplace) {
+  TORCH_CHECK(x.dim() == 4 && x.is_contiguous() && x.is_cuda(),
+              "rope expects [B,S,H,D]");
+  for (auto& t : {cos_table, sin_table})
+    TORCH_CHECK(t.scalar_type() == at::kFloat && t.is_contiguous() &&
+                t.is_cuda(), "tables must be fp32");
+  const int64_t B = x.size(0), S = x.size(1), D = x.size(3);
   TORCH_CHECK(cos_table.size(-1) == D / 2, "table dim mismatch");
   TORCH_CHECK(cos_table.size(0) >= S || positions.has_value(),
               "cos table shorter than sequence");
@@ -701,9 +708,21 @@ void rope(at::Tensor x, at::Tensor cos_table, at::Tensor sin_table,
                 "positions must be int32 [B,S]");
     pos_ptr = positions->data_ptr<int>();
   }
-  ds_rope(x.data_ptr(), cos_table.data_ptr<float>(),
-          sin_table.data_ptr<float>(), pos_ptr, B, S, Hh, D, backward ? 1 : 0,
+  std::vector<at::Tensor> in = {x}, out;
+  if (x2.has_value()) {
+    TORCH_CHECK(x2->dim() == 4 && x2->is_contiguous() && x2->is_cuda() &&
+                x2->size(0) == B && x2->size(1) == S && x2->size(3) == D &&
+                x2->scalar_type() == x.scalar_type(), "rope: second tensor");
+    in.push_back(*x2);
+  }
+  for (auto& t : in) out.push_back(inplace ? t : at::empty_like(t));
+  const bool two = in.size() == 2;
+  ds_rope(in[0].data_ptr(), out[0].data_ptr(), (int)x.size(2),
+          two ? in[1].data_ptr() : nullptr, two ? out[1].data_ptr() : nullptr,
+          two ? (int)in[1].size(2) : 0, cos_table.data_ptr<float>(),
+          sin_table.data_ptr<float>(), pos_ptr, B, S, D, backward ? 1 : 0,
           dtype_code(x), cur_stream());
+  return out;
 }
 
 at::Tensor gated_act_fwd(at::Tensor gate, at::Tensor up, int64_t act) {
@@ -912,7 +931,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         pybind11::arg("invrms"), pybind11::arg("mean"),
         pybind11::arg("layernorm"), pybind11::arg("dres") = c10::nullopt);
   m.def("add_norm_fwd", &add_norm_fwd, "RMS norm of a sum, and the sum");
-  m.def("rope", &rope, "Rotary position embedding (in-place)");
+  m.def("rope", &rope, "Rotary position embedding of one or two tensors",
+        pybind11::arg("x"), pybind11::arg("x2"), pybind11::arg("cos"),
+        pybind11::arg("sin"), pybind11::arg("positions"),
+        pybind11::arg("backward"), pybind11::arg("inplace") = false);
   m.def("token_gather", &token_gather,
         "row-coalesced token gather [B,S,D] x [B,K] -> [B,K,D]");
   m.def("token_scatter", &token_scatter,

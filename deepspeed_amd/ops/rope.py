@@ -129,7 +129,7 @@ def _torch_rope(x, cos, sin, positions=None, backward=False):
 
 
 class _RopeFn(torch.autograd.Function):
-    """Out-of-place autograd wrapper (kernel itself is in-place on a copy)."""
+    """Out-of-place autograd wrapper."""
 
     @staticmethod
     def forward(ctx, x, cos, sin, positions):
@@ -138,9 +138,8 @@ class _RopeFn(torch.autograd.Function):
                               torch.empty(0))
         ext = get_ext()
         if ext is not None and x.is_cuda:
-            out = x.contiguous().clone()
-            ext.rope(out, cos, sin, positions, False)
-            return out
+            return ext.rope(x.contiguous(), None, cos, sin, positions,
+                            False)[0]
         return _torch_rope(x, cos, sin, positions, backward=False)
 
     @staticmethod
@@ -149,8 +148,7 @@ class _RopeFn(torch.autograd.Function):
         positions = positions if positions.numel() else None
         ext = get_ext()
         if ext is not None and dy.is_cuda:
-            dx = dy.contiguous().clone()
-            ext.rope(dx, cos, sin, positions, True)
+            dx = ext.rope(dy.contiguous(), None, cos, sin, positions, True)[0]
             return dx, None, None, None
         return _torch_rope(dy, cos, sin, positions, backward=True), None, None, None
 

@@ -106,3 +106,52 @@ def test_backward_repeats():
     a = torch.autograd.grad(o, (q, k, v), do, retain_graph=True)
     b = torch.autograd.grad(o, (q, k, v), do)
     assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("d", [64, 96, 128])
+@pytest.mark.parametrize("given", [False, True])
+def test_rope_flash_is_rope_then_flash(d, given):
+    from deepspeed_amd.ops.rope import apply_rope, rope_tables
+    torch.manual_seed(d)
+    cos, sin = rope_tables(d, 200, 1e4, device="cuda")
+    q = torch.randn(2, 75, 6, d, device="cuda").bfloat16()
+    k, v = (torch.randn(2, 75, 2, d, device="cuda").bfloat16()
+            for _ in range(2))
+    pos = torch.randint(0, 200, (2, 75), device="cuda", dtype=torch.int32) \
+        if given else None
+    do = torch.randn_like(q)
+    res = []
+    for f in (lambda a, b, c: attention.rope_flash_attention(a, b, c, cos, sin,
+                                                             pos),
+              lambda a, b, c: attention.flash_attn_func(
+                  apply_rope(a, cos, sin, pos), apply_rope(b, cos, sin, pos),
+                  c)):
+        x = [t.clone().requires_grad_() for t in (q, k, v)]
+        o = f(*x)
+        o.backward(do)
+        res.append([o] + [t.grad for t in x])
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+    with torch.no_grad():
+        assert torch.equal(attention.rope_flash_attention(q, k, v, cos, sin,
+                                                          pos), res[0][0])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16,
+                                   torch.float32])
+@pytest.mark.parametrize("d,h", [(2, 3), (34, 1), (64, 5), (96, 2), (128, 8)])
+def test_rope_pairs(dtype, d, h):
+    from deepspeed_amd.ops import _C
+    from deepspeed_amd.ops.rope import _torch_rope, rope_tables
+    torch.manual_seed(0)
+    cos, sin = rope_tables(d, 50, 1e4, device="cuda")
+    x = torch.randn(2, 33, h, d, device="cuda").to(dtype)
+    y = torch.randn(2, 33, 2, d, device="cuda").to(dtype)
+    for back in (False, True):
+        got = _C.rope(x, y, cos, sin, None, back)
+        for g, t in zip(got, (x, y)):
+            torch.testing.assert_close(
+                g, _torch_rope(t, cos, sin, None, back),
+                rtol=2 * torch.finfo(dtype).eps, atol=1e-6)
+        a = x.clone()
+        _C.rope(a, None, cos, sin, None, back, True)
+        assert torch.equal(a, got[0])
