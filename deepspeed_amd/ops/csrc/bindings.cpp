@@ -67,6 +67,9 @@ extern "C" void ds_groupwise_dequant(const void* q, const float* scales,
 extern "C" void ds_fp_quantize(const void* x, int dtype, void* out,
                                float* scales, long long n, int group_size,
                                int bits, int dequant, void* stream);
+extern "C" int ds_sumsq_parts(const long long* n, int count);
+extern "C" void ds_sumsq(const void* const* p, const long long* n, int count,
+                         int dtype, float* part, float* out, void* stream);
 extern "C" void ds_flash_fwd(const void* q, const void* k, const void* v,
                              void* o, float* lse, const long long* strides,
                              int B, int S, int H, int Hkv, int D, float scale,
@@ -490,6 +493,28 @@ std::vector<at::Tensor> rows_linear(
   return out;
 }
 
+at::Tensor sum_of_squares(std::vector<at::Tensor> ts) {
+  TORCH_CHECK(!ts.empty(), "sum_of_squares: no tensors");
+  std::vector<const void*> p;
+  std::vector<long long> n;
+  for (auto& t : ts) {
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
+                t.scalar_type() == ts[0].scalar_type() &&
+                t.device() == ts[0].device() &&
+                (t.scalar_type() == at::kFloat ||
+                 t.scalar_type() == at::kBFloat16) &&
+                t.numel() < (1ll << 45), "sum_of_squares: bf16 or fp32 GPU");
+    p.push_back(t.data_ptr());
+    n.push_back(t.numel());
+  }
+  auto f32 = ts[0].options().dtype(at::kFloat);
+  auto part = at::empty({ds_sumsq_parts(n.data(), (int)n.size())}, f32);
+  auto out = at::empty({}, f32);
+  ds_sumsq(p.data(), n.data(), (int)n.size(), dtype_code(ts[0]),
+           part.data_ptr<float>(), out.data_ptr<float>(), cur_stream());
+  return out;
+}
+
 class ShmComm {
  public:
   ShmComm(const std::string& name, int64_t rank, int64_t world,
@@ -891,6 +916,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "split-KV decode attention over a paged KV block table");
   m.def("rows_linear", &rows_linear,
         "linear layers of a few rows, bf16 or groupwise int8 weights");
+  m.def("sum_of_squares", &sum_of_squares,
+        "sum of squares over a list of tensors");
   m.def("paged_rows", &paged_rows,
         "attention of a serving step's runs of tokens over the paged pool");
   m.def("paged_append", &paged_append,

@@ -36,6 +36,7 @@ from ... import accel
 from ... import comm as dist
 from ...utils.logging import log_dist
 from ..fp16.loss_scaler import LossScalerBase, LossScaler
+from ...ops.grad_norm import sum_of_squares
 from ..utils import ALIGNMENT
 from ...utils.nvtx import instrument_w_nvtx
 
@@ -400,8 +401,7 @@ class ZeroStage12Optimizer:
                 dist.all_reduce(norm_sq_dev,
                                 group=self.mpu.get_model_parallel_group())
         elif owned:
-            norms = torch._foreach_norm(owned, 2.0)
-            norm_sq_dev = torch.stack([n.float() for n in norms]).pow(2).sum()
+            norm_sq_dev = sum_of_squares(owned)
             if dist.is_initialized() and self.world_size > 1:
                 dist.all_reduce(norm_sq_dev, group=self.dp_group)
             if self.mpu is not None:

@@ -45,6 +45,7 @@ from ... import accel
 from ... import comm as dist
 from ...utils.logging import log_dist
 from ..fp16.loss_scaler import LossScalerBase, LossScaler
+from ...ops.grad_norm import sum_of_squares
 from ..utils import ALIGNMENT
 from ...utils.nvtx import instrument_w_nvtx
 
@@ -871,8 +872,7 @@ class ZeroStage3Optimizer:
             owned = [g for g in self.group_owned_grads if g.numel() > 0]
         norm_sq = None
         if owned:
-            norms = torch._foreach_norm(owned, 2.0)
-            norm_sq = torch.stack([n.float() for n in norms]).pow(2).sum()
+            norm_sq = sum_of_squares(owned)
             if dist.is_initialized() and self.world_size > 1:
                 if norm_sq.is_cuda or not self.cpu_offload:
                     dist.all_reduce(norm_sq, group=self.dp_group)

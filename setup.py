@@ -25,6 +25,7 @@ ext = CUDAExtension(
         os.path.join(CSRC, "shm_comm.cpp"),
         os.path.join(CSRC, "adam.hip"),
         os.path.join(CSRC, "optim.hip"),
+        os.path.join(CSRC, "grad_norm.hip"),
         os.path.join(CSRC, "fp_quant.hip"),
         os.path.join(CSRC, "transpose.hip"),
         os.path.join(CSRC, "softmax_dropout.hip"),
