@@ -118,6 +118,11 @@ class ZeroStage12Optimizer:
         self.group_params: List[List[torch.nn.Parameter]] = []
         self.group_shard_numel: List[int] = []
 
+        # One rank, nothing to exchange: the flat gradient buffers ARE the
+        # rank's shards. No reduction, no second copy of the gradients.
+        self._local = (self.world_size == 1 and not cpu_offload and all(
+            dist.get_world_size(self._group_pg(g)) == 1
+            for g in self.optimizer.param_groups))
         self._build_flat_buffers()
         self._replace_inner_params()
         self._register_hooks()
@@ -212,7 +217,8 @@ class ZeroStage12Optimizer:
 
             master_device = torch.device("cpu") if self.cpu_offload else device
             master = torch.empty(shard_total, dtype=torch.float32, device=master_device)
-            owned = torch.empty(shard_total, dtype=gdtype, device=master_device)
+            owned = torch.empty(0 if self._local else shard_total, dtype=gdtype,
+                                device=master_device)
             if self.cpu_offload and self.offload_pin_memory and accel.available():
                 master = master.pin_memory()
                 owned = owned.pin_memory()
@@ -283,6 +289,8 @@ class ZeroStage12Optimizer:
     def _reduce_bucket(self, bucket: _Bucket):
         """Reduce-scatter (stage 2) or all-reduce (stage 1) one bucket."""
         bucket.reduced = True
+        if self._local:
+            return
         grad = bucket.grad_flat
         master = self.group_masters[bucket.group_idx]
         owned = self.group_owned_grads[bucket.group_idx]
@@ -387,7 +395,8 @@ class ZeroStage12Optimizer:
 
         # overflow check (fp16 path) + grad norm on owned shards
         scale = self.loss_scaler.loss_scale
-        owned = [g for g in self.group_owned_grads if g.numel() > 0]
+        owned = [b.grad_flat for b in self.buckets] if self._local else \
+            [g for g in self.group_owned_grads if g.numel() > 0]
         norm_sq_dev = None
         if self.cpu_offload and self._dev_norm_sq is not None:
             # per-rank shard norms are partial sums — the global norm (and
@@ -406,8 +415,9 @@ class ZeroStage12Optimizer:
                 dist.all_reduce(norm_sq_dev, group=self.dp_group)
             if self.mpu is not None:
                 dist.all_reduce(norm_sq_dev, group=self.mpu.get_model_parallel_group())
-        self.overflow = bool(norm_sq_dev is not None and
-                             (torch.isinf(norm_sq_dev) or torch.isnan(norm_sq_dev)))
+        # one transfer: what follows is decided and scaled on the host
+        norm_sq = None if norm_sq_dev is None else float(norm_sq_dev)
+        self.overflow = norm_sq is not None and not math.isfinite(norm_sq)
         self.loss_scaler.update_scale(self.overflow)
         if self.overflow:
             log_dist(f"overflow detected, skipping step "
@@ -416,12 +426,11 @@ class ZeroStage12Optimizer:
             self._reset_buckets()
             return
 
-        global_norm = (norm_sq_dev.sqrt() / scale) if norm_sq_dev is not None else None
+        global_norm = math.sqrt(norm_sq) / scale if norm_sq is not None else 0.0
         combined_scale = scale
-        if self.clip_grad > 0 and global_norm is not None:
-            clip = (global_norm / self.clip_grad).clamp(min=1.0)
-            combined_scale = scale * clip
-        self._global_grad_norm = float(global_norm) if global_norm is not None else 0.0
+        if self.clip_grad > 0:
+            combined_scale = scale * max(1.0, global_norm / self.clip_grad)
+        self._global_grad_norm = global_norm
 
         stepped = wrote_params = False
         if self.fused_adam_fn is not None:
@@ -456,7 +465,8 @@ class ZeroStage12Optimizer:
                                    (b.pg_rank + 1) * b.shard_size]
                 else:
                     wrote_params = False
-                segments.append((b.master_offset, b.shard_size, out16))
+                segments.append((b.master_offset, b.shard_size, out16) + (
+                    (b.grad_flat,) if self._local else ()))
                 seg_buckets.append(b)
             if self.cpu_offload:
                 # pipelined: wait only THIS bucket's D2H, step it on the
@@ -484,7 +494,11 @@ class ZeroStage12Optimizer:
             master = self.group_masters[gi]
             if master.numel() == 0:
                 continue
-            g = self.group_owned_grads[gi].to(dtype=torch.float32)
+            if self._local:
+                g = torch.cat([b.grad_flat for b in self.buckets
+                               if b.group_idx == gi]).to(dtype=torch.float32)
+            else:
+                g = self.group_owned_grads[gi].to(dtype=torch.float32)
             if isinstance(combined_scale, torch.Tensor) or combined_scale != 1.0:
                 g = g / combined_scale
             master.grad = g

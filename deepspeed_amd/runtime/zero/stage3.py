@@ -668,17 +668,33 @@ class ZeroStage3Optimizer:
         copied in by the post-accumulate hook (first arrival = copy, later
         arrivals = add), which removes the per-microstep fill kernel and the
         autograd `p.grad +=` read-modify-write of the preset-view scheme."""
-        if not u.trainable:
+        if not u.trainable or self._takes_grad(u):
             return
-        if u.grad_full is None:
+        self._grad_buffer(u)
+
+    def _grad_buffer(self, u: _Unit):
+        if u.trainable and u.grad_full is None:
             u.grad_full = torch.empty(u.numel, dtype=self._dtype,
                                       device=self._device)
             u.grad_seen = [False] * len(u.params)
 
+    def _takes_grad(self, u: _Unit) -> bool:
+        """One rank and one parameter without padding: the gradient that
+        autograd hands over is the unit's buffer, no copy of it is made."""
+        return (self.world_size == 1 and len(u.params) == 1
+                and u.params[0].ds_numel == u.numel)
+
     def _make_grad_hook(self, u: _Unit, idx: int, off: int):
         def hook(param):
-            if u.grad_full is None:
-                self._ensure_grad_buffer(u)
+            g = param.grad
+            if (g is not None and u.grad_full is None and self._takes_grad(u)
+                    and g.dtype == self._dtype and g.device == self._device
+                    and g.layout is torch.strided and g.is_contiguous()
+                    and g.data_ptr() % 16 == 0):
+                u.grad_full = g.detach().view(-1)
+                u.grad_seen = [True]
+                param.grad = None
+            self._grad_buffer(u)
             if param.grad is not None:
                 g = param.grad.detach().reshape(-1)
                 dst = u.grad_full[off:off + param.ds_numel]
@@ -849,7 +865,8 @@ class ZeroStage3Optimizer:
     def _post_backward(self):
         # flush units whose grads partially arrived (unused params)
         for u in self.units:
-            if u.grad_full is not None and u.in_backward:
+            if u.in_backward:
+                self._grad_buffer(u)
                 self._reduce_unit(u)
         self._drain_inflight_rs(limit=0)
         self._flush_pending_releases()
@@ -882,8 +899,9 @@ class ZeroStage3Optimizer:
                     norm_sq = t.cpu()
             if self.mpu is not None:
                 dist.all_reduce(norm_sq, group=self.mpu.get_model_parallel_group())
-        self.overflow = bool(norm_sq is not None and
-                             (torch.isinf(norm_sq) or torch.isnan(norm_sq)))
+        # one transfer: what follows is decided and scaled on the host
+        norm_sq = None if norm_sq is None else float(norm_sq)
+        self.overflow = norm_sq is not None and not math.isfinite(norm_sq)
         self.loss_scaler.update_scale(self.overflow)
         if self.overflow:
             log_dist(f"overflow detected, skipping step "
@@ -892,12 +910,11 @@ class ZeroStage3Optimizer:
             self.micro_step_id = 0
             return
 
-        global_norm = (norm_sq.sqrt() / scale) if norm_sq is not None else None
+        global_norm = math.sqrt(norm_sq) / scale if norm_sq is not None else 0.0
         combined_scale = scale
-        if self.clip_grad > 0 and global_norm is not None:
-            clip = (global_norm / self.clip_grad).clamp(min=1.0)
-            combined_scale = scale * clip
-        self._global_grad_norm = float(global_norm) if global_norm is not None else 0.0
+        if self.clip_grad > 0:
+            combined_scale = scale * max(1.0, global_norm / self.clip_grad)
+        self._global_grad_norm = global_norm
 
         stepped = wrote_params = False
         if self.nvme_offload:
