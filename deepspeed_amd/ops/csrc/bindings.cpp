@@ -99,6 +99,11 @@ extern "C" void ds_rows_linear(const void* x, int layers, const void* const* w,
                                const void* const* bias, void* const* out,
                                const int* n, int M,
                                int K, int group, int mode, void* stream);
+extern "C" int ds_batch_linear_splits(const int* n, int layers, int M, int K);
+extern "C" void ds_batch_linear(const void* x, int layers,
+                                const void* const* w, const void* const* bias,
+                                void* const* out, const int* n, int M, int K,
+                                int splits, float* part, void* stream);
 extern "C" void ds_transpose_bf16(const void* src, void* dst, int n_batch,
                                   int R, int C, long long row_stride,
                                   int inner, long long inner_stride,
@@ -437,9 +442,10 @@ at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
   return out;
 }
 
-// Linear layers on one input of a few rows (rows_linear.hip). weights: bf16
-// [N, K], or int8 (any shape, N * K long) with their groupwise scales.
-// mode 1 returns silu(layer 0) * layer 1.
+// Linear layers on one input of a few rows (rows_linear.hip), or of up to 256
+// with bf16 weights (batch_linear.hip). weights: bf16 [N, K], or int8 (any
+// shape, N * K long) with their groupwise scales. mode 1 returns
+// silu(layer 0) * layer 1.
 std::vector<at::Tensor> rows_linear(
     at::Tensor x, std::vector<at::Tensor> weights,
     std::vector<at::Tensor> scales,
@@ -449,8 +455,8 @@ std::vector<at::Tensor> rows_linear(
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
               x.is_contiguous() && x.dim() == 2, "rows_linear: x");
   const int64_t M = x.size(0), K = x.size(1);
-  TORCH_CHECK(M >= 1 && M <= (scales.empty() ? 32 : 64) && K > 0 && K % 256 == 0 && L >= 1 &&
-              L <= 3 && (mode == 0 || L == 2) &&
+  TORCH_CHECK(M >= 1 && M <= (scales.empty() ? 256 : 64) && K > 0 &&
+              K % 256 == 0 && L >= 1 && L <= 3 && (mode == 0 || L == 2) &&
               (scales.empty() || (int)scales.size() == L) &&
               (int)biases.size() == L, "rows_linear: shape");
   const bool i8 = !scales.empty();
@@ -488,6 +494,22 @@ std::vector<at::Tensor> rows_linear(
   }
   TORCH_CHECK(mode == 0 || n[0] == n[1], "rows_linear: gate and up");
   TORCH_CHECK(((uintptr_t)x.data_ptr() & 15) == 0, "rows_linear: alignment");
+  if (!i8 && M > 32) {
+    TORCH_CHECK(mode == 0, "rows_linear: no activation past 32 rows");
+    int64_t all = 0;
+    for (int i = 0; i < L; ++i) {
+      TORCH_CHECK(n[i] % 4 == 0, "rows_linear: features in fours");
+      all += n[i];
+    }
+    const int splits = ds_batch_linear_splits(n, L, (int)M, (int)K);
+    at::Tensor part;
+    if (splits > 1)
+      part = at::empty({splits * M * all}, x.options().dtype(at::kFloat));
+    ds_batch_linear(x.data_ptr(), L, w, b, o, n, (int)M, (int)K, splits,
+                    splits > 1 ? part.data_ptr<float>() : nullptr,
+                    cur_stream());
+    return out;
+  }
   ds_rows_linear(x.data_ptr(), L, w, i8 ? sc : nullptr, b, o, n, (int)M,
                  (int)K, (int)group, (int)mode, cur_stream());
   return out;

@@ -5,7 +5,9 @@ the contiguous axis (see ``_Linear``).
 
 ``rows_linear``, for a few rows (decoding): the weight-streaming kernel of
 csrc/rows_linear.hip in place of a library GEMM, with several layers of one
-input in one launch and the gate's activation in its epilogue.
+input in one launch and the gate's activation in its epilogue. For up to 256 rows
+(many requests, short prompts) the kernel of csrc/batch_linear.hip where
+``batch_pays``.
 
 It takes the modules themselves and returns None wherever calling them is the
 thing to do: with gradients, hooks, autocast, other types, sharded
@@ -17,9 +19,10 @@ from torch.nn.modules import module as _module
 
 from ._loader import get_ext
 
-# Most rows: at 64 the library's product takes half the kernel's time (N 14336:
-# 26.6 to 49.8 us); with int8 weights it needs them dequantized first (85 us).
-ROWS, ROWS_INT8 = 32, 64
+# Most rows for rows_linear.hip: at 64 the library's product takes half the
+# kernel's time (N 14336: 26.6 to 49.8 us); with int8 weights it needs them
+# dequantized first. Past them, up to BATCH, batch_linear.hip where it pays.
+ROWS, ROWS_INT8, BATCH = 32, 64, 256
 
 PLAIN, SWIGLU = 0, 1
 
@@ -131,6 +134,26 @@ def unhooked(mod: nn.Module, internal_ok: bool = False) -> bool:
                 or _module._global_backward_pre_hooks)
 
 
+def batch_pays(ns, K: int) -> bool:
+    """Whether batch_linear.hip takes layers of ``ns`` features on one input, of
+    33 to 256 rows. Several layers: one launch that fills the chip in place of
+    products that leave it idle (us, library and kernel, at 64 and 224 rows:
+    4096 + 1024 + 1024, K 4096 44 / 21 and 47 / 36; 3 x 3072, K 3072 48 / 23 and
+    53 / 44; 3 x 5120, K 5120 65 / 43, 150 / 77 at 256; 8192 + 1024 + 1024, K
+    8192 60 / 41 and 111 / 98). One layer: where
+    the contraction is long and the library's product splits it badly (4096, K
+    14336 39 / 33, 60 / 59, 76 / 43 at 128; 3072, K 8192 24 / 21, 33 / 34, 43 /
+    27 at 128; 8192, K 28672 134 / 103, 257 / 198). The library is ahead where
+    its tiles fill the chip (14336 + 14336, K 4096 54 / 61, 91 / 98) and at
+    small or square layers (4096, K 4096 15 / 17, 23 / 25; 2048, K 4096 11 / 15,
+    16 / 21)."""
+    if any(n % 4 for n in ns):
+        return False
+    if len(ns) > 1:
+        return sum(ns) <= 16384
+    return K >= 2 * ns[0] and ns[0] * K >= 1 << 24
+
+
 def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
                 hooks_ran: bool = False):
     """Outputs of the linear modules ``mods`` on x [..., K], a list: one each,
@@ -141,7 +164,7 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
         return None
     K = x.shape[-1]
     M = x.numel() // K if K else 0
-    if not 1 <= M <= ROWS_INT8 or K % 256 or get_ext() is None or \
+    if not 1 <= M <= BATCH or K % 256 or get_ext() is None or \
             torch.is_autocast_enabled() or torch.compiler.is_compiling():
         return None
     from ..linear.optimized_linear import WOQLinear
@@ -152,13 +175,13 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
             return None
         if kind is Linear or kind is nn.Linear:
             w = m.weight
-            if M > ROWS or w.dtype is not torch.bfloat16 or \
+            if w.dtype is not torch.bfloat16 or \
                     type(w) is not nn.Parameter or w.shape[1:] != (K,):
                 return None
         elif kind is WOQLinear:
             p = m.qweight
             w, group = p.q, p.cfg.group_size
-            if p.cfg.q_bits != 8 or group % 256 or \
+            if M > ROWS_INT8 or p.cfg.q_bits != 8 or group % 256 or \
                     group != mods[0].qweight.cfg.group_size or \
                     p.shape[1:] != (K,) or \
                     w.numel() != p.shape[0] * K or not unhooked(p):
@@ -173,6 +196,9 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
             return None
         weights.append(w)
         biases.append(b)
+    if M > ROWS and not scales and (mode != PLAIN or not batch_pays(
+            [w.shape[0] for w in weights], K)):
+        return None
     x2 = x.reshape(M, K).contiguous()
     if x2.data_ptr() % 16:
         return None

@@ -7,7 +7,8 @@ import torch.nn as nn
 
 from deepspeed_amd.linear.optimized_linear import (QuantizationConfig,
                                                    WOQLinear)
-from deepspeed_amd.ops.linear import SWIGLU, rows_linear, unhooked
+from deepspeed_amd.ops.linear import (SWIGLU, batch_pays, rows_linear,
+                                      unhooked)
 
 
 def test_unhooked():
@@ -69,7 +70,7 @@ def test_rows_linear_gpu(int8, m, sizes):
     both = [_layer(n, k, i % 2 == 0, int8, g) for i, n in enumerate(ns)]
     x = torch.randn(1, m, k, generator=g).bfloat16().cuda()
     got = rows_linear(x, [b[0] for b in both])
-    if m > (64 if int8 else 32):
+    if m > 64 if int8 else m > 32 and not batch_pays(ns, k):
         assert got is None
         return
     for (lin, want), y in zip(both, got):
@@ -80,6 +81,35 @@ def test_rows_linear_gpu(int8, m, sizes):
     h = both[0][0].register_forward_hook(lambda *a: None)
     assert rows_linear(x, (both[0][0],)) is None
     h.remove()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [33, 48, 49, 64, 65, 80, 96, 112, 127, 128, 129,
+                               200, 225, 256, 257])
+@pytest.mark.parametrize("sizes", [((4, 132, 124), 256), ((100, 36), 512),
+                                   ((1024, 256, 256), 1280),
+                                   ((128,), 131072)])
+@torch.no_grad()
+def test_batch_linear_gpu(m, sizes):
+    ns, k = sizes
+    g = torch.Generator().manual_seed(m)
+    both = [_layer(n, k, i % 2 == 0, False, g) for i, n in enumerate(ns)]
+    x = torch.randn(m, k, generator=g).bfloat16().cuda()
+    got = rows_linear(x, [b[0] for b in both])
+    if m > 256:
+        assert got is None
+        return
+    for (lin, want), y in zip(both, got):
+        _close(y, want(x))
+    assert rows_linear(x, [both[0][0]] * 2, SWIGLU) is None
+
+
+def test_batch_rule():
+    assert batch_pays((4096, 1024, 1024), 4096)
+    assert batch_pays((4096,), 14336)
+    assert not batch_pays((4096,), 4096)
+    assert not batch_pays((14336, 14336), 4096)
+    assert not batch_pays((4096, 1022), 4096)
 
 
 @pytest.mark.gpu
