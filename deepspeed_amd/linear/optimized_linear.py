@@ -14,6 +14,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
+from ..ops.linear import movable, rows_linear
 from ..ops.quantizer import dequantize, quantize
 
 
@@ -48,6 +49,7 @@ class QuantizedParameter(nn.Module):
                           self.dtype).view(self.shape)
 
 
+@movable
 class WOQLinear(nn.Module):
     """Inference linear on a quantized weight (weight-only quantization): few
     rows read the int8 weight as it is, many have it dequantized first."""
@@ -58,7 +60,6 @@ class WOQLinear(nn.Module):
         self.bias = lin.bias
 
     def forward(self, x):
-        from ..ops.linear import rows_linear
         y = rows_linear(x, (self,), hooks_ran=True)
         if y is not None:
             return y[0]

@@ -18,7 +18,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ..ops.attention import rope_flash_attention
-from ..ops.linear import SWIGLU, Linear, rows_linear, unhooked
+from ..ops.linear import SWIGLU, Linear, movable, rows_linear, unhooked
 from ..ops.norms import RMSNorm
 from ..ops.rope import apply_rope, rope_tables
 from ..ops.swiglu import swiglu
@@ -252,7 +252,7 @@ class LlamaMLP(nn.Module):
 
 def add_norm(norm, x, delta):
     """(norm of the residual stream x with a sublayer's output added, the new
-    stream); one kernel where nothing watches or replaces the norm."""
+    stream); one kernel where nothing watches or replaces the norm's call."""
     if delta is None:
         return norm(x), x
     if type(norm) is RMSNorm and unhooked(norm, internal_ok=True):
@@ -261,6 +261,7 @@ def add_norm(norm, x, delta):
     return norm(x), x
 
 
+@movable
 class LlamaDecoderLayer(nn.Module):
     def __init__(self, cfg: LlamaConfig, layer_idx: int):
         super().__init__()

@@ -104,6 +104,18 @@ def _plain_autograd() -> bool:
             and not torch.jit.is_tracing())
 
 
+# The forward that each class had when its work was given another way round it.
+_TORCHS = nn.Linear.forward
+_FORWARD = {nn.Linear: _TORCHS}
+
+
+def movable(cls):
+    """Class decorator: ``unhooked`` may say yes to modules of this class."""
+    _FORWARD[cls] = cls.forward
+    return cls
+
+
+@movable
 class Linear(nn.Linear):
     """nn.Linear with the backward of ``_Linear`` on a GPU."""
 
@@ -115,15 +127,22 @@ class Linear(nn.Linear):
                 and w.is_contiguous() and w.dim() == 2
                 and x.numel() and x.shape[-1] == w.shape[1]
                 and any(backward_plan(x.numel() // w.shape[1], *w.shape))
-                and get_ext() is not None and _plain_autograd()):
+                and get_ext() is not None and _plain_autograd()
+                and nn.Linear.forward is _TORCHS):
             return _Linear.apply(x, w, self.bias)
-        return nn.functional.linear(x, w, self.bias)
+        return super().forward(x)
 
 
 def unhooked(mod: nn.Module, internal_ok: bool = False) -> bool:
-    """No hook sees the module's call: its work may move elsewhere. With
-    ``internal_ok`` the call itself stays, in another form that the
-    framework's own hooks (marked ``_ds_internal``) take as well."""
+    """No hook sees the module's call and no other forward takes it (one set on
+    the module or on its class, or a compiled one): its work may move
+    elsewhere. With ``internal_ok`` the call itself stays, in another form that
+    the framework's own hooks (marked ``_ds_internal``) take as well."""
+    cls = type(mod)
+    if "forward" in mod.__dict__ or mod._compiled_call_impl is not None or \
+            cls.forward is not _FORWARD.get(cls) or \
+            nn.Linear.forward is not _TORCHS:
+        return False
     own = (mod._forward_hooks, mod._forward_pre_hooks, mod._backward_hooks,
            mod._backward_pre_hooks)
     return not (any(not (internal_ok and getattr(h, "_ds_internal", False))
@@ -167,7 +186,7 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
     if not 1 <= M <= BATCH or K % 256 or get_ext() is None or \
             torch.is_autocast_enabled() or torch.compiler.is_compiling():
         return None
-    from ..linear.optimized_linear import WOQLinear
+    from ..linear.optimized_linear import QuantizedParameter, WOQLinear
     kind = type(mods[0])
     weights, scales, biases, group = [], [], [], 0
     for m in mods:
@@ -181,10 +200,13 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
         elif kind is WOQLinear:
             p = m.qweight
             w, group = p.q, p.cfg.group_size
+            if type(p) is not QuantizedParameter or \
+                    "dequantized" in p.__dict__:
+                return None
             if M > ROWS_INT8 or p.cfg.q_bits != 8 or group % 256 or \
                     group != mods[0].qweight.cfg.group_size or \
                     p.shape[1:] != (K,) or \
-                    w.numel() != p.shape[0] * K or not unhooked(p):
+                    w.numel() != p.shape[0] * K:
                 return None
             scales.append(p.scales)
         else:

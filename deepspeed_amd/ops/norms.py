@@ -8,6 +8,7 @@ matching torch implementation (fp32 math internally, like the kernels).
 import torch
 
 from ._loader import get_ext
+from .linear import movable
 
 
 class _RMSNormFn(torch.autograd.Function):
@@ -140,6 +141,7 @@ def layer_norm(x, weight, bias=None, eps=1e-5):
     return _LayerNormFn.apply(x, weight, bias, eps)
 
 
+@movable
 class RMSNorm(torch.nn.Module):
     def __init__(self, hidden_size, eps=1e-6, dtype=None, device=None):
         super().__init__()

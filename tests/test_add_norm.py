@@ -41,6 +41,59 @@ def test_hooked_or_replaced_layers_see_their_calls():
     assert torch.equal(model(ids, labels=ids), want)
 
 
+@pytest.mark.parametrize("where", ["module", "class"])
+@pytest.mark.parametrize("grad", [False, True])
+def test_replaced_forwards_are_taken(where, grad, monkeypatch):
+    """A forward set on a layer, a norm or a projection, or on its class."""
+    torch.manual_seed(0)
+    model = llama.LlamaForCausalLM(llama.llama_tiny())
+    ids = torch.randint(0, 512, (2, 9))
+    layer = model.model.layers[1]
+    for mod in (layer, layer.input_layernorm, model.model.norm,
+                layer.self_attn.q_proj, layer.mlp.down_proj, model.lm_head):
+        with monkeypatch.context() as m, torch.set_grad_enabled(grad):
+            want, calls = model(ids), []
+            old = type(mod).forward
+
+            def forward(self, x, *a, **k):
+                calls.append(0)
+                assert not k.keys() - {"positions", "kv_cache"}
+                y = old(self, x, *a, **k)
+                return 2 * y if self is mod else y
+
+            if where == "class":
+                m.setattr(type(mod), "forward", forward)
+            else:
+                m.setitem(mod.__dict__, "forward", forward.__get__(mod))
+            assert not unhooked(mod) and not unhooked(mod, internal_ok=True)
+            got = model(ids)
+            assert calls and not torch.equal(got, want)
+        assert unhooked(mod)
+
+
+def test_torchs_linear_replaced(monkeypatch):
+    model = llama.LlamaForCausalLM(llama.llama_tiny())
+    lin = model.lm_head
+    monkeypatch.setattr(torch.nn.Linear, "forward", lambda self, x: x)
+    assert not unhooked(lin)
+    x = torch.randn(2, 64)
+    assert lin(x) is x
+
+
+@pytest.mark.parametrize("name", ["", ".input_layernorm", ".mlp.up_proj"])
+def test_compiled_modules_run_compiled(name):
+    torch.manual_seed(0)
+    model = llama.LlamaForCausalLM(llama.llama_tiny())
+    ids = torch.randint(0, 512, (2, 9))
+    want = model(ids)
+    mod = model.get_submodule("model.layers.0" + name)
+    graphs = []
+    mod.compile(backend=lambda g, _: graphs.append(g) or g.forward)
+    assert not unhooked(mod)
+    torch.testing.assert_close(model(ids), want)
+    assert graphs
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,h", [(1, 8), (3, 2040), (7, 2048), (1030, 4096),

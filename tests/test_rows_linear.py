@@ -128,6 +128,24 @@ def test_rows_swiglu_gpu(int8, m):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("int8", [False, True])
+@torch.no_grad()
+def test_replaced_forward_gpu(int8):
+    lin, _ = _layer(64, 256, False, int8, torch.Generator().manual_seed(0))
+    x = torch.randn(2, 256, device="cuda").bfloat16()
+    want = rows_linear(x, (lin,))[0]
+    lin.forward = lambda x: 0 * x
+    assert rows_linear(x, (lin,)) is None
+    del lin.forward
+    assert torch.equal(rows_linear(x, (lin,))[0], want)
+    if int8:
+        w = 2 * lin.qweight.dequantized()
+        lin.qweight.dequantized = lambda: w
+        assert rows_linear(x, (lin,)) is None
+        _close(lin(x), x.double() @ w.double().t())
+
+
+@pytest.mark.gpu
 @torch.no_grad()
 def test_model_with_and_without_rows_linear(monkeypatch):
     """A decoding step's logits by either way, through a whole model."""
