@@ -934,6 +934,9 @@ class AioHandle {
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  pybind11::class_<ShmComm>(m, "ShmComm")
+      .def(pybind11::init<const std::string&, int64_t, int64_t, int64_t>())
+      .def("all_reduce", &ShmComm::all_reduce);
   m.def("paged_decode", &paged_decode,
         "split-KV decode attention over a paged KV block table");
   m.def("rows_linear", &rows_linear,
