@@ -21,6 +21,8 @@ from typing import Dict, List, Optional
 
 import torch
 
+from ..ops.linear import untransformed
+
 
 class RaggedKVCache:
     """Slot-pooled KV: [slots, Hkv, max_seq, D] per layer + per-slot
@@ -547,7 +549,8 @@ class PagedKVCache:
         causal attention over the paged pool. None when ineligible (the caller
         rotates and takes ``decode_attention`` or ``update``)."""
         if not self._eligible(layer_idx, q, k, v) or (
-                torch.is_grad_enabled() and q.requires_grad):
+                torch.is_grad_enabled() and q.requires_grad) or \
+                not untransformed():
             return None
         if positions is not None and (
                 positions.dtype != torch.int32 or not positions.is_cuda

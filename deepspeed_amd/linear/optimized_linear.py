@@ -59,6 +59,16 @@ class WOQLinear(nn.Module):
         self.qweight = QuantizedParameter(lin.weight.data, cfg)
         self.bias = lin.bias
 
+    def int8_rows(self, K: int):
+        """(int8 weight, scales, group size) of a weight [N, K] as it was
+        quantized; None where it is another."""
+        p = self.qweight
+        if type(p) is not QuantizedParameter or "dequantized" in p.__dict__ \
+                or p.cfg.q_bits != 8 or p.shape[1:] != (K,) or \
+                p.q.numel() != p.shape[0] * K:
+            return None
+        return p.q, p.scales, p.cfg.group_size
+
     def forward(self, x):
         y = rows_linear(x, (self,), hooks_ran=True)
         if y is not None:

@@ -9,6 +9,7 @@ from typing import Optional
 import torch
 
 from ._loader import get_ext
+from .linear import _plain_autograd, untransformed
 
 
 def _eligible(q: torch.Tensor, k: torch.Tensor) -> bool:
@@ -32,7 +33,6 @@ def flash_train_available(q: torch.Tensor, k: torch.Tensor) -> bool:
     opts out."""
     if os.environ.get("DS_AMD_FLASH_TRAIN", "1") == "0":
         return False
-    from .linear import _plain_autograd
     return _eligible(q, k) and _plain_autograd()
 
 
@@ -160,7 +160,7 @@ def rope_flash_attention(q, k, v, cos, sin, positions=None):
     the kernels do not apply."""
     grad = torch.is_grad_enabled()
     if not (flash_train_available(q, k) if grad else
-            flash_attn_available(q, k)) or (
+            flash_attn_available(q, k) and untransformed()) or (
             positions is None and cos.size(0) < q.size(1)) or (
             positions is not None and positions.dtype != torch.int32):
         return None

@@ -10,11 +10,12 @@ input in one launch and the gate's activation in its epilogue. For up to 256 row
 ``batch_pays``.
 
 It takes the modules themselves and returns None wherever calling them is the
-thing to do: with gradients, hooks, autocast, other types, sharded
-or replaced modules, or more rows than the kernel is the faster one for."""
+thing to do: with gradients, hooks, autocast, function transforms, tangents or
+traces, other types, sharded or replaced modules, or more rows than the kernel is the faster one for."""
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
 
 from ._loader import get_ext
@@ -94,14 +95,23 @@ def _transposed(a: torch.Tensor) -> torch.Tensor:
     return get_ext().transpose_2d(a.contiguous())
 
 
+_interpreter = torch._C._functorch.peek_interpreter_stack
+_modes = torch._C._len_torch_dispatch_stack
+_trace = torch._C._get_tracing_state
+
+
+def untransformed() -> bool:
+    """No function transform, tangent, trace or dispatch mode is about: these
+    see torch's own operations, and a kernel called directly passes them by."""
+    return (_interpreter() is None and forward_ad._current_level < 0
+            and _modes() == 0 and _trace() is None)
+
+
 def _plain_autograd() -> bool:
-    """No transform or tangent is about that an autograd function without
-    rules of its own would stop."""
-    return (torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0
-            and not torch.compiler.is_compiling()
-            and not torch.is_autocast_enabled()
-            and not torch.jit.is_tracing())
+    """Neither one of these nor autocast or a compiler is about: an autograd
+    function without rules for them would stop them."""
+    return (untransformed() and not torch.compiler.is_compiling()
+            and not torch.is_autocast_enabled())
 
 
 # The forward that each class had when its work was given another way round it.
@@ -178,15 +188,15 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
     """Outputs of the linear modules ``mods`` on x [..., K], a list: one each,
     or with ``SWIGLU`` silu(first) * second. ``hooks_ran``: called from inside
     the module's own call. None when ineligible."""
-    if torch.is_grad_enabled() or not x.is_cuda or \
-            x.dtype is not torch.bfloat16 or type(x) is not torch.Tensor:
+    if type(x) is not torch.Tensor or torch.is_grad_enabled() or \
+            not x.is_cuda or x.dtype is not torch.bfloat16:
         return None
     K = x.shape[-1]
     M = x.numel() // K if K else 0
     if not 1 <= M <= BATCH or K % 256 or get_ext() is None or \
-            torch.is_autocast_enabled() or torch.compiler.is_compiling():
+            torch.is_autocast_enabled() or torch.compiler.is_compiling() or \
+            not untransformed():
         return None
-    from ..linear.optimized_linear import QuantizedParameter, WOQLinear
     kind = type(mods[0])
     weights, scales, biases, group = [], [], [], 0
     for m in mods:
@@ -197,18 +207,12 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
             if w.dtype is not torch.bfloat16 or \
                     type(w) is not nn.Parameter or w.shape[1:] != (K,):
                 return None
-        elif kind is WOQLinear:
-            p = m.qweight
-            w, group = p.q, p.cfg.group_size
-            if type(p) is not QuantizedParameter or \
-                    "dequantized" in p.__dict__:
+        elif hasattr(kind, "int8_rows"):
+            p = m.int8_rows(K) if M <= ROWS_INT8 else None
+            if p is None or p[2] % 256 or group not in (0, p[2]):
                 return None
-            if M > ROWS_INT8 or p.cfg.q_bits != 8 or group % 256 or \
-                    group != mods[0].qweight.cfg.group_size or \
-                    p.shape[1:] != (K,) or \
-                    w.numel() != p.shape[0] * K:
-                return None
-            scales.append(p.scales)
+            w, scale, group = p
+            scales.append(scale)
         else:
             return None
         b = m.bias

@@ -8,7 +8,7 @@ import torch.nn as nn
 from deepspeed_amd.linear.optimized_linear import (QuantizationConfig,
                                                    WOQLinear)
 from deepspeed_amd.ops.linear import (SWIGLU, batch_pays, rows_linear,
-                                      unhooked)
+                                      unhooked, untransformed)
 
 
 def test_unhooked():
@@ -33,6 +33,42 @@ def test_cpu_and_grad_calls_are_left_alone():
     with torch.no_grad():
         assert rows_linear(x, (lin,)) is None
     assert rows_linear(x, (lin,)) is None
+
+
+def _under_transforms(f, x):
+    """f(x) as transforms, tangents, a trace and a dispatch mode make the
+    call, by name."""
+    import torch.autograd.forward_ad as fwad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+    out = {"vmap": torch.func.vmap(f)(x),
+           "jvp": torch.func.jvp(f, (x,), (2 * x,))[1]}
+    with fwad.dual_level():
+        out["dual"] = fwad.unpack_dual(f(fwad.make_dual(x, 2 * x))).tangent
+    with FlopCounterMode(display=False) as mode:
+        f(x)
+    out["flops"] = mode.get_total_flops()
+    # traced on one input, run on another
+    out["make_fx"] = make_fx(f)(x)(3 * x)
+    out["trace"] = torch.jit.trace(f, x, check_trace=False)(3 * x)
+    return out
+
+
+def test_untransformed():
+    seen = []
+
+    def f(x):
+        seen.append(untransformed())
+        return x @ x.t()
+
+    f(torch.ones(2, 2))
+    assert seen == [True]
+    seen.clear()
+    with torch.no_grad():
+        assert untransformed()
+        _under_transforms(f, torch.ones(2, 2, 2)[0])
+    assert len(seen) >= 6 and not any(seen)
+    assert untransformed()
 
 
 def _layer(n, k, bias, int8, g):
@@ -125,6 +161,22 @@ def test_rows_swiglu_gpu(int8, m):
     x = torch.randn(m, 512, generator=g).bfloat16().cuda()
     y, = rows_linear(x, (gate, up), SWIGLU)
     _close(y, torch.nn.functional.silu(fg(x)) * fu(x))
+
+
+@pytest.mark.gpu
+@torch.no_grad()
+def test_quantized_linear_under_transforms_gpu():
+    """A quantized layer, which takes the kernel by itself, under each."""
+    lin, want = _layer(64, 256, False, True, torch.Generator().manual_seed(0))
+    x = torch.randn(4, 256, device="cuda").bfloat16()
+    assert rows_linear(x, (lin,)) is not None
+    got = _under_transforms(lin, x)
+    assert got.pop("flops") == 2 * 4 * 64 * 256
+    for name, scale in (("vmap", 1), ("jvp", 2), ("dual", 2), ("make_fx", 3),
+                        ("trace", 3)):
+        err = got[name].double() - scale * want(x)
+        # weights rounded to bf16 on this way round, and inputs 3 * x
+        assert err.norm() <= 0.01 * scale * want(x).norm(), name
 
 
 @pytest.mark.gpu
