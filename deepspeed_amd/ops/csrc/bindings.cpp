@@ -3,6 +3,7 @@
 // Uses torch-ROCm's native HIP stream API (c10::hip) — no CUDA shims.
 
 #include <torch/extension.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
 #include <tuple>
@@ -163,6 +164,27 @@ void* cur_stream() {
   return reinterpret_cast<void*>(c10::hip::getCurrentHIPStream().stream());
 }
 
+// A call's tensors lie on one device, the first's, and its kernels run there,
+// whichever device is the current one. Pointers of another device are no error
+// to a kernel: it faults on them or reads what is not its own.
+struct OneDevice {
+  const char* what;
+  const c10::Device device;
+  const c10::DeviceGuard guard;
+  template <typename... Ts>
+  OneDevice(const char* what_, const at::Tensor& first, const Ts&... more)
+      : what(what_), device(first.device()), guard(device) {
+    (check(more), ...);
+  }
+  void check(const at::Tensor& t) const {
+    TORCH_CHECK(t.device() == device, what, ": tensors on different devices, ",
+                device, " and ", t.device());
+  }
+  void check(const c10::optional<at::Tensor>& t) const {
+    if (t.has_value() && t->defined()) check(*t);
+  }
+};
+
 void fused_adam_flat(at::Tensor p, at::Tensor g, at::Tensor m, at::Tensor v,
                      c10::optional<at::Tensor> p16, double lr, double beta1,
                      double beta2, double eps, double weight_decay,
@@ -265,6 +287,7 @@ at::Tensor transpose_bf16(at::Tensor src, int64_t n_batch, int64_t R,
 // x [R, C] bf16 -> its transpose [C, R], whose rows start on 16 bytes (their
 // stride is R rounded up to 8).
 at::Tensor transpose_2d(at::Tensor x) {
+  const OneDevice on("transpose_2d", x);
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
               x.dim() == 2 && x.is_contiguous(), "transpose_2d: bf16 matrix");
   const int64_t R = x.size(0), C = x.size(1), ld = (R + 7) / 8 * 8;
@@ -344,6 +367,7 @@ static void check_pool(const at::Tensor& q, const at::Tensor& kpool,
 at::Tensor paged_decode(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
                         at::Tensor block_table, at::Tensor lens,
                         int64_t splits, double scale) {
+  const OneDevice on("paged_decode", q, kpool, vpool, block_table, lens);
   check_pool(q, kpool, vpool, "paged_decode");
   const int n = q.size(0), H = q.size(1);
   const int Hkv = kpool.size(1), BS = kpool.size(2);
@@ -376,6 +400,7 @@ at::Tensor paged_rows(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
                       at::Tensor meta, int64_t n_items, int64_t n_runs,
                       int64_t n_merges, bool any_merge, int64_t nq,
                       double scale) {
+  const OneDevice on("paged_rows", q, kpool, vpool, meta);
   check_pool(q, kpool, vpool, "paged_rows");
   TORCH_CHECK(meta.scalar_type() == at::kInt && meta.is_cuda() &&
               meta.is_contiguous() &&
@@ -405,6 +430,8 @@ at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
                         c10::optional<at::Tensor> cos_table,
                         c10::optional<at::Tensor> sin_table,
                         c10::optional<at::Tensor> positions, int64_t S) {
+  const OneDevice on("paged_append", q, k, v, kpool, vpool, dst, cos_table,
+                     sin_table, positions);
   check_pool(q, kpool, vpool, "paged_append");
   const int T = q.size(0), H = q.size(1), Hkv = kpool.size(1);
   for (auto& x : {k, v})
@@ -451,6 +478,10 @@ std::vector<at::Tensor> rows_linear(
     std::vector<at::Tensor> scales,
     std::vector<c10::optional<at::Tensor>> biases, int64_t group,
     int64_t mode) {
+  const OneDevice on("rows_linear", x);
+  for (auto& t : weights) on.check(t);
+  for (auto& t : scales) on.check(t);
+  for (auto& t : biases) on.check(t);
   const int L = weights.size();
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
               x.is_contiguous() && x.dim() == 2, "rows_linear: x");
@@ -517,6 +548,7 @@ std::vector<at::Tensor> rows_linear(
 
 at::Tensor sum_of_squares(std::vector<at::Tensor> ts) {
   TORCH_CHECK(!ts.empty(), "sum_of_squares: no tensors");
+  const OneDevice on("sum_of_squares", ts[0]);
   std::vector<const void*> p;
   std::vector<long long> n;
   for (auto& t : ts) {
@@ -611,6 +643,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_bwd(
     at::Tensor dy, at::Tensor x, at::Tensor w, at::Tensor invrms,
     c10::optional<at::Tensor> mean, bool layernorm,
     c10::optional<at::Tensor> dres) {
+  const OneDevice on("norm_bwd", x, dy, w, invrms, mean, dres);
   TORCH_CHECK(dy.is_contiguous() && x.is_contiguous() && w.is_contiguous(),
               "must be contiguous");
   const int64_t H = x.size(-1);
@@ -647,6 +680,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_bwd(
 // (ops/norms.py, add_norm_eligible).
 std::tuple<at::Tensor, at::Tensor, at::Tensor> add_norm_fwd(
     at::Tensor x, at::Tensor res, at::Tensor w, double eps) {
+  const OneDevice on("add_norm_fwd", x, res, w);
   const int64_t H = x.size(-1);
   for (auto& t : {x, res})
     TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
@@ -739,6 +773,7 @@ std::vector<at::Tensor> rope(at::Tensor x, c10::optional<at::Tensor> x2,
                              at::Tensor cos_table, at::Tensor sin_table,
                              c10::optional<at::Tensor> positions,
                              bool backward, bool inplace) {
+  const OneDevice on("rope", x, x2, cos_table, sin_table, positions);
   TORCH_CHECK(x.dim() == 4 && x.is_contiguous() && x.is_cuda(),
               "rope expects [B,S,H,D]");
   for (auto& t : {cos_table, sin_table})
@@ -855,6 +890,7 @@ struct FlashArgs {
 std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
     at::Tensor q, at::Tensor k, at::Tensor v, double scale, bool causal,
     bool with_lse) {
+  const OneDevice on("flash_attn_fwd", q, k, v);
   FlashArgs a(q, k, v, scale);
   auto o = at::empty({a.B, a.S, a.H, a.D}, q.options());
   auto lse = at::empty({with_lse ? a.B : 0, a.H, a.S},
@@ -871,6 +907,7 @@ std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(
 std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(
     at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor o, at::Tensor dout,
     at::Tensor lse, double scale, bool causal, int64_t splits) {
+  const OneDevice on("flash_attn_bwd", q, k, v, o, dout, lse);
   FlashArgs a(q, k, v, scale);
   if (splits == 0) splits = ds_flash_bwd_splits(a.B, a.S, a.H, a.Hkv);
   TORCH_CHECK(splits >= 1 && splits <= a.H / a.Hkv, "flash_bwd: splits");
