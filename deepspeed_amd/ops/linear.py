@@ -59,20 +59,23 @@ class _Linear(torch.autograd.Function):
     """x W^T + b whose backward lays operands out for the matrix product:
     dx = dy W reads W across its rows, and dW = dy^T x reads both across
     theirs, at two thirds of the forward product's rate. Transposing costs a
-    read and a write of an operand and pays where ``backward_plan`` says."""
+    read and a write of an operand and pays where ``backward_plan`` says. Kept
+    for the backward is what it needs: a frozen layer holds no input."""
 
     @staticmethod
     def forward(ctx, x, weight, bias):
-        ctx.save_for_backward(x, weight)
+        need_x, need_w, _ = ctx.needs_input_grad
+        ctx.save_for_backward(x if need_w else None, weight if need_x else None)
+        ctx.shape, ctx.features = x.shape, weight.shape
         return nn.functional.linear(x, weight, bias)
 
     @staticmethod
     def backward(ctx, dy):
         x, weight = ctx.saved_tensors
         need_x, need_w, need_b = ctx.needs_input_grad
-        N, K = weight.shape
-        dy2, x2 = dy.reshape(-1, N), x.reshape(-1, K)
-        T = x2.shape[0]
+        N, K = ctx.features
+        dy2 = dy.reshape(-1, N)
+        T = dy2.shape[0]
         w_t = dy_t = x_t = False
         # differentiable products where the gradient itself is differentiated
         if not torch.is_grad_enabled() and dy.dtype is torch.bfloat16:
@@ -81,8 +84,9 @@ class _Linear(torch.autograd.Function):
         if need_x:
             dx = nn.functional.linear(dy2, _transposed(weight)) if w_t \
                 else dy2 @ weight
-            dx = dx.view(x.shape)
+            dx = dx.view(ctx.shape)
         if need_w:
+            x2 = x.reshape(-1, K)
             a = _transposed(dy2) if dy_t else dy2.t()
             b = _transposed(x2).t() if x_t else x2
             dw = a @ b

@@ -33,6 +33,27 @@ def test_is_torchs_linear_elsewhere():
     assert torch.equal(ja, jb)
 
 
+@pytest.mark.parametrize("frozen", ["weight", "input", "bias", None])
+def test_saves_what_the_backward_needs(frozen):
+    """As torch's layer does: a frozen weight holds no input (adapters over a
+    frozen model), an input without gradient no weight."""
+    torch.manual_seed(0)
+    t = {"input": torch.randn(2, 3, 6), "weight": torch.randn(5, 6),
+         "bias": torch.randn(5)}
+    grads, kept = [], []
+    for f in (L._Linear.apply, nn.functional.linear):
+        x, w, b = (t[n].clone().requires_grad_(n != frozen) for n in t)
+        seen = []
+        with torch.autograd.graph.saved_tensors_hooks(
+                lambda s: seen.append(s.numel()) or s, lambda s: s):
+            f(x, w, b).sum().backward()
+        grads.append([x.grad, w.grad, b.grad])
+        kept.append(sorted(seen))
+    assert kept[0] == kept[1]
+    for a, b in zip(*grads):
+        assert a is b is None or torch.equal(a, b)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("r,c", [(1, 1), (8, 64), (127, 63), (128, 64),
                                  (129, 72), (1000, 264), (4000, 3072),
