@@ -548,9 +548,9 @@ class PagedKVCache:
         positions int32 [n, S] or each row's index in S), cache write and
         causal attention over the paged pool. None when ineligible (the caller
         rotates and takes ``decode_attention`` or ``update``)."""
-        if not self._eligible(layer_idx, q, k, v) or (
-                torch.is_grad_enabled() and q.requires_grad) or \
-                not untransformed():
+        if not self._eligible(layer_idx, q, k, v) or not untransformed() or (
+                torch.is_grad_enabled()
+                and any(x.requires_grad for x in (q, k, v))):
             return None
         if positions is not None and (
                 positions.dtype != torch.int32 or not positions.is_cuda

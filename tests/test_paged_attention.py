@@ -71,6 +71,22 @@ def test_step_plan_covers_every_key_once(name, bs, heads):
     assert plan.items == merges[:, 1].sum()
 
 
+@pytest.mark.parametrize("which", [0, 1, 2, None])
+def test_rope_attention_leaves_gradients_alone(which, monkeypatch):
+    """With a gradient for queries, keys or values the caller's own path, which
+    has one, is taken."""
+    cache = PagedKVCache(1, 1, 2, 64, 128)
+    monkeypatch.setattr(cache, "_eligible", lambda *a: True)
+    monkeypatch.setattr(cache, "_attend", lambda *a: "kernels")
+    qkv = [torch.zeros(1, 3, h, 128) for h in (4, 2, 2)]
+    if which is not None:
+        qkv[which].requires_grad_()
+    want = None if which is not None else "kernels"
+    assert cache.rope_attention(0, *qkv, None, None) == want
+    with torch.no_grad():
+        assert cache.rope_attention(0, *qkv, None, None) == "kernels"
+
+
 def _reference(q, k, v, pos, scale):
     """q [m, H, D] at positions ``pos`` over k, v [L, Hkv, D], in fp64."""
     G = q.shape[1] // k.shape[1]
