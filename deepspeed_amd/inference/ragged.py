@@ -517,8 +517,9 @@ class PagedKVCache:
 
     def _eligible(self, layer_idx: int, q, k, v) -> bool:
         from ..ops.paged_attention import paged_decode_available
-        kp = self.k[layer_idx]
+        kp, vp = self.k[layer_idx], self.v[layer_idx]
         return (q.is_cuda and kp.is_cuda and kp.dtype == torch.bfloat16
+                and (kp.data_ptr() | vp.data_ptr()) % 16 == 0
                 and k.dtype == v.dtype == torch.bfloat16
                 and paged_decode_available(
                     q.reshape(-1, q.size(-2), q.size(-1)), kp))
@@ -527,7 +528,7 @@ class PagedKVCache:
                 positions=None, scale=None):
         """New rows into the pool, then attention over it: three launches (two
         where no history is split) for the whole step."""
-        from ..ops.paged_attention import (StepPlan, paged_append,
+        from ..ops.paged_attention import (StepPlan, aligned, paged_append,
                                            paged_attention)
         kp, vp = self.k[layer_idx], self.v[layer_idx]
         n, S, H, D = q.shape
@@ -536,7 +537,7 @@ class PagedKVCache:
             plan = self._plans[H, kp.size(1)] = StepPlan.build(
                 *self._row_places(), self.block_table, self.block_size, H,
                 kp.size(1), kp.device)
-        q, k, v = (x.reshape(n * S, -1, D).contiguous() for x in (q, k, v))
+        q, k, v = (aligned(x.reshape(n * S, -1, D)) for x in (q, k, v))
         q = paged_append(plan, q, k, v, kp, vp, cos, sin, positions, S)
         o = paged_attention(plan, q, kp, vp, scale)
         return o.view(n, S, H, D)

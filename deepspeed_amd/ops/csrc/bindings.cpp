@@ -360,6 +360,9 @@ static void check_pool(const at::Tensor& q, const at::Tensor& kpool,
               what, ": bf16 cuda contiguous");
   TORCH_CHECK(q.size(2) == 128 && kpool.size(3) == 128, what,
               ": D must be 128");
+  for (auto& t : {q, kpool, vpool})
+    TORCH_CHECK(((uintptr_t)t.data_ptr() & 15) == 0, what,
+                ": 16-byte accesses");
   TORCH_CHECK(kpool.size(1) > 0 && q.size(1) % kpool.size(1) == 0, what,
               ": H must be a multiple of Hkv");
 }
@@ -437,7 +440,8 @@ at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
   for (auto& x : {k, v})
     TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
                 x.is_contiguous() && x.dim() == 3 && x.size(0) == T &&
-                x.size(1) == Hkv && x.size(2) == 128, "paged_append: k/v");
+                x.size(1) == Hkv && x.size(2) == 128 &&
+                ((uintptr_t)x.data_ptr() & 15) == 0, "paged_append: k/v");
   TORCH_CHECK(dst.scalar_type() == at::kInt && dst.is_cuda() &&
               dst.is_contiguous() && dst.numel() == T, "paged_append: dst");
   TORCH_CHECK(S >= 1 && T % S == 0, "paged_append: S");

@@ -28,6 +28,12 @@ def paged_decode_available(q: torch.Tensor, kpool: torch.Tensor) -> bool:
             and 1 <= q.size(1) // kpool.size(1) <= 16)
 
 
+def aligned(x: torch.Tensor) -> torch.Tensor:
+    """x as the kernels read it: contiguous, on 16 bytes."""
+    x = x.contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
 def paged_decode_attention(q: torch.Tensor, kpool: torch.Tensor,
                            vpool: torch.Tensor, block_table: torch.Tensor,
                            lens: torch.Tensor, splits: Optional[int] = None,
@@ -41,7 +47,7 @@ def paged_decode_attention(q: torch.Tensor, kpool: torch.Tensor,
     if splits is None:
         nw = max(1, q.size(0) * kpool.size(1))
         splits = max(1, min(32, WORKGROUPS // nw))
-    return ext.paged_decode(q.contiguous(), kpool, vpool,
+    return ext.paged_decode(aligned(q), aligned(kpool), aligned(vpool),
                             block_table.contiguous().int(),
                             lens.contiguous().int(), splits, scale)
 

@@ -87,6 +87,50 @@ def test_rope_attention_leaves_gradients_alone(which, monkeypatch):
         assert cache.rope_attention(0, *qkv, None, None) == "kernels"
 
 
+def test_kernels_get_aligned_tensors(monkeypatch):
+    """16-byte accesses: a slice at an odd offset, or a pool of another layout
+    than the cache's own, is laid out anew; a misaligned cache is left to the
+    general path."""
+    from deepspeed_amd.ops import paged_attention as P
+    seen = []
+
+    class Ext:
+        def __getattr__(self, name):
+            def call(*args):
+                seen.append(name)
+                for t in args:
+                    if torch.is_tensor(t) and t.dtype is torch.bfloat16:
+                        assert t.is_contiguous() and t.data_ptr() % 16 == 0
+                return args[0]
+            return call
+
+    monkeypatch.setattr(P, "get_ext", Ext)
+
+    def odd(*shape):
+        n = int(np.prod(shape))
+        return torch.randn(n + 1).bfloat16()[1:].view(shape)
+
+    q, k, v = odd(1, 1, 4, 128), odd(1, 1, 2, 128), odd(1, 1, 2, 128)
+    pool = odd(3, 2, 64, 128)
+    P.paged_decode_attention(q[0], pool, pool, torch.zeros(1, 1),
+                             torch.ones(1))
+    cache = PagedKVCache(1, 1, 2, 64, 128, dtype=torch.bfloat16)
+    cache.begin_step([0], 1)
+    assert torch.equal(cache._attend(0, q, k, v), q)
+    assert seen == ["paged_decode", "paged_append", "paged_rows"]
+
+    class OnGpu(torch.Tensor):
+        is_cuda = True
+
+    q = torch.zeros(1, 1, 4, 128, dtype=torch.bfloat16).as_subclass(OnGpu)
+    for p, want in ((torch.zeros(3, 2, 64, 128).bfloat16(), True),
+                    (pool, False)):
+        cache.k[0], cache.v[0] = p.as_subclass(OnGpu), p
+        assert cache._eligible(0, q, q, q) is want
+        cache.k[0], cache.v[0] = cache.v[0].as_subclass(OnGpu), pool
+        assert cache._eligible(0, q, q, q) is False
+
+
 def _reference(q, k, v, pos, scale):
     """q [m, H, D] at positions ``pos`` over k, v [L, Hkv, D], in fp64."""
     G = q.shape[1] // k.shape[1]
