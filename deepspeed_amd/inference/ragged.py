@@ -445,7 +445,10 @@ class PagedKVCache:
         self.max_seq = max_seq
         self.device = device
         self._slots: Optional[List[int]] = None
-        self._plans = {}     # of the current step, by (heads, key heads)
+        # of the current step, each made when a layer first asks for it
+        self._plans = {}     # by (heads, key heads)
+        self._mask: Optional[torch.Tensor] = None
+        self._places = None
 
     def free(self, slot: int):
         self.free_blocks.extend(reversed(self.block_table[slot]))
@@ -473,18 +476,25 @@ class PagedKVCache:
             self._ensure_blocks(s, st + q_len)
         self._L = L
         self._starts = starts
-        self._plans = {}
+        self._forget_step()
+
+    def _forget_step(self):
+        self._plans, self._mask, self._places = {}, None, None
 
     @property
     def last_mask(self) -> Optional[torch.Tensor]:
-        """[n, 1, q_len, L] validity of the padded views of ``update``; None
-        outside a step."""
-        if self._slots is None:
-            return None
-        pos = torch.arange(self._L, device=self.device)
-        qpos = (self._starts.to(self.device)[:, None, None] +
-                torch.arange(self._q_len, device=self.device)[None, :, None])
-        return (pos[None, None, :] <= qpos).unsqueeze(1)
+        """[n, 1, q_len, L] validity of the padded views of ``update``, or what
+        it was set to in this step; None outside a step."""
+        if self._mask is None and self._slots is not None:
+            pos = torch.arange(self._L, device=self.device)
+            qpos = (self._starts.to(self.device)[:, None, None] + torch.arange(
+                self._q_len, device=self.device)[None, :, None])
+            self._mask = (pos[None, None, :] <= qpos).unsqueeze(1)
+        return self._mask
+
+    @last_mask.setter
+    def last_mask(self, mask: Optional[torch.Tensor]):
+        self._mask = mask
 
     def _row_places(self):
         """Slot and position of every row of the step, in order."""
@@ -497,18 +507,21 @@ class PagedKVCache:
     def update(self, layer_idx: int, k: torch.Tensor, v: torch.Tensor):
         n, Hkv, q_len, D = k.shape
         bs = self.block_size
-        from ..ops.paged_attention import StepPlan
-        dst, _, _ = StepPlan.rows(*self._row_places(), self.block_table, bs)
-        dst = torch.from_numpy(dst).to(self.device)
-        blk, at = dst // bs, dst % bs
+        nblk = (self._L + bs - 1) // bs
+        if self._places is None:
+            from ..ops.paged_attention import StepPlan
+            dst, _, _ = StepPlan.rows(*self._row_places(), self.block_table,
+                                      bs)
+            dst = torch.from_numpy(dst).to(self.device)
+            self._places = dst // bs, dst % bs, torch.tensor(
+                [(self.block_table[s] + [0] * nblk)[:nblk]
+                 for s in self._slots], dtype=torch.long,
+                device=self.device)                         # [n, nblk]
+        blk, at, idx = self._places
         for pool, x in ((self.k[layer_idx], k), (self.v[layer_idx], v)):
             pool[blk, :, at] = x.transpose(1, 2).reshape(
                 n * q_len, Hkv, D).to(pool.dtype)
         # materialize padded views: gather each slot's blocks
-        nblk = (self._L + bs - 1) // bs
-        idx = torch.tensor([ (self.block_table[s] + [0] * nblk)[:nblk]
-                             for s in self._slots ], dtype=torch.long,
-                           device=self.device)              # [n, nblk]
         kb = self.k[layer_idx][idx]                          # [n,nblk,Hkv,bs,D]
         vb = self.v[layer_idx][idx]
         kb = kb.permute(0, 2, 1, 3, 4).reshape(n, Hkv, nblk * bs, D)
@@ -579,4 +592,4 @@ class PagedKVCache:
         else:
             self.lens[idx] += self._q_len
         self._slots = None
-        self._plans = {}
+        self._forget_step()

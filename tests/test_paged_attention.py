@@ -71,6 +71,33 @@ def test_step_plan_covers_every_key_once(name, bs, heads):
     assert plan.items == merges[:, 1].sum()
 
 
+def test_mask_and_places_are_made_once_a_step(monkeypatch):
+    """Every layer of a step reads the same mask and row places; the mask can be
+    set, for the step, and both are new in the next one."""
+    made = []
+    rows = StepPlan.rows
+    monkeypatch.setattr(StepPlan, "rows",
+                        lambda *a: made.append(0) or rows(*a))
+    cache = PagedKVCache(3, 2, 2, 32, 8, block_size=4)
+    assert cache.last_mask is None
+    for step, n in enumerate((5, 1, 6)):
+        cache.begin_step([1, 0], n)
+        mask = cache.last_mask
+        lo = int(cache._starts[0])
+        assert mask.shape == (2, 1, n, lo + n)
+        assert torch.equal(mask[0, 0].sum(1), lo + 1 + torch.arange(n))
+        k = torch.randn(3, 2, 2, n, 8)
+        for layer in range(3):
+            assert cache.last_mask is mask
+            got, _ = cache.update(layer, k[layer], k[layer])
+            assert torch.equal(got[:, :, lo:], k[layer])
+        assert len(made) == step + 1
+        cache.last_mask = other = ~mask
+        assert cache.last_mask is other
+        cache.end_step()
+        assert cache.last_mask is None
+
+
 @pytest.mark.parametrize("which", [0, 1, 2, None])
 def test_rope_attention_leaves_gradients_alone(which, monkeypatch):
     """With a gradient for queries, keys or values the caller's own path, which
