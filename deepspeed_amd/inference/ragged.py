@@ -499,7 +499,8 @@ class PagedKVCache:
     def _row_places(self):
         """Slot and position of every row of the step, in order."""
         n = self._q_len
-        pos = (self._starts[:, None] + torch.arange(n)).reshape(-1).numpy()
+        starts = self._starts.cpu()       # wherever the lengths are kept
+        pos = (starts[:, None] + torch.arange(n)).reshape(-1).numpy()
         slots = self._slots if n == 1 else \
             [s for s in self._slots for _ in range(n)]
         return slots, pos

@@ -236,6 +236,28 @@ def test_paged_attention_gpu(name, bs, heads):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("device", ["cuda", "cpu"])
+def test_lengths_kept_on_the_gpu(device):
+    """The cache's lengths may lie beside its pool."""
+    res = []
+    for lens in ("cpu", "cuda"):
+        torch.manual_seed(0)
+        cache = PagedKVCache(1, 2, 2, 64, 128, dtype=torch.bfloat16,
+                             device=device)
+        cache.lens = cache.lens.to(lens)
+        for n in (3, 1):
+            cache.begin_step([1, 0], n)
+            q, k, v = (torch.randn(2, n, h, 128).bfloat16().to(device)
+                       for h in (4, 2, 2))
+            o = cache.decode_attention(0, q, k, v)
+            if o is None:
+                o, _ = cache.update(0, k.transpose(1, 2), v.transpose(1, 2))
+            cache.end_step()
+        res.append(o)
+    assert torch.equal(*res)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("scale", [0.05, -0.05, 0.0])
 @pytest.mark.parametrize("splits", [None, 1, 5])
 def test_paged_decode_scales_and_splits(scale, splits):
