@@ -47,11 +47,11 @@ def _rows(x: torch.Tensor) -> torch.Tensor:
 
 def _scaled(q, scale):
     """(q, scale, factor of dq) with a positive scale: the kernels take maxima
-    of unscaled scores."""
+    of unscaled scores. A scale of nought or no number goes into q."""
     scale = scale if scale is not None else 1.0 / math.sqrt(q.size(-1))
     if scale > 0:
         return q, scale, 1
-    return (-q, -scale, -1) if scale < 0 else (torch.zeros_like(q), 1.0, 0)
+    return (-q, -scale, -1) if scale < 0 else (q * scale, 1.0, scale)
 
 
 def _vt_from_bshd(v):

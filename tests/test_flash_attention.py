@@ -76,6 +76,15 @@ def test_splits_agree(splits):
         _close(g, w, n)
 
 
+def test_a_scale_that_is_no_number_shows():
+    torch.manual_seed(0)
+    q, k, v = (torch.randn(1, 40, 2, 64, device="cuda").bfloat16()
+               .requires_grad_() for _ in range(3))
+    o = attention.flash_attn_func(q, k, v, True, math.nan)
+    o.sum().backward()
+    assert o.isnan().all() and q.grad.isnan().all() and k.grad.isnan().all()
+
+
 @pytest.mark.parametrize("scale", [0.3, -0.2, 0.0])
 def test_scales_and_strides(scale):
     """Slices of one buffer, as a joint projection leaves them, BHSD views and
