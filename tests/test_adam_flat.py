@@ -6,15 +6,17 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 2048, 2053, (1 << 25) + 5])
-@pytest.mark.parametrize("offset", [0, 1, 2])
+LARGE = (1 << 25) + 5     # past the caches: the nontemporal kernel
+
+
+@pytest.mark.parametrize("n,offset", [
+    (n, offset) for n in (1, 3, 4, 5, 1023, 2048, 2053)
+    for offset in (0, 1, 2)] + [(LARGE, 0), (LARGE, 1)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16,
                                    torch.float32])
 @pytest.mark.parametrize("adamw", [True, False])
 def test_adam_flat(n, offset, dtype, adamw):
     from deepspeed_amd.ops import _C
-    if n > 1 << 20 and (offset == 2 or not adamw):
-        return
     torch.manual_seed(n)
 
     def buf(dt):

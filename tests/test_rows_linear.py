@@ -35,19 +35,21 @@ def test_cpu_and_grad_calls_are_left_alone():
     assert rows_linear(x, (lin,)) is None
 
 
-def _under_transforms(f, x):
+def _under_transforms(f, x, all=True):
     """f(x) as transforms, tangents, a trace and a dispatch mode make the
     call, by name."""
     import torch.autograd.forward_ad as fwad
     from torch.fx.experimental.proxy_tensor import make_fx
     from torch.utils.flop_counter import FlopCounterMode
-    out = {"vmap": torch.func.vmap(f)(x),
-           "jvp": torch.func.jvp(f, (x,), (2 * x,))[1]}
+    out = {"vmap": torch.func.vmap(f)(x)}
     with fwad.dual_level():
         out["dual"] = fwad.unpack_dual(f(fwad.make_dual(x, 2 * x))).tangent
     with FlopCounterMode(display=False) as mode:
         f(x)
     out["flops"] = mode.get_total_flops()
+    if not all:
+        return out
+    out["jvp"] = torch.func.jvp(f, (x,), (2 * x,))[1]
     # traced on one input, run on another
     out["make_fx"] = make_fx(f)(x)(3 * x)
     out["trace"] = torch.jit.trace(f, x, check_trace=False)(3 * x)
@@ -153,28 +155,38 @@ def test_batch_rule():
 @pytest.mark.parametrize("m", [1, 16, 17, 32, 50])
 @torch.no_grad()
 def test_rows_swiglu_gpu(int8, m):
-    if m > 32 and not int8:
-        return
     g = torch.Generator().manual_seed(m)
     (gate, fg), (up, fu) = (_layer(1000, 512, False, int8, g)
                             for _ in range(2))
     x = torch.randn(m, 512, generator=g).bfloat16().cuda()
-    y, = rows_linear(x, (gate, up), SWIGLU)
+    got = rows_linear(x, (gate, up), SWIGLU)
+    if m > 32 and not int8:
+        assert got is None
+        return
+    y, = got
     _close(y, torch.nn.functional.silu(fg(x)) * fu(x))
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("int8", [False, True])
 @torch.no_grad()
-def test_quantized_linear_under_transforms_gpu():
-    """A quantized layer, which takes the kernel by itself, under each."""
-    lin, want = _layer(64, 256, False, True, torch.Generator().manual_seed(0))
+def test_under_transforms_gpu(int8):
+    """A layer's call as a model makes it, and a quantized layer's own (whose
+    dequantization no tangent transform and no trace has ever passed)."""
+    lin, want = _layer(64, 256, False, int8, torch.Generator().manual_seed(0))
     x = torch.randn(4, 256, device="cuda").bfloat16()
     assert rows_linear(x, (lin,)) is not None
-    got = _under_transforms(lin, x)
+    lin.requires_grad_(False)      # constants of a trace
+
+    def call(x):
+        y = rows_linear(x, (lin,))
+        return lin(x) if y is None else y[0]
+
+    got = _under_transforms(lin if int8 else call, x, all=not int8)
     assert got.pop("flops") == 2 * 4 * 64 * 256
-    for name, scale in (("vmap", 1), ("jvp", 2), ("dual", 2), ("make_fx", 3),
-                        ("trace", 3)):
-        err = got[name].double() - scale * want(x)
+    for name, y in got.items():
+        scale = {"vmap": 1, "jvp": 2, "dual": 2, "make_fx": 3, "trace": 3}[name]
+        err = y.double() - scale * want(x)
         # weights rounded to bf16 on this way round, and inputs 3 * x
         assert err.norm() <= 0.01 * scale * want(x).norm(), name
 
