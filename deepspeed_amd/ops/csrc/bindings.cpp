@@ -680,8 +680,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_bwd(
           layernorm ? dwb.narrow(0, H, H) : at::empty({0}, f32opts)};
 }
 
-// RMS norm of x + res -> (norm, sum, 1/rms). The caller sees to the sizes
-// (ops/norms.py, add_norm_eligible).
+// RMS norm of x + res -> (norm, sum, 1/rms); add_rms_norm in ops/norms.py
+// takes another way for what the kernel does not.
 std::tuple<at::Tensor, at::Tensor, at::Tensor> add_norm_fwd(
     at::Tensor x, at::Tensor res, at::Tensor w, double eps) {
   const OneDevice on("add_norm_fwd", x, res, w);

@@ -1,17 +1,14 @@
-// Tiled bf16 matrix transpose for MI355X (gfx950).
+// bf16 matrix transposes for MI355X (gfx950).
 //
-// torch's permute(...).contiguous() runs the generic strided-copy kernel
-// at ~250 GB/s on these shapes; this LDS-tiled version reads AND writes
-// 16 B-coalesced (64x64 bf16 tiles, padded LDS) and is HBM-bound.
-// Used by the flash-attention wrappers for the V^T / q^T / k^T / do^T
-// layout changes (fwd vt and the bwd BHSD->BHDS copies).
+// transpose_2d: one matrix of any size, the operands of a linear layer's
+// backward (ops/linear.py).
 //
-// Batched: for batch index bh, the source matrix [R, C] starts at
+// transpose_bf16: a batch of matrices out of [B, H, R, C] or [B, R, H, C]
+// through LDS tiles of 64 x 64 (padded), 16-byte accesses both ways. A general
+// layout helper: attention reads its operands transposed by itself. For batch
+// index bh the source matrix [R, C] starts at
 //   src + (bh / inner) * outer_stride + (bh % inner) * inner_stride
-// with row stride row_stride (elements). This covers both
-//   [B, H, R, C] (inner=H, inner_stride=R*C... plain contiguous) and
-//   [B, R, H, C] (inner=H, inner_stride=C, row_stride=H*C) layouts.
-// Destination is contiguous [bh][C][R].
+// with row stride row_stride (elements); the destination is [bh][C][R].
 
 #include "ds_kernels.h"
 

@@ -499,7 +499,7 @@ class ZeroStage12Optimizer:
                                if b.group_idx == gi]).to(dtype=torch.float32)
             else:
                 g = self.group_owned_grads[gi].to(dtype=torch.float32)
-            if isinstance(combined_scale, torch.Tensor) or combined_scale != 1.0:
+            if combined_scale != 1.0:
                 g = g / combined_scale
             master.grad = g
         self.optimizer.step()

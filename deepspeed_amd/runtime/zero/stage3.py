@@ -1008,9 +1008,7 @@ class ZeroStage3Optimizer:
         from ...ops._loader import get_ext
         ext = get_ext()
         have_cpu_adam = ext is not None and hasattr(ext, "cpu_adam_flat")
-        scale = float(combined_scale) if not torch.is_tensor(combined_scale) \
-            else float(combined_scale.item())
-        inv_scale = 1.0 / scale
+        inv_scale = 1.0 / combined_scale
         self._nvme_step_count += 1
         step = self._nvme_step_count
         for gi, group in enumerate(self.optimizer.param_groups):
@@ -1087,7 +1085,7 @@ class ZeroStage3Optimizer:
             if master.numel() == 0:
                 continue
             g = self.group_owned_grads[gi]
-            if isinstance(combined_scale, torch.Tensor) or combined_scale != 1.0:
+            if combined_scale != 1.0:
                 g = g / combined_scale
             master.grad = g
         self.optimizer.step()
