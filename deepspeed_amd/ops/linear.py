@@ -40,18 +40,32 @@ def backward_plan(T: int, N: int, K: int):
     weight's). A product reads an operand along the contracted axis faster than
     across it, and transposing costs a read and a write.
 
-    Weight: pays from some 3000 rows (N 14336, K 4096, us as stored and
-    transposed: 2048 rows 211 / 257, 4000 340 / 344, 8192 708 / 647).
+    Weight (us as stored and transposed, the copy included): pays where the
+    product's gain, at the rates above, is more than the copy: from 2500 to 3500
+    rows by the weight's size (4096 x 4096 over 3500 rows 116 / 107, 4096 x
+    14336 over 3072 305 / 284, 8192 x 3072 196 / 153). Weights that are more
+    than three times as long as wide lose there and gain from some 3600 rows
+    (14336 x 4096: 2560 rows 260 / 273, 3072 294 / 305, 3500 331 / 333, 4000
+    362 / 350, 8192 704 / 640; 128256 x 4096: 3072 rows 2514 / 2657, 4000 3154 /
+    3050). Between 5000 and 6144 rows the longest can lose some percent (32064 x
+    3072: 1142 / 1244 and 1733 / 1781, 8192 rows 1284 / 1198).
     Gradient of the weight: both operands lie across. Transposing the narrower
     is within 7% of the best choice over all sizes measured (8192 rows: 14336 x
     4096 993 / 756, both 741; 4096 x 14336 994 / 785, both 734; 128256 x 4096
     7178 / 6247, both 6364). Outputs under 256 tiles of 256 x 256 and fewer
     rows stay: there the library splits the contraction over more of the chip
     in its own layout (3072 x 3072 over 32768 rows 598 / 994, 14336 x 4096 over
-    1000 rows 160 / 161)."""
+    1000 rows 160 / 161). So do, from 16384 rows, outputs that nearly fill a
+    second round of the 256 CUs (tiles, over 16384 rows: 384 752 / 702, 400 904 /
+    1017, 416 1022 / 1056, 448 984 / 1052 and 927 / 1091, 480 1008 / 998, 512 951
+    / 790); over 8192 rows they gain a fifth, between the two some gain and some
+    lose."""
     flops = 2.0 * T * N * K
-    w = flops / DGRAD_T + 4.0 * N * K / STREAM + LAUNCH < flops / DGRAD
-    big = N * K >= 1 << 24 and T >= 2048
+    w = flops / DGRAD_T + 4.0 * N * K / STREAM + LAUNCH < flops / DGRAD and (
+        N <= 3 * K or T >= 3600)
+    tiles = -(-N // 256) * -(-K // 256)
+    big = N * K >= 1 << 24 and T >= 2048 and not (
+        T >= 16384 and 384 < tiles < 512)
     return w, big and N < K, big and N >= K
 
 
