@@ -240,7 +240,13 @@ void launch(Args a, int layers, hipStream_t st) {
 // FT 1 / 2 / 4): M 8: N 4096 10.8 / 13.8 / 37, N 14336 29.2 / 29.2 / 51;
 // M 16: N 6144 19.5 / 17.0 / 40, N 14336 35.7 / 31.5 / 52; M 32: N 4096 15.7 /
 // 18.6 / 25, N 6144 26.1 / 20.3 / 25.5, N 14336 48 / 36.5 / 29.6. Gate and up
-// (two streams share x): M 16 52.6 / 92, M 32 61.9 / 55.1.
+// (two streams share x): M 16 52.6 / 92, M 32 61.9 / 55.1. int8, for which x
+// weighs twice as much, is within a tenth of its best by the same rule: M 8: N
+// 4096 8.3 / 10.8 / 18, N 6144 13.0 / 11.8 / 19, N 14336 20.7 / 20.9 / 20.1; M
+// 16: N 6144 15.4 / 12.8 / 20, N 14336 25.9 / 23.0 / 20.8, N 128256 176 / 163 /
+// 152; M 32: N 6144 23 / 16.3 / 23, N 14336 40 / 29.7 / 24.0; M 64: N 4096 21.1 /
+// 23.8 / 44, N 14336 74 / 46 / 51; gate and up M 8 35.9 / 34.8, M 16 39.5 / 37.2,
+// M 32 53.8 / 42.6, M 64 88 / 67.
 template <bool I8>
 void launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
   int tiles = 0;
