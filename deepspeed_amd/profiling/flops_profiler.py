@@ -17,6 +17,7 @@ from collections import defaultdict
 import torch
 import torch.nn as nn
 
+from ..ops.linear import Linear
 from ..utils.logging import logger
 
 
@@ -94,7 +95,8 @@ class FlopsProfiler:
 
         self._names = {id(m): n for n, m in self.model.named_modules()}
         for m in self.model.modules():
-            if type(m) in ignore:
+            # the framework's linear layer is torch's to its user
+            if type(m) in ignore or type(m) is Linear and nn.Linear in ignore:
                 continue
             self._hooks.append(m.register_forward_pre_hook(pre_hook))
             self._hooks.append(m.register_forward_hook(post_hook))

@@ -482,6 +482,22 @@ def test_flops_profiler_counts_gemms():
     assert params == 64 * 128 + 128 + 128 * 10 + 10
 
 
+def test_flops_profiler_ignores_torchs_linear():
+    """Ignoring nn.Linear leaves out the models' own linear layers."""
+    from deepspeed_amd.models import llama
+    from deepspeed_amd.ops.linear import Linear
+    from deepspeed_amd.profiling.flops_profiler import FlopsProfiler
+    model = llama.LlamaForCausalLM(llama.llama_tiny())
+    ids = torch.randint(0, 512, (1, 8))
+    for ignore in ([torch.nn.Linear], [Linear]):
+        prof = FlopsProfiler(model)
+        prof.start_profile(ignore_list=ignore)
+        model(ids)
+        prof.stop_profile()
+        assert not any("_proj" in n or "lm_head" in n for n in prof._macs)
+        assert any("norm" in n for n in prof._macs)
+
+
 def test_evoformer_attention_reference_math():
     """DS4Sci_EvoformerAttention vs an index-loop fp32 reference with both
     bias patterns (mask bias [B,N,1,1,S] + pair bias [B,1,H,S,S])."""
