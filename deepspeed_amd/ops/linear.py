@@ -40,15 +40,17 @@ def backward_plan(T: int, N: int, K: int):
     weight's). A product reads an operand along the contracted axis faster than
     across it, and transposing costs a read and a write.
 
-    Weight (us as stored and transposed, the copy included): pays where the
-    product's gain, at the rates above, is more than the copy: from 2500 to 3500
-    rows by the weight's size (4096 x 4096 over 3500 rows 116 / 107, 4096 x
-    14336 over 3072 305 / 284, 8192 x 3072 196 / 153). Weights that are more
-    than three times as long as wide lose there and gain from some 3600 rows
-    (14336 x 4096: 2560 rows 260 / 273, 3072 294 / 305, 3500 331 / 333, 4000
-    362 / 350, 8192 704 / 640; 128256 x 4096: 3072 rows 2514 / 2657, 4000 3154 /
-    3050). Between 5000 and 6144 rows the longest can lose some percent (32064 x
-    3072: 1142 / 1244 and 1733 / 1781, 8192 rows 1284 / 1198).
+    Weight: the library's times jump by up to 1.9 between neighbouring numbers of
+    rows (128256 x 4096: 2560 rows 2245 us, 2561 3724), so a rule by rows holds
+    on balance only. Over 15 weights of 3072 x 3072 to 152064 x 3584 (us as
+    stored and transposed, the copy included): below some 3100 rows large ones
+    mostly lose (14336 x 4096: 2560 rows 264 / 271, 3000 285 / 296; 4096 x
+    14336: 2700 345 / 399; 128256 x 4096: 2700 3820 / 4378, 3000 2560 / 2585;
+    8192 x 8192: 3000 337 / 347), from there on two in three gain (14336 x 4096:
+    3111 496 / 390, 3500 324 / 327, 4000 351 / 342, 8192 704 / 640; 128256 x
+    4096: 3111 4088 / 3224, 4000 3190 / 2973; 4096 x 4096: 3500 117 / 108; but
+    4096 x 14336: 3500 404 / 448, 4000 400 / 370; 32064 x 3072: 3500 904 / 968,
+    4000 632 / 626). Small ones wait for the copy to be worth it.
     Gradient of the weight: both operands lie across. Transposing the narrower
     is within 7% of the best choice over all sizes measured (8192 rows: 14336 x
     4096 993 / 756, both 741; 4096 x 14336 994 / 785, both 734; 128256 x 4096
@@ -61,8 +63,8 @@ def backward_plan(T: int, N: int, K: int):
     / 790); over 8192 rows they gain a fifth, between the two some gain and some
     lose."""
     flops = 2.0 * T * N * K
-    w = flops / DGRAD_T + 4.0 * N * K / STREAM + LAUNCH < flops / DGRAD and (
-        N <= 3 * K or T >= 3600)
+    w = T >= 3100 and flops / DGRAD_T + 4.0 * N * K / STREAM + LAUNCH < \
+        flops / DGRAD
     tiles = -(-N // 256) * -(-K // 256)
     big = N * K >= 1 << 24 and T >= 2048 and not (
         T >= 16384 and 384 < tiles < 512)

@@ -16,10 +16,11 @@ def test_backward_plan():
     assert L.backward_plan(32768, 3072, 3072) == (True, False, False)
     assert L.backward_plan(16, 64, 64) == (False, False, False)
     # the weight: where the copy has been measured to pay
-    for n, k, rows in ((14336, 4096, 3600), (128256, 4096, 3600),
-                       (4096, 14336, 2700), (8192, 3072, 3050)):
-        for t in (2048, 2560, 3000, 3072, 3500, 4000, 8192):
-            assert L.backward_plan(t, n, k)[0] == (t >= rows), (t, n, k)
+    for n, k in ((14336, 4096), (128256, 4096), (4096, 14336), (8192, 3072)):
+        for t in (2048, 2560, 3000, 3111, 4000, 8192):
+            assert L.backward_plan(t, n, k)[0] == (t > 3100), (t, n, k)
+    assert [L.backward_plan(t, 4096, 4096)[0] for t in (3111, 3500)] == \
+        [False, True]
     # its gradient: not where the output nearly fills a second round of CUs
     for n, k, much in ((5120, 5120, False), (7168, 4096, False),
                        (6144, 4096, True), (6144, 6144, True)):
