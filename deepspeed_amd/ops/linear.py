@@ -171,16 +171,20 @@ def unhooked(mod: nn.Module, internal_ok: bool = False) -> bool:
     cls = type(mod)
     if "forward" in mod.__dict__ or mod._compiled_call_impl is not None or \
             cls.forward is not _FORWARD.get(cls) or \
-            nn.Linear.forward is not _TORCHS:
+            nn.Linear.forward is not _TORCHS or \
+            _module._global_forward_hooks or \
+            _module._global_forward_pre_hooks or \
+            _module._global_backward_hooks or \
+            _module._global_backward_pre_hooks:
         return False
-    own = (mod._forward_hooks, mod._forward_pre_hooks, mod._backward_hooks,
-           mod._backward_pre_hooks)
-    return not (any(not (internal_ok and getattr(h, "_ds_internal", False))
-                    for hooks in own if hooks for h in hooks.values())
-                or _module._global_forward_hooks
-                or _module._global_forward_pre_hooks
-                or _module._global_backward_hooks
-                or _module._global_backward_pre_hooks)
+    if not (mod._forward_hooks or mod._forward_pre_hooks
+            or mod._backward_hooks or mod._backward_pre_hooks):
+        return True
+    return internal_ok and all(
+        getattr(h, "_ds_internal", False)
+        for hooks in (mod._forward_hooks, mod._forward_pre_hooks,
+                      mod._backward_hooks, mod._backward_pre_hooks)
+        for h in hooks.values())
 
 
 def batch_pays(ns, K: int) -> bool:
