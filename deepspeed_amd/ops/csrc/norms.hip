@@ -8,7 +8,8 @@
 //  * forward caches the row in registers when H <= 16384 (one HBM read)
 //  * the residual stream's add belongs to the norm: the forward reads the
 //    sublayer's output and the stream, writes their sum and its norm (taken
-//    from the fp32 sum, not from its rounding); the backward adds the stream's
+//    from the fp32 sum, not from its rounding, which is what the backward reads
+//    again, with the fp32 sum's 1/rms); the backward adds the stream's
 //    gradient before it rounds. An add kernel each way moved three more
 //    tensors and rounded once more.
 //  * backward: a row in registers (one read), the weight's gradient in

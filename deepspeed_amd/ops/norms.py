@@ -96,7 +96,11 @@ class _LayerNormFn(torch.autograd.Function):
 
 
 class _AddNormFn(torch.autograd.Function):
-    """RMS norm of x + residual, and the sum itself (GPU, 16-bit)."""
+    """RMS norm of x + residual, and the sum itself (GPU, 16-bit). The norm is
+    that of the fp32 sum; kept for the backward is the sum that is handed on,
+    rounded to 16 bits, with the 1/rms of the fp32 one. The gradient is so that
+    of a point half a unit in the last place of each value away, as it was with
+    an add of its own, whose norm began at that point too."""
 
     @staticmethod
     def forward(ctx, x, residual, weight, eps):
