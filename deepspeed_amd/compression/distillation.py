@@ -2,7 +2,7 @@
 deepspeed/compression: layer_reduction / distillation config in
 compress.py + the schedule_offset machinery in basic_layer.py).
 
-Three pieces the round-1 miniature lacked:
+Three pieces:
 
 * ``KDLoss`` — the standard distillation objective: KL(student/T ||
   teacher/T) * T^2 blended with the hard-label loss, plus optional

@@ -2,9 +2,9 @@
 
 See csrc/cross_entropy.hip. The autograd wrapper recomputes nothing: the
 forward saves (logits, labels, lse) and the backward emits bf16 dlogits in
-one elementwise pass. Enabled in the chunked-CE loss path with
-DS_AMD_FUSED_CE=1 (GPU numerics validation is a round-2 gate; the torch
-fallback defines the semantics and runs everywhere)."""
+one elementwise pass. The default of the chunked-CE loss path on a GPU
+(DS_AMD_FUSED_CE=0 opts out); the torch fallback defines the semantics and
+runs everywhere."""
 
 import os
 
@@ -33,10 +33,9 @@ class _FusedCE(torch.autograd.Function):
 
 
 def fused_ce_available(logits) -> bool:
-    """Default ON (GPU-numerics-validated round 2, r2_call3): the fused
-    kernel computes loss+lse from bf16 logits and emits bf16 dlogits in
-    one pass — no [tokens, vocab] fp32 materialization, no cunn_SoftMax
-    pair. DS_AMD_FUSED_CE=0 opts out."""
+    """Default ON: the fused kernel computes loss+lse from bf16 logits and
+    emits bf16 dlogits in one pass — no [tokens, vocab] fp32 materialization,
+    no cunn_SoftMax pair. DS_AMD_FUSED_CE=0 opts out."""
     return (os.environ.get("DS_AMD_FUSED_CE", "1") != "0"
             and get_ext() is not None and logits.is_cuda
             and logits.dtype == torch.bfloat16)

@@ -183,9 +183,8 @@ def test_init_inference_fp6_weight_only_gpu():
 
 
 def test_llama_mini_fp16_loss_scaling_gpu():
-    """fp16 + dynamic loss scaling on device (VERDICT: fp16 dtype matrix
-    had no GPU runtime): losses stay finite, the scale survives, and
-    training moves."""
+    """fp16 + dynamic loss scaling on device: losses stay finite, the scale
+    survives, and training moves."""
     import deepspeed_amd
     from deepspeed_amd.models import LlamaConfig, LlamaForCausalLM
     _init_env()
