@@ -448,6 +448,7 @@ class PagedKVCache:
         # of the current step, each made when a layer first asks for it
         self._plans = {}     # by (heads, key heads)
         self._mask: Optional[torch.Tensor] = None
+        self._mask_made = True
         self._places = None
 
     def free(self, slot: int):
@@ -480,21 +481,22 @@ class PagedKVCache:
 
     def _forget_step(self):
         self._plans, self._mask, self._places = {}, None, None
+        self._mask_made = False
 
     @property
     def last_mask(self) -> Optional[torch.Tensor]:
         """[n, 1, q_len, L] validity of the padded views of ``update``, or what
         it was set to in this step; None outside a step."""
-        if self._mask is None and self._slots is not None:
+        if not self._mask_made and self._slots is not None:
             pos = torch.arange(self._L, device=self.device)
             qpos = (self._starts.to(self.device)[:, None, None] + torch.arange(
                 self._q_len, device=self.device)[None, :, None])
-            self._mask = (pos[None, None, :] <= qpos).unsqueeze(1)
+            self.last_mask = (pos[None, None, :] <= qpos).unsqueeze(1)
         return self._mask
 
     @last_mask.setter
     def last_mask(self, mask: Optional[torch.Tensor]):
-        self._mask = mask
+        self._mask, self._mask_made = mask, True
 
     def _row_places(self):
         """Slot and position of every row of the step, in order."""

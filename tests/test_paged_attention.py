@@ -94,6 +94,8 @@ def test_mask_and_places_are_made_once_a_step(monkeypatch):
         assert len(made) == step + 1
         cache.last_mask = other = ~mask
         assert cache.last_mask is other
+        cache.last_mask = None
+        assert cache.last_mask is None
         cache.end_step()
         assert cache.last_mask is None
 
