@@ -448,7 +448,7 @@ class PagedKVCache:
         # of the current step, each made when a layer first asks for it
         self._plans = {}     # by (heads, key heads)
         self._mask: Optional[torch.Tensor] = None
-        self._mask_made = True
+        self._mask_given = False
         self._places = None
 
     def free(self, slot: int):
@@ -481,22 +481,23 @@ class PagedKVCache:
 
     def _forget_step(self):
         self._plans, self._mask, self._places = {}, None, None
-        self._mask_made = False
+        self._mask_given = False
 
     @property
     def last_mask(self) -> Optional[torch.Tensor]:
         """[n, 1, q_len, L] validity of the padded views of ``update``, or what
         it was set to in this step; None outside a step."""
-        if not self._mask_made and self._slots is not None:
+        if self._mask is None and not self._mask_given and \
+                self._slots is not None:
             pos = torch.arange(self._L, device=self.device)
             qpos = (self._starts.to(self.device)[:, None, None] + torch.arange(
                 self._q_len, device=self.device)[None, :, None])
-            self.last_mask = (pos[None, None, :] <= qpos).unsqueeze(1)
+            self._mask = (pos[None, None, :] <= qpos).unsqueeze(1)
         return self._mask
 
     @last_mask.setter
     def last_mask(self, mask: Optional[torch.Tensor]):
-        self._mask, self._mask_made = mask, True
+        self._mask, self._mask_given = mask, True
 
     def _row_places(self):
         """Slot and position of every row of the step, in order."""
@@ -564,8 +565,10 @@ class PagedKVCache:
         and k, v [n, S, Hkv, D]: rotary embedding (tables [max_pos, D/2];
         positions int32 [n, S] or each row's index in S), cache write and
         causal attention over the paged pool. None when ineligible (the caller
-        rotates and takes ``decode_attention`` or ``update``)."""
-        if not self._eligible(layer_idx, q, k, v) or not untransformed() or (
+        rotates and takes ``decode_attention`` or ``update``), as with a mask
+        of the caller's own."""
+        if self._mask_given or not self._eligible(layer_idx, q, k, v) or \
+                not untransformed() or (
                 torch.is_grad_enabled()
                 and any(x.requires_grad for x in (q, k, v))):
             return None

@@ -114,6 +114,14 @@ def test_rope_attention_leaves_gradients_alone(which, monkeypatch):
     assert cache.rope_attention(0, *qkv, None, None) == want
     with torch.no_grad():
         assert cache.rope_attention(0, *qkv, None, None) == "kernels"
+        # a mask of the caller's own is for the path that has one
+        cache.begin_step([0], 3)
+        cache.last_mask
+        assert cache.rope_attention(0, *qkv, None, None) == "kernels"
+        cache.last_mask = torch.ones(1, 1, 3, 3, dtype=torch.bool)
+        assert cache.rope_attention(0, *qkv, None, None) is None
+        cache.end_step()
+        assert cache.rope_attention(0, *qkv, None, None) == "kernels"
 
 
 def test_kernels_get_aligned_tensors(monkeypatch):
