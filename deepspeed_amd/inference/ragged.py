@@ -559,6 +559,12 @@ class PagedKVCache:
         o = paged_attention(plan, q, kp, vp, scale)
         return o.view(n, S, H, D)
 
+    def _replaced(self) -> bool:
+        cls, own = type(self), self.__dict__
+        return (cls.update is not PagedKVCache.update
+                or cls.decode_attention is not PagedKVCache.decode_attention
+                or "update" in own or "decode_attention" in own)
+
     def rope_attention(self, layer_idx: int, q, k, v, cos, sin,
                        positions=None, scale=None):
         """A step's attention from the unrotated projections q [n, S, H, D]
@@ -566,8 +572,9 @@ class PagedKVCache:
         positions int32 [n, S] or each row's index in S), cache write and
         causal attention over the paged pool. None when ineligible (the caller
         rotates and takes ``decode_attention`` or ``update``), as with a mask
-        of the caller's own."""
-        if self._mask_given or not self._eligible(layer_idx, q, k, v) or \
+        of the caller's own or another class's ``update``."""
+        if self._mask_given or self._replaced() or \
+                not self._eligible(layer_idx, q, k, v) or \
                 not untransformed() or (
                 torch.is_grad_enabled()
                 and any(x.requires_grad for x in (q, k, v))):

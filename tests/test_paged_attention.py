@@ -124,6 +124,21 @@ def test_rope_attention_leaves_gradients_alone(which, monkeypatch):
         assert cache.rope_attention(0, *qkv, None, None) == "kernels"
 
 
+@pytest.mark.parametrize("name", ["update", "decode_attention"])
+def test_caches_with_methods_of_their_own(name, monkeypatch):
+    """A subclass's or an instance's update and decode_attention are called."""
+    own = type("Own", (PagedKVCache,), {name: lambda self, *a: None})
+    qkv = [torch.zeros(1, 1, 2, 128)] * 3
+    for cls in (own, PagedKVCache):
+        cache = cls(1, 1, 2, 64, 128)
+        monkeypatch.setattr(cache, "_eligible", lambda *a: True)
+        monkeypatch.setattr(cache, "_attend", lambda *a: "kernels")
+        assert cache.rope_attention(0, *qkv, None, None) == \
+            (None if cls is own else "kernels")
+    setattr(cache, name, lambda *a: None)
+    assert cache.rope_attention(0, *qkv, None, None) is None
+
+
 def test_kernels_get_aligned_tensors(monkeypatch):
     """16-byte accesses: a slice at an odd offset, or a pool of another layout
     than the cache's own, is laid out anew; a misaligned cache is left to the
