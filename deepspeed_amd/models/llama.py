@@ -7,8 +7,8 @@ theta=500000, SwiGLU MLP, RMSNorm, tied-off lm_head).
 
 Hot ops: RMSNorm / RoPE / SwiGLU are the hand-written HIP kernels in
 ``deepspeed_amd.ops``, and so is attention (flash forward and backward, paged
-serving) wherever its kernels apply, else torch SDPA; GEMMs go through torch
-(hipBLASLt).
+serving) wherever its kernels apply, else torch SDPA; linear layers of inference
+are ``ops.linear``'s kernels, GEMMs of training go through torch (hipBLASLt).
 """
 
 from dataclasses import dataclass
@@ -18,7 +18,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ..ops.attention import rope_flash_attention
-from ..ops.linear import SWIGLU, Linear, movable, rows_linear, unhooked
+from ..ops.linear import (SWIGLU, Linear, movable, rows_linear, tile_linear,
+                          unhooked)
 from ..ops.norms import RMSNorm
 from ..ops.rope import apply_rope, rope_tables
 from ..ops.swiglu import swiglu
@@ -128,13 +129,14 @@ class LlamaAttention(nn.Module):
         self.o_proj = Linear(cfg.num_heads * self.head_dim, h, bias=False)
 
     def _out(self, o):
-        y = rows_linear(o, (self.o_proj,))
+        y = rows_linear(o, (self.o_proj,)) or tile_linear(o, (self.o_proj,))
         return self.o_proj(o) if y is None else y[0]
 
     def forward(self, x, cos, sin, positions=None, kv_cache=None,
                 attention_fn=None):
         B, S, _ = x.shape
-        qkv = rows_linear(x, (self.q_proj, self.k_proj, self.v_proj))
+        mods = self.q_proj, self.k_proj, self.v_proj
+        qkv = rows_linear(x, mods) or tile_linear(x, mods)
         if qkv is None:
             qkv = self.q_proj(x), self.k_proj(x), self.v_proj(x)
         q = qkv[0].view(B, S, self.num_heads, self.head_dim)
@@ -244,9 +246,11 @@ class LlamaMLP(nn.Module):
         self.down_proj = Linear(i, h, bias=False)
 
     def forward(self, x):
-        h = rows_linear(x, (self.gate_proj, self.up_proj), SWIGLU)
+        mods = self.gate_proj, self.up_proj
+        h = rows_linear(x, mods, SWIGLU) or tile_linear(x, mods, SWIGLU)
         h = swiglu(self.gate_proj(x), self.up_proj(x)) if h is None else h[0]
-        y = rows_linear(h, (self.down_proj,))
+        mods = self.down_proj,
+        y = rows_linear(h, mods) or tile_linear(h, mods)
         return self.down_proj(h) if y is None else y[0]
 
 
@@ -347,7 +351,8 @@ class LlamaForCausalLM(nn.Module):
             # [B*S, vocab] fp32 logits (vocab=128256 -> ~2 GB per 4k tokens).
             # Routed through the lm_head MODULE so ZeRO-3 fetch hooks fire.
             return chunked_cross_entropy(hidden, self.lm_head, labels)
-        logits = rows_linear(hidden, (self.lm_head,))
+        mods = self.lm_head,
+        logits = rows_linear(hidden, mods) or tile_linear(hidden, mods)
         return self.lm_head(hidden) if logits is None else logits[0]
 
     def num_parameters(self):

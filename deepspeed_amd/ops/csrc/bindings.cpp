@@ -100,11 +100,13 @@ extern "C" void ds_rows_linear(const void* x, int layers, const void* const* w,
                                const void* const* bias, void* const* out,
                                const int* n, int M,
                                int K, int group, int mode, void* stream);
-extern "C" int ds_batch_linear_splits(const int* n, int layers, int M, int K);
-extern "C" void ds_batch_linear(const void* x, int layers,
-                                const void* const* w, const void* const* bias,
-                                void* const* out, const int* n, int M, int K,
-                                int splits, float* part, void* stream);
+extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
+                                   int mode, int* splits);
+extern "C" int ds_tile_linear_stages(int tile, int mode);
+extern "C" int ds_tile_linear(const void* x, int layers, const void* const* w,
+                              const void* const* bias, void* const* out,
+                              const int* n, int M, int K, int mode, int tile,
+                              int splits, float* part, void* stream);
 extern "C" void ds_transpose_bf16(const void* src, void* dst, int n_batch,
                                   int R, int C, long long row_stride,
                                   int inner, long long inner_stride,
@@ -473,10 +475,73 @@ at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
   return out;
 }
 
-// Linear layers on one input of a few rows (rows_linear.hip), or of up to 256
-// with bf16 weights (batch_linear.hip). weights: bf16 [N, K], or int8 (any
+// bf16 weights on one input, pointers and features of each; outputs made anew:
+// one each, or with mode 1 silu(layer 0) * layer 1.
+struct Layers {
+  const void *w[3], *b[3];
+  void* o[3];
+  int n[3];
+  int count = 0;
+  int64_t all = 0;
+  std::vector<at::Tensor> out;
+
+  void add(const char* what, const at::Tensor& x, const at::Tensor& weight,
+           const c10::optional<at::Tensor>& bias, at::ScalarType type,
+           int64_t mode) {
+    const int64_t M = x.size(0), K = x.size(1);
+    const int i = count++;
+    TORCH_CHECK(weight.is_cuda() && weight.is_contiguous() &&
+                weight.scalar_type() == type && weight.numel() % K == 0 &&
+                weight.numel() > 0 && weight.numel() / K < (1 << 30) &&
+                ((uintptr_t)weight.data_ptr() & 15) == 0, what, ": weight");
+    n[i] = weight.numel() / K;
+    all += n[i];
+    w[i] = weight.data_ptr();
+    b[i] = nullptr;
+    if (bias.has_value()) {
+      TORCH_CHECK(bias->is_cuda() && bias->is_contiguous() &&
+                  bias->scalar_type() == at::kBFloat16 &&
+                  bias->numel() == n[i], what, ": bias");
+      b[i] = bias->data_ptr();
+    }
+    if (mode == 0 || i == 0) out.push_back(at::empty({M, n[i]}, x.options()));
+    o[i] = out.back().data_ptr();
+    TORCH_CHECK(mode == 0 || n[0] == n[i], what, ": gate and up");
+  }
+  // Whether tile_linear.hip takes them; does it if so. A tile and a number of
+  // splits may be asked for.
+  bool tiled(const at::Tensor& x, int64_t mode, int tile = -1,
+             int splits = 1) {
+    const int64_t M = x.size(0), K = x.size(1);
+    if (K % 64 || K > (1 << 22) || M >= (1 << 30)) return false;
+    for (int i = 0; i < count; ++i)
+      if (n[i] % 4) return false;
+    if (tile < 0)
+      tile = ds_tile_linear_plan(n, count, (int)M, (int)K, (int)mode, &splits);
+    const int stages = ds_tile_linear_stages(tile, (int)mode);
+    if (stages < 1 || splits < 1 || K / 64 / splits < stages ||
+        (mode && splits > 1))
+      return false;
+    at::Tensor part;
+    if (splits > 1)
+      part = at::empty({splits * M * all}, x.options().dtype(at::kFloat));
+    const int e = ds_tile_linear(
+        x.data_ptr(), count, w, b, o, n, (int)M, (int)K, (int)mode, tile,
+        splits, splits > 1 ? part.data_ptr<float>() : nullptr, cur_stream());
+    TORCH_CHECK(e == 0, "tile_linear: launch failed with error ", e);
+    return true;
+  }
+};
+
+// Linear layers on one input of a few rows: rows_linear.hip, or tile_linear.hip
+// for bf16 weights and more than 16 of them. weights: bf16 [N, K], or int8 (any
 // shape, N * K long) with their groupwise scales. mode 1 returns
 // silu(layer 0) * layer 1.
+//
+// 16: above it tile_linear.hip shares x in LDS where rows_linear.hip reads it
+// out of L2 for every 16 to 64 features (us, rows_linear at 32 rows and
+// tile_linear at 33: N 4096, K 4096 15.7 / 11.7; q, k and v of that 20.3 / 16.5;
+// N 4096, K 14336 33 / 26; gate and up 14336 60 / 52; N 128256 226 / 179).
 std::vector<at::Tensor> rows_linear(
     at::Tensor x, std::vector<at::Tensor> weights,
     std::vector<at::Tensor> scales,
@@ -494,60 +559,50 @@ std::vector<at::Tensor> rows_linear(
               K % 256 == 0 && L >= 1 && L <= 3 && (mode == 0 || L == 2) &&
               (scales.empty() || (int)scales.size() == L) &&
               (int)biases.size() == L, "rows_linear: shape");
+  TORCH_CHECK(((uintptr_t)x.data_ptr() & 15) == 0, "rows_linear: alignment");
   const bool i8 = !scales.empty();
-  const void *w[3], *b[3];
   const float* sc[3];
-  void* o[3];
-  int n[3];
-  std::vector<at::Tensor> out;
+  Layers y;
   for (int i = 0; i < L; ++i) {
-    const auto& t = weights[i];
-    TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
-                t.scalar_type() == (i8 ? at::kChar : at::kBFloat16) &&
-                t.numel() % K == 0 && t.numel() > 0 &&
-                ((uintptr_t)t.data_ptr() & 15) == 0, "rows_linear: weight");
-    n[i] = t.numel() / K;
-    w[i] = t.data_ptr();
-    b[i] = nullptr;
-    if (biases[i].has_value()) {
-      TORCH_CHECK(biases[i]->is_cuda() && biases[i]->is_contiguous() &&
-                  biases[i]->scalar_type() == at::kBFloat16 &&
-                  biases[i]->numel() == n[i], "rows_linear: bias");
-      b[i] = biases[i]->data_ptr();
-    }
+    y.add("rows_linear", x, weights[i], biases[i],
+          i8 ? at::kChar : at::kBFloat16, mode);
     if (i8) {
       TORCH_CHECK(scales[i].is_cuda() && scales[i].is_contiguous() &&
                   scales[i].scalar_type() == at::kFloat && group > 0 &&
                   group % 256 == 0 &&
-                  scales[i].numel() == (t.numel() + group - 1) / group,
+                  scales[i].numel() ==
+                      (weights[i].numel() + group - 1) / group,
                   "rows_linear: scales");
       sc[i] = scales[i].data_ptr<float>();
     }
-    if (mode == 0 || i == 0)
-      out.push_back(at::empty({M, n[i]}, x.options()));
-    o[i] = out.back().data_ptr();
   }
-  TORCH_CHECK(mode == 0 || n[0] == n[1], "rows_linear: gate and up");
-  TORCH_CHECK(((uintptr_t)x.data_ptr() & 15) == 0, "rows_linear: alignment");
-  if (!i8 && M > 32) {
-    TORCH_CHECK(mode == 0, "rows_linear: no activation past 32 rows");
-    int64_t all = 0;
-    for (int i = 0; i < L; ++i) {
-      TORCH_CHECK(n[i] % 4 == 0, "rows_linear: features in fours");
-      all += n[i];
-    }
-    const int splits = ds_batch_linear_splits(n, L, (int)M, (int)K);
-    at::Tensor part;
-    if (splits > 1)
-      part = at::empty({splits * M * all}, x.options().dtype(at::kFloat));
-    ds_batch_linear(x.data_ptr(), L, w, b, o, n, (int)M, (int)K, splits,
-                    splits > 1 ? part.data_ptr<float>() : nullptr,
-                    cur_stream());
-    return out;
-  }
-  ds_rows_linear(x.data_ptr(), L, w, i8 ? sc : nullptr, b, o, n, (int)M,
-                 (int)K, (int)group, (int)mode, cur_stream());
-  return out;
+  if (!i8 && M > 16 && y.tiled(x, mode)) return y.out;
+  TORCH_CHECK(i8 || M <= 32, "rows_linear: features in fours past 32 rows");
+  ds_rows_linear(x.data_ptr(), L, y.w, i8 ? sc : nullptr, y.b, y.o, y.n,
+                 (int)M, (int)K, (int)group, (int)mode, cur_stream());
+  return y.out;
+}
+
+// Linear layers on one input of any number of rows, bf16 (tile_linear.hip).
+std::vector<at::Tensor> tile_linear(
+    at::Tensor x, std::vector<at::Tensor> weights,
+    std::vector<c10::optional<at::Tensor>> biases, int64_t mode, int64_t tile,
+    int64_t splits) {
+  const OneDevice on("tile_linear", x);
+  for (auto& t : weights) on.check(t);
+  for (auto& t : biases) on.check(t);
+  const int L = weights.size();
+  TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
+              x.is_contiguous() && x.dim() == 2 && x.numel() > 0 &&
+              ((uintptr_t)x.data_ptr() & 15) == 0, "tile_linear: x");
+  TORCH_CHECK(L >= 1 && L <= 3 && (mode == 0 || (mode == 1 && L == 2)) &&
+              (int)biases.size() == L, "tile_linear: shape");
+  Layers y;
+  for (int i = 0; i < L; ++i)
+    y.add("tile_linear", x, weights[i], biases[i], at::kBFloat16, mode);
+  TORCH_CHECK(y.tiled(x, mode, (int)tile, (int)splits),
+              "tile_linear: features in fours, inputs in 64s, 192 or more");
+  return y.out;
 }
 
 at::Tensor sum_of_squares(std::vector<at::Tensor> ts) {
@@ -982,6 +1037,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "split-KV decode attention over a paged KV block table");
   m.def("rows_linear", &rows_linear,
         "linear layers of a few rows, bf16 or groupwise int8 weights");
+  m.def("tile_linear", &tile_linear, "linear layers of many rows, bf16",
+        py::arg("x"), py::arg("weights"), py::arg("biases"), py::arg("mode"),
+        py::arg("tile") = -1, py::arg("splits") = 1);
   m.def("sum_of_squares", &sum_of_squares,
         "sum of squares over a list of tensors");
   m.def("paged_rows", &paged_rows,

@@ -1,0 +1,537 @@
+// Linear layers of many rows for MI355X (gfx950): y = x W^T, x [M, K] bf16,
+// W [N, K] bf16, M past what rows_linear.hip takes: decoding for many requests,
+// portions of prompts, whole prompts.
+//
+// Reference analogue: the GEMMs of inference/v2/kernels/core_ops/blas_kernels
+// and the gated ones of core_ops/gated_activations.
+//
+// A workgroup owns a tile of BM rows by BN features. Stages of 64 inputs of
+// both go from memory straight into a ring of NS buffers in LDS
+// (global_load_lds, 16 bytes a lane; 16-byte chunk c of a row lies at
+// c ^ (row & 7), which the lanes' addresses bring about, since a wave's load
+// fills 1 KB of LDS in lane order: no bank conflicts counted). Operands of the
+// products are read into registers one phase ahead. A stage's inputs take four
+// phases: the first half of the wave's rows over inputs 0-31 and 32-63, then
+// the second half; so W and the first half of x are read out after a quarter of
+// the stage, their buffer is loaded anew from there on, and loads have one and
+// a half stages to arrive in with only two buffers.
+//
+//   * Loads are spread between the products, two in a phase of 16: a burst of
+//     them stalls its wave behind the address units, and the products after it
+//     wait (8192 x 8192 x 8192: 805 us with the loads at once, 747 spread;
+//     without loads 655, loads alone 650; the library's product 690 to 750).
+//   * Several layers on one input (q, k, v) are one launch, so that narrow ones
+//     fill the chip together; with SWIGLU a tile holds gate and up, 16 features
+//     of each in turn, and the activation is taken from the fp32 sums.
+//   * Where tiles leave CUs idle, the contraction is split; partial sums stay
+//     fp32 and are added in their order by a second kernel.
+
+#include "ds_kernels.h"
+
+#include <cmath>
+
+#pragma clang diagnostic ignored "-Winline-asm"     // m0 among the clobbers
+
+namespace {
+
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int MAXL = 3;     // layers a launch
+constexpr int BK = 64;      // inputs a stage
+constexpr int ROW = BK * 2; // bytes of a row of a stage
+
+enum { PLAIN = 0, SWIGLU = 1 };
+
+struct Args {
+  const short* w[MAXL];
+  const short* bias[MAXL];
+  short* out[MAXL];
+  int n[MAXL];          // features, multiples of four
+  int tile_end[MAXL];   // tiles of features up to and with a layer
+  int n_end[MAXL];      // features up to and with a layer
+  const short* x;
+  float* part;          // [splits, M, all features], splits > 1
+  int M, K, layers, tiles, mtiles, splits;
+};
+
+__device__ __forceinline__ f32x4 mfma(s16x8 a, s16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+      __builtin_bit_cast(b16x8, a), __builtin_bit_cast(b16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ short bits(float x) {
+  return __builtin_bit_cast(short, (__bf16)x);
+}
+__device__ __forceinline__ float value(short x) {
+  return __builtin_bit_cast(float, (unsigned)(unsigned short)x << 16);
+}
+__device__ __forceinline__ f32x4 add_bias(f32x4 y, const short* bias, int n) {
+  if (bias)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] += value(bias[n + e]);
+  return y;
+}
+__device__ __forceinline__ s16x4 packed(f32x4 y) {
+  return s16x4{bits(y[0]), bits(y[1]), bits(y[2]), bits(y[3])};
+}
+
+__device__ __forceinline__ int uni(int x) {
+  return __builtin_amdgcn_readfirstlane(x);
+}
+__device__ __forceinline__ const char* uni(const char* p) {
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)p);
+  const unsigned hi =
+      __builtin_amdgcn_readfirstlane((unsigned)((uintptr_t)p >> 32));
+  return (const char*)(((uintptr_t)hi << 32) | lo);
+}
+
+// 16 bytes a lane from base + off to LDS, lane after lane from `lds` on. Not the
+// builtin: behind that the compiler waits for all loads before it reads LDS.
+__device__ __forceinline__ void load_lds(const char* base, unsigned off,
+                                         int lds) {
+  asm volatile("s_mov_b32 m0, %2\n\t"
+               "s_nop 0\n\t"
+               "global_load_lds_dwordx4 %0, %1"
+               :: "v"(off), "s"(uni(base)), "s"(uni(lds)) : "memory", "m0");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() {  // but for the N youngest
+  static_assert(N < 64, "vmcnt has six bits");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void barrier() {   // and what was read from LDS
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// MT products with NR reads from LDS in their first half and ND loads spread
+// over all of them.
+template <int MT, int NR, int ND, typename Mul, typename Read, typename Load>
+__device__ __forceinline__ void phase(Mul mul, Read read, Load load) {
+  constexpr int HALF = MT / 2 > 0 ? MT / 2 : 1;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+      if (q * HALF / (NR > 0 ? NR : 1) == i) {
+        read(q);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+    for (int q = 0; q < ND; ++q)
+      if ((2 * q + 1) * MT / (ND > 0 ? 2 * ND : 1) == i) {
+        load(q);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    mul(i);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int I>
+struct Int {
+  static constexpr int value = I;
+};
+template <int R, typename F>
+__device__ __forceinline__ void last_steps(F& step, int it, int buf) {
+  buf = step(Int<R>{}, it, buf);
+  if constexpr (R > 0) last_steps<R - 1>(step, it + 1, buf);
+}
+
+template <int BM, int BN, int WM, int WN, int NS, int MODE>
+__global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
+    const Args a) {
+  constexpr bool GLU = MODE == SWIGLU;
+  constexpr int NW = WM * WN;
+  // 16-row tiles of a wave: features, rows of x, the halves of these
+  constexpr int FN = BN / WN / 16, FM = BM / WM / 16;
+  constexpr int H0 = FM / 2, H1 = FM - H0;
+  // A stage in LDS: W, the first halves of all waves' rows of x, the second
+  constexpr int X0 = H0 * 16 * WM, X1 = H1 * 16 * WM;
+  constexpr int AT_X0 = BN * ROW, AT_X1 = AT_X0 + X0 * ROW;
+  constexpr int STAGE = (BN + BM) * ROW;
+  // loads of 8 rows a wave: of W, of the first halves, of the second ones
+  constexpr int PW = BN / 8 / NW, P0 = X0 / 8 / NW, P1 = X1 / 8 / NW;
+  static_assert(PW * NW * 8 == BN && P0 * NW * 8 == X0 && P1 * NW * 8 == X1 &&
+                H0 > 0 && NW % 4 == 0 && (!GLU || FN % 2 == 0), "");
+  constexpr int PA = PW + P0, P = PA + P1;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int lane = threadIdx.x & 63;
+  const int wid = uni(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int wm = wid / WN, wn = wid % WN;
+
+  // Consecutive workgroups go to the 8 XCDs in turn: each XCD takes a run of
+  // tiles, rows first in groups of 4 or 8, so that its L2 serves W and x to many
+  // (8192 x 8192 x 8192: groups of 1 1149 us, 2 858, 4 824, 8 844, 32 1024).
+  constexpr int GROUP = BM >= 192 ? 4 : 8;
+  const int per = a.tiles * a.mtiles, total = per * a.splits;
+  int id = blockIdx.x;
+  {
+    const int q = total / 8, r = total % 8, xcd = id % 8;
+    id = xcd * q + min(xcd, r) + id / 8;
+  }
+  const int split = uni(id / per);
+  id -= split * per;
+  const int group = id / (GROUP * a.tiles);
+  const int high = min(GROUP, a.mtiles - GROUP * group);
+  id -= group * GROUP * a.tiles;
+  const int mt = uni(GROUP * group + id % high);
+  int nt = uni(id / high);
+  int layer = 0;
+  if (!GLU) {
+    while (nt >= a.tile_end[layer]) ++layer;
+    if (layer) nt -= a.tile_end[layer - 1];
+  }
+  const int N = a.n[layer], K = a.K;
+  const int n0 = nt * (GLU ? BN / 2 : BN), m0 = mt * BM;
+  const int steps = K / BK;
+  const int s0 = uni(split * steps / a.splits);
+  const int n_it = uni((split + 1) * steps / a.splits) - s0;    // NS or more
+
+  // The lane's place in each load: rows past the end repeat the last one.
+  unsigned off[P];
+  const int lr = lane >> 3, lc = lane & 7;
+#pragma unroll
+  for (int j = 0; j < P; ++j) {
+    int r;
+    if (j < PW) {
+      const int row = (j * NW + wid) * 8 + lr;
+      r = min(n0 + (GLU ? (row >> 5) * 16 + (row & 15) : row), N - 1) - n0;
+    } else {
+      constexpr int C0 = H0 * 16, C1 = H1 * 16;
+      const int row = ((j < PA ? j - PW : j - PA) * NW + wid) * 8 + lr;
+      const int c = j < PA ? C0 : C1;
+      r = row / c * (BM / WM) + row % c + (j < PA ? 0 : C0);
+      r = min(m0 + r, a.M - 1) - m0;
+    }
+    off[j] = (unsigned)r * K * 2 + ((lc ^ lr) << 4);
+  }
+  const short* w = GLU ? (wid & 2 ? a.w[1] : a.w[0]) : a.w[layer];
+  const char* wb = uni((const char*)(w + (long long)n0 * K + s0 * BK));
+  const char* xb = uni((const char*)(a.x + (long long)m0 * K + s0 * BK));
+  const int lds0 =
+      (int)(uintptr_t)(__attribute__((address_space(3))) char*)lds + wid * 1024;
+  // load j of a stage: W, the first halves (A, j < PA), the second ones
+  auto fetch = [&](int it, int buf, int j) {
+    const int at = j < PW ? j * NW * 1024 : j < PA
+        ? AT_X0 + (j - PW) * NW * 1024 : AT_X1 + (j - PA) * NW * 1024;
+    load_lds((j < PW ? wb : xb) + (long long)it * ROW, off[j], lds0 + buf + at);
+  };
+
+  f32x4 acc[FN][FM];
+#pragma unroll
+  for (int f = 0; f < FN; ++f)
+#pragma unroll
+    for (int m = 0; m < FM; ++m) acc[f][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int i = 0; i < NS; ++i)
+#pragma unroll
+    for (int j = 0; j < (i < NS - 1 ? P : PA); ++j) fetch(i, i * STAGE, j);
+  wait_loads<(NS - 1) * P>();
+  barrier();
+
+  const int o0 = (g ^ (col & 7)) << 4, o1 = o0 ^ 64;
+  const char* wl = lds + (wn * (BN / WN) + col) * ROW;
+  const char* x0l = lds + AT_X0 + (wm * H0 * 16 + col) * ROW;
+  const char* x1l = lds + AT_X1 + (wm * H1 * 16 + col) * ROW;
+  s16x8 wa[2][FN], x0[2][H0], x1[2][H1];
+  auto tile_of = [](const char* p, int i) {
+    return *(const s16x8*)(p + i * 16 * ROW);
+  };
+#pragma unroll
+  for (int f = 0; f < FN; ++f) wa[0][f] = tile_of(wl + o0, f);
+#pragma unroll
+  for (int m = 0; m < H0; ++m) x0[0][m] = tile_of(x0l + o0, m);
+
+  // Loads of A of stage it + NS in three parts behind the stage's first barrier
+  // (by then all waves have read A), those of the second halves of it - 1 + NS
+  // before it. R: stages left after this one, NS for "at least NS".
+  constexpr int A1 = (PA + 2) / 3, A2 = A1 + (PA - A1 + 1) / 2;
+  auto step = [&](auto left, int it, int buf) {
+    constexpr int R = decltype(left)::value;
+    const int prev = buf == 0 ? (NS - 1) * STAGE : buf - STAGE;
+    const int next = buf == (NS - 1) * STAGE ? 0 : buf + STAGE;
+    phase<H0 * FN, FN + H0, (R >= NS - 1 ? P1 : 0)>(
+        [&](int i) {
+          acc[i % FN][i / FN] =
+              mfma(wa[0][i % FN], x0[0][i / FN], acc[i % FN][i / FN]);
+        },
+        [&](int q) {
+          if (q < FN) wa[1][q] = tile_of(wl + buf + o1, q);
+          else x0[1][q - FN] = tile_of(x0l + buf + o1, q - FN);
+        },
+        [&](int q) { fetch(it - 1 + NS, prev, PA + q); });
+    // the second halves of this stage have arrived
+    wait_loads<(R < NS - 1 ? R : NS - 1) * P>();
+    barrier();
+    phase<H0 * FN, H1, (R >= NS ? A1 : 0)>(
+        [&](int i) {
+          acc[i % FN][i / FN] =
+              mfma(wa[1][i % FN], x0[1][i / FN], acc[i % FN][i / FN]);
+        },
+        [&](int q) { x1[0][q] = tile_of(x1l + buf + o0, q); },
+        [&](int q) { fetch(it + NS, buf, q); });
+    phase<H1 * FN, H1, (R >= NS ? A2 - A1 : 0)>(
+        [&](int i) {
+          acc[i % FN][i / FN + H0] =
+              mfma(wa[0][i % FN], x1[0][i / FN], acc[i % FN][i / FN + H0]);
+        },
+        [&](int q) { x1[1][q] = tile_of(x1l + buf + o1, q); },
+        [&](int q) { fetch(it + NS, buf, A1 + q); });
+    // A of the next stage has arrived
+    if constexpr (R >= NS) wait_loads<(NS - 2) * P + P1 + A2>();
+    else if constexpr (R > 0) wait_loads<(R - 1) * P + P1>();
+    barrier();
+    phase<H1 * FN, (R > 0 ? FN + H0 : 0), (R >= NS ? PA - A2 : 0)>(
+        [&](int i) {
+          acc[i % FN][i / FN + H0] =
+              mfma(wa[1][i % FN], x1[1][i / FN], acc[i % FN][i / FN + H0]);
+        },
+        [&](int q) {
+          if (q < FN) wa[0][q] = tile_of(wl + next + o0, q);
+          else x0[0][q - FN] = tile_of(x0l + next + o0, q - FN);
+        },
+        [&](int q) { fetch(it + NS, buf, A2 + q); });
+    return next;
+  };
+  int it = 0, buf = 0;
+  for (; it + NS < n_it; ++it) buf = step(Int<NS>{}, it, buf);
+  last_steps<NS - 1>(step, it, buf);
+
+  // lane: row col of a tile of x, features 4 g + r of a tile of W
+  if constexpr (!GLU && BN >= 192) {
+    // Through LDS, so that whole lines are stored (8192 x 8192 x 4096: 10 us
+    // less; narrower tiles gain nothing).
+    if (a.splits == 1 && N % 8 == 0) {
+      constexpr int RB = BN * 2 + 16;               // bytes a row
+      constexpr int PASS = (BM * RB + NS * STAGE - 1) / (NS * STAGE);
+      constexpr int MP = (FM + PASS - 1) / PASS;    // tiles of a wave a pass
+      constexpr int VPR = BN / 8;                   // vectors a row
+      static_assert(WM * MP * 16 * RB <= NS * STAGE, "");
+#pragma unroll
+      for (int p = 0; p < PASS; ++p) {
+        barrier();
+#pragma unroll
+        for (int i = 0; i < MP; ++i) {
+          const int m = p * MP + i;
+          if (m >= FM) break;
+          char* row = lds + ((wm * MP + i) * 16 + col) * RB;
+#pragma unroll
+          for (int f = 0; f < FN; ++f) {
+            const int n = (wn * FN + f) * 16 + 4 * g;
+            f32x4 y = acc[f][m];
+            if (n0 + n < N) y = add_bias(y, a.bias[layer], n0 + n);
+            *(s16x4*)(row + n * 2) = packed(y);
+          }
+        }
+        barrier();
+        for (int i = threadIdx.x; i < WM * MP * 16 * VPR; i += NW * 64) {
+          const int at = i / VPR, n = n0 + i % VPR * 8;
+          const int mr = at % (MP * 16) + p * MP * 16;
+          const int r = m0 + at / (MP * 16) * (BM / WM) + mr;
+          if (mr >= FM * 16 || r >= a.M || n >= N) continue;
+          *(s16x8*)(a.out[layer] + (long long)r * N + n) =
+              *(const s16x8*)(lds + at * RB + i % VPR * 16);
+        }
+      }
+      return;
+    }
+  }
+  const int all = a.n_end[a.layers - 1];
+#pragma unroll
+  for (int m = 0; m < FM; ++m) {
+    const int r = m0 + wm * (BM / WM) + 16 * m + col;
+    if (r >= a.M) continue;
+    if constexpr (GLU) {
+#pragma unroll
+      for (int f = 0; f < FN; f += 2) {
+        const int n = n0 + (wn * FN + f) * 8 + 4 * g;
+        if (n >= N) continue;
+        const f32x4 y = add_bias(acc[f][m], a.bias[0], n);
+        f32x4 o = add_bias(acc[f + 1][m], a.bias[1], n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] *= y[e] / (1.f + expf(-y[e]));
+        *(s16x4*)(a.out[0] + (long long)r * N + n) = packed(o);
+      }
+    } else {
+#pragma unroll
+      for (int f = 0; f < FN; ++f) {
+        const int n = n0 + (wn * FN + f) * 16 + 4 * g;
+        if (n >= N) continue;
+        if (a.splits > 1)
+          *(f32x4*)(a.part + ((long long)split * a.M + r) * all +
+                    (layer ? a.n_end[layer - 1] : 0) + n) = acc[f][m];
+        else
+          *(s16x4*)(a.out[layer] + (long long)r * N + n) =
+              packed(add_bias(acc[f][m], a.bias[layer], n));
+      }
+    }
+  }
+}
+
+// Adds the splits up: four features of a row a thread.
+__global__ __launch_bounds__(256) void tile_merge_kernel(const Args a) {
+  const int all = a.n_end[a.layers - 1];
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long long)a.M * (all / 4)) return;
+  const int r = (int)(i / (all / 4)), n = (int)(i % (all / 4)) * 4;
+  f32x4 y = {0.f, 0.f, 0.f, 0.f};
+  const float* p = a.part + (long long)r * all + n;
+#pragma unroll 4
+  for (int s = 0; s < a.splits; ++s)
+    y += *(const f32x4*)(p + (long long)s * a.M * all);
+  int l = 0;
+  while (n >= a.n_end[l]) ++l;
+  const int at = n - (l ? a.n_end[l - 1] : 0);
+  *(s16x4*)(a.out[l] + (long long)r * a.n[l] + at) =
+      packed(add_bias(y, a.bias[l], at));
+}
+
+template <int BM, int BN, int WM, int WN, int NS, int MODE>
+int launch(Args a, hipStream_t st) {
+  constexpr int LDS = NS * (BM + BN) * ROW;
+  static_assert(LDS <= 160 * 1024, "");
+  const int bn = MODE == SWIGLU ? BN / 2 : BN;
+  int tiles = 0;
+  for (int i = 0; i < (MODE == SWIGLU ? 1 : a.layers); ++i)
+    a.tile_end[i] = tiles += (a.n[i] + bn - 1) / bn;
+  a.tiles = tiles;
+  a.mtiles = (a.M + BM - 1) / BM;
+  auto kernel = tile_linear_kernel<BM, BN, WM, WN, NS, MODE>;
+  const hipError_t e = hipFuncSetAttribute(
+      (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL(kernel, dim3(tiles * a.mtiles * a.splits),
+                     dim3(WM * WN * 64), LDS, st, a);
+  if (a.splits > 1) {
+    const long long q = (long long)a.M * (a.n_end[a.layers - 1] / 4);
+    hipLaunchKernelGGL(tile_merge_kernel, dim3((unsigned)((q + 255) / 256)),
+                       dim3(256), 0, st, a);
+  }
+  return (int)hipGetLastError();
+}
+
+// number, BM, BN, waves along rows and features, stages in LDS; us a stage and
+// a tile of a chip full of them (fitted to 20 layers of 1024 x 1024 to 128256 x
+// 4096 and 33 to 8192 rows; root mean square error 6%). The largest make the
+// most products of what they load, the smaller ones fill the chip with fewer
+// rows or features. 256 x 192 has waves of three tiles of features: no gates.
+#define TILES(X)                           \
+  X(0, 64, 64, 2, 2, 8, 0.280f, 1.7f)      \
+  X(1, 64, 128, 2, 2, 6, 0.405f, 2.4f)     \
+  X(2, 128, 64, 4, 2, 6, 0.349f, 2.3f)     \
+  X(3, 128, 128, 4, 2, 5, 0.523f, 3.7f)    \
+  X(4, 128, 256, 2, 4, 3, 0.807f, 6.3f)    \
+  X(5, 192, 128, 4, 2, 4, 0.646f, 4.8f)    \
+  X(6, 192, 256, 4, 2, 2, 1.060f, 7.5f)    \
+  X(7, 256, 128, 4, 2, 3, 0.790f, 5.7f)    \
+  X(8, 256, 192, 2, 4, 2, 1.038f, 7.0f)    \
+  X(9, 256, 256, 2, 4, 2, 1.342f, 8.4f)
+
+struct Tile {
+  int bm, bn, stages;
+  bool gates;
+  float stage, fixed;
+};
+const Tile tiles_[] = {
+#define X(I, BM, BN, WM, WN, NS, U, F) \
+  {BM, BN, NS, BN / WN / 16 % 2 == 0, U, F},
+    TILES(X)
+#undef X
+};
+
+// us that a tile and a number of splits take: rounds of the 256 CUs (the last
+// one, in part empty, runs faster: less power, less traffic) or W and x from
+// memory at 4.15 TB/s, whichever is longer, then adding the splits up.
+float estimate(const Tile& t, const int* n, int layers, int M, int K, int mode,
+               int splits) {
+  const int bn = mode == SWIGLU ? t.bn / 2 : t.bn;
+  double tiles = 0, all = 0;
+  for (int i = 0; i < layers; ++i) {
+    if (mode != SWIGLU || i == 0) tiles += (n[i] + bn - 1) / bn;
+    all += n[i];
+  }
+  tiles *= (double)((M + t.bm - 1) / t.bm) * splits;
+  const double whole = (double)(long long)(tiles / 256);
+  const double rest = tiles / 256 - whole;
+  double us = (whole + (rest > 0 ? 0.76 + 0.24 * rest : 0)) *
+      (K / BK / (double)splits * t.stage + t.fixed);
+  double mem = (all * K + (double)M * (K + all)) * 2 / 4.15e6;
+  us *= us * us;
+  mem *= mem * mem;
+  us = cbrt(sqrt(us * us + mem * mem));
+  if (splits > 1) us += 2.7 + 0.296e-6 * splits * M * all * 4;
+  return (float)us;
+}
+
+}  // namespace
+
+// The tile for 1..3 weights on one input and the splits of the contraction, by
+// ``estimate``: over those layers and rows within 1% of the fastest on average,
+// 23% at worst. Each split needs the ring's stages. -1: no tile for this K.
+extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
+                                   int mode, int* splits) {
+  static const int some[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+  int best = -1;
+  float least = 0;
+  for (int i = 0; i < (int)(sizeof(tiles_) / sizeof(Tile)); ++i) {
+    const Tile& t = tiles_[i];
+    if (mode == SWIGLU && !t.gates) continue;
+    long long tiles = 0;
+    for (int l = 0; l < layers; ++l) tiles += (n[l] + t.bn - 1) / t.bn;
+    tiles *= (M + t.bm - 1) / t.bm;
+    for (int s : some) {
+      if (s > 1 && (mode == SWIGLU || tiles * s > 520)) break;
+      if (K / BK / s < t.stages) break;
+      const float us = estimate(t, n, layers, M, K, mode, s);
+      if (best < 0 || us < least) {
+        best = i;
+        least = us;
+        *splits = s;
+      }
+    }
+  }
+  return best;
+}
+
+// Stages of inputs that a split has to hold at least; 0: no such tile.
+extern "C" int ds_tile_linear_stages(int tile, int mode) {
+  if (tile < 0 || tile >= (int)(sizeof(tiles_) / sizeof(Tile))) return 0;
+  return mode == SWIGLU && !tiles_[tile].gates ? 0 : tiles_[tile].stages;
+}
+
+// K is a multiple of 64, every n of four, x and every w lie at 16 bytes; mode 1:
+// silu(layer 0) * layer 1. tile and splits from the plan; part: splits * M * all
+// features, null for one split. Returns a hipError_t.
+extern "C" int ds_tile_linear(const void* x, int layers, const void* const* w,
+                              const void* const* bias, void* const* out,
+                              const int* n, int M, int K, int mode, int tile,
+                              int splits, float* part, void* stream) {
+  Args a = {};
+  int total = 0;
+  for (int i = 0; i < layers; ++i) {
+    a.w[i] = (const short*)w[i];
+    a.bias[i] = (const short*)bias[i];
+    a.out[i] = (short*)out[i];
+    a.n[i] = n[i];
+    a.n_end[i] = total += n[i];
+  }
+  a.x = (const short*)x;
+  a.part = part;
+  a.M = M; a.K = K; a.layers = layers; a.splits = splits;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  switch (tile) {
+#define X(I, BM, BN, WM, WN, NS, U, F)                                    \
+  case I:                                                                 \
+    if (mode == SWIGLU)                                                   \
+      return launch<BM, BN, WM, WN, NS,                                   \
+                    BN / WN / 16 % 2 == 0 ? SWIGLU : PLAIN>(a, st);       \
+    return launch<BM, BN, WM, WN, NS, PLAIN>(a, st);
+    TILES(X)
+#undef X
+  }
+  return (int)hipErrorInvalidValue;
+}

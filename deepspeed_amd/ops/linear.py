@@ -3,15 +3,14 @@
 ``Linear`` is torch's, with a backward whose products read their operands along
 the contiguous axis (see ``_Linear``).
 
-``rows_linear``, for a few rows (decoding): the weight-streaming kernel of
-csrc/rows_linear.hip in place of a library GEMM, with several layers of one
-input in one launch and the gate's activation in its epilogue. For up to 256 rows
-(many requests, short prompts) the kernel of csrc/batch_linear.hip where
-``batch_pays``.
+``rows_linear``, for a few rows (decoding), and ``tile_linear``, for any more:
+the framework's kernels (csrc/rows_linear.hip, csrc/tile_linear.hip) in place of
+a library GEMM, with several layers of one input in one launch and the gate's
+activation in the epilogue.
 
-It takes the modules themselves and returns None wherever calling them is the
+Both take the modules themselves and return None wherever calling them is the
 thing to do: with gradients, hooks, autocast, function transforms, tangents or
-traces, other types, sharded or replaced modules, or more rows than the kernel is the faster one for."""
+traces, other types, sharded or replaced modules."""
 
 import torch
 import torch.nn as nn
@@ -20,9 +19,8 @@ from torch.nn.modules import module as _module
 
 from ._loader import get_ext
 
-# Most rows for rows_linear.hip: at 64 the library's product takes half the
-# kernel's time (N 14336: 26.6 to 49.8 us); with int8 weights it needs them
-# dequantized first. Past them, up to BATCH, batch_linear.hip where it pays.
+# Most rows that ``rows_linear`` takes: bf16, int8 (past it the weights are
+# dequantized first), and bf16 where ``batch_pays``.
 ROWS, ROWS_INT8, BATCH = 32, 64, 256
 
 PLAIN, SWIGLU = 0, 1
@@ -188,18 +186,9 @@ def unhooked(mod: nn.Module, internal_ok: bool = False) -> bool:
 
 
 def batch_pays(ns, K: int) -> bool:
-    """Whether batch_linear.hip takes layers of ``ns`` features on one input, of
-    33 to 256 rows. Several layers: one launch that fills the chip in place of
-    products that leave it idle (us, library and kernel, at 64 and 224 rows:
-    4096 + 1024 + 1024, K 4096 44 / 21 and 47 / 36; 3 x 3072, K 3072 48 / 23 and
-    53 / 44; 3 x 5120, K 5120 65 / 43, 150 / 77 at 256; 8192 + 1024 + 1024, K
-    8192 60 / 41 and 111 / 98). One layer: where
-    the contraction is long and the library's product splits it badly (4096, K
-    14336 39 / 33, 60 / 59, 76 / 43 at 128; 3072, K 8192 24 / 21, 33 / 34, 43 /
-    27 at 128; 8192, K 28672 134 / 103, 257 / 198). The library is ahead where
-    its tiles fill the chip (14336 + 14336, K 4096 54 / 61, 91 / 98) and at
-    small or square layers (4096, K 4096 15 / 17, 23 / 25; 2048, K 4096 11 / 15,
-    16 / 21)."""
+    """Whether ``rows_linear`` takes layers of ``ns`` features on one input of 33
+    to 256 rows: several layers of moderate size, and one with a long
+    contraction. Others are for ``tile_linear``."""
     if any(n % 4 for n in ns):
         return False
     if len(ns) > 1:
@@ -253,4 +242,47 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
     if x2.data_ptr() % 16:
         return None
     out = get_ext().rows_linear(x2, weights, scales, biases, group, mode)
+    return [o.view(*x.shape[:-1], o.shape[-1]) for o in out]
+
+
+def tile_linear(x: torch.Tensor, mods, mode: int = PLAIN):
+    """``rows_linear`` for more than ``ROWS`` rows and torch's or the models' own
+    bf16 layers. Over 20 layers of 1024 x 1024 to 128256 x 4096 and 33 to 8192
+    rows the kernel takes 0.65 of the library's time in the geometric mean (us,
+    library and kernel: gate and up 14336, K 4096, 224 rows 95 + activation / 67;
+    4096, K 14336, 1024 rows 138 / 108; 3584, K 18944, 2331 rows 489 / 302).
+
+    One plain layer of many rows stays the library's: its products of whole
+    rounds of tiles reach 5% more (4096 rows: N 4096, K 4096 91 / 98; N 4096, K
+    14336 304 / 324; N 128256 2930 / 3060; elsewhere 3300 rows: N 4096, K 14336
+    343 / 305), but for contractions from 16384 on (3584, K 18944: 4096 rows 540
+    / 418, 5000 958 / 658)."""
+    if type(x) is not torch.Tensor or torch.is_grad_enabled() or \
+            not x.is_cuda or x.dtype is not torch.bfloat16:
+        return None
+    K = x.shape[-1]
+    M = x.numel() // K if K else 0
+    if M <= ROWS or K % 64 or not 192 <= K <= 1 << 22 or (
+            M >= 2560 and len(mods) == 1 and K < 16384) or \
+            get_ext() is None or torch.is_autocast_enabled() or \
+            torch.compiler.is_compiling() or not untransformed():
+        return None
+    weights, biases = [], []
+    for m in mods:
+        if type(m) not in (Linear, nn.Linear) or not unhooked(m):
+            return None
+        w, b = m.weight, m.bias
+        if w.dtype is not torch.bfloat16 or type(w) is not nn.Parameter or \
+                w.shape[1:] != (K,) or w.shape[0] % 4 or not w.is_cuda or \
+                not w.is_contiguous() or w.data_ptr() % 16 or (
+                    mode == SWIGLU and w.shape != mods[0].weight.shape) or (
+                    b is not None and (b.dtype is not torch.bfloat16
+                                       or not b.is_contiguous())):
+            return None
+        weights.append(w)
+        biases.append(b)
+    x2 = x.reshape(M, K).contiguous()
+    if x2.data_ptr() % 16:
+        return None
+    out = get_ext().tile_linear(x2, weights, biases, mode)
     return [o.view(*x.shape[:-1], o.shape[-1]) for o in out]

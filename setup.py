@@ -31,7 +31,7 @@ ext = CUDAExtension(
         os.path.join(CSRC, "softmax_dropout.hip"),
         os.path.join(CSRC, "paged_attention.hip"),
         os.path.join(CSRC, "rows_linear.hip"),
-        os.path.join(CSRC, "batch_linear.hip"),
+        os.path.join(CSRC, "tile_linear.hip"),
         os.path.join(CSRC, "quantize.hip"),
         os.path.join(CSRC, "attention.hip"),
         os.path.join(CSRC, "cross_entropy.hip"),
