@@ -7,8 +7,8 @@ theta=500000, SwiGLU MLP, RMSNorm, tied-off lm_head).
 
 Hot ops: RMSNorm / RoPE / SwiGLU are the hand-written HIP kernels in
 ``deepspeed_amd.ops``, and so is attention (flash forward and backward, paged
-serving) wherever its kernels apply, else torch SDPA; linear layers of inference
-are ``ops.linear``'s kernels, GEMMs of training go through torch (hipBLASLt).
+serving) wherever its kernels apply, else torch SDPA; linear layers are
+``ops.linear``'s, with the library's products where these are faster.
 """
 
 from dataclasses import dataclass
@@ -18,8 +18,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ..ops.attention import rope_flash_attention
-from ..ops.linear import (SWIGLU, Linear, movable, rows_linear, tile_linear,
-                          unhooked)
+from ..ops.linear import (SWIGLU, Linear, call, movable, rows_linear,
+                          tile_linear, unhooked)
 from ..ops.norms import RMSNorm
 from ..ops.rope import apply_rope, rope_tables
 from ..ops.swiglu import swiglu
@@ -130,7 +130,7 @@ class LlamaAttention(nn.Module):
 
     def _out(self, o):
         y = rows_linear(o, (self.o_proj,)) or tile_linear(o, (self.o_proj,))
-        return self.o_proj(o) if y is None else y[0]
+        return call(self.o_proj, o) if y is None else y[0]
 
     def forward(self, x, cos, sin, positions=None, kv_cache=None,
                 attention_fn=None):
@@ -138,7 +138,7 @@ class LlamaAttention(nn.Module):
         mods = self.q_proj, self.k_proj, self.v_proj
         qkv = rows_linear(x, mods) or tile_linear(x, mods)
         if qkv is None:
-            qkv = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+            qkv = [call(m, x) for m in mods]
         q = qkv[0].view(B, S, self.num_heads, self.head_dim)
         k = qkv[1].view(B, S, self.num_kv_heads, self.head_dim)
         v = qkv[2].view(B, S, self.num_kv_heads, self.head_dim)
@@ -248,10 +248,11 @@ class LlamaMLP(nn.Module):
     def forward(self, x):
         mods = self.gate_proj, self.up_proj
         h = rows_linear(x, mods, SWIGLU) or tile_linear(x, mods, SWIGLU)
-        h = swiglu(self.gate_proj(x), self.up_proj(x)) if h is None else h[0]
+        if h is None:
+            h = [swiglu(*(tile_linear(x, mods) or [call(m, x) for m in mods]))]
         mods = self.down_proj,
-        y = rows_linear(h, mods) or tile_linear(h, mods)
-        return self.down_proj(h) if y is None else y[0]
+        y = rows_linear(h[0], mods) or tile_linear(h[0], mods)
+        return call(self.down_proj, h[0]) if y is None else y[0]
 
 
 def add_norm(norm, x, delta):
@@ -353,7 +354,7 @@ class LlamaForCausalLM(nn.Module):
             return chunked_cross_entropy(hidden, self.lm_head, labels)
         mods = self.lm_head,
         logits = rows_linear(hidden, mods) or tile_linear(hidden, mods)
-        return self.lm_head(hidden) if logits is None else logits[0]
+        return call(self.lm_head, hidden) if logits is None else logits[0]
 
     def num_parameters(self):
         return sum(p.numel() for p in self.parameters())
@@ -373,7 +374,7 @@ def chunked_cross_entropy(hidden, lm_head, labels, chunk_tokens=8192):
     count = hidden.new_zeros((), dtype=torch.float32)
     for s in range(0, n, chunk_tokens):
         e = min(s + chunk_tokens, n)
-        logits = lm_head(hidden[s:e])
+        logits = call(lm_head, hidden[s:e])
         l, c = fused_cross_entropy_sum(logits, labels[s:e])
         total = total + l
         count = count + c

@@ -103,10 +103,11 @@ extern "C" void ds_rows_linear(const void* x, int layers, const void* const* w,
 extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
                                    int mode, int* splits);
 extern "C" int ds_tile_linear_stages(int tile, int mode);
-extern "C" int ds_tile_linear(const void* x, int layers, const void* const* w,
-                              const void* const* bias, void* const* out,
-                              const int* n, int M, int K, int mode, int tile,
-                              int splits, float* part, void* stream);
+extern "C" int ds_tile_linear(const void* const* x, int layers,
+                              const void* const* w, const void* const* bias,
+                              void* const* out, const int* n, int M, int K,
+                              int mode, int tile, int splits, float* part,
+                              void* stream);
 extern "C" void ds_transpose_bf16(const void* src, void* dst, int n_batch,
                                   int R, int C, long long row_stride,
                                   int inner, long long inner_stride,
@@ -525,9 +526,10 @@ struct Layers {
     at::Tensor part;
     if (splits > 1)
       part = at::empty({splits * M * all}, x.options().dtype(at::kFloat));
+    const void* xs[1] = {x.data_ptr()};
     const int e = ds_tile_linear(
-        x.data_ptr(), count, w, b, o, n, (int)M, (int)K, (int)mode, tile,
-        splits, splits > 1 ? part.data_ptr<float>() : nullptr, cur_stream());
+        xs, count, w, b, o, n, (int)M, (int)K, (int)mode, tile, splits,
+        splits > 1 ? part.data_ptr<float>() : nullptr, cur_stream());
     TORCH_CHECK(e == 0, "tile_linear: launch failed with error ", e);
     return true;
   }
@@ -603,6 +605,76 @@ std::vector<at::Tensor> tile_linear(
   TORCH_CHECK(y.tiled(x, mode, (int)tile, (int)splits),
               "tile_linear: features in fours, inputs in 64s, 192 or more");
   return y.out;
+}
+
+// Gradients of linear layers y = x W^T on one input, bf16 (tile_linear.hip). mode
+// 2: of the input, the sum over the layers of dy W; mode 3: of each weight, dy^T
+// x. others: the weights, or the input alone.
+std::vector<at::Tensor> tile_linear_grad(const std::vector<at::Tensor>& dys,
+                                         const std::vector<at::Tensor>& others,
+                                         int mode, int tile, int splits) {
+  const int L = dys.size();
+  TORCH_CHECK(L >= 1 && L <= 3 && (int)others.size() == (mode == 2 ? L : 1),
+              "tile_linear_grad: layers");
+  const OneDevice on("tile_linear_grad", dys[0]);
+  for (auto& t : dys) on.check(t);
+  for (auto& t : others) on.check(t);
+  const int64_t M = dys[0].size(0), K = others[0].size(1);
+  const void *x[3], *w[3], *b[3] = {};
+  void* o[3];
+  int n[3];
+  int64_t all = 0;
+  auto good = [](const at::Tensor& t) {
+    return t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() == 2 &&
+        t.is_contiguous() && t.numel() > 0 &&
+        ((uintptr_t)t.data_ptr() & 15) == 0;
+  };
+  std::vector<at::Tensor> out;
+  for (int i = 0; i < L; ++i) {
+    const auto& other = others[mode == 2 ? i : 0];
+    TORCH_CHECK(good(dys[i]) && good(other) && dys[i].size(0) == M &&
+                other.size(1) == K &&
+                other.size(0) == (mode == 2 ? dys[i].size(1) : M) &&
+                dys[i].size(1) < (1 << 30) && K % 8 == 0 &&
+                dys[i].size(1) % (mode == 2 ? 64 : 8) == 0,
+                "tile_linear_grad: operands");
+    x[i] = dys[i].data_ptr();
+    w[i] = other.data_ptr();
+    n[i] = dys[i].size(1);
+    all += n[i];
+    if (mode == 3 || i == 0)
+      out.push_back(at::empty({mode == 2 ? M : n[i], K}, dys[0].options()));
+    o[i] = out.back().data_ptr();
+  }
+  TORCH_CHECK(K <= (1 << 22) && M < (1 << 30) && all < (1ll << 31),
+              "tile_linear_grad: size");
+  if (tile < 0)
+    tile = ds_tile_linear_plan(n, L, (int)M, (int)K, mode, &splits);
+  const int stages = ds_tile_linear_stages(tile, mode);
+  const int64_t steps = mode == 2 ? all / 64 : (M + 63) / 64;
+  TORCH_CHECK(stages > 0 && splits > 0 && steps / splits >= stages,
+              "tile_linear_grad: too little to add up");
+  at::Tensor part;
+  if (splits > 1)
+    part = at::empty({splits * (mode == 2 ? M : all) * K},
+                     dys[0].options().dtype(at::kFloat));
+  const int e = ds_tile_linear(
+      x, L, w, b, o, n, (int)M, (int)K, mode, tile, splits,
+      splits > 1 ? part.data_ptr<float>() : nullptr, cur_stream());
+  TORCH_CHECK(e == 0, "tile_linear_grad: launch failed with error ", e);
+  return out;
+}
+
+at::Tensor tile_linear_dx(std::vector<at::Tensor> dys,
+                          std::vector<at::Tensor> weights, int64_t tile,
+                          int64_t splits) {
+  return tile_linear_grad(dys, weights, 2, (int)tile, (int)splits)[0];
+}
+
+std::vector<at::Tensor> tile_linear_dw(at::Tensor x,
+                                       std::vector<at::Tensor> dys,
+                                       int64_t tile, int64_t splits) {
+  return tile_linear_grad(dys, {x}, 3, (int)tile, (int)splits);
 }
 
 at::Tensor sum_of_squares(std::vector<at::Tensor> ts) {
@@ -1040,6 +1112,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_linear", &tile_linear, "linear layers of many rows, bf16",
         py::arg("x"), py::arg("weights"), py::arg("biases"), py::arg("mode"),
         py::arg("tile") = -1, py::arg("splits") = 1);
+  m.def("tile_linear_dx", &tile_linear_dx,
+        "input's gradient, summed over linear layers", py::arg("dys"),
+        py::arg("weights"), py::arg("tile") = -1, py::arg("splits") = 1);
+  m.def("tile_linear_dw", &tile_linear_dw, "weights' gradients",
+        py::arg("x"), py::arg("dys"), py::arg("tile") = -1,
+        py::arg("splits") = 1);
   m.def("sum_of_squares", &sum_of_squares,
         "sum of squares over a list of tensors");
   m.def("paged_rows", &paged_rows,

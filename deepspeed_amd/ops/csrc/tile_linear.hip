@@ -1,6 +1,6 @@
 // Linear layers of many rows for MI355X (gfx950): y = x W^T, x [M, K] bf16,
 // W [N, K] bf16, M past what rows_linear.hip takes: decoding for many requests,
-// portions of prompts, whole prompts.
+// portions of prompts, whole prompts; and both gradients of training.
 //
 // Reference analogue: the GEMMs of inference/v2/kernels/core_ops/blas_kernels
 // and the gated ones of core_ops/gated_activations.
@@ -38,23 +38,34 @@ typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int MAXL = 3;     // layers a launch
 constexpr int BK = 64;      // inputs a stage
 constexpr int ROW = BK * 2; // bytes of a row of a stage
 
-enum { PLAIN = 0, SWIGLU = 1 };
+// on lambdas: one that is not inlined takes what it captures to scratch memory
+#define INLINE __attribute__((always_inline))
 
+// y = x W^T, silu(x W0^T) * (x W1^T), and of y = x W^T the gradients of x, a sum
+// over the layers, and of each W.
+enum { PLAIN = 0, SWIGLU = 1, GRAD_X = 2, GRAD_W = 3 };
+
+// Operands by their place in the kernel: "w" brings the columns of an output,
+// "x" its rows. GRAD_X: w are the weights [n, K], x the gradients dy [M, n], and
+// the contraction runs over the features of one layer after the other. GRAD_W: w
+// is the layers' input [M, K], x the gradients, contracted over M.
 struct Args {
   const short* w[MAXL];
+  const short* x[MAXL];
   const short* bias[MAXL];
   short* out[MAXL];
-  int n[MAXL];          // features, multiples of four
-  int tile_end[MAXL];   // tiles of features up to and with a layer
-  int n_end[MAXL];      // features up to and with a layer
-  const short* x;
-  float* part;          // [splits, M, all features], splits > 1
-  int M, K, layers, tiles, mtiles, splits;
+  int n[MAXL];          // features
+  int n_end[MAXL];      // up to and with a layer: features,
+  int tile_end[MAXL];   // tiles of the outputs' columns, or GRAD_W of its rows,
+  int step_end[MAXL];   // and GRAD_X: stages
+  float* part;          // [splits, rows, columns] of all outputs, splits > 1
+  int M, K, layers, tiles, mtiles, splits, steps;
 };
 
 __device__ __forceinline__ f32x4 mfma(s16x8 a, s16x8 b, f32x4 c) {
@@ -105,6 +116,11 @@ __device__ __forceinline__ void barrier() {   // and what was read from LDS
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+__device__ __forceinline__ s16x4 tr_read(const char* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s16x4*)p);
+}
+
 // MT products with NR reads from LDS in their first half and ND loads spread
 // over all of them.
 template <int MT, int NR, int ND, typename Mul, typename Read, typename Load>
@@ -129,6 +145,12 @@ __device__ __forceinline__ void phase(Mul mul, Read read, Load load) {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// By value: choosing among a lambda's captures would keep them in memory.
+template <typename T>
+__device__ __forceinline__ T pick(int i, T a, T b, T c) {
+  return i == 2 ? c : i == 1 ? b : a;
+}
+
 template <int I>
 struct Int {
   static constexpr int value = I;
@@ -143,18 +165,22 @@ template <int BM, int BN, int WM, int WN, int NS, int MODE>
 __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
     const Args a) {
   constexpr bool GLU = MODE == SWIGLU;
+  // operands that lie across the contraction
+  constexpr bool WT = MODE == GRAD_X || MODE == GRAD_W, XT = MODE == GRAD_W;
   constexpr int NW = WM * WN;
   // 16-row tiles of a wave: features, rows of x, the halves of these
   constexpr int FN = BN / WN / 16, FM = BM / WM / 16;
   constexpr int H0 = FM / 2, H1 = FM - H0;
+  constexpr int C0 = H0 * 16, C1 = H1 * 16;
   // A stage in LDS: W, the first halves of all waves' rows of x, the second
-  constexpr int X0 = H0 * 16 * WM, X1 = H1 * 16 * WM;
+  constexpr int X0 = C0 * WM, X1 = C1 * WM;
   constexpr int AT_X0 = BN * ROW, AT_X1 = AT_X0 + X0 * ROW;
   constexpr int STAGE = (BN + BM) * ROW;
-  // loads of 8 rows a wave: of W, of the first halves, of the second ones
+  // loads of 1 KB a wave: of W, of the first halves, of the second ones
   constexpr int PW = BN / 8 / NW, P0 = X0 / 8 / NW, P1 = X1 / 8 / NW;
   static_assert(PW * NW * 8 == BN && P0 * NW * 8 == X0 && P1 * NW * 8 == X1 &&
-                H0 > 0 && NW % 4 == 0 && (!GLU || FN % 2 == 0), "");
+                H0 > 0 && NW % 4 == 0 && (!GLU || FN % 2 == 0) &&
+                (!XT || (X0 % 64 == 0 && X1 % 64 == 0)), "");
   constexpr int PA = PW + P0, P = PA + P1;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int lane = threadIdx.x & 63;
@@ -177,47 +203,95 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
   const int group = id / (GROUP * a.tiles);
   const int high = min(GROUP, a.mtiles - GROUP * group);
   id -= group * GROUP * a.tiles;
-  const int mt = uni(GROUP * group + id % high);
+  int mt = uni(GROUP * group + id % high);
   int nt = uni(id / high);
   int layer = 0;
-  if (!GLU) {
+  if (MODE == PLAIN) {
     while (nt >= a.tile_end[layer]) ++layer;
     if (layer) nt -= a.tile_end[layer - 1];
   }
-  const int N = a.n[layer], K = a.K;
+  if (MODE == GRAD_W) {
+    while (mt >= a.tile_end[layer]) ++layer;
+    if (layer) mt -= a.tile_end[layer - 1];
+  }
+  // rows and columns of the output, its tile's first ones
+  const int K = a.K, N = WT ? K : a.n[layer];
+  const int rows = MODE == GRAD_W ? a.n[layer] : a.M;
   const int n0 = nt * (GLU ? BN / 2 : BN), m0 = mt * BM;
-  const int steps = K / BK;
+  const int steps = MODE == GRAD_X ? a.steps
+      : MODE == GRAD_W ? (a.M + BK - 1) / BK : K / BK;
   const int s0 = uni(split * steps / a.splits);
   const int n_it = uni((split + 1) * steps / a.splits) - s0;    // NS or more
 
-  // The lane's place in each load: rows past the end repeat the last one.
+  // The lane's place in each load, which fills 1 KB: 8 rows of 64 inputs, or
+  // 8 inputs of 64 columns. Rows and columns past the end repeat the last ones;
+  // what comes of them is not stored.
+  //   Along the contraction: chunk c of row r lies at c ^ (r & 7).
+  //   Across it: blocks of 64 columns, [64 inputs][8 chunks], chunk c of input k
+  // at c ^ (2 bit 1 of k + 4 bit 3): a transposing read takes 4 inputs by 32
+  // bytes from each of four groups of 8 inputs, half of which share no bank.
   unsigned off[P];
   const int lr = lane >> 3, lc = lane & 7;
 #pragma unroll
   for (int j = 0; j < P; ++j) {
-    int r;
-    if (j < PW) {
-      const int row = (j * NW + wid) * 8 + lr;
-      r = min(n0 + (GLU ? (row >> 5) * 16 + (row & 15) : row), N - 1) - n0;
-    } else {
-      constexpr int C0 = H0 * 16, C1 = H1 * 16;
-      const int row = ((j < PA ? j - PW : j - PA) * NW + wid) * 8 + lr;
+    const bool of_w = j < PW;
+    const int piece = (of_w ? j : j < PA ? j - PW : j - PA) * NW + wid;
+    const bool t = of_w ? WT : XT;
+    const int h = 2 * ((lr >> 1) & 1) + 4 * (piece & 1);
+    int r = t ? piece / 8 * 64 + 8 * (lc ^ h) : piece * 8 + lr;
+    if (!of_w) {
       const int c = j < PA ? C0 : C1;
-      r = row / c * (BM / WM) + row % c + (j < PA ? 0 : C0);
-      r = min(m0 + r, a.M - 1) - m0;
+      r = r / c * (BM / WM) + r % c + (j < PA ? 0 : C0);
+    } else if (GLU) {
+      r = (r >> 5) * 16 + (r & 15);
     }
-    off[j] = (unsigned)r * K * 2 + ((lc ^ lr) << 4);
+    const int last = (of_w ? N - n0 : rows - m0) - (t ? 8 : 1);
+    r = min(r, last);
+    if (t) off[j] = 2 * r;
+    else if (MODE == GRAD_X) off[j] = r;    // its layer's stride comes later
+    else off[j] = (unsigned)r * K * 2 + ((lc ^ lr) << 4);
   }
-  const short* w = GLU ? (wid & 2 ? a.w[1] : a.w[0]) : a.w[layer];
-  const char* wb = uni((const char*)(w + (long long)n0 * K + s0 * BK));
-  const char* xb = uni((const char*)(a.x + (long long)m0 * K + s0 * BK));
+  const short* w = GLU ? (wid & 2 ? a.w[1] : a.w[0]) : a.w[MODE == PLAIN ? layer : 0];
+  const char* wb = uni((const char*)(w + (WT ? n0 : (long long)n0 * K)));
+  const char* xb = uni((const char*)(
+      a.x[MODE == GRAD_W ? layer : 0] +
+      (XT ? m0 : MODE == GRAD_X ? 0 : (long long)m0 * K)));
   const int lds0 =
       (int)(uintptr_t)(__attribute__((address_space(3))) char*)lds + wid * 1024;
+  // GRAD_X: where the layers begin and what is theirs
+  const int e0 = a.layers > 1 ? a.step_end[0] : 1 << 30;
+  const int e1 = a.layers > 2 ? a.step_end[1] : 1 << 30;
+  const int f0 = a.n[0], f1 = a.n[1], f2 = a.n[2];
+  const short *w0 = a.w[0], *w1 = a.w[1], *w2 = a.w[2];
+  const short *d0 = a.x[0], *d1 = a.x[1], *d2 = a.x[2];
   // load j of a stage: W, the first halves (A, j < PA), the second ones
-  auto fetch = [&](int it, int buf, int j) {
+  auto fetch = [&](int it, int buf, int j) INLINE {
     const int at = j < PW ? j * NW * 1024 : j < PA
         ? AT_X0 + (j - PW) * NW * 1024 : AT_X1 + (j - PA) * NW * 1024;
-    load_lds((j < PW ? wb : xb) + (long long)it * ROW, off[j], lds0 + buf + at);
+    const bool t = j < PW ? WT : XT;
+    const char* p = j < PW ? wb : xb;
+    unsigned o = off[j];
+    int step = s0 + it, ld = j < PW ? K : rows;
+    if (MODE == GRAD_X) {
+      const int l = (step >= e0) + (step >= e1);
+      step -= pick(l, 0, e0, e1);
+      if (j < PW) {
+        p = (const char*)(pick(l, w0, w1, w2) + n0);
+      } else {
+        ld = pick(l, f0, f1, f2);
+        p = (const char*)(pick(l, d0, d1, d2) + (long long)m0 * ld);
+      }
+    }
+    if (t) {
+      int k = ((j < PW ? j : j < PA ? j - PW : j - PA) * NW + wid) % 8 * 8 + lr;
+      if (MODE == GRAD_W) k = min(k, a.M - 1 - step * BK);
+      p += (long long)step * BK * ld * 2;
+      o += (unsigned)k * ld * 2;
+    } else {
+      if (MODE == GRAD_X) o = o * ld * 2 + ((lc ^ lr) << 4);
+      p += (long long)step * ROW;
+    }
+    load_lds(p, o, lds0 + buf + at);
   };
 
   f32x4 acc[FN][FM];
@@ -233,68 +307,111 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
   wait_loads<(NS - 1) * P>();
   barrier();
 
+  // 16 rows (or columns) by the inputs 32 h + 8 g + j, from tile i of a part of
+  // a stage on
   const int o0 = (g ^ (col & 7)) << 4, o1 = o0 ^ 64;
-  const char* wl = lds + (wn * (BN / WN) + col) * ROW;
-  const char* x0l = lds + AT_X0 + (wm * H0 * 16 + col) * ROW;
-  const char* x1l = lds + AT_X1 + (wm * H1 * 16 + col) * ROW;
+  const int tr0 = (8 * g + (col >> 2)) * 128 + (col & 3) * 8;
+  const int trh = 32 * ((col >> 3) & 1) + 64 * (g & 1);
+  auto read = [&](auto across, int part, int first, int i, int h) INLINE {
+    if constexpr (decltype(across)::value) {
+      const int c = first / 16 + i;
+      const char* p = lds + part + c / 4 * 8192 + h * 4096 +
+          (tr0 ^ trh ^ (c % 4 * 32));
+      const s16x4 lo = tr_read(p), hi = tr_read(p + 512);
+      return s16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    } else {
+      return *(const s16x8*)(lds + part + (first + col) * ROW +
+                             (h ? o1 : o0) + i * 16 * ROW);
+    }
+  };
+  const Int<WT> wt;
+  const Int<XT> xt;
   s16x8 wa[2][FN], x0[2][H0], x1[2][H1];
-  auto tile_of = [](const char* p, int i) {
-    return *(const s16x8*)(p + i * 16 * ROW);
+  auto get_w = [&](int buf, int i, int h) INLINE {
+    wa[h][i] = read(wt, buf, wn * (BN / WN), i, h);
+  };
+  auto get_x0 = [&](int buf, int i, int h) INLINE {
+    x0[h][i] = read(xt, buf + AT_X0, wm * C0, i, h);
+  };
+  auto get_x1 = [&](int buf, int i, int h) INLINE {
+    x1[h][i] = read(xt, buf + AT_X1, wm * C1, i, h);
+  };
+  // GRAD_W: inputs past the last one (of the last stage) count for nothing
+  const int beyond = MODE == GRAD_W && split == a.splits - 1
+      ? a.M - (steps - 1) * BK : BK;
+  auto cut = [&](s16x8& v, int h) INLINE {
+    u32x4 d = __builtin_bit_cast(u32x4, v);
+    const int left = beyond - 32 * h - 8 * g;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      d[e] &= left > 2 * e + 1 ? ~0u : left > 2 * e ? 0xffffu : 0u;
+    v = __builtin_bit_cast(s16x8, d);
   };
 #pragma unroll
-  for (int f = 0; f < FN; ++f) wa[0][f] = tile_of(wl + o0, f);
+  for (int f = 0; f < FN; ++f) get_w(0, f, 0);
 #pragma unroll
-  for (int m = 0; m < H0; ++m) x0[0][m] = tile_of(x0l + o0, m);
+  for (int m = 0; m < H0; ++m) get_x0(0, m, 0);
 
   // Loads of A of stage it + NS in three parts behind the stage's first barrier
   // (by then all waves have read A), those of the second halves of it - 1 + NS
   // before it. R: stages left after this one, NS for "at least NS".
   constexpr int A1 = (PA + 2) / 3, A2 = A1 + (PA - A1 + 1) / 2;
-  auto step = [&](auto left, int it, int buf) {
+  auto step = [&](auto left, int it, int buf) INLINE {
     constexpr int R = decltype(left)::value;
+    auto cut_last = [&](auto& of_w, int nw, auto& of_x, int nx,
+                        int h) INLINE {
+      if constexpr (MODE == GRAD_W && R == 0) {
+        for (int i = 0; i < nw; ++i) cut(of_w[i], h);
+        for (int i = 0; i < nx; ++i) cut(of_x[i], h);
+      }
+    };
     const int prev = buf == 0 ? (NS - 1) * STAGE : buf - STAGE;
     const int next = buf == (NS - 1) * STAGE ? 0 : buf + STAGE;
+    cut_last(wa[0], FN, x0[0], H0, 0);
     phase<H0 * FN, FN + H0, (R >= NS - 1 ? P1 : 0)>(
-        [&](int i) {
+        [&](int i) INLINE {
           acc[i % FN][i / FN] =
               mfma(wa[0][i % FN], x0[0][i / FN], acc[i % FN][i / FN]);
         },
-        [&](int q) {
-          if (q < FN) wa[1][q] = tile_of(wl + buf + o1, q);
-          else x0[1][q - FN] = tile_of(x0l + buf + o1, q - FN);
+        [&](int q) INLINE {
+          if (q < FN) get_w(buf, q, 1);
+          else get_x0(buf, q - FN, 1);
         },
-        [&](int q) { fetch(it - 1 + NS, prev, PA + q); });
+        [&](int q) INLINE { fetch(it - 1 + NS, prev, PA + q); });
     // the second halves of this stage have arrived
     wait_loads<(R < NS - 1 ? R : NS - 1) * P>();
     barrier();
+    cut_last(wa[1], FN, x0[1], H0, 1);
     phase<H0 * FN, H1, (R >= NS ? A1 : 0)>(
-        [&](int i) {
+        [&](int i) INLINE {
           acc[i % FN][i / FN] =
               mfma(wa[1][i % FN], x0[1][i / FN], acc[i % FN][i / FN]);
         },
-        [&](int q) { x1[0][q] = tile_of(x1l + buf + o0, q); },
-        [&](int q) { fetch(it + NS, buf, q); });
+        [&](int q) INLINE { get_x1(buf, q, 0); },
+        [&](int q) INLINE { fetch(it + NS, buf, q); });
+    cut_last(wa[0], 0, x1[0], H1, 0);
     phase<H1 * FN, H1, (R >= NS ? A2 - A1 : 0)>(
-        [&](int i) {
+        [&](int i) INLINE {
           acc[i % FN][i / FN + H0] =
               mfma(wa[0][i % FN], x1[0][i / FN], acc[i % FN][i / FN + H0]);
         },
-        [&](int q) { x1[1][q] = tile_of(x1l + buf + o1, q); },
-        [&](int q) { fetch(it + NS, buf, A1 + q); });
+        [&](int q) INLINE { get_x1(buf, q, 1); },
+        [&](int q) INLINE { fetch(it + NS, buf, A1 + q); });
     // A of the next stage has arrived
     if constexpr (R >= NS) wait_loads<(NS - 2) * P + P1 + A2>();
     else if constexpr (R > 0) wait_loads<(R - 1) * P + P1>();
     barrier();
+    cut_last(wa[1], 0, x1[1], H1, 1);
     phase<H1 * FN, (R > 0 ? FN + H0 : 0), (R >= NS ? PA - A2 : 0)>(
-        [&](int i) {
+        [&](int i) INLINE {
           acc[i % FN][i / FN + H0] =
               mfma(wa[1][i % FN], x1[1][i / FN], acc[i % FN][i / FN + H0]);
         },
-        [&](int q) {
-          if (q < FN) wa[0][q] = tile_of(wl + next + o0, q);
-          else x0[0][q - FN] = tile_of(x0l + next + o0, q - FN);
+        [&](int q) INLINE {
+          if (q < FN) get_w(next, q, 0);
+          else get_x0(next, q - FN, 0);
         },
-        [&](int q) { fetch(it + NS, buf, A2 + q); });
+        [&](int q) INLINE { fetch(it + NS, buf, A2 + q); });
     return next;
   };
   int it = 0, buf = 0;
@@ -332,7 +449,7 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
           const int at = i / VPR, n = n0 + i % VPR * 8;
           const int mr = at % (MP * 16) + p * MP * 16;
           const int r = m0 + at / (MP * 16) * (BM / WM) + mr;
-          if (mr >= FM * 16 || r >= a.M || n >= N) continue;
+          if (mr >= FM * 16 || r >= rows || n >= N) continue;
           *(s16x8*)(a.out[layer] + (long long)r * N + n) =
               *(const s16x8*)(lds + at * RB + i % VPR * 16);
         }
@@ -340,11 +457,14 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
       return;
     }
   }
-  const int all = a.n_end[a.layers - 1];
+  // partial sums: rows and columns before this layer's
+  const int before = layer ? a.n_end[layer - 1] : 0;
+  const int all = WT ? K : a.n_end[a.layers - 1];
+  const int all_rows = MODE == GRAD_W ? a.n_end[a.layers - 1] : a.M;
 #pragma unroll
   for (int m = 0; m < FM; ++m) {
     const int r = m0 + wm * (BM / WM) + 16 * m + col;
-    if (r >= a.M) continue;
+    if (r >= rows) continue;
     if constexpr (GLU) {
 #pragma unroll
       for (int f = 0; f < FN; f += 2) {
@@ -362,8 +482,9 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
         const int n = n0 + (wn * FN + f) * 16 + 4 * g;
         if (n >= N) continue;
         if (a.splits > 1)
-          *(f32x4*)(a.part + ((long long)split * a.M + r) * all +
-                    (layer ? a.n_end[layer - 1] : 0) + n) = acc[f][m];
+          *(f32x4*)(a.part + ((long long)split * all_rows + r +
+                              (MODE == GRAD_W ? before : 0)) * all +
+                    (MODE == GRAD_W ? 0 : before) + n) = acc[f][m];
         else
           *(s16x4*)(a.out[layer] + (long long)r * N + n) =
               packed(add_bias(acc[f][m], a.bias[layer], n));
@@ -372,44 +493,61 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
   }
 }
 
-// Adds the splits up: four features of a row a thread.
-__global__ __launch_bounds__(256) void tile_merge_kernel(const Args a) {
-  const int all = a.n_end[a.layers - 1];
+// Adds the splits up: four columns of a row a thread.
+template <int MODE>
+__global__ __launch_bounds__(256) void tile_merge_kernel(const Args a,
+                                                         const int rows,
+                                                         const int all) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long long)a.M * (all / 4)) return;
-  const int r = (int)(i / (all / 4)), n = (int)(i % (all / 4)) * 4;
+  if (i >= (long long)rows * (all / 4)) return;
+  int r = (int)(i / (all / 4)), n = (int)(i % (all / 4)) * 4;
   f32x4 y = {0.f, 0.f, 0.f, 0.f};
   const float* p = a.part + (long long)r * all + n;
 #pragma unroll 4
   for (int s = 0; s < a.splits; ++s)
-    y += *(const f32x4*)(p + (long long)s * a.M * all);
-  int l = 0;
-  while (n >= a.n_end[l]) ++l;
-  const int at = n - (l ? a.n_end[l - 1] : 0);
-  *(s16x4*)(a.out[l] + (long long)r * a.n[l] + at) =
-      packed(add_bias(y, a.bias[l], at));
+    y += *(const f32x4*)(p + (long long)s * rows * all);
+  int l = 0, ld = all;
+  if (MODE == PLAIN) {
+    while (n >= a.n_end[l]) ++l;
+    if (l) n -= a.n_end[l - 1];
+    ld = a.n[l];
+  }
+  if (MODE == GRAD_W) {
+    while (r >= a.n_end[l]) ++l;
+    if (l) r -= a.n_end[l - 1];
+  }
+  *(s16x4*)(a.out[l] + (long long)r * ld + n) =
+      packed(add_bias(y, a.bias[l], n));
 }
 
 template <int BM, int BN, int WM, int WN, int NS, int MODE>
 int launch(Args a, hipStream_t st) {
   constexpr int LDS = NS * (BM + BN) * ROW;
   static_assert(LDS <= 160 * 1024, "");
-  const int bn = MODE == SWIGLU ? BN / 2 : BN;
-  int tiles = 0;
-  for (int i = 0; i < (MODE == SWIGLU ? 1 : a.layers); ++i)
-    a.tile_end[i] = tiles += (a.n[i] + bn - 1) / bn;
-  a.tiles = tiles;
-  a.mtiles = (a.M + BM - 1) / BM;
+  constexpr int bn = MODE == SWIGLU ? BN / 2 : BN;
+  int sum = 0, steps = 0;
+  for (int i = 0; i < a.layers; ++i) {
+    if (MODE != SWIGLU || i == 0)
+      sum += MODE == GRAD_W ? (a.n[i] + BM - 1) / BM : (a.n[i] + bn - 1) / bn;
+    a.tile_end[i] = sum;
+    a.step_end[i] = steps += a.n[i] / BK;
+  }
+  a.steps = steps;
+  a.tiles = MODE >= GRAD_X ? (a.K + bn - 1) / bn : sum;
+  a.mtiles = MODE == GRAD_W ? sum : (a.M + BM - 1) / BM;
   auto kernel = tile_linear_kernel<BM, BN, WM, WN, NS, MODE>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (e != hipSuccess) return (int)e;
-  hipLaunchKernelGGL(kernel, dim3(tiles * a.mtiles * a.splits),
+  hipLaunchKernelGGL(kernel, dim3(a.tiles * a.mtiles * a.splits),
                      dim3(WM * WN * 64), LDS, st, a);
   if (a.splits > 1) {
-    const long long q = (long long)a.M * (a.n_end[a.layers - 1] / 4);
-    hipLaunchKernelGGL(tile_merge_kernel, dim3((unsigned)((q + 255) / 256)),
-                       dim3(256), 0, st, a);
+    const int n = a.n_end[a.layers - 1];
+    const int rows = MODE == GRAD_W ? n : a.M, all = MODE >= GRAD_X ? a.K : n;
+    const long long q = (long long)rows * (all / 4);
+    hipLaunchKernelGGL(tile_merge_kernel<MODE>,
+                       dim3((unsigned)((q + 255) / 256)), dim3(256), 0, st, a,
+                       rows, all);
   }
   return (int)hipGetLastError();
 }
@@ -431,14 +569,21 @@ int launch(Args a, hipStream_t st) {
   X(8, 256, 192, 2, 4, 2, 1.038f, 7.0f)    \
   X(9, 256, 256, 2, 4, 2, 1.342f, 8.4f)
 
+// A wave's gate and up tiles in pairs; halves of x in blocks of 64 columns.
+#define GATES(BN, WN) (BN / WN / 16 % 2 == 0)
+#define BLOCKS(BM, WM) (BM / WM / 32 * 16 * WM % 64 == 0)
+
 struct Tile {
   int bm, bn, stages;
-  bool gates;
+  bool gates, blocks;
   float stage, fixed;
+  bool takes(int mode) const {
+    return (gates || mode != SWIGLU) && (blocks || mode != GRAD_W);
+  }
 };
 const Tile tiles_[] = {
 #define X(I, BM, BN, WM, WN, NS, U, F) \
-  {BM, BN, NS, BN / WN / 16 % 2 == 0, U, F},
+  {BM, BN, NS, GATES(BN, WN), BLOCKS(BM, WM), U, F},
     TILES(X)
 #undef X
 };
@@ -446,24 +591,18 @@ const Tile tiles_[] = {
 // us that a tile and a number of splits take: rounds of the 256 CUs (the last
 // one, in part empty, runs faster: less power, less traffic) or W and x from
 // memory at 4.15 TB/s, whichever is longer, then adding the splits up.
-float estimate(const Tile& t, const int* n, int layers, int M, int K, int mode,
-               int splits) {
-  const int bn = mode == SWIGLU ? t.bn / 2 : t.bn;
-  double tiles = 0, all = 0;
-  for (int i = 0; i < layers; ++i) {
-    if (mode != SWIGLU || i == 0) tiles += (n[i] + bn - 1) / bn;
-    all += n[i];
-  }
-  tiles *= (double)((M + t.bm - 1) / t.bm) * splits;
+float estimate(const Tile& t, double tiles, int steps, double rows,
+               double columns, double bytes, int splits) {
+  tiles *= splits;
   const double whole = (double)(long long)(tiles / 256);
   const double rest = tiles / 256 - whole;
   double us = (whole + (rest > 0 ? 0.76 + 0.24 * rest : 0)) *
-      (K / BK / (double)splits * t.stage + t.fixed);
-  double mem = (all * K + (double)M * (K + all)) * 2 / 4.15e6;
+      (steps / (double)splits * t.stage + t.fixed);
+  double mem = bytes / 4.15e6;
   us *= us * us;
   mem *= mem * mem;
   us = cbrt(sqrt(us * us + mem * mem));
-  if (splits > 1) us += 2.7 + 0.296e-6 * splits * M * all * 4;
+  if (splits > 1) us += 2.7 + 0.296e-6 * splits * rows * columns * 4;
   return (float)us;
 }
 
@@ -475,18 +614,30 @@ float estimate(const Tile& t, const int* n, int layers, int M, int K, int mode,
 extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
                                    int mode, int* splits) {
   static const int some[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+  double all = 0;
+  for (int l = 0; l < layers; ++l) all += n[l];
+  const int steps = mode == GRAD_X ? (int)(all / BK)
+      : mode == GRAD_W ? (M + BK - 1) / BK : K / BK;
+  const double rows = mode == GRAD_W ? all : M;
+  const double columns = mode >= GRAD_X ? K : all;
+  const double bytes = 2 * (all * K + (double)M * (K + all));
   int best = -1;
   float least = 0;
   for (int i = 0; i < (int)(sizeof(tiles_) / sizeof(Tile)); ++i) {
     const Tile& t = tiles_[i];
-    if (mode == SWIGLU && !t.gates) continue;
-    long long tiles = 0;
-    for (int l = 0; l < layers; ++l) tiles += (n[l] + t.bn - 1) / t.bn;
-    tiles *= (M + t.bm - 1) / t.bm;
+    if (!t.takes(mode)) continue;
+    double tiles = 0;
+    for (int l = 0; l < layers; ++l)    // SWIGLU: a gate and an up each
+      tiles += mode == GRAD_W ? (n[l] + t.bm - 1) / t.bm
+          : mode == SWIGLU ? 0.5 * ((2 * n[l] + t.bn - 1) / t.bn)
+          : (n[l] + t.bn - 1) / t.bn;
+    if (mode == GRAD_X) tiles = 1;
+    tiles *= mode >= GRAD_X ? (K + t.bn - 1) / t.bn : 1;
+    tiles *= mode == GRAD_W ? 1 : (M + t.bm - 1) / t.bm;
     for (int s : some) {
       if (s > 1 && (mode == SWIGLU || tiles * s > 520)) break;
-      if (K / BK / s < t.stages) break;
-      const float us = estimate(t, n, layers, M, K, mode, s);
+      if (steps / s < t.stages) break;
+      const float us = estimate(t, tiles, steps, rows, columns, bytes, s);
       if (best < 0 || us < least) {
         best = i;
         least = us;
@@ -500,35 +651,44 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
 // Stages of inputs that a split has to hold at least; 0: no such tile.
 extern "C" int ds_tile_linear_stages(int tile, int mode) {
   if (tile < 0 || tile >= (int)(sizeof(tiles_) / sizeof(Tile))) return 0;
-  return mode == SWIGLU && !tiles_[tile].gates ? 0 : tiles_[tile].stages;
+  return tiles_[tile].takes(mode) ? tiles_[tile].stages : 0;
 }
 
-// K is a multiple of 64, every n of four, x and every w lie at 16 bytes; mode 1:
-// silu(layer 0) * layer 1. tile and splits from the plan; part: splits * M * all
-// features, null for one split. Returns a hipError_t.
-extern "C" int ds_tile_linear(const void* x, int layers, const void* const* w,
-                              const void* const* bias, void* const* out,
-                              const int* n, int M, int K, int mode, int tile,
-                              int splits, float* part, void* stream) {
+// 1..3 weights [n, K] of layers on one input of M rows. PLAIN and SWIGLU: x[0]
+// [M, K] to out [M, n], one each or one; K is a multiple of 64, n of four.
+// GRAD_X: x are the gradients dy [M, n], out[0] [M, K]; n is a multiple of 64, K
+// of eight. GRAD_W: w[0] is the input, x the gradients, out [n, K]; n and K are
+// multiples of eight. All operands at 16 bytes; bias only for the first two.
+// tile and splits from the plan; part: splits * rows * columns of all outputs,
+// null for one split. Returns a hipError_t.
+extern "C" int ds_tile_linear(const void* const* x, int layers,
+                              const void* const* w, const void* const* bias,
+                              void* const* out, const int* n, int M, int K,
+                              int mode, int tile, int splits, float* part,
+                              void* stream) {
   Args a = {};
   int total = 0;
   for (int i = 0; i < layers; ++i) {
-    a.w[i] = (const short*)w[i];
-    a.bias[i] = (const short*)bias[i];
-    a.out[i] = (short*)out[i];
+    a.w[i] = (const short*)w[mode == GRAD_W ? 0 : i];
+    a.x[i] = (const short*)x[mode >= GRAD_X ? i : 0];
+    a.bias[i] = mode >= GRAD_X ? nullptr : (const short*)bias[i];
+    a.out[i] = (short*)out[mode == GRAD_X || mode == SWIGLU ? 0 : i];
     a.n[i] = n[i];
     a.n_end[i] = total += n[i];
   }
-  a.x = (const short*)x;
   a.part = part;
   a.M = M; a.K = K; a.layers = layers; a.splits = splits;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   switch (tile) {
 #define X(I, BM, BN, WM, WN, NS, U, F)                                    \
   case I:                                                                 \
+    if (mode == GRAD_X) return launch<BM, BN, WM, WN, NS, GRAD_X>(a, st); \
+    if (mode == GRAD_W)                                                   \
+      return launch<BM, BN, WM, WN, NS,                                   \
+                    BLOCKS(BM, WM) ? GRAD_W : PLAIN>(a, st);              \
     if (mode == SWIGLU)                                                   \
       return launch<BM, BN, WM, WN, NS,                                   \
-                    BN / WN / 16 % 2 == 0 ? SWIGLU : PLAIN>(a, st);       \
+                    GATES(BN, WN) ? SWIGLU : PLAIN>(a, st);               \
     return launch<BM, BN, WM, WN, NS, PLAIN>(a, st);
     TILES(X)
 #undef X

@@ -1,7 +1,6 @@
 """Linear layers.
 
-``Linear`` is torch's, with a backward whose products read their operands along
-the contiguous axis (see ``_Linear``).
+``Linear`` is torch's, with the backward of ``_Linears``.
 
 ``rows_linear``, for a few rows (decoding), and ``tile_linear``, for any more:
 the framework's kernels (csrc/rows_linear.hip, csrc/tile_linear.hip) in place of
@@ -9,7 +8,7 @@ a library GEMM, with several layers of one input in one launch and the gate's
 activation in the epilogue.
 
 Both take the modules themselves and return None wherever calling them is the
-thing to do: with gradients, hooks, autocast, function transforms, tangents or
+thing to do: with gradients (but for several layers of ``tile_linear``), hooks, autocast, function transforms, tangents or
 traces, other types, sharded or replaced modules."""
 
 import torch
@@ -69,50 +68,152 @@ def backward_plan(T: int, N: int, K: int):
     return w, big and N < K, big and N >= K
 
 
-class _Linear(torch.autograd.Function):
-    """x W^T + b whose backward lays operands out for the matrix product:
-    dx = dy W reads W across its rows, and dW = dy^T x reads both across
-    theirs, at two thirds of the forward product's rate. Transposing costs a
-    read and a write of an operand and pays where ``backward_plan`` says. Kept
-    for the backward is what it needs: a frozen layer holds no input."""
+def own_products(T: int, N: int, K: int):
+    """Which products of the backward of a layer [N, K] over T rows are
+    csrc/tile_linear.hip's: (the input's gradient, the weight's). It reads either
+    operand across the contraction as fast as along it, without a transposed copy
+    (us, library with the copies of ``backward_plan`` and kernel).
+
+    Input: N 4096, K 14336, 2331 rows 351 / 256; 3072, K 8192, 1024 rows 53 / 50;
+    1024, K 1024, 1024 rows 22 / 9; 32000, K 1024, 1024 rows 194 / 75. From 2560
+    rows on the library's whole rounds of tiles are ahead at large weights (14336,
+    K 4096, 8192 rows 647 / 728; 128256, K 4096, 4000 rows 3050 / 3300) and no
+    longer at smaller ones (3072, K 8192, 4000 rows 162 / 159, 5000 307 / 220).
+    Weight: 4096, K 4096, 4000 rows 122 / 102; 14336, K 4096, 4000 rows 453 / 383,
+    32768 rows 3555 / 3162; 3072, K 3072, 4000 rows 88 / 72; but 128256, K 4096,
+    8192 rows 6289 / 6630 (4000 rows 3454 / 3324)."""
+    dx = N % 64 == 0 and K % 8 == 0 and N >= 192 and T > ROWS and \
+        (T < 2560 or N * K < 1 << 25)
+    dw = N % 8 == 0 and K % 8 == 0 and T > 192 and \
+        (T < 6144 or N * K < 1 << 28)
+    return dx, dw
+
+
+def own_forward(T: int, ns, K: int) -> bool:
+    """Whether the forward product of layers of ``ns`` features is
+    csrc/tile_linear.hip's, as in ``tile_linear``."""
+    return T > ROWS and K % 64 == 0 and 192 <= K <= 1 << 22 and \
+        all(n % 4 == 0 for n in ns) and (
+            T < 2560 or K >= 16384
+            or (len(ns) > 1 and max(ns) * K < 1 << 25))
+
+
+def _aligned(*ts) -> bool:
+    return all(t.data_ptr() % 16 == 0 for t in ts)
+
+
+def _forward(x, weights, biases):
+    """Outputs of the layers on x, by the kernel where that pays."""
+    ns, K = [w.shape[0] for w in weights], x.shape[-1]
+    x2 = x.reshape(-1, K).contiguous()
+    if own_forward(x2.shape[0], ns, K) and _aligned(x2, *weights) and all(
+            b is None or (b.dtype is torch.bfloat16 and b.is_contiguous())
+            for b in biases):
+        out = get_ext().tile_linear(x2, weights, biases, PLAIN)
+        return [o.view(*x.shape[:-1], o.shape[-1]) for o in out]
+    return [nn.functional.linear(x, w, b) for w, b in zip(weights, biases)]
+
+
+def _dx(dys, weights, own: bool):
+    """Sum of dy W over the layers."""
+    T, K = dys[0].shape[0], weights[0].shape[1]
+    sizes = [w.shape[0] for w in weights]
+    if own and all(own_products(T, n, K)[0] for n in sizes) and \
+            _aligned(*dys, *weights):
+        return get_ext().tile_linear_dx(dys, weights)
+    dx = None
+    for dy, w in zip(dys, weights):
+        if own and backward_plan(T, *w.shape)[0]:
+            part = nn.functional.linear(dy, _transposed(w))
+        else:
+            part = dy @ w
+        dx = part if dx is None else dx + part
+    return dx
+
+
+def _dw(x, dys, own: bool):
+    """dy^T x of the layers."""
+    T, K = x.shape
+    if own and all(own_products(T, dy.shape[1], K)[1] for dy in dys) and \
+            _aligned(x, *dys):
+        return get_ext().tile_linear_dw(x, dys)
+    dws = []
+    for dy in dys:
+        dy_t = x_t = False
+        if own:
+            _, dy_t, x_t = backward_plan(T, dy.shape[1], K)
+        a = _transposed(dy) if dy_t else dy.t()
+        b = _transposed(x).t() if x_t else x
+        dws.append(a @ b)
+    return dws
+
+
+class _Linears(torch.autograd.Function):
+    """x W^T + b of one to three layers on one input. The backward's products lie
+    across their operands (dx = dy W across W, dW = dy^T x across both): those of
+    ``own_products`` are csrc/tile_linear.hip's, with the input's gradient summed
+    over the layers in the product; for the others operands are transposed where
+    ``backward_plan`` says. Kept for the backward is what it needs: a frozen layer
+    holds no input. ``own``: the forward product may be the kernel's as well."""
 
     @staticmethod
-    def forward(ctx, x, weight, bias):
-        need_x, need_w, _ = ctx.needs_input_grad
-        ctx.save_for_backward(x if need_w else None, weight if need_x else None)
-        ctx.shape, ctx.features = x.shape, weight.shape
-        return nn.functional.linear(x, weight, bias)
+    def forward(ctx, x, own, *params):
+        weights, biases = params[::2], params[1::2]
+        need = ctx.needs_input_grad
+        ctx.save_for_backward(x if any(need[2::2]) else None,
+                              *(w if need[0] else None for w in weights))
+        ctx.shape, ctx.features = x.shape, [w.shape for w in weights]
+        if own:
+            out = _forward(x, weights, biases)
+        else:
+            out = [nn.functional.linear(x, w, b)
+                   for w, b in zip(weights, biases)]
+        return out[0] if len(out) == 1 else tuple(out)
 
     @staticmethod
-    def backward(ctx, dy):
-        x, weight = ctx.saved_tensors
-        need_x, need_w, need_b = ctx.needs_input_grad
-        N, K = ctx.features
-        dy2 = dy.reshape(-1, N)
-        T = dy2.shape[0]
-        w_t = dy_t = x_t = False
-        # differentiable products where the gradient itself is differentiated
-        if not torch.is_grad_enabled() and dy.dtype is torch.bfloat16:
-            w_t, dy_t, x_t = backward_plan(T, N, K)
-        dx = dw = db = None
-        if need_x:
-            dx = nn.functional.linear(dy2, _transposed(weight)) if w_t \
-                else dy2 @ weight
-            dx = dx.view(ctx.shape)
-        if need_w:
+    def backward(ctx, *dys):
+        x, *weights = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        K = ctx.shape[-1]
+        dys = [dy.reshape(-1, n) for dy, (n, _) in zip(dys, ctx.features)]
+        # differentiable products where the gradient itself is differentiated,
+        # torch's own where something watches them
+        own = (not torch.is_grad_enabled() and untransformed()
+               and all(dy.dtype is torch.bfloat16 and not _batched(dy)
+                       for dy in dys))
+        if own:
+            dys = [dy.contiguous() for dy in dys]
+        dx = None
+        grads = [None] * (2 * len(dys))
+        if need[0]:
+            dx = _dx(dys, weights, own).view(ctx.shape)
+        some = [i for i in range(len(dys)) if need[2 + 2 * i]]
+        if some:
             x2 = x.reshape(-1, K)
-            a = _transposed(dy2) if dy_t else dy2.t()
-            b = _transposed(x2).t() if x_t else x2
-            dw = a @ b
-        if need_b:
-            db = dy2.sum(0)
-        return dx, dw, db
+            if own:
+                x2 = x2.contiguous()
+            for i, dw in zip(some, _dw(x2, [dys[i] for i in some], own)):
+                grads[2 * i] = dw
+        for i, dy in enumerate(dys):
+            if need[3 + 2 * i]:
+                grads[2 * i + 1] = dy.sum(0)
+        return dx, None, *grads
+
+
+class _Linear:
+    """One layer with torch's forward product."""
+
+    @staticmethod
+    def apply(x, weight, bias):
+        return _Linears.apply(x, False, weight, bias)
 
 
 def _transposed(a: torch.Tensor) -> torch.Tensor:
     return get_ext().transpose_2d(a.contiguous())
 
 
+# Gradients asked for in batches (``is_grads_batched``) have no memory of their own.
+_batched = torch._C._functorch.is_legacy_batchedtensor
 _interpreter = torch._C._functorch.peek_interpreter_stack
 _modes = torch._C._len_torch_dispatch_stack
 _trace = torch._C._get_tracing_state
@@ -143,22 +244,40 @@ def movable(cls):
     return cls
 
 
+def _differentiable(x, weights) -> bool:
+    """``_Linears`` takes these with gradients: plain bf16 tensors on a GPU."""
+    return (torch.is_grad_enabled() and x.is_cuda and x.dim() > 1
+            and type(x) is torch.Tensor and x.dtype is torch.bfloat16
+            and x.numel() > 0
+            and all(type(w) is nn.Parameter and w.dtype is torch.bfloat16
+                    and w.dim() == 2 and w.shape[1] == x.shape[-1]
+                    and w.is_contiguous() for w in weights)
+            and get_ext() is not None and _plain_autograd()
+            and nn.Linear.forward is _TORCHS)
+
+
 @movable
 class Linear(nn.Linear):
-    """nn.Linear with the backward of ``_Linear`` on a GPU."""
+    """nn.Linear with the backward of ``_Linears`` on a GPU, and with ``own`` its
+    forward."""
 
-    def forward(self, x):
+    def forward(self, x, own: bool = False):
         w = self.weight
-        if (torch.is_grad_enabled() and x.is_cuda and x.dim() > 1
-                and type(x) is torch.Tensor and type(w) is nn.Parameter
-                and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16
-                and w.is_contiguous() and w.dim() == 2
-                and x.numel() and x.shape[-1] == w.shape[1]
-                and any(backward_plan(x.numel() // w.shape[1], *w.shape))
-                and get_ext() is not None and _plain_autograd()
-                and nn.Linear.forward is _TORCHS):
-            return _Linear.apply(x, w, self.bias)
+        if _differentiable(x, (w,)):
+            T = x.numel() // w.shape[1]
+            if any(own_products(T, *w.shape)) or \
+                    any(backward_plan(T, *w.shape)) or \
+                    (own and own_forward(T, w.shape[:1], w.shape[1])):
+                return _Linears.apply(x, own, w, self.bias)
         return super().forward(x)
+
+
+def call(mod: nn.Module, x):
+    """The module on x: a layer of this framework that at most the framework's
+    own hooks watch may take its forward product itself."""
+    if type(mod) is Linear and unhooked(mod, internal_ok=True):
+        return mod(x, own=True)
+    return mod(x)
 
 
 def unhooked(mod: nn.Module, internal_ok: bool = False) -> bool:
@@ -245,6 +364,22 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
     return [o.view(*x.shape[:-1], o.shape[-1]) for o in out]
 
 
+def _with_gradients(x, mods):
+    """Several layers of a training step's rows in one function, or None: their
+    products are one launch each way and nothing adds the input's gradients up."""
+    if len(mods) < 2 or not all(type(m) is Linear and unhooked(m)
+                                for m in mods) or \
+            not _differentiable(x, [m.weight for m in mods]):
+        return None
+    T, K = x.numel() // x.shape[-1], x.shape[-1]
+    ns = [m.weight.shape[0] for m in mods]
+    if not own_forward(T, ns, K) and \
+            not any(any(own_products(T, n, K)) for n in ns):
+        return None
+    return _Linears.apply(x, True, *(p for m in mods
+                                     for p in (m.weight, m.bias)))
+
+
 def tile_linear(x: torch.Tensor, mods, mode: int = PLAIN):
     """``rows_linear`` for more than ``ROWS`` rows and torch's or the models' own
     bf16 layers. Over 20 layers of 1024 x 1024 to 128256 x 4096 and 33 to 8192
@@ -257,7 +392,9 @@ def tile_linear(x: torch.Tensor, mods, mode: int = PLAIN):
     14336 304 / 324; N 128256 2930 / 3060; elsewhere 3300 rows: N 4096, K 14336
     343 / 305), but for contractions from 16384 on (3584, K 18944: 4096 rows 540
     / 418, 5000 958 / 658)."""
-    if type(x) is not torch.Tensor or torch.is_grad_enabled() or \
+    if torch.is_grad_enabled():
+        return _with_gradients(x, mods) if mode == PLAIN else None
+    if type(x) is not torch.Tensor or \
             not x.is_cuda or x.dtype is not torch.bfloat16:
         return None
     K = x.shape[-1]

@@ -1,11 +1,12 @@
 """Linear layers of many rows: which calls take the kernel (CPU) and every tile
-of the kernel against fp64 products (GPU)."""
+of the kernel against fp64 products, forward and backward (GPU)."""
 
 import pytest
 import torch
 import torch.nn as nn
 
-from deepspeed_amd.ops.linear import SWIGLU, Linear, tile_linear
+from deepspeed_amd.ops import linear as L
+from deepspeed_amd.ops.linear import SWIGLU, Linear, call, tile_linear
 
 # rows, features and stages of the tiles, in the kernel's order
 TILES = [(64, 64, 8), (64, 128, 6), (128, 64, 6), (128, 128, 5), (128, 256, 3),
@@ -107,3 +108,148 @@ def test_refused_gpu():
     assert call(40, 224, 64) is None
     assert call(40, 128, 64) is None
     assert call(40, 256, 64, torch.float16) is None
+
+
+def _limit(want, terms):
+    # one rounding to bf16 of an fp32 sum
+    return 2.0 ** -8 * want.abs() + 2.0 ** -20 * terms ** 0.5 * \
+        want.abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@torch.no_grad()
+def test_every_tile_backward_gpu(tile):
+    from deepspeed_amd.ops import _C
+    bm, bn, stages = TILES[tile]
+    for rows, more in ((-1, 8), (0, 0), (1, -8)):      # beside a whole tile
+        for steps, splits in ((stages, 1), (stages + 1, 1),
+                              (3 * stages + 4, 3)):
+            # the input's gradient: over one layer, and over three
+            for ns in ((64 * steps,), (64 * (steps - 1), 64), (64, 64 * steps,
+                                                              128)):
+                x, ws, _ = _inputs(bm + rows, ns, bn + more, steps)
+                dys = [_inputs(bm + rows, (), n, n)[0] for n in ns]
+                want = sum(d.double() @ w.double() for d, w in zip(dys, ws))
+                err = (_C.tile_linear_dx(dys, ws, tile, splits).double()
+                       - want).abs()
+                assert (err <= _limit(want, sum(ns))).all()
+            if bm == 64:        # its rows' halves are narrower than a block
+                with pytest.raises(RuntimeError):
+                    _C.tile_linear_dw(x, dys, tile, 1)
+                continue
+            # the weights': rows that end anywhere in a stage
+            for end in (-63, -31, -8, -1, 0):
+                m, ns = 64 * steps + end, (bm + more, 8, 2 * bm - 8)
+                x, _, _ = _inputs(m, (), bn + more, steps)
+                dys = [_inputs(m, (), n, n)[0] for n in ns]
+                for got, d in zip(_C.tile_linear_dw(x, dys, tile, splits),
+                                  dys):
+                    want = d.double().t() @ x.double()
+                    err = (got.double() - want).abs()
+                    assert (err <= _limit(want, m)).all()
+
+
+@pytest.mark.gpu
+def test_what_lies_past_the_last_row_gpu():
+    """Rows past the end count for nothing, whatever the last one holds: each
+    value of the weight's gradient comes from its own column."""
+    from deepspeed_amd.ops import _C
+    x, _, _ = _inputs(257, (), 256, 0)
+    dy, _, _ = _inputs(257, (), 264, 1)
+    x[-1, 5] = float("inf")
+    dy[-1, 7] = 0.0
+    got, = _C.tile_linear_dw(x, [dy])
+    want = dy.double().t() @ x.double()
+    finite = want.isfinite()
+    assert torch.equal(finite, got.isfinite())
+    assert torch.equal(want.isnan(), got.isnan())
+    err = (got.double() - want)[finite].abs()
+    assert (err <= _limit(want[finite], 257)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [40, 250, 1000, 2600])
+@pytest.mark.parametrize("ns,k", [((512, 128, 128), 256), ((1000, 1000), 264),
+                                  ((640,), 512)])
+@pytest.mark.parametrize("frozen", [None, "input", 0])
+def test_training_layers_gpu(m, ns, k, frozen):
+    x, ws, bs = _inputs(m, ns, k, m)
+    mods = []
+    for w, b in zip(ws, bs):
+        lin = Linear(k, len(w), bias=b is not None, device="cuda",
+                     dtype=torch.bfloat16)
+        with torch.no_grad():
+            lin.weight.copy_(w)
+            if b is not None:
+                lin.bias.copy_(b)
+        mods.append(lin)
+    if frozen == 0:
+        mods[0].weight.requires_grad_(False)
+    x = x.view(2, m // 2, k).requires_grad_(frozen != "input")
+    ys = tile_linear(x, mods) or [call(lin, x) for lin in mods]
+    dys = [torch.randn_like(y) for y in ys]
+    torch.autograd.backward(ys, dys)
+    x2 = x.detach().reshape(-1, k).double()
+    d2 = [d.reshape(-1, d.shape[-1]).double() for d in dys]
+    for y, want in zip(ys, _want(x2, ws, bs, 0)):
+        _close(y.detach().reshape(want.shape), want)
+    if frozen != "input":
+        want = sum(d @ w.double() for d, w in zip(d2, ws))
+        got = x.grad.view(-1, k).double()
+        # layers whose parts are added up outside are rounded one by one
+        parts = sum((d @ w.double()).abs() for d, w in zip(d2, ws))
+        assert ((got - want).abs() <= 2.0 ** -7 * parts
+                + _limit(want, sum(ns))).all()
+    for i, (lin, d) in enumerate(zip(mods, d2)):
+        if frozen == i:
+            assert lin.weight.grad is None
+        else:
+            want = d.t() @ x2
+            err = (lin.weight.grad.double() - want).abs()
+            assert (err <= _limit(want, m)).all()
+        if lin.bias is not None:
+            torch.testing.assert_close(lin.bias.grad.double(), d.sum(0),
+                                       rtol=2.0 ** -7, atol=0.05)
+
+
+@pytest.mark.gpu
+def test_training_layers_watched_gpu():
+    """Hooks, dispatch modes, batched and twice differentiated gradients go
+    through torch's own products."""
+    from torch.utils.flop_counter import FlopCounterMode
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn(300, 256, device="cuda", generator=g).bfloat16()
+    x.requires_grad_()
+    mods = [Linear(256, 256, bias=False, device="cuda", dtype=torch.bfloat16)
+            for _ in range(2)]
+    a, b = tile_linear(x, mods)
+    with FlopCounterMode(display=False) as mode:
+        (a * b).sum().backward(retain_graph=True)
+    assert mode.get_total_flops() == 4 * 2 * 300 * 256 * 256
+    gx, = torch.autograd.grad((a.float() * b.float()).sum(), x,
+                              create_graph=True)
+    gx.float().sum().backward(retain_graph=True)
+    v = torch.randn(3, 300, 256, device="cuda", generator=g).bfloat16()
+    many, = torch.autograd.grad(a, x, v, is_grads_batched=True,
+                                retain_graph=True)
+    for got, d in zip(many, v):
+        one, = torch.autograd.grad(a, x, d, retain_graph=True)
+        assert (got.float() - one.float()).norm() <= 0.01 * one.float().norm()
+    h = mods[0].register_forward_hook(lambda *a: None)
+    assert tile_linear(x, mods) is None
+    h.remove()
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(
+            lambda t: seen.append(t.shape) or t, lambda t: t):
+        tile_linear(x, mods)
+    assert seen == [x.shape, mods[0].weight.shape, mods[1].weight.shape]
+
+
+def test_own_products():
+    assert L.own_products(4000, 3072, 3072) == (True, True)
+    assert L.own_products(8192, 14336, 4096) == (False, True)
+    assert L.own_products(8192, 128256, 4096) == (False, False)
+    assert L.own_products(1000, 1000, 512) == (False, True)
+    assert L.own_products(1000, 1024, 516) == (False, False)
+    assert L.own_products(32, 1024, 512) == (False, False)
