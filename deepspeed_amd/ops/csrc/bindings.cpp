@@ -95,11 +95,11 @@ extern "C" void ds_paged_rows(const void* q, const void* kpool,
                               int n_merges, int any_merge, int nq, int H,
                               int Hkv, int BS, int max_blocks, int splits,
                               float scale, void* stream);
-extern "C" void ds_rows_linear(const void* x, int layers, const void* const* w,
-                               const float* const* scales,
-                               const void* const* bias, void* const* out,
-                               const int* n, int M,
-                               int K, int group, int mode, void* stream);
+extern "C" int ds_rows_linear(const void* x, int layers, const void* const* w,
+                              const float* const* scales,
+                              const void* const* bias, void* const* out,
+                              const int* n, int M, int K, int group, int mode,
+                              void* stream);
 extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
                                    int mode, int* splits);
 extern "C" int ds_tile_linear_stages(int tile, int mode);
@@ -580,8 +580,10 @@ std::vector<at::Tensor> rows_linear(
   }
   if (!i8 && M > 16 && y.tiled(x, mode)) return y.out;
   TORCH_CHECK(i8 || M <= 32, "rows_linear: features in fours past 32 rows");
-  ds_rows_linear(x.data_ptr(), L, y.w, i8 ? sc : nullptr, y.b, y.o, y.n,
-                 (int)M, (int)K, (int)group, (int)mode, cur_stream());
+  const int e = ds_rows_linear(x.data_ptr(), L, y.w, i8 ? sc : nullptr, y.b,
+                               y.o, y.n, (int)M, (int)K, (int)group, (int)mode,
+                               cur_stream());
+  TORCH_CHECK(e == 0, "rows_linear: launch failed with error ", e);
   return y.out;
 }
 

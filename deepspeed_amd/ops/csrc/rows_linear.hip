@@ -8,22 +8,25 @@
 //
 // A workgroup of 8 waves owns 16 FT output features; the waves take every
 // eighth chunk of inputs and add up through LDS, so that the 256 CUs have work
-// at N = 4096 and each wave has a chunk's loads in flight while it computes the
-// one before. W goes from memory straight into the A operand of
-// mfma_f32_16x16x32_bf16 (16 features by 64 or, int8, 64 contiguous bytes an
-// instruction), x into B (columns past M repeat the last row).
+// at N = 4096. W goes from memory straight into the A operand of
+// mfma_f32_16x16x32_bf16 (16 features by 64 contiguous bytes an instruction), x
+// into B (columns past M repeat the last row).
 //
-//   * Bound by the stream of W at few rows (N 128256, K 4096, M 1: 169 us, 6.2
-//     TB/s; the library's product 187 us) and by x out of L2 at many; at 32
-//     rows the library's GPU time is 5 to 30% less (N 14336 25.2 to 29.6 us, N
-//     4096 12.5 to 15.7), but its calls cost the host 20 us each, which a step
-//     of one layer's seven calls cannot hide, against 5 us here.
+//   * Up to 16 rows, few_rows_kernel: W and x are loaded D chunks of 128 inputs
+// ahead, so that a wave waits for neither, and the scales lie in LDS. Bound by
+// the stream of W in large layers, by launch and first loads in small ones. us
+// at 8 rows, before (chunks of 256, x loaded where it is used) and now: gate and
+// up 14336, K 4096 bf16 50.7 / 45.8, int8 36.6 / 32.8; q, k, v 4096 + 2 x 1024,
+// K 4096 16.0 / 13.3 and 12.2 / 10.8; N 128256 199 / 192 and 140 / 121; N 4096,
+// K 14336 27.7 / 27.3 and 19.7 / 18.9; N 4096, K 4096 10.2 / 10.1 and 8.2 / 8.6.
+// Three to six chunks ahead gained nothing more.
+//   * More rows, rows_linear_kernel: bound by x out of L2. Only int8 weights and
+// numbers of features that tile_linear.hip does not take come here.
 //   * int8: a lane's 16 bytes are 16 inputs, split over two products; the order
 //     of the inputs inside a product is free, x is read in the same order. The
 //     bytes become bf16 exactly (8 bits), are summed in fp32 and multiplied by
 //     their group's scale in fp32: nothing is rounded before the output, and
-//     the weight is not written out as bf16 and read again. N 14336, K 4096, M
-//     8: 21.8 us; dequantizing takes 28 us and the product 28.
+//     the weight is not written out as bf16 and read again.
 //   * Several layers on one input (q, k, v; gate and up) are one launch, and
 //     the epilogue takes the gate's activation and the bias with it: four
 //     launches a decoder layer instead of eight.
@@ -39,6 +42,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int NW = 8;       // waves a workgroup
 constexpr int MAXL = 3;     // layers a launch
+constexpr int CH = 128;     // inputs a chunk
 
 enum { PLAIN = 0, SWIGLU = 1 };
 
@@ -63,13 +67,12 @@ __device__ __forceinline__ float value(short x) {
   return __builtin_bit_cast(float, (unsigned)(unsigned short)x << 16);
 }
 
-// four signed bytes to four bf16, exactly: u = b + 128 is 0..255
+// four signed bytes to four bf16, exactly (an instruction a byte and one a pair)
 __device__ __forceinline__ void widen(unsigned b, unsigned& lo, unsigned& hi) {
-  b ^= 0x80808080u;
-  const float f0 = (float)(b & 255u) - 128.f;
-  const float f1 = (float)((b >> 8) & 255u) - 128.f;
-  const float f2 = (float)((b >> 16) & 255u) - 128.f;
-  const float f3 = (float)(b >> 24) - 128.f;
+  const float f0 = (float)(int)(signed char)b;
+  const float f1 = (float)(int)(signed char)(b >> 8);
+  const float f2 = (float)(int)(signed char)(b >> 16);
+  const float f3 = (float)(int)(signed char)(b >> 24);
   lo = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, f1),
                              __builtin_bit_cast(unsigned, f0), 0x07060302u);
   hi = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, f3),
@@ -77,7 +80,7 @@ __device__ __forceinline__ void widen(unsigned b, unsigned& lo, unsigned& hi) {
 }
 
 // CH inputs of 16 features: CH / 32 A operands.
-template <bool I8, int CH>
+template <bool I8>
 struct Weights {
   u32x4 r[I8 ? CH / 64 : CH / 32];
 
@@ -112,7 +115,6 @@ __device__ __forceinline__ int input_at(int i, int g) {
 
 template <bool I8, int MT, int MODE, int FT>
 __global__ __launch_bounds__(NW * 64) void rows_linear_kernel(const Args a) {
-  constexpr int CH = MT == 1 ? 256 : 128;     // inputs a chunk
   constexpr int L = MODE == SWIGLU ? 2 : 1;   // weight streams a workgroup
   constexpr int S = L * FT;                   // tiles of 16 features a wave
   __shared__ float lds[NW][S][256];
@@ -143,7 +145,7 @@ __global__ __launch_bounds__(NW * 64) void rows_linear_kernel(const Args a) {
     for (int m = 0; m < MT; ++m) acc[s][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int chunks = a.K / CH;
-  Weights<I8, CH> w[S];
+  Weights<I8> w[S];
   int c = wid;
   if (c < chunks)
 #pragma unroll
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(NW * 64) void rows_linear_kernel(const Args a) {
           sc[s][r] = a.scales[layer + s / FT][
               ((long long)min(n0 + 16 * (s % FT) + 4 * g + r, N - 1) * a.K +
                c * CH) / a.group];
-    Weights<I8, CH> cur[S];
+    Weights<I8> cur[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) cur[s] = w[s];
     if (c + NW < chunks)
@@ -225,60 +227,185 @@ __global__ __launch_bounds__(NW * 64) void rows_linear_kernel(const Args a) {
   }
 }
 
+template <bool I8, int MODE, int FT, int D, int OCC>
+__global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
+  constexpr int L = MODE == SWIGLU ? 2 : 1;   // weight streams a workgroup
+  constexpr int S = L * FT;                   // tiles of 16 features a wave
+  // [waves][S][256] sums, then int8's scales [chunks][S][16]
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* const sums = lds;
+  float* const scales = lds + NW * S * 256;
+
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int col = lane & 15, g = lane >> 4;
+  int layer = 0, tile = blockIdx.x;
+  if (MODE == PLAIN) {
+    while (tile >= a.tile_end[layer]) ++layer;
+    if (layer) tile -= a.tile_end[layer - 1];
+  }
+  const int N = a.n[layer], n0 = tile * 16 * FT;
+  const short* xp = a.x + (long long)min(col, a.M - 1) * a.K;
+  long long row[FT];
+#pragma unroll
+  for (int f = 0; f < FT; ++f)
+    row[f] = (long long)min(n0 + 16 * f + col, N - 1) * a.K;
+
+  const int chunks = a.K / CH;
+  const int mine = (chunks - wid + NW - 1) / NW;    // wid, wid + NW, ..
+  Weights<I8> w[D][S];
+  s16x8 x[D][CH / 32];
+  auto load = [&](int d, int i) __attribute__((always_inline)) {
+    const int at = (wid + min(i, mine - 1) * NW) * CH;
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      w[d][s].load(a.w[layer + s / FT], row[s % FT] + at, g);
+#pragma unroll
+    for (int k = 0; k < CH / 32; ++k)
+      x[d][k] = *(const s16x8*)(xp + at + input_at<I8>(k, g));
+  };
+  f32x4 acc[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (mine > 0)
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, d);
+  if (I8) {
+    for (int e = threadIdx.x; e < chunks * S * 16; e += NW * 64) {
+      const int c = e / (S * 16), f = e % (S * 16);
+      const long long r = min(n0 + f % (16 * FT), N - 1);
+      scales[e] = a.scales[layer + f / (16 * FT)][(r * a.K + c * CH) / a.group];
+    }
+    // not __syncthreads: that waits for the loads above as well
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+  auto use = [&](int d, int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      f32x4 part = I8 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[s];
+#pragma unroll
+      for (int k = 0; k < CH / 32; ++k)
+        part = mfma(w[d][s].operand(k), x[d][k], part);
+      if (I8) {     // of the rows 4 g + r that the lane holds the sums of
+        const f32x4 sc = *(const f32x4*)(
+            scales + ((wid + i * NW) * S + s) * 16 + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[s][r] += part[r] * sc[r];
+      } else {
+        acc[s] = part;
+      }
+    }
+  };
+  if (mine > 0) {
+    int i = 0;
+    for (; i + D < mine; i += D)
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        use(d, i + d);
+        load(d, i + d + D);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (i + d < mine) use(d, i + d);
+  }
+
+  // ---- add the waves up; features 4 g + r of a column lie side by side
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    *(f32x4*)(sums + (wid * S + s) * 256 + col * 16 + 4 * g) = acc[s];
+  __syncthreads();
+  for (int e = threadIdx.x; e < FT * 256; e += NW * 64) {
+    const int f = e >> 8, at = e & 255;
+    const int r = at >> 4, n = n0 + 16 * f + (at & 15);
+    if (r >= a.M || n >= N) continue;
+    float y[L];
+#pragma unroll
+    for (int s = 0; s < L; ++s) {
+      float t = 0.f;
+#pragma unroll
+      for (int w_ = 0; w_ < NW; ++w_)
+        t += sums[(w_ * S + s * FT + f) * 256 + at];
+      if (a.bias[layer + s]) t += value(a.bias[layer + s][n]);
+      y[s] = t;
+    }
+    float o = y[0];
+    if (MODE == SWIGLU) o = y[0] / (1.f + expf(-y[0])) * y[L - 1];
+    a.out[layer][(long long)r * N + n] = bits(o);
+  }
+}
+
+template <bool I8, int MODE, int FT, int D, int OCC>
+int launch_few(Args a, int layers, hipStream_t st) {
+  int tiles = 0;
+  for (int i = 0; i < (MODE == SWIGLU ? 1 : layers); ++i)
+    a.tile_end[i] = tiles += (a.n[i] + 16 * FT - 1) / (16 * FT);
+  constexpr int S = (MODE == SWIGLU ? 2 : 1) * FT;
+  const int lds = NW * S * 1024 + (I8 ? a.K / CH * S * 64 : 0);
+  auto kernel = few_rows_kernel<I8, MODE, FT, D, OCC>;
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(
+        (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return (int)e;
+  }
+  hipLaunchKernelGGL(kernel, dim3(tiles), dim3(NW * 64), lds, st, a);
+  return (int)hipGetLastError();
+}
+
 template <bool I8, int MT, int MODE, int FT>
-void launch(Args a, int layers, hipStream_t st) {
+int launch(Args a, int layers, hipStream_t st) {
   int tiles = 0;
   for (int i = 0; i < (MODE == SWIGLU ? 1 : layers); ++i)
     a.tile_end[i] = tiles += (a.n[i] + 16 * FT - 1) / (16 * FT);
   hipLaunchKernelGGL((rows_linear_kernel<I8, MT, MODE, FT>), dim3(tiles),
                      dim3(NW * 64), 0, st, a);
+  return (int)hipGetLastError();
 }
 
 // Tiles of features a wave. Every workgroup reads all of x, which costs M rows
-// out of L2 for 16 FT features of W: with more rows FT has to grow, but half
-// the workgroups leave CUs idle where the layer is small. Measured (us, bf16,
-// FT 1 / 2 / 4): M 8: N 4096 10.8 / 13.8 / 37, N 14336 29.2 / 29.2 / 51;
-// M 16: N 6144 19.5 / 17.0 / 40, N 14336 35.7 / 31.5 / 52; M 32: N 4096 15.7 /
-// 18.6 / 25, N 6144 26.1 / 20.3 / 25.5, N 14336 48 / 36.5 / 29.6. Gate and up
-// (two streams share x): M 16 52.6 / 92, M 32 61.9 / 55.1. int8, for which x
-// weighs twice as much, is within a tenth of its best by the same rule: M 8: N
-// 4096 8.3 / 10.8 / 18, N 6144 13.0 / 11.8 / 19, N 14336 20.7 / 20.9 / 20.1; M
-// 16: N 6144 15.4 / 12.8 / 20, N 14336 25.9 / 23.0 / 20.8, N 128256 176 / 163 /
-// 152; M 32: N 6144 23 / 16.3 / 23, N 14336 40 / 29.7 / 24.0; M 64: N 4096 21.1 /
-// 23.8 / 44, N 14336 74 / 46 / 51; gate and up M 8 35.9 / 34.8, M 16 39.5 / 37.2,
-// M 32 53.8 / 42.6, M 64 88 / 67.
+// out of L2 for 16 FT features of W; half the workgroups leave CUs idle where the
+// layer is small. Up to 16 rows (us, FT 1 / 2): N 4096 bf16 9.6 / 13, int8 8.6 /
+// 10.4; N 6144 15.7 / 13.3 and 12.3 / 10.8; N 128256 8 rows 205 / 192 and 148 /
+// 121, 16 rows 250 / 209 and 178 / 139, but bf16 1 row 168 / 178; gate and up,
+// whose two streams share x, 45.8 / 50.7 and 32.8 / 34.1. With two tiles bf16
+// has four chunks ahead (N 6144 13.3, two 14.5), int8 two (10.8, four 11.5).
+// More rows, int8 (FT 1 / 2 / 4): M 32: N 4096 11 / 14 / 20, N 6144 23 / 16.3 /
+// 23, N 14336 40 / 29.7 / 24.0; M 64: N 4096 21.1 / 23.8 / 44, N 14336 74 / 46 /
+// 51; gate and up M 32 53.8 / 42.6, M 64 88 / 67.
 template <bool I8>
-void launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
+int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
   int tiles = 0;
   for (int i = 0; i < layers; ++i) tiles += (a.n[i] + 15) / 16;
   const bool big = tiles >= 384, huge = tiles >= 896;
-  if (mode == SWIGLU) {
-    if (a.M <= 16) launch<I8, 1, SWIGLU, 1>(a, layers, st);
-    else if (a.M <= 32) launch<I8, 2, SWIGLU, 2>(a, layers, st);
-    else if (I8) launch<true, 4, SWIGLU, 2>(a, layers, st);
-  } else if (a.M <= 16) {
-    if (a.M > 8 && big) launch<I8, 1, PLAIN, 2>(a, layers, st);
-    else launch<I8, 1, PLAIN, 1>(a, layers, st);
-  } else if (a.M <= 32) {
-    if (huge) launch<I8, 2, PLAIN, 4>(a, layers, st);
-    else if (big) launch<I8, 2, PLAIN, 2>(a, layers, st);
-    else launch<I8, 2, PLAIN, 1>(a, layers, st);
-  } else if (I8) {
-    if (big) launch<true, 4, PLAIN, 2>(a, layers, st);
-    else launch<true, 4, PLAIN, 1>(a, layers, st);
+  // int8's scales in LDS: beside the sums 64 bytes a chunk and stream
+  if (a.M <= 16 && (!I8 || a.K <= 1 << 16)) {
+    if (mode == SWIGLU) return launch_few<I8, SWIGLU, 1, 2, 4>(a, layers, st);
+    if (big && (I8 || a.M > 4 || tiles < 2048))
+      return launch_few<I8, PLAIN, 2, I8 ? 2 : 4, I8 ? 4 : 2>(a, layers, st);
+    return launch_few<I8, PLAIN, 1, 2, 4>(a, layers, st);
   }
+  if (mode == SWIGLU) {
+    if (a.M <= 32) return launch<I8, 2, SWIGLU, 2>(a, layers, st);
+    return launch<true, 4, SWIGLU, 2>(a, layers, st);
+  }
+  if (a.M <= 32) {
+    if (huge) return launch<I8, 2, PLAIN, 4>(a, layers, st);
+    if (big) return launch<I8, 2, PLAIN, 2>(a, layers, st);
+    return launch<I8, 2, PLAIN, 1>(a, layers, st);
+  }
+  if (big) return launch<true, 4, PLAIN, 2>(a, layers, st);
+  return launch<true, 4, PLAIN, 1>(a, layers, st);
 }
 
 }  // namespace
 
 // layers: 1..3 weights on one input; mode 1: silu(layer 0) * layer 1. K and,
 // int8, the group are multiples of 256: a chunk of a feature has one scale.
-extern "C" void ds_rows_linear(const void* x, int layers, const void* const* w,
-                               const float* const* scales,
-                               const void* const* bias, void* const* out,
-                               const int* n, int M,
-                               int K, int group, int mode,
-                               void* stream) {
+// M up to 32, int8 64. Returns a hipError_t.
+extern "C" int ds_rows_linear(const void* x, int layers, const void* const* w,
+                              const float* const* scales,
+                              const void* const* bias, void* const* out,
+                              const int* n, int M, int K, int group, int mode,
+                              void* stream) {
   Args a = {};
   for (int i = 0; i < layers; ++i) {
     a.w[i] = w[i];
@@ -290,6 +417,6 @@ extern "C" void ds_rows_linear(const void* x, int layers, const void* const* w,
   a.x = (const short*)x;
   a.M = M; a.K = K; a.group = group;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (scales) launch_rows<true>(a, layers, mode, st);
-  else launch_rows<false>(a, layers, mode, st);
+  return scales ? launch_rows<true>(a, layers, mode, st)
+                : launch_rows<false>(a, layers, mode, st);
 }

@@ -1,0 +1,29 @@
+"""Linear layers of up to 16 rows where chunks of inputs end unevenly among the
+waves, features in a tile, and scales past what is kept in LDS, against fp64."""
+
+import pytest
+import torch
+
+from deepspeed_amd.ops.linear import SWIGLU, rows_linear
+from tests.test_rows_linear import _close, _layer
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("k", [256, 768, 1280, 2048, 2304, 4352, 65536, 65792])
+@pytest.mark.parametrize("m", [1, 5, 16])
+@torch.no_grad()
+def test_few_rows_gpu(int8, k, m):
+    g = torch.Generator().manual_seed(k + m)
+    x = torch.randn(m, k, generator=g).bfloat16().cuda()
+    # one tile a wave and two, gate and up
+    for ns, mode in (((17,), 0), ((6145, 3, 16), 0), ((33, 33), SWIGLU)):
+        if k > 5000 and ns[0] > 1000:
+            ns = (33, 3)
+        both = [_layer(n, k, i == 0, int8, g) for i, n in enumerate(ns)]
+        got = rows_linear(x, [b[0] for b in both], mode)
+        want = [f(x) for _, f in both]
+        if mode == SWIGLU:
+            want = [torch.nn.functional.silu(want[0]) * want[1]]
+        for y, w in zip(got, want):
+            _close(y, w)
