@@ -545,15 +545,11 @@ class PagedKVCache:
                 positions=None, scale=None):
         """New rows into the pool, then attention over it: three launches (two
         where no history is split) for the whole step."""
-        from ..ops.paged_attention import (StepPlan, aligned, paged_append,
+        from ..ops.paged_attention import (aligned, paged_append,
                                            paged_attention)
         kp, vp = self.k[layer_idx], self.v[layer_idx]
         n, S, H, D = q.shape
-        plan = self._plans.get((H, kp.size(1)))
-        if plan is None:
-            plan = self._plans[H, kp.size(1)] = StepPlan.build(
-                *self._row_places(), self.block_table, self.block_size, H,
-                kp.size(1), kp.device)
+        plan = self._plan(H, kp.size(1))
         q, k, v = (aligned(x.reshape(n * S, -1, D)) for x in (q, k, v))
         q = paged_append(plan, q, k, v, kp, vp, cos, sin, positions, S)
         o = paged_attention(plan, q, kp, vp, scale)
@@ -587,6 +583,42 @@ class PagedKVCache:
             positions = positions.contiguous()
         return self._attend(layer_idx, q, k, v, cos, sin, positions, scale)
 
+    def layers_plan(self, x, heads: int, kv_heads: int, positions=None):
+        """The step's plan if whole decoder layers on the residual stream x
+        [n, S, H] may append to and attend over the pools themselves, as
+        ``rope_attention`` would for each of them; None otherwise."""
+        own = self.__dict__
+        if self._mask_given or self._slots is None or \
+                type(self) is not PagedKVCache or \
+                any(getattr(PagedKVCache, name) is not f or name in own
+                    for name, f in _METHODS.items()) or \
+                not untransformed() or (
+                    positions is not None and (
+                        positions.dtype != torch.int32
+                        or not positions.is_cuda
+                        or not positions.is_contiguous()
+                        or positions.numel() != x.size(0) * x.size(1))):
+            return None
+        for kp, vp in zip(self.k, self.v):
+            if not kp.is_cuda or kp.dtype != torch.bfloat16 or \
+                    vp.dtype != torch.bfloat16 or kp.shape != vp.shape or \
+                    kp.size(1) != kv_heads or kp.size(3) != 128 or \
+                    not kp.is_contiguous() or not vp.is_contiguous() or \
+                    (kp.data_ptr() | vp.data_ptr()) % 16:
+                return None
+        if heads % kv_heads or not 1 <= heads // kv_heads <= 16:
+            return None
+        return self._plan(heads, kv_heads)
+
+    def _plan(self, heads: int, kv_heads: int):
+        from ..ops.paged_attention import StepPlan
+        plan = self._plans.get((heads, kv_heads))
+        if plan is None:
+            plan = self._plans[heads, kv_heads] = StepPlan.build(
+                *self._row_places(), self.block_table, self.block_size, heads,
+                kv_heads, self.k[0].device)
+        return plan
+
     def decode_attention(self, layer_idx: int, q, k, v, scale=None):
         """Single-token decode THROUGH the paged pool: writes the new
         token's k/v into its block and attends over the block lists — the
@@ -606,3 +638,9 @@ class PagedKVCache:
             self.lens[idx] += self._q_len
         self._slots = None
         self._forget_step()
+
+
+# What ``layers_plan`` stands for: replaced, they are called.
+_METHODS = {name: getattr(PagedKVCache, name) for name in (
+    "rope_attention", "_attend", "_eligible", "_replaced", "_row_places",
+    "_plan", "update", "decode_attention")}

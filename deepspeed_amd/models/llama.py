@@ -17,6 +17,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from ..ops import linear as _linear
+from ..ops._loader import get_ext
 from ..ops.attention import rope_flash_attention
 from ..ops.linear import (SWIGLU, Linear, call, movable, rows_linear,
                           tile_linear, unhooked)
@@ -114,6 +116,7 @@ def llama_mini():
                        num_kv_heads=4, max_seq_len=4096)
 
 
+@movable
 class LlamaAttention(nn.Module):
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
@@ -237,6 +240,7 @@ def sdpa_gqa(q, k, v, causal=True, attn_mask=None):
                                               is_causal=causal)
 
 
+@movable
 class LlamaMLP(nn.Module):
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
@@ -290,6 +294,67 @@ class LlamaDecoderLayer(nn.Module):
         return x + delta
 
 
+# What ``_native_layer`` stands for: replaced, they are called.
+_CHAIN, _OUT = LlamaDecoderLayer.chain, LlamaAttention._out
+
+
+def _operands(layer, rows: int):
+    """What a decoder layer brings to ``paged_decoder_layer``, or None where its
+    modules are to be called: (norm weights, their eps, linear weights, scales,
+    biases, group)."""
+    attn, mlp = layer.self_attn, layer.mlp
+    if type(attn) is not LlamaAttention or type(mlp) is not LlamaMLP or \
+            not unhooked(attn) or not unhooked(mlp) or \
+            "chain" in layer.__dict__ or "_out" in attn.__dict__ or \
+            attn.head_dim != 128:
+        return None
+    norms = layer.input_layernorm, layer.post_attention_layernorm
+    H = attn.num_heads * 128
+    weights, scales, biases, group = [], [], [], 0
+    for norm in norms:
+        if type(norm) is not RMSNorm or not unhooked(norm, internal_ok=True):
+            return None
+        w = norm.weight
+        if w.dtype is not torch.bfloat16 or not w.is_contiguous():
+            return None
+    mods = (attn.q_proj, attn.k_proj, attn.v_proj, attn.o_proj, mlp.gate_proj,
+            mlp.up_proj, mlp.down_proj)
+    kind = type(mods[0])
+    K = H
+    for m in mods:
+        if type(m) is not kind or not unhooked(m):
+            return None
+        if m is mods[6]:
+            K = n
+        if kind is Linear or kind is nn.Linear:
+            w = m.weight
+            if type(w) is not nn.Parameter or \
+                    w.dtype is not torch.bfloat16 or w.dim() != 2 or \
+                    w.shape[1] != K:
+                return None
+        elif hasattr(kind, "int8_rows"):
+            p = m.int8_rows(K) if rows <= _linear.ROWS_INT8 else None
+            if p is None or p[2] % 256 or group not in (0, p[2]):
+                return None
+            w, scale, group = p
+            scales.append(scale)
+        else:
+            return None
+        n, b = w.numel() // K, m.bias
+        if K % 256 or n % 4 or not w.is_contiguous() or w.data_ptr() % 16 or (
+                b is not None and (b.dtype is not torch.bfloat16
+                                   or not b.is_contiguous())):
+            return None
+        weights.append(w)
+        biases.append(b)
+    n = [w.numel() // H for w in weights[:6]]
+    if n != [H, attn.num_kv_heads * 128, n[1], H, n[4], n[4]] or \
+            weights[6].numel() != H * n[4]:
+        return None
+    return ([norms[0].weight, norms[1].weight], norms[0].eps, norms[1].eps,
+            weights, scales, biases, group)
+
+
 class LlamaModel(nn.Module):
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
@@ -310,17 +375,49 @@ class LlamaModel(nn.Module):
         if recompute:
             from ..runtime.activation_checkpointing import checkpoint
         delta = None
+        plan = self._paged_plan(x, positions, kv_cache)
         for layer in self.layers:
             if recompute:
                 x = checkpoint(lambda x_, l=layer: l(x_, cos, sin, positions,
                                                      kv_cache), x)
             elif type(layer) is LlamaDecoderLayer and unhooked(layer):
+                ops = plan and _operands(layer, x.shape[0] * x.shape[1])
+                if ops:
+                    at = layer.self_attn.layer_idx
+                    x, delta = get_ext().paged_decoder_layer(
+                        x, delta, *ops, cos, sin, positions, x.shape[1],
+                        kv_cache.k[at], kv_cache.v[at], plan.dst, plan.meta,
+                        plan.items, plan.runs, plan.merges, plan.any_merge,
+                        plan.nq, 128 ** -0.5)
+                    kv_cache.last_decoded = x.shape[1] == 1
+                    continue
                 x, delta = layer.chain(x, delta, cos, sin, positions,
                                        kv_cache)
             else:
                 x = x if delta is None else x + delta
                 x, delta = layer(x, cos, sin, positions, kv_cache), None
         return add_norm(self.norm, x, delta)[0]
+
+    def _paged_plan(self, x, positions, kv_cache):
+        """The plan of a serving step whose layers may run as native calls of
+        nine launches each, or None. A step of few tokens is bound by the host
+        otherwise (one request, four layers: 740 us of host time for 640 us of
+        kernels)."""
+        cfg = self.cfg
+        if not hasattr(kv_cache, "layers_plan") or torch.is_grad_enabled() or \
+                type(x) is not torch.Tensor or not x.is_cuda or \
+                x.dtype is not torch.bfloat16 or not x.numel() or \
+                x.shape[-1] != cfg.num_heads * 128 or x.shape[-1] > 16384 or \
+                not x.is_contiguous() or x.data_ptr() % 16 or \
+                get_ext() is None or torch.is_autocast_enabled() or \
+                torch.compiler.is_compiling() or \
+                LlamaDecoderLayer.chain is not _CHAIN or \
+                LlamaAttention._out is not _OUT or \
+                rows_linear is not _linear.rows_linear or \
+                tile_linear is not _linear.tile_linear:
+            return None
+        return kv_cache.layers_plan(x, cfg.num_heads, cfg.num_kv_heads,
+                                    positions)
 
     def gradient_checkpointing_enable(self):
         self.gradient_checkpointing = True

@@ -835,6 +835,66 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> add_norm_fwd(
   return {y, sum, inv};
 }
 
+// A decoder layer of a serving step over the paged pool, from the residual
+// stream x [.., H] that still lacks the last layer's output delta, to the same:
+// norm, q k v, rotation and append, attention, output, norm, gated MLP. What the
+// modules of models/llama.py call one by one, without their host time between
+// the launches (a layer of nine 180 us there, 45 here). norms: two weights.
+// weights: q, k, v, o, gate, up, down; int8 with scales. meta.. nq: StepPlan.
+std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
+    at::Tensor x, c10::optional<at::Tensor> delta,
+    const std::vector<at::Tensor>& norms, double eps0, double eps1,
+    const std::vector<at::Tensor>& weights,
+    const std::vector<at::Tensor>& scales,
+    const std::vector<c10::optional<at::Tensor>>& biases, int64_t group,
+    at::Tensor cos_table, at::Tensor sin_table,
+    c10::optional<at::Tensor> positions, int64_t S, at::Tensor kpool,
+    at::Tensor vpool, at::Tensor dst, at::Tensor meta, int64_t n_items,
+    int64_t n_runs, int64_t n_merges, bool any_merge, int64_t nq,
+    double scale) {
+  const OneDevice on("paged_decoder_layer", x, delta, cos_table, sin_table,
+                     positions, kpool, vpool, dst, meta);
+  TORCH_CHECK(norms.size() == 2 && weights.size() == 7 && biases.size() == 7 &&
+              (scales.empty() || scales.size() == 7) && x.is_contiguous() &&
+              x.numel() > 0 && x.scalar_type() == at::kBFloat16 &&
+              kpool.dim() == 4, "paged_decoder_layer");
+  const int64_t H = x.size(-1), M = x.numel() / H;
+  auto linears = [&](const at::Tensor& in, int first, int count,
+                     int64_t mode) {
+    const std::vector<at::Tensor> w(weights.begin() + first,
+                                    weights.begin() + first + count);
+    const std::vector<c10::optional<at::Tensor>> b(
+        biases.begin() + first, biases.begin() + first + count);
+    if (!scales.empty() || M <= 32) {
+      std::vector<at::Tensor> s;
+      if (!scales.empty())
+        s.assign(scales.begin() + first, scales.begin() + first + count);
+      return rows_linear(in, w, s, b, group, mode);
+    }
+    // as tile_linear in ops/linear.py has it
+    if (count == 1 && M >= 2560 && in.size(1) < 16384)
+      return std::vector<at::Tensor>{at::linear(in, w[0], b[0])};
+    return tile_linear(in, w, b, mode, -1, 1);
+  };
+  at::Tensor stream = x.view({M, H}), h;
+  if (delta.has_value())
+    std::tie(h, stream, std::ignore) = add_norm_fwd(
+        delta->view({M, H}), stream, norms[0], eps0);
+  else
+    h = std::get<0>(norm_fwd(stream, norms[0], c10::nullopt, eps0, false));
+  auto qkv = linears(h, 0, 3, 0);
+  for (auto& t : qkv) t = t.view({M, -1, 128});
+  auto q = paged_append(qkv[0], qkv[1], qkv[2], kpool, vpool, dst, cos_table,
+                        sin_table, positions, S);
+  auto o = paged_rows(q, kpool, vpool, meta, n_items, n_runs, n_merges,
+                      any_merge, nq, scale);
+  auto a = linears(o.view({M, -1}), 3, 1, 0)[0];
+  std::tie(h, stream, std::ignore) = add_norm_fwd(a, stream, norms[1], eps1);
+  h = linears(h, 4, 2, 1)[0];
+  h = linears(h, 6, 1, 0)[0];
+  return {stream.view(x.sizes()), h.view(x.sizes())};
+}
+
 at::Tensor token_gather(at::Tensor x, at::Tensor idx) {
   TORCH_CHECK(x.dim() == 3 && x.is_cuda() && x.is_contiguous(),
               "token_gather: contiguous [B,S,D] GPU tensor");
@@ -1161,6 +1221,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         pybind11::arg("dy"), pybind11::arg("x"), pybind11::arg("w"),
         pybind11::arg("invrms"), pybind11::arg("mean"),
         pybind11::arg("layernorm"), pybind11::arg("dres") = c10::nullopt);
+  m.def("paged_decoder_layer", &paged_decoder_layer,
+        "a decoder layer of a serving step over the paged pool");
   m.def("add_norm_fwd", &add_norm_fwd, "RMS norm of a sum, and the sum");
   m.def("rope", &rope, "Rotary position embedding of one or two tensors",
         pybind11::arg("x"), pybind11::arg("x2"), pybind11::arg("cos"),

@@ -1,0 +1,128 @@
+"""Serving steps whose decoder layers run as native calls: the same outputs and
+cache as the modules give one by one (GPU), and what keeps the modules called
+(CPU)."""
+
+import pytest
+import torch
+import torch.nn as nn
+
+from deepspeed_amd.inference.ragged import PagedKVCache
+from deepspeed_amd.linear.optimized_linear import (QuantizationConfig,
+                                                   WOQLinear)
+from deepspeed_amd.models import llama
+
+
+def _model(device, bias=False, int8=False):
+    torch.manual_seed(0)
+    cfg = llama.LlamaConfig(vocab_size=500, hidden_size=512,
+                            intermediate_size=768, num_layers=3, num_heads=4,
+                            num_kv_heads=2, max_seq_len=512,
+                            attention_bias=bias)
+    model = llama.LlamaForCausalLM(cfg).to(device, torch.bfloat16).eval()
+    model.requires_grad_(False)
+    if bias:
+        for p in model.named_parameters():
+            if p[0].endswith("bias"):
+                p[1].normal_()
+    if int8:
+        for m in list(model.modules()):
+            for name, lin in list(m.named_children()):
+                if isinstance(lin, nn.Linear):
+                    setattr(m, name, WOQLinear(lin, QuantizationConfig()))
+    return model, cfg
+
+
+def test_operands():
+    """A hook, a replaced forward, another class anywhere in the layer: its
+    modules are called."""
+    model, _ = _model("cpu")
+    layer = model.model.layers[0]
+    assert llama._operands(layer, 1) is not None
+    for m in (layer.self_attn, layer.mlp, layer.input_layernorm,
+              layer.self_attn.o_proj, layer.mlp.down_proj):
+        h = m.register_forward_hook(lambda *a: None)
+        assert llama._operands(layer, 1) is None
+        h.remove()
+        m.forward = lambda x: x
+        assert llama._operands(layer, 1) is None
+        del m.forward
+    own = type("Own", (llama.LlamaMLP,), {})
+    layer.mlp.__class__ = own
+    assert llama._operands(layer, 1) is None
+    layer.mlp.__class__ = llama.LlamaMLP
+    layer.chain = lambda *a: a
+    assert llama._operands(layer, 1) is None
+    del layer.chain
+    layer.mlp.up_proj = nn.Linear(512, 768, bias=False)
+    assert llama._operands(layer, 1) is None
+    model, _ = _model("cpu", int8=True)
+    assert llama._operands(model.model.layers[0], 64) is not None
+    assert llama._operands(model.model.layers[0], 65) is None
+
+
+def test_plan_is_the_caches_own():
+    """With methods of another kind, a mask of the caller's or outside a step
+    there is no plan."""
+    x = torch.zeros(1, 1, 512)
+    cache = PagedKVCache(1, 1, 2, 64, 128)
+    assert cache.layers_plan(x, 4, 2) is None
+    cache.begin_step([0], 1)
+    cache.last_mask = None
+    assert cache.layers_plan(x, 4, 2) is None
+    sub = type("Sub", (PagedKVCache,), {})(1, 1, 2, 64, 128)
+    sub.begin_step([0], 1)
+    assert sub.layers_plan(x, 4, 2) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["plain", "bias", "int8"])
+@pytest.mark.parametrize("positions", [False, True])
+@torch.no_grad()
+def test_same_as_modules_gpu(kind, positions, monkeypatch):
+    model, cfg = _model("cuda", kind == "bias", kind == "int8")
+    # prompt portions, single tokens, both packed; rows on either side of each
+    # kernel's line
+    steps = [([0], 20, None), ([1], 33, None), ([2], 130, None),
+             ([0, 1, 2], 1, None), ([2] * 2 + [0] * 30, 1,
+                                    [0, 1] + list(range(30))), ([1], 1, None)]
+    calls = []
+    native = llama.get_ext().paged_decoder_layer
+
+    class Ext:
+        def __getattr__(self, name):
+            return getattr(ext, name)
+
+        def paged_decoder_layer(self, *a):
+            calls.append(1)
+            return native(*a)
+
+    ext = llama.get_ext()
+    monkeypatch.setattr(llama, "get_ext", Ext)
+    out = []
+    for own in (True, False):
+        if not own:
+            monkeypatch.setattr(llama.LlamaModel, "_paged_plan",
+                                lambda *a: None)
+        g = torch.Generator().manual_seed(1)
+        cache = PagedKVCache(3, 3, 2, 512, 128, dtype=torch.bfloat16,
+                             device="cuda")
+        got = []
+        for slots, n, offsets in steps:
+            if offsets is not None and not positions:
+                continue            # rows of one slot stand at their own places
+            ids = torch.randint(0, 500, (len(slots), n), generator=g)
+            start = cache.lens[slots]
+            if offsets is not None:
+                start = start + torch.tensor(offsets)
+            pos = (start[:, None] + torch.arange(n)).int().cuda()
+            cache.begin_step(slots, n, offsets=offsets)
+            got.append(model(ids.cuda(), positions=pos if positions else None,
+                             kv_cache=cache))
+            assert cache.last_decoded == (n == 1)
+            cache.end_step()
+        out.append(got + cache.k + cache.v)
+    rows = [len(s) * n for s, n, o in steps if positions or o is None]
+    want = sum(3 for r in rows if kind != "int8" or r <= 64)
+    assert len(calls) == want
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
