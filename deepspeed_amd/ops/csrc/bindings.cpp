@@ -87,7 +87,7 @@ extern "C" void ds_paged_append(const void* q, const void* k, const void* v,
                                 const int* dst, const float* cs,
                                 const float* sn, const int* positions, int T,
                                 int S, int H, int Hkv, int BS, void* stream);
-extern "C" void ds_paged_rows(const void* q, const void* kpool,
+extern "C" int ds_paged_rows(const void* q, const void* kpool,
                               const void* vpool, const int* table,
                               const int* runs, const int* items,
                               const int* merges, const int* lens, void* out,
@@ -391,12 +391,13 @@ at::Tensor paged_decode(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
   auto part_ml = at::empty({splits > 1 ? items * Hkv * 16 * 2 : 0}, f32);
   auto o = at::empty_like(q);
   if (n == 0) return o;
-  ds_paged_rows(q.data_ptr(), kpool.data_ptr(), vpool.data_ptr(),
-                block_table.data_ptr<int>(), nullptr, nullptr, nullptr,
-                lens.data_ptr<int>(), o.data_ptr(), part.data_ptr<float>(),
-                part_ml.data_ptr<float>(), (int)items, n, splits > 1, 1, H,
-                Hkv, BS, (int)block_table.size(1), (int)splits, (float)scale,
-                cur_stream());
+  const int e = ds_paged_rows(
+      q.data_ptr(), kpool.data_ptr(), vpool.data_ptr(),
+      block_table.data_ptr<int>(), nullptr, nullptr, nullptr,
+      lens.data_ptr<int>(), o.data_ptr(), part.data_ptr<float>(),
+      part_ml.data_ptr<float>(), (int)items, n, splits > 1, 1, H, Hkv, BS,
+      (int)block_table.size(1), (int)splits, (float)scale, cur_stream());
+  TORCH_CHECK(e == 0, "paged_decode: launch failed, hipError_t ", e);
   return o;
 }
 
@@ -411,7 +412,7 @@ at::Tensor paged_rows(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
   TORCH_CHECK(meta.scalar_type() == at::kInt && meta.is_cuda() &&
               meta.is_contiguous() &&
               meta.numel() >= 4 * n_items + 4 * n_runs + 2 * n_merges &&
-              (nq == 1 || nq == 2), "paged_rows: plan");
+              (nq == 1 || nq == 2 || nq == 8), "paged_rows: plan");
   const int H = q.size(1), Hkv = kpool.size(1);
   const int* p = meta.data_ptr<int>();
   auto f32 = q.options().dtype(at::kFloat);
@@ -420,12 +421,14 @@ at::Tensor paged_rows(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
   auto part_ml = at::empty({cols * 2}, f32);
   auto o = at::empty_like(q);
   if (n_items == 0) return o;
-  ds_paged_rows(q.data_ptr(), kpool.data_ptr(), vpool.data_ptr(),
-                p + 4 * (n_items + n_runs) + 2 * n_merges, p + 4 * n_items, p,
-                p + 4 * (n_items + n_runs), nullptr, o.data_ptr(),
-                part.data_ptr<float>(), part_ml.data_ptr<float>(),
-                (int)n_items, (int)n_merges, any_merge, (int)nq, H, Hkv,
-                (int)kpool.size(2), 0, 0, (float)scale, cur_stream());
+  const int e = ds_paged_rows(
+      q.data_ptr(), kpool.data_ptr(), vpool.data_ptr(),
+      p + 4 * (n_items + n_runs) + 2 * n_merges, p + 4 * n_items, p,
+      p + 4 * (n_items + n_runs), nullptr, o.data_ptr(),
+      part.data_ptr<float>(), part_ml.data_ptr<float>(), (int)n_items,
+      (int)n_merges, any_merge, (int)nq, H, Hkv, (int)kpool.size(2), 0, 0,
+      (float)scale, cur_stream());
+  TORCH_CHECK(e == 0, "paged_rows: launch failed, hipError_t ", e);
   return o;
 }
 

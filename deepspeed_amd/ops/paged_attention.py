@@ -19,6 +19,14 @@ from ._loader import get_ext
 WORKGROUPS = 1024
 # Keys of the shortest split: one tile of 32 for each of a workgroup's waves.
 MIN_SPLIT = 128
+# Items of 128 columns (rows times heads a key head), eight waves of them a CU,
+# take steps of runs of BLOCK columns and more each that have BLOCK_WORK columns
+# times keys times key heads. us, 32 on 8 heads, tiles of 32 columns and of 128:
+# 16 rows behind 4000 23 / 23, 32 behind 1500 19 / 20 and 4000 29 / 26, 64 behind
+# 600 19 / 21 and 1500 26 / 25, 256 behind 64 19 / 23 and 600 37 / 30, 1024 behind
+# 1500 112 / 82, 2048 behind 4000 445 / 290. Beside decoding requests a launch of
+# their own is no gain (24 of 1000 and 200 rows 60 / 75).
+BLOCK, BLOCK_WORK, CUS = 64, 1 << 21, 256
 
 
 def paged_decode_available(q: torch.Tensor, kpool: torch.Tensor) -> bool:
@@ -97,9 +105,12 @@ class StepPlan:
         kv_len = pos[row0] + m
         runs = np.stack([row0, m, kv_len, offs[row0]], 1)
         G = heads // kv_heads
-        # columns (rows times heads a key head) go in tiles of 16; two tiles
-        # share the loads of a key tile where runs are long enough
+        # two tiles of 16 columns share the loads of a key tile where runs are
+        # long enough, eight where they are longer
         nq = 2 if int(m.max()) * G > 16 else 1
+        if int(m.min()) * G >= BLOCK and kv_heads * G * int(
+                (m * (kv_len - m // 2)).sum()) >= BLOCK_WORK:
+            nq = 8
         width = 16 * nq
         tiles = -(-m * G // width)
         run_of = np.repeat(np.arange(len(m)), tiles)
@@ -108,12 +119,23 @@ class StepPlan:
         tok = np.minimum((tile + 1) * width, m[run_of] * G) - 1
         end = kv_len[run_of] - m[run_of] + tok // G + 1
         # split long histories until the chip is full
-        if len(end) * kv_heads >= WORKGROUPS:
+        grain = 32
+        if nq == 8:
+            # the longest first; at most one round of workgroups, steps of 128
+            order = np.argsort(-end, kind="stable")
+            run_of, tile, end = run_of[order], tile[order], end[order]
+            room, per, grain = CUS // kv_heads, int(end[0]), MIN_SPLIT
+            if len(end) < room:
+                per = max(MIN_SPLIT, int(end.sum()) // room)
+                while per < end[0] and (-(-end // per)).sum() > room:
+                    per += MIN_SPLIT
+            n = -(-end // per)
+        elif len(end) * kv_heads >= WORKGROUPS:
             n = np.ones_like(end)
         else:
             per = max(MIN_SPLIT, int(end.sum()) * kv_heads // WORKGROUPS)
             n = -(-end // per)
-        step = -(-(-(-end // n)) // 32) * 32
+        step = -(-(-(-end // n)) // grain) * grain
         n = -(-end // step)
         of = np.repeat(np.arange(len(end)), n)
         first = np.cumsum(n) - n

@@ -303,3 +303,46 @@ def test_paged_decode_scales_and_splits(scale, splits):
                           torch.tensor([n - 1], device="cuda"), scale)
         err = (got[i:i + 1].double() - want).abs()
         assert (err <= 2.0 ** -8 * want.abs() + 2.0 ** -13).all(), err.max()
+
+
+@pytest.fixture
+def blocks(monkeypatch):
+    """Every run's items have 128 columns."""
+    from deepspeed_amd.ops import paged_attention as P
+    monkeypatch.setattr(P, "BLOCK", 1)
+    monkeypatch.setattr(P, "BLOCK_WORK", 0)
+
+
+@pytest.mark.parametrize("name", list(STEPS))
+@pytest.mark.parametrize("heads", [(14, 2), (32, 8)])
+def test_block_plan_covers_every_key_once(name, heads, blocks):
+    test_step_plan_covers_every_key_once(name, 64, heads)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(STEPS))
+@pytest.mark.parametrize("bs", [24, 64])
+@pytest.mark.parametrize("heads", [(1, 1), (14, 2), (32, 8)])
+def test_block_attention_gpu(name, bs, heads, blocks):
+    test_paged_attention_gpu(name, bs, heads)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [0.05, -0.05, 0.0])
+def test_block_scales(scale, blocks):
+    """Splits in which a column sees no key, and every key alike at scale 0."""
+    from deepspeed_amd.ops.paged_attention import paged_attention
+    torch.manual_seed(1)
+    slots, pos, _ = _rows([(0, 300)], [130])
+    table = torch.randperm(9)[:7]
+    plan = StepPlan.build(slots, pos, {0: table.tolist()}, 64, 14, 2, "cuda")
+    assert plan.nq == 8 and plan.any_merge
+    kp, vp = (torch.randn(9, 2, 64, 128, device="cuda").bfloat16()
+              for _ in range(2))
+    q = (4 * torch.randn(300, 14, 128, device="cuda")).bfloat16()
+    got = paged_attention(plan, q, kp, vp, scale)
+    kk, vv = (p[table.cuda()].transpose(1, 2).reshape(-1, 2, 128)[:430]
+              for p in (kp, vp))
+    want = _reference(q, kk, vv, torch.tensor(pos, device="cuda"), scale)
+    err = (got.double() - want).abs()
+    assert (err <= 2.0 ** -8 * want.abs() + 2.0 ** -13).all(), err.max()
