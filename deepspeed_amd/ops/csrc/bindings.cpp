@@ -614,16 +614,18 @@ std::vector<at::Tensor> tile_linear(
 
 // Gradients of linear layers y = x W^T on one input, bf16 (tile_linear.hip). mode
 // 2: of the input, the sum over the layers of dy W; mode 3: of each weight, dy^T
-// x. others: the weights, or the input alone.
-std::vector<at::Tensor> tile_linear_grad(const std::vector<at::Tensor>& dys,
-                                         const std::vector<at::Tensor>& others,
-                                         int mode, int tile, int splits) {
+// x, to `into` where that holds a tensor. others: the weights, or the input alone.
+std::vector<at::Tensor> tile_linear_grad(
+    const std::vector<at::Tensor>& dys, const std::vector<at::Tensor>& others,
+    int mode, int tile, int splits,
+    const std::vector<c10::optional<at::Tensor>>& into = {}) {
   const int L = dys.size();
   TORCH_CHECK(L >= 1 && L <= 3 && (int)others.size() == (mode == 2 ? L : 1),
               "tile_linear_grad: layers");
   const OneDevice on("tile_linear_grad", dys[0]);
   for (auto& t : dys) on.check(t);
   for (auto& t : others) on.check(t);
+  for (auto& t : into) on.check(t);
   const int64_t M = dys[0].size(0), K = others[0].size(1);
   const void *x[3], *w[3], *b[3] = {};
   void* o[3];
@@ -647,8 +649,14 @@ std::vector<at::Tensor> tile_linear_grad(const std::vector<at::Tensor>& dys,
     w[i] = other.data_ptr();
     n[i] = dys[i].size(1);
     all += n[i];
-    if (mode == 3 || i == 0)
-      out.push_back(at::empty({mode == 2 ? M : n[i], K}, dys[0].options()));
+    const int64_t rows = mode == 2 ? M : n[i];
+    if (i < (int)into.size() && into[i].has_value()) {
+      TORCH_CHECK(good(*into[i]) && into[i]->size(0) == rows &&
+                  into[i]->size(1) == K, "tile_linear_grad: into");
+      out.push_back(*into[i]);
+    } else if (mode == 3 || i == 0) {
+      out.push_back(at::empty({rows, K}, dys[0].options()));
+    }
     o[i] = out.back().data_ptr();
   }
   TORCH_CHECK(K <= (1 << 22) && M < (1 << 30) && all < (1ll << 31),
@@ -678,8 +686,10 @@ at::Tensor tile_linear_dx(std::vector<at::Tensor> dys,
 
 std::vector<at::Tensor> tile_linear_dw(at::Tensor x,
                                        std::vector<at::Tensor> dys,
-                                       int64_t tile, int64_t splits) {
-  return tile_linear_grad(dys, {x}, 3, (int)tile, (int)splits);
+                                       int64_t tile, int64_t splits,
+                                       std::vector<c10::optional<at::Tensor>>
+                                           into) {
+  return tile_linear_grad(dys, {x}, 3, (int)tile, (int)splits, into);
 }
 
 at::Tensor sum_of_squares(std::vector<at::Tensor> ts) {
@@ -1182,7 +1192,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("weights"), py::arg("tile") = -1, py::arg("splits") = 1);
   m.def("tile_linear_dw", &tile_linear_dw, "weights' gradients",
         py::arg("x"), py::arg("dys"), py::arg("tile") = -1,
-        py::arg("splits") = 1);
+        py::arg("splits") = 1,
+        py::arg("into") = std::vector<c10::optional<at::Tensor>>());
   m.def("sum_of_squares", &sum_of_squares,
         "sum of squares over a list of tensors");
   m.def("paged_rows", &paged_rows,

@@ -131,20 +131,54 @@ def _dx(dys, weights, own: bool):
     return dx
 
 
-def _dw(x, dys, own: bool):
-    """dy^T x of the layers."""
+class GradSlot:
+    """Where the gradient of a parameter belongs: ``view``, a part of its owner's
+    flat buffer, set as the parameter's ``_ds_grad_slot``. While it is ``open``
+    (the owner's backward, no gradient there yet) the product of the parameter's
+    one layer may be written into it. Autograd then keeps that very tensor as the
+    gradient, where it added a new one to the buffer: two reads and a write of
+    every weight's gradient, 20 us for 25M values.
+
+    uses: forward products since the owner's last backward; a weight of several
+    keeps to the addition. void: the owner took the gradient away, and what the
+    buffer holds is not part of what arrives."""
+
+    __slots__ = ("view", "uses", "open", "void")
+
+    def __init__(self, view):
+        self.view = view
+        self.uses = 0
+        self.open = self.void = False
+
+    def __reduce__(self):       # a saved module's parameters have none
+        return _nothing, ()
+
+    def take(self):
+        if not self.open or self.uses != 1:
+            return None
+        self.open = False
+        return self.view.detach()
+
+
+def _nothing():
+    return None
+
+
+def _dw(x, dys, own: bool, slots):
+    """dy^T x of the layers, in their slots where these are open."""
     T, K = x.shape
+    into = [slot and slot.take() for slot in slots] if own else [None] * len(dys)
     if own and all(own_products(T, dy.shape[1], K)[1] for dy in dys) and \
             _aligned(x, *dys):
-        return get_ext().tile_linear_dw(x, dys)
+        return get_ext().tile_linear_dw(x, dys, into=into)
     dws = []
-    for dy in dys:
+    for dy, out in zip(dys, into):
         dy_t = x_t = False
         if own:
             _, dy_t, x_t = backward_plan(T, dy.shape[1], K)
         a = _transposed(dy) if dy_t else dy.t()
         b = _transposed(x).t() if x_t else x
-        dws.append(a @ b)
+        dws.append(a @ b if out is None else torch.mm(a, b, out=out))
     return dws
 
 
@@ -154,7 +188,8 @@ class _Linears(torch.autograd.Function):
     ``own_products`` are csrc/tile_linear.hip's, with the input's gradient summed
     over the layers in the product; for the others operands are transposed where
     ``backward_plan`` says. Kept for the backward is what it needs: a frozen layer
-    holds no input. ``own``: the forward product may be the kernel's as well."""
+    holds no input. ``own``: the forward product may be the kernel's as well.
+    Weights' gradients go to their ``GradSlot``."""
 
     @staticmethod
     def forward(ctx, x, own, *params):
@@ -163,6 +198,10 @@ class _Linears(torch.autograd.Function):
         ctx.save_for_backward(x if any(need[2::2]) else None,
                               *(w if need[0] else None for w in weights))
         ctx.shape, ctx.features = x.shape, [w.shape for w in weights]
+        for w in weights:
+            slot = getattr(w, "_ds_grad_slot", None)
+            if slot is not None:
+                slot.uses += 1
         if own:
             out = _forward(x, weights, biases)
         else:
@@ -192,7 +231,8 @@ class _Linears(torch.autograd.Function):
             x2 = x.reshape(-1, K)
             if own:
                 x2 = x2.contiguous()
-            for i, dw in zip(some, _dw(x2, [dys[i] for i in some], own)):
+            slots = [getattr(weights[i], "_ds_grad_slot", None) for i in some]
+            for i, dw in zip(some, _dw(x2, [dys[i] for i in some], own, slots)):
                 grads[2 * i] = dw
         for i, dy in enumerate(dys):
             if need[3 + 2 * i]:

@@ -37,6 +37,7 @@ from ... import comm as dist
 from ...utils.logging import log_dist
 from ..fp16.loss_scaler import LossScalerBase, LossScaler
 from ...ops.grad_norm import sum_of_squares
+from ...ops.linear import GradSlot
 from ..utils import ALIGNMENT
 from ...utils.nvtx import instrument_w_nvtx
 
@@ -44,7 +45,7 @@ from ...utils.nvtx import instrument_w_nvtx
 class _Bucket:
     __slots__ = ("group_idx", "index", "flat", "grad_flat", "params", "offsets",
                  "numel", "shard_size", "pending", "reduced", "comm_event",
-                 "master_offset", "pg", "pg_rank", "pg_world")
+                 "master_offset", "pg", "pg_rank", "pg_world", "clean")
 
     def __init__(self, group_idx, index, numel, shard_size):
         self.group_idx = group_idx
@@ -56,6 +57,7 @@ class _Bucket:
         self.params: List[torch.nn.Parameter] = []
         self.offsets: List[int] = []
         self.pending = 0
+        self.clean = None       # version of grad_flat in which it is all zeros
         self.reduced = False
         self.comm_event = None
         self.master_offset = 0  # offset of this bucket's shard in the group master
@@ -123,6 +125,8 @@ class ZeroStage12Optimizer:
         self._local = (self.world_size == 1 and not cpu_offload and all(
             dist.get_world_size(self._group_pg(g)) == 1
             for g in self.optimizer.param_groups))
+        self._slots = []        # (parameter, its GradSlot, its bucket)
+        self._opened = []
         self._build_flat_buffers()
         self._replace_inner_params()
         self._register_hooks()
@@ -210,7 +214,11 @@ class ZeroStage12Optimizer:
                     p.data = b.flat[off:off + p.numel()].view_as(p.data)
                     if gdtype == dtype:
                         p.grad = b.grad_flat[off:off + p.numel()].view_as(p.data)
+                        if p.dim() == 2 and p.grad.data_ptr() % 16 == 0:
+                            p._ds_grad_slot = GradSlot(p.grad)
+                            self._slots.append((p, p._ds_grad_slot, b))
                     self.param_to_bucket[p] = b
+                b.clean = b.grad_flat._version
                 b.master_offset = shard_total
                 shard_total += b.shard_size
                 self.buckets.append(b)
@@ -261,16 +269,43 @@ class ZeroStage12Optimizer:
                     expected.add_(param.grad.detach().view(-1)
                                   .to(expected.dtype))
                     param.grad = None
-            elif param.grad is not None and \
-                    param.grad.data_ptr() != expected.data_ptr():
-                expected.add_(param.grad.detach().view(-1))
-                param.grad = expected.view_as(param)
+            elif param.grad is not None:
+                self._place(param, expected)
             if not self.is_gradient_accumulation_boundary:
                 return
             bucket.pending -= 1
             if bucket.pending == 0:
+                if not self._local:
+                    self._place_late(bucket)
                 self._reduce_bucket(bucket)
         return hook
+
+    @staticmethod
+    def _place(param, expected):
+        """A gradient has arrived: to its place, if it is not there."""
+        slot = getattr(param, "_ds_grad_slot", None)
+        there = param.grad.data_ptr() == expected.data_ptr()
+        if slot is not None and slot.void and (there or slot.open):
+            if not there:
+                expected.copy_(param.grad.detach().view(-1))
+            slot.open = slot.void = False
+        elif slot is not None and slot.void:
+            # A product has written to the place, and this is a sum with what it
+            # wrote or another pass's gradient, which that has still to be added
+            # to: it stays where it is until all have arrived.
+            return
+        elif not there:
+            expected.add_(param.grad.detach().view(-1))
+        if not there:
+            param.grad = expected.view_as(param)
+
+    def _place_late(self, bucket=None):
+        for p, slot, b in self._opened:
+            if (bucket is None or b is bucket) and slot.void and \
+                    not slot.open and p.grad is not None:
+                slot.view.copy_(p.grad.detach())
+                p.grad = slot.view
+                slot.void = False
 
     def _try_fused_adam(self):
         try:
@@ -376,10 +411,45 @@ class ZeroStage12Optimizer:
 
     def backward(self, loss, retain_graph=False):
         self.micro_step_id += 1
-        if self.custom_loss_scaler:
-            (loss * self.external_loss_scale).backward(retain_graph=retain_graph)
-        else:
-            self.loss_scaler.backward(loss.float(), retain_graph=retain_graph)
+        self._open_slots()
+        try:
+            if self.custom_loss_scaler:
+                (loss * self.external_loss_scale).backward(
+                    retain_graph=retain_graph)
+            else:
+                self.loss_scaler.backward(loss.float(),
+                                          retain_graph=retain_graph)
+        finally:
+            self._close_slots()
+
+    def _open_slots(self):
+        """Products write the first gradients of their weights into the flat
+        buffers, where nothing has been added to these since they were cleared:
+        the parameter has no gradient then until that one arrives. A parameter
+        whose gradient hooks see keeps to the addition."""
+        for p, slot, b in self._slots:
+            g = p.grad
+            if slot.uses == 1 and b.clean == b.grad_flat._version and \
+                    g is not None and g.dtype == slot.view.dtype and \
+                    g.data_ptr() == slot.view.data_ptr() and \
+                    not p._backward_hooks:
+                p.grad = None
+                slot.open = slot.void = True
+                self._opened.append((p, slot, b))
+        for _, _, b in self._opened:
+            b.clean = None      # the kernels' writes do not count as versions
+
+    def _close_slots(self):
+        self._place_late()
+        for p, slot, _ in self._opened:
+            if slot.void and not slot.open:     # written, but not handed on
+                slot.view.zero_()
+            slot.open = slot.void = False
+            if p.grad is None:
+                p.grad = slot.view
+        self._opened.clear()
+        for _, slot, _ in self._slots:
+            slot.uses = 0
 
     @instrument_w_nvtx
     def reduce_gradients(self):
@@ -541,6 +611,7 @@ class ZeroStage12Optimizer:
         # grads are views into flat buffers: zero in place, keep the views.
         for b in self.buckets:
             b.grad_flat.zero_()
+            b.clean = b.grad_flat._version
 
     # --------------------------------------------------------------- plumbing
 
