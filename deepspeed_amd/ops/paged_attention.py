@@ -60,6 +60,16 @@ def paged_decode_attention(q: torch.Tensor, kpool: torch.Tensor,
                             lens.contiguous().int(), splits, scale)
 
 
+def _to_device(values: np.ndarray, device) -> torch.Tensor:
+    """As int32, in the order of the device's current stream. From pageable memory
+    the host would wait there for all that the stream still has to do, the whole
+    step before; torch gives the pinned block to nobody else before it is read."""
+    pinned = torch.device(device).type == "cuda"
+    out = torch.empty(len(values), dtype=torch.int32, pin_memory=pinned)
+    out.numpy()[:] = values
+    return out.to(device, non_blocking=pinned)
+
+
 @dataclass
 class StepPlan:
     """One serving step for the kernels: where each new row goes (``dst``) and
@@ -146,9 +156,8 @@ class StepPlan:
         items = np.stack([run_of[of], tile[of], lo, hi], 1)
         merges = np.stack([first, n], 1)
         head = 4 * len(items) + 4 * len(runs) + 2 * len(merges) + len(flat)
-        both = torch.from_numpy(np.concatenate(
-            [items.ravel(), runs.ravel(), merges.ravel(), flat, dst]).astype(
-                np.int32)).to(device)
+        both = _to_device(np.concatenate(
+            [items.ravel(), runs.ravel(), merges.ravel(), flat, dst]), device)
         return cls(dst=both[head:], meta=both, items=len(items),
                    runs=len(runs), merges=len(merges),
                    any_merge=bool((n > 1).any()), nq=nq)

@@ -346,3 +346,19 @@ def test_block_scales(scale, blocks):
     want = _reference(q, kk, vv, torch.tensor(pos, device="cuda"), scale)
     err = (got.double() - want).abs()
     assert (err <= 2.0 ** -8 * want.abs() + 2.0 ** -13).all(), err.max()
+
+
+@pytest.mark.gpu
+def test_plans_made_ahead_of_the_gpu():
+    """The host goes on while a plan is on its way: later ones do not touch it."""
+    plans, want = [], []
+    a = torch.randn(4096, 4096, device="cuda")
+    for _ in range(20):
+        a = a @ a * 1e-2
+    for n in range(1, 9):
+        args = ([0] * n, np.arange(5, 5 + n), {0: [n, 7]}, 16, 8, 2)
+        plans.append(StepPlan.build(*args, "cuda"))
+        want.append(StepPlan.build(*args, "cpu"))
+    for p, w in zip(plans, want):
+        assert torch.equal(p.meta.cpu(), w.meta)
+        assert torch.equal(p.dst.cpu(), w.dst)
