@@ -376,21 +376,30 @@ class LlamaModel(nn.Module):
             from ..runtime.activation_checkpointing import checkpoint
         delta = None
         plan = self._paged_plan(x, positions, kv_cache)
-        for layer in self.layers:
+        layers = list(self.layers)
+
+        def operands(i):
+            if plan is None or i == len(layers) or \
+                    type(layers[i]) is not LlamaDecoderLayer or \
+                    not unhooked(layers[i]):
+                return None
+            return _operands(layers[i], x.shape[0] * x.shape[1])
+
+        after = operands(0)
+        for i, layer in enumerate(layers):
+            ops, after = after, operands(i + 1)
             if recompute:
                 x = checkpoint(lambda x_, l=layer: l(x_, cos, sin, positions,
                                                      kv_cache), x)
+            elif ops:
+                at = layer.self_attn.layer_idx
+                x, delta = get_ext().paged_decoder_layer(
+                    x, delta, *ops, cos, sin, positions, x.shape[1],
+                    kv_cache.k[at], kv_cache.v[at], plan.dst, plan.meta,
+                    plan.items, plan.runs, plan.merges, plan.any_merge,
+                    plan.nq, 128 ** -0.5, after is not None)
+                kv_cache.last_decoded = x.shape[1] == 1
             elif type(layer) is LlamaDecoderLayer and unhooked(layer):
-                ops = plan and _operands(layer, x.shape[0] * x.shape[1])
-                if ops:
-                    at = layer.self_attn.layer_idx
-                    x, delta = get_ext().paged_decoder_layer(
-                        x, delta, *ops, cos, sin, positions, x.shape[1],
-                        kv_cache.k[at], kv_cache.v[at], plan.dst, plan.meta,
-                        plan.items, plan.runs, plan.merges, plan.any_merge,
-                        plan.nq, 128 ** -0.5)
-                    kv_cache.last_decoded = x.shape[1] == 1
-                    continue
                 x, delta = layer.chain(x, delta, cos, sin, positions,
                                        kv_cache)
             else:

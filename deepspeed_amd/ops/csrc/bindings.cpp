@@ -29,6 +29,10 @@ extern "C" void ds_norm_fwd(const void* x, const void* w, const void* b,
 extern "C" void ds_add_norm_fwd(const void* x, const void* res, const void* w,
                                 void* sum, void* y, float* invrms, int rows,
                                 int H, float eps, int dtype, void* stream);
+extern "C" void ds_add_norm_parts(const float* part, int splits,
+                                  const void* res, const void* w, void* sum,
+                                  void* y, int rows, int H, float eps,
+                                  void* stream);
 extern "C" long long ds_norm_bwd_parts(const void* dy, const void* x,
                                        const void* dres, const void* dx,
                                        int rows, int H, int ln, int dtype);
@@ -83,10 +87,11 @@ extern "C" void ds_flash_bwd(const void* q, const void* k, const void* v,
                              int B, int S, int H, int Hkv, int D, float scale,
                              int causal, void* stream);
 extern "C" void ds_paged_append(const void* q, const void* k, const void* v,
-                                void* qout, void* kpool, void* vpool,
-                                const int* dst, const float* cs,
-                                const float* sn, const int* positions, int T,
-                                int S, int H, int Hkv, int BS, void* stream);
+                                const float* part, int splits, void* qout,
+                                void* kpool, void* vpool, const int* dst,
+                                const float* cs, const float* sn,
+                                const int* positions, int T, int S, int H,
+                                int Hkv, int BS, void* stream);
 extern "C" int ds_paged_rows(const void* q, const void* kpool,
                               const void* vpool, const int* table,
                               const int* runs, const int* items,
@@ -107,7 +112,7 @@ extern "C" int ds_tile_linear(const void* const* x, int layers,
                               const void* const* w, const void* const* bias,
                               void* const* out, const int* n, int M, int K,
                               int mode, int tile, int splits, float* part,
-                              void* stream);
+                              int merge, void* stream);
 extern "C" void ds_transpose_bf16(const void* src, void* dst, int n_batch,
                                   int R, int C, long long row_stride,
                                   int inner, long long inner_stride,
@@ -432,28 +437,21 @@ at::Tensor paged_rows(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
   return o;
 }
 
-// New rows k, v [T, Hkv, 128] into the pool rows dst [T]; with tables also
-// the rotary embedding of k on its way there and of q [T, H, 128], returned.
-at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
-                        at::Tensor kpool, at::Tensor vpool, at::Tensor dst,
-                        c10::optional<at::Tensor> cos_table,
-                        c10::optional<at::Tensor> sin_table,
-                        c10::optional<at::Tensor> positions, int64_t S) {
-  const OneDevice on("paged_append", q, k, v, kpool, vpool, dst, cos_table,
-                     sin_table, positions);
-  check_pool(q, kpool, vpool, "paged_append");
+// What both forms below share; q of T rows and H heads: its values, or what it
+// is like.
+at::Tensor append_rows(const at::Tensor& q, const void* k, const void* v,
+                       const void* q_or_bias, const float* part, int splits,
+                       at::Tensor kpool, at::Tensor vpool, at::Tensor dst,
+                       c10::optional<at::Tensor> cos_table,
+                       c10::optional<at::Tensor> sin_table,
+                       c10::optional<at::Tensor> positions, int64_t S,
+                       at::Tensor out) {
   const int T = q.size(0), H = q.size(1), Hkv = kpool.size(1);
-  for (auto& x : {k, v})
-    TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
-                x.is_contiguous() && x.dim() == 3 && x.size(0) == T &&
-                x.size(1) == Hkv && x.size(2) == 128 &&
-                ((uintptr_t)x.data_ptr() & 15) == 0, "paged_append: k/v");
   TORCH_CHECK(dst.scalar_type() == at::kInt && dst.is_cuda() &&
               dst.is_contiguous() && dst.numel() == T, "paged_append: dst");
   TORCH_CHECK(S >= 1 && T % S == 0, "paged_append: S");
   const float *cs = nullptr, *sn = nullptr;
   const int* pos = nullptr;
-  at::Tensor out = q;
   if (cos_table.has_value()) {
     for (auto& t : {*cos_table, *sin_table})
       TORCH_CHECK(t.scalar_type() == at::kFloat && t.is_cuda() &&
@@ -469,14 +467,33 @@ at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
     } else {
       TORCH_CHECK(cos_table->size(0) >= S, "table shorter than sequence");
     }
-    out = at::empty_like(q);
   }
   if (T == 0) return out;
-  ds_paged_append(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+  ds_paged_append(q_or_bias, k, v, part, splits, out.data_ptr(),
                   kpool.data_ptr(), vpool.data_ptr(), dst.data_ptr<int>(), cs,
                   sn, pos, T, (int)S, H, Hkv, (int)kpool.size(2),
                   cur_stream());
   return out;
+}
+
+// New rows k, v [T, Hkv, 128] into the pool rows dst [T]; with tables also
+// the rotary embedding of k on its way there and of q [T, H, 128], returned.
+at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
+                        at::Tensor kpool, at::Tensor vpool, at::Tensor dst,
+                        c10::optional<at::Tensor> cos_table,
+                        c10::optional<at::Tensor> sin_table,
+                        c10::optional<at::Tensor> positions, int64_t S) {
+  const OneDevice on("paged_append", q, k, v, kpool, vpool, dst, cos_table,
+                     sin_table, positions);
+  check_pool(q, kpool, vpool, "paged_append");
+  for (auto& x : {k, v})
+    TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
+                x.is_contiguous() && x.dim() == 3 && x.size(0) == q.size(0) &&
+                x.size(1) == kpool.size(1) && x.size(2) == 128 &&
+                ((uintptr_t)x.data_ptr() & 15) == 0, "paged_append: k/v");
+  return append_rows(q, k.data_ptr(), v.data_ptr(), q.data_ptr(), nullptr, 1,
+                     kpool, vpool, dst, cos_table, sin_table, positions, S,
+                     cos_table.has_value() ? at::empty_like(q) : q);
 }
 
 // bf16 weights on one input, pointers and features of each; outputs made anew:
@@ -513,9 +530,10 @@ struct Layers {
     TORCH_CHECK(mode == 0 || n[0] == n[i], what, ": gate and up");
   }
   // Whether tile_linear.hip takes them; does it if so. A tile and a number of
-  // splits may be asked for.
-  bool tiled(const at::Tensor& x, int64_t mode, int tile = -1,
-             int splits = 1) {
+  // splits may be asked for. With `parts`, sums in parts [splits, M, all] are left
+  // there, and the outputs are not written.
+  bool tiled(const at::Tensor& x, int64_t mode, int tile = -1, int splits = 1,
+             at::Tensor* parts = nullptr) {
     const int64_t M = x.size(0), K = x.size(1);
     if (K % 64 || K > (1 << 22) || M >= (1 << 30)) return false;
     for (int i = 0; i < count; ++i)
@@ -528,12 +546,14 @@ struct Layers {
       return false;
     at::Tensor part;
     if (splits > 1)
-      part = at::empty({splits * M * all}, x.options().dtype(at::kFloat));
+      part = at::empty({splits, M, all}, x.options().dtype(at::kFloat));
     const void* xs[1] = {x.data_ptr()};
     const int e = ds_tile_linear(
         xs, count, w, b, o, n, (int)M, (int)K, (int)mode, tile, splits,
-        splits > 1 ? part.data_ptr<float>() : nullptr, cur_stream());
+        splits > 1 ? part.data_ptr<float>() : nullptr, parts == nullptr,
+        cur_stream());
     TORCH_CHECK(e == 0, "tile_linear: launch failed with error ", e);
+    if (parts) *parts = part;
     return true;
   }
 };
@@ -673,7 +693,7 @@ std::vector<at::Tensor> tile_linear_grad(
                      dys[0].options().dtype(at::kFloat));
   const int e = ds_tile_linear(
       x, L, w, b, o, n, (int)M, (int)K, mode, tile, splits,
-      splits > 1 ? part.data_ptr<float>() : nullptr, cur_stream());
+      splits > 1 ? part.data_ptr<float>() : nullptr, 1, cur_stream());
   TORCH_CHECK(e == 0, "tile_linear_grad: launch failed with error ", e);
   return out;
 }
@@ -854,6 +874,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> add_norm_fwd(
 // modules of models/llama.py call one by one, without their host time between
 // the launches (a layer of nine 180 us there, 45 here). norms: two weights.
 // weights: q, k, v, o, gate, up, down; int8 with scales. meta.. nq: StepPlan.
+// Products whose contraction is split leave their sums in parts to what reads
+// them next: the append, the norms, and with `parts` the next layer's, whose
+// delta is fp32 [splits, rows, H] then.
 std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
     at::Tensor x, c10::optional<at::Tensor> delta,
     const std::vector<at::Tensor>& norms, double eps0, double eps1,
@@ -864,7 +887,7 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
     c10::optional<at::Tensor> positions, int64_t S, at::Tensor kpool,
     at::Tensor vpool, at::Tensor dst, at::Tensor meta, int64_t n_items,
     int64_t n_runs, int64_t n_merges, bool any_merge, int64_t nq,
-    double scale) {
+    double scale, bool parts) {
   const OneDevice on("paged_decoder_layer", x, delta, cos_table, sin_table,
                      positions, kpool, vpool, dst, meta);
   TORCH_CHECK(norms.size() == 2 && weights.size() == 7 && biases.size() == 7 &&
@@ -889,23 +912,73 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
       return std::vector<at::Tensor>{at::linear(in, w[0], b[0])};
     return tile_linear(in, w, b, mode, -1, 1);
   };
+  // outputs, or their sums in parts
+  using Sums = std::pair<std::vector<at::Tensor>, at::Tensor>;
+  auto sums = [&](const at::Tensor& in, int first, int count) -> Sums {
+    if (!scales.empty() || M <= 16 ||
+        (count == 1 && M >= 2560 && in.size(1) < 16384))
+      return {linears(in, first, count, 0), at::Tensor()};
+    Layers y;
+    at::Tensor part;
+    for (int i = first; i < first + count; ++i)
+      y.add("paged_decoder_layer", in, weights[i], biases[i], at::kBFloat16, 0);
+    if (!y.tiled(in, 0, -1, 1, &part))
+      return {linears(in, first, count, 0), at::Tensor()};
+    return {y.out, part};
+  };
   at::Tensor stream = x.view({M, H}), h;
+  auto add_norm = [&](const at::Tensor& d, const at::Tensor& w, double eps) {
+    if (d.scalar_type() != at::kFloat) {
+      std::tie(h, stream, std::ignore) =
+          add_norm_fwd(d.view({M, H}), stream, w, eps);
+      return;
+    }
+    TORCH_CHECK(d.dim() == 3 && d.size(1) == M && d.size(2) == H &&
+                d.is_contiguous() && w.is_contiguous() && w.numel() == H &&
+                w.scalar_type() == at::kBFloat16 && H % 8 == 0 &&
+                H <= 16384 && ((uintptr_t)stream.data_ptr() & 15) == 0,
+                "paged_decoder_layer: norm");
+    auto sum = at::empty_like(stream);
+    h = at::empty_like(stream);
+    ds_add_norm_parts(d.data_ptr<float>(), (int)d.size(0), stream.data_ptr(),
+                      w.data_ptr(), sum.data_ptr(), h.data_ptr(), (int)M,
+                      (int)H, (float)eps, cur_stream());
+    stream = sum;
+  };
+  for (auto& w : norms) on.check(w);
   if (delta.has_value())
-    std::tie(h, stream, std::ignore) = add_norm_fwd(
-        delta->view({M, H}), stream, norms[0], eps0);
+    add_norm(*delta, norms[0], eps0);
   else
     h = std::get<0>(norm_fwd(stream, norms[0], c10::nullopt, eps0, false));
-  auto qkv = linears(h, 0, 3, 0);
+  at::Tensor q;
+  auto [qkv, qkv_part] = sums(h, 0, 3);
   for (auto& t : qkv) t = t.view({M, -1, 128});
-  auto q = paged_append(qkv[0], qkv[1], qkv[2], kpool, vpool, dst, cos_table,
-                        sin_table, positions, S);
+  check_pool(qkv[0], kpool, vpool, "paged_decoder_layer");
+  TORCH_CHECK(qkv[1].size(1) == kpool.size(1) &&
+              qkv[2].size(1) == kpool.size(1), "paged_decoder_layer: heads");
+  if (qkv_part.defined()) {
+    const void* b[3];
+    for (int i = 0; i < 3; ++i)
+      b[i] = biases[i].has_value() ? biases[i]->data_ptr() : nullptr;
+    q = append_rows(qkv[0], b[1], b[2], b[0], qkv_part.data_ptr<float>(),
+                    (int)qkv_part.size(0), kpool, vpool, dst, cos_table,
+                    sin_table, positions, S, qkv[0]);
+  } else {
+    q = paged_append(qkv[0], qkv[1], qkv[2], kpool, vpool, dst, cos_table,
+                     sin_table, positions, S);
+  }
   auto o = paged_rows(q, kpool, vpool, meta, n_items, n_runs, n_merges,
                       any_merge, nq, scale);
-  auto a = linears(o.view({M, -1}), 3, 1, 0)[0];
-  std::tie(h, stream, std::ignore) = add_norm_fwd(a, stream, norms[1], eps1);
-  h = linears(h, 4, 2, 1)[0];
-  h = linears(h, 6, 1, 0)[0];
-  return {stream.view(x.sizes()), h.view(x.sizes())};
+  // the norm of sums in parts takes no bias
+  auto output = [&](const at::Tensor& in, int i, bool in_parts) {
+    if (!in_parts || biases[i].has_value()) return linears(in, i, 1, 0)[0];
+    auto [y, part] = sums(in, i, 1);
+    return part.defined() ? part : y[0];
+  };
+  add_norm(output(o.view({M, -1}), 3, true), norms[1], eps1);
+  h = output(linears(h, 4, 2, 1)[0], 6, parts);
+  return {stream.view(x.sizes()),
+          h.scalar_type() == at::kFloat ? h : h.view(x.sizes())};
 }
 
 at::Tensor token_gather(at::Tensor x, at::Tensor idx) {

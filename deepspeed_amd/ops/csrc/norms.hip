@@ -35,6 +35,82 @@ constexpr int VEC = 8;  // bf16 per 16B load
 // LN: also subtract mean. Saves fp32 invrms (and mean for LN) for backward.
 // ---------------------------------------------------------------------------
 
+// A row whose elements c.. c + VEC - 1 `load` brings. The weight is read with
+// the row, not behind the reduction: one wait for memory instead of two.
+template <typename T, bool LN, int ITERS, bool RES, typename Load>
+__device__ __forceinline__ void norm_row(Load load, const long long at,
+                                         const T* res, T* sum_out, const T* w,
+                                         const T* b, T* y, float* invrms_out,
+                                         float* mean_out, const int row,
+                                         const int H, const float eps,
+                                         float* red) {
+  using VecT = ds::bf16x8;  // same layout for f16 via reinterpret of 16B
+  const bool mine = threadIdx.x < BLOCK;
+  const bool vec = (reinterpret_cast<uintptr_t>(w) & 15) == 0;
+  float xv[ITERS][VEC];
+  T wv[ITERS][VEC];
+  float sum = 0.f, sumsq = 0.f;
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int c = (it * BLOCK + threadIdx.x) * VEC;
+    if (mine && c < H) {
+      if (vec)
+        *reinterpret_cast<VecT*>(wv[it]) =
+            *reinterpret_cast<const VecT*>(w + c);
+      else
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) wv[it][j] = w[c + j];
+      T v[VEC], r[VEC];
+      if (RES)
+        *reinterpret_cast<VecT*>(r) =
+            *reinterpret_cast<const VecT*>(res + at + c);
+      load(c, v);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        float f = ds::to_f32(v[j]);
+        if (RES) {
+          f += ds::to_f32(r[j]);
+          r[j] = ds::from_f32<T>(f);
+        }
+        xv[it][j] = f;
+        if (LN) sum += f;
+        sumsq += f * f;
+      }
+      if (RES)
+        *reinterpret_cast<VecT*>(sum_out + at + c) =
+            *reinterpret_cast<const VecT*>(r);
+    }
+  }
+  float mean = 0.f;
+  if (LN) {
+    mean = ds::block_reduce_sum<BLOCK>(sum, red) / H;
+    __syncthreads();
+  }
+  float var = ds::block_reduce_sum<BLOCK>(sumsq, red) / H;
+  if (LN) var -= mean * mean;
+  const float inv = rsqrtf(var + eps);
+  if (threadIdx.x == 0) {
+    if (invrms_out != nullptr) invrms_out[row] = inv;
+    if (LN) mean_out[row] = mean;
+  }
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int c = (it * BLOCK + threadIdx.x) * VEC;
+    if (mine && c < H) {
+      T out[VEC];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float f = xv[it][j];
+        float nw = (LN ? (f - mean) : f) * inv * ds::to_f32(wv[it][j]);
+        if (LN && b != nullptr) nw += ds::to_f32(b[c + j]);
+        out[j] = ds::from_f32<T>(nw);
+      }
+      *reinterpret_cast<VecT*>(y + at + c) =
+          *reinterpret_cast<const VecT*>(out);
+    }
+  }
+}
+
 template <typename T, bool LN, int ITERS, bool RES>
 __global__ void norm_fwd_cached_kernel(const T* __restrict__ x,
                                        const T* __restrict__ res,  // RES
@@ -47,66 +123,53 @@ __global__ void norm_fwd_cached_kernel(const T* __restrict__ x,
                                        const int rows, const int H,
                                        const float eps) {
   __shared__ float red[BLOCK / WAVE_SIZE];
-  using VecT = ds::bf16x8;  // same layout for f16 via reinterpret of 16B
   for (int row = blockIdx.x; row < rows; row += gridDim.x) {
-    const T* xr = x + (long long)row * H;
-    T* yr = y + (long long)row * H;
-    float xv[ITERS][VEC];
-    float sum = 0.f, sumsq = 0.f;
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-      const int c = (it * BLOCK + threadIdx.x) * VEC;
-      if (c < H) {
-        T v[VEC], r[VEC];
-        *reinterpret_cast<VecT*>(v) = *reinterpret_cast<const VecT*>(xr + c);
-        if (RES)
-          *reinterpret_cast<VecT*>(r) = *reinterpret_cast<const VecT*>(
-              res + (long long)row * H + c);
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) {
-          float f = ds::to_f32(v[j]);
-          if (RES) {
-            f += ds::to_f32(r[j]);
-            r[j] = ds::from_f32<T>(f);
-          }
-          xv[it][j] = f;
-          if (LN) sum += f;
-          sumsq += f * f;
-        }
-        if (RES)
-          *reinterpret_cast<VecT*>(sum_out + (long long)row * H + c) =
-              *reinterpret_cast<const VecT*>(r);
-      }
-    }
-    float mean = 0.f;
-    if (LN) {
-      mean = ds::block_reduce_sum<BLOCK>(sum, red) / H;
-      __syncthreads();
-    }
-    float var = ds::block_reduce_sum<BLOCK>(sumsq, red) / H;
-    if (LN) var -= mean * mean;
-    const float inv = rsqrtf(var + eps);
-    if (threadIdx.x == 0) {
-      invrms_out[row] = inv;
-      if (LN) mean_out[row] = mean;
-    }
-#pragma unroll
-    for (int it = 0; it < ITERS; ++it) {
-      const int c = (it * BLOCK + threadIdx.x) * VEC;
-      if (c < H) {
-        T out[VEC];
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) {
-          const float f = xv[it][j];
-          float nw = (LN ? (f - mean) : f) * inv * ds::to_f32(w[c + j]);
-          if (LN && b != nullptr) nw += ds::to_f32(b[c + j]);
-          out[j] = ds::from_f32<T>(nw);
-        }
-        *reinterpret_cast<VecT*>(yr + c) = *reinterpret_cast<const VecT*>(out);
-      }
-    }
+    const long long at = (long long)row * H;
+    norm_row<T, LN, ITERS, RES>(
+        [&](int c, T* v) {
+          *reinterpret_cast<ds::bf16x8*>(v) =
+              *reinterpret_cast<const ds::bf16x8*>(x + at + c);
+        },
+        at, res, sum_out, w, b, y, invrms_out, mean_out, row, H, eps, red);
     __syncthreads();
   }
+}
+
+// The same of res + x where x is still in parts, part[splits][rows][H], that
+// tile_linear.hip's split contraction left: added up in their order and rounded
+// as its merge would, by all 1024 threads (the loads of 8 splits in flight) into
+// LDS, from where 256 go on as above. A launch and a pass less: 32 x 4096 5.5 us,
+// the merge and the norm 4.2 and 4.0 under the profiler, which shows the launches
+// longer than they are; four layers of 32 requests 895 -> 880 us with the append's.
+constexpr int WIDE = 1024;
+
+template <int ITERS>
+__global__ __launch_bounds__(WIDE) void add_norm_parts_kernel(
+    const float* __restrict__ part, const int splits,
+    const ds::bf16* __restrict__ res, ds::bf16* __restrict__ sum_out,
+    const ds::bf16* __restrict__ w, ds::bf16* __restrict__ y, const int rows,
+    const int H, const float eps) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  __shared__ float red[WIDE / WAVE_SIZE];
+  __shared__ __attribute__((aligned(16))) ds::bf16 x[ITERS * BLOCK * VEC];
+  const int row = blockIdx.x;
+  const long long at = (long long)row * H, step = (long long)rows * H;
+  for (int c = threadIdx.x * 4; c < H; c += WIDE * 4) {
+    f4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int s = 0; s < splits; ++s)
+      t += *reinterpret_cast<const f4*>(part + s * step + at + c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[c + e] = ds::from_f32<ds::bf16>(t[e]);
+  }
+  __syncthreads();
+  norm_row<ds::bf16, false, ITERS, true>(
+      [&](int c, ds::bf16* v) {
+        *reinterpret_cast<ds::bf16x8*>(v) =
+            *reinterpret_cast<const ds::bf16x8*>(x + c);
+      },
+      at, res, sum_out, w, (const ds::bf16*)nullptr, y, (float*)nullptr,
+      (float*)nullptr, row, H, eps, red);
 }
 
 // Generic fallback (any H, scalar loads, row re-read).
@@ -508,6 +571,25 @@ extern "C" void ds_add_norm_fwd(const void* x, const void* res, const void* w,
   if (dtype == 1) { BY_H(ds::bf16); }
   else { BY_H(ds::f16); }
 #undef BY_H
+#undef GO
+}
+
+// The same, bf16, with x in parts [splits][rows][H] fp32; no 1/rms.
+extern "C" void ds_add_norm_parts(const float* part, int splits,
+                                  const void* res, const void* w, void* sum,
+                                  void* y, int rows, int H, float eps,
+                                  void* stream) {
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int iters = (H + BLOCK * VEC - 1) / (BLOCK * VEC);
+#define GO(ITERS)                                                           \
+  hipLaunchKernelGGL((add_norm_parts_kernel<ITERS>), dim3(rows),            \
+                     dim3(WIDE), 0, s, part, splits, (const ds::bf16*)res,  \
+                     (ds::bf16*)sum, (const ds::bf16*)w, (ds::bf16*)y, rows,\
+                     H, eps)
+  if (iters <= 1) GO(1);
+  else if (iters <= 2) GO(2);
+  else if (iters <= 4) GO(4);
+  else GO(8);
 #undef GO
 }
 

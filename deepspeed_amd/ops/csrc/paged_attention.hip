@@ -676,10 +676,17 @@ __global__ __launch_bounds__(128) void merge_kernel(const Args a,
                              bits(o[2] * inv), bits(o[3] * inv)};
 }
 
-// Eight threads a head row of 128: coordinates j..j+7 and j+64..j+71 of it.
+// Eight threads a head row of 128: coordinates j..j+7 and j+64..j+71 of it. With
+// PARTS q, k and v are still in parts, part[splits][T][(H + 2 Hkv) 128], that
+// tile_linear.hip's split contraction left, added up here in their order, with
+// the bias and rounded as its merge would: a launch of 4 us at 32 requests less,
+// for one more in this one.
+template <bool PARTS>
 __global__ __launch_bounds__(256) void append_kernel(
     const short* __restrict__ q, const short* __restrict__ k,
-    const short* __restrict__ v, short* __restrict__ qout,
+    const short* __restrict__ v,         // PARTS: the biases, or null
+    const float* __restrict__ part, const int splits,
+    short* __restrict__ qout,
     short* __restrict__ kpool, short* __restrict__ vpool,
     const int* __restrict__ dst,         // [T] block * BS + row in it
     const float* __restrict__ cs, const float* __restrict__ sn,  // or null
@@ -692,23 +699,50 @@ __global__ __launch_bounds__(256) void append_kernel(
   const int j = (int)(i & 7) * 8;
   const int t = (int)(u / per);
   int h = (int)(u % per);
+  const int all = h;      // PARTS: the head among those of q, k and v
   const short* src;
   short* to;
   bool turn = cs != nullptr;
   if (cs && h < H) {
-    src = q + ((long long)t * H + h) * D;
+    src = PARTS ? (q ? q + h * D : nullptr) : q + ((long long)t * H + h) * D;
     to = qout + ((long long)t * H + h) * D;
   } else {
     if (cs) h -= H;
     const bool is_k = h < Hkv;
     if (!is_k) h -= Hkv;
-    src = (is_k ? k : v) + ((long long)t * Hkv + h) * D;
+    src = is_k ? k : v;
+    if (PARTS) src = src ? src + h * D : nullptr;
+    else src += ((long long)t * Hkv + h) * D;
     const int at = dst[t];
     to = (is_k ? kpool : vpool) +
          (((long long)(at / BS) * Hkv + h) * BS + at % BS) * D;
     turn = turn && is_k;
   }
-  s16x8 x1 = *(const s16x8*)(src + j), x2 = *(const s16x8*)(src + j + 64);
+  s16x8 x1, x2;
+  if (PARTS) {
+    f32x4 y[4] = {};
+    const float* p = part + ((long long)t * per + all) * D + j;
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s) {
+      const float* ps = p + (long long)s * T * per * D;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        y[e] += *(const f32x4*)(ps + (e >> 1) * 64 + (e & 1) * 4);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float a = y[e >> 2][e & 3], b = y[2 + (e >> 2)][e & 3];
+      if (src) {
+        a += value(src[j + e]);
+        b += value(src[j + 64 + e]);
+      }
+      x1[e] = bits(a);
+      x2[e] = bits(b);
+    }
+  } else {
+    x1 = *(const s16x8*)(src + j);
+    x2 = *(const s16x8*)(src + j + 64);
+  }
   if (turn) {
     const int pos = positions ? positions[t] : t % S;
     const float* cp = cs + (long long)pos * 64 + j;
@@ -758,17 +792,21 @@ int launch_rows(const Args& a, const int2* merges, int n_items, int n_merges,
 
 }  // namespace
 
+// part: null, or q, k and v in parts (then these are their biases, or null, and
+// there are tables).
 extern "C" void ds_paged_append(const void* q, const void* k, const void* v,
-                                void* qout, void* kpool, void* vpool,
-                                const int* dst, const float* cs,
-                                const float* sn, const int* positions, int T,
-                                int S, int H, int Hkv, int BS, void* stream) {
+                                const float* part, int splits, void* qout,
+                                void* kpool, void* vpool, const int* dst,
+                                const float* cs, const float* sn,
+                                const int* positions, int T, int S, int H,
+                                int Hkv, int BS, void* stream) {
   const long long threads = (long long)T * ((cs ? H : 0) + 2 * Hkv) * 8;
-  hipLaunchKernelGGL(append_kernel, dim3((unsigned)((threads + 255) / 256)),
+  auto kernel = part ? append_kernel<true> : append_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((threads + 255) / 256)),
                      dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                     (const short*)q, (const short*)k, (const short*)v,
-                     (short*)qout, (short*)kpool, (short*)vpool, dst, cs, sn,
-                     positions, T, S, H, Hkv, BS);
+                     (const short*)q, (const short*)k, (const short*)v, part,
+                     splits, (short*)qout, (short*)kpool, (short*)vpool, dst,
+                     cs, sn, positions, T, S, H, Hkv, BS);
 }
 
 // nq: tiles of 16 columns an item (1, 2 or 8). runs/items/merges null: `lens`

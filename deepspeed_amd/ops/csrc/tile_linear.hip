@@ -24,7 +24,7 @@
 //     fill the chip together; with SWIGLU a tile holds gate and up, 16 features
 //     of each in turn, and the activation is taken from the fp32 sums.
 //   * Where tiles leave CUs idle, the contraction is split; partial sums stay
-//     fp32 and are added in their order by a second kernel.
+//     fp32 and are added in their order by a second kernel, or by the next one.
 
 #include "ds_kernels.h"
 
@@ -521,7 +521,7 @@ __global__ __launch_bounds__(256) void tile_merge_kernel(const Args a,
 }
 
 template <int BM, int BN, int WM, int WN, int NS, int MODE>
-int launch(Args a, hipStream_t st) {
+int launch(Args a, bool merge, hipStream_t st) {
   constexpr int LDS = NS * (BM + BN) * ROW;
   static_assert(LDS <= 160 * 1024, "");
   constexpr int bn = MODE == SWIGLU ? BN / 2 : BN;
@@ -541,7 +541,7 @@ int launch(Args a, hipStream_t st) {
   if (e != hipSuccess) return (int)e;
   hipLaunchKernelGGL(kernel, dim3(a.tiles * a.mtiles * a.splits),
                      dim3(WM * WN * 64), LDS, st, a);
-  if (a.splits > 1) {
+  if (a.splits > 1 && merge) {
     const int n = a.n_end[a.layers - 1];
     const int rows = MODE == GRAD_W ? n : a.M, all = MODE >= GRAD_X ? a.K : n;
     const long long q = (long long)rows * (all / 4);
@@ -660,12 +660,14 @@ extern "C" int ds_tile_linear_stages(int tile, int mode) {
 // of eight. GRAD_W: w[0] is the input, x the gradients, out [n, K]; n and K are
 // multiples of eight. All operands at 16 bytes; bias only for the first two.
 // tile and splits from the plan; part: splits * rows * columns of all outputs,
-// null for one split. Returns a hipError_t.
+// null for one split; merge 0 leaves these for the next kernel to add up, in
+// their order and with the bias (norms.hip, paged_attention.hip). Returns a
+// hipError_t.
 extern "C" int ds_tile_linear(const void* const* x, int layers,
                               const void* const* w, const void* const* bias,
                               void* const* out, const int* n, int M, int K,
                               int mode, int tile, int splits, float* part,
-                              void* stream) {
+                              int merge, void* stream) {
   Args a = {};
   int total = 0;
   for (int i = 0; i < layers; ++i) {
@@ -682,14 +684,15 @@ extern "C" int ds_tile_linear(const void* const* x, int layers,
   switch (tile) {
 #define X(I, BM, BN, WM, WN, NS, U, F)                                    \
   case I:                                                                 \
-    if (mode == GRAD_X) return launch<BM, BN, WM, WN, NS, GRAD_X>(a, st); \
+    if (mode == GRAD_X)                                                   \
+      return launch<BM, BN, WM, WN, NS, GRAD_X>(a, merge, st);            \
     if (mode == GRAD_W)                                                   \
       return launch<BM, BN, WM, WN, NS,                                   \
-                    BLOCKS(BM, WM) ? GRAD_W : PLAIN>(a, st);              \
+                    BLOCKS(BM, WM) ? GRAD_W : PLAIN>(a, merge, st);       \
     if (mode == SWIGLU)                                                   \
       return launch<BM, BN, WM, WN, NS,                                   \
-                    GATES(BN, WN) ? SWIGLU : PLAIN>(a, st);               \
-    return launch<BM, BN, WM, WN, NS, PLAIN>(a, st);
+                    GATES(BN, WN) ? SWIGLU : PLAIN>(a, merge, st);        \
+    return launch<BM, BN, WM, WN, NS, PLAIN>(a, merge, st);
     TILES(X)
 #undef X
   }

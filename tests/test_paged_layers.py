@@ -126,3 +126,24 @@ def test_same_as_modules_gpu(kind, positions, monkeypatch):
     assert len(calls) == want
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["plain", "bias"])
+def test_sums_in_parts_gpu(kind, monkeypatch):
+    """Long contractions are split, and what reads their sums next adds them up."""
+    x = torch.zeros(20, 2048, device="cuda", dtype=torch.bfloat16)
+    w = torch.zeros(2048, 2048, device="cuda", dtype=torch.bfloat16)
+    with torch.profiler.profile() as prof:
+        llama.get_ext().tile_linear(x, [w], [None], 0)
+        torch.cuda.synchronize()
+    assert any("tile_merge" in e.key for e in prof.key_averages())
+
+    class Wide(llama.LlamaConfig):
+        def __init__(self, **kw):
+            for name in ("hidden_size", "intermediate_size", "num_heads"):
+                kw[name] *= 4
+            super().__init__(**kw)
+
+    monkeypatch.setattr(llama, "LlamaConfig", Wide)
+    test_same_as_modules_gpu(kind, True, monkeypatch)
