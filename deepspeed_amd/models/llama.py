@@ -471,11 +471,14 @@ def chunked_cross_entropy(hidden, lm_head, labels, chunk_tokens=8192):
     fp32 logits never exceed chunk_tokens x vocab. With DS_AMD_FUSED_CE=1
     the per-chunk softmax+nll runs as the fused bf16 HIP kernel and no
     fp32 logits are materialized at all."""
-    from ..ops.cross_entropy import fused_cross_entropy_sum
+    from ..ops.cross_entropy import (fused_cross_entropy_mean,
+                                     fused_cross_entropy_sum)
     B, S, H = hidden.shape
     hidden = hidden.reshape(-1, H)
     labels = labels.reshape(-1)
     n = hidden.shape[0]
+    if 0 < n <= chunk_tokens:
+        return fused_cross_entropy_mean(call(lm_head, hidden), labels)
     total = hidden.new_zeros((), dtype=torch.float32)
     count = hidden.new_zeros((), dtype=torch.float32)
     for s in range(0, n, chunk_tokens):

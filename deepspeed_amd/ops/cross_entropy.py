@@ -14,22 +14,26 @@ from ._loader import get_ext
 
 
 class _FusedCE(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, logits, labels, ignore_index):
-        ext = get_ext()
-        loss, lse = ext.ce_fwd(logits, labels, ignore_index)
-        ctx.save_for_backward(logits, labels, lse)
-        ctx.ignore_index = ignore_index
-        count = (labels != ignore_index).sum().float()
-        ctx.mark_non_differentiable(count)
-        return loss.sum(), count
+    """(sum of the rows' losses, labels that count), or with ``mean`` their
+    quotient; what torch makes of it takes ten launches more."""
 
     @staticmethod
-    def backward(ctx, gsum, _gcount):
-        logits, labels, lse = ctx.saved_tensors
-        gscale = gsum.expand(logits.size(0)).contiguous().float()
-        d = get_ext().ce_bwd(logits, labels, lse, gscale, ctx.ignore_index)
-        return d, None, None
+    def forward(ctx, logits, labels, ignore_index, mean=False):
+        total, count, quotient, lse = get_ext().ce_loss(logits, labels,
+                                                        ignore_index)
+        ctx.save_for_backward(logits, labels, lse, count if mean else None)
+        ctx.ignore_index = ignore_index
+        if mean:
+            return quotient
+        ctx.mark_non_differentiable(count)
+        return total, count
+
+    @staticmethod
+    def backward(ctx, g, _gcount=None):
+        logits, labels, lse, count = ctx.saved_tensors
+        d = get_ext().ce_bwd(logits, labels, lse, g.contiguous().float(),
+                             ctx.ignore_index, count)
+        return d, None, None, None
 
 
 def fused_ce_available(logits) -> bool:
@@ -52,3 +56,12 @@ def fused_cross_entropy_sum(logits, labels, ignore_index=-100):
                                              ignore_index=ignore_index,
                                              reduction="sum")
     return loss, (labels != ignore_index).sum().float()
+
+
+def fused_cross_entropy_mean(logits, labels, ignore_index=-100):
+    """The mean over the labels that count (0 without any)."""
+    if fused_ce_available(logits):
+        return _FusedCE.apply(logits.contiguous(), labels.contiguous(),
+                              ignore_index, True)
+    loss, count = fused_cross_entropy_sum(logits, labels, ignore_index)
+    return loss / count.clamp(min=1)

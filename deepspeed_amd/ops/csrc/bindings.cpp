@@ -151,10 +151,13 @@ extern "C" void ds_cpu_lion_flat(float* p, const void* g, int grad_dtype,
 extern "C" void ds_ce_fwd(const void* logits, const long long* labels,
                           float* loss, float* lse, int N, long long V,
                           long long ignore_index, void* stream);
+extern "C" void ds_ce_total(const float* loss, const long long* labels,
+                            float* sum, float* count, float* mean, int N,
+                            long long ignore_index, void* stream);
 extern "C" void ds_ce_bwd(const void* logits, const long long* labels,
-                          const float* lse, const float* gscale,
-                          void* dlogits, int N, long long V,
-                          long long ignore_index, void* stream);
+                          const float* lse, const float* gscale, int stride,
+                          const float* count, void* dlogits, int N,
+                          long long V, long long ignore_index, void* stream);
 
 namespace {
 
@@ -981,6 +984,56 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
           h.scalar_type() == at::kFloat ? h : h.view(x.sizes())};
 }
 
+// Cross-entropy of bf16 logits [N, V] with labels [N]: (sum of the rows, labels
+// other than ignore_index, mean over these, lse [N]).
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> ce_loss(
+    at::Tensor logits, at::Tensor labels, int64_t ignore_index) {
+  const OneDevice on("ce_loss", logits, labels);
+  TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() &&
+              logits.dim() == 2 && logits.scalar_type() == at::kBFloat16 &&
+              labels.scalar_type() == at::kLong && labels.is_contiguous() &&
+              labels.numel() == logits.size(0) &&
+              logits.size(0) < (1ll << 31), "ce_loss args");
+  const int N = logits.size(0);
+  auto f32 = logits.options().dtype(at::kFloat);
+  auto loss = at::empty({N}, f32), lse = at::empty({N}, f32);
+  // apart: the caller may change one in place
+  auto sum = at::empty({}, f32), count = at::empty({}, f32),
+       mean = at::empty({}, f32);
+  const long long* y = (const long long*)labels.data_ptr<int64_t>();
+  ds_ce_fwd(logits.data_ptr(), y, loss.data_ptr<float>(),
+            lse.data_ptr<float>(), N, logits.size(1), ignore_index,
+            cur_stream());
+  ds_ce_total(loss.data_ptr<float>(), y, sum.data_ptr<float>(),
+              count.data_ptr<float>(), mean.data_ptr<float>(), N,
+              ignore_index, cur_stream());
+  return {sum, count, mean, lse};
+}
+
+// gscale: [N], or one for all rows; of the mean over `count` labels, if given.
+at::Tensor ce_bwd(at::Tensor logits, at::Tensor labels, at::Tensor lse,
+                  at::Tensor gscale, int64_t ignore_index,
+                  c10::optional<at::Tensor> count) {
+  const OneDevice on("ce_bwd", logits, labels, lse, gscale, count);
+  const int64_t N = logits.size(0);
+  TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() &&
+              logits.dim() == 2 && logits.scalar_type() == at::kBFloat16 &&
+              labels.scalar_type() == at::kLong && labels.is_contiguous() &&
+              labels.numel() == N && lse.is_contiguous() &&
+              lse.scalar_type() == at::kFloat && lse.numel() == N &&
+              gscale.is_contiguous() && gscale.scalar_type() == at::kFloat &&
+              (gscale.numel() == N || gscale.numel() == 1) &&
+              (!count || (count->scalar_type() == at::kFloat &&
+                          count->numel() == 1)), "ce_bwd args");
+  auto d = at::empty_like(logits);
+  ds_ce_bwd(logits.data_ptr(), (const long long*)labels.data_ptr<int64_t>(),
+            lse.data_ptr<float>(), gscale.data_ptr<float>(),
+            gscale.numel() == 1 ? 0 : 1,
+            count ? count->data_ptr<float>() : nullptr, d.data_ptr(), (int)N,
+            logits.size(1), ignore_index, cur_stream());
+  return d;
+}
+
 at::Tensor token_gather(at::Tensor x, at::Tensor idx) {
   TORCH_CHECK(x.dim() == 3 && x.is_cuda() && x.is_contiguous(),
               "token_gather: contiguous [B,S,D] GPU tensor");
@@ -1345,18 +1398,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           return std::make_tuple(loss, lse);
         },
         "fused CE forward: bf16 logits -> per-token loss + lse");
-  m.def("ce_bwd",
-        [](at::Tensor logits, at::Tensor labels, at::Tensor lse,
-           at::Tensor gscale, int64_t ignore_index) {
-          const int N = logits.size(0);
-          const long long V = logits.size(1);
-          auto d = at::empty_like(logits);
-          ds_ce_bwd(logits.data_ptr(), (const long long*)labels.data_ptr<int64_t>(),
-                    lse.data_ptr<float>(), gscale.data_ptr<float>(),
-                    d.data_ptr(), N, V, ignore_index, cur_stream());
-          return d;
-        },
-        "fused CE backward: dlogits in bf16");
+  m.def("ce_loss", &ce_loss,
+        "fused CE forward: bf16 logits -> sum, labels, mean, lse");
+  m.def("ce_bwd", &ce_bwd, "fused CE backward: dlogits in bf16",
+        py::arg("logits"), py::arg("labels"), py::arg("lse"),
+        py::arg("gscale"), py::arg("ignore_index"),
+        py::arg("count") = c10::nullopt);
   m.def("flash_attn_fwd", &flash_attn_fwd,
         "flash attention forward (bf16, MFMA): (o, logsumexp)");
   m.def("flash_attn_bwd", &flash_attn_bwd,

@@ -37,3 +37,31 @@ def test_cross_entropy_rows(v, offset):
     p = p * (gs * live).double()[:, None]
     # rounded to bf16 once
     assert ((d.double() - p).abs() <= 2.0 ** -8 * p.abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 9001])
+@pytest.mark.parametrize("ignored", ["none", "some", "all"])
+def test_sum_and_mean(n, ignored):
+    from deepspeed_amd.ops import _C
+    from deepspeed_amd.ops.cross_entropy import (fused_cross_entropy_mean,
+                                                 fused_cross_entropy_sum)
+    g = torch.Generator().manual_seed(n)
+    x = (3 * torch.randn(n, 24, generator=g)).bfloat16().cuda()
+    y = torch.randint(0, 24, (n,), generator=g).cuda()
+    if ignored != "none":
+        y[:: 1 if ignored == "all" else 3] = -100
+    x.requires_grad_()
+    rows, lse = _C.ce_fwd(x.detach(), y, -100)
+    live = int((y != -100).sum())
+    total, count = fused_cross_entropy_sum(x, y)
+    mean = fused_cross_entropy_mean(x, y)
+    assert count.item() == live
+    # fp64 sums, rounded once and once more divided
+    want = rows.double().sum()
+    torch.testing.assert_close(total.double(), want, rtol=2.0 ** -24, atol=0)
+    torch.testing.assert_close(mean.double(), want / max(live, 1),
+                               rtol=2.0 ** -23, atol=0)
+    mean *= 1.0                                   # its own memory
+    (d,) = torch.autograd.grad(mean * 8, x)
+    scale = torch.full((n,), 8.0, device="cuda") / max(live, 1)
+    assert torch.equal(d, _C.ce_bwd(x.detach(), y, lse, scale, -100))
