@@ -38,7 +38,7 @@ extern "C" long long ds_norm_bwd_parts(const void* dy, const void* x,
                                        int rows, int H, int ln, int dtype);
 extern "C" void ds_norm_bwd(const void* dy, const void* x, const void* w,
                             const float* invrms, const float* mean,
-                            const void* dres, void* dx, float* dwb,
+                            const void* dres, void* dx, void* dwb, int narrow,
                             float* part, int rows, int H, int ln, int dtype,
                             void* stream);
 extern "C" void ds_rope(const void* x1, void* y1, int heads1, const void* x2,
@@ -808,11 +808,12 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_fwd(
 }
 
 // dres (RMS only): a further gradient of x, added to dx.
+// (dx, dw, LN: db); dw and db in fp32, or dw in `into`, which has x's type.
 std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_bwd(
     at::Tensor dy, at::Tensor x, at::Tensor w, at::Tensor invrms,
     c10::optional<at::Tensor> mean, bool layernorm,
-    c10::optional<at::Tensor> dres) {
-  const OneDevice on("norm_bwd", x, dy, w, invrms, mean, dres);
+    c10::optional<at::Tensor> dres, c10::optional<at::Tensor> into) {
+  const OneDevice on("norm_bwd", x, dy, w, invrms, mean, dres, into);
   TORCH_CHECK(dy.is_contiguous() && x.is_contiguous() && w.is_contiguous(),
               "must be contiguous");
   const int64_t H = x.size(-1);
@@ -832,15 +833,25 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_bwd(
       code) : 0;
   auto part = at::empty({n}, f32opts);
   const int64_t width = layernorm ? 2 * H : H;
-  auto dwb = n ? at::empty({width}, f32opts) : at::zeros({width}, f32opts);
+  TORCH_CHECK(!into || (!layernorm && into->is_contiguous() &&
+                        into->numel() == H &&
+                        into->scalar_type() == x.scalar_type()),
+              "norm_bwd: into");
+  const bool narrow = into.has_value() && n;
+  auto dwb = narrow ? *into
+      : n ? at::empty({width}, f32opts) : at::zeros({width}, f32opts);
   if (rows)
     ds_norm_bwd(dy.data_ptr(), x.data_ptr(), w.data_ptr(),
                 invrms.data_ptr<float>(),
                 layernorm ? mean->data_ptr<float>() : nullptr, n ? rp : nullptr,
-                dx.data_ptr(), dwb.data_ptr<float>(),
+                dx.data_ptr(), dwb.data_ptr(), narrow,
                 n ? part.data_ptr<float>() : nullptr, (int)rows, (int)H, ln,
                 code, cur_stream());
   if (rp != nullptr && !n) dx.add_(*dres);
+  if (into) {
+    if (!narrow) into->copy_(dwb.view(into->sizes()));
+    return {dx, *into, at::empty({0}, f32opts)};
+  }
   return {dx, dwb.narrow(0, 0, H),
           layernorm ? dwb.narrow(0, H, H) : at::empty({0}, f32opts)};
 }
@@ -1360,7 +1371,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("norm_bwd", &norm_bwd, "RMSNorm/LayerNorm backward",
         pybind11::arg("dy"), pybind11::arg("x"), pybind11::arg("w"),
         pybind11::arg("invrms"), pybind11::arg("mean"),
-        pybind11::arg("layernorm"), pybind11::arg("dres") = c10::nullopt);
+        pybind11::arg("layernorm"), pybind11::arg("dres") = c10::nullopt,
+        pybind11::arg("into") = c10::nullopt);
   m.def("paged_decoder_layer", &paged_decoder_layer,
         "a decoder layer of a serving step over the paged pool");
   m.def("add_norm_fwd", &add_norm_fwd, "RMS norm of a sum, and the sum");

@@ -399,9 +399,12 @@ __global__ __launch_bounds__(BLOCK) void norm_bwd_rows_kernel(
 }
 
 // out[c] = sum over n rows of part[., c]: 64 columns a workgroup, 16 waves
-// each with every sixteenth row.
+// each with every sixteenth row. In the weight's type where that is asked for: a
+// conversion behind it was a launch a norm, ten a step of two layers with the
+// additions to the flat buffer that went with it.
+template <typename O>
 __global__ __launch_bounds__(1024) void norm_parts_kernel(
-    const float* __restrict__ part, float* __restrict__ out, const int n,
+    const float* __restrict__ part, O* __restrict__ out, const int n,
     const int width) {
   __shared__ float sums[16][64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -416,7 +419,7 @@ __global__ __launch_bounds__(1024) void norm_parts_kernel(
   if (wid == 0 && c < width) {
 #pragma unroll
     for (int i = 1; i < 16; ++i) s += sums[i][lane];
-    out[c] = s;
+    out[c] = ds::from_f32<O>(s);
   }
 }
 
@@ -478,8 +481,8 @@ int bwd_blocks(int rows) {
 template <typename T, bool LN, bool RES>
 void launch_norm_bwd_rows(const T* dy, const T* x, const T* w,
                           const float* invrms, const float* mean,
-                          const T* dres, T* dx, float* dwb, float* part,
-                          int rows, int H, hipStream_t s) {
+                          const T* dres, T* dx, void* dwb, bool narrow,
+                          float* part, int rows, int H, hipStream_t s) {
   const int grid = bwd_blocks(rows);
   const int iters = (H + BLOCK * VEC - 1) / (BLOCK * VEC);
 #define ROWS(ITERS)                                                          \
@@ -491,16 +494,21 @@ void launch_norm_bwd_rows(const T* dy, const T* x, const T* w,
   else ROWS(4);
 #undef ROWS
   const int width = (LN ? 2 : 1) * H;
-  hipLaunchKernelGGL(norm_parts_kernel, dim3((width + 63) / 64), dim3(1024),
-                     0, s, part, dwb, grid, width);
+  const dim3 columns((width + 63) / 64);
+  if (narrow)
+    hipLaunchKernelGGL(norm_parts_kernel<T>, columns, dim3(1024), 0, s, part,
+                       (T*)dwb, grid, width);
+  else
+    hipLaunchKernelGGL(norm_parts_kernel<float>, columns, dim3(1024), 0, s,
+                       part, (float*)dwb, grid, width);
 }
 
-// dwb: fp32 dw [H] and, LN, db [H] behind it
+// dwb: dw [H] and, LN, db [H] behind it; fp32, or with `narrow` (and part) T
 template <typename T>
 void launch_norm_bwd(const void* dy, const void* x, const void* w,
                      const float* invrms, const float* mean, const void* dres,
-                     void* dx, float* dwb, float* part, int rows, int H,
-                     bool ln, hipStream_t s) {
+                     void* dx, void* dwb, bool narrow, float* part, int rows,
+                     int H, bool ln, hipStream_t s) {
   const T* dyt = reinterpret_cast<const T*>(dy);
   const T* xt = reinterpret_cast<const T*>(x);
   const T* wt = reinterpret_cast<const T*>(w);
@@ -510,20 +518,20 @@ void launch_norm_bwd(const void* dy, const void* x, const void* w,
     if constexpr (sizeof(T) == 2) {
       if (ln)
         launch_norm_bwd_rows<T, true, false>(dyt, xt, wt, invrms, mean, rt,
-                                             dxt, dwb, part, rows, H, s);
+                                             dxt, dwb, narrow, part, rows, H, s);
       else if (dres != nullptr)
         launch_norm_bwd_rows<T, false, true>(dyt, xt, wt, invrms, mean, rt,
-                                             dxt, dwb, part, rows, H, s);
+                                             dxt, dwb, narrow, part, rows, H, s);
       else
         launch_norm_bwd_rows<T, false, false>(dyt, xt, wt, invrms, mean, rt,
-                                              dxt, dwb, part, rows, H, s);
+                                              dxt, dwb, narrow, part, rows, H, s);
     }
     return;
   }
   int grid = rows < 2048 ? rows : 2048;
   const size_t lds_bytes = (size_t)H * sizeof(float) * (ln ? 2 : 1);
-  float* dw = dwb;
-  float* db = dwb + H;
+  float* dw = (float*)dwb;
+  float* db = dw + H;
   if (ln) {
     hipLaunchKernelGGL((norm_bwd_kernel<T, true>), dim3(grid), dim3(BLOCK),
                        lds_bytes, s, dyt, xt, wt, invrms, mean, dxt, dw, db,
@@ -606,17 +614,17 @@ extern "C" long long ds_norm_bwd_parts(const void* dy, const void* x,
 
 extern "C" void ds_norm_bwd(const void* dy, const void* x, const void* w,
                             const float* invrms, const float* mean,
-                            const void* dres, void* dx, float* dwb,
+                            const void* dres, void* dx, void* dwb, int narrow,
                             float* part, int rows, int H, int ln, int dtype,
                             void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (dtype == 1)
-    launch_norm_bwd<ds::bf16>(dy, x, w, invrms, mean, dres, dx, dwb, part,
-                              rows, H, ln, s);
+    launch_norm_bwd<ds::bf16>(dy, x, w, invrms, mean, dres, dx, dwb, narrow,
+                              part, rows, H, ln, s);
   else if (dtype == 2)
-    launch_norm_bwd<ds::f16>(dy, x, w, invrms, mean, dres, dx, dwb, part, rows,
-                             H, ln, s);
+    launch_norm_bwd<ds::f16>(dy, x, w, invrms, mean, dres, dx, dwb, narrow,
+                             part, rows, H, ln, s);
   else
-    launch_norm_bwd<float>(dy, x, w, invrms, mean, dres, dx, dwb, part, rows,
-                           H, ln, s);
+    launch_norm_bwd<float>(dy, x, w, invrms, mean, dres, dx, dwb, narrow, part,
+                           rows, H, ln, s);
 }

@@ -164,10 +164,24 @@ def _nothing():
     return None
 
 
-def _dw(x, dys, own: bool, slots):
-    """dy^T x of the layers, in their slots where these are open."""
+def uses(*weights):
+    """A product that may write the weights' gradients is being made."""
+    for w in weights:
+        slot = getattr(w, "_ds_grad_slot", None)
+        if slot is not None:
+            slot.uses += 1
+
+
+def place(weight):
+    """Where the weight's gradient may be written now, or None."""
+    slot = getattr(weight, "_ds_grad_slot", None)
+    return None if slot is None else slot.take()
+
+
+def _dw(x, dys, own: bool, weights):
+    """dy^T x of the layers, in their weights' places where these are open."""
     T, K = x.shape
-    into = [slot and slot.take() for slot in slots] if own else [None] * len(dys)
+    into = [place(w) if own else None for w in weights]
     if own and all(own_products(T, dy.shape[1], K)[1] for dy in dys) and \
             _aligned(x, *dys):
         return get_ext().tile_linear_dw(x, dys, into=into)
@@ -198,10 +212,7 @@ class _Linears(torch.autograd.Function):
         ctx.save_for_backward(x if any(need[2::2]) else None,
                               *(w if need[0] else None for w in weights))
         ctx.shape, ctx.features = x.shape, [w.shape for w in weights]
-        for w in weights:
-            slot = getattr(w, "_ds_grad_slot", None)
-            if slot is not None:
-                slot.uses += 1
+        uses(*weights)
         if own:
             out = _forward(x, weights, biases)
         else:
@@ -231,8 +242,8 @@ class _Linears(torch.autograd.Function):
             x2 = x.reshape(-1, K)
             if own:
                 x2 = x2.contiguous()
-            slots = [getattr(weights[i], "_ds_grad_slot", None) for i in some]
-            for i, dw in zip(some, _dw(x2, [dys[i] for i in some], own, slots)):
+            for i, dw in zip(some, _dw(x2, [dys[i] for i in some], own,
+                                       [weights[i] for i in some])):
                 grads[2 * i] = dw
         for i, dy in enumerate(dys):
             if need[3 + 2 * i]:

@@ -8,7 +8,21 @@ matching torch implementation (fp32 math internally, like the kernels).
 import torch
 
 from ._loader import get_ext
-from .linear import movable
+from .linear import movable, place, uses
+
+
+def _backward(dy, x, weight, invrms, dres=None):
+    """(dx, dw) of the RMS norm; dw in the weight's type, at its place if there
+    is one."""
+    w = weight.contiguous()
+    if w.dtype != x.dtype:
+        dx, dw, _ = get_ext().norm_bwd(dy, x, w, invrms, None, False, dres)
+        return dx, dw.to(w.dtype)
+    into = place(weight)
+    dx, dw, _ = get_ext().norm_bwd(
+        dy, x, w, invrms, None, False, dres,
+        torch.empty_like(w) if into is None else into)
+    return dx, dw
 
 
 class _RMSNormFn(torch.autograd.Function):
@@ -32,8 +46,7 @@ class _RMSNormFn(torch.autograd.Function):
         ext = get_ext()
         dy = dy.contiguous()
         if ext is not None and x.is_cuda:
-            dx, dw, _ = ext.norm_bwd(dy, x, weight.contiguous(), invrms, None,
-                                     False)
+            dx, dw = _backward(dy, x, weight, invrms)
         else:
             H = x.shape[-1]
             xf = x.float().reshape(-1, H)
@@ -116,10 +129,8 @@ class _AddNormFn(torch.autograd.Function):
             return dtotal, dtotal, None, None
         if dtotal is not None:
             dtotal = dtotal.contiguous()
-        dx, dw, _ = get_ext().norm_bwd(dy.contiguous(), total,
-                                       weight.contiguous(), invrms, None,
-                                       False, dtotal)
-        return dx, dx, dw.to(weight.dtype), None
+        dx, dw = _backward(dy.contiguous(), total, weight, invrms, dtotal)
+        return dx, dx, dw, None
 
 
 def add_rms_norm(x, residual, weight, eps=1e-6):
@@ -132,12 +143,16 @@ def add_rms_norm(x, residual, weight, eps=1e-6):
         x, residual = x.contiguous(), residual.contiguous()
         weight = weight.contiguous()
         if x.data_ptr() % 16 == 0 and residual.data_ptr() % 16 == 0:
+            if torch.is_grad_enabled():
+                uses(weight)
             return _AddNormFn.apply(x, residual, weight, eps)
     total = residual + x
-    return _RMSNormFn.apply(total, weight, eps), total
+    return rms_norm(total, weight, eps), total
 
 
 def rms_norm(x, weight, eps=1e-6):
+    if torch.is_grad_enabled():
+        uses(weight)
     return _RMSNormFn.apply(x, weight, eps)
 
 
@@ -160,7 +175,7 @@ class RMSNorm(torch.nn.Module):
         """The norm of x; with ``residual`` that of residual + x, and the
         sum."""
         if residual is None:
-            return _RMSNormFn.apply(x, self.weight, self.eps)
+            return rms_norm(x, self.weight, self.eps)
         return add_rms_norm(x, residual, self.weight, self.eps)
 
     def extra_repr(self):

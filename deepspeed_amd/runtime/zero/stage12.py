@@ -214,7 +214,7 @@ class ZeroStage12Optimizer:
                     p.data = b.flat[off:off + p.numel()].view_as(p.data)
                     if gdtype == dtype:
                         p.grad = b.grad_flat[off:off + p.numel()].view_as(p.data)
-                        if p.dim() == 2 and p.grad.data_ptr() % 16 == 0:
+                        if p.grad.data_ptr() % 16 == 0:
                             p._ds_grad_slot = GradSlot(p.grad)
                             self._slots.append((p, p._ds_grad_slot, b))
                     self.param_to_bucket[p] = b

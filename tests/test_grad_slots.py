@@ -136,3 +136,27 @@ def test_same_gradients_gpu(monkeypatch):
         for n in want[0]:
             if "around" not in n:
                 assert torch.equal(got[0][n], want[0][n]), n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,h", [(3, 8), (700, 1024), (40, 8192), (5, 9000),
+                                    (9, 33)])
+@pytest.mark.parametrize("dres", [False, True])
+def test_norm_gradient_in_its_type_gpu(rows, h, dres):
+    """As the fp32 one rounded, by the rows kernel and the general one."""
+    from deepspeed_amd.ops import _C
+    g = torch.Generator().manual_seed(h)
+    x, dy, r = (torch.randn(rows, h, generator=g).bfloat16().cuda()
+                for _ in range(3))
+    w = torch.randn(h, generator=g).bfloat16().cuda()
+    inv = torch.rand(rows, generator=g).cuda()
+    r = r if dres else None
+    dx, dw, _ = _C.norm_bwd(dy, x, w, inv, None, False, r)
+    into = torch.empty_like(w)
+    dx2, dw2, _ = _C.norm_bwd(dy, x, w, inv, None, False, r, into)
+    assert dw2.data_ptr() == into.data_ptr()
+    # the general kernel adds rows up with atomics, in any order
+    exact = h % 8 == 0 and h <= 8192
+    assert torch.equal(dx, dx2)
+    torch.testing.assert_close(dw2, dw.bfloat16(), rtol=0 if exact else 2.0**-7,
+                               atol=0 if exact else 1e-4)
