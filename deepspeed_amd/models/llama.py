@@ -20,6 +20,7 @@ import torch.nn.functional as F
 from ..ops import linear as _linear
 from ..ops._loader import get_ext
 from ..ops.attention import rope_flash_attention
+from ..ops.embedding import Embedding
 from ..ops.linear import (SWIGLU, Linear, call, movable, rows_linear,
                           tile_linear, unhooked)
 from ..ops.norms import RMSNorm
@@ -359,7 +360,7 @@ class LlamaModel(nn.Module):
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
         self.cfg = cfg
-        self.embed_tokens = nn.Embedding(cfg.vocab_size, cfg.hidden_size)
+        self.embed_tokens = Embedding(cfg.vocab_size, cfg.hidden_size)
         self.layers = nn.ModuleList(
             [LlamaDecoderLayer(cfg, i) for i in range(cfg.num_layers)])
         self.norm = RMSNorm(cfg.hidden_size, eps=cfg.rms_eps)

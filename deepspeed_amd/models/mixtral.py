@@ -12,6 +12,7 @@ import torch
 import torch.nn as nn
 
 from ..moe import MoE
+from ..ops.embedding import Embedding
 from ..ops.norms import RMSNorm
 from ..ops.rope import rope_tables
 from .llama import LlamaAttention, LlamaMLP, LlamaConfig, chunked_cross_entropy
@@ -101,7 +102,7 @@ class MixtralModel(nn.Module):
     def __init__(self, cfg: MixtralConfig):
         super().__init__()
         self.cfg = cfg
-        self.embed_tokens = nn.Embedding(cfg.vocab_size, cfg.hidden_size)
+        self.embed_tokens = Embedding(cfg.vocab_size, cfg.hidden_size)
         self.layers = nn.ModuleList(
             [MixtralDecoderLayer(cfg, i) for i in range(cfg.num_layers)])
         self.norm = RMSNorm(cfg.hidden_size, eps=cfg.rms_eps)

@@ -151,6 +151,11 @@ extern "C" void ds_cpu_lion_flat(float* p, const void* g, int grad_dtype,
 extern "C" void ds_ce_fwd(const void* logits, const long long* labels,
                           float* loss, float* lse, int N, long long V,
                           long long ignore_index, void* stream);
+extern "C" int ds_embedding_block();
+extern "C" void ds_embedding_bwd(const long long* ids, const void* grad,
+                                 int* order, int* key, unsigned* has,
+                                 int* spans, void* out, int T, int V, int H,
+                                 long long padding, void* stream);
 extern "C" void ds_ce_total(const float* loss, const long long* labels,
                             float* sum, float* count, float* mean, int N,
                             long long ignore_index, void* stream);
@@ -995,6 +1000,36 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
           h.scalar_type() == at::kFloat ? h : h.view(x.sizes())};
 }
 
+// Gradient [V, H] of an embedding's table for tokens ids [T] with the gradients
+// grad [T, H] bf16; rows of `padding` (-1: none) get nothing. `into` is zero.
+at::Tensor embedding_bwd(at::Tensor ids, at::Tensor grad, int64_t V,
+                         int64_t padding, c10::optional<at::Tensor> into) {
+  const OneDevice on("embedding_bwd", grad, ids, into);
+  const int64_t T = ids.numel(), H = grad.size(-1);
+  TORCH_CHECK(ids.scalar_type() == at::kLong && ids.is_contiguous() &&
+              grad.is_cuda() && grad.is_contiguous() && grad.dim() == 2 &&
+              grad.scalar_type() == at::kBFloat16 && grad.size(0) == T &&
+              T > 0 && T <= 32768 && H > 0 && H % 8 == 0 && H <= (1 << 20) &&
+              V > 0 && V < (1 << 30) &&
+              ((uintptr_t)grad.data_ptr() & 15) == 0, "embedding_bwd");
+  TORCH_CHECK(!into || (into->is_contiguous() && into->dim() == 2 &&
+                        into->scalar_type() == at::kBFloat16 &&
+                        into->size(0) == V && into->size(1) == H &&
+                        ((uintptr_t)into->data_ptr() & 15) == 0),
+              "embedding_bwd: into");
+  auto out = into ? *into : at::zeros({V, H}, grad.options());
+  const int64_t blk = ds_embedding_block(), blocks = (T + blk - 1) / blk;
+  auto i32 = grad.options().dtype(at::kInt);
+  auto places = at::empty({2 * T}, i32), spans = at::empty({V * blocks}, i32);
+  auto has = at::zeros({V * ((blocks + 31) / 32)}, i32);
+  ds_embedding_bwd((const long long*)ids.data_ptr<int64_t>(),
+                   grad.data_ptr(), places.data_ptr<int>(),
+                   places.data_ptr<int>() + T, (unsigned*)has.data_ptr<int>(),
+                   spans.data_ptr<int>(), out.data_ptr(), (int)T, (int)V,
+                   (int)H, padding, cur_stream());
+  return out;
+}
+
 // Cross-entropy of bf16 logits [N, V] with labels [N]: (sum of the rows, labels
 // other than ignore_index, mean over these, lse [N]).
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> ce_loss(
@@ -1410,6 +1445,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           return std::make_tuple(loss, lse);
         },
         "fused CE forward: bf16 logits -> per-token loss + lse");
+  m.def("embedding_bwd", &embedding_bwd, "gradient of an embedding's table",
+        py::arg("ids"), py::arg("grad"), py::arg("rows"), py::arg("padding"),
+        py::arg("into") = c10::nullopt);
   m.def("ce_loss", &ce_loss,
         "fused CE forward: bf16 logits -> sum, labels, mean, lse");
   m.def("ce_bwd", &ce_bwd, "fused CE backward: dlogits in bf16",

@@ -40,6 +40,7 @@ ext = CUDAExtension(
         os.path.join(CSRC, "swiglu.hip"),
         os.path.join(CSRC, "spatial.hip"),
         os.path.join(CSRC, "token_ops.hip"),
+        os.path.join(CSRC, "embedding.hip"),
     ],
     extra_compile_args={
         "cxx": ["-O3", "-std=c++17", "-fopenmp", "-mavx2", "-mfma"],
