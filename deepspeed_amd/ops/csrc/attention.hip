@@ -59,9 +59,10 @@ __device__ __forceinline__ void place(int id, int blocks, int heads, int& blk,
 // the vector unit does one multiply-add, one exp2, half a maximum, one add and
 // half a conversion; the maximum is raised only where it grows by more than
 // 2^8, so that most steps rescale nothing. Bound by the vector unit beside the
-// matrix cores. 32 on 8 heads of 128, causal: 1 x 4096 173 us (793 TFLOP/s), 8
-// x 4096 1340 us (820); with V transposed beforehand, fp32 scaling and
-// conversions bit by bit it took 350 us, torch's attention 389 and 2716.
+// matrix cores. 32 on 8 heads of 128, causal: 1 x 4096 163 us (842 TFLOP/s), 8 x
+// 4096 1260 us (873), 173 and 1340 while every step waited for the next
+// one's loads; with V transposed beforehand, fp32 scaling and conversions bit by
+// bit it took 350 us, torch's attention 389 and 2716.
 
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(512) void fwd_kernel(
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(512) void fwd_kernel(
 
   T::template fetch<KB, 512>(kp, (int)vk.s, S, kt[0], tid);
   T::template fetch<KB, 512>(vp, (int)vv.s, S, vt[0], tid);
-  __syncthreads();
+  arrive();
 
   for (int it = 0; it < steps; ++it) {
     const int k0 = it * KB, cur = it & 1;
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(512) void fwd_kernel(
         }
       __builtin_amdgcn_s_setprio(0);
     }
-    __syncthreads();
+    arrive();
   }
 
   l += __shfl_xor(l, 32, 64);
@@ -294,15 +295,13 @@ __global__ __launch_bounds__(256, 2) void dkdv_kernel(
                                (int)vd.s, S - s0, dt[buf], tid);
     if (wid < 2) {
       const float* p = stat + wid * rows + ((long long)b * H + h) * S + s0;
-      __builtin_amdgcn_global_load_lds(
-          (const unsigned int*)(p + min(lane, S - s0 - 1)),
-          (unsigned int*)(&st[buf][wid][lane]), 4, 0, 0);
+      load_lds<4>(p, 4u * min(lane, S - s0 - 1), lds_at(&st[buf][wid][0]));
     }
   };
 
   int h = hkv * G + g0, s0 = first;
   fetch(h, s0, 0, tid);
-  __syncthreads();
+  arrive();
   for (int it = 0; it < steps; ++it) {
     const int cur = it & 1;
     int s1 = s0 + QB;
@@ -371,7 +370,7 @@ __global__ __launch_bounds__(256, 2) void dkdv_kernel(
       }
       __builtin_amdgcn_s_setprio(0);
     }
-    __syncthreads();
+    arrive();
     s0 = s1;
   }
 
@@ -472,7 +471,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(
   const int steps = (end_b + KB - 1) / KB;
   T::template fetch<KB, 256>(kp, (int)vk.s, S, kt[0], tid);
   T::template fetch<KB, 256>(vp, (int)vv.s, S, vt[0], tid);
-  __syncthreads();
+  arrive();
   for (int it = 0; it < steps; ++it) {
     const int k0 = it * KB, cur = it & 1;
     if (it + 1 < steps) {
@@ -514,7 +513,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(
       }
       __builtin_amdgcn_s_setprio(0);
     }
-    __syncthreads();
+    arrive();
   }
   if (row >= S) return;
   typedef int i32x2 __attribute__((ext_vector_type(2)));

@@ -6,6 +6,8 @@
 
 #include <hip/hip_runtime.h>
 
+#pragma clang diagnostic ignored "-Winline-asm"     // m0 among the clobbers
+
 namespace attn {
 
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -29,6 +31,45 @@ __device__ __forceinline__ s16x4 tr_read(const short* p) {
 __device__ __forceinline__ int pack2(float a, float b) {
   return __builtin_bit_cast(
       int, __builtin_convertvector((f32x2{a, b}), b16x2));
+}
+
+// 16 bytes a lane to LDS, lane after lane from `lds` on; `arrive` waits for
+// them. Not the builtin: behind that the compiler waits for all loads before it
+// reads LDS, the next tile's among them.
+__device__ __forceinline__ int lds_at(const void* p) {
+  return (int)(uintptr_t)(__attribute__((address_space(3))) char*)p;
+}
+__device__ __forceinline__ void load_lds(const void* p, int lds) {
+  asm volatile("s_mov_b32 m0, %1\n\t"
+               "s_nop 0\n\t"
+               "global_load_lds_dwordx4 %0, off"
+               :: "v"(p), "s"(__builtin_amdgcn_readfirstlane(lds))
+               : "memory", "m0");
+}
+// The same from a base for all lanes and an offset in bytes: half the registers.
+template <int BYTES>
+__device__ __forceinline__ void load_lds(const void* base, unsigned off,
+                                         int lds) {
+  static_assert(BYTES == 16 || BYTES == 4, "");
+  const unsigned lo =
+      __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)base);
+  const unsigned hi =
+      __builtin_amdgcn_readfirstlane((unsigned)((uintptr_t)base >> 32));
+  const void* p = (const void*)(((uintptr_t)hi << 32) | lo);
+  lds = __builtin_amdgcn_readfirstlane(lds);
+  if (BYTES == 16)
+    asm volatile("s_mov_b32 m0, %2\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dwordx4 %0, %1"
+                 :: "v"(off), "s"(p), "s"(lds) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dword %0, %1"
+                 :: "v"(off), "s"(p), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void arrive() {   // own loads, then everybody's
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 // Registers 8 s .. 8 s + 7 of a result as the next product's B operand.
@@ -88,9 +129,8 @@ struct Tile {
       const int row = j / SC;
       int c = (j % SC) ^ turn(row);
       if (CH < SC) c = min(c, CH - 1);
-      const int off = min(row, left - 1) * stride + c * 8;
-      __builtin_amdgcn_global_load_lds((const unsigned int*)(src + off),
-                                       (unsigned int*)(t + j * 8), 16, 0, 0);
+      const unsigned off = (unsigned)min(row, left - 1) * stride + c * 8;
+      load_lds<16>(src, 2u * off, lds_at(t) + ((tid & ~63) + i * TPB) * 16);
     }
   }
 };

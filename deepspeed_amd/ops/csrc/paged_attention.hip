@@ -50,8 +50,6 @@
 #include "attention_tile.h"
 #include "ds_kernels.h"
 
-#pragma clang diagnostic ignored "-Winline-asm"     // m0 among the clobbers
-
 namespace {
 
 using namespace attn;
@@ -347,18 +345,6 @@ constexpr int AHEAD = 2;              // operands read before their product
 __device__ __forceinline__ int uni(int x) {
   return __builtin_amdgcn_readfirstlane(x);
 }
-// 16 bytes a lane to LDS, lane after lane from `lds` on. Not the builtin: behind
-// that the compiler waits for all loads before it reads LDS.
-__device__ __forceinline__ void load_lds(const short* p, int lds) {
-  asm volatile("s_mov_b32 m0, %1\n\t"
-               "s_nop 0\n\t"
-               "global_load_lds_dwordx4 %0, off"
-               :: "v"(p), "s"(uni(lds)) : "memory", "m0");
-}
-__device__ __forceinline__ void arrive() {   // own loads, then everybody's
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 struct True { static constexpr bool value = true; };
 struct False { static constexpr bool value = false; };
@@ -427,7 +413,7 @@ __global__ __launch_bounds__(BNW * 64) void block_kernel(const Args a) {
   // aligned block holds the four rows of a wave's load. Rows past the last key
   // repeat it.
   const int lr = 4 * wid + (lane >> 4);
-  const int lds0 = (int)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const int lds0 = lds_at(lds);
   int ids[2][4];      // blocks of the next values, of the next keys but one
   auto find = [&](int (&id)[4], int kb) INLINE {
 #pragma unroll
