@@ -8,8 +8,9 @@ a library GEMM, with several layers of one input in one launch and the gate's
 activation in the epilogue.
 
 Both take the modules themselves and return None wherever calling them is the
-thing to do: with gradients (but for several layers of ``tile_linear``), hooks, autocast, function transforms, tangents or
-traces, other types, sharded or replaced modules."""
+thing to do: with gradients (but for several layers of ``tile_linear``), hooks,
+autocast, function transforms, tangents or traces, other types, sharded or
+replaced modules."""
 
 import torch
 import torch.nn as nn
