@@ -670,7 +670,7 @@ std::vector<at::Tensor> tile_linear_grad(
     TORCH_CHECK(good(dys[i]) && good(other) && dys[i].size(0) == M &&
                 other.size(1) == K &&
                 other.size(0) == (mode == 2 ? dys[i].size(1) : M) &&
-                dys[i].size(1) < (1 << 30) && K % 8 == 0 &&
+                dys[i].size(1) <= (1 << 23) && K % 8 == 0 &&
                 dys[i].size(1) % (mode == 2 ? 64 : 8) == 0,
                 "tile_linear_grad: operands");
     x[i] = dys[i].data_ptr();

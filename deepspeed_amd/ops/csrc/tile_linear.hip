@@ -658,7 +658,9 @@ extern "C" int ds_tile_linear_stages(int tile, int mode) {
 // [M, K] to out [M, n], one each or one; K is a multiple of 64, n of four.
 // GRAD_X: x are the gradients dy [M, n], out[0] [M, K]; n is a multiple of 64, K
 // of eight. GRAD_W: w[0] is the input, x the gradients, out [n, K]; n and K are
-// multiples of eight. All operands at 16 bytes; bias only for the first two.
+// multiples of eight. K is at most 2^22 and the gradients' n 2^23: a lane's offset
+// in a tile, up to 255 rows, is 32 bits. All operands at 16 bytes; bias only for the
+// first two.
 // tile and splits from the plan; part: splits * rows * columns of all outputs,
 // null for one split; merge 0 leaves these for the next kernel to add up, in
 // their order and with the bias (norms.hip, paged_attention.hip). Returns a

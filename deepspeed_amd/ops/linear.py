@@ -31,6 +31,11 @@ PLAIN, SWIGLU = 0, 1
 DGRAD, DGRAD_T = 1220e12, 1530e12
 STREAM, LAUNCH = 5e12, 5e-6
 
+# Largest layers of csrc/tile_linear.hip: a lane's offset in a tile is 32 bits, up
+# to 255 rows of 2 bytes a feature (of the output's gradient) or input and a row's
+# 128 bytes.
+FEATURES, INPUTS = 1 << 23, 1 << 22
+
 
 def backward_plan(T: int, N: int, K: int):
     """Which operands to transpose in the backward of a layer [N, K] over T
@@ -82,7 +87,11 @@ def own_products(T: int, N: int, K: int):
     longer at smaller ones (3072, K 8192, 4000 rows 162 / 159, 5000 307 / 220).
     Weight: 4096, K 4096, 4000 rows 122 / 102; 14336, K 4096, 4000 rows 453 / 383,
     32768 rows 3555 / 3162; 3072, K 3072, 4000 rows 88 / 72; but 128256, K 4096,
-    8192 rows 6289 / 6630 (4000 rows 3454 / 3324)."""
+    8192 rows 6289 / 6630 (4000 rows 3454 / 3324).
+
+    ``FEATURES``, ``INPUTS`` and 2^30 rows are what the kernel's offsets hold."""
+    if N > FEATURES or K > INPUTS or T >= 1 << 30:
+        return False, False
     dx = N % 64 == 0 and K % 8 == 0 and N >= 192 and T > ROWS and \
         (T < 2560 or N * K < 1 << 25)
     dw = N % 8 == 0 and K % 8 == 0 and T > 192 and \
@@ -93,7 +102,7 @@ def own_products(T: int, N: int, K: int):
 def own_forward(T: int, ns, K: int) -> bool:
     """Whether the forward product of layers of ``ns`` features is
     csrc/tile_linear.hip's, as in ``tile_linear``."""
-    return T > ROWS and K % 64 == 0 and 192 <= K <= 1 << 22 and \
+    return T > ROWS and K % 64 == 0 and 192 <= K <= INPUTS and \
         all(n % 4 == 0 for n in ns) and (
             T < 2560 or K >= 16384
             or (len(ns) > 1 and max(ns) * K < 1 << 25))
@@ -451,7 +460,7 @@ def tile_linear(x: torch.Tensor, mods, mode: int = PLAIN):
         return None
     K = x.shape[-1]
     M = x.numel() // K if K else 0
-    if M <= ROWS or K % 64 or not 192 <= K <= 1 << 22 or (
+    if M <= ROWS or K % 64 or not 192 <= K <= INPUTS or (
             M >= 2560 and len(mods) == 1 and K < 16384) or \
             get_ext() is None or torch.is_autocast_enabled() or \
             torch.compiler.is_compiling() or not untransformed():

@@ -253,3 +253,38 @@ def test_own_products():
     assert L.own_products(1000, 1000, 512) == (False, True)
     assert L.own_products(1000, 1024, 516) == (False, False)
     assert L.own_products(32, 1024, 512) == (False, False)
+
+
+def test_largest_layers():
+    """Past what a lane's 32 bits of offset reach the library has the products."""
+    for n, k in ((L.FEATURES, 64), (64, L.INPUTS)):
+        # the last of 256 rows, or of the 64 of a stage across the contraction
+        assert 255 * 2 * max(n, k) + 128 < 2 ** 32
+        assert any(L.own_products(256, n, k))
+    assert L.own_products(256, L.FEATURES + 64, 64) == (False, False)
+    assert L.own_products(256, 64, L.INPUTS + 64) == (False, False)
+    assert L.own_products((1 << 30) - 1, 8, 8) == (False, True)
+    assert L.own_products(1 << 30, 8, 8) == (False, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [L.FEATURES, L.FEATURES + 64, 9_000_000])
+def test_largest_layers_gpu(n):
+    """Every row's gradient of the input from its own row of the output's."""
+    from deepspeed_amd.ops import _C
+    m, k = 256, 64
+    lin = Linear(k, n, bias=False, device="cuda", dtype=torch.bfloat16)
+    x = torch.randn(m, k, device="cuda").bfloat16().requires_grad_()
+    y = lin(x)
+    assert ("_Linears" in type(y.grad_fn).__name__) == (n <= L.FEATURES)
+    at = torch.arange(m, device="cuda") * 33203 % n
+    dy = torch.zeros_like(y)
+    dy[torch.arange(m, device="cuda"), at] = 1.0
+    y.backward(dy)
+    assert torch.equal(x.grad, lin.weight.detach()[at])
+    assert torch.equal(lin.weight.grad[at], x.detach())
+    if n > L.FEATURES:
+        for call in (lambda: _C.tile_linear_dx([dy], [lin.weight.detach()]),
+                     lambda: _C.tile_linear_dw(x.detach(), [dy])):
+            with pytest.raises(RuntimeError, match="operands"):
+                call()
