@@ -964,7 +964,11 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
                       (int)H, (float)eps, cur_stream());
     stream = sum;
   };
+  // here, not where each is used: sums() launches on what it is given
   for (auto& w : norms) on.check(w);
+  for (auto& w : weights) on.check(w);
+  for (auto& s : scales) on.check(s);
+  for (auto& b : biases) on.check(b);
   if (delta.has_value())
     add_norm(*delta, norms[0], eps0);
   else
