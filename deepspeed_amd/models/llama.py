@@ -295,7 +295,7 @@ class LlamaDecoderLayer(nn.Module):
         return x + delta
 
 
-# What ``_native_layer`` stands for: replaced, they are called.
+# What a native layer stands for: replaced, they are called.
 _CHAIN, _OUT = LlamaDecoderLayer.chain, LlamaAttention._out
 
 
@@ -356,6 +356,13 @@ def _operands(layer, rows: int):
             weights, scales, biases, group)
 
 
+def _plain(x) -> bool:
+    """A stream, or an output to be added to it, that native layers take."""
+    return type(x) is torch.Tensor and x.is_cuda and \
+        x.dtype is torch.bfloat16 and x.is_contiguous() and \
+        x.data_ptr() % 16 == 0
+
+
 class LlamaModel(nn.Module):
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
@@ -386,13 +393,21 @@ class LlamaModel(nn.Module):
                 return None
             return _operands(layers[i], x.shape[0] * x.shape[1])
 
-        after = operands(0)
+        after, native = operands(0), True
         for i, layer in enumerate(layers):
-            ops, after = after, operands(i + 1)
+            # behind modules, which may hand on or change anything, all is
+            # looked at anew
+            ops = after if native else operands(i)
+            if not native and ops and not (
+                    (delta is None or _plain(delta) and delta.shape == x.shape)
+                    and self._paged_plan(x, positions, kv_cache) is plan):
+                ops = None
+            native = ops is not None
+            after = operands(i + 1) if native else None
             if recompute:
                 x = checkpoint(lambda x_, l=layer: l(x_, cos, sin, positions,
                                                      kv_cache), x)
-            elif ops:
+            elif native:
                 at = layer.self_attn.layer_idx
                 x, delta = get_ext().paged_decoder_layer(
                     x, delta, *ops, cos, sin, positions, x.shape[1],
@@ -415,10 +430,8 @@ class LlamaModel(nn.Module):
         kernels)."""
         cfg = self.cfg
         if not hasattr(kv_cache, "layers_plan") or torch.is_grad_enabled() or \
-                type(x) is not torch.Tensor or not x.is_cuda or \
-                x.dtype is not torch.bfloat16 or not x.numel() or \
+                not _plain(x) or not x.numel() or \
                 x.shape[-1] != cfg.num_heads * 128 or x.shape[-1] > 16384 or \
-                not x.is_contiguous() or x.data_ptr() % 16 or \
                 get_ext() is None or torch.is_autocast_enabled() or \
                 torch.compiler.is_compiling() or \
                 LlamaDecoderLayer.chain is not _CHAIN or \

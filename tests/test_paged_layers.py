@@ -152,6 +152,64 @@ def test_same_as_modules_gpu(kind, positions, monkeypatch):
         assert torch.equal(a, b)
 
 
+class _Strided(llama.LlamaDecoderLayer):
+    """Hands on a stream that lies across."""
+
+    def forward(self, *a):
+        y = super().forward(*a)
+        return y.transpose(1, 2).contiguous().transpose(1, 2)
+
+
+class _Offset(llama.LlamaMLP):
+    """Its output starts off 16 bytes."""
+
+    def forward(self, x):
+        y = super().forward(x)
+        return torch.cat([y.new_zeros(1), y.flatten()])[1:].view_as(y)
+
+
+class _Masked(llama.LlamaDecoderLayer):
+    """Sets the step's mask for the layers behind it: nothing but itself."""
+
+    def forward(self, x, cos, sin, positions, kv_cache):
+        y = super().forward(x, cos, sin, positions, kv_cache)
+        kv_cache.last_mask = torch.eye(
+            x.shape[1], dtype=torch.bool, device=x.device)[None, None]
+        return y
+
+
+class _Fp32(llama.LlamaDecoderLayer):
+    def forward(self, *a):
+        return super().forward(*a).float()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("own", [_Strided, _Offset, _Masked, _Fp32])
+@torch.no_grad()
+def test_behind_other_classes_gpu(own, monkeypatch):
+    """What a layer or MLP of another class hands on reaches the layers behind it
+    as if there were modules only, or is refused as there."""
+    model, _ = _model("cuda")
+    part = model.model.layers[1]
+    part = part.mlp if issubclass(own, llama.LlamaMLP) else part
+    part.__class__ = own
+    ids = torch.randint(0, 500, (1, 20), device="cuda")
+    out = []
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(llama.LlamaModel, "_paged_plan",
+                                lambda *a: None)
+        cache = PagedKVCache(3, 1, 2, 512, 128, dtype=torch.bfloat16,
+                             device="cuda")
+        cache.begin_step([0], 20)
+        if own is _Fp32:
+            with pytest.raises(RuntimeError, match="same dtype"):
+                model(ids, kv_cache=cache)
+            continue
+        out.append(model(ids, kv_cache=cache))
+    assert own is _Fp32 or torch.equal(*out)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["plain", "bias"])
 def test_sums_in_parts_gpu(kind, monkeypatch):
