@@ -397,8 +397,9 @@ class LlamaModel(nn.Module):
         for i, layer in enumerate(layers):
             # behind modules, which may hand on or change anything, all is
             # looked at anew
-            ops = after if native else operands(i)
-            if not native and ops and not (
+            behind = native
+            ops = after if behind else operands(i)
+            if not behind and ops and not (
                     (delta is None or _plain(delta) and delta.shape == x.shape)
                     and self._paged_plan(x, positions, kv_cache) is plan):
                 ops = None
@@ -413,7 +414,7 @@ class LlamaModel(nn.Module):
                     x, delta, *ops, cos, sin, positions, x.shape[1],
                     kv_cache.k[at], kv_cache.v[at], plan.dst, plan.meta,
                     plan.items, plan.runs, plan.merges, plan.any_merge,
-                    plan.nq, 128 ** -0.5, after is not None)
+                    plan.nq, 128 ** -0.5, behind, after is not None)
                 kv_cache.last_decoded = x.shape[1] == 1
             elif type(layer) is LlamaDecoderLayer and unhooked(layer):
                 x, delta = layer.chain(x, delta, cos, sin, positions,

@@ -895,7 +895,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> add_norm_fwd(
 // weights: q, k, v, o, gate, up, down; int8 with scales. meta.. nq: StepPlan.
 // Products whose contraction is split leave their sums in parts to what reads
 // them next: the append, the norms, and with `parts` the next layer's, whose
-// delta is fp32 [splits, rows, H] then.
+// delta is fp32 [splits, rows, H] then (and which is called with `behind`: another
+// delta has x's type).
 std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
     at::Tensor x, c10::optional<at::Tensor> delta,
     const std::vector<at::Tensor>& norms, double eps0, double eps1,
@@ -906,13 +907,15 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
     c10::optional<at::Tensor> positions, int64_t S, at::Tensor kpool,
     at::Tensor vpool, at::Tensor dst, at::Tensor meta, int64_t n_items,
     int64_t n_runs, int64_t n_merges, bool any_merge, int64_t nq,
-    double scale, bool parts) {
+    double scale, bool behind, bool parts) {
   const OneDevice on("paged_decoder_layer", x, delta, cos_table, sin_table,
                      positions, kpool, vpool, dst, meta);
   TORCH_CHECK(norms.size() == 2 && weights.size() == 7 && biases.size() == 7 &&
               (scales.empty() || scales.size() == 7) && x.is_contiguous() &&
               x.numel() > 0 && x.scalar_type() == at::kBFloat16 &&
               kpool.dim() == 4, "paged_decoder_layer");
+  TORCH_CHECK(!delta || behind || delta->scalar_type() == x.scalar_type(),
+              "paged_decoder_layer: delta");
   const int64_t H = x.size(-1), M = x.numel() / H;
   auto linears = [&](const at::Tensor& in, int first, int count,
                      int64_t mode) {

@@ -74,28 +74,35 @@ def test_plan_is_the_caches_own():
     assert sub.layers_plan(x, 4, 2) is None
 
 
-@pytest.mark.parametrize("where", ["weight", "bias", "scales", "norm"])
-def test_one_device(where):
-    """Refused before anything is launched, whichever product reads it."""
+@pytest.mark.parametrize("where", ["weight", "bias", "scales", "norm",
+                                   "delta"])
+def test_refused(where):
+    """Before anything is launched: tensors on another device, whichever product
+    reads them, and an fp32 delta that is no layer's sums in parts."""
     _C = pytest.importorskip("deepspeed_amd.ops._C")
     bf16 = dict(dtype=torch.bfloat16)
     ws = [torch.zeros(512, 512, **bf16) for _ in range(7)]
     norms, bs, scales = [torch.zeros(512, **bf16)] * 2, [None] * 7, []
+    delta = None
     if where == "weight":
         ws[3] = ws[3].to("meta")
     elif where == "bias":
         bs[2] = torch.zeros(512, device="meta", **bf16)
     elif where == "scales":
         scales = [torch.zeros(128)] * 6 + [torch.zeros(128, device="meta")]
-    else:
+    elif where == "norm":
         norms = [norms[0], norms[1].to("meta")]
+    else:
+        delta = torch.zeros(1, 20, 512)
     pool, plan = torch.zeros(1, 4, 64, 128, **bf16), torch.zeros(
         99, dtype=torch.int32)
-    with pytest.raises(RuntimeError, match="on different devices"):
+    with pytest.raises(RuntimeError, match="delta" if where == "delta" else
+                       "on different devices"):
         _C.paged_decoder_layer(
-            torch.zeros(1, 20, 512, **bf16), None, norms, 1e-6, 1e-6, ws,
+            torch.zeros(1, 20, 512, **bf16), delta, norms, 1e-6, 1e-6, ws,
             scales, bs, 2048, torch.zeros(64, 64), torch.zeros(64, 64), None,
-            20, pool, pool, plan[:20], plan, 1, 1, 1, False, 1, 1.0, False)
+            20, pool, pool, plan[:20], plan, 1, 1, 1, False, 1, 1.0,
+            False, False)
 
 
 @pytest.mark.gpu
