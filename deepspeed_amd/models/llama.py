@@ -313,7 +313,7 @@ def _operands(layer, rows: int):
     H = attn.num_heads * 128
     weights, scales, biases, group = [], [], [], 0
     for norm in norms:
-        if type(norm) is not RMSNorm or not unhooked(norm, internal_ok=True):
+        if type(norm) is not RMSNorm or not unhooked(norm):
             return None
         w = norm.weight
         if w.dtype is not torch.bfloat16 or not w.is_contiguous():

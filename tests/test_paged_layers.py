@@ -46,6 +46,14 @@ def test_operands():
         m.forward = lambda x: x
         assert llama._operands(layer, 1) is None
         del m.forward
+    # the norms' calls do not take place, so neither would their hooks
+    for norm in (layer.input_layernorm, layer.post_attention_layernorm):
+        def fetch(*a):
+            return None
+        fetch._ds_internal = True
+        h = norm.register_forward_pre_hook(fetch)
+        assert llama._operands(layer, 1) is None
+        h.remove()
     own = type("Own", (llama.LlamaMLP,), {})
     layer.mlp.__class__ = own
     assert llama._operands(layer, 1) is None
