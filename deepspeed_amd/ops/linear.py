@@ -222,6 +222,7 @@ class _Linears(torch.autograd.Function):
         ctx.save_for_backward(x if any(need[2::2]) else None,
                               *(w if need[0] else None for w in weights))
         ctx.shape, ctx.features = x.shape, [w.shape for w in weights]
+        ctx.set_materialize_grads(False)
         uses(*weights)
         if own:
             out = _forward(x, weights, biases)
@@ -235,19 +236,23 @@ class _Linears(torch.autograd.Function):
         x, *weights = ctx.saved_tensors
         need = ctx.needs_input_grad
         K = ctx.shape[-1]
-        dys = [dy.reshape(-1, n) for dy, (n, _) in zip(dys, ctx.features)]
+        grads = [None] * (2 * len(dys))
+        used = [i for i, dy in enumerate(dys) if dy is not None]
+        if not used:
+            return None, None, *grads
+        dys = {i: dys[i].reshape(-1, ctx.features[i][0]) for i in used}
         # differentiable products where the gradient itself is differentiated,
         # torch's own where something watches them
         own = (not torch.is_grad_enabled() and untransformed()
                and all(dy.dtype is torch.bfloat16 and not _batched(dy)
-                       for dy in dys))
+                       for dy in dys.values()))
         if own:
-            dys = [dy.contiguous() for dy in dys]
+            dys = {i: dy.contiguous() for i, dy in dys.items()}
         dx = None
-        grads = [None] * (2 * len(dys))
         if need[0]:
-            dx = _dx(dys, weights, own).view(ctx.shape)
-        some = [i for i in range(len(dys)) if need[2 + 2 * i]]
+            dx = _dx(list(dys.values()), [weights[i] for i in used],
+                     own).view(ctx.shape)
+        some = [i for i in used if need[2 + 2 * i]]
         if some:
             x2 = x.reshape(-1, K)
             if own:
@@ -255,7 +260,7 @@ class _Linears(torch.autograd.Function):
             for i, dw in zip(some, _dw(x2, [dys[i] for i in some], own,
                                        [weights[i] for i in some])):
                 grads[2 * i] = dw
-        for i, dy in enumerate(dys):
+        for i, dy in dys.items():
             if need[3 + 2 * i]:
                 grads[2 * i + 1] = dy.sum(0)
         return dx, None, *grads

@@ -255,6 +255,34 @@ def test_own_products():
     assert L.own_products(32, 1024, 512) == (False, False)
 
 
+@pytest.mark.parametrize("used", [(0,), (2,), (0, 2), ()])
+def test_unused_outputs_have_no_gradients(used):
+    g = torch.Generator().manual_seed(0)
+    mods = [nn.Linear(8, n) for n in (4, 6, 2)]
+    x = torch.randn(3, 5, 8, generator=g).requires_grad_()
+    ys = L._Linears.apply(x, False, *(p for m in mods
+                                      for p in (m.weight, m.bias)))
+    if not used:
+        # nothing but a gradient of None arrives
+        class Off(torch.autograd.Function):
+            forward = staticmethod(lambda ctx, *ys: ys[0].detach().sum())
+            backward = staticmethod(lambda ctx, g: (None,) * 3)
+        Off.apply(*ys).backward()
+    else:
+        sum(ys[i].square().sum() for i in used).backward()
+    got = [x.grad] + [p.grad for m in mods for p in (m.weight, m.bias)]
+    x.grad = None
+    for m in mods:
+        m.zero_grad()
+    if used:
+        sum(mods[i](x).square().sum() for i in used).backward()
+    want = [x.grad] + [p.grad for m in mods for p in (m.weight, m.bias)]
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        if a is not None:
+            torch.testing.assert_close(a, b)
+
+
 def test_largest_layers():
     """Past what a lane's 32 bits of offset reach the library has the products."""
     for n, k in ((L.FEATURES, 64), (64, L.INPUTS)):
