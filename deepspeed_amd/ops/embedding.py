@@ -6,7 +6,7 @@ import torch
 import torch.nn as nn
 
 from ._loader import get_ext
-from .linear import _batched, _plain_autograd, untransformed, uses
+from .linear import _batched, _plain_autograd, slot_of, untransformed, uses
 
 # Most tokens: the table of places takes 4 bytes for each row of the embedding's
 # and 256 tokens (78 MB for 152064 rows).
@@ -21,7 +21,7 @@ class _Embed(torch.autograd.Function):
     def forward(ctx, ids, weight, padding):
         ctx.save_for_backward(ids)
         ctx.shape, ctx.padding = weight.shape, padding
-        ctx.slot = getattr(weight, "_ds_grad_slot", None)
+        ctx.slot = slot_of(weight)
         return nn.functional.embedding(ids, weight)
 
     @staticmethod

@@ -12,6 +12,8 @@ thing to do: with gradients (but for several layers of ``tile_linear``), hooks,
 autocast, function transforms, tangents or traces, other types, sharded or
 replaced modules."""
 
+import weakref
+
 import torch
 import torch.nn as nn
 from torch.autograd import forward_ad
@@ -143,25 +145,26 @@ def _dx(dys, weights, own: bool):
 
 class GradSlot:
     """Where the gradient of a parameter belongs: ``view``, a part of its owner's
-    flat buffer, set as the parameter's ``_ds_grad_slot``. While it is ``open``
-    (the owner's backward, no gradient there yet) the product of the parameter's
-    one layer may be written into it. Autograd then keeps that very tensor as the
-    gradient, where it added a new one to the buffer: two reads and a write of
-    every weight's gradient, 20 us for 25M values.
+    flat buffer. While it is ``open`` (the owner's backward, no gradient there
+    yet) the product of the parameter's one layer may be written into it. Autograd
+    then keeps that very tensor as the gradient, where it added a new one to the
+    buffer: two reads and a write of every weight's gradient, 20 us for 25M values.
 
     uses: forward products since the owner's last backward; a weight of several
     keeps to the addition. void: the owner took the gradient away, and what the
-    buffer holds is not part of what arrives."""
+    buffer holds is not part of what arrives.
 
-    __slots__ = ("view", "uses", "open", "void")
+    Beside the parameter, not on it: what is on it is saved with it. It lives as
+    long as its owner keeps it, and keeps the parameter no longer than that lives."""
 
-    def __init__(self, view):
+    __slots__ = ("view", "uses", "open", "void", "weight", "__weakref__")
+
+    def __init__(self, weight, view):
         self.view = view
         self.uses = 0
         self.open = self.void = False
-
-    def __reduce__(self):       # a saved module's parameters have none
-        return _nothing, ()
+        self.weight = weakref.ref(weight)
+        _slots[id(weight)] = self
 
     def take(self):
         if not self.open or self.uses != 1:
@@ -170,21 +173,26 @@ class GradSlot:
         return self.view.detach()
 
 
-def _nothing():
-    return None
+_slots = weakref.WeakValueDictionary()      # by the id of the parameter
+
+
+def slot_of(weight):
+    """The parameter's ``GradSlot``, or None."""
+    slot = _slots.get(id(weight))
+    return slot if slot is not None and slot.weight() is weight else None
 
 
 def uses(*weights):
     """A product that may write the weights' gradients is being made."""
     for w in weights:
-        slot = getattr(w, "_ds_grad_slot", None)
+        slot = slot_of(w)
         if slot is not None:
             slot.uses += 1
 
 
 def place(weight):
     """Where the weight's gradient may be written now, or None."""
-    slot = getattr(weight, "_ds_grad_slot", None)
+    slot = slot_of(weight)
     return None if slot is None else slot.take()
 
 

@@ -536,6 +536,8 @@ class Engine(torch.nn.Module):
                     h.remove()
                 except Exception:
                     pass
+        if isinstance(opt, ZeroStage12Optimizer):
+            opt.drop_slots()
         self.optimizer = None
 
     def set_custom_curriculum_learning_schedule(self, fn):

@@ -37,7 +37,7 @@ from ... import comm as dist
 from ...utils.logging import log_dist
 from ..fp16.loss_scaler import LossScalerBase, LossScaler
 from ...ops.grad_norm import sum_of_squares
-from ...ops.linear import GradSlot
+from ...ops.linear import GradSlot, slot_of
 from ..utils import ALIGNMENT
 from ...utils.nvtx import instrument_w_nvtx
 
@@ -215,8 +215,7 @@ class ZeroStage12Optimizer:
                     if gdtype == dtype:
                         p.grad = b.grad_flat[off:off + p.numel()].view_as(p.data)
                         if p.grad.data_ptr() % 16 == 0:
-                            p._ds_grad_slot = GradSlot(p.grad)
-                            self._slots.append((p, p._ds_grad_slot, b))
+                            self._slots.append((p, GradSlot(p, p.grad), b))
                     self.param_to_bucket[p] = b
                 b.clean = b.grad_flat._version
                 b.master_offset = shard_total
@@ -283,7 +282,7 @@ class ZeroStage12Optimizer:
     @staticmethod
     def _place(param, expected):
         """A gradient has arrived: to its place, if it is not there."""
-        slot = getattr(param, "_ds_grad_slot", None)
+        slot = slot_of(param)
         there = param.grad.data_ptr() == expected.data_ptr()
         if slot is not None and slot.void and (there or slot.open):
             if not there:
@@ -450,6 +449,11 @@ class ZeroStage12Optimizer:
         self._opened.clear()
         for _, slot, _ in self._slots:
             slot.uses = 0
+
+    def drop_slots(self):
+        """Gradients are autograd's own again, and the parameters hold on to the
+        flat buffers by ``grad`` alone."""
+        self._slots.clear()
 
     @instrument_w_nvtx
     def reduce_gradients(self):

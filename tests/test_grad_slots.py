@@ -48,13 +48,11 @@ def _grads(stage, gas, own, device="cpu", rows=4):
         "optimizer": {"type": "AdamW", "params": {"lr": 1e-3}}})
     named = list(engine.module.named_parameters())
     if not own:
-        opt._slots = []
-        for _, p in named:
-            if hasattr(p, "_ds_grad_slot"):
-                del p._ds_grad_slot
+        opt.drop_slots()
     given = []
     for name, p in named:
-        slot = getattr(p, "_ds_grad_slot", None)
+        slot = L.slot_of(p)
+        assert (slot is not None) == own
         if slot is not None:
             class Seen(L.GradSlot):
                 __slots__ = ("name",)
@@ -64,7 +62,7 @@ def _grads(stage, gas, own, device="cpu", rows=4):
                     if out is not None:
                         given.append(self.name)
                     return out
-            p._ds_grad_slot = seen = Seen(slot.view)
+            seen = Seen(p, slot.view)
             seen.name = name
             opt._slots = [(q, seen if q is p else s, b)
                           for q, s, b in opt._slots]
@@ -114,13 +112,47 @@ def test_same_gradients(world, stage, gas):
     run_distributed(_check, world_size=world, args=(stage, gas))
 
 
-def test_saved_modules_hold_no_places(tmp_path):
-    lin = torch.nn.Linear(4, 4)
-    lin.weight._ds_grad_slot = L.GradSlot(torch.zeros(1000, 1000))
-    torch.save(lin, tmp_path / "m.pt")
-    assert (tmp_path / "m.pt").stat().st_size < 10000
-    back = torch.load(tmp_path / "m.pt", weights_only=False)
-    assert getattr(back.weight, "_ds_grad_slot", None) is None
+def _saved(rank, world, path):
+    import deepspeed_amd
+    from torch.multiprocessing.reductions import StorageWeakRef
+    engine, opt, _, _ = deepspeed_amd.initialize(
+        model=torch.nn.Linear(1000, 1000), config={
+            "train_micro_batch_size_per_gpu": 1, "bf16": {"enabled": True},
+            "zero_optimization": {"stage": 2},
+            "optimizer": {"type": "AdamW", "params": {"lr": 1e-3}}})
+    lin = engine.module
+    named = dict(lin.named_parameters())
+    assert all(L.slot_of(p) is not None for p in named.values())
+    torch.save(named, path)
+    back = torch.load(path, weights_only=True)
+    for n, p in named.items():
+        assert torch.equal(back[n], p) and L.slot_of(back[n]) is None
+    torch.save(lin.state_dict(keep_vars=True), path)
+    assert list(torch.load(path, weights_only=True)) == list(named)
+    # without its owner a place is gone, and with it the buffer
+    flat = StorageWeakRef(opt.buckets[0].grad_flat.untyped_storage())
+    engine.destroy()
+    assert all(L.slot_of(p) is None for p in named.values())
+    del engine, opt
+    lin.zero_grad(set_to_none=True)
+    import gc
+    gc.collect()
+    assert flat.expired()
+
+
+def test_saved_parameters_hold_no_places(tmp_path):
+    run_distributed(_saved, world_size=1, args=(str(tmp_path / "m.pt"),))
+
+
+def test_place_of_another_parameter():
+    """A place is its parameter's, not of one that came to lie where that was."""
+    a, b = (torch.nn.Parameter(torch.zeros(4)) for _ in range(2))
+    slot = L.GradSlot(a, torch.zeros(4))
+    assert L.slot_of(a) is slot and L.slot_of(b) is None
+    L._slots[id(b)] = slot
+    assert L.slot_of(b) is None
+    del slot
+    assert L.slot_of(a) is None and id(b) not in L._slots
 
 
 @pytest.mark.gpu
