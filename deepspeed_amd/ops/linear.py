@@ -151,8 +151,8 @@ class GradSlot:
     buffer: two reads and a write of every weight's gradient, 20 us for 25M values.
 
     uses: forward products since the owner's last backward; a weight of several
-    keeps to the addition. void: the owner took the gradient away, and what the
-    buffer holds is not part of what arrives.
+    keeps to the addition. void: a product was given the place, whose parameter
+    has no gradient until what that wrote arrives.
 
     Beside the parameter, not on it: what is on it is saved with it. It lives as
     long as its owner keeps it, and keeps the parameter no longer than that lives."""
@@ -167,9 +167,16 @@ class GradSlot:
         _slots[id(weight)] = self
 
     def take(self):
-        if not self.open or self.uses != 1:
+        """The place for a product that is made now, or None. Only from here on
+        has the parameter no gradient: hooks that read it see the buffer until
+        autograd goes on to it, which it does next (but where the weight is used
+        outside of products as well: then when its last gradient is made)."""
+        w = self.weight()
+        if not self.open or self.uses != 1 or w is None or w.grad is None or \
+                w.grad.data_ptr() != self.view.data_ptr():
             return None
-        self.open = False
+        self.open, self.void = False, True
+        w.grad = None
         return self.view.detach()
 
 

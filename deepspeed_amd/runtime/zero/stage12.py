@@ -284,24 +284,22 @@ class ZeroStage12Optimizer:
         """A gradient has arrived: to its place, if it is not there."""
         slot = slot_of(param)
         there = param.grad.data_ptr() == expected.data_ptr()
-        if slot is not None and slot.void and (there or slot.open):
-            if not there:
-                expected.copy_(param.grad.detach().view(-1))
-            slot.open = slot.void = False
-        elif slot is not None and slot.void:
-            # A product has written to the place, and this is a sum with what it
-            # wrote or another pass's gradient, which that has still to be added
-            # to: it stays where it is until all have arrived.
+        if slot is not None and slot.void:
+            # Elsewhere: a sum with what a product wrote to the place, or another
+            # pass's gradient, which that has still to be added to. It stays where
+            # it is until all have arrived.
+            slot.void = not there
             return
-        elif not there:
-            expected.add_(param.grad.detach().view(-1))
+        if slot is not None:
+            slot.open = False
         if not there:
+            expected.add_(param.grad.detach().view(-1))
             param.grad = expected.view_as(param)
 
     def _place_late(self, bucket=None):
         for p, slot, b in self._opened:
             if (bucket is None or b is bucket) and slot.void and \
-                    not slot.open and p.grad is not None:
+                    p.grad is not None:
                 slot.view.copy_(p.grad.detach())
                 p.grad = slot.view
                 slot.void = False
@@ -423,17 +421,15 @@ class ZeroStage12Optimizer:
 
     def _open_slots(self):
         """Products write the first gradients of their weights into the flat
-        buffers, where nothing has been added to these since they were cleared:
-        the parameter has no gradient then until that one arrives. A parameter
-        whose gradient hooks see keeps to the addition."""
+        buffers, where nothing has been added to these since they were cleared. A
+        parameter whose gradient hooks see keeps to the addition."""
         for p, slot, b in self._slots:
             g = p.grad
             if slot.uses == 1 and b.clean == b.grad_flat._version and \
                     g is not None and g.dtype == slot.view.dtype and \
                     g.data_ptr() == slot.view.data_ptr() and \
                     not p._backward_hooks:
-                p.grad = None
-                slot.open = slot.void = True
+                slot.open = True
                 self._opened.append((p, slot, b))
         for _, _, b in self._opened:
             b.clean = None      # the kernels' writes do not count as versions
@@ -441,11 +437,10 @@ class ZeroStage12Optimizer:
     def _close_slots(self):
         self._place_late()
         for p, slot, _ in self._opened:
-            if slot.void and not slot.open:     # written, but not handed on
+            if slot.void:       # written, but not handed on
                 slot.view.zero_()
-            slot.open = slot.void = False
-            if p.grad is None:
                 p.grad = slot.view
+            slot.open = slot.void = False
         self._opened.clear()
         for _, slot, _ in self._slots:
             slot.uses = 0

@@ -112,6 +112,51 @@ def test_same_gradients(world, stage, gas):
     run_distributed(_check, world_size=world, args=(stage, gas))
 
 
+def _seen(rank, world):
+    """What reads the parameters' gradients in the backward finds the buffers."""
+    import deepspeed_amd
+    engine, opt, _, _ = deepspeed_amd.initialize(model=Net(), config={
+        "train_micro_batch_size_per_gpu": 4, "bf16": {"enabled": True},
+        "zero_optimization": {"stage": 2},
+        "optimizer": {"type": "AdamW", "params": {"lr": 1e-3}}})
+    named = dict(engine.module.named_parameters())
+    # those used outside of their products as well come to theirs at the end
+    places = {n: p.grad.data_ptr() for n, p in named.items()
+              if n not in ("tied.weight", "around.weight")}
+    seen = []
+
+    def read(grad):
+        assert all(named[n].grad.data_ptr() == places[n] for n in places)
+        seen.append({n: named[n].grad.clone() for n in places})
+
+    apply_ = engine.module.apply_
+
+    def watched(mod, x):
+        y = apply_(mod, x)
+        y.register_hook(read)
+        return y
+
+    engine.module.apply_ = watched
+    g = torch.Generator().manual_seed(0)
+    for _ in range(2):
+        x = torch.randn(4, 64, generator=g).bfloat16()
+        loss = engine(x, labels=torch.randn(4, 64, generator=g))
+        del seen[:]
+        engine.backward(loss)
+        assert len(seen) == 7
+        # nothing has arrived at first; the last layer's is there when the one
+        # before it is reached, and stays
+        assert not any(v.any() for v in seen[0].values())
+        for s in seen[1:]:
+            assert torch.equal(s["out.weight"], named["out.weight"].grad)
+        engine.step()
+    engine.destroy()
+
+
+def test_gradients_are_seen_in_the_backward():
+    run_distributed(_seen, world_size=1)
+
+
 def _saved(rank, world, path):
     import deepspeed_amd
     from torch.multiprocessing.reductions import StorageWeakRef
