@@ -8,9 +8,19 @@ import torch.nn as nn
 from ._loader import get_ext
 from .linear import _batched, _plain_autograd, slot_of, untransformed, uses
 
-# Most tokens: the table of places takes 4 bytes for each row of the embedding's
-# and 256 tokens (78 MB for 152064 rows).
-TOKENS = 32768
+# Most tokens, rows and columns of the kernel's tables.
+TOKENS, ROWS, COLUMNS = 32768, (1 << 30) - 1, 1 << 20
+
+
+def fits(tokens: int, rows: int, columns: int) -> bool:
+    """Whether the kernel takes the gradient of a table. Its places, 4 bytes for
+    each row and 256 tokens and a bit more (80 MB for 152064 rows and 32768
+    tokens), may take as much memory as the gradient itself: ten million rows of
+    64 would want 5.3 GB of it beside one of 1.3."""
+    blocks = -(-tokens // 256)
+    return 0 < tokens <= TOKENS and 0 < rows <= ROWS and \
+        0 < columns <= COLUMNS and columns % 8 == 0 and \
+        4 * (blocks + -(-blocks // 32)) <= 2 * columns
 
 
 class _Embed(torch.autograd.Function):
@@ -51,9 +61,9 @@ class Embedding(nn.Embedding):
         if torch.is_grad_enabled() and type(w) is nn.Parameter and \
                 w.requires_grad and w.is_cuda and \
                 w.dtype is torch.bfloat16 and w.dim() == 2 and \
-                w.is_contiguous() and w.shape[1] % 8 == 0 and \
+                w.is_contiguous() and \
                 type(ids) is torch.Tensor and ids.dtype is torch.long and \
-                ids.device == w.device and 0 < ids.numel() <= TOKENS and \
+                ids.device == w.device and fits(ids.numel(), *w.shape) and \
                 self.max_norm is None and not self.sparse and \
                 not self.scale_grad_by_freq and get_ext() is not None and \
                 _plain_autograd() and nn.Embedding.forward is _TORCHS:

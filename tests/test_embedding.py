@@ -4,7 +4,7 @@ shared rows end, against fp64, and the module where its kernel is not taken."""
 import pytest
 import torch
 
-from deepspeed_amd.ops.embedding import Embedding
+from deepspeed_amd.ops.embedding import Embedding, fits
 
 
 def test_on_the_cpu_and_its_second_derivative():
@@ -15,6 +15,21 @@ def test_on_the_cpu_and_its_second_derivative():
     for m in (own, ref):
         m(ids).square().sum().backward()
     assert torch.equal(own.weight.grad, ref.weight.grad)
+
+
+def test_places_take_no_more_than_the_gradient():
+    for tokens, rows, columns, want in (
+            (32768, 152064, 3584, True), (4096, 32000, 1024, True),
+            (32768, 10_000_000, 64, False), (32768, 100, 264, True),
+            (32768, 100, 256, False), (256, 10, 8, True), (1000, 10, 8, False),
+            (32769, 100, 4096, False), (0, 100, 4096, False),
+            (8, 1 << 30, 8, False), (8, 100, (1 << 20) + 8, False),
+            (8, 100, 12, False)):
+        assert fits(tokens, rows, columns) == want, (tokens, rows, columns)
+        if want:
+            blocks = -(-tokens // 256)
+            spans, has = rows * blocks, rows * -(-blocks // 32)
+            assert 4 * (spans + has) <= 2 * rows * columns
 
 
 @pytest.mark.gpu
@@ -69,3 +84,17 @@ def test_module_gpu():
             torch.testing.assert_close(second, grads_dy[1], rtol=2.0 ** -6,
                                        atol=1e-2)
     torch.testing.assert_close(grads[0][0], grads[1][0], rtol=2.0 ** -7, atol=0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("columns", [64, 512])
+def test_narrow_tables_are_torchs_gpu(columns):
+    ids = torch.randint(0, 300, (32768,), device="cuda")
+    own = Embedding(300, columns, device="cuda", dtype=torch.bfloat16)
+    y = own(ids)
+    assert ("_Embed" in type(y.grad_fn).__name__) == (columns == 512)
+    y.backward(torch.ones_like(y))
+    want = torch.bincount(ids, minlength=300)[:, None]
+    torch.testing.assert_close(own.weight.grad.float(),
+                               want.expand(300, columns).float(),
+                               rtol=2.0 ** -8, atol=0)
