@@ -17,6 +17,7 @@ from collections import defaultdict
 import torch
 import torch.nn as nn
 
+from ..ops.embedding import Embedding
 from ..ops.linear import Linear
 from ..utils.logging import logger
 
@@ -62,6 +63,10 @@ def _macs_for(mod, inp, out):
     return 0
 
 
+# the framework's own layers, which are torch's to their user
+_TORCHS = {Linear: nn.Linear, Embedding: nn.Embedding}
+
+
 class FlopsProfiler:
     """Per-module MACs/params/latency accounting via forward hooks."""
 
@@ -95,8 +100,7 @@ class FlopsProfiler:
 
         self._names = {id(m): n for n, m in self.model.named_modules()}
         for m in self.model.modules():
-            # the framework's linear layer is torch's to its user
-            if type(m) in ignore or type(m) is Linear and nn.Linear in ignore:
+            if type(m) in ignore or _TORCHS.get(type(m)) in ignore:
                 continue
             self._hooks.append(m.register_forward_pre_hook(pre_hook))
             self._hooks.append(m.register_forward_hook(post_hook))

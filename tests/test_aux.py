@@ -498,6 +498,22 @@ def test_flops_profiler_ignores_torchs_linear():
         assert any("norm" in n for n in prof._macs)
 
 
+def test_flops_profiler_ignores_torchs_embedding():
+    """Ignoring nn.Embedding leaves out the models' own table of tokens."""
+    from deepspeed_amd.models import llama
+    from deepspeed_amd.ops.embedding import Embedding
+    from deepspeed_amd.profiling.flops_profiler import FlopsProfiler
+    model = llama.LlamaForCausalLM(llama.llama_tiny())
+    ids = torch.randint(0, 512, (1, 8))
+    for ignore in ([], [torch.nn.Embedding], [Embedding]):
+        prof = FlopsProfiler(model)
+        prof.start_profile(ignore_list=ignore)
+        model(ids)
+        prof.stop_profile()
+        assert any("embed" in n for n in prof._calls) == (not ignore)
+        assert any("_proj" in n for n in prof._macs)
+
+
 def test_evoformer_attention_reference_math():
     """DS4Sci_EvoformerAttention vs an index-loop fp32 reference with both
     bias patterns (mask bias [B,N,1,1,S] + pair bias [B,1,H,S,S])."""
