@@ -1135,3 +1135,21 @@ def _ltd_zero3_worker(rank=0, world=1):
         engine.step()
         assert torch.isfinite(loss)
     assert engine.random_ltd_scheduler.current_seq > 8
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("device", [
+    "cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_labels_of_more_tokens_than_there_are(dtype, device):
+    """Labels past the last token count for nothing, in one chunk as in many."""
+    from deepspeed_amd.models.llama import chunked_cross_entropy
+    g = torch.Generator().manual_seed(0)
+    hidden = torch.randn(2, 7, 16, generator=g).to(device, dtype)
+    labels = torch.randint(0, 24, (20,), generator=g).to(device)
+    labels[3] = -100
+    head = torch.nn.Linear(16, 24, bias=False).to(device, dtype)
+    want = torch.nn.functional.cross_entropy(
+        head(hidden).view(14, 24).double(), labels[:14])
+    for chunk in (4, 14, 8192):
+        got = chunked_cross_entropy(hidden, head, labels, chunk)
+        torch.testing.assert_close(got.double(), want, rtol=1e-5, atol=1e-5)
