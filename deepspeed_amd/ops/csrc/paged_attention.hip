@@ -406,8 +406,9 @@ __global__ __launch_bounds__(BNW * 64) void block_kernel(const Args a) {
   const int limit = min(first + tok, key1 - 1);
   const int low = uni(min(first + min(c0, ncols - 1) / G, key1 - 1));
   const bool active = c0 < ncols;
-  // a scale of 0, too, leaves the probability 0 to keys that are not seen
-  const float c = fmaxf(a.c, 1e-30f);
+  // a scale of 0, too, leaves the probability 0 to keys that are not seen, and
+  // one that is no number gives none
+  const float c = a.c < 1e-30f ? 1e-30f : a.c;
 
   // Rows i * 32 + 4 wid + lane / 16 of a step, chunks by the tile's swizzle; an
   // aligned block holds the four rows of a wave's load. Rows past the last key

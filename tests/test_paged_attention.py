@@ -349,6 +349,25 @@ def test_block_scales(scale, blocks):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["rows", "blocks"])
+@pytest.mark.parametrize("kept", [0, 130])
+def test_scale_that_is_no_number(kind, kept, request):
+    """Gives no numbers, whichever kernel the step's runs take and whether their
+    keys are split."""
+    from deepspeed_amd.ops.paged_attention import paged_attention
+    if kind == "blocks":
+        request.getfixturevalue("blocks")
+    slots, pos, _ = _rows([(0, 100)], [kept])
+    plan = StepPlan.build(slots, pos, {0: [3, 1, 0, 2]}, 64, 14, 2, "cuda")
+    assert (plan.nq == 8) == (kind == "blocks")
+    assert plan.any_merge == (kept > 0)
+    kp, vp = (torch.randn(4, 2, 64, 128, device="cuda").bfloat16()
+              for _ in range(2))
+    q = torch.randn(100, 14, 128, device="cuda").bfloat16()
+    assert paged_attention(plan, q, kp, vp, float("nan")).isnan().all()
+
+
+@pytest.mark.gpu
 def test_plans_made_ahead_of_the_gpu():
     """The host goes on while a plan is on its way: later ones do not touch it."""
     plans, want = [], []
