@@ -588,7 +588,7 @@ std::vector<at::Tensor> rows_linear(
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 &&
               x.is_contiguous() && x.dim() == 2, "rows_linear: x");
   const int64_t M = x.size(0), K = x.size(1);
-  TORCH_CHECK(M >= 1 && M <= (scales.empty() ? 256 : 64) && K > 0 &&
+  TORCH_CHECK(M >= 1 && M <= (scales.empty() ? 32 : 64) && K > 0 &&
               K % 256 == 0 && L >= 1 && L <= 3 && (mode == 0 || L == 2) &&
               (scales.empty() || (int)scales.size() == L) &&
               (int)biases.size() == L, "rows_linear: shape");
@@ -610,7 +610,6 @@ std::vector<at::Tensor> rows_linear(
     }
   }
   if (!i8 && M > 16 && y.tiled(x, mode)) return y.out;
-  TORCH_CHECK(i8 || M <= 32, "rows_linear: features in fours past 32 rows");
   const int e = ds_rows_linear(x.data_ptr(), L, y.w, i8 ? sc : nullptr, y.b,
                                y.o, y.n, (int)M, (int)K, (int)group, (int)mode,
                                cur_stream());

@@ -21,9 +21,9 @@ from torch.nn.modules import module as _module
 
 from ._loader import get_ext
 
-# Most rows that ``rows_linear`` takes: bf16, int8 (past it the weights are
-# dequantized first), and bf16 where ``batch_pays``.
-ROWS, ROWS_INT8, BATCH = 32, 64, 256
+# Most rows that ``rows_linear`` takes: bf16 (more are for ``tile_linear``), and
+# int8 (past it the weights are dequantized first).
+ROWS, ROWS_INT8 = 32, 64
 
 PLAIN, SWIGLU = 0, 1
 
@@ -385,17 +385,6 @@ def unhooked(mod: nn.Module, internal_ok: bool = False) -> bool:
         for h in hooks.values())
 
 
-def batch_pays(ns, K: int) -> bool:
-    """Whether ``rows_linear`` takes layers of ``ns`` features on one input of 33
-    to 256 rows: several layers of moderate size, and one with a long
-    contraction. Others are for ``tile_linear``."""
-    if any(n % 4 for n in ns):
-        return False
-    if len(ns) > 1:
-        return sum(ns) <= 16384
-    return K >= 2 * ns[0] and ns[0] * K >= 1 << 24
-
-
 def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
                 hooks_ran: bool = False):
     """Outputs of the linear modules ``mods`` on x [..., K], a list: one each,
@@ -406,7 +395,7 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
         return None
     K = x.shape[-1]
     M = x.numel() // K if K else 0
-    if not 1 <= M <= BATCH or K % 256 or get_ext() is None or \
+    if not 1 <= M <= ROWS_INT8 or K % 256 or get_ext() is None or \
             torch.is_autocast_enabled() or torch.compiler.is_compiling() or \
             not untransformed():
         return None
@@ -421,7 +410,7 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
                     type(w) is not nn.Parameter or w.shape[1:] != (K,):
                 return None
         elif hasattr(kind, "int8_rows"):
-            p = m.int8_rows(K) if M <= ROWS_INT8 else None
+            p = m.int8_rows(K)
             if p is None or p[2] % 256 or group not in (0, p[2]):
                 return None
             w, scale, group = p
@@ -435,8 +424,7 @@ def rows_linear(x: torch.Tensor, mods, mode: int = PLAIN,
             return None
         weights.append(w)
         biases.append(b)
-    if M > ROWS and not scales and (mode != PLAIN or not batch_pays(
-            [w.shape[0] for w in weights], K)):
+    if M > ROWS and not scales:
         return None
     x2 = x.reshape(M, K).contiguous()
     if x2.data_ptr() % 16:

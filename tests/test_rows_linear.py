@@ -7,7 +7,8 @@ import torch.nn as nn
 
 from deepspeed_amd.linear.optimized_linear import (QuantizationConfig,
                                                    WOQLinear)
-from deepspeed_amd.ops.linear import (SWIGLU, batch_pays, rows_linear,
+from deepspeed_amd.ops import linear as L
+from deepspeed_amd.ops.linear import (SWIGLU, rows_linear, tile_linear,
                                       unhooked, untransformed)
 
 
@@ -108,7 +109,7 @@ def test_rows_linear_gpu(int8, m, sizes):
     both = [_layer(n, k, i % 2 == 0, int8, g) for i, n in enumerate(ns)]
     x = torch.randn(1, m, k, generator=g).bfloat16().cuda()
     got = rows_linear(x, [b[0] for b in both])
-    if m > 64 if int8 else m > 32 and not batch_pays(ns, k):
+    if m > (64 if int8 else 32):
         assert got is None
         return
     for (lin, want), y in zip(both, got):
@@ -133,21 +134,23 @@ def test_batch_linear_gpu(m, sizes):
     g = torch.Generator().manual_seed(m)
     both = [_layer(n, k, i % 2 == 0, False, g) for i, n in enumerate(ns)]
     x = torch.randn(m, k, generator=g).bfloat16().cuda()
-    got = rows_linear(x, [b[0] for b in both])
-    if m > 256:
-        assert got is None
-        return
+    assert rows_linear(x, [b[0] for b in both]) is None
+    got = tile_linear(x, [b[0] for b in both])
     for (lin, want), y in zip(both, got):
         _close(y, want(x))
     assert rows_linear(x, [both[0][0]] * 2, SWIGLU) is None
 
 
-def test_batch_rule():
-    assert batch_pays((4096, 1024, 1024), 4096)
-    assert batch_pays((4096,), 14336)
-    assert not batch_pays((4096,), 4096)
-    assert not batch_pays((14336, 14336), 4096)
-    assert not batch_pays((4096, 1022), 4096)
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [32, 33])
+@torch.no_grad()
+def test_longest_contractions_gpu(m):
+    """Past what the tiled kernel takes, 33 rows and more are the module's own."""
+    lin = nn.Linear(L.INPUTS + 256, 4, bias=False, device="cuda",
+                    dtype=torch.bfloat16)
+    x = torch.randn(m, L.INPUTS + 256, device="cuda").bfloat16()
+    assert (rows_linear(x, (lin,)) is not None) == (m <= 32)
+    assert m <= 32 or tile_linear(x, (lin,)) is None
 
 
 @pytest.mark.gpu
