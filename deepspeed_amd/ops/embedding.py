@@ -6,7 +6,7 @@ import torch
 import torch.nn as nn
 
 from ._loader import get_ext
-from .linear import _batched, _plain_autograd, slot_of, untransformed, uses
+from .linear import _batched, _plain_autograd, untransformed, uses
 
 # Most tokens, rows and columns of the kernel's tables.
 TOKENS, ROWS, COLUMNS = 32768, (1 << 30) - 1, 1 << 20
@@ -31,7 +31,7 @@ class _Embed(torch.autograd.Function):
     def forward(ctx, ids, weight, padding):
         ctx.save_for_backward(ids)
         ctx.shape, ctx.padding = weight.shape, padding
-        ctx.slot = slot_of(weight)
+        ctx.slot = uses(weight)
         return nn.functional.embedding(ids, weight)
 
     @staticmethod
@@ -67,7 +67,6 @@ class Embedding(nn.Embedding):
                 self.max_norm is None and not self.sparse and \
                 not self.scale_grad_by_freq and get_ext() is not None and \
                 _plain_autograd() and nn.Embedding.forward is _TORCHS:
-            uses(w)
             return _Embed.apply(ids, w, -1 if self.padding_idx is None
                                 else self.padding_idx)
         return super().forward(ids)

@@ -146,7 +146,7 @@ def _dx(dys, weights, own: bool):
 class GradSlot:
     """Where the gradient of a parameter belongs: ``view``, a part of its owner's
     flat buffer. While it is ``open`` (the owner's backward, no gradient there
-    yet) the product of the parameter's one layer may be written into it. Autograd
+    yet; it is the tensor that the parameter has as its gradient) the product of the parameter's one layer may be written into it. Autograd
     then keeps that very tensor as the gradient, where it added a new one to the
     buffer: two reads and a write of every weight's gradient, 20 us for 25M values.
 
@@ -155,46 +155,49 @@ class GradSlot:
     has no gradient until what that wrote arrives.
 
     Beside the parameter, not on it: what is on it is saved with it. It lives as
-    long as its owner keeps it, and keeps the parameter no longer than that lives."""
+    long as its owner keeps it; since it keeps the parameter, that one's id is not
+    another's."""
 
     __slots__ = ("view", "uses", "open", "void", "weight", "__weakref__")
 
     def __init__(self, weight, view):
         self.view = view
         self.uses = 0
-        self.open = self.void = False
-        self.weight = weakref.ref(weight)
-        _slots[id(weight)] = self
+        self.open, self.void = None, False
+        self.weight = weight
+        key = id(weight)
+        _slots[key] = weakref.ref(
+            self, lambda ref: _slots.get(key) is ref and _slots.pop(key))
 
     def take(self):
         """The place for a product that is made now, or None. Only from here on
         has the parameter no gradient: hooks that read it see the buffer until
         autograd goes on to it, which it does next (but where the weight is used
         outside of products as well: then when its last gradient is made)."""
-        w = self.weight()
-        if not self.open or self.uses != 1 or w is None or w.grad is None or \
-                w.grad.data_ptr() != self.view.data_ptr():
+        w = self.weight
+        if self.open is None or self.uses != 1 or w.grad is not self.open:
             return None
-        self.open, self.void = False, True
+        self.open, self.void = None, True
         w.grad = None
         return self.view.detach()
 
 
-_slots = weakref.WeakValueDictionary()      # by the id of the parameter
+_slots = {}     # weak references by the id of the parameter
 
 
 def slot_of(weight):
     """The parameter's ``GradSlot``, or None."""
-    slot = _slots.get(id(weight))
-    return slot if slot is not None and slot.weight() is weight else None
+    ref = _slots.get(id(weight))
+    return None if ref is None else ref()
 
 
-def uses(*weights):
-    """A product that may write the weights' gradients is being made."""
-    for w in weights:
-        slot = slot_of(w)
-        if slot is not None:
-            slot.uses += 1
+def uses(weight):
+    """A product that may write the weight's gradient is being made; its slot."""
+    ref = _slots.get(id(weight))
+    slot = None if ref is None else ref()
+    if slot is not None:
+        slot.uses += 1
+    return slot
 
 
 def place(weight):
@@ -203,10 +206,10 @@ def place(weight):
     return None if slot is None else slot.take()
 
 
-def _dw(x, dys, own: bool, weights):
+def _dw(x, dys, own: bool, slots):
     """dy^T x of the layers, in their weights' places where these are open."""
     T, K = x.shape
-    into = [place(w) if own else None for w in weights]
+    into = [s.take() if own and s else None for s in slots]
     if own and all(own_products(T, dy.shape[1], K)[1] for dy in dys) and \
             _aligned(x, *dys):
         return get_ext().tile_linear_dw(x, dys, into=into)
@@ -237,8 +240,9 @@ class _Linears(torch.autograd.Function):
         ctx.save_for_backward(x if any(need[2::2]) else None,
                               *(w if need[0] else None for w in weights))
         ctx.shape, ctx.features = x.shape, [w.shape for w in weights]
-        ctx.set_materialize_grads(False)
-        uses(*weights)
+        if len(weights) > 1:
+            ctx.set_materialize_grads(False)
+        ctx.slots = [uses(w) for w in weights]
         if own:
             out = _forward(x, weights, biases)
         else:
@@ -255,27 +259,29 @@ class _Linears(torch.autograd.Function):
         used = [i for i, dy in enumerate(dys) if dy is not None]
         if not used:
             return None, None, *grads
-        dys = {i: dys[i].reshape(-1, ctx.features[i][0]) for i in used}
+        if len(used) < len(dys):
+            dys, weights = [dys[i] for i in used], [weights[i] for i in used]
+        dys = [dy.reshape(-1, ctx.features[i][0]) for i, dy in zip(used, dys)]
         # differentiable products where the gradient itself is differentiated,
         # torch's own where something watches them
         own = (not torch.is_grad_enabled() and untransformed()
                and all(dy.dtype is torch.bfloat16 and not _batched(dy)
-                       for dy in dys.values()))
+                       for dy in dys))
         if own:
-            dys = {i: dy.contiguous() for i, dy in dys.items()}
+            dys = [dy.contiguous() for dy in dys]
         dx = None
         if need[0]:
-            dx = _dx(list(dys.values()), [weights[i] for i in used],
-                     own).view(ctx.shape)
-        some = [i for i in used if need[2 + 2 * i]]
+            dx = _dx(dys, weights, own).view(ctx.shape)
+        some = [(i, dy) for i, dy in zip(used, dys) if need[2 + 2 * i]]
         if some:
             x2 = x.reshape(-1, K)
             if own:
                 x2 = x2.contiguous()
-            for i, dw in zip(some, _dw(x2, [dys[i] for i in some], own,
-                                       [weights[i] for i in some])):
+            for (i, _), dw in zip(some, _dw(x2, [dy for _, dy in some], own,
+                                            [need[0] and ctx.slots[i]
+                                             for i, _ in some])):
                 grads[2 * i] = dw
-        for i, dy in dys.items():
+        for i, dy in zip(used, dys):
             if need[3 + 2 * i]:
                 grads[2 * i + 1] = dy.sum(0)
         return dx, None, *grads

@@ -291,7 +291,7 @@ class ZeroStage12Optimizer:
             slot.void = not there
             return
         if slot is not None:
-            slot.open = False
+            slot.open = None
         if not there:
             expected.add_(param.grad.detach().view(-1))
             param.grad = expected.view_as(param)
@@ -429,7 +429,7 @@ class ZeroStage12Optimizer:
                     g is not None and g.dtype == slot.view.dtype and \
                     g.data_ptr() == slot.view.data_ptr() and \
                     not p._backward_hooks:
-                slot.open = True
+                slot.open = g
                 self._opened.append((p, slot, b))
         for _, _, b in self._opened:
             b.clean = None      # the kernels' writes do not count as versions
@@ -440,7 +440,7 @@ class ZeroStage12Optimizer:
             if slot.void:       # written, but not handed on
                 slot.view.zero_()
                 p.grad = slot.view
-            slot.open = slot.void = False
+            slot.open, slot.void = None, False
         self._opened.clear()
         for _, slot, _ in self._slots:
             slot.uses = 0

@@ -190,14 +190,17 @@ def test_saved_parameters_hold_no_places(tmp_path):
 
 
 def test_place_of_another_parameter():
-    """A place is its parameter's, not of one that came to lie where that was."""
+    """A place is its parameter's, and gone with its owner."""
     a, b = (torch.nn.Parameter(torch.zeros(4)) for _ in range(2))
-    slot = L.GradSlot(a, torch.zeros(4))
+    slot, key = L.GradSlot(a, torch.zeros(4)), id(a)
     assert L.slot_of(a) is slot and L.slot_of(b) is None
-    L._slots[id(b)] = slot
-    assert L.slot_of(b) is None
+    newer = L.GradSlot(a, torch.zeros(4))
     del slot
-    assert L.slot_of(a) is None and id(b) not in L._slots
+    assert L.slot_of(a) is newer
+    del a       # the id stays the parameter's while there is a place
+    assert L.slot_of(newer.weight) is newer and id(newer.weight) == key
+    del newer
+    assert key not in L._slots
 
 
 @pytest.mark.gpu
