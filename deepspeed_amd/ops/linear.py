@@ -76,29 +76,52 @@ def backward_plan(T: int, N: int, K: int):
     return w, big and N < K, big and N >= K
 
 
+def own_dx(T: int, ns, K: int) -> bool:
+    """Whether the input's gradient of layers [n, K] of ``ns`` features over T rows
+    is csrc/tile_linear.hip's, which adds the layers up in one product (us, library
+    with the copies of ``backward_plan`` and additions, and kernel).
+
+    N 14336, K 4096, 1000 rows 128 / 110, 2300 251 / 246; 18944, K 3584, 2048 rows
+    348 / 223; 32064, K 3072, 2559 rows 608 / 409; 3072, K 8192, 1024 rows 53 / 50.
+    From 2560 rows on the library's rounds of tiles are ahead past 7e10 products
+    (4096, K 4096: 4000 rows 104 / 102, 8192 187 / 201, 16384 361 / 419, 32768 715 /
+    871, but 10000 378 / 279; 8192, K 3072: 3000 159 / 147, 4000 190 / 203, 12288 451
+    / 519; 3072, K 3072: 4096 75 / 64, 8192 135 / 134, 16384 213 / 237; 1024, K 1024:
+    16384 39 / 33), where the features are many times the inputs past 1.7e11 (24576,
+    K 1024: 8192 rows 0.60 of the library's time, 10000 1.18; 32768, K 512: 10000
+    0.66, 12288 1.12; 32000, K 1024: 5000 427 / 262, 8192 389 / 431).
+    Several layers: the additions count for less the more features there are (2 of
+    8192, K 3072: 4096 rows 347 / 331, 6000 550 / 637, 16384 1104 / 1262; 2 of 6144,
+    K 4096 0.74 to 1.05 from 5000 rows on; 4096 + 2 of 1024, K 4096: 8192 rows 383 /
+    303, 32768 1413 / 1217; 3 of 3072, K 3072: 32768 rows 1473 / 1398)."""
+    if not ROWS < T < 1 << 30 or K % 8 or K > INPUTS or \
+            any(n % 64 or not 192 <= n <= FEATURES for n in ns):
+        return False
+    if T < 2560:
+        return True
+    if max(ns) * K >= 1 << 25:
+        return False
+    work = T * sum(ns) * K
+    if len(ns) > 1:
+        return work < 22e10 or sum(ns) <= 4 * K
+    return work < (17e10 if ns[0] >= 16 * K else 7e10)
+
+
 def own_products(T: int, N: int, K: int):
     """Which products of the backward of a layer [N, K] over T rows are
     csrc/tile_linear.hip's: (the input's gradient, the weight's). It reads either
     operand across the contraction as fast as along it, without a transposed copy
     (us, library with the copies of ``backward_plan`` and kernel).
 
-    Input: N 4096, K 14336, 2331 rows 351 / 256; 3072, K 8192, 1024 rows 53 / 50;
-    1024, K 1024, 1024 rows 22 / 9; 32000, K 1024, 1024 rows 194 / 75. From 2560
-    rows on the library's whole rounds of tiles are ahead at large weights (14336,
-    K 4096, 8192 rows 647 / 728; 128256, K 4096, 4000 rows 3050 / 3300) and no
-    longer at smaller ones (3072, K 8192, 4000 rows 162 / 159, 5000 307 / 220).
+    Input: ``own_dx``.
     Weight: 4096, K 4096, 4000 rows 122 / 102; 14336, K 4096, 4000 rows 453 / 383,
     32768 rows 3555 / 3162; 3072, K 3072, 4000 rows 88 / 72; but 128256, K 4096,
     8192 rows 6289 / 6630 (4000 rows 3454 / 3324).
 
     ``FEATURES``, ``INPUTS`` and 2^30 rows are what the kernel's offsets hold."""
-    if N > FEATURES or K > INPUTS or T >= 1 << 30:
-        return False, False
-    dx = N % 64 == 0 and K % 8 == 0 and N >= 192 and T > ROWS and \
-        (T < 2560 or N * K < 1 << 25)
-    dw = N % 8 == 0 and K % 8 == 0 and T > 192 and \
-        (T < 6144 or N * K < 1 << 28)
-    return dx, dw
+    dw = N % 8 == 0 and K % 8 == 0 and 192 < T < 1 << 30 and \
+        N <= FEATURES and K <= INPUTS and (T < 6144 or N * K < 1 << 28)
+    return own_dx(T, (N,), K), dw
 
 
 def own_forward(T: int, ns, K: int) -> bool:
@@ -130,8 +153,7 @@ def _dx(dys, weights, own: bool):
     """Sum of dy W over the layers."""
     T, K = dys[0].shape[0], weights[0].shape[1]
     sizes = [w.shape[0] for w in weights]
-    if own and all(own_products(T, n, K)[0] for n in sizes) and \
-            _aligned(*dys, *weights):
+    if own and own_dx(T, sizes, K) and _aligned(*dys, *weights):
         return get_ext().tile_linear_dx(dys, weights)
     dx = None
     for dy, w in zip(dys, weights):
@@ -448,8 +470,8 @@ def _with_gradients(x, mods):
         return None
     T, K = x.numel() // x.shape[-1], x.shape[-1]
     ns = [m.weight.shape[0] for m in mods]
-    if not own_forward(T, ns, K) and \
-            not any(any(own_products(T, n, K)) for n in ns):
+    if not own_forward(T, ns, K) and not own_dx(T, ns, K) and \
+            not any(own_products(T, n, K)[1] for n in ns):
         return None
     return _Linears.apply(x, True, *(p for m in mods
                                      for p in (m.weight, m.bias)))

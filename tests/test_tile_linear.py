@@ -255,6 +255,27 @@ def test_own_products():
     assert L.own_products(32, 1024, 512) == (False, False)
 
 
+def test_own_dx():
+    """The input's gradient of many rows is the library's where that is ahead."""
+    def one(t, n, k):
+        return L.own_dx(t, (n,), k)
+    assert one(2559, 128256, 4096) and not one(2560, 128256, 4096)
+    assert one(4096, 4096, 4096) and not one(8192, 4096, 4096)
+    assert one(2700, 3072, 8192) and not one(32768, 8192, 3072)
+    assert one(5000, 32000, 1024) and not one(8192, 32000, 1024)
+    assert one(32768, 1024, 1024)
+    # several at once save the additions
+    assert L.own_dx(32768, (4096, 1024, 1024), 4096)
+    assert L.own_dx(32768, (3072,) * 3, 3072)
+    assert L.own_dx(4096, (8192,) * 2, 3072)
+    assert not L.own_dx(6000, (8192,) * 2, 3072)
+    assert not L.own_dx(2560, (14336,) * 2, 4096)
+    # what the kernel does not take
+    for t, ns, k in ((32, (256,), 64), (1 << 30, (256,), 64), (64, (128,), 64),
+                     (64, (256, 224), 64), (64, (256,), 68)):
+        assert not L.own_dx(t, ns, k)
+
+
 @pytest.mark.parametrize("used", [(0,), (2,), (0, 2), ()])
 def test_unused_outputs_have_no_gradients(used):
     g = torch.Generator().manual_seed(0)
