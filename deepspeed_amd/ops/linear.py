@@ -124,6 +124,20 @@ def own_products(T: int, N: int, K: int):
     return own_dx(T, (N,), K), dw
 
 
+def one_dw(T: int, ns, K: int) -> bool:
+    """Whether the weights' gradients of several layers over T rows are one launch.
+    Not where that is a bit more than a round of the 256 CUs over operands past the
+    256 MB that the chip caches: the second round is then as long as the first (us,
+    one launch, one each, library: 4096 + 2 of 1024, K 4096, 384 tiles: 12288 rows
+    525 / 530 / 574, 14000 702 / 544 / 718, 32768 1718 / 1217 / 1434; 3 of 3072, K
+    2048, 288 tiles: 10000 348 / 351 / 434, 16384 704 / 544 / 682; 4096 + 2 of 512, K
+    4096, 320 tiles: 16384 605 / 559 / 712; but 4096 + 2 of 1536, 448 tiles: 16384 739
+    / 757 / 894; 5120 + 2 of 1024, K 5120, 560 tiles: 16384 954 / 1096 / 1549)."""
+    tiles = sum(-(-n // 256) for n in ns) * -(-K // 256)
+    return len(ns) == 1 or not (
+        256 < tiles < 400 and 2 * T * (K + sum(ns)) > 1 << 28)
+
+
 def own_forward(T: int, ns, K: int) -> bool:
     """Whether the forward product of layers of ``ns`` features is
     csrc/tile_linear.hip's, as in ``tile_linear``."""
@@ -234,7 +248,10 @@ def _dw(x, dys, own: bool, slots):
     into = [s.take() if own and s else None for s in slots]
     if own and all(own_products(T, dy.shape[1], K)[1] for dy in dys) and \
             _aligned(x, *dys):
-        return get_ext().tile_linear_dw(x, dys, into=into)
+        if one_dw(T, [dy.shape[1] for dy in dys], K):
+            return get_ext().tile_linear_dw(x, dys, into=into)
+        return [get_ext().tile_linear_dw(x, [dy], into=[out])[0]
+                for dy, out in zip(dys, into)]
     dws = []
     for dy, out in zip(dys, into):
         dy_t = x_t = False

@@ -276,6 +276,37 @@ def test_own_dx():
         assert not L.own_dx(t, ns, k)
 
 
+@pytest.mark.parametrize("t,ns,k,want", [
+    (12288, (4096, 1024, 1024), 4096, [3]),
+    (14000, (4096, 1024, 1024), 4096, [1, 1, 1]),
+    (32768, (4096, 1536, 1536), 4096, [3]),
+    (16384, (3072, 3072, 3072), 2048, [1, 1, 1]),
+    (32768, (1024, 256, 256), 1024, [3]),
+    (32768, (4096,), 4096, [1])])
+def test_launches_of_weight_gradients(t, ns, k, want, monkeypatch):
+    """Each gradient arrives at its own weight, in one launch or in several."""
+    calls = []
+
+    class Ext:
+        @staticmethod
+        def tile_linear_dw(x, dys, into):
+            calls.append(len(dys))
+            assert len(into) == len(dys)
+            return [(dy.shape[1], out) for dy, out in zip(dys, into)]
+
+    class Slot:
+        def __init__(self, n):
+            self.take = lambda: n
+
+    monkeypatch.setattr(L, "get_ext", Ext)
+    x = torch.empty(t, k, device="meta", dtype=torch.bfloat16)
+    dys = [torch.empty(t, n, device="meta", dtype=torch.bfloat16) for n in ns]
+    slots = [None if i == 1 else Slot(i) for i in range(len(ns))]
+    assert L._dw(x, dys, True, slots) == [
+        (n, None if i == 1 else i) for i, n in enumerate(ns)]
+    assert calls == want
+
+
 @pytest.mark.parametrize("used", [(0,), (2,), (0, 2), ()])
 def test_unused_outputs_have_no_gradients(used):
     g = torch.Generator().manual_seed(0)
