@@ -791,10 +791,13 @@ void cpu_adam_flat(at::Tensor p, at::Tensor g, at::Tensor m, at::Tensor v,
 std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_fwd(
     at::Tensor x, at::Tensor w, c10::optional<at::Tensor> b, double eps,
     bool layernorm) {
+  const OneDevice on("norm_fwd", x, w, b);
   TORCH_CHECK(x.is_contiguous() && w.is_contiguous(), "must be contiguous");
   const int64_t H = x.size(-1);
   const int64_t rows = x.numel() / H;
   TORCH_CHECK(w.numel() == H, "weight shape mismatch");
+  // the kernel reads the weight in x's type
+  TORCH_CHECK(w.scalar_type() == x.scalar_type(), "norm_fwd: types");
   auto y = at::empty_like(x);
   auto f32opts = x.options().dtype(at::kFloat);
   auto invrms = at::empty({rows}, f32opts);
@@ -802,8 +805,10 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_fwd(
   const void* bptr = nullptr;
   if (b.has_value() && b->defined()) {
     TORCH_CHECK(b->is_contiguous() && b->numel() == H, "bias shape mismatch");
+    TORCH_CHECK(b->scalar_type() == x.scalar_type(), "norm_fwd: types");
     bptr = b->data_ptr();
   }
+  TORCH_CHECK(x.is_cuda(), "norm_fwd: GPU tensors");
   ds_norm_fwd(x.data_ptr(), w.data_ptr(), bptr, y.data_ptr(),
               invrms.data_ptr<float>(),
               layernorm ? mean.data_ptr<float>() : nullptr, (int)rows, (int)H,
@@ -822,6 +827,15 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> norm_bwd(
               "must be contiguous");
   const int64_t H = x.size(-1);
   const int64_t rows = x.numel() / H;
+  TORCH_CHECK(w.numel() == H && dy.numel() == x.numel() &&
+              w.scalar_type() == x.scalar_type() &&
+              dy.scalar_type() == x.scalar_type() &&
+              invrms.scalar_type() == at::kFloat && invrms.numel() == rows &&
+              invrms.is_contiguous() &&
+              (!layernorm || (mean.has_value() && mean->numel() == rows &&
+                              mean->scalar_type() == at::kFloat &&
+                              mean->is_contiguous())),
+              "norm_bwd: types or sizes");
   auto dx = at::empty_like(x);
   auto f32opts = x.options().dtype(at::kFloat);
   const void* rp = nullptr;

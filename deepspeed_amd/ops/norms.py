@@ -11,13 +11,22 @@ from ._loader import get_ext
 from .linear import movable, place, uses
 
 
+def _kernels(x, *others):
+    """The extension if its norms take x with these tensors (or None): on a GPU,
+    and all of one type, since the kernels read them in x's."""
+    ext = get_ext()
+    if ext is None or not x.is_cuda:
+        return None
+    for t in others:
+        if t is not None and t.dtype is not x.dtype:
+            return None
+    return ext
+
+
 def _backward(dy, x, weight, invrms, dres=None):
     """(dx, dw) of the RMS norm; dw in the weight's type, at its place if there
     is one."""
     w = weight.contiguous()
-    if w.dtype != x.dtype:
-        dx, dw, _ = get_ext().norm_bwd(dy, x, w, invrms, None, False, dres)
-        return dx, dw.to(w.dtype)
     into = place(weight)
     dx, dw, _ = get_ext().norm_bwd(
         dy, x, w, invrms, None, False, dres,
@@ -28,9 +37,9 @@ def _backward(dy, x, weight, invrms, dres=None):
 class _RMSNormFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, eps):
-        ext = get_ext()
+        ext = _kernels(x, weight)
         x = x.contiguous()
-        if ext is not None and x.is_cuda:
+        if ext is not None:
             y, invrms, _ = ext.norm_fwd(x, weight.contiguous(), None, eps, False)
         else:
             xf = x.float()
@@ -43,9 +52,9 @@ class _RMSNormFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, weight, invrms = ctx.saved_tensors
-        ext = get_ext()
+        ext = _kernels(x, weight, dy)
         dy = dy.contiguous()
-        if ext is not None and x.is_cuda:
+        if ext is not None:
             dx, dw = _backward(dy, x, weight, invrms)
         else:
             H = x.shape[-1]
@@ -63,9 +72,9 @@ class _RMSNormFn(torch.autograd.Function):
 class _LayerNormFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, eps):
-        ext = get_ext()
+        ext = _kernels(x, weight, bias)
         x = x.contiguous()
-        if ext is not None and x.is_cuda:
+        if ext is not None:
             y, invrms, mean = ext.norm_fwd(
                 x, weight.contiguous(),
                 bias.contiguous() if bias is not None else None, eps, True)
@@ -87,9 +96,9 @@ class _LayerNormFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, weight, invrms, mean = ctx.saved_tensors
-        ext = get_ext()
+        ext = _kernels(x, weight, dy)
         dy = dy.contiguous()
-        if ext is not None and x.is_cuda:
+        if ext is not None:
             dx, dw, db = ext.norm_bwd(dy, x, weight.contiguous(), invrms, mean,
                                       True)
         else:

@@ -150,3 +150,63 @@ def test_norm_weight_gradient_repeats(rows):
         rms_norm(x, w).backward(dy)
         grads.append(w.grad)
     assert torch.equal(grads[0], grads[1]) and torch.equal(grads[0], grads[2])
+
+
+@pytest.mark.parametrize("which", ["fwd", "bias", "bwd", "dy"])
+def test_kernels_refuse_other_types(which):
+    """A weight, bias or gradient in another type than x's would be read past its
+    end, or as other numbers."""
+    _C = pytest.importorskip("deepspeed_amd.ops._C")
+    x, w = torch.zeros(2, 64), torch.zeros(64)
+    bf16 = torch.zeros(64, dtype=torch.bfloat16)
+    inv = torch.zeros(2)
+    with pytest.raises(RuntimeError, match="types"):
+        if which == "fwd":
+            _C.norm_fwd(x, bf16, None, 1e-5, False)
+        elif which == "bias":
+            _C.norm_fwd(x, w, bf16, 1e-5, True)
+        elif which == "bwd":
+            _C.norm_bwd(x, x, bf16, inv, None, False)
+        else:
+            _C.norm_bwd(x.bfloat16(), x, w, inv, None, False)
+
+
+@pytest.mark.parametrize("device", [
+    "cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("kind", ["rms", "add", "layer"])
+@pytest.mark.parametrize("x_type", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("w_type", [torch.float32, torch.bfloat16])
+def test_weights_of_another_type(kind, x_type, w_type, device):
+    """The norm in x's type, the gradients each in its own."""
+    from deepspeed_amd.ops.norms import layer_norm
+    g = torch.Generator().manual_seed(0)
+    x, r, dy = (torch.randn(5, 512, generator=g).to(device, x_type)
+                for _ in range(3))
+    w, b = (torch.randn(512, generator=g).to(device, w_type)
+            for _ in range(2))
+    ps = [x, w, b] if kind == "layer" else [x, w]
+    for p in ps:
+        p.requires_grad_()
+
+    def norm(x, w, b=None, r=r, own=True):
+        if not own:
+            if kind == "layer":
+                return torch.nn.functional.layer_norm(x, (512,), w, b, 1e-5)
+            x = x + r.double() if kind == "add" else x
+            return x * torch.rsqrt(x.square().mean(-1, keepdim=True)
+                                   + 1e-5) * w
+        if kind == "layer":
+            return layer_norm(x, w, b, 1e-5)
+        return add_rms_norm(x, r, w, 1e-5)[0] if kind == "add" else \
+            rms_norm(x, w, 1e-5)
+
+    y = norm(*ps)
+    got = [y, *torch.autograd.grad(y, ps, dy)]
+    assert [t.dtype for t in got] == [x_type] + [p.dtype for p in ps]
+    qs = [p.detach().double().requires_grad_() for p in ps]
+    y = norm(*qs, own=False)
+    for a, c in zip(got, [y, *torch.autograd.grad(y, qs, dy.double())]):
+        # fp32 within, rounded to the result's type; the sum of add to x's, too
+        half = torch.bfloat16 in (a.dtype, x_type)
+        assert (a.double() - c).norm() <= \
+            (2.0 ** -7 if half else 2.0 ** -18) * c.norm()
