@@ -1206,8 +1206,10 @@ std::vector<at::Tensor> rope(at::Tensor x, c10::optional<at::Tensor> x2,
 }
 
 at::Tensor gated_act_fwd(at::Tensor gate, at::Tensor up, int64_t act) {
+  const OneDevice on("gated_act_fwd", gate, up);
   TORCH_CHECK(gate.is_contiguous() && up.is_contiguous() &&
               gate.sizes() == up.sizes(), "shape mismatch");
+  TORCH_CHECK(gate.scalar_type() == up.scalar_type(), "gated_act_fwd: types");
   auto out = at::empty_like(gate);
   ds_gated_act_fwd(gate.data_ptr(), up.data_ptr(), out.data_ptr(),
                    gate.numel(), (int)act, dtype_code(gate), cur_stream());
@@ -1217,8 +1219,13 @@ at::Tensor gated_act_fwd(at::Tensor gate, at::Tensor up, int64_t act) {
 std::tuple<at::Tensor, at::Tensor> gated_act_bwd(at::Tensor dout,
                                                  at::Tensor gate,
                                                  at::Tensor up, int64_t act) {
+  const OneDevice on("gated_act_bwd", gate, dout, up);
   TORCH_CHECK(dout.is_contiguous() && gate.is_contiguous() &&
               up.is_contiguous(), "must be contiguous");
+  TORCH_CHECK(gate.scalar_type() == up.scalar_type() &&
+              gate.scalar_type() == dout.scalar_type() &&
+              gate.numel() == up.numel() && gate.numel() == dout.numel(),
+              "gated_act_bwd: types or sizes");
   auto dgate = at::empty_like(gate);
   auto dup = at::empty_like(up);
   ds_gated_act_bwd(dout.data_ptr(), gate.data_ptr(), up.data_ptr(),

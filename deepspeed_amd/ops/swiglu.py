@@ -11,14 +11,21 @@ from ._loader import get_ext
 _SILU, _GELU = 0, 1
 
 
+def _kernels(gate, *others):
+    """The extension if it takes these: on a GPU and of one type."""
+    ext = get_ext()
+    return ext if ext is not None and gate.is_cuda and all(
+        t.dtype is gate.dtype for t in others) else None
+
+
 class _GatedActFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, gate, up, act):
         ctx.act = act
         gate, up = gate.contiguous(), up.contiguous()
         ctx.save_for_backward(gate, up)
-        ext = get_ext()
-        if ext is not None and gate.is_cuda:
+        ext = _kernels(gate, up)
+        if ext is not None:
             return ext.gated_act_fwd(gate, up, act)
         gf = gate.float()
         a = torch.nn.functional.silu(gf) if act == _SILU else \
@@ -28,9 +35,9 @@ class _GatedActFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         gate, up = ctx.saved_tensors
-        ext = get_ext()
+        ext = _kernels(gate, up, dout)
         dout = dout.contiguous()
-        if ext is not None and gate.is_cuda:
+        if ext is not None:
             dgate, dup = ext.gated_act_bwd(dout, gate, up, ctx.act)
             return dgate, dup, None
         gf, uf, dof = gate.float(), up.float(), dout.float()

@@ -1153,3 +1153,36 @@ def test_labels_of_more_tokens_than_there_are(dtype, device):
     for chunk in (4, 14, 8192):
         got = chunked_cross_entropy(hidden, head, labels, chunk)
         torch.testing.assert_close(got.double(), want, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("which", ["fwd", "up", "dout"])
+def test_gated_kernels_refuse_other_types(which):
+    """They read all operands in the gate's type."""
+    _C = pytest.importorskip("deepspeed_amd.ops._C")
+    x, y = torch.zeros(64), torch.zeros(64, dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError, match="types"):
+        if which == "fwd":
+            _C.gated_act_fwd(x, y, 0)
+        else:
+            _C.gated_act_bwd(*((x, x, y) if which == "up" else (y, x, x)), 0)
+
+
+@pytest.mark.parametrize("device", [
+    "cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("types", [(torch.float32, torch.bfloat16),
+                                   (torch.bfloat16, torch.float32)])
+def test_gates_of_another_type(types, device):
+    from deepspeed_amd.ops.swiglu import swiglu
+    g = torch.Generator().manual_seed(0)
+    gate, up = (torch.randn(3, 512, generator=g).to(device, t)
+                .requires_grad_() for t in types)
+    y = swiglu(gate, up)
+    dy = torch.randn(3, 512, generator=g).to(y)
+    got = [y, *torch.autograd.grad(y, (gate, up), dy)]
+    assert [t.dtype for t in got] == [types[0], *types]
+    a, b = (t.detach().double().requires_grad_() for t in (gate, up))
+    y = torch.nn.functional.silu(a) * b
+    for x, want in zip(got, [y, *torch.autograd.grad(y, (a, b),
+                                                     dy.double())]):
+        eps = 2.0 ** (-8 if x.dtype == torch.bfloat16 else -18)
+        assert (x.double() - want).norm() <= eps * want.norm()
