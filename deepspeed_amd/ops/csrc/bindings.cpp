@@ -930,6 +930,20 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
   TORCH_CHECK(!delta || behind || delta->scalar_type() == x.scalar_type(),
               "paged_decoder_layer: delta");
   const int64_t H = x.size(-1), M = x.numel() / H;
+  // as own_forward in ops/linear.py has it
+  auto own_forward = [&](const at::Tensor& in, int first, int count,
+                         int64_t mode) {
+    if (M < 2560 || mode == 1) return true;
+    const int64_t K = in.size(1);
+    int64_t most = 0, all = 0;
+    for (int i = first; i < first + count; ++i) {
+      const int64_t n = weights[i].numel() / K;
+      most = std::max(most, n);
+      all += n;
+    }
+    if (count == 1) return K >= 16384 && all % 4096 != 0;
+    return most * K < (1 << 25) && (M < 16384 || 1.0 * M * all * K < 4e11);
+  };
   auto linears = [&](const at::Tensor& in, int first, int count,
                      int64_t mode) {
     const std::vector<at::Tensor> w(weights.begin() + first,
@@ -942,16 +956,17 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
         s.assign(scales.begin() + first, scales.begin() + first + count);
       return rows_linear(in, w, s, b, group, mode);
     }
-    // as tile_linear in ops/linear.py has it
-    if (count == 1 && M >= 2560 && in.size(1) < 16384)
-      return std::vector<at::Tensor>{at::linear(in, w[0], b[0])};
+    if (!own_forward(in, first, count, mode)) {
+      std::vector<at::Tensor> y;
+      for (int i = 0; i < count; ++i) y.push_back(at::linear(in, w[i], b[i]));
+      return y;
+    }
     return tile_linear(in, w, b, mode, -1, 1);
   };
   // outputs, or their sums in parts
   using Sums = std::pair<std::vector<at::Tensor>, at::Tensor>;
   auto sums = [&](const at::Tensor& in, int first, int count) -> Sums {
-    if (!scales.empty() || M <= 16 ||
-        (count == 1 && M >= 2560 && in.size(1) < 16384))
+    if (!scales.empty() || M <= 16 || !own_forward(in, first, count, 0))
       return {linears(in, first, count, 0), at::Tensor()};
     Layers y;
     at::Tensor part;

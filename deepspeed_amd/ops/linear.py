@@ -138,13 +138,32 @@ def one_dw(T: int, ns, K: int) -> bool:
         256 < tiles < 400 and 2 * T * (K + sum(ns)) > 1 << 28)
 
 
-def own_forward(T: int, ns, K: int) -> bool:
+def own_forward(T: int, ns, K: int, mode: int = PLAIN) -> bool:
     """Whether the forward product of layers of ``ns`` features is
-    csrc/tile_linear.hip's, as in ``tile_linear``."""
-    return T > ROWS and K % 64 == 0 and 192 <= K <= INPUTS and \
-        all(n % 4 == 0 for n in ns) and (
-            T < 2560 or K >= 16384
-            or (len(ns) > 1 and max(ns) * K < 1 << 25))
+    csrc/tile_linear.hip's. Over 20 layers of 1024 x 1024 to 128256 x 4096 and 33 to
+    8192 rows the kernel takes 0.65 of the library's time in the geometric mean (us,
+    library and kernel: gate and up 14336, K 4096, 224 rows 95 + activation / 67;
+    4096, K 14336, 1024 rows 138 / 108; 3584, K 18944, 2331 rows 489 / 302).
+
+    From 2560 rows on the library's whole rounds of tiles reach 5% more for one layer
+    (4096 rows: N 4096, K 4096 91 / 98; N 4096, K 14336 304 / 324; N 128256 2930 /
+    3060; elsewhere 3300 rows: N 4096, K 14336 343 / 305), but for contractions from
+    16384 on where the features are no whole rounds (geometric mean over 2560 to 16384
+    rows and K 16384 to 28672, library 1: N 3584 0.71, 4608 0.73, 5120 0.85, 7168
+    0.83; 2048 0.89; 4096 1.05, 8192 1.01). Several layers stay here (3 of 3072, K 3072,
+    8192 rows 360 / 329; 2 of 5632, K 2048, 0.78 to 1.07), but not large ones
+    (8192 + 2 of 1024, K 8192: 4096 rows 473 / 527, 12288 1330 / 1466) and not from
+    16384 rows on (4096 + 2 of 1024, K 4096: 12288 rows 424 / 458, 16384 528 / 560,
+    32768 1071 / 1156; 2 of 8192, K 3072, 16384 rows 1081 / 1168); gate and up with
+    their activation are even (14336, K 4096: 8192 rows 1349 / 1385, 16384 2706 /
+    2708)."""
+    if T <= ROWS or K % 64 or not 192 <= K <= INPUTS or any(n % 4 for n in ns):
+        return False
+    if T < 2560 or mode == SWIGLU:
+        return True
+    if len(ns) == 1:
+        return K >= 16384 and ns[0] % 4096 != 0
+    return max(ns) * K < 1 << 25 and (T < 16384 or T * sum(ns) * K < 4e11)
 
 
 def _aligned(*ts) -> bool:
@@ -496,16 +515,7 @@ def _with_gradients(x, mods):
 
 def tile_linear(x: torch.Tensor, mods, mode: int = PLAIN):
     """``rows_linear`` for more than ``ROWS`` rows and torch's or the models' own
-    bf16 layers. Over 20 layers of 1024 x 1024 to 128256 x 4096 and 33 to 8192
-    rows the kernel takes 0.65 of the library's time in the geometric mean (us,
-    library and kernel: gate and up 14336, K 4096, 224 rows 95 + activation / 67;
-    4096, K 14336, 1024 rows 138 / 108; 3584, K 18944, 2331 rows 489 / 302).
-
-    One plain layer of many rows stays the library's: its products of whole
-    rounds of tiles reach 5% more (4096 rows: N 4096, K 4096 91 / 98; N 4096, K
-    14336 304 / 324; N 128256 2930 / 3060; elsewhere 3300 rows: N 4096, K 14336
-    343 / 305), but for contractions from 16384 on (3584, K 18944: 4096 rows 540
-    / 418, 5000 958 / 658)."""
+    bf16 layers, where ``own_forward`` says so."""
     if torch.is_grad_enabled():
         return _with_gradients(x, mods) if mode == PLAIN else None
     if type(x) is not torch.Tensor or \
@@ -513,9 +523,7 @@ def tile_linear(x: torch.Tensor, mods, mode: int = PLAIN):
         return None
     K = x.shape[-1]
     M = x.numel() // K if K else 0
-    if M <= ROWS or K % 64 or not 192 <= K <= INPUTS or (
-            M >= 2560 and len(mods) == 1 and K < 16384) or \
-            get_ext() is None or torch.is_autocast_enabled() or \
+    if M <= ROWS or get_ext() is None or torch.is_autocast_enabled() or \
             torch.compiler.is_compiling() or not untransformed():
         return None
     weights, biases = [], []
@@ -524,7 +532,7 @@ def tile_linear(x: torch.Tensor, mods, mode: int = PLAIN):
             return None
         w, b = m.weight, m.bias
         if w.dtype is not torch.bfloat16 or type(w) is not nn.Parameter or \
-                w.shape[1:] != (K,) or w.shape[0] % 4 or not w.is_cuda or \
+                w.shape[1:] != (K,) or not w.is_cuda or \
                 not w.is_contiguous() or w.data_ptr() % 16 or (
                     mode == SWIGLU and w.shape != mods[0].weight.shape) or (
                     b is not None and (b.dtype is not torch.bfloat16
@@ -532,6 +540,8 @@ def tile_linear(x: torch.Tensor, mods, mode: int = PLAIN):
             return None
         weights.append(w)
         biases.append(b)
+    if not own_forward(M, [w.shape[0] for w in weights], K, mode):
+        return None
     x2 = x.reshape(M, K).contiguous()
     if x2.data_ptr() % 16:
         return None

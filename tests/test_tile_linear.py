@@ -276,6 +276,24 @@ def test_own_dx():
         assert not L.own_dx(t, ns, k)
 
 
+def test_own_forward():
+    own = L.own_forward
+    assert own(2559, (128256,), 4096) and not own(2560, (128256,), 4096)
+    # long contractions, but for whole rounds of tiles
+    assert own(8192, (3584,), 18944) and own(2560, (5120,), 16384)
+    assert not own(8192, (4096,), 16384) and not own(2560, (8192,), 28672)
+    assert own(2559, (4096,), 16384)
+    # several layers
+    assert own(12288, (4096, 1024, 1024), 4096)
+    assert not own(16384, (4096, 1024, 1024), 4096)
+    assert own(32768, (1024, 256, 256), 1024)
+    assert not own(4096, (8192, 1024, 1024), 8192)
+    assert own(32768, (14336, 14336), 4096, SWIGLU)
+    for t, ns, k in ((32, (64,), 256), (64, (62,), 256), (64, (64,), 224),
+                     (64, (64,), 128), (64, (64,), L.INPUTS + 64)):
+        assert not own(t, ns, k) and not own(t, ns * 2, k, SWIGLU)
+
+
 @pytest.mark.parametrize("t,ns,k,want", [
     (12288, (4096, 1024, 1024), 4096, [3]),
     (14000, (4096, 1024, 1024), 4096, [1, 1, 1]),
