@@ -493,7 +493,9 @@ def chunked_cross_entropy(hidden, lm_head, labels, chunk_tokens=8192):
     labels = labels.reshape(-1)
     n = hidden.shape[0]
     if 0 < n <= chunk_tokens:
-        return fused_cross_entropy_mean(call(lm_head, hidden), labels[:n])
+        if labels.shape[0] > n:
+            labels = labels[:n]
+        return fused_cross_entropy_mean(call(lm_head, hidden), labels)
     total = hidden.new_zeros((), dtype=torch.float32)
     count = hidden.new_zeros((), dtype=torch.float32)
     for s in range(0, n, chunk_tokens):

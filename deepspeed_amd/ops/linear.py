@@ -94,9 +94,11 @@ def own_dx(T: int, ns, K: int) -> bool:
     8192, K 3072: 4096 rows 347 / 331, 6000 550 / 637, 16384 1104 / 1262; 2 of 6144,
     K 4096 0.74 to 1.05 from 5000 rows on; 4096 + 2 of 1024, K 4096: 8192 rows 383 /
     303, 32768 1413 / 1217; 3 of 3072, K 3072: 32768 rows 1473 / 1398)."""
-    if not ROWS < T < 1 << 30 or K % 8 or K > INPUTS or \
-            any(n % 64 or not 192 <= n <= FEATURES for n in ns):
+    if T <= ROWS or T >= 1 << 30 or K % 8 or K > INPUTS:
         return False
+    for n in ns:
+        if n % 64 or n < 192 or n > FEATURES:
+            return False
     if T < 2560:
         return True
     if max(ns) * K >= 1 << 25:
@@ -107,21 +109,22 @@ def own_dx(T: int, ns, K: int) -> bool:
     return work < (17e10 if ns[0] >= 16 * K else 7e10)
 
 
+def own_dw(T: int, N: int, K: int) -> bool:
+    """Whether the gradient of a weight [N, K] over T rows is
+    csrc/tile_linear.hip's (us, library with the copies of ``backward_plan`` and
+    kernel): 4096, K 4096, 4000 rows 122 / 102; 14336, K 4096, 4000 rows 453 / 383,
+    8192 767 / 796, 10000 1148 / 970, 32768 3529 / 3265; 3072, K 3072, 4000 rows 88 /
+    72; but 128256, K 4096, 8192 rows 6289 / 6630 (4000 rows 3454 / 3324)."""
+    return T > 192 and N % 8 == 0 and K % 8 == 0 and T < 1 << 30 and \
+        N <= FEATURES and K <= INPUTS and (T < 6144 or N * K < 1 << 28)
+
+
 def own_products(T: int, N: int, K: int):
     """Which products of the backward of a layer [N, K] over T rows are
     csrc/tile_linear.hip's: (the input's gradient, the weight's). It reads either
-    operand across the contraction as fast as along it, without a transposed copy
-    (us, library with the copies of ``backward_plan`` and kernel).
-
-    Input: ``own_dx``.
-    Weight: 4096, K 4096, 4000 rows 122 / 102; 14336, K 4096, 4000 rows 453 / 383,
-    32768 rows 3555 / 3162; 3072, K 3072, 4000 rows 88 / 72; but 128256, K 4096,
-    8192 rows 6289 / 6630 (4000 rows 3454 / 3324).
-
-    ``FEATURES``, ``INPUTS`` and 2^30 rows are what the kernel's offsets hold."""
-    dw = N % 8 == 0 and K % 8 == 0 and 192 < T < 1 << 30 and \
-        N <= FEATURES and K <= INPUTS and (T < 6144 or N * K < 1 << 28)
-    return own_dx(T, (N,), K), dw
+    operand across the contraction as fast as along it, without a transposed copy.
+    """
+    return own_dx(T, (N,), K), own_dw(T, N, K)
 
 
 def one_dw(T: int, ns, K: int) -> bool:
@@ -133,9 +136,9 @@ def one_dw(T: int, ns, K: int) -> bool:
     2048, 288 tiles: 10000 348 / 351 / 434, 16384 704 / 544 / 682; 4096 + 2 of 512, K
     4096, 320 tiles: 16384 605 / 559 / 712; but 4096 + 2 of 1536, 448 tiles: 16384 739
     / 757 / 894; 5120 + 2 of 1024, K 5120, 560 tiles: 16384 954 / 1096 / 1549)."""
-    tiles = sum(-(-n // 256) for n in ns) * -(-K // 256)
-    return len(ns) == 1 or not (
-        256 < tiles < 400 and 2 * T * (K + sum(ns)) > 1 << 28)
+    if 2 * T * (K + sum(ns)) <= 1 << 28:
+        return True
+    return not 256 < sum(-(-n // 256) for n in ns) * -(-K // 256) < 400
 
 
 def own_forward(T: int, ns, K: int, mode: int = PLAIN) -> bool:
@@ -213,10 +216,10 @@ class GradSlot:
     long as its owner keeps it; since it keeps the parameter, that one's id is not
     another's."""
 
-    __slots__ = ("view", "uses", "open", "void", "weight", "__weakref__")
+    __slots__ = ("view", "at", "uses", "open", "void", "weight", "__weakref__")
 
     def __init__(self, weight, view):
-        self.view = view
+        self.view, self.at = view, view.data_ptr()
         self.uses = 0
         self.open, self.void = None, False
         self.weight = weight
@@ -265,9 +268,9 @@ def _dw(x, dys, own: bool, slots):
     """dy^T x of the layers, in their weights' places where these are open."""
     T, K = x.shape
     into = [s.take() if own and s else None for s in slots]
-    if own and all(own_products(T, dy.shape[1], K)[1] for dy in dys) and \
-            _aligned(x, *dys):
-        if one_dw(T, [dy.shape[1] for dy in dys], K):
+    ns = [dy.shape[1] for dy in dys]
+    if own and all(own_dw(T, n, K) for n in ns) and _aligned(x, *dys):
+        if len(ns) == 1 or one_dw(T, ns, K):
             return get_ext().tile_linear_dw(x, dys, into=into)
         return [get_ext().tile_linear_dw(x, [dy], into=[out])[0]
                 for dy, out in zip(dys, into)]
@@ -314,10 +317,11 @@ class _Linears(torch.autograd.Function):
         need = ctx.needs_input_grad
         K = ctx.shape[-1]
         grads = [None] * (2 * len(dys))
-        used = [i for i, dy in enumerate(dys) if dy is not None]
-        if not used:
-            return None, None, *grads
-        if len(used) < len(dys):
+        used = range(len(dys))
+        if len(dys) > 1 and any(dy is None for dy in dys):
+            used = [i for i in used if dys[i] is not None]
+            if not used:
+                return None, None, *grads
             dys, weights = [dys[i] for i in used], [weights[i] for i in used]
         dys = [dy.reshape(-1, ctx.features[i][0]) for i, dy in zip(used, dys)]
         # differentiable products where the gradient itself is differentiated,
@@ -330,14 +334,16 @@ class _Linears(torch.autograd.Function):
         dx = None
         if need[0]:
             dx = _dx(dys, weights, own).view(ctx.shape)
-        some = [(i, dy) for i, dy in zip(used, dys) if need[2 + 2 * i]]
+        some = [i for i in used if need[2 + 2 * i]]
         if some:
             x2 = x.reshape(-1, K)
             if own:
                 x2 = x2.contiguous()
-            for (i, _), dw in zip(some, _dw(x2, [dy for _, dy in some], own,
-                                            [need[0] and ctx.slots[i]
-                                             for i, _ in some])):
+            theirs = dys if len(some) == len(dys) else \
+                [dy for i, dy in zip(used, dys) if i in some]
+            for i, dw in zip(some, _dw(x2, theirs, own,
+                                       [need[0] and ctx.slots[i]
+                                        for i in some])):
                 grads[2 * i] = dw
         for i, dy in zip(used, dys):
             if need[3 + 2 * i]:
@@ -507,7 +513,7 @@ def _with_gradients(x, mods):
     T, K = x.numel() // x.shape[-1], x.shape[-1]
     ns = [m.weight.shape[0] for m in mods]
     if not own_forward(T, ns, K) and not own_dx(T, ns, K) and \
-            not any(own_products(T, n, K)[1] for n in ns):
+            not any(own_dw(T, n, K) for n in ns):
         return None
     return _Linears.apply(x, True, *(p for m in mods
                                      for p in (m.weight, m.bias)))

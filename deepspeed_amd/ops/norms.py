@@ -11,15 +11,13 @@ from ._loader import get_ext
 from .linear import movable, place, uses
 
 
-def _kernels(x, *others):
-    """The extension if its norms take x with these tensors (or None): on a GPU,
-    and all of one type, since the kernels read them in x's."""
+def _kernels(x, a, b=None):
+    """The extension if its norms take x with these tensors: on a GPU, and all of
+    one type, since the kernels read them in x's."""
     ext = get_ext()
-    if ext is None or not x.is_cuda:
+    if ext is None or not x.is_cuda or a.dtype is not x.dtype or (
+            b is not None and b.dtype is not x.dtype):
         return None
-    for t in others:
-        if t is not None and t.dtype is not x.dtype:
-            return None
     return ext
 
 

@@ -11,11 +11,13 @@ from ._loader import get_ext
 _SILU, _GELU = 0, 1
 
 
-def _kernels(gate, *others):
+def _kernels(gate, a, b=None):
     """The extension if it takes these: on a GPU and of one type."""
     ext = get_ext()
-    return ext if ext is not None and gate.is_cuda and all(
-        t.dtype is gate.dtype for t in others) else None
+    if ext is None or not gate.is_cuda or a.dtype is not gate.dtype or (
+            b is not None and b.dtype is not gate.dtype):
+        return None
+    return ext
 
 
 class _GatedActFn(torch.autograd.Function):

@@ -260,16 +260,18 @@ class ZeroStage12Optimizer:
         def hook(param):
             # autograd accumulates directly into the preset flat view; if torch
             # ever replaced .grad (it should not), fold it back in.
-            expected = bucket.grad_flat[offset:offset + param.numel()]
-            if expected.dtype != param.dtype:
-                # fp32 accumulation mode: fold the fresh 16-bit grad into the
-                # fp32 flat and free it
-                if param.grad is not None:
-                    expected.add_(param.grad.detach().view(-1)
-                                  .to(expected.dtype))
+            grad, slot = param.grad, slot_of(param)
+            if grad is not None and not (slot is not None
+                                         and self._placed(slot, grad)):
+                expected = bucket.grad_flat[offset:offset + param.numel()]
+                if expected.dtype != param.dtype:
+                    # fp32 accumulation mode: fold the fresh 16-bit grad into
+                    # the fp32 flat and free it
+                    expected.add_(grad.detach().view(-1).to(expected.dtype))
                     param.grad = None
-            elif param.grad is not None:
-                self._place(param, expected)
+                elif grad.data_ptr() != expected.data_ptr():
+                    expected.add_(grad.detach().view(-1))
+                    param.grad = expected.view_as(param)
             if not self.is_gradient_accumulation_boundary:
                 return
             bucket.pending -= 1
@@ -280,21 +282,17 @@ class ZeroStage12Optimizer:
         return hook
 
     @staticmethod
-    def _place(param, expected):
-        """A gradient has arrived: to its place, if it is not there."""
-        slot = slot_of(param)
-        there = param.grad.data_ptr() == expected.data_ptr()
-        if slot is not None and slot.void:
+    def _placed(slot, grad):
+        """A gradient has arrived: is it in its place, or has it to wait?"""
+        there = grad.data_ptr() == slot.at
+        if slot.void:
             # Elsewhere: a sum with what a product wrote to the place, or another
             # pass's gradient, which that has still to be added to. It stays where
             # it is until all have arrived.
             slot.void = not there
-            return
-        if slot is not None:
-            slot.open = None
-        if not there:
-            expected.add_(param.grad.detach().view(-1))
-            param.grad = expected.view_as(param)
+            return True
+        slot.open = None
+        return there
 
     def _place_late(self, bucket=None):
         for p, slot, b in self._opened:
@@ -427,8 +425,7 @@ class ZeroStage12Optimizer:
             g = p.grad
             if slot.uses == 1 and b.clean == b.grad_flat._version and \
                     g is not None and g.dtype == slot.view.dtype and \
-                    g.data_ptr() == slot.view.data_ptr() and \
-                    not p._backward_hooks:
+                    g.data_ptr() == slot.at and not p._backward_hooks:
                 slot.open = g
                 self._opened.append((p, slot, b))
         for _, _, b in self._opened:
