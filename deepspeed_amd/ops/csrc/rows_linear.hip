@@ -227,7 +227,13 @@ __global__ __launch_bounds__(NW * 64) void rows_linear_kernel(const Args a) {
   }
 }
 
-template <bool I8, int MODE, int FT, int D, int OCC>
+// EVEN: every wave's chunks are a multiple of D, so that no load runs ahead of the
+// last one. Otherwise each is asked for by itself, and costs a branch (K 4096, q, k
+// and v of 4096 + 2 x 1024, 8 rows 13.6 / 15.1). us at 8 rows, loads past the end
+// repeating the last chunk and now: N 32000, K 1024 41.6 / 14.4; 3 of 3072, K 3072
+// 22.2 / 16.6; gate and up 2816, K 1024 7.3 / 5.1; 8192, K 3072 24.3 / 20.1; 3584, K
+// 18944 35.1 / 32.2.
+template <bool I8, int MODE, int FT, int D, int OCC, bool EVEN>
 __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
   constexpr int L = MODE == SWIGLU ? 2 : 1;   // weight streams a workgroup
   constexpr int S = L * FT;                   // tiles of 16 features a wave
@@ -236,7 +242,9 @@ __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
   float* const sums = lds;
   float* const scales = lds + NW * S * 256;
 
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wid = EVEN ? threadIdx.x >> 6
+                       : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, g = lane >> 4;
   int layer = 0, tile = blockIdx.x;
   if (MODE == PLAIN) {
@@ -255,7 +263,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
   Weights<I8> w[D][S];
   s16x8 x[D][CH / 32];
   auto load = [&](int d, int i) __attribute__((always_inline)) {
-    const int at = (wid + min(i, mine - 1) * NW) * CH;
+    const int at = (wid + (EVEN ? min(i, mine - 1) : i) * NW) * CH;
 #pragma unroll
     for (int s = 0; s < S; ++s)
       w[d][s].load(a.w[layer + s / FT], row[s % FT] + at, g);
@@ -266,9 +274,10 @@ __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
   f32x4 acc[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (mine > 0)
+  if (!EVEN || mine > 0)
 #pragma unroll
-    for (int d = 0; d < D; ++d) load(d, d);
+    for (int d = 0; d < D; ++d)
+      if (EVEN || d < mine) load(d, d);
   if (I8) {
     for (int e = threadIdx.x; e < chunks * S * 16; e += NW * 64) {
       const int c = e / (S * 16), f = e % (S * 16);
@@ -301,7 +310,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
 #pragma unroll
       for (int d = 0; d < D; ++d) {
         use(d, i + d);
-        load(d, i + d + D);
+        if (EVEN || i + d + D < mine) load(d, i + d + D);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -334,6 +343,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
   }
 }
 
+// D of chunks ahead, and the waves a SIMD that its registers leave.
 template <bool I8, int MODE, int FT, int D, int OCC>
 int launch_few(Args a, int layers, hipStream_t st) {
   int tiles = 0;
@@ -341,7 +351,9 @@ int launch_few(Args a, int layers, hipStream_t st) {
     a.tile_end[i] = tiles += (a.n[i] + 16 * FT - 1) / (16 * FT);
   constexpr int S = (MODE == SWIGLU ? 2 : 1) * FT;
   const int lds = NW * S * 1024 + (I8 ? a.K / CH * S * 64 : 0);
-  auto kernel = few_rows_kernel<I8, MODE, FT, D, OCC>;
+  auto kernel = a.K / CH % (NW * D) == 0
+      ? few_rows_kernel<I8, MODE, FT, D, OCC, true>
+      : few_rows_kernel<I8, MODE, FT, D, OCC, false>;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(
         (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -367,7 +379,13 @@ int launch(Args a, int layers, hipStream_t st) {
 // 10.4; N 6144 15.7 / 13.3 and 12.3 / 10.8; N 128256 8 rows 205 / 192 and 148 /
 // 121, 16 rows 250 / 209 and 178 / 139, but bf16 1 row 168 / 178; gate and up,
 // whose two streams share x, 45.8 / 50.7 and 32.8 / 34.1. With two tiles bf16
-// has four chunks ahead (N 6144 13.3, two 14.5), int8 two (10.8, four 11.5).
+// has four chunks ahead where these are a wave's whole parts (N 6144 13.3, two
+// 14.5; N 32000, K 1024 two 14.4, four 17.7), int8 two (10.8, four 11.5).
+// Two tiles take two rounds of the CUs' time: not where the rounds grow by it (8
+// rows, FT 1 / 2, bf16: N 9216, K 4096 20.7 / 25.0; 12288 22.8 / 26.2; 10240, K 8192
+// 46 / 51; int8 of long layers and few rows: 10240, K 8192 28.0 / 31.3, but 12288, K
+// 4096 17.8 / 17.0), nor, there, where it leaves a CU one workgroup (8192, K 8192, 1
+// row 16.5 / 20.9).
 // More rows, int8 (FT 1 / 2 / 4): M 32: N 4096 11 / 14 / 20, N 6144 23 / 16.3 /
 // 23, N 14336 40 / 29.7 / 24.0; M 64: N 4096 21.1 / 23.8 / 44, N 14336 74 / 46 /
 // 51; gate and up M 32 53.8 / 42.6, M 64 88 / 67.
@@ -379,9 +397,14 @@ int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
   // int8's scales in LDS: beside the sums 64 bytes a chunk and stream
   if (a.M <= 16 && (!I8 || a.K <= 1 << 16)) {
     if (mode == SWIGLU) return launch_few<I8, SWIGLU, 1, 2, 4>(a, layers, st);
-    if (big && (I8 || a.M > 4 || tiles < 2048))
-      return launch_few<I8, PLAIN, 2, I8 ? 2 : 4, I8 ? 4 : 2>(a, layers, st);
-    return launch_few<I8, PLAIN, 1, 2, 4>(a, layers, st);
+    const bool rounds = 2 * ((tiles + 511) / 512) <= (tiles + 255) / 256;
+    const bool full = tiles > 448 && tiles <= 512;
+    if (!big || (I8 ? a.M <= 8 && a.K > 4096 && (!rounds || full)
+                    : !rounds || (a.M <= 4 && tiles >= 2048)))
+      return launch_few<I8, PLAIN, 1, 2, 4>(a, layers, st);
+    if (!I8 && a.K / CH % (4 * NW) == 0)
+      return launch_few<I8, PLAIN, 2, 4, 2>(a, layers, st);
+    return launch_few<I8, PLAIN, 2, 2, 4>(a, layers, st);
   }
   if (mode == SWIGLU) {
     if (a.M <= 32) return launch<I8, 2, SWIGLU, 2>(a, layers, st);

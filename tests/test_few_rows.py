@@ -27,3 +27,18 @@ def test_few_rows_gpu(int8, k, m):
             want = [torch.nn.functional.silu(want[0]) * want[1]]
         for y, w in zip(got, want):
             _close(y, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("n,k", [(6144, 4096), (8192, 4352), (9216, 1024),
+                                 (9216, 4096), (32000, 256), (33000, 512)])
+@pytest.mark.parametrize("m", [1, 8, 9])
+@torch.no_grad()
+def test_tiles_a_wave_gpu(int8, n, k, m):
+    """One and two tiles on either side of their lines, with chunks that are a
+    wave's whole parts and others."""
+    g = torch.Generator().manual_seed(m)
+    lin, want = _layer(n, k, False, int8, g)
+    x = torch.randn(m, k, generator=g).bfloat16().cuda()
+    _close(rows_linear(x, (lin,))[0], want(x))
