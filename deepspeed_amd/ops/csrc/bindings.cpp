@@ -504,6 +504,18 @@ at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
                      cos_table.has_value() ? at::empty_like(q) : q);
 }
 
+// Whether rows_linear.hip is ahead of tile_linear.hip for bf16 layers of `all`
+// features: up to 16 rows, past which the latter shares x in LDS where the former
+// reads it out of L2 for every 16 to 64 features, and up to 32 for small layers (us,
+// either at 17 and 32 rows: N 4096, K 4096 11.9 / 11.6 and 15 / 12; q, k and v of
+// that 17 / 15 and 20 / 17; N 128256 215 / 185 and 228 / 185; but N 1024, K 1024 4.8 /
+// 7.0 and 5.5 / 7.0; 6144, K 1024 6.6 / 7.2 and 7.1 / 7.5; 4096, K 1792 7.2 / 9.6 and
+// 8.3 / 9.6; and 8192, K 512 5.3 / 5.2 and 5.6 / 5.3; 512, K 2048 6.8 / 7.6 and 8.1 /
+// 7.7; gate and up 2816, K 1024 8.3 / 7.1 and 9.0 / 7.0).
+bool few_rows(int64_t M, int64_t all, int64_t K, int64_t mode) {
+  return M <= 16 || (M <= 32 && mode == 0 && K < 2048 && all <= 6144);
+}
+
 // bf16 weights on one input, pointers and features of each; outputs made anew:
 // one each, or with mode 1 silu(layer 0) * layer 1.
 struct Layers {
@@ -566,15 +578,10 @@ struct Layers {
   }
 };
 
-// Linear layers on one input of a few rows: rows_linear.hip, or tile_linear.hip
-// for bf16 weights and more than 16 of them. weights: bf16 [N, K], or int8 (any
+// Linear layers on one input of a few rows, by rows_linear.hip or tile_linear.hip
+// (few_rows). weights: bf16 [N, K], or int8 (any
 // shape, N * K long) with their groupwise scales. mode 1 returns
 // silu(layer 0) * layer 1.
-//
-// 16: above it tile_linear.hip shares x in LDS where rows_linear.hip reads it
-// out of L2 for every 16 to 64 features (us, rows_linear at 32 rows and
-// tile_linear at 33: N 4096, K 4096 15.7 / 11.7; q, k and v of that 20.3 / 16.5;
-// N 4096, K 14336 33 / 26; gate and up 14336 60 / 52; N 128256 226 / 179).
 std::vector<at::Tensor> rows_linear(
     at::Tensor x, std::vector<at::Tensor> weights,
     std::vector<at::Tensor> scales,
@@ -609,7 +616,7 @@ std::vector<at::Tensor> rows_linear(
       sc[i] = scales[i].data_ptr<float>();
     }
   }
-  if (!i8 && M > 16 && y.tiled(x, mode)) return y.out;
+  if (!i8 && !few_rows(M, y.all, K, mode) && y.tiled(x, mode)) return y.out;
   const int e = ds_rows_linear(x.data_ptr(), L, y.w, i8 ? sc : nullptr, y.b,
                                y.o, y.n, (int)M, (int)K, (int)group, (int)mode,
                                cur_stream());
@@ -966,7 +973,11 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
   // outputs, or their sums in parts
   using Sums = std::pair<std::vector<at::Tensor>, at::Tensor>;
   auto sums = [&](const at::Tensor& in, int first, int count) -> Sums {
-    if (!scales.empty() || M <= 16 || !own_forward(in, first, count, 0))
+    int64_t all = 0;
+    for (int i = first; i < first + count; ++i)
+      all += weights[i].numel() / in.size(1);
+    if (!scales.empty() || few_rows(M, all, in.size(1), 0) ||
+        !own_forward(in, first, count, 0))
       return {linears(in, first, count, 0), at::Tensor()};
     Layers y;
     at::Tensor part;

@@ -42,3 +42,17 @@ def test_tiles_a_wave_gpu(int8, n, k, m):
     lin, want = _layer(n, k, False, int8, g)
     x = torch.randn(m, k, generator=g).bfloat16().cuda()
     _close(rows_linear(x, (lin,))[0], want(x))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ns,k", [((1024,), 1024), ((4096, 1024, 1024), 1792),
+                                  ((4096, 1024, 1028), 1792), ((512,), 2048),
+                                  ((130, 64), 256)])
+@pytest.mark.parametrize("m", [16, 17, 32])
+@torch.no_grad()
+def test_small_layers_of_up_to_32_rows_gpu(ns, k, m):
+    g = torch.Generator().manual_seed(m)
+    both = [_layer(n, k, i == 0, False, g) for i, n in enumerate(ns)]
+    x = torch.randn(m, k, generator=g).bfloat16().cuda()
+    for y, (_, want) in zip(rows_linear(x, [b[0] for b in both]), both):
+        _close(y, want(x))
