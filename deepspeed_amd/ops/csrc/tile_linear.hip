@@ -590,15 +590,17 @@ const Tile tiles_[] = {
 
 // us that a tile and a number of splits take: rounds of the 256 CUs (the last
 // one, in part empty, runs faster: less power, less traffic) or W and x from
-// memory at 4.15 TB/s, whichever is longer, then adding the splits up.
+// memory at 4.15 TB/s, a sixth less by few workgroups (8192 x 8192, 64 rows: 128 of
+// them 43.7 us, 256 36.1; 10240 x 8192, 128 rows: 160 59, 240 45; but 11008 x 4096,
+// 17 rows: 172 22.7, 344 25.5), whichever is longer, then adding the splits up.
 float estimate(const Tile& t, double tiles, int steps, double rows,
-               double columns, double bytes, int splits) {
+               double columns, double bytes, int splits, int mode) {
   tiles *= splits;
   const double whole = (double)(long long)(tiles / 256);
   const double rest = tiles / 256 - whole;
   double us = (whole + (rest > 0 ? 0.76 + 0.24 * rest : 0)) *
       (steps / (double)splits * t.stage + t.fixed);
-  double mem = bytes / 4.15e6;
+  double mem = bytes / (mode == PLAIN && tiles < 168 ? 3.46e6 : 4.15e6);
   us *= us * us;
   mem *= mem * mem;
   us = cbrt(sqrt(us * us + mem * mem));
@@ -637,7 +639,8 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
     for (int s : some) {
       if (s > 1 && (mode == SWIGLU || tiles * s > 520)) break;
       if (steps / s < t.stages) break;
-      const float us = estimate(t, tiles, steps, rows, columns, bytes, s);
+      const float us = estimate(t, tiles, steps, rows, columns, bytes, s,
+                                mode);
       if (best < 0 || us < least) {
         best = i;
         least = us;
