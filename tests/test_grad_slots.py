@@ -218,6 +218,92 @@ def test_same_gradients_gpu(monkeypatch):
                 assert torch.equal(got[0][n], want[0][n]), n
 
 
+def _model_grads(own, gas, tied, tokens, frozen=False):
+    """Gradients and weights of a model's steps; the second batch has none of the
+    first one's tokens, so that rows of the table are to be zero again."""
+    import deepspeed_amd
+    from deepspeed_amd.models import llama
+    torch.manual_seed(0)
+    cfg = llama.LlamaConfig(vocab_size=512, hidden_size=256,
+                            intermediate_size=512, num_layers=2, num_heads=2,
+                            num_kv_heads=1, max_seq_len=4096,
+                            tie_embeddings=tied)
+    model = llama.LlamaForCausalLM(cfg).cuda()
+    if frozen:
+        model.model.norm.weight.requires_grad_(False)
+    engine, opt, _, _ = deepspeed_amd.initialize(model=model, config={
+        "train_micro_batch_size_per_gpu": 3,
+        "gradient_accumulation_steps": gas, "bf16": {"enabled": True},
+        "zero_optimization": {"stage": 2}, "gradient_clipping": 1.0,
+        "optimizer": {"type": "AdamW", "params": {"lr": 1e-3}}})
+    named = dict(engine.module.named_parameters())
+    taken = []
+    if not own:
+        opt.drop_slots()
+    else:
+        class Seen(L.GradSlot):
+            __slots__ = ("name",)
+
+            def take(self):
+                out = super().take()
+                if out is not None:
+                    taken.append(self.name)
+                return out
+
+        slots = {}
+        for n, p in named.items():
+            if L.slot_of(p) is not None:
+                slots[p] = Seen(p, L.slot_of(p).view)
+                slots[p].name = n
+        opt._slots = [(p, slots[p], b) for p, _, b in opt._slots]
+    g = torch.Generator().manual_seed(1)
+    out = []
+    for i in range(3 * gas):
+        lo = 256 * (i % 2)
+        ids = torch.randint(lo, lo + 256, (3, tokens // 3), generator=g).cuda()
+        engine.backward(engine(ids, labels=ids))
+        out.append({n: p.grad.clone() for n, p in named.items()
+                    if p.grad is not None})
+        engine.step()
+    out.append({n: p.detach().clone() for n, p in named.items()})
+    engine.destroy()
+    return out, set(taken)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gas,tied,tokens,frozen", [
+    (1, False, 600, False), (2, False, 600, False), (1, True, 600, False),
+    (1, False, 9000, False), (1, False, 600, True)])
+def test_places_of_a_model_gpu(gas, tied, tokens, frozen):
+    """Embedding, norms and layers, each in its place, as added up there: over
+    accumulation, with a tied head, with a head in several chunks."""
+    import os
+    os.environ.setdefault("MASTER_ADDR", "127.0.0.1")
+    os.environ.setdefault("MASTER_PORT", "29548")
+    got, taken = _model_grads(True, gas, tied, tokens, frozen)
+    want, none = _model_grads(False, gas, tied, tokens, frozen)
+    assert not none
+    norms = {n for n in got[-1] if "norm" in n}
+    if frozen:
+        norms.remove("model.norm.weight")
+    assert norms <= taken
+    # several uses of one weight are added up
+    assert ("model.embed_tokens.weight" in taken) == (not tied)
+    assert ("lm_head.weight" in taken) == (not tied and tokens <= 8192)
+    for a, b in zip(got, want):
+        assert a.keys() == b.keys()
+        for n in b:
+            # one rounding to bf16 either way, but where two are added up first
+            if tied and "embed" in n or tokens > 8192 and "lm_head" in n:
+                assert torch.allclose(a[n].float(), b[n].float(),
+                                      rtol=2.0 ** -6, atol=1e-3), n
+            elif gas == 1 and not tied:
+                assert torch.equal(a[n], b[n]), n
+            else:
+                assert (a[n].float() - b[n].float()).norm() <= \
+                    2.0 ** -6 * b[n].float().norm(), n
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,h", [(3, 8), (700, 1024), (40, 8192), (5, 9000),
                                     (9, 33)])

@@ -19,7 +19,7 @@ def test_calls_left_alone():
     x = torch.randn(40, 256).bfloat16()
     with torch.no_grad():
         assert tile_linear(x, (lin,)) is None      # on the CPU
-    assert tile_linear(x, (lin,)) is None          # with gradients
+    assert tile_linear(x, (lin, lin)) is None
 
 
 def _inputs(m, ns, k, seed):
@@ -108,6 +108,13 @@ def test_refused_gpu():
     assert call(40, 224, 64) is None
     assert call(40, 128, 64) is None
     assert call(40, 256, 64, torch.float16) is None
+    with torch.enable_grad():              # one layer is the module's own
+        assert call(40, 256, 64) is None
+        lin = Linear(256, 64, device="cuda", dtype=torch.bfloat16)
+        x = torch.randn(40, 256, device="cuda", dtype=torch.bfloat16)
+        assert "_Linears" in type(tile_linear(x, (lin, lin))[0].grad_fn
+                                  ).__name__
+        assert tile_linear(x, (lin, lin), SWIGLU) is None
 
 
 def _limit(want, terms):
