@@ -59,10 +59,11 @@ __device__ __forceinline__ void place(int id, int blocks, int heads, int& blk,
 // the vector unit does one multiply-add, one exp2, half a maximum, one add and
 // half a conversion; the maximum is raised only where it grows by more than
 // 2^8, so that most steps rescale nothing. Bound by the vector unit beside the
-// matrix cores. 32 on 8 heads of 128, causal: 1 x 4096 163 us (842 TFLOP/s), 8 x
-// 4096 1260 us (873), 173 and 1340 while every step waited for the next
-// one's loads; with V transposed beforehand, fp32 scaling and conversions bit by
-// bit it took 350 us, torch's attention 389 and 2716.
+// matrix cores. 32 on 8 heads of 128, causal: 1 x 4096 170 us (810 TFLOP/s; 189
+// beside a prompt's products), 2 x 4096 302 (911), 8 x 4096 1250 (879), 5% more while
+// every step waited for the next one's loads; with V transposed beforehand, fp32
+// scaling and conversions bit by bit 1 x 4096 took 350 us, torch's attention 389 and
+// 2716 at 8 x 4096.
 
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(512) void fwd_kernel(

@@ -20,8 +20,8 @@
 // K 4096 16.0 / 13.3 and 12.2 / 10.8; N 128256 199 / 192 and 140 / 121; N 4096,
 // K 14336 27.7 / 27.3 and 19.7 / 18.9; N 4096, K 4096 10.2 / 10.1 and 8.2 / 8.6.
 // Three to six chunks ahead gained nothing more.
-//   * More rows, rows_linear_kernel: bound by x out of L2. Only int8 weights and
-// numbers of features that tile_linear.hip does not take come here.
+//   * More rows, rows_linear_kernel: bound by x out of L2. Only int8 weights, small
+// layers and numbers of features that tile_linear.hip does not take come here.
 //   * int8: a lane's 16 bytes are 16 inputs, split over two products; the order
 //     of the inputs inside a product is free, x is read in the same order. The
 //     bytes become bf16 exactly (8 bits), are summed in fp32 and multiplied by
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
       const long long r = min(n0 + f % (16 * FT), N - 1);
       scales[e] = a.scales[layer + f / (16 * FT)][(r * a.K + c * CH) / a.group];
     }
-    // not __syncthreads: that waits for the loads above as well
+    // the scales have arrived, and with them the loads above, which were first
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
   auto use = [&](int d, int i) __attribute__((always_inline)) {

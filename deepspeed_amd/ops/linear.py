@@ -112,9 +112,10 @@ def own_dx(T: int, ns, K: int) -> bool:
 def own_dw(T: int, N: int, K: int) -> bool:
     """Whether the gradient of a weight [N, K] over T rows is
     csrc/tile_linear.hip's (us, library with the copies of ``backward_plan`` and
-    kernel): 4096, K 4096, 4000 rows 122 / 102; 14336, K 4096, 4000 rows 453 / 383,
-    8192 767 / 796, 10000 1148 / 970, 32768 3529 / 3265; 3072, K 3072, 4000 rows 88 /
-    72; but 128256, K 4096, 8192 rows 6289 / 6630 (4000 rows 3454 / 3324)."""
+    kernel): 4096, K 4096, 4000 rows 126 / 103; 14336, K 4096, 4000 rows 437 / 398,
+    6144 573 / 598, 7000 687 / 667, 8192 767 / 796, 10000 1148 / 970, 32768 3529 /
+    3265; 3072, K 3072, 4000 rows 100 / 78, 24576 411 / 438; but 128256, K 4096, 8192
+    rows 6289 / 6630 (4000 rows 3454 / 3324)."""
     return T > 192 and N % 8 == 0 and K % 8 == 0 and T < 1 << 30 and \
         N <= FEATURES and K <= INPUTS and (T < 6144 or N * K < 1 << 28)
 
@@ -203,10 +204,11 @@ def _dx(dys, weights, own: bool):
 
 class GradSlot:
     """Where the gradient of a parameter belongs: ``view``, a part of its owner's
-    flat buffer. While it is ``open`` (the owner's backward, no gradient there
-    yet; it is the tensor that the parameter has as its gradient) the product of the parameter's one layer may be written into it. Autograd
-    then keeps that very tensor as the gradient, where it added a new one to the
-    buffer: two reads and a write of every weight's gradient, 20 us for 25M values.
+    flat buffer. While it is ``open`` (the owner's backward, nothing there yet; it
+    holds the tensor that the parameter has as its gradient) the product of the
+    parameter's one layer may be written into it. Autograd then keeps that very
+    tensor as the gradient, where it added a new one to the buffer: two reads and a
+    write of every weight's gradient, 20 us for 25M values.
 
     uses: forward products since the owner's last backward; a weight of several
     keeps to the addition. void: a product was given the place, whose parameter
