@@ -29,6 +29,7 @@
 #include "ds_kernels.h"
 
 #include <cmath>
+#include <utility>
 
 #pragma clang diagnostic ignored "-Winline-asm"     // m0 among the clobbers
 
@@ -493,6 +494,568 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
   }
 }
 
+template <int... I, typename F>
+__device__ __forceinline__ void each(std::integer_sequence<int, I...>, F& f) {
+  (f(Int<I>{}), ...);
+}
+
+// One operand's descriptor: loads past `left` bytes from `base` on bring zeros,
+// stores there are dropped.
+__device__ __forceinline__ u32x4 descriptor(const char* base, long long left) {
+  const unsigned long long b = (unsigned long long)(uintptr_t)base;
+  u32x4 d;
+  d[0] = __builtin_amdgcn_readfirstlane((unsigned)b);
+  d[1] = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32) & 0xffffu);
+  d[2] = __builtin_amdgcn_readfirstlane(
+      left > 0xffffffffll ? 0xffffffffu : left < 0 ? 0u : (unsigned)left);
+  d[3] = 0x00020000u;
+  return d;
+}
+// 16 bytes a lane from descriptor + off + soff to LDS at m0, lane after lane. In
+// two parts: m0 has to be written an instruction ahead, which a product fills.
+__device__ __forceinline__ void load_to(int lds, int n) {
+  asm volatile("s_add_u32 m0, %0, %1" :: "s"(lds), "i"(n) : "memory", "m0", "scc");
+}
+__device__ __forceinline__ void load(u32x4 from, unsigned off, int soff) {
+  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds"
+               :: "v"(off), "s"(from), "s"(soff) : "memory");
+}
+// The sums of a wave that has all 256 accumulation registers: four from R on. They
+// are named, not variables: those the compiler moves to other registers and, as they
+// run out, to memory. It has to have no use for these registers itself (nothing is
+// spilled: some 170 to 190 of 256 others are taken). Operands have to be written, and
+// products made, some instructions before they are read.
+__device__ __forceinline__ void take_sums() {
+  asm volatile("" ::: "a0", "a255");
+}
+template <int R>
+__device__ __forceinline__ void add_product(s16x8 a, s16x8 b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, a[%2:%3]"
+               :: "v"(a), "v"(b), "n"(R), "n"(R + 3));
+}
+template <int R>
+__device__ __forceinline__ void zero(s16x8 zeros) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 a[%1:%2], %0, %0, 0"
+               :: "v"(zeros), "n"(R), "n"(R + 3));
+}
+template <int R>
+__device__ __forceinline__ float sum() {
+  float x;
+  asm volatile("v_accvgpr_read_b32 %0, a[%1:%1]" : "=v"(x) : "n"(R));
+  return x;
+}
+__device__ __forceinline__ void wait_reads() {    // of LDS
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+}
+__device__ __forceinline__ s16x8 lds_read(int at) {
+  return *(const __attribute__((address_space(3))) s16x8*)(uintptr_t)(unsigned)at;
+}
+__device__ __forceinline__ s16x4 lds_tr_read(int at) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s16x4*)(uintptr_t)(unsigned)at);
+}
+__device__ __forceinline__ unsigned packed2(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned,
+                            __builtin_convertvector((f32x2{lo, hi}), b16x2));
+}
+
+// The largest tiles, 256 x 256, by four waves of 128 x 128, one a SIMD: a wave's
+// 256 sums are the accumulation registers, and LDS is read for 64 products of a
+// half stage by 16 operands (eight waves of 128 x 64: 12 for 32). The chip's power
+// bounds these products, so reads that are not made become clock.
+//
+//   * A workgroup stays on its CU and goes on from tile to tile: the ring is
+// filled across the border, so that a tile's first stages load while the one before
+// is computed and stored.
+//   * One barrier a stage, behind the reads of its second half: from there on the
+// stage's places in the ring are free (x two stages, W three), and the next stage
+// has arrived. A barrier costs some 70 of a stage's 2500 cycles, a load between two
+// products 17 (of 2048 that are products), their arrival nothing.
+//   * PLAIN and SWIGLU: x is the first operand of the products and a lane's tiles
+// of W are neighbouring features (brought about by which row is loaded where), so
+// that 16 lanes store 256 bytes of a row without a pass through LDS. The gradients,
+// whose W lies across, exchange halves between rows of 16 lanes.
+//
+// us, eight waves with a tile a workgroup, and now: 8192 x 8192 x 8192 786 / 735;
+// 4096 rows, K 4096: 28672 690 / 653, 6144 175 / 164, gate and up 14336 712 / 680;
+// gate and up 18944, K 3584, 2331 rows 517 / 497; dx of 14336, K 4096, 8192 rows 738 /
+// 685; dW of that 765 / 762 (its transposing reads are two an operand).
+template <int MODE, bool PARTS>
+__global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
+  constexpr bool GLU = MODE == SWIGLU;
+  constexpr bool WT = MODE == GRAD_X || MODE == GRAD_W, XT = MODE == GRAD_W;
+  constexpr int BM = 256, BN = 256, F = 8;      // tiles of 16 a wave, either way
+  constexpr int P = 8;                          // loads of 1 KB a wave, each
+  constexpr int SW = BN * ROW, SX = BM * ROW, XAT = 3 * SW;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int lane = threadIdx.x & 63;
+  const int wid = uni(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int wm = wid >> 1, wn = wid & 1;
+  const int K = a.K;
+
+  // Tiles in the order of the kernel above; an XCD's workgroups take its run in
+  // turn, so that they work side by side.
+  constexpr int GROUP = 4;
+  const int per = a.tiles * a.mtiles, total = per * a.splits;
+  const int slots = gridDim.x / 8, xcd = blockIdx.x % 8;
+  int item = xcd * (total / 8) + min(xcd, total % 8);
+  const int end = item + total / 8 + (xcd < total % 8);
+  item += blockIdx.x / 8;
+  if (item >= end) return;
+
+  struct Place {
+    int m0, n0, s0, n_it, layer, split;
+  };
+  auto locate = [&](int id) INLINE {
+    Place p;
+    p.split = uni(id / per);
+    id -= p.split * per;
+    const int group = id / (GROUP * a.tiles);
+    const int high = min(GROUP, a.mtiles - GROUP * group);
+    id -= group * GROUP * a.tiles;
+    int mt = GROUP * group + id % high, nt = id / high, l = 0;
+    if (MODE == PLAIN) {
+      while (nt >= a.tile_end[l]) ++l;
+      if (l) nt -= a.tile_end[l - 1];
+    }
+    if (MODE == GRAD_W) {
+      while (mt >= a.tile_end[l]) ++l;
+      if (l) mt -= a.tile_end[l - 1];
+    }
+    p.layer = uni(l);
+    p.n0 = uni(nt * (GLU ? BN / 2 : BN));
+    p.m0 = uni(mt * BM);
+    const int steps = MODE == GRAD_X ? a.steps
+        : MODE == GRAD_W ? (a.M + BK - 1) / BK : K / BK;
+    p.s0 = uni(p.split * steps / a.splits);
+    p.n_it = uni((p.split + 1) * steps / a.splits) - p.s0;
+    return p;
+  };
+  Place at = locate(item), next = at;
+  bool more = item + slots < end;
+  if (more) next = locate(item + slots);
+
+  // ---- loads: the lanes' places in the pieces of 1 KB, as above. Rows past the
+  // end lie past the descriptor's; columns past the end are not stored.
+  const int lr = lane >> 3, lc = lane & 7;
+  auto place_w = [&](int j) INLINE {
+    const int piece = j * 4 + wid;
+    if (WT)
+      return (unsigned)(piece % 8 * 8 + lr) * K * 2 +
+          2 * (piece / 8 * 64 +
+               8 * (lc ^ (2 * ((lr >> 1) & 1) + 4 * (wid & 1))));
+    // tile f of a wave: features F c + f, or gate and up of 4 c + f / 2
+    const int half = piece / 16, f = piece / 2 % 8, c = piece % 2 * 8 + lr;
+    const int r = GLU ? half * 64 + F / 2 * c + (f >> 1) : half * 128 + F * c + f;
+    return (unsigned)r * K * 2 + ((lc ^ lr) << 4);
+  };
+  auto place_x = [&](int j, int ld) INLINE {
+    const int piece = j * 4 + wid;
+    if (XT)
+      return (unsigned)(piece % 8 * 8 + lr) * ld * 2 +
+          2 * (piece / 8 * 64 +
+               8 * (lc ^ (2 * ((lr >> 1) & 1) + 4 * (wid & 1))));
+    return (unsigned)(piece * 8 + lr) * ld * 2 + ((lc ^ lr) << 4);
+  };
+  unsigned woff[P], xoff[P];
+#pragma unroll
+  for (int j = 0; j < P; ++j) {
+    woff[j] = place_w(j);
+    xoff[j] = place_x(j, K);
+  }
+  // From contraction step `step` of a tile on: descriptor, bytes to its end (the
+  // operands that lie across move it), stages that follow one another there.
+  u32x4 wfrom, xfrom;
+  const char *wbase, *xbase;
+  long long wend, xend;
+  int wsoff = 0, xsoff = 0, wrow = ROW, xrow = ROW, wleft, xleft;
+  int wstep, xstep, wstop, xstop, xld = K;
+  auto seek_w = [&](int n0, int layer, int step, int stop) INLINE {
+    wstop = uni(stop);
+    wleft = stop - step;
+    if (MODE == GRAD_X) {
+      int l = 0;
+      while (step >= a.step_end[l]) ++l;
+      const int k = (step - (l ? a.step_end[l - 1] : 0)) * BK;
+      wbase = (const char*)(a.w[l] + (long long)k * K + n0);
+      wend = ((long long)(a.n[l] - k) * K - n0) * 2;
+      wleft = min(stop, a.step_end[l]) - step;
+    } else if (MODE == GRAD_W) {
+      wbase = (const char*)(a.w[0] + (long long)step * BK * K + n0);
+      wend = ((long long)(a.M - step * BK) * K - n0) * 2;
+    } else {
+      const short* w = GLU ? (wid & 2 ? a.w[1] : a.w[0]) : a.w[layer];
+      wbase = (const char*)(w + (long long)n0 * K);
+      wend = (long long)(a.n[layer] - n0) * K * 2;
+      wsoff = uni(step * ROW);
+    }
+    wstep = uni(step);
+    wleft = uni(wleft);
+    wfrom = descriptor(wbase, wend);
+  };
+  auto seek_x = [&](int m0, int layer, int step, int stop) INLINE {
+    xstop = uni(stop);
+    xleft = stop - step;
+    if (MODE == GRAD_X) {
+      int l = 0;
+      while (step >= a.step_end[l]) ++l;
+      xld = uni(a.n[l]);
+      xbase = (const char*)(a.x[l] + (long long)m0 * xld);
+      xend = (long long)(a.M - m0) * xld * 2;
+      xsoff = uni((step - (l ? a.step_end[l - 1] : 0)) * ROW);
+      xleft = min(stop, a.step_end[l]) - step;
+    } else if (MODE == GRAD_W) {
+      xld = uni(a.n[layer]);
+      xbase = (const char*)(a.x[layer] + (long long)step * BK * xld + m0);
+      xend = ((long long)(a.M - step * BK) * xld - m0) * 2;
+    } else {
+      xbase = (const char*)(a.x[0] + (long long)m0 * K);
+      xend = (long long)(a.M - m0) * K * 2;
+      xsoff = uni(step * ROW);
+    }
+    xstep = uni(step);
+    xleft = uni(xleft);
+    xfrom = descriptor(xbase, xend);
+    if (MODE >= GRAD_X)
+#pragma unroll
+      for (int j = 0; j < P; ++j) xoff[j] = place_x(j, xld);
+  };
+  // Behind the last of these: the next layer, the next tile, or nothing, which is
+  // a descriptor of no bytes.
+  bool wover = false, xover = false;
+  auto turn_w = [&]() INLINE {
+    if (MODE == GRAD_X && wstep + 1 < wstop) {
+      seek_w(wover ? next.n0 : at.n0, 0, wstep + 1, wstop);
+    } else if (more && !wover) {
+      wover = true;
+      seek_w(next.n0, next.layer, next.s0, next.s0 + next.n_it);
+    } else {
+      wfrom[2] = 0;
+      wsoff = wrow = 0;
+      wend = 0;
+      wleft = 1 << 30;
+    }
+  };
+  auto turn_x = [&]() INLINE {
+    if (MODE == GRAD_X && xstep + 1 < xstop) {
+      seek_x(xover ? next.m0 : at.m0, 0, xstep + 1, xstop);
+    } else if (more && !xover) {
+      xover = true;
+      seek_x(next.m0, next.layer, next.s0, next.s0 + next.n_it);
+    } else {
+      xfrom[2] = 0;
+      xsoff = xrow = 0;
+      xend = 0;
+      xleft = 1 << 30;
+    }
+  };
+  auto move_w = [&]() INLINE {
+    if (WT) {
+      const long long d = wrow ? (long long)BK * K * 2 : 0;
+      wbase += d;
+      wend -= d;
+      wfrom = descriptor(wbase, wend);
+      if (MODE == GRAD_X) ++wstep;
+    } else {
+      wsoff += wrow;
+    }
+  };
+  auto move_x = [&]() INLINE {
+    if (XT) {
+      const long long d = xrow ? (long long)BK * xld * 2 : 0;
+      xbase += d;
+      xend -= d;
+      xfrom = descriptor(xbase, xend);
+    } else {
+      xsoff += xrow;
+      if (MODE == GRAD_X) ++xstep;
+    }
+  };
+  const int lds_at = (int)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const int put = lds_at + wid * 1024;
+  int wput = put, xput = put + XAT, wget = 0, xget = 0;
+  auto next_w = [&](int b, int first) INLINE {
+    return b == first + 2 * SW ? first : b + SW;
+  };
+  auto fill_w = [&]() INLINE {
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      load_to(wput, j * 4096);
+      asm volatile("s_nop 0");
+      load(wfrom, woff[j], wsoff);
+    }
+    wput = next_w(wput, put);
+    if (--wleft == 0) turn_w();
+    else move_w();
+  };
+  auto fill_x = [&]() INLINE {
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      load_to(xput, j * 4096);
+      asm volatile("s_nop 0");
+      load(xfrom, xoff[j], xsoff);
+    }
+    xput = xput == put + XAT ? xput + SX : put + XAT;
+    if (--xleft == 0) turn_x();
+    else move_x();
+  };
+
+  // ---- operands: 16 rows (or columns) by inputs 32 h + 8 g + j, at the lane's
+  // addresses and constants. Across, tiles of 16 columns have four of them.
+  const int tr = (8 * g + (col >> 2)) * 128 + (col & 3) * 8 +
+      32 * ((col >> 3) & 1) + 64 * (g & 1);
+  const int o0 = (g ^ (col & 7)) << 4;
+  const int w0 = WT ? lds_at + wn * 16384 + tr
+                    : lds_at + (wn * (BN / 2) + col) * ROW + o0;
+  const int x0 = XAT + (XT ? lds_at + wm * 16384 + tr
+                           : lds_at + (wm * (BM / 2) + col) * ROW + o0);
+  int wat[WT ? 4 : 1], xat[XT ? 4 : 1];
+  auto aim = [&](int h) INLINE {    // at a half of the stage
+    if (!WT || h == 0)
+#pragma unroll
+      for (int c = 0; c < (WT ? 4 : 1); ++c) {
+        wat[c] = (w0 ^ (WT ? 32 * c : 64 * h)) + wget;
+        asm volatile("" : "+v"(wat[c]));
+      }
+    if (!XT || h == 0)
+#pragma unroll
+      for (int c = 0; c < (XT ? 4 : 1); ++c) {
+        xat[c] = (x0 ^ (XT ? 32 * c : 64 * h)) + xget;
+        asm volatile("" : "+v"(xat[c]));
+      }
+  };
+  s16x8 wa[2][F], xa[2][F];
+  auto across = [&](int at, int i, int h) INLINE {
+    const s16x4 lo = lds_tr_read(at + i / 4 * 8192 + h * 4096);
+    const s16x4 hi = lds_tr_read(at + i / 4 * 8192 + h * 4096 + 512);
+    return s16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  };
+  auto get = [&](int q, int h) INLINE {
+    if (q < F)
+      wa[h][q] = WT ? across(wat[WT ? q % 4 : 0], q, h)
+                    : lds_read(wat[0] + q * 16 * ROW);
+    else
+      xa[h][q - F] = XT ? across(xat[XT ? q % 4 : 0], q - F, h)
+                        : lds_read(xat[0] + (q - F) * 16 * ROW);
+  };
+  // sums of a tile of W and one of x
+#define acc(f, m) (((f) * F + (m)) * 4)
+  take_sums();
+  auto clear = [&]() INLINE {
+    s16x8 zeros = {};
+    asm volatile("s_nop 4" : "+v"(zeros));    // written before it is multiplied
+    auto one = [&](auto i) INLINE { zero<decltype(i)::value * 4>(zeros); };
+    each(std::make_integer_sequence<int, F * F>{}, one);
+  };
+  clear();
+
+  seek_w(at.n0, at.layer, at.s0, at.s0 + at.n_it);
+  seek_x(at.m0, at.layer, at.s0, at.s0 + at.n_it);
+  fill_w();
+  fill_x();
+  fill_w();
+  fill_x();
+  fill_w();
+  wait_loads<3 * P>();
+  barrier();
+  aim(0);
+#pragma unroll
+  for (int q = 0; q < 2 * F; ++q) get(q, 0);
+
+  // A stage's 128 products. Reads of its second half lie between the first ones,
+  // those of the next stage's first half behind the middle; x two stages ahead and
+  // W three are loaded behind the barrier.
+  constexpr int N2 = 2 * F * F, BARRIER = 30;
+  constexpr int STORES = 4 * F;     // of a tile, at least
+  int young = 0;        // a tile's stores are behind the loads that are waited for
+  while (true) {
+#pragma clang loop unroll(disable)
+    for (int it = 0; it < at.n_it; ++it) {
+      __builtin_amdgcn_sched_barrier(0);
+      wait_reads();
+      aim(1);
+      auto product = [&](auto at) INLINE {
+        constexpr int i = decltype(at)::value, h = i / (F * F), m = i / F % F;
+        constexpr int f = m % 2 ? F - 1 - i % F : i % F;
+        if constexpr (i == BARRIER) {
+          asm volatile("s_cmp_lg_u32 %0, 0\n\t"
+                       "s_cbranch_scc1 1f\n\t"
+                       "s_waitcnt vmcnt(%1)\n"
+                       "1:\n\t"
+                       "s_waitcnt vmcnt(%2)"
+                       :: "s"(young), "n"(P), "n"(P + STORES) : "memory", "scc");
+          wait_reads();
+          __builtin_amdgcn_s_barrier();
+          wget = next_w(wget, 0);
+          xget ^= SX;
+          aim(0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = 0; q < P; ++q) {
+          if (i == BARRIER + 2 + 6 * q) load_to(xput, q * 4096);
+          if (i == BARRIER + 52 + 6 * q) load_to(wput, q * 4096);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = 0; q < 2 * F; ++q) {
+          if (i == q * 3 / 2) get(q, 1);
+          if (i == 67 + 2 * q) get(q, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (WT) add_product<acc(f, m)>(wa[h][f], xa[h][m]);
+        else add_product<acc(f, m)>(xa[h][m], wa[h][f]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < P; ++q) {
+          if (i == BARRIER + 2 + 6 * q) load(xfrom, xoff[q], xsoff);
+          if (i == BARRIER + 52 + 6 * q) load(wfrom, woff[q], wsoff);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      each(std::make_integer_sequence<int, N2>{}, product);
+      young = 0;
+      xput = xput == put + XAT ? xput + SX : put + XAT;
+      wput = next_w(wput, put);
+      --wleft;
+      --xleft;
+      if (min(wleft, xleft) > 0) {
+        move_w();
+        move_x();
+      } else {
+        if (wleft == 0) turn_w();
+        else move_w();
+        if (xleft == 0) turn_x();
+        else move_x();
+      }
+    }
+
+    asm volatile("s_nop 15");     // the last products
+    // Every store is made, past the tile's rows or columns to nowhere: the waits
+    // above count them.
+    const int N = WT ? K : a.n[at.layer];
+    const int rows = MODE == GRAD_W ? a.n[at.layer] : a.M;
+    const int m_of = uni(at.m0 + wm * (BM / 2));
+    const int have = uni(max(0, min(rows - m_of, BM / 2)));
+    constexpr unsigned NOWHERE = 0x80000000u;
+    if constexpr (PARTS) {
+      const int before = a.n_end[at.layer] - a.n[at.layer];
+      const int all = WT ? K : a.n_end[a.layers - 1];
+      const int all_rows = MODE == GRAD_W ? a.n_end[a.layers - 1] : a.M;
+      const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(a.part + ((long long)at.split * all_rows + m_of +
+                            (MODE == GRAD_W ? before : 0)) * all +
+                  (MODE == PLAIN ? before : 0)),
+          (short)0, (int)((unsigned)have * all * 4), 0x00020000);
+      // gradients: row col, columns 4 g ..; otherwise rows 4 g + r, half of eight
+      const int n1 = at.n0 + wn * (BN / 2) + (WT ? 4 * g : F * col);
+      const int r1 = WT ? col : 4 * g;
+      auto store = [&](auto at) INLINE {
+        constexpr int m = decltype(at)::value / F, i = decltype(at)::value % F;
+        constexpr int f = 4 * (i & 1), r = i >> 1;
+        f32x4 v;
+        if constexpr (WT)
+          v = f32x4{sum<acc(i, m)>(), sum<acc(i, m) + 1>(), sum<acc(i, m) + 2>(),
+                    sum<acc(i, m) + 3>()};
+        else
+          v = f32x4{sum<acc(f, m) + r>(), sum<acc(f + 1, m) + r>(),
+                    sum<acc(f + 2, m) + r>(), sum<acc(f + 3, m) + r>()};
+        const int row = r1 + 16 * m + (WT ? 0 : r);
+        const int n = n1 + (WT ? 16 * i : f);
+        __builtin_amdgcn_raw_buffer_store_b128(
+            __builtin_bit_cast(u32x4, v), to,
+            n < N && row < have ? (unsigned)(row * all + n) * 4 : NOWHERE, 0, 0);
+      };
+      each(std::make_integer_sequence<int, F * F>{}, store);
+    } else {
+      short* out = a.out[MODE == GRAD_X || GLU ? 0 : at.layer];
+      const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(out + (long long)m_of * N), (short)0,
+          (int)((unsigned)have * N * 2), 0x00020000);
+      if constexpr (WT) {
+        // columns 4 g .. of two tiles to 8 of one: odd rows of lanes of the first
+        // change places with even ones of the second
+        const int n1 = at.n0 + wn * (BN / 2) + (g & 1) * 16 + (g >> 1) * 8;
+        auto store = [&](auto at) INLINE {
+          constexpr int f = decltype(at)::value / F * 2, m = decltype(at)::value % F;
+          constexpr int A = acc(f, m), B = acc(f + 1, m);
+          const unsigned y0 = packed2(sum<A>(), sum<A + 1>());
+          const unsigned y1 = packed2(sum<A + 2>(), sum<A + 3>());
+          const unsigned z0 = packed2(sum<B>(), sum<B + 1>());
+          const unsigned z1 = packed2(sum<B + 2>(), sum<B + 3>());
+          const auto lo = __builtin_amdgcn_permlane16_swap(y0, z0, false, false);
+          const auto hi = __builtin_amdgcn_permlane16_swap(y1, z1, false, false);
+          const int n = n1 + 16 * f;
+          __builtin_amdgcn_raw_buffer_store_b128(
+              u32x4{lo[0], hi[0], lo[1], hi[1]}, to,
+              n < N ? (unsigned)((16 * m + col) * N + n) * 2 : NOWHERE, 0, 0);
+        };
+        each(std::make_integer_sequence<int, F / 2 * F>{}, store);
+      } else {
+        constexpr int W = GLU ? F / 2 : F;      // features a lane
+        const int n = at.n0 + wn * (GLU ? BN / 4 : BN / 2) + W * col;
+        float b[GLU ? 2 : 1][W];
+#pragma unroll
+        for (int l = 0; l < (GLU ? 2 : 1); ++l) {
+          const short* bias = a.bias[GLU ? l : at.layer];   // of none: zeros
+          const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
+              (void*)bias, (short)0, bias ? N * 2 : 0, 0x00020000);
+#pragma unroll
+          for (int e = 0; e < W; ++e)
+            b[l][e] = value((short)__builtin_amdgcn_raw_buffer_load_b16(
+                from, (n + e) * 2, 0, 0));
+        }
+        typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+        auto store = [&](auto at) INLINE {
+          constexpr int m = decltype(at)::value / 4, r = decltype(at)::value % 4;
+          const unsigned o =
+              n < N ? (unsigned)((4 * g + 16 * m + r) * N + n) * 2 : NOWHERE;
+          auto one = [&](auto at) INLINE {
+            constexpr int e = decltype(at)::value;
+            if constexpr (GLU) {
+              const float t = sum<acc(2 * e, m) + r>() + b[0][e];
+              return t / (1.f + expf(-t)) *
+                  (sum<acc(2 * e + 1, m) + r>() + b[GLU][e]);
+            } else {
+              return sum<acc(e, m) + r>() + b[0][e];
+            }
+          };
+          const u32x2 v = {packed2(one(Int<0>{}), one(Int<1>{})),
+                           packed2(one(Int<2>{}), one(Int<3>{}))};
+          if constexpr (GLU)
+            __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, 0);
+          else {
+            const u32x2 u = {packed2(one(Int<4>{}), one(Int<5>{})),
+                             packed2(one(Int<6>{}), one(Int<7>{}))};
+            if (N % 8 == 0) {
+              __builtin_amdgcn_raw_buffer_store_b128(u32x4{v[0], v[1], u[0], u[1]},
+                                                     to, o, 0, 0);
+            } else {
+              __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, 0);
+              __builtin_amdgcn_raw_buffer_store_b64(
+                  u, to, n + 4 < N ? o + 8 : NOWHERE, 0, 0);
+            }
+          }
+        };
+        each(std::make_integer_sequence<int, 4 * F>{}, store);
+      }
+    }
+    if (!more) break;
+    at = next;
+    item += slots;
+    more = item + slots < end;
+    if (more) next = locate(item + slots);
+    wover = xover = false;
+    young = 1;
+    clear();
+  }
+  wait_loads<0>();
+}
+#undef acc
+
 // Adds the splits up: four columns of a row a thread.
 template <int MODE>
 __global__ __launch_bounds__(256) void tile_merge_kernel(const Args a,
@@ -520,10 +1083,9 @@ __global__ __launch_bounds__(256) void tile_merge_kernel(const Args a,
       packed(add_bias(y, a.bias[l], n));
 }
 
-template <int BM, int BN, int WM, int WN, int NS, int MODE>
-int launch(Args a, bool merge, hipStream_t st) {
-  constexpr int LDS = NS * (BM + BN) * ROW;
-  static_assert(LDS <= 160 * 1024, "");
+// Tiles and stages of a launch, before the kernel's own numbers of them.
+template <int BM, int BN, int MODE>
+int count(Args& a) {
   constexpr int bn = MODE == SWIGLU ? BN / 2 : BN;
   int sum = 0, steps = 0;
   for (int i = 0; i < a.layers; ++i) {
@@ -535,20 +1097,50 @@ int launch(Args a, bool merge, hipStream_t st) {
   a.steps = steps;
   a.tiles = MODE >= GRAD_X ? (a.K + bn - 1) / bn : sum;
   a.mtiles = MODE == GRAD_W ? sum : (a.M + BM - 1) / BM;
+  return a.tiles * a.mtiles * a.splits;
+}
+
+template <int MODE>
+int merge_splits(const Args& a, hipStream_t st) {
+  const int n = a.n_end[a.layers - 1];
+  const int rows = MODE == GRAD_W ? n : a.M, all = MODE >= GRAD_X ? a.K : n;
+  const long long q = (long long)rows * (all / 4);
+  hipLaunchKernelGGL(tile_merge_kernel<MODE>, dim3((unsigned)((q + 255) / 256)),
+                     dim3(256), 0, st, a, rows, all);
+  return (int)hipGetLastError();
+}
+
+template <int BM, int BN, int WM, int WN, int NS, int MODE>
+int launch(Args a, bool merge, hipStream_t st) {
+  constexpr int LDS = NS * (BM + BN) * ROW;
+  static_assert(LDS <= 160 * 1024, "");
+  const int items = count<BM, BN, MODE>(a);
   auto kernel = tile_linear_kernel<BM, BN, WM, WN, NS, MODE>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (e != hipSuccess) return (int)e;
-  hipLaunchKernelGGL(kernel, dim3(a.tiles * a.mtiles * a.splits),
-                     dim3(WM * WN * 64), LDS, st, a);
-  if (a.splits > 1 && merge) {
-    const int n = a.n_end[a.layers - 1];
-    const int rows = MODE == GRAD_W ? n : a.M, all = MODE >= GRAD_X ? a.K : n;
-    const long long q = (long long)rows * (all / 4);
-    hipLaunchKernelGGL(tile_merge_kernel<MODE>,
-                       dim3((unsigned)((q + 255) / 256)), dim3(256), 0, st, a,
-                       rows, all);
-  }
+  hipLaunchKernelGGL(kernel, dim3(items), dim3(WM * WN * 64), LDS, st, a);
+  if (a.splits > 1 && merge) return merge_splits<MODE>(a, st);
+  return (int)hipGetLastError();
+}
+
+template <int MODE>
+int launch_wide(Args a, bool merge, hipStream_t st) {
+  constexpr int LDS = 160 * 1024, CUS = 256;
+  const int items = count<256, 256, MODE>(a);
+  const int steps = MODE == GRAD_X ? a.steps
+      : MODE == GRAD_W ? (a.M + BK - 1) / BK : a.K / BK;
+  // W is loaded up to three stages ahead, into the next tile but not the one
+  // behind it: shorter contractions have a workgroup a tile
+  const int grid = items < CUS || steps / a.splits < 4 ? (items + 7) / 8 * 8 : CUS;
+  auto kernel = MODE != SWIGLU && a.splits > 1
+      ? wide_linear_kernel<MODE, MODE != SWIGLU>
+      : wide_linear_kernel<MODE, false>;
+  const hipError_t e = hipFuncSetAttribute(
+      (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), LDS, st, a);
+  if (a.splits > 1 && merge) return merge_splits<MODE>(a, st);
   return (int)hipGetLastError();
 }
 
@@ -566,8 +1158,8 @@ int launch(Args a, bool merge, hipStream_t st) {
   X(5, 192, 128, 4, 2, 4, 0.646f, 4.8f)    \
   X(6, 192, 256, 4, 2, 2, 1.060f, 7.5f)    \
   X(7, 256, 128, 4, 2, 3, 0.790f, 5.7f)    \
-  X(8, 256, 192, 2, 4, 2, 1.038f, 7.0f)    \
-  X(9, 256, 256, 2, 4, 2, 1.342f, 8.4f)
+  X(8, 256, 192, 2, 4, 2, 1.038f, 7.0f)
+constexpr int WIDE = 9;
 
 // A wave's gate and up tiles in pairs; halves of x in blocks of 64 columns.
 #define GATES(BN, WN) (BN / WN / 16 % 2 == 0)
@@ -586,6 +1178,7 @@ const Tile tiles_[] = {
   {BM, BN, NS, GATES(BN, WN), BLOCKS(BM, WM), U, F},
     TILES(X)
 #undef X
+    {256, 256, 2, true, true, 1.262f, 7.9f},    // WIDE
 };
 
 // us that a tile and a number of splits take: rounds of the 256 CUs (the last
@@ -627,7 +1220,7 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
   float least = 0;
   for (int i = 0; i < (int)(sizeof(tiles_) / sizeof(Tile)); ++i) {
     const Tile& t = tiles_[i];
-    if (!t.takes(mode)) continue;
+    if (!t.takes(mode) || (i == WIDE && columns >= 1 << 22)) continue;
     double tiles = 0;
     for (int l = 0; l < layers; ++l)    // SWIGLU: a gate and an up each
       tiles += mode == GRAD_W ? (n[l] + t.bm - 1) / t.bm
@@ -686,6 +1279,9 @@ extern "C" int ds_tile_linear(const void* const* x, int layers,
   a.part = part;
   a.M = M; a.K = K; a.layers = layers; a.splits = splits;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  // WIDE stores at 32-bit offsets in 128 rows
+  if (tile == WIDE && (mode >= GRAD_X ? K : total) >= 1 << 22)
+    return (int)hipErrorInvalidValue;
   switch (tile) {
 #define X(I, BM, BN, WM, WN, NS, U, F)                                    \
   case I:                                                                 \
@@ -700,6 +1296,11 @@ extern "C" int ds_tile_linear(const void* const* x, int layers,
     return launch<BM, BN, WM, WN, NS, PLAIN>(a, merge, st);
     TILES(X)
 #undef X
+  case WIDE:
+    if (mode == GRAD_X) return launch_wide<GRAD_X>(a, merge, st);
+    if (mode == GRAD_W) return launch_wide<GRAD_W>(a, merge, st);
+    if (mode == SWIGLU) return launch_wide<SWIGLU>(a, merge, st);
+    return launch_wide<PLAIN>(a, merge, st);
   }
   return (int)hipErrorInvalidValue;
 }

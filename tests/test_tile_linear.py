@@ -158,6 +158,35 @@ def test_every_tile_backward_gpu(tile):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("steps", [2, 3, 4, 5, 9])
+@torch.no_grad()
+def test_widest_tile_goes_on_gpu(steps):
+    """256 x 256: more tiles than workgroups, which go on from tile to tile, over
+    the shortest contractions (of which each has a workgroup) and longer ones."""
+    from deepspeed_amd.ops import _C
+    wide, k = len(TILES) - 1, 64 * steps
+    for m, ns, mode in ((4100, (4360,), 0), (2305, (6148, 516, 264), 0),
+                        (2100, (4100, 4100), SWIGLU)):
+        x, ws, bs = _inputs(m, ns, k, steps)
+        for y, want in zip(_C.tile_linear(x, ws, bs, mode, wide, 1),
+                           _want(x, ws, bs, mode)):
+            _close(y, want)
+    for splits in (1, 2):       # dx [4100, 4360] over two layers, dW of as many
+        ns = (64 * splits * steps - 64, 64)
+        _, ws, _ = _inputs(1, ns, 4360, steps)
+        dys = [_inputs(4100, (), n, n)[0] for n in ns]
+        want = sum(d.double() @ w.double() for d, w in zip(dys, ws))
+        err = (_C.tile_linear_dx(dys, ws, wide, splits).double() - want).abs()
+        assert (err <= _limit(want, sum(ns))).all()
+        m = 64 * splits * steps - 3
+        x, _, _ = _inputs(m, (), 4360, steps)
+        dys = [_inputs(m, (), n, n)[0] for n in (4104, 264)]
+        for got, d in zip(_C.tile_linear_dw(x, dys, wide, splits), dys):
+            want = d.double().t() @ x.double()
+            assert ((got.double() - want).abs() <= _limit(want, m)).all()
+
+
+@pytest.mark.gpu
 def test_what_lies_past_the_last_row_gpu():
     """Rows past the end count for nothing, whatever the last one holds: each
     value of the weight's gradient comes from its own column."""
