@@ -277,8 +277,21 @@ __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
   const int mine = (chunks - wid + NW - 1) / NW;    // wid, wid + NW, ..
   Weights<I8> w[D][S];
   s16x8 x[D][CH / 32];
+  // Workgroups that all begin at the rows' beginnings read the same few memory
+  // channels at a time where rows are whole multiples of 16 KB (int8: 4 KB) apart; each
+  // begins elsewhere there (us, 8 rows, before / now: bf16 8192, K 8192 31.6 / 25.0,
+  // 28672 x 2, K 8192 165 / 156; int8 14336 x 2, K 4096 33.8 / 30.8, 4096 8.6 / 7.8,
+  // 128256 117 / 113, of 1 row 109 / 97; but apart by 6 KB, 8192 x 2, K 3072 bf16 19.7 /
+  // 20.4, by 28, 4096, K 14336 of 1 row 22.7 / 23.9, by 8, 128256, K 4096 185 / 189).
+  const int turn = a.K % (I8 ? 4096 : 8192) ? 0
+      : __builtin_amdgcn_readfirstlane(
+            (blockIdx.x / 8 * 13 + blockIdx.x % 8 * 7) % 32 * chunks / 32);
+  auto chunk = [&](int i) __attribute__((always_inline)) {
+    const int c = wid + i * NW + turn;
+    return c < chunks ? c : c - chunks;
+  };
   auto load = [&](int d, int i) __attribute__((always_inline)) {
-    const int at = (wid + (EVEN ? min(i, mine - 1) : i) * NW) * CH;
+    const int at = chunk(EVEN ? min(i, mine - 1) : i) * CH;
 #pragma unroll
     for (int s = 0; s < S; ++s)
       w[d][s].load(a.w[layer + s / FT], row[s % FT] + at, g);
@@ -311,7 +324,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
         part = mfma(w[d][s].operand(k), x[d][k], part);
       if (I8) {     // of the rows 4 g + r that the lane holds the sums of
         const f32x4 sc = *(const f32x4*)(
-            scales + ((wid + i * NW) * S + s) * 16 + 4 * g);
+            scales + (chunk(i) * S + s) * 16 + 4 * g);
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[s][r] += part[r] * sc[r];
       } else {

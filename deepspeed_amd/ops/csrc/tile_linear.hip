@@ -67,6 +67,7 @@ struct Args {
   int step_end[MAXL];   // and GRAD_X: stages
   float* part;          // [splits, rows, columns] of all outputs, splits > 1
   int M, K, layers, tiles, mtiles, splits, steps;
+  bool turn;            // each workgroup begins elsewhere in its contraction
 };
 
 __device__ __forceinline__ f32x4 mfma(s16x8 a, s16x8 b, f32x4 c) {
@@ -223,6 +224,8 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
       : MODE == GRAD_W ? (a.M + BK - 1) / BK : K / BK;
   const int s0 = uni(split * steps / a.splits);
   const int n_it = uni((split + 1) * steps / a.splits) - s0;    // NS or more
+  const int turn = MODE > SWIGLU || !a.turn ? 0
+      : uni((blockIdx.x / 8 * 13 + blockIdx.x % 8 * 7) % 32 * n_it / 32);
 
   // The lane's place in each load, which fills 1 KB: 8 rows of 64 inputs, or
   // 8 inputs of 64 columns. Rows and columns past the end repeat the last ones;
@@ -273,6 +276,7 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
     const char* p = j < PW ? wb : xb;
     unsigned o = off[j];
     int step = s0 + it, ld = j < PW ? K : rows;
+    if (MODE <= SWIGLU) step += it + turn < n_it ? turn : turn - n_it;
     if (MODE == GRAD_X) {
       const int l = (step >= e0) + (step >= e1);
       step -= pick(l, 0, e0, e1);
@@ -1115,6 +1119,14 @@ int launch(Args a, bool merge, hipStream_t st) {
   constexpr int LDS = NS * (BM + BN) * ROW;
   static_assert(LDS <= 160 * 1024, "");
   const int items = count<BM, BN, MODE>(a);
+  // One tile of rows reads W once, nothing of it is shared: tiles that all begin at
+  // their rows' beginnings read the same few memory channels at a time where rows
+  // are whole multiples of 4 KB apart. Begun apart over an XCD and over the XCDs (us,
+  // before / now): 48 rows 16384, K 4096 31.5 / 25.2, 32000 60 / 47, 28672, K 8192 106 /
+  // 82, gate and up 14336, K 4096 54.9 / 42.6, 11008 43.0 / 36.5; 128 rows 128256 222 /
+  // 197, 32000 63 / 51; 224 rows 32000 73 / 69, gate and up 14336 65.2 / 64.4; even at
+  // K 3072, 4608 and 5120. Other steps than 13 and 7 leave 18432, K 4096 at 43 to 52.
+  a.turn = a.mtiles == 1 && a.splits == 1 && a.K * 2 % 4096 == 0;
   auto kernel = tile_linear_kernel<BM, BN, WM, WN, NS, MODE>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);

@@ -187,6 +187,21 @@ def test_widest_tile_goes_on_gpu(steps):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,ns,k,mode,tile", [
+    (40, (20000,), 2048, 0, 0), (33, (9000, 9000), 4096, SWIGLU, 1),
+    (100, (8200, 4100), 2048, 0, 3), (190, (16396,), 4096, 0, 6)])
+@torch.no_grad()
+def test_one_tile_of_rows_gpu(m, ns, k, mode, tile):
+    """Rows of whole multiples of 4 KB: every workgroup begins elsewhere in them,
+    and comes to all of them."""
+    from deepspeed_amd.ops import _C
+    x, ws, bs = _inputs(m, ns, k, m)
+    for y, want in zip(_C.tile_linear(x, ws, bs, mode, tile, 1),
+                       _want(x, ws, bs, mode)):
+        _close(y, want)
+
+
+@pytest.mark.gpu
 def test_what_lies_past_the_last_row_gpu():
     """Rows past the end count for nothing, whatever the last one holds: each
     value of the weight's gradient comes from its own column."""
