@@ -538,9 +538,9 @@ __device__ __forceinline__ void add_product(s16x8 a, s16x8 b) {
                :: "v"(a), "v"(b), "n"(R), "n"(R + 3));
 }
 template <int R>
-__device__ __forceinline__ void zero(s16x8 zeros) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 a[%1:%2], %0, %0, 0"
-               :: "v"(zeros), "n"(R), "n"(R + 3));
+__device__ __forceinline__ void first_product(s16x8 a, s16x8 b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, 0"
+               :: "v"(a), "v"(b), "n"(R), "n"(R + 3));
 }
 template <int R>
 __device__ __forceinline__ float sum() {
@@ -582,10 +582,13 @@ __device__ __forceinline__ unsigned packed2(float lo, float hi) {
 // that 16 lanes store 256 bytes of a row without a pass through LDS. The gradients,
 // whose W lies across, exchange halves between rows of 16 lanes.
 //
-// us, eight waves with a tile a workgroup, and now: 8192 x 8192 x 8192 786 / 735;
-// 4096 rows, K 4096: 28672 690 / 653, 6144 175 / 164, gate and up 14336 712 / 680;
-// gate and up 18944, K 3584, 2331 rows 517 / 497; dx of 14336, K 4096, 8192 rows 738 /
-// 685; dW of that 765 / 762 (its transposing reads are two an operand).
+//   * A tile's first products write its sums, those of no bias are stored as they
+// are, and outputs pass the caches by: 2 to 4%.
+//
+// us, eight waves with a tile a workgroup, and now: 8192 x 8192 x 8192 786 / 695;
+// 4096 rows, K 4096: 28672 690 / 632, 6144 175 / 159, gate and up 14336 712 / 665;
+// gate and up 18944, K 3584, 2331 rows 517 / 486; dx of 14336, K 4096, 8192 rows 738 /
+// 690; dW of that 765 / 735 (its transposing reads are two an operand).
 template <int MODE, bool PARTS>
 __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   constexpr bool GLU = MODE == SWIGLU;
@@ -848,13 +851,6 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   // sums of a tile of W and one of x
 #define acc(f, m) (((f) * F + (m)) * 4)
   take_sums();
-  auto clear = [&]() INLINE {
-    s16x8 zeros = {};
-    asm volatile("s_nop 4" : "+v"(zeros));    // written before it is multiplied
-    auto one = [&](auto i) INLINE { zero<decltype(i)::value * 4>(zeros); };
-    each(std::make_integer_sequence<int, F * F>{}, one);
-  };
-  clear();
 
   seek_w(at.n0, at.layer, at.s0, at.s0 + at.n_it);
   seek_x(at.m0, at.layer, at.s0, at.s0 + at.n_it);
@@ -875,67 +871,73 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   constexpr int N2 = 2 * F * F, BARRIER = 30;
   constexpr int STORES = 4 * F;     // of a tile, at least
   int young = 0;        // a tile's stores are behind the loads that are waited for
-  while (true) {
-#pragma clang loop unroll(disable)
-    for (int it = 0; it < at.n_it; ++it) {
-      __builtin_amdgcn_sched_barrier(0);
-      wait_reads();
-      aim(1);
-      auto product = [&](auto at) INLINE {
-        constexpr int i = decltype(at)::value, h = i / (F * F), m = i / F % F;
-        constexpr int f = m % 2 ? F - 1 - i % F : i % F;
-        if constexpr (i == BARRIER) {
+  auto stage = [&](auto first) INLINE {
+    constexpr bool FIRST = decltype(first)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    wait_reads();
+    aim(1);
+    auto product = [&](auto at) INLINE {
+      constexpr int i = decltype(at)::value, h = i / (F * F), m = i / F % F;
+      constexpr int f = m % 2 ? F - 1 - i % F : i % F;
+      if constexpr (i == BARRIER) {
+        if constexpr (FIRST)
           asm volatile("s_cmp_lg_u32 %0, 0\n\t"
                        "s_cbranch_scc1 1f\n\t"
                        "s_waitcnt vmcnt(%1)\n"
                        "1:\n\t"
                        "s_waitcnt vmcnt(%2)"
                        :: "s"(young), "n"(P), "n"(P + STORES) : "memory", "scc");
-          wait_reads();
-          __builtin_amdgcn_s_barrier();
-          wget = next_w(wget, 0);
-          xget ^= SX;
-          aim(0);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int q = 0; q < P; ++q) {
-          if (i == BARRIER + 2 + 6 * q) load_to(xput, q * 4096);
-          if (i == BARRIER + 52 + 6 * q) load_to(wput, q * 4096);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int q = 0; q < 2 * F; ++q) {
-          if (i == q * 3 / 2) get(q, 1);
-          if (i == 67 + 2 * q) get(q, 0);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        if (WT) add_product<acc(f, m)>(wa[h][f], xa[h][m]);
-        else add_product<acc(f, m)>(xa[h][m], wa[h][f]);
+        else
+          wait_loads<P>();
+        wait_reads();
+        __builtin_amdgcn_s_barrier();
+        wget = next_w(wget, 0);
+        xget ^= SX;
+        aim(0);
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int q = 0; q < P; ++q) {
-          if (i == BARRIER + 2 + 6 * q) load(xfrom, xoff[q], xsoff);
-          if (i == BARRIER + 52 + 6 * q) load(wfrom, woff[q], wsoff);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      };
-      each(std::make_integer_sequence<int, N2>{}, product);
-      young = 0;
-      xput = xput == put + XAT ? xput + SX : put + XAT;
-      wput = next_w(wput, put);
-      --wleft;
-      --xleft;
-      if (min(wleft, xleft) > 0) {
-        move_w();
-        move_x();
-      } else {
-        if (wleft == 0) turn_w();
-        else move_w();
-        if (xleft == 0) turn_x();
-        else move_x();
       }
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        if (i == BARRIER + 2 + 6 * q) load_to(xput, q * 4096);
+        if (i == BARRIER + 52 + 6 * q) load_to(wput, q * 4096);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int q = 0; q < 2 * F; ++q) {
+        if (i == q * 3 / 2) get(q, 1);
+        if (i == 66 + 3 * q) get(q, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const s16x8 u = WT ? wa[h][f] : xa[h][m], v = WT ? xa[h][m] : wa[h][f];
+      if constexpr (FIRST && h == 0) first_product<acc(f, m)>(u, v);
+      else add_product<acc(f, m)>(u, v);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        if (i == BARRIER + 2 + 6 * q) load(xfrom, xoff[q], xsoff);
+        if (i == BARRIER + 52 + 6 * q) load(wfrom, woff[q], wsoff);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    each(std::make_integer_sequence<int, N2>{}, product);
+    xput = xput == put + XAT ? xput + SX : put + XAT;
+    wput = next_w(wput, put);
+    --wleft;
+    --xleft;
+    if (min(wleft, xleft) > 0) {
+      move_w();
+      move_x();
+    } else {
+      if (wleft == 0) turn_w();
+      else move_w();
+      if (xleft == 0) turn_x();
+      else move_x();
     }
+  };
+  while (true) {
+    stage(Int<1>{});
+#pragma clang loop unroll(disable)
+    for (int it = 1; it < at.n_it; ++it) stage(Int<0>{});
 
     asm volatile("s_nop 15");     // the last products
     // Every store is made, past the tile's rows or columns to nowhere: the waits
@@ -975,6 +977,8 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       };
       each(std::make_integer_sequence<int, F * F>{}, store);
     } else {
+      // outputs pass the caches by, which hold what other tiles still read
+      constexpr int STREAM = 2;
       short* out = a.out[MODE == GRAD_X || GLU ? 0 : at.layer];
       const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(
           (void*)(out + (long long)m_of * N), (short)0,
@@ -995,13 +999,15 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
           const int n = n1 + 16 * f;
           __builtin_amdgcn_raw_buffer_store_b128(
               u32x4{lo[0], hi[0], lo[1], hi[1]}, to,
-              n < N ? (unsigned)((16 * m + col) * N + n) * 2 : NOWHERE, 0, 0);
+              n < N ? (unsigned)((16 * m + col) * N + n) * 2 : NOWHERE, 0, STREAM);
         };
         each(std::make_integer_sequence<int, F / 2 * F>{}, store);
       } else {
         constexpr int W = GLU ? F / 2 : F;      // features a lane
         const int n = at.n0 + wn * (GLU ? BN / 4 : BN / 2) + W * col;
         float b[GLU ? 2 : 1][W];
+        const bool biased = a.bias[GLU ? 0 : at.layer] || (GLU && a.bias[1]);
+        if (biased)
 #pragma unroll
         for (int l = 0; l < (GLU ? 2 : 1); ++l) {
           const short* bias = a.bias[GLU ? l : at.layer];   // of none: zeros
@@ -1013,38 +1019,42 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
                 from, (n + e) * 2, 0, 0));
         }
         typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-        auto store = [&](auto at) INLINE {
+        auto store = [&](auto bias, auto at) INLINE {
+          constexpr bool B = decltype(bias)::value;
           constexpr int m = decltype(at)::value / 4, r = decltype(at)::value % 4;
           const unsigned o =
               n < N ? (unsigned)((4 * g + 16 * m + r) * N + n) * 2 : NOWHERE;
           auto one = [&](auto at) INLINE {
             constexpr int e = decltype(at)::value;
             if constexpr (GLU) {
-              const float t = sum<acc(2 * e, m) + r>() + b[0][e];
+              const float t = sum<acc(2 * e, m) + r>() + (B ? b[0][e] : 0.f);
               return t / (1.f + expf(-t)) *
-                  (sum<acc(2 * e + 1, m) + r>() + b[GLU][e]);
+                  (sum<acc(2 * e + 1, m) + r>() + (B ? b[GLU][e] : 0.f));
             } else {
-              return sum<acc(e, m) + r>() + b[0][e];
+              return B ? sum<acc(e, m) + r>() + b[0][e] : sum<acc(e, m) + r>();
             }
           };
           const u32x2 v = {packed2(one(Int<0>{}), one(Int<1>{})),
                            packed2(one(Int<2>{}), one(Int<3>{}))};
           if constexpr (GLU)
-            __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, STREAM);
           else {
             const u32x2 u = {packed2(one(Int<4>{}), one(Int<5>{})),
                              packed2(one(Int<6>{}), one(Int<7>{}))};
             if (N % 8 == 0) {
               __builtin_amdgcn_raw_buffer_store_b128(u32x4{v[0], v[1], u[0], u[1]},
-                                                     to, o, 0, 0);
+                                                     to, o, 0, STREAM);
             } else {
-              __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, 0);
+              __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, STREAM);
               __builtin_amdgcn_raw_buffer_store_b64(
-                  u, to, n + 4 < N ? o + 8 : NOWHERE, 0, 0);
+                  u, to, n + 4 < N ? o + 8 : NOWHERE, 0, STREAM);
             }
           }
         };
-        each(std::make_integer_sequence<int, 4 * F>{}, store);
+        auto with = [&](auto at) INLINE { store(Int<1>{}, at); };
+        auto without = [&](auto at) INLINE { store(Int<0>{}, at); };
+        if (biased) each(std::make_integer_sequence<int, 4 * F>{}, with);
+        else each(std::make_integer_sequence<int, 4 * F>{}, without);
       }
     }
     if (!more) break;
@@ -1054,7 +1064,6 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
     if (more) next = locate(item + slots);
     wover = xover = false;
     young = 1;
-    clear();
   }
   wait_loads<0>();
 }
