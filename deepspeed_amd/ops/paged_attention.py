@@ -14,9 +14,19 @@ import torch
 
 from ._loader import get_ext
 
-# Workgroups wanted in flight: four waves each, two to three to a CU of 256.
-# More splits than that only add partial results to write and merge.
+# Workgroups wanted in flight where the lengths stay on the device: four waves each,
+# two to three to a CU of 256. More splits than that only add partial results to
+# write and merge.
 WORKGROUPS = 1024
+# Where they are known, splits fill whole rounds of the workgroups that the 256 CUs
+# hold, three each of one tile of columns: a few more would begin when the others end,
+# and read alone (us, 8 key heads, some 1024 of them / at most a round: 32 x 2000 59.6
+# / 55.8, 8 x 16000 108.1 / 98.2, 16 x 8000 107.8 / 98.9, 40 x 3000 100.9 / 94.2). Of two
+# tiles two each, two rounds (24 of 1000 and 200 rows 47.8 / 42.7, 29 of 2000 and 100
+# rows 68.0 / 64.5). With less than KEYS keys each, two a CU: the rest merges longer
+# than it reads (1 x 16000 27.0 / 21.1, 64 x 500 34.9 / 30.9, 15 of 200 and 250 rows
+# 23.9 / 19.5).
+ROUND, FEWER, KEYS = {1: 768, 2: 1024}, 512, 384
 # Keys of the shortest split: one tile of 32 for each of a workgroup's waves.
 MIN_SPLIT = 128
 # Items of 128 columns (rows times heads a key head), eight waves of them a CU,
@@ -140,11 +150,17 @@ class StepPlan:
                 while per < end[0] and (-(-end // per)).sum() > room:
                     per += MIN_SPLIT
             n = -(-end // per)
-        elif len(end) * kv_heads >= WORKGROUPS:
-            n = np.ones_like(end)
         else:
-            per = max(MIN_SPLIT, int(end.sum()) * kv_heads // WORKGROUPS)
+            total, full = int(end.sum()), ROUND[nq]
+            if total * kv_heads < KEYS * full:
+                full = FEWER
+            room = -(-len(end) * kv_heads // full) * full // kv_heads
+            # half a split more for each tile, where it ends unevenly
+            per = max(MIN_SPLIT, total // max(1, room - len(end) // 2))
             n = -(-end // per)
+            while n.sum() > max(room, len(end)):
+                per += per // 16
+                n = -(-end // per)
         step = -(-(-(-end // n)) // grain) * grain
         n = -(-end // step)
         of = np.repeat(np.arange(len(end)), n)

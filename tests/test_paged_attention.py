@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from deepspeed_amd.inference.ragged import PagedKVCache
+from deepspeed_amd.ops import paged_attention as plans
 from deepspeed_amd.ops.paged_attention import StepPlan
 
 # (slots with the new rows of each, kept tokens by slot)
@@ -27,6 +28,33 @@ def _rows(step, lens):
         pos += range(at[s], at[s] + m)
         at[s] += m
     return slots, np.array(pos), at
+
+
+@pytest.mark.parametrize("lens,rows,kv_heads", [
+    ([1], 1, 8), ([127] * 3, 1, 8), ([16000], 1, 8), ([16000] * 8, 1, 8),
+    (range(1000, 3000, 63), 1, 8), ([2000] * 97, 1, 8), ([900] * 33, 1, 32),
+    ([2000] * 24, 200, 8), ([200] * 15, 250, 8), ([30000] * 2, 7, 1)])
+def test_splits_fill_whole_rounds(lens, rows, kv_heads):
+    """Decoding requests beside a run of more rows: no more workgroups than whole
+    rounds of those that the CUs hold, or than there are tiles; every key once."""
+    lens = list(lens)
+    slots = list(range(len(lens))) + [len(lens)] * (rows - 1)
+    pos = np.array([*lens, *range(rows - 1)])
+    tables = {s: list(range(500)) for s in range(len(lens) + 1)}
+    plan = StepPlan.build(slots, pos, tables, 64, 4 * kv_heads, kv_heads, "cpu")
+    meta = plan.meta.numpy()
+    items = meta[:4 * plan.items].reshape(-1, 4)
+    merges = meta[4 * (plan.items + plan.runs):][:2 * plan.merges].reshape(-1, 2)
+    tiles = -(-plan.merges * kv_heads // plans.ROUND[plan.nq])
+    assert plan.items * kv_heads <= tiles * plans.ROUND[plan.nq] or \
+        plan.items == plan.merges
+    for first, n in merges:
+        at = 0
+        for it in items[first:first + n]:
+            assert it[2] == at < abs(it[3])
+            at = abs(it[3])
+    assert {int(abs(items[f + n - 1][3])) for f, n in merges} >= \
+        {n + 1 for n in lens}
 
 
 @pytest.mark.parametrize("name", list(STEPS))
