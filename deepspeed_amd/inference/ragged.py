@@ -472,8 +472,9 @@ class PagedKVCache:
             assert q_len == 1, "packed mode is per-token (q_len 1)"
             starts = starts + torch.as_tensor(offsets,
                                               device=self.lens.device)
-        L = int((starts + q_len).max())
-        for s, st in zip(self._slots, starts.tolist()):
+        at = starts.tolist()
+        L = max(at) + q_len
+        for s, st in zip(self._slots, at):
             self._ensure_blocks(s, st + q_len)
         self._L = L
         self._starts = starts
@@ -503,7 +504,8 @@ class PagedKVCache:
         """Slot and position of every row of the step, in order."""
         n = self._q_len
         starts = self._starts.cpu()       # wherever the lengths are kept
-        pos = (starts[:, None] + torch.arange(n)).reshape(-1).numpy()
+        pos = starts.numpy() if n == 1 else \
+            (starts[:, None] + torch.arange(n)).reshape(-1).numpy()
         slots = self._slots if n == 1 else \
             [s for s in self._slots for _ in range(n)]
         return slots, pos

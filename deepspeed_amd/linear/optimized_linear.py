@@ -62,12 +62,14 @@ class WOQLinear(nn.Module):
     def int8_rows(self, K: int):
         """(int8 weight, scales, group size) of a weight [N, K] as it was
         quantized; None where it is another."""
-        p = self.qweight
+        p = self._modules.get("qweight")
         if type(p) is not QuantizedParameter or "dequantized" in p.__dict__ \
-                or p.cfg.q_bits != 8 or p.shape[1:] != (K,) or \
-                p.q.numel() != p.shape[0] * K:
+                or p.cfg.q_bits != 8 or p.shape[1:] != (K,):
             return None
-        return p.q, p.scales, p.cfg.group_size
+        q, scales = p._buffers.get("q"), p._buffers.get("scales")
+        if q is None or scales is None or q.numel() != p.shape[0] * K:
+            return None
+        return q, scales, p.cfg.group_size
 
     def forward(self, x):
         y = rows_linear(x, (self,), hooks_ran=True)

@@ -21,8 +21,8 @@ from ..ops import linear as _linear
 from ..ops._loader import get_ext
 from ..ops.attention import rope_flash_attention
 from ..ops.embedding import Embedding
-from ..ops.linear import (SWIGLU, Linear, call, movable, rows_linear,
-                          tile_linear, unhooked)
+from ..ops.linear import (SWIGLU, Linear, all_unhooked, call, movable,
+                          rows_linear, tile_linear, unhooked)
 from ..ops.norms import RMSNorm
 from ..ops.rope import apply_rope, rope_tables
 from ..ops.swiglu import swiglu
@@ -299,6 +299,10 @@ class LlamaDecoderLayer(nn.Module):
 _CHAIN, _OUT = LlamaDecoderLayer.chain, LlamaAttention._out
 
 
+_ATTN = "q_proj", "k_proj", "v_proj", "o_proj"
+_MLP = "gate_proj", "up_proj", "down_proj"
+
+
 def _operands(layer, rows: int):
     """What a decoder layer brings to ``paged_decoder_layer``, or None where its
     modules are to be called: (norm weights, their eps, linear weights, scales,
@@ -309,51 +313,40 @@ def _operands(layer, rows: int):
             "chain" in layer.__dict__ or "_out" in attn.__dict__ or \
             attn.head_dim != 128:
         return None
-    norms = layer.input_layernorm, layer.post_attention_layernorm
-    H = attn.num_heads * 128
-    weights, scales, biases, group = [], [], [], 0
-    for norm in norms:
-        if type(norm) is not RMSNorm or not unhooked(norm):
-            return None
-        w = norm.weight
-        if w.dtype is not torch.bfloat16 or not w.is_contiguous():
-            return None
-    mods = (attn.q_proj, attn.k_proj, attn.v_proj, attn.o_proj, mlp.gate_proj,
-            mlp.up_proj, mlp.down_proj)
+    H, parts = attn.num_heads * 128, layer._modules
+    norms = parts.get("input_layernorm"), parts.get("post_attention_layernorm")
+    mods = [attn._modules.get(name) for name in _ATTN]
+    mods += [mlp._modules.get(name) for name in _MLP]
     kind = type(mods[0])
-    K = H
-    for m in mods:
-        if type(m) is not kind or not unhooked(m):
+    if type(norms[0]) is not RMSNorm or type(norms[1]) is not RMSNorm or \
+            any(type(m) is not kind for m in mods):
+        return None
+    scales, group = [], 0
+    if kind is Linear or kind is nn.Linear:
+        weights = [m._parameters.get("weight") for m in mods]
+        if any(type(w) is not nn.Parameter for w in weights):
             return None
-        if m is mods[6]:
-            K = n
-        if kind is Linear or kind is nn.Linear:
-            w = m.weight
-            if type(w) is not nn.Parameter or \
-                    w.dtype is not torch.bfloat16 or w.dim() != 2 or \
-                    w.shape[1] != K:
-                return None
-        elif hasattr(kind, "int8_rows"):
-            p = m.int8_rows(K) if rows <= _linear.ROWS_INT8 else None
+    elif hasattr(kind, "int8_rows") and rows <= _linear.ROWS_INT8:
+        weights = []
+        for m in mods:
+            p = m.int8_rows(H if len(weights) < 6 else
+                            weights[5].numel() // H)
             if p is None or p[2] % 256 or group not in (0, p[2]):
                 return None
-            w, scale, group = p
-            scales.append(scale)
-        else:
-            return None
-        n, b = w.numel() // K, m.bias
-        if K % 256 or n % 4 or not w.is_contiguous() or w.data_ptr() % 16 or (
-                b is not None and (b.dtype is not torch.bfloat16
-                                   or not b.is_contiguous())):
-            return None
-        weights.append(w)
-        biases.append(b)
-    n = [w.numel() // H for w in weights[:6]]
-    if n != [H, attn.num_kv_heads * 128, n[1], H, n[4], n[4]] or \
-            weights[6].numel() != H * n[4]:
+            group = p[2]
+            weights.append(p[0])
+            scales.append(p[1])
+    else:
         return None
-    return ([norms[0].weight, norms[1].weight], norms[0].eps, norms[1].eps,
-            weights, scales, biases, group)
+    if not all_unhooked((attn, mlp, *norms, *mods)):
+        return None
+    biases = [m._parameters["bias"] if "bias" in m._parameters else m.bias
+              for m in mods]
+    scaled = [n._parameters.get("weight") for n in norms]
+    if any(w is None for w in scaled) or not get_ext().paged_layer_fits(
+            scaled, weights, scales, biases, H, attn.num_kv_heads * 128):
+        return None
+    return (scaled, norms[0].eps, norms[1].eps, weights, scales, biases, group)
 
 
 def _plain(x) -> bool:

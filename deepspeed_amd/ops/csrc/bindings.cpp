@@ -3,10 +3,18 @@
 // Uses torch-ROCm's native HIP stream API (c10::hip) — no CUDA shims.
 
 #include <torch/extension.h>
+#include <pybind11/numpy.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
 #include <tuple>
+
+std::tuple<at::Tensor, int64_t, int64_t, int64_t, bool, int64_t, int64_t>
+step_plan(const pybind11::sequence& slots,
+          pybind11::array_t<int64_t, pybind11::array::c_style |
+                                         pybind11::array::forcecast> pos,
+          const pybind11::object& tables, int64_t block_size, int64_t heads,
+          int64_t kv_heads, const std::vector<int64_t>& lines, bool pinned);
 
 extern "C" void ds_fused_adam_flat(float* p, const void* g, int grad_dtype,
                                    float* m, float* v, void* p16, long long n,
@@ -1046,6 +1054,36 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
           h.scalar_type() == at::kFloat ? h : h.view(x.sizes())};
 }
 
+// What paged_decoder_layer asks of a layer's tensors, H wide, with kv features of
+// keys; int8 weights have scales, and are as large as their modules say. Looked at
+// one by one in Python, with their modules, they took 36 us of a layer's host time;
+// the modules alone take 15.
+bool paged_layer_fits(const std::vector<at::Tensor>& norms,
+                      const std::vector<at::Tensor>& weights,
+                      const std::vector<at::Tensor>& scales,
+                      const std::vector<c10::optional<at::Tensor>>& biases,
+                      int64_t H, int64_t kv) {
+  auto plain = [](const at::Tensor& t) {
+    return t.scalar_type() == at::kBFloat16 && t.is_contiguous();
+  };
+  if (weights.size() != 7 || biases.size() != 7 || H < 256 || H % 256)
+    return false;
+  for (auto& w : norms)
+    if (!plain(w)) return false;
+  const int64_t F = weights[4].numel() / H;
+  const int64_t N[] = {H, kv, kv, H, F, F, H};
+  for (int i = 0; i < 7; ++i) {
+    const auto& w = weights[i];
+    const int64_t K = i == 6 ? F : H;
+    if (K % 256 || N[i] % 4 || !N[i] || w.numel() != N[i] * K ||
+        !w.is_contiguous() || (uintptr_t)w.data_ptr() % 16 ||
+        (scales.empty() && (!plain(w) || w.dim() != 2 || w.size(1) != K)) ||
+        (biases[i].has_value() && !plain(*biases[i])))
+      return false;
+  }
+  return true;
+}
+
 // Gradient [V, H] of an embedding's table for tokens ids [T] with the gradients
 // grad [T, H] bf16; rows of `padding` (-1: none) get nothing. `into` is zero.
 at::Tensor embedding_bwd(at::Tensor ids, at::Tensor grad, int64_t V,
@@ -1463,6 +1501,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         pybind11::arg("into") = c10::nullopt);
   m.def("paged_decoder_layer", &paged_decoder_layer,
         "a decoder layer of a serving step over the paged pool");
+  m.def("paged_layer_fits", &paged_layer_fits,
+        "whether paged_decoder_layer takes a layer's tensors");
+  m.def("step_plan", &step_plan, "plan of a serving step over the paged pool");
   m.def("add_norm_fwd", &add_norm_fwd, "RMS norm of a sum, and the sum");
   m.def("rope", &rope, "Rotary position embedding of one or two tensors",
         pybind11::arg("x"), pybind11::arg("x2"), pybind11::arg("cos"),

@@ -433,6 +433,28 @@ def call(mod: nn.Module, x):
     return mod(x)
 
 
+def _watched() -> bool:
+    return bool(nn.Linear.forward is not _TORCHS
+                or _module._global_forward_hooks
+                or _module._global_forward_pre_hooks
+                or _module._global_backward_hooks
+                or _module._global_backward_pre_hooks)
+
+
+def all_unhooked(mods) -> bool:
+    """``unhooked`` of each of them."""
+    if _watched():
+        return False
+    for mod in mods:
+        cls = type(mod)
+        if "forward" in mod.__dict__ or mod._compiled_call_impl is not None or \
+                cls.forward is not _FORWARD.get(cls) or \
+                mod._forward_hooks or mod._forward_pre_hooks or \
+                mod._backward_hooks or mod._backward_pre_hooks:
+            return False
+    return True
+
+
 def unhooked(mod: nn.Module, internal_ok: bool = False) -> bool:
     """No hook sees the module's call and no other forward takes it (one set on
     the module or on its class, or a compiled one): its work may move
@@ -440,12 +462,7 @@ def unhooked(mod: nn.Module, internal_ok: bool = False) -> bool:
     the framework's own hooks (marked ``_ds_internal``) take as well."""
     cls = type(mod)
     if "forward" in mod.__dict__ or mod._compiled_call_impl is not None or \
-            cls.forward is not _FORWARD.get(cls) or \
-            nn.Linear.forward is not _TORCHS or \
-            _module._global_forward_hooks or \
-            _module._global_forward_pre_hooks or \
-            _module._global_backward_hooks or \
-            _module._global_backward_pre_hooks:
+            cls.forward is not _FORWARD.get(cls) or _watched():
         return False
     if not (mod._forward_hooks or mod._forward_pre_hooks
             or mod._backward_hooks or mod._backward_pre_hooks):

@@ -12,6 +12,7 @@ from typing import List, Optional
 import numpy as np
 import torch
 
+from . import _loader
 from ._loader import get_ext
 
 # Workgroups wanted in flight where the lengths stay on the device: four waves each,
@@ -70,16 +71,6 @@ def paged_decode_attention(q: torch.Tensor, kpool: torch.Tensor,
                             lens.contiguous().int(), splits, scale)
 
 
-def _to_device(values: np.ndarray, device) -> torch.Tensor:
-    """As int32, in the order of the device's current stream. From pageable memory
-    the host would wait there for all that the stream still has to do, the whole
-    step before; torch gives the pinned block to nobody else before it is read."""
-    pinned = torch.device(device).type == "cuda"
-    out = torch.empty(len(values), dtype=torch.int32, pin_memory=pinned)
-    out.numpy()[:] = values
-    return out.to(device, non_blocking=pinned)
-
-
 @dataclass
 class StepPlan:
     """One serving step for the kernels: where each new row goes (``dst``) and
@@ -116,67 +107,81 @@ class StepPlan:
         """``slots[i]`` and ``pos[i]``: request slot and position of row i.
         Neighbouring rows of one slot at following positions form a run and
         share the reads of its keys and values."""
-        T = len(slots)
-        dst, flat, offs = cls.rows(slots, pos, tables, block_size)
-        sl = np.asarray(slots)
-        cut = np.flatnonzero((sl[1:] != sl[:-1]) | (pos[1:] != pos[:-1] + 1))
-        row0 = np.concatenate(([0], cut + 1))
-        m = np.diff(np.append(row0, T))
-        kv_len = pos[row0] + m
-        runs = np.stack([row0, m, kv_len, offs[row0]], 1)
-        G = heads // kv_heads
-        # two tiles of 16 columns share the loads of a key tile where runs are
-        # long enough, eight where they are longer
-        nq = 2 if int(m.max()) * G > 16 else 1
-        if int(m.min()) * G >= BLOCK and kv_heads * G * int(
-                (m * (kv_len - m // 2)).sum()) >= BLOCK_WORK:
-            nq = 8
-        width = 16 * nq
-        tiles = -(-m * G // width)
-        run_of = np.repeat(np.arange(len(m)), tiles)
-        tile = np.arange(len(run_of)) - np.repeat(np.cumsum(tiles) - tiles,
-                                                  tiles)
-        tok = np.minimum((tile + 1) * width, m[run_of] * G) - 1
-        end = kv_len[run_of] - m[run_of] + tok // G + 1
-        # split long histories until the chip is full
-        grain = 32
-        if nq == 8:
-            # the longest first; at most one round of workgroups, steps of 128
-            order = np.argsort(-end, kind="stable")
-            run_of, tile, end = run_of[order], tile[order], end[order]
-            room, per, grain = CUS // kv_heads, int(end[0]), MIN_SPLIT
-            if len(end) < room:
-                per = max(MIN_SPLIT, int(end.sum()) // room)
-                while per < end[0] and (-(-end // per)).sum() > room:
-                    per += MIN_SPLIT
+        ext = _loader.get_ext()
+        args = slots, pos, tables, block_size, heads, kv_heads
+        values, items, runs, merges, any_merge, nq, head = _planned(*args) \
+            if ext is None else ext.step_plan(
+                *args, [ROUND[1], ROUND[2], FEWER, KEYS, MIN_SPLIT, BLOCK,
+                        BLOCK_WORK, CUS], torch.device(device).type == "cuda")
+        # in the order of the current stream; from pageable memory the host would
+        # wait there for all that the stream still has to do, the whole step before
+        # (torch gives the pinned block to nobody else before it is read)
+        meta = values.to(device, non_blocking=True)
+        return cls(dst=meta[head:], meta=meta, items=items, runs=runs,
+                   merges=merges, any_merge=any_merge, nq=nq)
+
+
+def _planned(slots, pos, tables, block_size: int, heads: int, kv_heads: int):
+    """``step_plan`` of csrc/step_plan.cpp, for a host without the extension."""
+    T = len(slots)
+    dst, flat, offs = StepPlan.rows(slots, pos, tables, block_size)
+    sl = np.asarray(slots)
+    cut = np.flatnonzero((sl[1:] != sl[:-1]) | (pos[1:] != pos[:-1] + 1))
+    row0 = np.concatenate(([0], cut + 1))
+    m = np.diff(np.append(row0, T))
+    kv_len = pos[row0] + m
+    runs = np.stack([row0, m, kv_len, offs[row0]], 1)
+    G = heads // kv_heads
+    # two tiles of 16 columns share the loads of a key tile where runs are
+    # long enough, eight where they are longer
+    nq = 2 if int(m.max()) * G > 16 else 1
+    if int(m.min()) * G >= BLOCK and kv_heads * G * int(
+            (m * (kv_len - m // 2)).sum()) >= BLOCK_WORK:
+        nq = 8
+    width = 16 * nq
+    tiles = -(-m * G // width)
+    run_of = np.repeat(np.arange(len(m)), tiles)
+    tile = np.arange(len(run_of)) - np.repeat(np.cumsum(tiles) - tiles,
+                                              tiles)
+    tok = np.minimum((tile + 1) * width, m[run_of] * G) - 1
+    end = kv_len[run_of] - m[run_of] + tok // G + 1
+    # split long histories until the chip is full
+    grain = 32
+    if nq == 8:
+        # the longest first; at most one round of workgroups, steps of 128
+        order = np.argsort(-end, kind="stable")
+        run_of, tile, end = run_of[order], tile[order], end[order]
+        room, per, grain = CUS // kv_heads, int(end[0]), MIN_SPLIT
+        if len(end) < room:
+            per = max(MIN_SPLIT, int(end.sum()) // room)
+            while per < end[0] and (-(-end // per)).sum() > room:
+                per += MIN_SPLIT
+        n = -(-end // per)
+    else:
+        total, full = int(end.sum()), ROUND[nq]
+        if total * kv_heads < KEYS * full:
+            full = FEWER
+        room = -(-len(end) * kv_heads // full) * full // kv_heads
+        # half a split more for each tile, where it ends unevenly
+        per = max(MIN_SPLIT, total // max(1, room - len(end) // 2))
+        n = -(-end // per)
+        while n.sum() > max(room, len(end)):
+            per += per // 16
             n = -(-end // per)
-        else:
-            total, full = int(end.sum()), ROUND[nq]
-            if total * kv_heads < KEYS * full:
-                full = FEWER
-            room = -(-len(end) * kv_heads // full) * full // kv_heads
-            # half a split more for each tile, where it ends unevenly
-            per = max(MIN_SPLIT, total // max(1, room - len(end) // 2))
-            n = -(-end // per)
-            while n.sum() > max(room, len(end)):
-                per += per // 16
-                n = -(-end // per)
-        step = -(-(-(-end // n)) // grain) * grain
-        n = -(-end // step)
-        of = np.repeat(np.arange(len(end)), n)
-        first = np.cumsum(n) - n
-        part = np.arange(len(of)) - first[of]
-        lo = part * step[of]
-        hi = np.minimum(lo + step[of], end[of])
-        hi = np.where(n[of] == 1, -hi, hi)
-        items = np.stack([run_of[of], tile[of], lo, hi], 1)
-        merges = np.stack([first, n], 1)
-        head = 4 * len(items) + 4 * len(runs) + 2 * len(merges) + len(flat)
-        both = _to_device(np.concatenate(
-            [items.ravel(), runs.ravel(), merges.ravel(), flat, dst]), device)
-        return cls(dst=both[head:], meta=both, items=len(items),
-                   runs=len(runs), merges=len(merges),
-                   any_merge=bool((n > 1).any()), nq=nq)
+    step = -(-(-(-end // n)) // grain) * grain
+    n = -(-end // step)
+    of = np.repeat(np.arange(len(end)), n)
+    first = np.cumsum(n) - n
+    part = np.arange(len(of)) - first[of]
+    lo = part * step[of]
+    hi = np.minimum(lo + step[of], end[of])
+    hi = np.where(n[of] == 1, -hi, hi)
+    items = np.stack([run_of[of], tile[of], lo, hi], 1)
+    merges = np.stack([first, n], 1)
+    meta = np.concatenate([items.ravel(), runs.ravel(), merges.ravel(), flat,
+                           dst])
+    return torch.from_numpy(meta.astype(np.int32)), len(items), len(runs), \
+        len(merges), bool((n > 1).any()), nq, len(meta) - T
 
 
 def paged_append(plan: StepPlan, q, k, v, kpool, vpool, cos=None, sin=None,

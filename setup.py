@@ -23,6 +23,7 @@ ext = CUDAExtension(
         os.path.join(CSRC, "cpu_adam.cpp"),
         os.path.join(CSRC, "aio.cpp"),
         os.path.join(CSRC, "shm_comm.cpp"),
+        os.path.join(CSRC, "step_plan.cpp"),
         os.path.join(CSRC, "adam.hip"),
         os.path.join(CSRC, "optim.hip"),
         os.path.join(CSRC, "grad_norm.hip"),

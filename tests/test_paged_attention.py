@@ -57,6 +57,43 @@ def test_splits_fill_whole_rounds(lens, rows, kv_heads):
         {n + 1 for n in lens}
 
 
+@pytest.mark.parametrize("heads", [(8, 8), (14, 2), (32, 8), (16, 1)])
+def test_step_plan_equals_numpys(heads):
+    """Single rows and runs of every length, slots that come again, tables of any
+    kind, ties in length and long histories; what is no step is refused."""
+    rng = np.random.default_rng(0)
+    seen = set()
+    for case in range(200):
+        bs = int(rng.choice([1, 16, 24, 64]))
+        slots, pos, ends = [], [], {}
+        for _ in range(rng.integers(1, 40)):
+            s = int(rng.integers(0, 30))
+            n = int(rng.choice([1, 1, 2, 17, 64, 300]))
+            at = int(rng.choice([0, 5, 130, 500, 500, 4000]))
+            slots += [s] * n
+            pos += range(at, at + n)
+            ends[s] = max(ends.get(s, 0), at + n)
+        if case % 5 == 0:       # long runs only: tiles of 128 columns
+            slots, pos = [0] * 300 + [1] * 70, [*range(900, 1200), *range(70)]
+            pos[300:] = [p + 13 * case for p in pos[300:]]
+            ends = {0: 1200, 1: 70 + 13 * case}
+        tables = {s: rng.integers(0, 1000, -(-n // bs)) for s, n in ends.items()}
+        if case % 2:
+            tables = {s: t.tolist() for s, t in tables.items()}
+        args = slots, np.array(pos), tables, bs, *heads
+        want, items, runs, merges, any_merge, nq, head = plans._planned(*args)
+        plan = StepPlan.build(*args, "cpu")
+        assert torch.equal(plan.meta, want) and torch.equal(plan.dst, want[head:])
+        assert (plan.items, plan.runs, plan.merges, plan.any_merge, plan.nq) == \
+            (items, runs, merges, any_merge, nq)
+        seen.add(nq)
+    assert seen >= {2, 8}
+    for slots, pos in (([], []), ([0], [64]), ([0, 1], [1]), ([0], [-1])):
+        with pytest.raises((ValueError, IndexError)):
+            StepPlan.build(slots, np.array(pos, np.int64), {0: [3], 1: []}, 64, 8,
+                           8, "cpu")
+
+
 @pytest.mark.parametrize("name", list(STEPS))
 @pytest.mark.parametrize("bs", [16, 24, 64])
 @pytest.mark.parametrize("heads", [(8, 8), (14, 2), (32, 8)])
