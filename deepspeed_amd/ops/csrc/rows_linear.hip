@@ -19,7 +19,8 @@
 // up 14336, K 4096 bf16 50.7 / 45.8, int8 36.6 / 32.8; q, k, v 4096 + 2 x 1024,
 // K 4096 16.0 / 13.3 and 12.2 / 10.8; N 128256 199 / 192 and 140 / 121; N 4096,
 // K 14336 27.7 / 27.3 and 19.7 / 18.9; N 4096, K 4096 10.2 / 10.1 and 8.2 / 8.6.
-// Three to six chunks ahead gained nothing more.
+// Three to six chunks ahead gained nothing more. Most layers of K 2048 to 4096 go
+// on to going_rows_kernel, which was measured against this.
 //   * More rows, rows_linear_kernel: bound by x out of L2. Only int8 weights, small
 // layers and numbers of features that tile_linear.hip does not take come here.
 //   * int8: a lane's 16 bytes are 16 inputs, split over two products; the order
@@ -371,6 +372,193 @@ __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
   }
 }
 
+// The same over contractions of X chunks a wave, for which x stays in registers: one
+// workgroup a CU that goes on from tile to tile, with all chunks of the next tile on
+// their way while this one's are multiplied and added up (sums and int8's scales
+// have two places in LDS, and a tile one barrier). Reading x again for each tile
+// takes the more of the time the more rows there are, and first loads and the last
+// round's end are a quarter of a workgroup's life that reads one tile. As many
+// workgroups as fill every round alike. us, few_rows_kernel / here, at 1, 8 and 16
+// rows: gate and up 14336, K 4096 bf16 44.0 / 40.9, 46.0 / 42.1, 51.1 / 43.9, int8 at 8
+// and 16 30.6 / 28.1, 35.4 / 29.7; 128256, K 4096 bf16 163 / 164, 186 / 174, 208 /
+// 181, int8 96 / 87, 112 / 92, 134 / 99; 9216, K 3072 bf16 14.3 / 12.8, 16.7 / 13.6, 18.2
+// (12 rows) / 14.2. Now 5.2 to 6.3 TB/s of W where it is large.
+template <bool I8, int MODE, int FT, int X>
+__global__ __launch_bounds__(NW * 64, 2) void going_rows_kernel(const Args a,
+                                                                int tiles) {
+  constexpr int L = MODE == SWIGLU ? 2 : 1;   // weight streams a workgroup
+  constexpr int S = L * FT;                   // tiles of 16 features a wave
+  constexpr int C = X * NW, R = I8 ? (C * S * 16 + NW * 64 - 1) / (NW * 64) : 1;
+  __shared__ float sums[2][NW * S * 256];
+  __shared__ __attribute__((aligned(16)))
+  float scales[I8 ? 2 : 1][I8 ? C * S * 16 : 4];
+
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int turn = !I8 || a.K % 4096 ? 0      // as above
+      : __builtin_amdgcn_readfirstlane(
+            (blockIdx.x / 8 * 13 + blockIdx.x % 8 * 7) % 32 * C / 32);
+  auto chunk = [&](int i) __attribute__((always_inline)) {
+    const int c = wid + i * NW + turn;
+    return c < C ? c : c - C;
+  };
+  struct Place { int layer, n0; };
+  auto locate = [&](int tile) __attribute__((always_inline)) {
+    int l = 0;
+    if (MODE == PLAIN) {
+      while (tile >= a.tile_end[l]) ++l;
+      if (l) tile -= a.tile_end[l - 1];
+    }
+    return Place{l, tile * 16 * FT};
+  };
+  int tile = blockIdx.x;
+  Place at = locate(tile);
+  Weights<I8> w[X][S];
+  long long row[FT];
+  Place from = at;
+  auto rows_of = [&](Place p) __attribute__((always_inline)) {
+    from = p;
+#pragma unroll
+    for (int f = 0; f < FT; ++f)
+      row[f] = (long long)min(p.n0 + 16 * f + col, a.n[p.layer] - 1) * a.K;
+  };
+  auto load = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      w[i][s].load(a.w[from.layer + s / FT], row[s % FT] + chunk(i) * CH, g);
+  };
+  // int8's scales of a tile [chunks][S][16], by way of registers
+  float sc[R];
+  auto load_scales = [&](Place p) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int e = min((int)threadIdx.x + r * NW * 64, C * S * 16 - 1);
+      const int c = e / (S * 16), f = e % (S * 16);
+      const long long n = min(p.n0 + f % (16 * FT), a.n[p.layer] - 1);
+      sc[r] = a.scales[p.layer + f / (16 * FT)][(n * a.K + c * CH) / a.group];
+    }
+  };
+  auto put_scales = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int e = threadIdx.x + r * NW * 64;
+      if (e < C * S * 16) scales[I8 ? b : 0][e] = sc[r];
+    }
+  };
+  if (I8) load_scales(at);
+  rows_of(at);
+#pragma unroll
+  for (int i = 0; i < X; ++i) load(i);
+  s16x8 x[X][CH / 32];
+  const short* xp = a.x + (long long)min(col, a.M - 1) * a.K;
+#pragma unroll
+  for (int i = 0; i < X; ++i)
+#pragma unroll
+    for (int k = 0; k < CH / 32; ++k)
+      x[i][k] = *(const s16x8*)(xp + chunk(i) * CH + input_at<I8>(k, g));
+  if (I8) {
+    put_scales(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+  int b = 0;
+  while (true) {
+    const int then = tile + gridDim.x;
+    const bool more = then < tiles;
+    const Place next = more ? locate(then) : at;
+    if (I8 && more) load_scales(next);
+    f32x4 acc[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < X; ++i) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        f32x4 part = I8 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[s];
+#pragma unroll
+        for (int k = 0; k < CH / 32; ++k)
+          part = mfma(w[i][s].operand(k), x[i][k], part);
+        if (I8) {     // of the rows 4 g + r that the lane holds the sums of
+          const f32x4 v = *(const f32x4*)(
+              &scales[I8 ? b : 0][(chunk(i) * S + s) * 16 + 4 * g]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[s][r] += part[r] * v[r];
+        } else {
+          acc[s] = part;
+        }
+      }
+      if (i == 0) rows_of(next);
+      if (more) load(i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    float* const sum = sums[b];
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+      *(f32x4*)(sum + (wid * S + s) * 256 + col * 16 + 4 * g) = acc[s];
+    if (I8 && more) put_scales(b ^ 1);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const int N = a.n[at.layer];
+    for (int e = threadIdx.x; e < FT * 256; e += NW * 64) {
+      const int f = e >> 8, o_ = e & 255;
+      const int r = o_ >> 4, n = at.n0 + 16 * f + (o_ & 15);
+      if (r >= a.M || n >= N) continue;
+      float y[L];
+#pragma unroll
+      for (int s = 0; s < L; ++s) {
+        float t = 0.f;
+#pragma unroll
+        for (int w_ = 0; w_ < NW; ++w_)
+          t += sum[(w_ * S + s * FT + f) * 256 + o_];
+        if (a.bias[at.layer + s]) t += value(a.bias[at.layer + s][n]);
+        y[s] = t;
+      }
+      float o = y[0];
+      if (MODE == SWIGLU) o = y[0] / (1.f + expf(-y[0])) * y[L - 1];
+      a.out[at.layer][(long long)r * N + n] = bits(o);
+    }
+    if (!more) break;
+    tile = then;
+    at = next;
+    b ^= 1;
+  }
+}
+
+template <bool I8, int MODE, int X>
+int launch_going(Args a, int layers, hipStream_t st) {
+  constexpr int FT = I8 && MODE == PLAIN ? 2 : 1, CUS = 256;
+  int tiles = 0;
+  for (int i = 0; i < (MODE == SWIGLU ? 1 : layers); ++i)
+    a.tile_end[i] = tiles += (a.n[i] + 16 * FT - 1) / (16 * FT);
+  const int rounds = (tiles + CUS - 1) / CUS;
+  hipLaunchKernelGGL((going_rows_kernel<I8, MODE, FT, X>),
+                     dim3((tiles + rounds - 1) / rounds), dim3(NW * 64), 0, st,
+                     a, tiles);
+  return (int)hipGetLastError();
+}
+
+// Where they go on, for tiles of 16 features (us, few_rows_kernel / going on, K 4096
+// unless said): not a single round (bf16 4096 of 1 row 8.8 / 8.9, int8 6.9 / 9.1). Gates
+// whose rounds are whole from 9 rows on only (8192 of 1 row 25.2 / 25.9, 12288 35.1 /
+// 36.0, of 16 rows 29.1 / 27.9; 8448 of 1 row 31.6 / 28.3), int8's from 5 on unless
+// they are short (14336, K 3072 of 1 row 20.6 / 21.8, of 8 24.2 / 22.7; K 2048 of 1
+// 15.7 / 14.8). bf16 of one or two rows up to 4096 tiles (50304 67.9 / 65.9, 128256 163
+// / 164, K 3072 123 / 125). int8 of up to four rows not where the last round, of
+// tiles of 32, is filled (13824, K 3072 11.9 / 12.2, 16384 15.2 / 16.0; 12288 14.6 /
+// 14.1, 16640 20.2 / 18.7).
+// K 2048 bf16, where a wave has two chunks on their way, stays (14336 x 2 of 1 row
+// 23.9 / 26.4, 32000 of 8 25.2 / 27.2), as do 5 and more chunks a wave, for which the
+// registers do not reach, and contractions that are not whole chunks of eight waves.
+template <bool I8>
+bool goes_on(const Args& a, int mode, int tiles) {
+  const int X = a.K % (CH * NW) ? 0 : a.K / (CH * NW), pairs = tiles / 2;
+  if (X < (I8 ? 2 : 3) || X > 4) return false;
+  if (mode == SWIGLU)
+    return pairs > 256 && (a.M > 8 || pairs % 256) &&
+           (!I8 || a.M > 4 || X == 2);
+  if (!I8) return tiles > 256 && (a.M > 2 || tiles < 4096);
+  return a.M > 4 ? tiles > 256 : pairs > 512 || (pairs > 256 && pairs <= 384);
+}
+
 // D of chunks ahead, and the waves a SIMD that its registers leave.
 template <bool I8, int MODE, int FT, int D, int OCC>
 int launch_few(Args a, int layers, hipStream_t st) {
@@ -401,7 +589,7 @@ int launch(Args a, int layers, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// Tiles of features a wave. Every workgroup reads all of x, which costs M rows
+// Tiles of features a wave, where workgroups have one tile. Every workgroup reads all of x, which costs M rows
 // out of L2 for 16 FT features of W; half the workgroups leave CUs idle where the
 // layer is small. Up to 16 rows (us, FT 1 / 2): N 4096 bf16 9.6 / 13, int8 8.6 /
 // 10.4; N 6144 15.7 / 13.3 and 12.3 / 10.8; N 128256 8 rows 205 / 192 and 148 /
@@ -423,6 +611,16 @@ int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
   for (int i = 0; i < layers; ++i) tiles += (a.n[i] + 15) / 16;
   const bool big = tiles >= 384, huge = tiles >= 896;
   // int8's scales in LDS: beside the sums 64 bytes a chunk and stream
+  if (a.M <= 16 && goes_on<I8>(a, mode, tiles)) {
+#define GO(X)                                                             \
+  if (a.K == X * CH * NW)                                                 \
+    return mode == SWIGLU ? launch_going<I8, SWIGLU, X>(a, layers, st)    \
+                          : launch_going<I8, PLAIN, X>(a, layers, st);
+    GO(4)
+    GO(3)
+    if constexpr (I8) { GO(2) }
+#undef GO
+  }
   if (a.M <= 16 && (!I8 || a.K <= 1 << 16)) {
     if (mode == SWIGLU) return launch_few<I8, SWIGLU, 1, 2, 4>(a, layers, st);
     const bool rounds = 2 * ((tiles + 511) / 512) <= (tiles + 255) / 256;

@@ -45,6 +45,28 @@ def test_tiles_a_wave_gpu(int8, n, k, m):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("k", [2048, 3072, 4096])
+@pytest.mark.parametrize("m", [1, 5, 16])
+@torch.no_grad()
+def test_workgroups_go_on_gpu(int8, k, m):
+    """More tiles than CUs: one that begins the second round, rounds that end in
+    part and whole, the last tile in part, and layers that end inside a tile."""
+    g = torch.Generator().manual_seed(k + m)
+    x = torch.randn(m, k, generator=g).bfloat16().cuda()
+    for ns, mode in (((4100,), 0), ((8196,), 0), ((16384,), 0),
+                     ((8200, 4100, 5000), 0), ((4100, 4100), SWIGLU),
+                     ((8200, 8200), SWIGLU), ((8192, 8192), SWIGLU)):
+        both = [_layer(n, k, i == 0, int8, g) for i, n in enumerate(ns)]
+        got = rows_linear(x, [b[0] for b in both], mode)
+        want = [f(x) for _, f in both]
+        if mode == SWIGLU:
+            want = [torch.nn.functional.silu(want[0]) * want[1]]
+        for y, w in zip(got, want):
+            _close(y, w)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("ns,k", [((1024,), 1024), ((4096, 1024, 1024), 1792),
                                   ((4096, 1024, 1028), 1792), ((512,), 2048),
                                   ((130, 64), 256)])
