@@ -202,6 +202,17 @@ def test_one_tile_of_rows_gpu(m, ns, k, mode, tile):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [-1, 0, 1, None])
+def test_square_tile_gpu(rows, monkeypatch):
+    """192 x 192, as the tiles before it."""
+    monkeypatch.setitem(globals(), "TILES", TILES + [(192, 192, 3)])
+    if rows is None:
+        test_every_tile_backward_gpu(len(TILES) - 1)
+    else:
+        test_every_tile_gpu(len(TILES) - 1, rows)
+
+
+@pytest.mark.gpu
 def test_what_lies_past_the_last_row_gpu():
     """Rows past the end count for nothing, whatever the last one holds: each
     value of the weight's gradient comes from its own column."""
