@@ -433,17 +433,13 @@ def call(mod: nn.Module, x):
     return mod(x)
 
 
-def _watched() -> bool:
-    return bool(nn.Linear.forward is not _TORCHS
-                or _module._global_forward_hooks
-                or _module._global_forward_pre_hooks
-                or _module._global_backward_hooks
-                or _module._global_backward_pre_hooks)
-
-
 def all_unhooked(mods) -> bool:
     """``unhooked`` of each of them."""
-    if _watched():
+    if nn.Linear.forward is not _TORCHS or \
+            _module._global_forward_hooks or \
+            _module._global_forward_pre_hooks or \
+            _module._global_backward_hooks or \
+            _module._global_backward_pre_hooks:
         return False
     for mod in mods:
         cls = type(mod)
@@ -462,7 +458,12 @@ def unhooked(mod: nn.Module, internal_ok: bool = False) -> bool:
     the framework's own hooks (marked ``_ds_internal``) take as well."""
     cls = type(mod)
     if "forward" in mod.__dict__ or mod._compiled_call_impl is not None or \
-            cls.forward is not _FORWARD.get(cls) or _watched():
+            cls.forward is not _FORWARD.get(cls) or \
+            nn.Linear.forward is not _TORCHS or \
+            _module._global_forward_hooks or \
+            _module._global_forward_pre_hooks or \
+            _module._global_backward_hooks or \
+            _module._global_backward_pre_hooks:
         return False
     if not (mod._forward_hooks or mod._forward_pre_hooks
             or mod._backward_hooks or mod._backward_pre_hooks):
