@@ -1166,20 +1166,20 @@ int launch_wide(Args a, bool merge, hipStream_t st) {
 }
 
 // number, BM, BN, waves along rows and features, stages in LDS; us a stage and
-// a tile of a chip full of them (fitted to 20 layers of 1024 x 1024 to 128256 x
-// 4096 and 33 to 8192 rows; root mean square error 6%). The largest make the
-// most products of what they load, the smaller ones fill the chip with fewer
-// rows or features. 256 x 192 has waves of three tiles of features: no gates.
+// a tile of a chip full of them (fitted to 8000 calls in all four modes, of 33 to
+// 8192 rows and 1024 x 1024 to 32000 x 18944; root mean square error 10%). The
+// largest make the most products of what they load, the smaller ones fill the chip
+// with fewer rows or features. 256 x 192 has waves of three tiles of features: no gates.
 #define TILES(X)                           \
-  X(0, 64, 64, 2, 2, 8, 0.280f, 1.7f)      \
-  X(1, 64, 128, 2, 2, 6, 0.405f, 2.4f)     \
-  X(2, 128, 64, 4, 2, 6, 0.349f, 2.3f)     \
-  X(3, 128, 128, 4, 2, 5, 0.523f, 3.7f)    \
-  X(4, 128, 256, 2, 4, 3, 0.807f, 6.3f)    \
-  X(5, 192, 128, 4, 2, 4, 0.646f, 4.8f)    \
-  X(6, 192, 256, 4, 2, 2, 1.060f, 7.5f)    \
-  X(7, 256, 128, 4, 2, 3, 0.790f, 5.7f)    \
-  X(8, 256, 192, 2, 4, 2, 1.038f, 7.0f)
+  X(0, 64, 64, 2, 2, 8, 0.305f, 1.2f)      \
+  X(1, 64, 128, 2, 2, 6, 0.437f, 2.6f)     \
+  X(2, 128, 64, 4, 2, 6, 0.365f, 2.6f)     \
+  X(3, 128, 128, 4, 2, 5, 0.532f, 3.4f)    \
+  X(4, 128, 256, 2, 4, 3, 0.759f, 4.9f)    \
+  X(5, 192, 128, 4, 2, 4, 0.674f, 5.2f)    \
+  X(6, 192, 256, 4, 2, 2, 1.047f, 6.3f)    \
+  X(7, 256, 128, 4, 2, 3, 0.754f, 5.2f)    \
+  X(8, 256, 192, 2, 4, 2, 1.023f, 6.3f)
 constexpr int WIDE = 9;
 // 192 x 192, for what lies between the rounds of the others (us, the earlier choice /
 // this, over 150 layers that it is chosen for 0.89 forward, 0.92 backward, at worst
@@ -1189,7 +1189,7 @@ constexpr int WIDE = 9;
 // a little more than its terms say (3000 rows, n 32000, K 3072 in three splits of 256 x
 // 256 508, in this 549).
 constexpr int SQUARE = 10;
-#define BETWEEN(X) X(SQUARE, 192, 192, 4, 2, 3, 0.860f, 8.5f)
+#define BETWEEN(X) X(SQUARE, 192, 192, 4, 2, 3, 0.804f, 6.3f)
 
 // A wave's gate and up tiles in pairs; halves of x in blocks of 64 columns.
 #define GATES(BN, WN) (BN / WN / 16 % 2 == 0)
@@ -1207,36 +1207,40 @@ const Tile tiles_[] = {
 #define X(I, BM, BN, WM, WN, NS, U, F) \
   {BM, BN, NS, GATES(BN, WN), BLOCKS(BM, WM), U, F},
     TILES(X)
-    {256, 256, 2, true, true, 1.262f, 7.9f},    // WIDE
+    {256, 256, 2, true, true, 1.149f, 8.8f},    // WIDE
     BETWEEN(X)
 #undef X
 };
 
 // us that a tile and a number of splits take: rounds of the 256 CUs (the last
 // one, in part empty, runs faster: less power, less traffic) or W and x from
-// memory at 4.15 TB/s, a sixth less by few workgroups (8192 x 8192, 64 rows: 128 of
-// them 43.7 us, 256 36.1; 10240 x 8192, 128 rows: 160 59, 240 45; but 11008 x 4096,
-// 17 rows: 172 22.7, 344 25.5), whichever is longer, then adding the splits up.
+// memory, whichever is longer, then adding the splits up. Memory gives less to few
+// workgroups (8192 x 8192, 64 rows: 128 of them 43.7 us, 256 36.1; but 11008 x 4096,
+// 17 rows: 172 22.7, 344 25.5) and to W read across in columns of 64, 128 bytes a row
+// (its gradient's input, 128 rows, 14336 x 14336: 128 x 64 133 us, 192 x 256 95; 64
+// rows, 32000 x 18944 by 64 x 128 304, by 128 x 256 206).
 float estimate(const Tile& t, double tiles, int steps, double rows,
                double columns, double bytes, int splits, int mode) {
   tiles *= splits;
   const double whole = (double)(long long)(tiles / 256);
   const double rest = tiles / 256 - whole;
-  double us = (whole + (rest > 0 ? 0.76 + 0.24 * rest : 0)) *
-      (steps / (double)splits * t.stage + t.fixed);
-  double mem = bytes / (mode == PLAIN && tiles < 168 ? 3.46e6 : 4.15e6);
+  double us = (whole + (rest > 0 ? 0.82 + 0.18 * rest : 0)) *
+      (steps / (double)splits * t.stage * (mode == GRAD_W ? 0.95 : 1) + t.fixed);
+  double mem = bytes / (mode == GRAD_X && t.bn == 64 ? 4.3e6
+                        : mode == PLAIN && tiles < 168 ? 4.0e6 : 5.7e6);
   us *= us * us;
   mem *= mem * mem;
   us = cbrt(sqrt(us * us + mem * mem));
-  if (splits > 1) us += 2.7 + 0.296e-6 * splits * rows * columns * 4;
+  if (splits > 1) us += 2.65 + 0.276e-6 * splits * rows * columns * 4;
   return (float)us;
 }
 
 }  // namespace
 
 // The tile for 1..3 weights on one input and the splits of the contraction, by
-// ``estimate``: over those layers and rows within 1% of the fastest on average,
-// 23% at worst. Each split needs the ring's stages. -1: no tile for this K.
+// ``estimate``: over those calls 0.6% over the fastest on average, 0.9% for the
+// input's gradient (4.4% by an earlier fit). Each split needs the ring's stages. -1:
+// no tile for this K.
 extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
                                    int mode, int* splits) {
   static const int some[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
@@ -1264,7 +1268,7 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
       if (s > 1 && (mode == SWIGLU || tiles * s > 520)) break;
       if (steps / s < t.stages) break;
       float us = estimate(t, tiles, steps, rows, columns, bytes, s, mode);
-      if (i == SQUARE && mode == GRAD_X) us *= 1.06f;
+      if (i == SQUARE && mode == GRAD_X) us *= 1.04f;
       if (best < 0 || us < least) {
         best = i;
         least = us;
