@@ -950,14 +950,17 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
                          int64_t mode) {
     if (M < 2560 || mode == 1) return true;
     const int64_t K = in.size(1);
-    int64_t most = 0, all = 0;
+    int64_t most = 0, all = 0, tiles = 0;
     for (int i = first; i < first + count; ++i) {
       const int64_t n = weights[i].numel() / K;
       most = std::max(most, n);
       all += n;
+      tiles += (M + 255) / 256 * ((n + 255) / 256);
     }
-    if (count == 1) return K >= 16384 && all % 4096 != 0;
-    return most * K < (1 << 25) && (M < 16384 || 1.0 * M * all * K < 4e11);
+    if (count == 1)
+      return K < 3072 || tiles % 256 != 0 || (K >= 16384 && all % 4096 != 0);
+    return M % 256 != 0 || (most * K < (1 << 26) &&
+                            (M < 16384 || 1.0 * M * all * K < 4e11));
   };
   auto linears = [&](const at::Tensor& in, int first, int count,
                      int64_t mode) {

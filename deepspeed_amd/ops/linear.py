@@ -76,6 +76,11 @@ def backward_plan(T: int, N: int, K: int):
     return w, big and N < K, big and N >= K
 
 
+def _tiles(T: int, ns) -> int:
+    """Tiles of 256 x 256 of outputs [T, n]."""
+    return -(-T // 256) * sum(-(-n // 256) for n in ns)
+
+
 def own_dx(T: int, ns, K: int) -> bool:
     """Whether the input's gradient of layers [n, K] of ``ns`` features over T rows
     is csrc/tile_linear.hip's, which adds the layers up in one product (us, library
@@ -83,17 +88,17 @@ def own_dx(T: int, ns, K: int) -> bool:
 
     N 14336, K 4096, 1000 rows 128 / 110, 2300 251 / 246; 18944, K 3584, 2048 rows
     348 / 223; 32064, K 3072, 2559 rows 608 / 409; 3072, K 8192, 1024 rows 53 / 50.
-    From 2560 rows on the library's rounds of tiles are ahead past 7e10 products
-    (4096, K 4096: 4000 rows 104 / 102, 8192 187 / 201, 16384 361 / 419, 32768 715 /
-    871, but 10000 378 / 279; 8192, K 3072: 3000 159 / 147, 4000 190 / 203, 12288 451
-    / 519; 3072, K 3072: 4096 75 / 64, 8192 135 / 134, 16384 213 / 237; 1024, K 1024:
-    16384 39 / 33), where the features are many times the inputs past 1.7e11 (24576,
-    K 1024: 8192 rows 0.60 of the library's time, 10000 1.18; 32768, K 512: 10000
-    0.66, 12288 1.12; 32000, K 1024: 5000 427 / 262, 8192 389 / 431).
-    Several layers: the additions count for less the more features there are (2 of
-    8192, K 3072: 4096 rows 347 / 331, 6000 550 / 637, 16384 1104 / 1262; 2 of 6144,
-    K 4096 0.74 to 1.05 from 5000 rows on; 4096 + 2 of 1024, K 4096: 8192 rows 383 /
-    303, 32768 1413 / 1217; 3 of 3072, K 3072: 32768 rows 1473 / 1398)."""
+    From 2560 rows on, over 3400 layers and rows, the library is ahead past 7e10
+    products where the rows are whole tiles of 256 (14336, K 4096: 4096 rows 343 / 340,
+    8192 637 / 692; 4096, K 4096, 8192 rows 192 / 202; 14336, K 3072, 8192 544 / 619),
+    but for features many times the inputs up to 1.7e11. Elsewhere the kernel is, by
+    5% in the geometric mean (128256, K 3072, 4000 rows 4160 / 2676; 3072, K 8192 158 /
+    153), but not where it has a bit more than a round of tiles (14336, K 2048, 10000
+    rows 459 / 593), if there are not too many features.
+    Several layers, over 1900: 0.83 of the library's time, whose additions count for
+    less the more features there are (4096 + 2 of 1024, K 4096: 8192 rows 383 / 297; 3
+    of 3072, K 8192: 4096 rows 546 / 437; whole tiles of rows and 2 of 14336, K 4096:
+    4096 rows 712 / 695, 8192 1332 / 1396; 2 of 8192, K 3072, 8192 655 / 683)."""
     if T <= ROWS or T >= 1 << 30 or K % 8 or K > INPUTS:
         return False
     for n in ns:
@@ -101,12 +106,13 @@ def own_dx(T: int, ns, K: int) -> bool:
             return False
     if T < 2560:
         return True
-    if max(ns) * K >= 1 << 25:
-        return False
-    work = T * sum(ns) * K
+    work, tiles = T * sum(ns) * K, _tiles(T, (K,))
     if len(ns) > 1:
-        return work < 22e10 or sum(ns) <= 4 * K
-    return work < (17e10 if ns[0] >= 16 * K else 7e10)
+        return T % 256 != 0 or sum(ns) <= 4 * K or (
+            work < 22e10 and max(ns) * K < 1 << 25)
+    if max(ns) * K < 1 << 25 and work < (17e10 if ns[0] >= 16 * K else 7e10):
+        return True
+    return T % 256 != 0 and (not 256 < tiles < 400 or ns[0] >= 28672)
 
 
 def own_dw(T: int, N: int, K: int) -> bool:
@@ -149,25 +155,24 @@ def own_forward(T: int, ns, K: int, mode: int = PLAIN) -> bool:
     library and kernel: gate and up 14336, K 4096, 224 rows 95 + activation / 67;
     4096, K 14336, 1024 rows 138 / 108; 3584, K 18944, 2331 rows 489 / 302).
 
-    From 2560 rows on the library's whole rounds of tiles reach 5% more for one layer
-    (4096 rows: N 4096, K 4096 91 / 98; N 4096, K 14336 304 / 324; N 128256 2930 /
-    3060; elsewhere 3300 rows: N 4096, K 14336 343 / 305), but for contractions from
-    16384 on where the features are no whole rounds (geometric mean over 2560 to 16384
-    rows and K 16384 to 28672, library 1: N 3584 0.71, 4608 0.73, 5120 0.85, 7168
-    0.83; 2048 0.89; 4096 1.05, 8192 1.01). Several layers stay here (3 of 3072, K 3072,
-    8192 rows 360 / 329; 2 of 5632, K 2048, 0.78 to 1.07), but not large ones
-    (8192 + 2 of 1024, K 8192: 4096 rows 473 / 527, 12288 1330 / 1466) and not from
-    16384 rows on (4096 + 2 of 1024, K 4096: 12288 rows 424 / 458, 16384 528 / 560,
-    32768 1071 / 1156; 2 of 8192, K 3072, 16384 rows 1081 / 1168); gate and up with
-    their activation are even (14336, K 4096: 8192 rows 1349 / 1385, 16384 2706 /
-    2708)."""
+    From 2560 rows on, over 2700 layers and rows: 0.92 of the library's time for one
+    layer, but where 256 x 256 tiles fill whole rounds of the 256 CUs and contractions
+    are long, the library is ahead (4096 rows: N 4096, K 14336 295 / 307; 8192 rows: N
+    14336, K 4096 628 / 644; else N 128256, K 4096, 4096 rows 2970 / 2930, N 3072, K
+    4096 80 / 76). Several layers, over 1500: 0.86 (3 of 3072, K 3072, 8192 rows 370 /
+    330; 2 of 11008, K 4096, 8192 rows 1285 / 973), but not large ones of whole tiles of
+    rows (2 of 8192, K 14336, 4096 rows 1223 / 1257) nor, from 16384 of these on, many
+    products (3 of 4096, K 4096: 16384 rows 1063 / 1090); gate and up with their
+    activation stay (14336, K 4096, 8192 rows 1240 + activation / 1290)."""
     if T <= ROWS or K % 64 or not 192 <= K <= INPUTS or any(n % 4 for n in ns):
         return False
     if T < 2560 or mode == SWIGLU:
         return True
     if len(ns) == 1:
-        return K >= 16384 and ns[0] % 4096 != 0
-    return max(ns) * K < 1 << 25 and (T < 16384 or T * sum(ns) * K < 4e11)
+        return K < 3072 or _tiles(T, ns) % 256 != 0 or (
+            K >= 16384 and ns[0] % 4096 != 0)
+    return T % 256 != 0 or max(ns) * K < 1 << 26 and (
+        T < 16384 or T * sum(ns) * K < 4e11)
 
 
 def _aligned(*ts) -> bool:
