@@ -26,8 +26,8 @@
 //   * Bound by the stream of K and V (decode): 16-byte loads, the next tile in
 //     flight while the softmax and the second product of this one run, three
 //     waves a SIMD. 55 us a layer at 32 requests of 2000 tokens and 8 key
-//     heads (4.8 TB/s), 100 us at 8 of 16000 (5.2 TB/s; a large copy reaches
-//     5.0). One position a wave at a time (2-byte loads, a six-step shuffle
+//     heads (4.8 TB/s), 98 us at 8 of 16000 (5.3 TB/s; a large copy reaches
+//     4.9). One position a wave at a time (2-byte loads, a six-step shuffle
 //     chain each) took 240 and 459 us.
 //   * S^T = K Q^T on mfma_f32_16x16x32_bf16: K rows go from global memory
 //     straight into A fragments (64 contiguous bytes a row and instruction).
