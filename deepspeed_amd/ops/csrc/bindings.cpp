@@ -957,8 +957,9 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
       all += n;
       tiles += (M + 255) / 256 * ((n + 255) / 256);
     }
+    if (count == 1 && K >= 16384) return all % 4096 != 0;
     if (count == 1)
-      return K < 3072 || tiles % 256 != 0 || (K >= 16384 && all % 4096 != 0);
+      return M % 256 != 0 || (all < 65536 && (K < 3072 || tiles % 256 != 0));
     return M % 256 != 0 || (most * K < (1 << 26) &&
                             (M < 16384 || 1.0 * M * all * K < 4e11));
   };

@@ -98,7 +98,8 @@ def own_dx(T: int, ns, K: int) -> bool:
     Several layers, over 1900: 0.83 of the library's time, whose additions count for
     less the more features there are (4096 + 2 of 1024, K 4096: 8192 rows 383 / 297; 3
     of 3072, K 8192: 4096 rows 546 / 437; whole tiles of rows and 2 of 14336, K 4096:
-    4096 rows 712 / 695, 8192 1332 / 1396; 2 of 8192, K 3072, 8192 655 / 683)."""
+    4096 rows 712 / 695, 8192 1332 / 1396; 2 of 8192, K 3072, 8192 655 / 683; a bit more
+    than a round of tiles: 2 of 11008, K 2048, 10000 rows 730 / 914)."""
     if T <= ROWS or T >= 1 << 30 or K % 8 or K > INPUTS:
         return False
     for n in ns:
@@ -107,12 +108,14 @@ def own_dx(T: int, ns, K: int) -> bool:
     if T < 2560:
         return True
     work, tiles = T * sum(ns) * K, _tiles(T, (K,))
+    uneven = T % 256 != 0 and (not 256 < tiles < 400 or
+                               (len(ns) == 1 and ns[0] >= 28672))
     if len(ns) > 1:
-        return T % 256 != 0 or sum(ns) <= 4 * K or (
+        return uneven or sum(ns) <= 4 * K or (
             work < 22e10 and max(ns) * K < 1 << 25)
     if max(ns) * K < 1 << 25 and work < (17e10 if ns[0] >= 16 * K else 7e10):
         return True
-    return T % 256 != 0 and (not 256 < tiles < 400 or ns[0] >= 28672)
+    return uneven
 
 
 def own_dw(T: int, N: int, K: int) -> bool:
@@ -158,8 +161,11 @@ def own_forward(T: int, ns, K: int, mode: int = PLAIN) -> bool:
     From 2560 rows on, over 2700 layers and rows: 0.92 of the library's time for one
     layer, but where 256 x 256 tiles fill whole rounds of the 256 CUs and contractions
     are long, the library is ahead (4096 rows: N 4096, K 14336 295 / 307; 8192 rows: N
-    14336, K 4096 628 / 644; else N 128256, K 4096, 4096 rows 2970 / 2930, N 3072, K
-    4096 80 / 76). Several layers, over 1500: 0.86 (3 of 3072, K 3072, 8192 rows 370 /
+    14336, K 4096 628 / 644; else N 3072, K 4096, 4096 rows 80 / 76, 8192 126 / 117 at K
+    3072), and from 65536 features on whole tiles of rows are within 2% either way
+    (128256, K 4096, 4096 rows 2970 / 2930). K from 16384 on: but for whole rounds
+    (geometric mean over 2560 to 16384 rows by the kernel before, library 1: N 3584
+    0.71, 5120 0.85, 4096 1.05, 8192 1.01). Several layers, over 1500: 0.86 (3 of 3072, K 3072, 8192 rows 370 /
     330; 2 of 11008, K 4096, 8192 rows 1285 / 973), but not large ones of whole tiles of
     rows (2 of 8192, K 14336, 4096 rows 1223 / 1257) nor, from 16384 of these on, many
     products (3 of 4096, K 4096: 16384 rows 1063 / 1090); gate and up with their
@@ -169,8 +175,10 @@ def own_forward(T: int, ns, K: int, mode: int = PLAIN) -> bool:
     if T < 2560 or mode == SWIGLU:
         return True
     if len(ns) == 1:
-        return K < 3072 or _tiles(T, ns) % 256 != 0 or (
-            K >= 16384 and ns[0] % 4096 != 0)
+        if K >= 16384:
+            return ns[0] % 4096 != 0
+        return T % 256 != 0 or ns[0] < 65536 and (
+            K < 3072 or _tiles(T, ns) % 256 != 0)
     return T % 256 != 0 or max(ns) * K < 1 << 26 and (
         T < 16384 or T * sum(ns) * K < 4e11)
 
