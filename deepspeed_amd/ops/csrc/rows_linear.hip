@@ -589,7 +589,8 @@ int launch(Args a, int layers, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// Tiles of features a wave, where workgroups have one tile. Every workgroup reads all of x, which costs M rows
+// Tiles of features a wave, where workgroups have one tile. Every workgroup reads
+// all of x, which costs M rows
 // out of L2 for 16 FT features of W; half the workgroups leave CUs idle where the
 // layer is small. Up to 16 rows (us, FT 1 / 2): N 4096 bf16 9.6 / 13, int8 8.6 /
 // 10.4; N 6144 15.7 / 13.3 and 12.3 / 10.8; N 128256 8 rows 205 / 192 and 148 /
