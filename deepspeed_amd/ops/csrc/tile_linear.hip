@@ -527,7 +527,7 @@ __device__ __forceinline__ void load(u32x4 from, unsigned off, int soff) {
 // The sums of a wave that has all 256 accumulation registers: four from R on. They
 // are named, not variables: those the compiler moves to other registers and, as they
 // run out, to memory. It has to have no use for these registers itself (nothing is
-// spilled: some 170 to 190 of 256 others are taken). Operands have to be written, and
+// spilled: 147 to 176 of 256 others are taken). Operands have to be written, and
 // products made, some instructions before they are read.
 __device__ __forceinline__ void take_sums() {
   asm volatile("" ::: "a0", "a255");
@@ -570,9 +570,14 @@ __device__ __forceinline__ unsigned packed2(float lo, float hi) {
 // half stage by 16 operands (eight waves of 128 x 64: 12 for 32). The chip's power
 // bounds these products, so reads that are not made become clock.
 //
-//   * A workgroup stays on its CU and goes on from tile to tile: the ring is
-// filled across the border, so that a tile's first stages load while the one before
-// is computed and stored.
+//   * A tile a workgroup. One that goes on from tile to tile, its ring filled across
+// the border, gains up to 1.3% alone on the chip (2.5 at K 2048, 4.5 at 1024), but
+// where another kernel holds some of the CUs, a collective above all, the tiles of
+// the workgroups that wait for these are late together, and the collective waits for
+// the whole product (us with 8 CUs held, eight waves / one tile / going on: 4096 rows
+// 28672, K 4096 771 / 796 / 1105; 8192 x 8192 x 8192 894 / 923 / 1234; dx of 14336, K
+// 4096, 8192 rows 988 / 1003 / 1187; with 32 held 840 / 787 / 1098, 978 / 914 / 1224,
+// 1054 / 1000 / 1186).
 //   * One barrier a stage, behind the reads of its second half: from there on the
 // stage's places in the ring are free (x two stages, W three), and the next stage
 // has arrived. A barrier costs some 70 of a stage's 2500 cycles, a load between two
@@ -585,10 +590,10 @@ __device__ __forceinline__ unsigned packed2(float lo, float hi) {
 //   * A tile's first products write its sums, those of no bias are stored as they
 // are, and outputs pass the caches by: 2 to 4%.
 //
-// us, eight waves with a tile a workgroup, and now: 8192 x 8192 x 8192 786 / 695;
-// 4096 rows, K 4096: 28672 690 / 632, 6144 175 / 159, gate and up 14336 712 / 665;
-// gate and up 18944, K 3584, 2331 rows 517 / 486; dx of 14336, K 4096, 8192 rows 738 /
-// 690; dW of that 765 / 735 (its transposing reads are two an operand).
+// us one after another, eight waves and now: 8192 x 8192 x 8192 764 / 720; 4096 rows,
+// K 4096: 28672 696 / 648, 6144 166 / 159, gate and up 14336 712 / 680; gate and up
+// 18944, K 3584, 2331 rows 536 / 503; dx of 14336, K 4096, 8192 rows 745 / 706; dW of
+// that 789 / 727 (its transposing reads are two an operand).
 template <int MODE, bool PARTS>
 __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   constexpr bool GLU = MODE == SWIGLU;
@@ -607,11 +612,8 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   // turn, so that they work side by side.
   constexpr int GROUP = 4;
   const int per = a.tiles * a.mtiles, total = per * a.splits;
-  const int slots = gridDim.x / 8, xcd = blockIdx.x % 8;
-  int item = xcd * (total / 8) + min(xcd, total % 8);
-  const int end = item + total / 8 + (xcd < total % 8);
-  item += blockIdx.x / 8;
-  if (item >= end) return;
+  const int xcd = blockIdx.x % 8;
+  const int item = xcd * (total / 8) + min(xcd, total % 8) + blockIdx.x / 8;
 
   struct Place {
     int m0, n0, s0, n_it, layer, split;
@@ -641,9 +643,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
     p.n_it = uni((p.split + 1) * steps / a.splits) - p.s0;
     return p;
   };
-  Place at = locate(item), next = at;
-  bool more = item + slots < end;
-  if (more) next = locate(item + slots);
+  const Place at = locate(item);
 
   // ---- loads: the lanes' places in the pieces of 1 KB, as above. Rows past the
   // end lie past the descriptor's; columns past the end are not stored.
@@ -730,15 +730,11 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
 #pragma unroll
       for (int j = 0; j < P; ++j) xoff[j] = place_x(j, xld);
   };
-  // Behind the last of these: the next layer, the next tile, or nothing, which is
-  // a descriptor of no bytes.
-  bool wover = false, xover = false;
+  // Behind the last of these: the next layer, or nothing, which is a descriptor of no
+  // bytes.
   auto turn_w = [&]() INLINE {
     if (MODE == GRAD_X && wstep + 1 < wstop) {
-      seek_w(wover ? next.n0 : at.n0, 0, wstep + 1, wstop);
-    } else if (more && !wover) {
-      wover = true;
-      seek_w(next.n0, next.layer, next.s0, next.s0 + next.n_it);
+      seek_w(at.n0, 0, wstep + 1, wstop);
     } else {
       wfrom[2] = 0;
       wsoff = wrow = 0;
@@ -748,10 +744,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   };
   auto turn_x = [&]() INLINE {
     if (MODE == GRAD_X && xstep + 1 < xstop) {
-      seek_x(xover ? next.m0 : at.m0, 0, xstep + 1, xstop);
-    } else if (more && !xover) {
-      xover = true;
-      seek_x(next.m0, next.layer, next.s0, next.s0 + next.n_it);
+      seek_x(at.m0, 0, xstep + 1, xstop);
     } else {
       xfrom[2] = 0;
       xsoff = xrow = 0;
@@ -869,8 +862,6 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   // those of the next stage's first half behind the middle; x two stages ahead and
   // W three are loaded behind the barrier.
   constexpr int N2 = 2 * F * F, BARRIER = 30;
-  constexpr int STORES = 4 * F;     // of a tile, at least
-  int young = 0;        // a tile's stores are behind the loads that are waited for
   auto stage = [&](auto first) INLINE {
     constexpr bool FIRST = decltype(first)::value;
     __builtin_amdgcn_sched_barrier(0);
@@ -880,15 +871,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       constexpr int i = decltype(at)::value, h = i / (F * F), m = i / F % F;
       constexpr int f = m % 2 ? F - 1 - i % F : i % F;
       if constexpr (i == BARRIER) {
-        if constexpr (FIRST)
-          asm volatile("s_cmp_lg_u32 %0, 0\n\t"
-                       "s_cbranch_scc1 1f\n\t"
-                       "s_waitcnt vmcnt(%1)\n"
-                       "1:\n\t"
-                       "s_waitcnt vmcnt(%2)"
-                       :: "s"(young), "n"(P), "n"(P + STORES) : "memory", "scc");
-        else
-          wait_loads<P>();
+        wait_loads<P>();
         wait_reads();
         __builtin_amdgcn_s_barrier();
         wget = next_w(wget, 0);
@@ -934,136 +917,126 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       else move_x();
     }
   };
-  while (true) {
-    stage(Int<1>{});
+  stage(Int<1>{});
 #pragma clang loop unroll(disable)
-    for (int it = 1; it < at.n_it; ++it) stage(Int<0>{});
+  for (int it = 1; it < at.n_it; ++it) stage(Int<0>{});
 
-    asm volatile("s_nop 15");     // the last products
-    // Every store is made, past the tile's rows or columns to nowhere: the waits
-    // above count them.
-    const int N = WT ? K : a.n[at.layer];
-    const int rows = MODE == GRAD_W ? a.n[at.layer] : a.M;
-    const int m_of = uni(at.m0 + wm * (BM / 2));
-    const int have = uni(max(0, min(rows - m_of, BM / 2)));
-    constexpr unsigned NOWHERE = 0x80000000u;
-    if constexpr (PARTS) {
-      const int before = a.n_end[at.layer] - a.n[at.layer];
-      const int all = WT ? K : a.n_end[a.layers - 1];
-      const int all_rows = MODE == GRAD_W ? a.n_end[a.layers - 1] : a.M;
-      const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(a.part + ((long long)at.split * all_rows + m_of +
-                            (MODE == GRAD_W ? before : 0)) * all +
-                  (MODE == PLAIN ? before : 0)),
-          (short)0, (int)((unsigned)have * all * 4), 0x00020000);
-      // gradients: row col, columns 4 g ..; otherwise rows 4 g + r, half of eight
-      const int n1 = at.n0 + wn * (BN / 2) + (WT ? 4 * g : F * col);
-      const int r1 = WT ? col : 4 * g;
+  asm volatile("s_nop 15");     // the last products
+  // past the tile's rows or columns to nowhere
+  const int N = WT ? K : a.n[at.layer];
+  const int rows = MODE == GRAD_W ? a.n[at.layer] : a.M;
+  const int m_of = uni(at.m0 + wm * (BM / 2));
+  const int have = uni(max(0, min(rows - m_of, BM / 2)));
+  constexpr unsigned NOWHERE = 0x80000000u;
+  if constexpr (PARTS) {
+    const int before = a.n_end[at.layer] - a.n[at.layer];
+    const int all = WT ? K : a.n_end[a.layers - 1];
+    const int all_rows = MODE == GRAD_W ? a.n_end[a.layers - 1] : a.M;
+    const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(a.part + ((long long)at.split * all_rows + m_of +
+                          (MODE == GRAD_W ? before : 0)) * all +
+                (MODE == PLAIN ? before : 0)),
+        (short)0, (int)((unsigned)have * all * 4), 0x00020000);
+    // gradients: row col, columns 4 g ..; otherwise rows 4 g + r, half of eight
+    const int n1 = at.n0 + wn * (BN / 2) + (WT ? 4 * g : F * col);
+    const int r1 = WT ? col : 4 * g;
+    auto store = [&](auto at) INLINE {
+      constexpr int m = decltype(at)::value / F, i = decltype(at)::value % F;
+      constexpr int f = 4 * (i & 1), r = i >> 1;
+      f32x4 v;
+      if constexpr (WT)
+        v = f32x4{sum<acc(i, m)>(), sum<acc(i, m) + 1>(), sum<acc(i, m) + 2>(),
+                  sum<acc(i, m) + 3>()};
+      else
+        v = f32x4{sum<acc(f, m) + r>(), sum<acc(f + 1, m) + r>(),
+                  sum<acc(f + 2, m) + r>(), sum<acc(f + 3, m) + r>()};
+      const int row = r1 + 16 * m + (WT ? 0 : r);
+      const int n = n1 + (WT ? 16 * i : f);
+      __builtin_amdgcn_raw_buffer_store_b128(
+          __builtin_bit_cast(u32x4, v), to,
+          n < N && row < have ? (unsigned)(row * all + n) * 4 : NOWHERE, 0, 0);
+    };
+    each(std::make_integer_sequence<int, F * F>{}, store);
+  } else {
+    // outputs pass the caches by, which hold what other tiles still read
+    constexpr int STREAM = 2;
+    short* out = a.out[MODE == GRAD_X || GLU ? 0 : at.layer];
+    const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(out + (long long)m_of * N), (short)0,
+        (int)((unsigned)have * N * 2), 0x00020000);
+    if constexpr (WT) {
+      // columns 4 g .. of two tiles to 8 of one: odd rows of lanes of the first
+      // change places with even ones of the second
+      const int n1 = at.n0 + wn * (BN / 2) + (g & 1) * 16 + (g >> 1) * 8;
       auto store = [&](auto at) INLINE {
-        constexpr int m = decltype(at)::value / F, i = decltype(at)::value % F;
-        constexpr int f = 4 * (i & 1), r = i >> 1;
-        f32x4 v;
-        if constexpr (WT)
-          v = f32x4{sum<acc(i, m)>(), sum<acc(i, m) + 1>(), sum<acc(i, m) + 2>(),
-                    sum<acc(i, m) + 3>()};
-        else
-          v = f32x4{sum<acc(f, m) + r>(), sum<acc(f + 1, m) + r>(),
-                    sum<acc(f + 2, m) + r>(), sum<acc(f + 3, m) + r>()};
-        const int row = r1 + 16 * m + (WT ? 0 : r);
-        const int n = n1 + (WT ? 16 * i : f);
+        constexpr int f = decltype(at)::value / F * 2, m = decltype(at)::value % F;
+        constexpr int A = acc(f, m), B = acc(f + 1, m);
+        const unsigned y0 = packed2(sum<A>(), sum<A + 1>());
+        const unsigned y1 = packed2(sum<A + 2>(), sum<A + 3>());
+        const unsigned z0 = packed2(sum<B>(), sum<B + 1>());
+        const unsigned z1 = packed2(sum<B + 2>(), sum<B + 3>());
+        const auto lo = __builtin_amdgcn_permlane16_swap(y0, z0, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(y1, z1, false, false);
+        const int n = n1 + 16 * f;
         __builtin_amdgcn_raw_buffer_store_b128(
-            __builtin_bit_cast(u32x4, v), to,
-            n < N && row < have ? (unsigned)(row * all + n) * 4 : NOWHERE, 0, 0);
+            u32x4{lo[0], hi[0], lo[1], hi[1]}, to,
+            n < N ? (unsigned)((16 * m + col) * N + n) * 2 : NOWHERE, 0, STREAM);
       };
-      each(std::make_integer_sequence<int, F * F>{}, store);
+      each(std::make_integer_sequence<int, F / 2 * F>{}, store);
     } else {
-      // outputs pass the caches by, which hold what other tiles still read
-      constexpr int STREAM = 2;
-      short* out = a.out[MODE == GRAD_X || GLU ? 0 : at.layer];
-      const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(out + (long long)m_of * N), (short)0,
-          (int)((unsigned)have * N * 2), 0x00020000);
-      if constexpr (WT) {
-        // columns 4 g .. of two tiles to 8 of one: odd rows of lanes of the first
-        // change places with even ones of the second
-        const int n1 = at.n0 + wn * (BN / 2) + (g & 1) * 16 + (g >> 1) * 8;
-        auto store = [&](auto at) INLINE {
-          constexpr int f = decltype(at)::value / F * 2, m = decltype(at)::value % F;
-          constexpr int A = acc(f, m), B = acc(f + 1, m);
-          const unsigned y0 = packed2(sum<A>(), sum<A + 1>());
-          const unsigned y1 = packed2(sum<A + 2>(), sum<A + 3>());
-          const unsigned z0 = packed2(sum<B>(), sum<B + 1>());
-          const unsigned z1 = packed2(sum<B + 2>(), sum<B + 3>());
-          const auto lo = __builtin_amdgcn_permlane16_swap(y0, z0, false, false);
-          const auto hi = __builtin_amdgcn_permlane16_swap(y1, z1, false, false);
-          const int n = n1 + 16 * f;
-          __builtin_amdgcn_raw_buffer_store_b128(
-              u32x4{lo[0], hi[0], lo[1], hi[1]}, to,
-              n < N ? (unsigned)((16 * m + col) * N + n) * 2 : NOWHERE, 0, STREAM);
-        };
-        each(std::make_integer_sequence<int, F / 2 * F>{}, store);
-      } else {
-        constexpr int W = GLU ? F / 2 : F;      // features a lane
-        const int n = at.n0 + wn * (GLU ? BN / 4 : BN / 2) + W * col;
-        float b[GLU ? 2 : 1][W];
-        const bool biased = a.bias[GLU ? 0 : at.layer] || (GLU && a.bias[1]);
-        if (biased)
+      constexpr int W = GLU ? F / 2 : F;      // features a lane
+      const int n = at.n0 + wn * (GLU ? BN / 4 : BN / 2) + W * col;
+      float b[GLU ? 2 : 1][W];
+      const bool biased = a.bias[GLU ? 0 : at.layer] || (GLU && a.bias[1]);
+      if (biased)
 #pragma unroll
-        for (int l = 0; l < (GLU ? 2 : 1); ++l) {
-          const short* bias = a.bias[GLU ? l : at.layer];   // of none: zeros
-          const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
-              (void*)bias, (short)0, bias ? N * 2 : 0, 0x00020000);
+      for (int l = 0; l < (GLU ? 2 : 1); ++l) {
+        const short* bias = a.bias[GLU ? l : at.layer];   // of none: zeros
+        const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)bias, (short)0, bias ? N * 2 : 0, 0x00020000);
 #pragma unroll
-          for (int e = 0; e < W; ++e)
-            b[l][e] = value((short)__builtin_amdgcn_raw_buffer_load_b16(
-                from, (n + e) * 2, 0, 0));
-        }
-        typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-        auto store = [&](auto bias, auto at) INLINE {
-          constexpr bool B = decltype(bias)::value;
-          constexpr int m = decltype(at)::value / 4, r = decltype(at)::value % 4;
-          const unsigned o =
-              n < N ? (unsigned)((4 * g + 16 * m + r) * N + n) * 2 : NOWHERE;
-          auto one = [&](auto at) INLINE {
-            constexpr int e = decltype(at)::value;
-            if constexpr (GLU) {
-              const float t = sum<acc(2 * e, m) + r>() + (B ? b[0][e] : 0.f);
-              return t / (1.f + expf(-t)) *
-                  (sum<acc(2 * e + 1, m) + r>() + (B ? b[GLU][e] : 0.f));
-            } else {
-              return B ? sum<acc(e, m) + r>() + b[0][e] : sum<acc(e, m) + r>();
-            }
-          };
-          const u32x2 v = {packed2(one(Int<0>{}), one(Int<1>{})),
-                           packed2(one(Int<2>{}), one(Int<3>{}))};
-          if constexpr (GLU)
-            __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, STREAM);
-          else {
-            const u32x2 u = {packed2(one(Int<4>{}), one(Int<5>{})),
-                             packed2(one(Int<6>{}), one(Int<7>{}))};
-            if (N % 8 == 0) {
-              __builtin_amdgcn_raw_buffer_store_b128(u32x4{v[0], v[1], u[0], u[1]},
-                                                     to, o, 0, STREAM);
-            } else {
-              __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, STREAM);
-              __builtin_amdgcn_raw_buffer_store_b64(
-                  u, to, n + 4 < N ? o + 8 : NOWHERE, 0, STREAM);
-            }
+        for (int e = 0; e < W; ++e)
+          b[l][e] = value((short)__builtin_amdgcn_raw_buffer_load_b16(
+              from, (n + e) * 2, 0, 0));
+      }
+      typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+      auto store = [&](auto bias, auto at) INLINE {
+        constexpr bool B = decltype(bias)::value;
+        constexpr int m = decltype(at)::value / 4, r = decltype(at)::value % 4;
+        const unsigned o =
+            n < N ? (unsigned)((4 * g + 16 * m + r) * N + n) * 2 : NOWHERE;
+        auto one = [&](auto at) INLINE {
+          constexpr int e = decltype(at)::value;
+          if constexpr (GLU) {
+            const float t = sum<acc(2 * e, m) + r>() + (B ? b[0][e] : 0.f);
+            return t / (1.f + expf(-t)) *
+                (sum<acc(2 * e + 1, m) + r>() + (B ? b[GLU][e] : 0.f));
+          } else {
+            return B ? sum<acc(e, m) + r>() + b[0][e] : sum<acc(e, m) + r>();
           }
         };
-        auto with = [&](auto at) INLINE { store(Int<1>{}, at); };
-        auto without = [&](auto at) INLINE { store(Int<0>{}, at); };
-        if (biased) each(std::make_integer_sequence<int, 4 * F>{}, with);
-        else each(std::make_integer_sequence<int, 4 * F>{}, without);
-      }
+        const u32x2 v = {packed2(one(Int<0>{}), one(Int<1>{})),
+                         packed2(one(Int<2>{}), one(Int<3>{}))};
+        if constexpr (GLU)
+          __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, STREAM);
+        else {
+          const u32x2 u = {packed2(one(Int<4>{}), one(Int<5>{})),
+                           packed2(one(Int<6>{}), one(Int<7>{}))};
+          if (N % 8 == 0) {
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4{v[0], v[1], u[0], u[1]},
+                                                   to, o, 0, STREAM);
+          } else {
+            __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, STREAM);
+            __builtin_amdgcn_raw_buffer_store_b64(
+                u, to, n + 4 < N ? o + 8 : NOWHERE, 0, STREAM);
+          }
+        }
+      };
+      auto with = [&](auto at) INLINE { store(Int<1>{}, at); };
+      auto without = [&](auto at) INLINE { store(Int<0>{}, at); };
+      if (biased) each(std::make_integer_sequence<int, 4 * F>{}, with);
+      else each(std::make_integer_sequence<int, 4 * F>{}, without);
     }
-    if (!more) break;
-    at = next;
-    item += slots;
-    more = item + slots < end;
-    if (more) next = locate(item + slots);
-    wover = xover = false;
-    young = 1;
   }
   wait_loads<0>();
 }
@@ -1147,20 +1120,15 @@ int launch(Args a, bool merge, hipStream_t st) {
 
 template <int MODE>
 int launch_wide(Args a, bool merge, hipStream_t st) {
-  constexpr int LDS = 160 * 1024, CUS = 256;
+  constexpr int LDS = 160 * 1024;
   const int items = count<256, 256, MODE>(a);
-  const int steps = MODE == GRAD_X ? a.steps
-      : MODE == GRAD_W ? (a.M + BK - 1) / BK : a.K / BK;
-  // W is loaded up to three stages ahead, into the next tile but not the one
-  // behind it: shorter contractions have a workgroup a tile
-  const int grid = items < CUS || steps / a.splits < 4 ? (items + 7) / 8 * 8 : CUS;
   auto kernel = MODE != SWIGLU && a.splits > 1
       ? wide_linear_kernel<MODE, MODE != SWIGLU>
       : wide_linear_kernel<MODE, false>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (e != hipSuccess) return (int)e;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), LDS, st, a);
+  hipLaunchKernelGGL(kernel, dim3(items), dim3(256), LDS, st, a);
   if (a.splits > 1 && merge) return merge_splits<MODE>(a, st);
   return (int)hipGetLastError();
 }

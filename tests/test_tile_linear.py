@@ -12,6 +12,7 @@ from deepspeed_amd.ops.linear import SWIGLU, Linear, call, tile_linear
 TILES = [(64, 64, 8), (64, 128, 6), (128, 64, 6), (128, 128, 5), (128, 256, 3),
          (192, 128, 4), (192, 256, 2), (256, 128, 3), (256, 192, 2),
          (256, 256, 2)]
+WIDE = len(TILES) - 1
 
 
 def test_calls_left_alone():
@@ -160,16 +161,21 @@ def test_every_tile_backward_gpu(tile):
 @pytest.mark.gpu
 @pytest.mark.parametrize("steps", [2, 3, 4, 5, 9])
 @torch.no_grad()
-def test_widest_tile_goes_on_gpu(steps):
-    """256 x 256: more tiles than workgroups, which go on from tile to tile, over
-    the shortest contractions (of which each has a workgroup) and longer ones."""
+def test_widest_tile_in_rounds_gpu(steps):
+    """256 x 256: more tiles than the chip has CUs, over the shortest contractions
+    and longer ones, in one part and in uneven ones."""
     from deepspeed_amd.ops import _C
-    wide, k = len(TILES) - 1, 64 * steps
+    wide, k = WIDE, 64 * steps
     for m, ns, mode in ((4100, (4360,), 0), (2305, (6148, 516, 264), 0),
                         (2100, (4100, 4100), SWIGLU)):
         x, ws, bs = _inputs(m, ns, k, steps)
         for y, want in zip(_C.tile_linear(x, ws, bs, mode, wide, 1),
                            _want(x, ws, bs, mode)):
+            _close(y, want)
+    for splits in (2, 3):
+        x, ws, bs = _inputs(2305, (4100, 516, 264), 64 * (splits * steps + 1), steps)
+        for y, want in zip(_C.tile_linear(x, ws, bs, 0, wide, splits),
+                           _want(x, ws, bs, 0)):
             _close(y, want)
     for splits in (1, 2):       # dx [4100, 4360] over two layers, dW of as many
         ns = (64 * splits * steps - 64, 64)
