@@ -528,7 +528,8 @@ __device__ __forceinline__ void load(u32x4 from, unsigned off, int soff) {
 // are named, not variables: those the compiler moves to other registers and, as they
 // run out, to memory. It has to have no use for these registers itself (nothing is
 // spilled: 147 to 176 of 256 others are taken). Operands have to be written, and
-// products made, some instructions before they are read.
+// products made, some instructions before they are read. Each build looks through the
+// compiler's assembly for all of this but the products (ops/named_registers.py).
 __device__ __forceinline__ void take_sums() {
   asm volatile("" ::: "a0", "a255");
 }

@@ -3,8 +3,9 @@ registers which they name in inline assembly (csrc/tile_linear.hip). The compile
 knows neither that these hold anything nor what the assembly does, so a build ends
 where its output would not go with it: ``faults`` of every such kernel.
 
-  * An accumulation register outside the kernel's own assembly, a vector register
-    spilled, scratch memory (both are how the compiler would come to take one).
+  * An accumulation register outside the kernel's own assembly, or m0, where its
+    loads to LDS go; a vector register spilled, scratch memory (both are how the
+    compiler would come to take an accumulation register).
   * What the hardware does not wait for and the compiler, which does not read inline
     assembly, does not fill in: a vector register written less than two instructions
     before a product of the assembly reads it, a scalar register written by a vector
@@ -14,14 +15,12 @@ It is run by setup.py and stands alone: no import of the package is needed."""
 
 import re
 import subprocess
-import sys
-
-FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC",
-         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+import tempfile
 
 _KERNEL = re.compile(r"^(\w+):\s*; @\1$")
 _LABEL = re.compile(r"^(\.L\w+):")
 _REGISTER = re.compile(r"\b([asv])(?:(\d+)\b|\[(\w+):(\w+)\])")
+_M0 = re.compile(r"\bm0\b")
 # written by a vector instruction besides its first operand
 _PAIR = re.compile(r"^v_(?:swap|permlane\d+_swap|mad_[ui]64|div_scale|"
                    r"(?:add|sub|subrev)(?:c|b|brev)?_co)")
@@ -133,7 +132,7 @@ def faults(assembly: str):
             if isinstance(b, str):
                 continue
             if not b.own:
-                if any(k == "a" for k, _ in b.all):
+                if any(k == "a" for k, _ in b.all) or _M0.search(b.text):
                     bad.append("%s: %s, outside of the assembly" % (name, b.text))
                 continue
             if "mfma" in b.name:
@@ -147,21 +146,37 @@ def faults(assembly: str):
     return bad, kernels
 
 
-def assembly_of(source: str, hipcc: str = "hipcc"):
-    """The process that writes the source's assembly for the GPU to its output."""
-    return subprocess.Popen(
-        [hipcc, *FLAGS, "--offload-device-only", "-S", source, "-o", "-"],
-        stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
+class assembly_of:
+    """The compiler that writes the source's assembly for the GPU, at work."""
+
+    def __init__(self, source: str, flags, hipcc: str = "hipcc"):
+        # by way of files: a full pipe would hold the compiler up
+        self._out, self._err = tempfile.TemporaryFile(), tempfile.TemporaryFile()
+        self._process = subprocess.Popen(
+            [hipcc, *flags, "-fPIC", "--offload-device-only", "-S", source, "-o",
+             "-"], stdout=self._out, stderr=self._err)
+
+    def text(self) -> str:
+        code = self._process.wait()
+        for f in (self._out, self._err):
+            f.seek(0)
+        if code:
+            raise RuntimeError(self._err.read().decode())
+        return self._out.read().decode()
+
+    def close(self):
+        if self._process.poll() is None:
+            self._process.kill()
+            self._process.wait()
+        self._out.close()
+        self._err.close()
 
 
-def check(process, source: str, kernels: int):
+def check(assembly: assembly_of, source: str, kernels: int):
     """Ends the build where the assembly will not do, or where there are not
     ``kernels`` of these: another way of naming registers would pass unseen."""
-    out, err = process.communicate()
-    if process.returncode:
-        sys.exit("%s: no assembly:\n%s" % (source, err))
-    bad, found = faults(out)
+    bad, found = faults(assembly.text())
     if found != kernels:
         bad.append("%d kernels name registers, not %d" % (found, kernels))
     if bad:
-        sys.exit("\n".join(["%s:" % source] + bad[:20]))
+        raise RuntimeError("\n".join(["%s:" % source] + bad[:20]))

@@ -6,15 +6,45 @@ The resulting deepspeed_amd/ops/_C*.so is git-ignored but ships to the GPU
 box with the repo snapshot.
 """
 
+import importlib.util
 import os
 
 from setuptools import setup
 
 os.environ.setdefault("PYTORCH_ROCM_ARCH", "gfx950")
 
-from torch.utils.cpp_extension import BuildExtension, CUDAExtension  # noqa: E402
+from torch.utils.cpp_extension import (BuildExtension, CUDAExtension,  # noqa: E402
+                                       ROCM_HOME)
 
-CSRC = os.path.join("deepspeed_amd", "ops", "csrc")
+OPS = os.path.join("deepspeed_amd", "ops")
+CSRC = os.path.join(OPS, "csrc")
+
+DEVICE_FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950",
+                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# The source whose kernels name accumulation registers, and how many these are: the
+# build ends where the compiler's assembly does not go with it.
+NAMING, KERNELS = os.path.join(CSRC, "tile_linear.hip"), 7
+
+
+def _named_registers():
+    path = os.path.join(OPS, "named_registers.py")    # without the package
+    spec = importlib.util.spec_from_file_location("named_registers", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
+class Build(BuildExtension):
+    def build_extensions(self):
+        look = _named_registers()
+        hipcc = os.path.join(ROCM_HOME, "bin", "hipcc") if ROCM_HOME else "hipcc"
+        assembly = look.assembly_of(NAMING, DEVICE_FLAGS, hipcc)
+        try:
+            super().build_extensions()
+            look.check(assembly, NAMING, KERNELS)
+        finally:
+            assembly.close()
+
 
 ext = CUDAExtension(
     name="deepspeed_amd.ops._C",
@@ -45,8 +75,7 @@ ext = CUDAExtension(
     ],
     extra_compile_args={
         "cxx": ["-O3", "-std=c++17", "-fopenmp", "-mavx2", "-mfma"],
-        "nvcc": ["-O3", "-std=c++17", "--offload-arch=gfx950",
-                 "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"],
+        "nvcc": DEVICE_FLAGS,
     },
     extra_link_args=["-fopenmp"],
 )
@@ -56,5 +85,5 @@ setup(
     version="0.1.0",
     packages=["deepspeed_amd"],
     ext_modules=[ext],
-    cmdclass={"build_ext": BuildExtension.with_options(use_ninja=True)},
+    cmdclass={"build_ext": Build.with_options(use_ninja=True)},
 )
