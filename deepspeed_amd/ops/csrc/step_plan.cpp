@@ -22,6 +22,7 @@ int64_t as_int(PyObject* o) {
   return v;
 }
 
+struct Blocks { int64_t at, count; };     // of a slot
 struct Run { int64_t row0, rows, keys, blocks; };
 struct Tile { int64_t run, tile, end, splits; };
 
@@ -48,32 +49,33 @@ step_plan(const pybind11::sequence& slots,
   // the rows' places and the runs of neighbours
   std::vector<int64_t> slot(T), offset(T);
   std::vector<int32_t> blocks;
-  std::unordered_map<int64_t, int64_t> first;
+  std::unordered_map<int64_t, Blocks> lists;
+  Blocks list = {0, 0};
   std::vector<Run> runs;
   const py::list rows(slots);
   for (int64_t i = 0; i < T; ++i) {
     PyObject* s = PyList_GET_ITEM(rows.ptr(), i);
     slot[i] = as_int(s);
     const bool same = i && slot[i] == slot[i - 1];
-    if (same) {
-      offset[i] = offset[i - 1];
-    } else {
-      const auto [it, unseen] = first.emplace(slot[i], (int64_t)blocks.size());
-      offset[i] = it->second;
+    if (!same) {
+      const auto [it, unseen] =
+          lists.emplace(slot[i], Blocks{(int64_t)blocks.size(), 0});
       if (unseen) {
         const py::list own(py::object(
             tables[py::reinterpret_borrow<py::object>(s)]));
         for (Py_ssize_t j = 0; j < PyList_GET_SIZE(own.ptr()); ++j)
           blocks.push_back((int32_t)as_int(PyList_GET_ITEM(own.ptr(), j)));
+        it->second.count = (int64_t)blocks.size() - it->second.at;
       }
+      list = it->second;
     }
+    offset[i] = list.at;
+    if (at[i] < 0 || at[i] / block_size >= list.count)
+      throw py::index_error("step_plan: a position outside its slot's blocks");
     if (!same || at[i] != at[i - 1] + 1)
       runs.push_back({i, 0, 0, offset[i]});
     ++runs.back().rows;
   }
-  for (int64_t i = 0; i < T; ++i)
-    if (at[i] < 0 || offset[i] + at[i] / block_size >= (int64_t)blocks.size())
-      throw py::index_error("step_plan: a position outside the blocks");
 
   int64_t most = 0, least = T, work = 0;
   for (auto& r : runs) {

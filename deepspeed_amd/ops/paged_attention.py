@@ -87,7 +87,8 @@ class StepPlan:
     @staticmethod
     def rows(slots: List[int], pos: np.ndarray, tables, block_size: int):
         """Pool row (block * block_size + offset) of every new token, and the
-        block lists of the step's slots, one after another."""
+        block lists of the step's slots, one after another. A position is to lie
+        in its own slot's blocks: the next ones are another request's."""
         used = list(dict.fromkeys(slots))
         lists = [tables[s] for s in used]
         flat = np.fromiter(itertools.chain.from_iterable(lists), np.int32,
@@ -97,6 +98,9 @@ class StepPlan:
             first[s] = at
             at += len(blocks)
         offs = np.array([first[s] for s in slots], np.int64)
+        own = np.array([len(tables[s]) for s in slots], np.int64)
+        if ((pos < 0) | (pos // block_size >= own)).any():
+            raise IndexError("StepPlan: a position outside its slot's blocks")
         dst = flat[offs + pos // block_size].astype(np.int64) * block_size \
             + pos % block_size
         return dst, flat, offs
@@ -124,6 +128,8 @@ class StepPlan:
 def _planned(slots, pos, tables, block_size: int, heads: int, kv_heads: int):
     """``step_plan`` of csrc/step_plan.cpp, for a host without the extension."""
     T = len(slots)
+    if T < 1 or pos.shape != (T,) or block_size < 1 or not 1 <= kv_heads <= heads:
+        raise ValueError("StepPlan: a step of rows, each with its position")
     dst, flat, offs = StepPlan.rows(slots, pos, tables, block_size)
     sl = np.asarray(slots)
     cut = np.flatnonzero((sl[1:] != sl[:-1]) | (pos[1:] != pos[:-1] + 1))

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from deepspeed_amd.inference.ragged import PagedKVCache
-from deepspeed_amd.ops import paged_attention as plans
+from deepspeed_amd.ops import _loader, paged_attention as plans
 from deepspeed_amd.ops.paged_attention import StepPlan
 
 # (slots with the new rows of each, kept tokens by slot)
@@ -60,7 +60,7 @@ def test_splits_fill_whole_rounds(lens, rows, kv_heads):
 @pytest.mark.parametrize("heads", [(8, 8), (14, 2), (32, 8), (16, 1)])
 def test_step_plan_equals_numpys(heads):
     """Single rows and runs of every length, slots that come again, tables of any
-    kind, ties in length and long histories; what is no step is refused."""
+    kind, ties in length and long histories."""
     rng = np.random.default_rng(0)
     seen = set()
     for case in range(200):
@@ -88,10 +88,25 @@ def test_step_plan_equals_numpys(heads):
             (items, runs, merges, any_merge, nq)
         seen.add(nq)
     assert seen >= {2, 8}
-    for slots, pos in (([], []), ([0], [64]), ([0, 1], [1]), ([0], [-1])):
-        with pytest.raises((ValueError, IndexError)):
-            StepPlan.build(slots, np.array(pos, np.int64), {0: [3], 1: []}, 64, 8,
-                           8, "cpu")
+
+
+@pytest.mark.parametrize("slots,pos", [
+    ([], []), ([0], [64]), ([0, 1], [1]), ([0], [-1]), ([0, 2], [0, 128]),
+    # in the next request's blocks, after rows of its own and in a run
+    ([0, 2], [64, 0]), ([0, 2], [100, 0]), ([2, 0, 0], [5, 63, 64])])
+@pytest.mark.parametrize("native", [True, False])
+def test_no_step(slots, pos, native, monkeypatch):
+    """Refused alike with the extension and on a host without it."""
+    if native and _loader.get_ext() is None:
+        pytest.skip("no extension")
+    if not native:
+        monkeypatch.setattr(_loader, "get_ext", lambda: None)
+    pos, tables = np.array(pos, np.int64), {0: [3], 1: [], 2: [7, 8]}
+    with pytest.raises((ValueError, IndexError)):
+        StepPlan.build(slots, pos, tables, 64, 8, 8, "cpu")
+    if len(slots) == len(pos) > 0:
+        with pytest.raises(IndexError):
+            StepPlan.rows(slots, pos, tables, 64)
 
 
 @pytest.mark.parametrize("name", list(STEPS))
