@@ -40,6 +40,11 @@ MIN_SPLIT = 128
 BLOCK, BLOCK_WORK, CUS = 64, 1 << 21, 256
 
 
+def _lines() -> List[int]:
+    """As csrc/step_plan.cpp reads them."""
+    return [ROUND[1], ROUND[2], FEWER, KEYS, MIN_SPLIT, BLOCK, BLOCK_WORK, CUS]
+
+
 def paged_decode_available(q: torch.Tensor, kpool: torch.Tensor) -> bool:
     return (get_ext() is not None and q.is_cuda
             and q.dtype == torch.bfloat16 and q.size(-1) == 128
@@ -115,8 +120,7 @@ class StepPlan:
         args = slots, pos, tables, block_size, heads, kv_heads
         values, items, runs, merges, any_merge, nq, head = _planned(*args) \
             if ext is None else ext.step_plan(
-                *args, [ROUND[1], ROUND[2], FEWER, KEYS, MIN_SPLIT, BLOCK,
-                        BLOCK_WORK, CUS], torch.device(device).type == "cuda")
+                *args, _lines(), torch.device(device).type == "cuda")
         # in the order of the current stream; from pageable memory the host would
         # wait there for all that the stream still has to do, the whole step before
         # (torch gives the pinned block to nobody else before it is read)

@@ -45,22 +45,27 @@ def test_splits_fill_whole_rounds(lens, rows, kv_heads):
     meta = plan.meta.numpy()
     items = meta[:4 * plan.items].reshape(-1, 4)
     merges = meta[4 * (plan.items + plan.runs):][:2 * plan.merges].reshape(-1, 2)
-    tiles = -(-plan.merges * kv_heads // plans.ROUND[plan.nq])
-    assert plan.items * kv_heads <= tiles * plans.ROUND[plan.nq] or \
-        plan.items == plan.merges
+    full = plans.ROUND[plan.nq]
+    ends = [abs(items[f + n - 1][3]) for f, n in merges]
+    if sum(ends) * kv_heads < plans.KEYS * full:
+        full = plans.FEWER
+    tiles = -(-plan.merges * kv_heads // full)
+    assert plan.items * kv_heads <= tiles * full or plan.items == plan.merges
     for first, n in merges:
         at = 0
         for it in items[first:first + n]:
             assert it[2] == at < abs(it[3])
             at = abs(it[3])
-    assert {int(abs(items[f + n - 1][3])) for f, n in merges} >= \
-        {n + 1 for n in lens}
+    assert {*map(int, ends)} >= {n + 1 for n in lens}
 
 
 @pytest.mark.parametrize("heads", [(8, 8), (14, 2), (32, 8), (16, 1)])
 def test_step_plan_equals_numpys(heads):
     """Single rows and runs of every length, slots that come again, tables of any
     kind, ties in length and long histories."""
+    ext = _loader.get_ext()
+    if ext is None:
+        pytest.skip("the native plan is the extension's")
     rng = np.random.default_rng(0)
     seen = set()
     for case in range(200):
@@ -81,7 +86,10 @@ def test_step_plan_equals_numpys(heads):
         if case % 2:
             tables = {s: t.tolist() for s, t in tables.items()}
         args = slots, np.array(pos), tables, bs, *heads
-        want, items, runs, merges, any_merge, nq, head = plans._planned(*args)
+        want, *counts = plans._planned(*args)
+        got, *native = ext.step_plan(*args, plans._lines(), False)
+        assert torch.equal(got, want) and native == counts
+        items, runs, merges, any_merge, nq, head = counts
         plan = StepPlan.build(*args, "cpu")
         assert torch.equal(plan.meta, want) and torch.equal(plan.dst, want[head:])
         assert (plan.items, plan.runs, plan.merges, plan.any_merge, plan.nq) == \
