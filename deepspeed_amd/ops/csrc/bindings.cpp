@@ -720,6 +720,23 @@ std::vector<at::Tensor> tile_linear_grad(
   return out;
 }
 
+// (tile, splits) that tile_linear.hip takes for layers of ns features.
+std::tuple<int64_t, int64_t> tile_linear_plan(const std::vector<int64_t>& ns,
+                                              int64_t M, int64_t K,
+                                              int64_t mode) {
+  TORCH_CHECK(ns.size() >= 1 && ns.size() <= 3 && M > 0 && M < (1 << 30) &&
+              K > 0 && K <= (1 << 22) && mode >= 0 && mode <= 3,
+              "tile_linear_plan: layers");
+  int n[3], splits = 1;
+  for (size_t i = 0; i < ns.size(); ++i) {
+    TORCH_CHECK(ns[i] > 0 && ns[i] <= (1 << 29), "tile_linear_plan: features");
+    n[i] = (int)ns[i];
+  }
+  const int tile = ds_tile_linear_plan(n, (int)ns.size(), (int)M, (int)K,
+                                       (int)mode, &splits);
+  return {tile, splits};
+}
+
 at::Tensor tile_linear_dx(std::vector<at::Tensor> dys,
                           std::vector<at::Tensor> weights, int64_t tile,
                           int64_t splits) {
@@ -1454,6 +1471,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("tile_linear", &tile_linear, "linear layers of many rows, bf16",
         py::arg("x"), py::arg("weights"), py::arg("biases"), py::arg("mode"),
         py::arg("tile") = -1, py::arg("splits") = 1);
+  m.def("tile_linear_plan", &tile_linear_plan,
+        "tile and splits of layers of ns features", pybind11::arg("ns"),
+        pybind11::arg("rows"), pybind11::arg("inputs"), pybind11::arg("mode"));
   m.def("tile_linear_dx", &tile_linear_dx,
         "input's gradient, summed over linear layers", py::arg("dys"),
         py::arg("weights"), py::arg("tile") = -1, py::arg("splits") = 1);

@@ -1134,6 +1134,13 @@ int launch_wide(Args a, bool merge, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+// What the largest tile does not take: outputs are stored at 32-bit offsets in 128
+// rows of ``columns`` sums, and the rows that GRAD_X reads lie behind a descriptor of
+// less than 2^32 bytes, which 256 rows of 2^23 features fill.
+bool past_wide(int mode, double columns, int most) {
+  return columns >= 1 << 22 || (mode == GRAD_X && most >= 1 << 23);
+}
+
 // number, BM, BN, waves along rows and features, stages in LDS; us a stage and
 // a tile of a chip full of them (fitted to 8000 calls in all four modes, of 33 to
 // 8192 rows and 1024 x 1024 to 32000 x 18944; root mean square error 10%). The
@@ -1214,7 +1221,11 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
                                    int mode, int* splits) {
   static const int some[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
   double all = 0;
-  for (int l = 0; l < layers; ++l) all += n[l];
+  int most = 0;
+  for (int l = 0; l < layers; ++l) {
+    all += n[l];
+    most = n[l] > most ? n[l] : most;
+  }
   const int steps = mode == GRAD_X ? (int)(all / BK)
       : mode == GRAD_W ? (M + BK - 1) / BK : K / BK;
   const double rows = mode == GRAD_W ? all : M;
@@ -1224,7 +1235,8 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
   float least = 0;
   for (int i = 0; i < (int)(sizeof(tiles_) / sizeof(Tile)); ++i) {
     const Tile& t = tiles_[i];
-    if (!t.takes(mode) || (i == WIDE && columns >= 1 << 22)) continue;
+    if (!t.takes(mode) || (i == WIDE && past_wide(mode, columns, most)))
+      continue;
     double tiles = 0;
     for (int l = 0; l < layers; ++l)    // SWIGLU: a gate and an up each
       tiles += mode == GRAD_W ? (n[l] + t.bm - 1) / t.bm
@@ -1271,8 +1283,9 @@ extern "C" int ds_tile_linear(const void* const* x, int layers,
                               int mode, int tile, int splits, float* part,
                               int merge, void* stream) {
   Args a = {};
-  int total = 0;
+  int total = 0, most = 0;
   for (int i = 0; i < layers; ++i) {
+    most = n[i] > most ? n[i] : most;
     a.w[i] = (const short*)w[mode == GRAD_W ? 0 : i];
     a.x[i] = (const short*)x[mode >= GRAD_X ? i : 0];
     a.bias[i] = mode >= GRAD_X ? nullptr : (const short*)bias[i];
@@ -1283,8 +1296,7 @@ extern "C" int ds_tile_linear(const void* const* x, int layers,
   a.part = part;
   a.M = M; a.K = K; a.layers = layers; a.splits = splits;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // WIDE stores at 32-bit offsets in 128 rows
-  if (tile == WIDE && (mode >= GRAD_X ? K : total) >= 1 << 22)
+  if (tile == WIDE && past_wide(mode, mode >= GRAD_X ? K : total, most))
     return (int)hipErrorInvalidValue;
   switch (tile) {
 #define X(I, BM, BN, WM, WN, NS, U, F)                                    \

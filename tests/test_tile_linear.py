@@ -6,6 +6,7 @@ import torch
 import torch.nn as nn
 
 from deepspeed_amd.ops import linear as L
+from deepspeed_amd.ops._loader import get_ext
 from deepspeed_amd.ops.linear import SWIGLU, Linear, call, tile_linear
 
 # rows, features and stages of the tiles, in the kernel's order
@@ -21,6 +22,24 @@ def test_calls_left_alone():
     with torch.no_grad():
         assert tile_linear(x, (lin,)) is None      # on the CPU
     assert tile_linear(x, (lin, lin)) is None
+
+
+def test_largest_of_the_widest_tile():
+    """256 x 256 reaches its rows and outputs by 32 bits: 2^23 features of the
+    output's gradient are one too many, as are 2^22 columns stored."""
+    ext = get_ext()
+    if ext is None:
+        pytest.skip("the plan is the extension's")
+    most = 1 << 23
+    assert ext.tile_linear_plan([most - 64], 8192, 4096, 2)[0] == WIDE
+    assert ext.tile_linear_plan([most], 8192, 4096, 2)[0] != WIDE
+    assert ext.tile_linear_plan([4096, most], 8192, 4096, 2)[0] != WIDE
+    assert ext.tile_linear_plan([most], 8192, 4096, 3)[0] == WIDE
+    most = 1 << 22
+    assert ext.tile_linear_plan([most - 8], 8192, 4096, 0)[0] == WIDE
+    assert ext.tile_linear_plan([most], 8192, 4096, 0)[0] != WIDE
+    assert ext.tile_linear_plan([4096], 8192, most - 8, 3)[0] == WIDE
+    assert ext.tile_linear_plan([4096], 8192, most, 3)[0] != WIDE
 
 
 def _inputs(m, ns, k, seed):
