@@ -932,6 +932,23 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> add_norm_fwd(
   return {y, sum, inv};
 }
 
+// own_forward of ops/linear.py, for what Layers::tiled takes.
+bool own_forward(int64_t M, const std::vector<int64_t>& ns, int64_t K,
+                 int64_t mode) {
+  if (M < 2560 || mode == 1) return true;
+  int64_t most = 0, all = 0, tiles = 0;
+  for (const int64_t n : ns) {
+    most = std::max(most, n);
+    all += n;
+    tiles += (M + 255) / 256 * ((n + 255) / 256);
+  }
+  if (ns.size() == 1 && K >= 16384) return all % 4096 != 0;
+  if (ns.size() == 1)
+    return M % 256 != 0 || (all < 65536 && (K < 3072 || tiles % 256 != 0));
+  return M % 256 != 0 || (most * K < (1 << 26) &&
+                          (M < 16384 || 1.0 * M * all * K < 4e11));
+}
+
 // A decoder layer of a serving step over the paged pool, from the residual
 // stream x [.., H] that still lacks the last layer's output delta, to the same:
 // norm, q k v, rotation and append, attention, output, norm, gated MLP. What the
@@ -962,23 +979,11 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
   TORCH_CHECK(!delta || behind || delta->scalar_type() == x.scalar_type(),
               "paged_decoder_layer: delta");
   const int64_t H = x.size(-1), M = x.numel() / H;
-  // as own_forward in ops/linear.py has it
-  auto own_forward = [&](const at::Tensor& in, int first, int count,
-                         int64_t mode) {
-    if (M < 2560 || mode == 1) return true;
-    const int64_t K = in.size(1);
-    int64_t most = 0, all = 0, tiles = 0;
-    for (int i = first; i < first + count; ++i) {
-      const int64_t n = weights[i].numel() / K;
-      most = std::max(most, n);
-      all += n;
-      tiles += (M + 255) / 256 * ((n + 255) / 256);
-    }
-    if (count == 1 && K >= 16384) return all % 4096 != 0;
-    if (count == 1)
-      return M % 256 != 0 || (all < 65536 && (K < 3072 || tiles % 256 != 0));
-    return M % 256 != 0 || (most * K < (1 << 26) &&
-                            (M < 16384 || 1.0 * M * all * K < 4e11));
+  auto own = [&](const at::Tensor& in, int first, int count, int64_t mode) {
+    std::vector<int64_t> ns;
+    for (int i = first; i < first + count; ++i)
+      ns.push_back(weights[i].numel() / in.size(1));
+    return own_forward(M, ns, in.size(1), mode);
   };
   auto linears = [&](const at::Tensor& in, int first, int count,
                      int64_t mode) {
@@ -992,7 +997,7 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
         s.assign(scales.begin() + first, scales.begin() + first + count);
       return rows_linear(in, w, s, b, group, mode);
     }
-    if (!own_forward(in, first, count, mode)) {
+    if (!own(in, first, count, mode)) {
       std::vector<at::Tensor> y;
       for (int i = 0; i < count; ++i) y.push_back(at::linear(in, w[i], b[i]));
       return y;
@@ -1006,7 +1011,7 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
     for (int i = first; i < first + count; ++i)
       all += weights[i].numel() / in.size(1);
     if (!scales.empty() || few_rows(M, all, in.size(1), 0) ||
-        !own_forward(in, first, count, 0))
+        !own(in, first, count, 0))
       return {linears(in, first, count, 0), at::Tensor()};
     Layers y;
     at::Tensor part;
@@ -1525,6 +1530,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         pybind11::arg("into") = c10::nullopt);
   m.def("paged_decoder_layer", &paged_decoder_layer,
         "a decoder layer of a serving step over the paged pool");
+  m.def("own_forward", &own_forward, "which products paged_decoder_layer makes",
+        pybind11::arg("rows"), pybind11::arg("ns"), pybind11::arg("inputs"),
+        pybind11::arg("mode"));
   m.def("paged_layer_fits", &paged_layer_fits,
         "whether paged_decoder_layer takes a layer's tensors");
   m.def("step_plan", &step_plan, "plan of a serving step over the paged pool");

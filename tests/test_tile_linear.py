@@ -381,6 +381,61 @@ def test_own_forward():
         assert not own(t, ns, k) and not own(t, ns * 2, k, SWIGLU)
 
 
+@pytest.mark.parametrize("own,other", [
+    # whole tiles of rows, and one row more
+    ((4097, (4096,), 4096), (4096, (4096,), 4096)),
+    ((4097, (8192, 8192), 8192), (4096, (8192, 8192), 8192)),
+    ((16385, (4096,) * 3, 4096), (16384, (4096,) * 3, 4096)),
+    # whole rounds of tiles and contractions that are not short
+    ((4096, (3840,), 4096), (4096, (4096,), 4096)),
+    ((4096, (4096,), 3008), (4096, (4096,), 3072)),
+    # vocabularies
+    ((4096, (65280,), 4096), (4096, (65536,), 4096)),
+    # the largest of several, their rows and their products
+    ((4096, (8128, 8128), 8192), (4096, (8192, 8192), 8192)),
+    ((16128, (4096,) * 3, 4096), (16384, (4096,) * 3, 4096)),
+    ((16384, (2048,) * 2, 4096), (16384, (4096,) * 2, 4096)),
+])
+def test_lines_of_forward(own, other):
+    assert L.own_forward(*own) and not L.own_forward(*other)
+
+
+@pytest.mark.parametrize("own,other", [
+    # whole tiles of rows, and one row more
+    ((8193, (14336,), 4096), (8192, (14336,), 4096)),
+    ((8193, (14336,) * 2, 4096), (8192, (14336,) * 2, 4096)),
+    # a bit more than a round of tiles, but for many features
+    ((8160, (14336,), 2048), (8200, (14336,), 2048)),
+    ((12700, (14336,), 2048), (12500, (14336,), 2048)),
+    ((10000, (28672,), 2048), (10000, (28608,), 2048)),
+    ((8160, (11008,) * 2, 2048), (10000, (11008,) * 2, 2048)),
+])
+def test_lines_of_dx(own, other):
+    assert L.own_dx(*own) and not L.own_dx(*other)
+
+
+def test_both_copies_of_forward():
+    """A serving step's native layer and the modules make the same products."""
+    ext = get_ext()
+    if ext is None:
+        pytest.skip("the copy is the extension's")
+    rows = [33, 2559, 2560, 2561, 3840, 4095, 4096, 8192, 16128, 16383, 16384,
+            16385, 32768, 100000]
+    widths = [4, 256, 1024, 3072, 4096, 4100, 8192, 12288, 16384, 28672, 65280,
+              65532, 65536, 128256]
+    inputs = [192, 1024, 3008, 3072, 4096, 8192, 16320, 16384, 28672, 1 << 22]
+    seen = set()
+    for t in rows:
+        for n in widths:
+            for ns in ((n,), (n, n), (n, 1024, 1024), (n,) * 3):
+                for k in inputs:
+                    for mode in (0, 1) if len(ns) == 2 else (0,):
+                        want = L.own_forward(t, ns, k, mode)
+                        assert ext.own_forward(t, ns, k, mode) == want, (t, ns, k)
+                        seen.add((len(ns), want))
+    assert len(seen) == 6
+
+
 @pytest.mark.parametrize("t,ns,k,want", [
     (12288, (4096, 1024, 1024), 4096, [3]),
     (14000, (4096, 1024, 1024), 4096, [1, 1, 1]),
