@@ -942,7 +942,9 @@ bool own_forward(int64_t M, const std::vector<int64_t>& ns, int64_t K,
     all += n;
     tiles += (M + 255) / 256 * ((n + 255) / 256);
   }
-  if (ns.size() == 1 && K >= 16384) return all % 4096 != 0;
+  if (ns.size() == 1 && K >= 16384)
+    return all % 4096 != 0 || (all < 16384 && M % 256 != 0) ||
+        (all < 8192 && tiles % 256 != 0);
   if (ns.size() == 1)
     return M % 256 != 0 || (all < 65536 && (K < 3072 || tiles % 256 != 0));
   return M % 256 != 0 || (most * K < (1 << 26) &&

@@ -155,28 +155,33 @@ def own_forward(T: int, ns, K: int, mode: int = PLAIN) -> bool:
     """Whether the forward product of layers of ``ns`` features is
     csrc/tile_linear.hip's. Over 20 layers of 1024 x 1024 to 128256 x 4096 and 33 to
     8192 rows the kernel takes 0.65 of the library's time in the geometric mean (us,
-    library and kernel: gate and up 14336, K 4096, 224 rows 95 + activation / 67;
-    4096, K 14336, 1024 rows 138 / 108; 3584, K 18944, 2331 rows 489 / 302).
+    library and kernel: gate and up 14336, K 4096, 224 rows 86 + activation / 57;
+    4096, K 14336, 1024 rows 114 / 104; 3584, K 18944, 2331 rows 495 / 256).
 
-    From 2560 rows on, over 2700 layers and rows: 0.92 of the library's time for one
+    From 2560 rows on, over 1000 layers and rows: 0.95 of the library's time for one
     layer, but where 256 x 256 tiles fill whole rounds of the 256 CUs and contractions
-    are long, the library is ahead (4096 rows: N 4096, K 14336 295 / 307; 8192 rows: N
-    14336, K 4096 628 / 644; else N 3072, K 4096, 4096 rows 80 / 76, 8192 126 / 117 at K
+    are long, the library is ahead (4096 rows: N 4096, K 14336 351 / 385; 8192 rows: N
+    14336, K 4096 644 / 675; else N 3072, K 4096, 4096 rows 81 / 78, 8192 127 / 120 at K
     3072), and from 65536 features on whole tiles of rows are within 2% either way
-    (128256, K 4096, 4096 rows 2970 / 2930). K from 16384 on: but for whole rounds
-    (geometric mean over 2560 to 16384 rows by the kernel before, library 1: N 3584
-    0.71, 5120 0.85, 4096 1.05, 8192 1.01). Several layers, over 1500: 0.86 (3 of 3072, K 3072, 8192 rows 370 /
-    330; 2 of 11008, K 4096, 8192 rows 1285 / 973), but not large ones of whole tiles of
-    rows (2 of 8192, K 14336, 4096 rows 1223 / 1257) nor, from 16384 of these on, many
-    products (3 of 4096, K 4096: 16384 rows 1063 / 1090); gate and up with their
-    activation stay (14336, K 4096, 8192 rows 1240 + activation / 1290)."""
+    (128256, K 4096, 4096 rows 3016 / 2961). K from 16384 on, over 1400: 0.84 of it, but
+    for features in 4096s, which the library's tiles fill best: 4096 of them 0.83
+    (4352 rows, K 16384 869 / 456) but in whole rounds (4096 rows, K 16384 354 / 384), 8192
+    0.96 and 12288 0.98 but of whole tiles of rows (both 1.00), more 1.02 (8192 rows N
+    24576, K 16384 4198 / 4533).
+    Several layers, over 1200: 0.80 (3 of 3072, K 3072, 8192 rows 372 / 340; 2 of 11008,
+    K 4096, 8192 rows 1306 / 976), but whole tiles of rows of large ones are the
+    library's (2 of 8192, K 14336, 4096 rows 1231 / 1286, though over 137 the kernel
+    takes 0.87), as are, from 16384 of these on, many products (3 of 4096, K 4096:
+    16384 rows 1084 / 1114); gate and up with their activation stay (14336, K 4096,
+    8192 rows 1260 + activation / 1379)."""
     if T <= ROWS or K % 64 or not 192 <= K <= INPUTS or any(n % 4 for n in ns):
         return False
     if T < 2560 or mode == SWIGLU:
         return True
     if len(ns) == 1:
         if K >= 16384:
-            return ns[0] % 4096 != 0
+            return ns[0] % 4096 != 0 or (ns[0] < 16384 and T % 256 != 0) or (
+                ns[0] < 8192 and _tiles(T, ns) % 256 != 0)
         return T % 256 != 0 or ns[0] < 65536 and (
             K < 3072 or _tiles(T, ns) % 256 != 0)
     return T % 256 != 0 or max(ns) * K < 1 << 26 and (

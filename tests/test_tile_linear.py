@@ -389,6 +389,12 @@ def test_own_forward():
     # whole rounds of tiles and contractions that are not short
     ((4096, (3840,), 4096), (4096, (4096,), 4096)),
     ((4096, (4096,), 3008), (4096, (4096,), 3072)),
+    # long contractions: features in 4096s
+    ((4096, (24640,), 16384), (4096, (24576,), 16384)),
+    ((4097, (12288,), 16384), (4096, (12288,), 16384)),
+    ((4097, (12288,), 16384), (4097, (16384,), 16384)),
+    ((3840, (4096,), 16384), (4096, (4096,), 16384)),
+    ((3840, (4096,), 16384), (3840, (8192,), 16384)),
     # vocabularies
     ((4096, (65280,), 4096), (4096, (65536,), 4096)),
     # the largest of several, their rows and their products
