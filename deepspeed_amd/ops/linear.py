@@ -86,20 +86,21 @@ def own_dx(T: int, ns, K: int) -> bool:
     is csrc/tile_linear.hip's, which adds the layers up in one product (us, library
     with the copies of ``backward_plan`` and additions, and kernel).
 
-    N 14336, K 4096, 1000 rows 128 / 110, 2300 251 / 246; 18944, K 3584, 2048 rows
-    348 / 223; 32064, K 3072, 2559 rows 608 / 409; 3072, K 8192, 1024 rows 53 / 50.
-    From 2560 rows on, over 3400 layers and rows, the library is ahead past 7e10
-    products where the rows are whole tiles of 256 (14336, K 4096: 4096 rows 343 / 340,
-    8192 637 / 692; 4096, K 4096, 8192 rows 192 / 202; 14336, K 3072, 8192 544 / 619),
-    but for features many times the inputs up to 1.7e11. Elsewhere the kernel is, by
-    5% in the geometric mean (128256, K 3072, 4000 rows 4160 / 2676; 3072, K 8192 158 /
-    153), but not where it has a bit more than a round of tiles (14336, K 2048, 10000
-    rows 459 / 593), if there are not too many features.
-    Several layers, over 1900: 0.83 of the library's time, whose additions count for
-    less the more features there are (4096 + 2 of 1024, K 4096: 8192 rows 383 / 297; 3
-    of 3072, K 8192: 4096 rows 546 / 437; whole tiles of rows and 2 of 14336, K 4096:
-    4096 rows 712 / 695, 8192 1332 / 1396; 2 of 8192, K 3072, 8192 655 / 683; a bit more
-    than a round of tiles: 2 of 11008, K 2048, 10000 rows 730 / 914)."""
+    N 14336, K 4096, 1000 rows 148 / 121, 2300 290 / 259; 18944, K 3584, 2048 rows
+    343 / 233; 32064, K 3072, 2559 rows 594 / 401; but 3072, K 8192, 1024 rows 51 / 52.
+    From 2560 rows on the library is ahead past 7e10 products where the rows are whole
+    tiles of 256 (14336, K 4096: 4096 rows 348 / 355, 8192 643 / 719; 4096, K 4096,
+    8192 rows 192 / 207; 14336, K 3072, 8192 544 / 621; over 508 of these the kernel
+    takes 0.96 all the same, since the library's times jump between neighbouring
+    layers), but for features many times the inputs up to 1.7e11.
+    Elsewhere the kernel is, by 7% in the geometric mean (128256, K 3072, 4000 rows
+    4175 / 2727; 3072, K 8192 155 / 158), but not where it has a bit more than a round
+    of tiles (14336, K 2048, 10000 rows 458 / 600), if there are not too many features.
+    Several layers, over 1200: 0.75 of the library's time, whose additions count for
+    less the more features there are (4096 + 2 of 1024, K 4096: 8192 rows 422 / 339; 3
+    of 3072, K 8192: 4096 rows 550 / 443; whole tiles of rows and 2 of 14336, K 4096:
+    4096 rows 715 / 694, 8192 1316 / 1402; 2 of 8192, K 3072, 8192 667 / 697; a bit more
+    than a round of tiles: 2 of 11008, K 2048, 10000 rows 729 / 882)."""
     if T <= ROWS or T >= 1 << 30 or K % 8 or K > INPUTS:
         return False
     for n in ns:
@@ -121,12 +122,16 @@ def own_dx(T: int, ns, K: int) -> bool:
 def own_dw(T: int, N: int, K: int) -> bool:
     """Whether the gradient of a weight [N, K] over T rows is
     csrc/tile_linear.hip's (us, library with the copies of ``backward_plan`` and
-    kernel): 4096, K 4096, 4000 rows 126 / 103; 14336, K 4096, 4000 rows 437 / 398,
-    6144 573 / 598, 7000 687 / 667, 8192 767 / 796, 10000 1148 / 970, 32768 3529 /
-    3265; 3072, K 3072, 4000 rows 100 / 78, 24576 411 / 438; but 128256, K 4096, 8192
-    rows 6289 / 6630 (4000 rows 3454 / 3324)."""
+    kernel): 4096, K 4096, 4000 rows 138 / 108; 14336, K 4096, 4000 rows 443 / 368,
+    6144 576 / 528, 8192 759 / 737, 10000 1147 / 901, 32768 3544 / 2990; 3072, K 3072,
+    4000 rows 108 / 78, 24576 447 / 419; 32064, K 8192, 16384 rows 6789 / 6191. Over
+    1200 layers and rows from 2560 on 0.87 of the library's time, 1.09 at most. The
+    library keeps where the two are closest, vocabularies over many whole tiles of
+    rows (0.96 over 44; 128256, K 4096, 8192 rows 6460 / 6284, but of other numbers of
+    rows 0.90)."""
     return T > 192 and N % 8 == 0 and K % 8 == 0 and T < 1 << 30 and \
-        N <= FEATURES and K <= INPUTS and (T < 6144 or N * K < 1 << 28)
+        N <= FEATURES and K <= INPUTS and (
+            T < 6144 or T % 256 != 0 or N < 65536 or N * K < 1 << 28)
 
 
 def own_products(T: int, N: int, K: int):
@@ -140,12 +145,14 @@ def own_products(T: int, N: int, K: int):
 def one_dw(T: int, ns, K: int) -> bool:
     """Whether the weights' gradients of several layers over T rows are one launch.
     Not where that is a bit more than a round of the 256 CUs over operands past the
-    256 MB that the chip caches: the second round is then as long as the first (us,
-    one launch, one each, library: 4096 + 2 of 1024, K 4096, 384 tiles: 12288 rows
-    525 / 530 / 574, 14000 702 / 544 / 718, 32768 1718 / 1217 / 1434; 3 of 3072, K
-    2048, 288 tiles: 10000 348 / 351 / 434, 16384 704 / 544 / 682; 4096 + 2 of 512, K
-    4096, 320 tiles: 16384 605 / 559 / 712; but 4096 + 2 of 1536, 448 tiles: 16384 739
-    / 757 / 894; 5120 + 2 of 1024, K 5120, 560 tiles: 16384 954 / 1096 / 1549)."""
+    256 MB that the chip caches: the second round is then as long as the first. Over
+    400 layers and rows past that size one launch takes, of the time of one each, 1.10
+    at up to 288 tiles, 1.12 to 320, 1.03 to 352, 0.99 to 400, 0.89 to 480 and 0.9 from
+    there (us, one launch, one each, library: 4096 + 2 of 1024, K 4096, 384 tiles: 14000
+    rows 597 / 526 / 765, 32768 1456 / 1185 / 1499; 3 of 3072, K 2048, 288 tiles: 10000
+    363 / 355 / 453, 16384 602 / 556 / 709; 4096 + 2 of 512, K 4096, 320 tiles: 16384
+    612 / 539 / 714; but 4096 + 2 of 1536, 448 tiles: 16384 739 / 758 / 925; 5120 + 2 of
+    1024, K 5120, 560 tiles: 16384 971 / 1035 / 1531)."""
     if 2 * T * (K + sum(ns)) <= 1 << 28:
         return True
     return not 256 < sum(-(-n // 256) for n in ns) * -(-K // 256) < 400

@@ -420,6 +420,14 @@ def test_lines_of_dx(own, other):
     assert L.own_dx(*own) and not L.own_dx(*other)
 
 
+def test_lines_of_dw():
+    """The library's: vocabularies over many whole tiles of rows."""
+    assert L.own_dw(8193, 128256, 4096) and not L.own_dw(8192, 128256, 4096)
+    assert L.own_dw(5888, 65536, 4096) and not L.own_dw(6144, 65536, 4096)
+    assert L.own_dw(6144, 65528, 8192) and not L.own_dw(32768, 65536, 8192)
+    assert L.own_dw(32768, 128256, 2048)
+
+
 def test_both_copies_of_forward():
     """A serving step's native layer and the modules make the same products."""
     ext = get_ext()
