@@ -383,6 +383,16 @@ __global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
 // and 16 30.6 / 28.1, 35.4 / 29.7; 128256, K 4096 bf16 163 / 164, 186 / 174, 208 /
 // 181, int8 96 / 87, 112 / 92, 134 / 99; 9216, K 3072 bf16 14.3 / 12.8, 16.7 / 13.6, 18.2
 // (12 rows) / 14.2. Now 5.2 to 6.3 TB/s of W where it is large.
+//
+// A workgroup's tiles are fixed at the launch and it takes a CU whole: where another
+// stream's kernel holds CUs and the workgroups are more than those left, some begin when
+// the first others end (us, few_rows_kernel / here, 8 rows, weights from memory, alone
+// and with 8 CUs held: 128256, K 4096 bf16 190 / 174 and 210 / 274, int8 128 / 97 and 132
+// / 152; 28672 bf16 51 / 42 and 54 / 65; but gate and up 14336, 224 workgroups, 45 / 42
+// and 46 / 41). Of the framework only ZeRO-3's gathers run beside such layers, and are
+// many times as long; a serving step's collectives wait for it and it for them. With
+// workgroups for 224 CUs nothing is lost where 8 are held, but alone 0 to 17% (int8
+// 32000, K 4096 28.4 / 32.3, 16384 16.6 / 19.5, bf16 12288 20.0 / 21.9, 128256 none).
 template <bool I8, int MODE, int FT, int X>
 __global__ __launch_bounds__(NW * 64, 2) void going_rows_kernel(const Args a,
                                                                 int tiles) {

@@ -1157,9 +1157,12 @@ bool past_wide(int mode, double columns, int most) {
   X(7, 256, 128, 4, 2, 3, 0.754f, 5.2f)    \
   X(8, 256, 192, 2, 4, 2, 1.023f, 6.3f)
 constexpr int WIDE = 9;
-// 192 x 192, for what lies between the rounds of the others (us, the earlier choice /
-// this, over 150 layers that it is chosen for 0.89 forward, 0.92 backward, at worst
-// 1.1): 2331 rows 3584, K 4096 62.4 / 57.7, K 18944 291 / 272; 573 rows 14336, K 3584
+// 192 x 192, for what lies between the rounds of the others (us, the choice without it /
+// this; over 500 layers that it is chosen for 0.94 of one's or several layers' forward,
+// 0.88 of gate and up, 0.97 of the input's gradient and 0.93 of the weights', 22 of them
+// more than 5% and at worst 20% slower, 185 rows of 32000 + 2 of 8000, K 16384, as
+// other tiles' are that the estimate does not hold for; taken for a lead of 2.5% and
+// more only, it would gain 0.2%): 2331 rows 3584, K 4096 62.4 / 57.7, K 18944 291 / 272; 573 rows 14336, K 3584
 // 60.2 / 50.3, gate and up of 543, K 4096 128 / 111; 1524 rows 11008, K 4096 127 / 109;
 // 540 rows 32000, K 4096 157 / 132. The input's gradient, whose W is read across, takes
 // a little more than its terms say (3000 rows, n 32000, K 3072 in three splits of 256 x
@@ -1215,8 +1218,9 @@ float estimate(const Tile& t, double tiles, int steps, double rows,
 
 // The tile for 1..3 weights on one input and the splits of the contraction, by
 // ``estimate``: over those calls 0.6% over the fastest on average, 0.9% for the
-// input's gradient (4.4% by an earlier fit). Each split needs the ring's stages. -1:
-// no tile for this K.
+// input's gradient (4.4% by an earlier fit). Each split needs the ring's stages. The
+// addition of the splits is counted also where the next kernel makes it as it reads
+// them. -1: no tile for this K.
 extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
                                    int mode, int* splits) {
   static const int some[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
