@@ -1109,7 +1109,12 @@ int launch(Args a, bool merge, hipStream_t st) {
   // 82, gate and up 14336, K 4096 54.9 / 42.6, 11008 43.0 / 36.5; 128 rows 128256 222 /
   // 197, 32000 63 / 51; 224 rows 32000 73 / 69, gate and up 14336 65.2 / 64.4; even at
   // K 3072, 4608 and 5120. Other steps than 13 and 7 leave 18432, K 4096 at 43 to 52.
-  a.turn = a.mtiles == 1 && a.splits == 1 && a.K * 2 % 4096 == 0;
+  // But each is at another place of x then, all of which has to stay in an XCD's 4 MB
+  // of L2 beside W's stream. Of the time of beginning together, over 7000 layers with
+  // weights from memory: x up to 1 MB 0.90, to 1.5 0.92, to 2 0.96, to 2.5 0.99, to 3
+  // 1.02, to 4 1.07, to 6 1.15, more 1.22 (256 rows 32064, K 16384 255 / 459 us).
+  a.turn = a.mtiles == 1 && a.splits == 1 && a.K * 2 % 4096 == 0 &&
+      (long long)a.M * a.K <= 1 << 20;
   auto kernel = tile_linear_kernel<BM, BN, WM, WN, NS, MODE>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);

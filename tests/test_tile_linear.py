@@ -214,11 +214,12 @@ def test_widest_tile_in_rounds_gpu(steps):
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,ns,k,mode,tile", [
     (40, (20000,), 2048, 0, 0), (33, (9000, 9000), 4096, SWIGLU, 1),
-    (100, (8200, 4100), 2048, 0, 3), (190, (16396,), 4096, 0, 6)])
+    (100, (8200, 4100), 2048, 0, 3), (190, (16396,), 4096, 0, 6),
+    (128, (8196,), 8192, 0, 3), (129, (8196,), 8192, 0, 6)])
 @torch.no_grad()
 def test_one_tile_of_rows_gpu(m, ns, k, mode, tile):
     """Rows of whole multiples of 4 KB: every workgroup begins elsewhere in them,
-    and comes to all of them."""
+    and comes to all of them; up to 2 MB of x, and past them."""
     from deepspeed_amd.ops import _C
     x, ws, bs = _inputs(m, ns, k, m)
     for y, want in zip(_C.tile_linear(x, ws, bs, mode, tile, 1),
