@@ -1167,13 +1167,28 @@ constexpr int WIDE = 9;
 // 0.88 of gate and up, 0.97 of the input's gradient and 0.93 of the weights', 22 of them
 // more than 5% and at worst 20% slower, 185 rows of 32000 + 2 of 8000, K 16384, as
 // other tiles' are that the estimate does not hold for; taken for a lead of 2.5% and
-// more only, it would gain 0.2%): 2331 rows 3584, K 4096 62.4 / 57.7, K 18944 291 / 272; 573 rows 14336, K 3584
-// 60.2 / 50.3, gate and up of 543, K 4096 128 / 111; 1524 rows 11008, K 4096 127 / 109;
-// 540 rows 32000, K 4096 157 / 132. The input's gradient, whose W is read across, takes
-// a little more than its terms say (3000 rows, n 32000, K 3072 in three splits of 256 x
-// 256 508, in this 549).
+// more only, it would gain 0.2%): 2331 rows 3584, K 4096 62.4 / 57.7, K 18944 291 /
+// 272; 573 rows 14336, K 3584 60.2 / 50.3, gate and up of 543, K 4096 128 / 111; 1524
+// rows 11008, K 4096 127 / 109; 540 rows 32000, K 4096 157 / 132. The input's gradient,
+// whose W is read across, takes a little more than its terms say (3000 rows, n 32000, K
+// 3072 in three splits of 256 x 256 508, in this 549).
 constexpr int SQUARE = 10;
 #define BETWEEN(X) X(SQUARE, 192, 192, 4, 2, 3, 0.804f, 6.3f)
+// The largest tile by eight waves, two a SIMD: a short contraction is as much its first
+// loads and its stores, which the waves make beside each other's products. In place of
+// WIDE up to so many stages. Over 7000 layers, of the four waves' time: gate and up
+// 0.98 at 8, 0.99 to 32, then even; the input's gradient 0.93 at 8, 0.98 at 16 and 1.02
+// at 32; the weights', of 5120 and more columns, 0.89 to 4, 0.93 to 8, 0.97 to 12, 0.99
+// to 16 and 1.02 from there. Gradients of fewer than 3072 columns are even or lose (K
+// 1536 1.00, 2048 1.07), and of columns that are a power of two, whose rows' stores meet
+// in the same memory channels (4096 1.05, 8192 1.02, 16384 0.99, but 3584 0.97). PLAIN,
+// whose outputs go through LDS here, 1.10 at 8 and 1.06 from 24 on: never.
+constexpr int EIGHT = 11;
+bool short_contraction(int mode, int stages, int columns) {
+  static const int most[] = {0, 24, 16, 12};    // by mode
+  return stages <= most[mode] &&
+      (mode == SWIGLU || (columns >= 3072 && (columns & (columns - 1))));
+}
 
 // A wave's gate and up tiles in pairs; halves of x in blocks of 64 columns.
 #define GATES(BN, WN) (BN / WN / 16 % 2 == 0)
@@ -1183,8 +1198,10 @@ struct Tile {
   int bm, bn, stages;
   bool gates, blocks;
   float stage, fixed;
+  bool plain = true;
   bool takes(int mode) const {
-    return (gates || mode != SWIGLU) && (blocks || mode != GRAD_W);
+    return (gates || mode != SWIGLU) && (blocks || mode != GRAD_W) &&
+        (plain || mode != PLAIN);
   }
 };
 const Tile tiles_[] = {
@@ -1193,6 +1210,7 @@ const Tile tiles_[] = {
     TILES(X)
     {256, 256, 2, true, true, 1.149f, 8.8f},    // WIDE
     BETWEEN(X)
+    {256, 256, 2, true, true, 0, 0, false},     // EIGHT
 #undef X
 };
 
@@ -1242,7 +1260,7 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
   const double bytes = 2 * (all * K + (double)M * (K + all));
   int best = -1;
   float least = 0;
-  for (int i = 0; i < (int)(sizeof(tiles_) / sizeof(Tile)); ++i) {
+  for (int i = 0; i < EIGHT; ++i) {
     const Tile& t = tiles_[i];
     if (!t.takes(mode) || (i == WIDE && past_wide(mode, columns, most)))
       continue;
@@ -1266,6 +1284,7 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
       }
     }
   }
+  if (best == WIDE && short_contraction(mode, steps / *splits, K)) return EIGHT;
   return best;
 }
 
@@ -1322,6 +1341,11 @@ extern "C" int ds_tile_linear(const void* const* x, int layers,
     TILES(X)
     BETWEEN(X)
 #undef X
+  case EIGHT:
+    if (mode == GRAD_X) return launch<256, 256, 2, 4, 2, GRAD_X>(a, merge, st);
+    if (mode == GRAD_W) return launch<256, 256, 2, 4, 2, GRAD_W>(a, merge, st);
+    if (mode == SWIGLU) return launch<256, 256, 2, 4, 2, SWIGLU>(a, merge, st);
+    break;
   case WIDE:
     if (mode == GRAD_X) return launch_wide<GRAD_X>(a, merge, st);
     if (mode == GRAD_W) return launch_wide<GRAD_W>(a, merge, st);

@@ -238,6 +238,44 @@ def test_square_tile_gpu(rows, monkeypatch):
         test_every_tile_gpu(len(TILES) - 1, rows)
 
 
+def test_short_contractions():
+    """256 x 256 by eight waves where the contraction, or a part of it, is short."""
+    ext = get_ext()
+    if ext is None:
+        pytest.skip("the plan is the extension's")
+    plan = ext.tile_linear_plan
+    eight = len(TILES) + 1
+    assert plan([14336] * 2, 8192, 1536, SWIGLU)[0] == eight
+    assert plan([14336] * 2, 8192, 1600, SWIGLU)[0] == WIDE
+    assert plan([1024], 8192, 14336, 2)[0] == eight
+    assert plan([512, 576], 8192, 14336, 2)[0] == WIDE
+    assert plan([14336], 768, 14336, 3)[0] == eight
+    assert plan([14336], 769, 14336, 3)[0] == WIDE
+    assert plan([14336], 8192, 512, 0)[0] != eight
+    for k in (2560, 4096, 8192):      # few columns, and powers of two
+        assert plan([32000], 768, k, 3)[0] == WIDE
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", [SWIGLU, 2])
+def test_short_contractions_gpu(mode, monkeypatch):
+    """256 x 256 by eight waves, as the tiles before it."""
+    from deepspeed_amd.ops import _C
+    eight = len(TILES) + 1
+    monkeypatch.setitem(globals(), "TILES",
+                        TILES + [(192, 192, 3), (256, 256, 2)])
+    if mode != SWIGLU:
+        return test_every_tile_backward_gpu(eight)
+    for rows in (-1, 0, 1):
+        for n in (132, 256):
+            for steps in (2, 3, 7):
+                x, ws, bs = _inputs(256 + rows, (n, n), 64 * steps, steps)
+                _close(_C.tile_linear(x, ws, bs, SWIGLU, eight, 1)[0],
+                       _want(x, ws, bs, SWIGLU)[0])
+    with pytest.raises(RuntimeError):
+        _C.tile_linear(x, ws, bs, 0, eight, 1)
+
+
 @pytest.mark.gpu
 def test_what_lies_past_the_last_row_gpu():
     """Rows past the end count for nothing, whatever the last one holds: each
