@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <unordered_map>
+#include <utility>
 #include <vector>
 
 namespace {
@@ -30,8 +31,9 @@ struct Tile { int64_t run, tile, end, splits; };
 
 // slots and pos: request slot and position of every row; tables[slot]: its blocks.
 // lines: ROUND of one and of two tiles, FEWER, KEYS, MIN_SPLIT, BLOCK, BLOCK_WORK,
-// CUS. -> (int32 values on the host: items, runs, merges, blocks, places of the
-// rows; items, runs, merges, whether any history is split, nq, index of the places).
+// CUS, WORKGROUPS, LONG. -> (int32 values on the host: items, runs, merges, blocks,
+// places of the rows; items, runs, merges, whether any history is split, nq, index of
+// the places).
 std::tuple<at::Tensor, int64_t, int64_t, int64_t, bool, int64_t, int64_t>
 step_plan(const pybind11::sequence& slots,
           pybind11::array_t<int64_t, pybind11::array::c_style |
@@ -41,7 +43,7 @@ step_plan(const pybind11::sequence& slots,
   namespace py = pybind11;
   const int64_t T = py::len(slots), G = kv_heads > 0 ? heads / kv_heads : 0;
   if (T < 1 || pos.ndim() != 1 || pos.size() != T || block_size < 1 || G < 1 ||
-      lines.size() != 8)
+      lines.size() != 10)
     throw py::value_error("step_plan: a step of rows, each with its position");
   const int64_t* at = pos.data();
   const int64_t min_split = lines[4];
@@ -121,14 +123,34 @@ step_plan(const pybind11::sequence& slots,
       while (per < longest && splits(per) > room) per += min_split;
     }
     splits(per);
-  } else {
+  } else if (n * kv_heads < lines[8]) {
     int64_t full = lines[nq - 1];
-    if (total * kv_heads < lines[3] * full) full = lines[2];
+    const int64_t fewer = lines[2];
+    if (total * kv_heads < lines[3] * full) full = fewer;
     const int64_t room = ceil_div(n * kv_heads, full) * full / kv_heads;
     // half a split more for each tile, where it ends unevenly
     int64_t per = std::max(min_split,
                            total / std::max<int64_t>(1, room - n / 2));
     while (splits(per) > std::max(room, n)) per += per / 16;
+    // keys of the longest part, and rounds of two tiles' workgroups
+    auto rounds = [&] {
+      int64_t longest = 0, count = 0;
+      for (auto& t : tiles) {
+        longest = std::max(longest, ceil_div(t.end, t.splits));
+        count += t.splits;
+      }
+      return std::make_pair(longest, ceil_div(count * kv_heads, fewer));
+    };
+    if (nq == 2) {
+      const auto [longest, k] = rounds();
+      if (k > 1 && longest > lines[9] &&
+          10 * total * kv_heads < 7 * k * fewer * longest) {
+        const auto before = tiles;
+        splits(std::max(min_split, total * kv_heads / lines[8]));
+        const auto [longest2, k2] = rounds();
+        if (longest2 * k2 >= longest * k) tiles = before;
+      }
+    }
   }
   int64_t items = 0;
   bool any = false;

@@ -15,9 +15,8 @@ import torch
 from . import _loader
 from ._loader import get_ext
 
-# Workgroups wanted in flight where the lengths stay on the device: four waves each,
-# two to three to a CU of 256. More splits than that only add partial results to
-# write and merge.
+# Workgroups wanted in flight: four waves each, two to three to a CU of 256. More splits
+# than that only add partial results to write and merge.
 WORKGROUPS = 1024
 # Where they are known, splits fill whole rounds of the workgroups that the 256 CUs
 # hold, three each of one tile of columns: a few more would begin when the others end,
@@ -28,6 +27,15 @@ WORKGROUPS = 1024
 # than it reads (1 x 16000 27.0 / 21.1, 64 x 500 34.9 / 30.9, 15 of 200 and 250 rows
 # 23.9 / 19.5).
 ROUND, FEWER, KEYS = {1: 768, 2: 1024}, 512, 384
+# But WORKGROUPS tiles and more stay whole, however their last round is filled (over 257
+# steps of two tiles of columns, splits that fill it 1.05 of the time, 1.36 at worst; 93
+# rows behind 382 beside 9 of as many, 32 key heads 50 / 39 us). And where rounds of two
+# tiles' workgroups, as long as the longest of them, hold less than 0.7 of what they
+# could, such as evenly long histories that do not fit in twice, parts of more than LONG
+# keys are cut for WORKGROUPS if that is less by this measure (65 of 4600 steps, 0.91 of
+# the time, 1.01 at worst; from 1024 keys on 91, 1.08 at worst; 319 rows behind 16000
+# beside 2 of as many 605 / 482).
+LONG = 2048
 # Keys of the shortest split: one tile of 32 for each of a workgroup's waves.
 MIN_SPLIT = 128
 # Items of 128 columns (rows times heads a key head), eight waves of them a CU,
@@ -42,7 +50,8 @@ BLOCK, BLOCK_WORK, CUS = 64, 1 << 21, 256
 
 def _lines() -> List[int]:
     """As csrc/step_plan.cpp reads them."""
-    return [ROUND[1], ROUND[2], FEWER, KEYS, MIN_SPLIT, BLOCK, BLOCK_WORK, CUS]
+    return [ROUND[1], ROUND[2], FEWER, KEYS, MIN_SPLIT, BLOCK, BLOCK_WORK, CUS,
+            WORKGROUPS, LONG]
 
 
 def paged_decode_available(q: torch.Tensor, kpool: torch.Tensor) -> bool:
@@ -129,6 +138,11 @@ class StepPlan:
                    merges=merges, any_merge=any_merge, nq=nq)
 
 
+def _rounds(end, n, kv_heads: int):
+    """Keys of the longest part, and rounds of two tiles' workgroups."""
+    return int((-(-end // n)).max()), -(-int(n.sum()) * kv_heads // FEWER)
+
+
 def _planned(slots, pos, tables, block_size: int, heads: int, kv_heads: int):
     """``step_plan`` of csrc/step_plan.cpp, for a host without the extension."""
     T = len(slots)
@@ -167,6 +181,8 @@ def _planned(slots, pos, tables, block_size: int, heads: int, kv_heads: int):
             while per < end[0] and (-(-end // per)).sum() > room:
                 per += MIN_SPLIT
         n = -(-end // per)
+    elif len(end) * kv_heads >= WORKGROUPS:
+        n = np.ones_like(end)
     else:
         total, full = int(end.sum()), ROUND[nq]
         if total * kv_heads < KEYS * full:
@@ -178,6 +194,13 @@ def _planned(slots, pos, tables, block_size: int, heads: int, kv_heads: int):
         while n.sum() > max(room, len(end)):
             per += per // 16
             n = -(-end // per)
+        if nq == 2:
+            longest, rounds = _rounds(end, n, kv_heads)
+            if rounds > 1 and longest > LONG and \
+                    10 * total * kv_heads < 7 * rounds * FEWER * longest:
+                other = -(-end // max(MIN_SPLIT, total * kv_heads // WORKGROUPS))
+                if math.prod(_rounds(end, other, kv_heads)) < rounds * longest:
+                    n = other
     step = -(-(-(-end // n)) // grain) * grain
     n = -(-end // step)
     of = np.repeat(np.arange(len(end)), n)

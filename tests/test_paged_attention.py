@@ -59,6 +59,22 @@ def test_splits_fill_whole_rounds(lens, rows, kv_heads):
     assert {*map(int, ends)} >= {n + 1 for n in lens}
 
 
+@pytest.mark.parametrize("lens,rows,heads,split", [
+    # tiles for all workgroups, and a few less
+    ([2000] * 128, 1, (32, 8), False), ([2000, 3000] * 55, 1, (32, 8), True),
+    ([382] * 9, 93, (256, 32), False), ([382] * 9, 40, (256, 32), True),
+    # evenly long, a round and a quarter: each in two
+    ([15828] * 2, 319, (64, 8), True)])
+def test_many_tiles_and_even_ones(lens, rows, heads, split):
+    slots = list(range(len(lens))) + [len(lens)] * (rows - 1)
+    pos = np.array([*lens, *range(lens[0], lens[0] + rows - 1)])
+    tables = {s: list(range(500)) for s in range(len(lens) + 1)}
+    plan = StepPlan.build(slots, pos, tables, 64, *heads, "cpu")
+    assert plan.any_merge == split
+    if rows == 319:
+        assert plan.items == 2 * plan.merges
+
+
 @pytest.mark.parametrize("heads", [(8, 8), (14, 2), (32, 8), (16, 1)])
 def test_step_plan_equals_numpys(heads):
     """Single rows and runs of every length, slots that come again, tables of any
