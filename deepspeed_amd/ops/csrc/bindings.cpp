@@ -513,15 +513,16 @@ at::Tensor paged_append(at::Tensor q, at::Tensor k, at::Tensor v,
 }
 
 // Whether rows_linear.hip is ahead of tile_linear.hip for bf16 layers of `all`
-// features: up to 16 rows, past which the latter shares x in LDS where the former
-// reads it out of L2 for every 16 to 64 features, and up to 32 for small layers (us,
-// either at 17 and 32 rows: N 4096, K 4096 11.9 / 11.6 and 15 / 12; q, k and v of
-// that 17 / 15 and 20 / 17; N 128256 215 / 185 and 228 / 185; but N 1024, K 1024 4.8 /
-// 7.0 and 5.5 / 7.0; 6144, K 1024 6.6 / 7.2 and 7.1 / 7.5; 4096, K 1792 7.2 / 9.6 and
-// 8.3 / 9.6; and 8192, K 512 5.3 / 5.2 and 5.6 / 5.3; 512, K 2048 6.8 / 7.6 and 8.1 /
-// 7.7; gate and up 2816, K 1024 8.3 / 7.1 and 9.0 / 7.0).
+// features: up to 16 rows, past which x is most of what it reads, and up to 32 for
+// layers of two rounds of tiles of 16 features (us, either at 24 and 32 rows, K 4096
+// unless said: 4096 9.1 / 11.5 and 9.8 / 11.8; q, k and v of that 12.2 / 14.7 and 12.9 /
+// 15.1; 2048, K 2048 5.8 / 8.3 and 6.0 / 8.3; gate and up 2816, K 1024 5.2 / 7.4 and 5.4 /
+// 7.5; but 9216, K 3072 15.8 / 15.5; gate and up 5632, K 2048 11.5 / 12.1 and 11.8 /
+// 12.2, 14336 38.1 / 38.2 and 39.5 / 38.0). Over 3700 layers of the time of the latter
+// 0.5 to 0.9 up to K 4096, 1.1 to 1.4 at 8192 and fewer than 192 tiles; gates 0.5 to 0.75
+// at any K; three rounds 1.1.
 bool few_rows(int64_t M, int64_t all, int64_t K, int64_t mode) {
-  return M <= 16 || (M <= 32 && mode == 0 && K < 2048 && all <= 6144);
+  return M <= 16 || (M <= 32 && all <= 8192 && (mode == 1 || K <= 4096));
 }
 
 // bf16 weights on one input, pointers and features of each; outputs made anew:

@@ -6,23 +6,16 @@
 // csrc/transformer/inference and the weight-only quantized linears of
 // inference/v2/kernels/core_ops (cuda_linear).
 //
-// A workgroup of 8 waves owns 16 FT output features; the waves take every
-// eighth chunk of inputs and add up through LDS, so that the 256 CUs have work
-// at N = 4096. W goes from memory straight into the A operand of
-// mfma_f32_16x16x32_bf16 (16 features by 64 contiguous bytes an instruction), x
-// into B (columns past M repeat the last row).
+// W is the A operand of mfma_f32_16x16x32_bf16 (16 features), x the B operand
+// (columns past M are not stored); the waves of a workgroup have parts of the
+// contraction and add up through LDS.
 //
-//   * Up to 16 rows, few_rows_kernel: W and x are loaded D chunks of 128 inputs
-// ahead, so that a wave waits for neither, and the scales lie in LDS. Bound by
-// the stream of W in large layers, by launch and first loads in small ones. us
-// at 8 rows, before (chunks of 256, x loaded where it is used) and now: gate and
-// up 14336, K 4096 bf16 50.7 / 45.8, int8 36.6 / 32.8; q, k, v 4096 + 2 x 1024,
-// K 4096 16.0 / 13.3 and 12.2 / 10.8; N 128256 199 / 192 and 140 / 121; N 4096,
-// K 14336 27.7 / 27.3 and 19.7 / 18.9; N 4096, K 4096 10.2 / 10.1 and 8.2 / 8.6.
-// Three to six chunks ahead gained nothing more. Most layers of K 2048 to 4096 go
-// on to going_rows_kernel, which was measured against this.
-//   * More rows, rows_linear_kernel: bound by x out of L2. Only int8 weights, small
-// layers and numbers of features that tile_linear.hip does not take come here.
+//   * Up to 16 rows, and up to 32 where the weights are int8 or the layer is small:
+// stream_rows_kernel, in which every load goes to LDS, 128 bytes of 8 rows an
+// instruction. Bound by the stream of W from memory, 6 to 7 TB/s where it is large,
+// by launch and first loads where it is small.
+//   * More rows of int8, rows_linear_kernel: W and x straight into registers, bound by
+// x out of L2. bf16 layers of more rows are tile_linear.hip's.
 //   * int8: a lane's 16 bytes are 16 inputs, split over two products; the order
 //     of the inputs inside a product is free, x is read in the same order. The
 //     bytes become bf16 exactly (8 bits), are summed in fp32 and multiplied by
@@ -41,9 +34,9 @@ typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int NW = 8;       // waves a workgroup
+constexpr int NW = 8;       // waves a workgroup, there
 constexpr int MAXL = 3;     // layers a launch
-constexpr int CH = 128;     // inputs a chunk
+constexpr int CH = 128;     // inputs a chunk of rows_linear_kernel
 
 enum { PLAIN = 0, SWIGLU = 1 };
 
@@ -243,175 +236,100 @@ __global__ __launch_bounds__(NW * 64) void rows_linear_kernel(const Args a) {
   }
 }
 
-// EVEN: every wave's chunks are a multiple of D, so that no load runs ahead of the
-// last one. Otherwise each is asked for by itself, and costs a branch (K 4096, q, k
-// and v of 4096 + 2 x 1024, 8 rows 13.6 / 15.1). us at 8 rows, loads past the end
-// repeating the last chunk and now: N 32000, K 1024 41.6 / 14.4; 3 of 3072, K 3072
-// 22.2 / 16.6; gate and up 2816, K 1024 7.3 / 5.1; 8192, K 3072 24.3 / 20.1; 3584, K
-// 18944 35.1 / 32.2.
-template <bool I8, int MODE, int FT, int D, int OCC, bool EVEN>
-__global__ __launch_bounds__(NW * 64, OCC) void few_rows_kernel(const Args a) {
-  constexpr int L = MODE == SWIGLU ? 2 : 1;   // weight streams a workgroup
-  constexpr int S = L * FT;                   // tiles of 16 features a wave
-  // [waves][S][256] sums, then int8's scales [chunks][S][16]
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  float* const sums = lds;
-  float* const scales = lds + NW * S * 256;
-
-  const int lane = threadIdx.x & 63;
-  const int wid = EVEN ? threadIdx.x >> 6
-                       : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col = lane & 15, g = lane >> 4;
-  int layer = 0, tile = blockIdx.x;
-  if (MODE == PLAIN) {
-    while (tile >= a.tile_end[layer]) ++layer;
-    if (layer) tile -= a.tile_end[layer - 1];
-  }
-  const int N = a.n[layer], n0 = tile * 16 * FT;
-  const short* xp = a.x + (long long)min(col, a.M - 1) * a.K;
-  long long row[FT];
-#pragma unroll
-  for (int f = 0; f < FT; ++f)
-    row[f] = (long long)min(n0 + 16 * f + col, N - 1) * a.K;
-
-  const int chunks = a.K / CH;
-  const int mine = (chunks - wid + NW - 1) / NW;    // wid, wid + NW, ..
-  Weights<I8> w[D][S];
-  s16x8 x[D][CH / 32];
-  // Workgroups that all begin at the rows' beginnings read the same few memory
-  // channels at a time where rows are whole multiples of 16 KB (int8: 4 KB) apart; each
-  // begins elsewhere there (us, 8 rows, before / now: bf16 8192, K 8192 31.6 / 25.0,
-  // 28672 x 2, K 8192 165 / 156; int8 14336 x 2, K 4096 33.8 / 30.8, 4096 8.6 / 7.8,
-  // 128256 117 / 113, of 1 row 109 / 97; but apart by 6 KB, 8192 x 2, K 3072 bf16 19.7 /
-  // 20.4, by 28, 4096, K 14336 of 1 row 22.7 / 23.9, by 8, 128256, K 4096 185 / 189).
-  const int turn = a.K % (I8 ? 4096 : 8192) ? 0
-      : __builtin_amdgcn_readfirstlane(
-            (blockIdx.x / 8 * 13 + blockIdx.x % 8 * 7) % 32 * chunks / 32);
-  auto chunk = [&](int i) __attribute__((always_inline)) {
-    const int c = wid + i * NW + turn;
-    return c < chunks ? c : c - chunks;
-  };
-  auto load = [&](int d, int i) __attribute__((always_inline)) {
-    const int at = chunk(EVEN ? min(i, mine - 1) : i) * CH;
-#pragma unroll
-    for (int s = 0; s < S; ++s)
-      w[d][s].load(a.w[layer + s / FT], row[s % FT] + at, g);
-#pragma unroll
-    for (int k = 0; k < CH / 32; ++k)
-      x[d][k] = *(const s16x8*)(xp + at + input_at<I8>(k, g));
-  };
-  f32x4 acc[S];
-#pragma unroll
-  for (int s = 0; s < S; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (!EVEN || mine > 0)
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-      if (EVEN || d < mine) load(d, d);
-  if (I8) {
-    for (int e = threadIdx.x; e < chunks * S * 16; e += NW * 64) {
-      const int c = e / (S * 16), f = e % (S * 16);
-      const long long r = min(n0 + f % (16 * FT), N - 1);
-      scales[e] = a.scales[layer + f / (16 * FT)][(r * a.K + c * CH) / a.group];
-    }
-    // the scales have arrived, and with them the loads above, which were first
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  }
-  auto use = [&](int d, int i) __attribute__((always_inline)) {
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      f32x4 part = I8 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[s];
-#pragma unroll
-      for (int k = 0; k < CH / 32; ++k)
-        part = mfma(w[d][s].operand(k), x[d][k], part);
-      if (I8) {     // of the rows 4 g + r that the lane holds the sums of
-        const f32x4 sc = *(const f32x4*)(
-            scales + (chunk(i) * S + s) * 16 + 4 * g);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[s][r] += part[r] * sc[r];
-      } else {
-        acc[s] = part;
-      }
-    }
-  };
-  if (mine > 0) {
-    int i = 0;
-    for (; i + D < mine; i += D)
-#pragma unroll
-      for (int d = 0; d < D; ++d) {
-        use(d, i + d);
-        if (EVEN || i + d + D < mine) load(d, i + d + D);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-      if (i + d < mine) use(d, i + d);
-  }
-
-  // ---- add the waves up; features 4 g + r of a column lie side by side
-#pragma unroll
-  for (int s = 0; s < S; ++s)
-    *(f32x4*)(sums + (wid * S + s) * 256 + col * 16 + 4 * g) = acc[s];
-  __syncthreads();
-  for (int e = threadIdx.x; e < FT * 256; e += NW * 64) {
-    const int f = e >> 8, at = e & 255;
-    const int r = at >> 4, n = n0 + 16 * f + (at & 15);
-    if (r >= a.M || n >= N) continue;
-    float y[L];
-#pragma unroll
-    for (int s = 0; s < L; ++s) {
-      float t = 0.f;
-#pragma unroll
-      for (int w_ = 0; w_ < NW; ++w_)
-        t += sums[(w_ * S + s * FT + f) * 256 + at];
-      if (a.bias[layer + s]) t += value(a.bias[layer + s][n]);
-      y[s] = t;
-    }
-    float o = y[0];
-    if (MODE == SWIGLU) o = y[0] / (1.f + expf(-y[0])) * y[L - 1];
-    a.out[layer][(long long)r * N + n] = bits(o);
-  }
+template <int N>
+__device__ __forceinline__ void wait_loads() {  // but for the N youngest
+  static_assert(N < 64, "vmcnt has six bits");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void barrier() {   // and what was read from LDS
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+__device__ __forceinline__ int uni(int x) {
+  return __builtin_amdgcn_readfirstlane(x);
+}
+// Loads past `left` bytes from `base` on bring zeros.
+__device__ __forceinline__ u32x4 descriptor(const void* base, long long left) {
+  const unsigned long long b = (unsigned long long)(uintptr_t)base;
+  u32x4 d;
+  d[0] = uni((unsigned)b);
+  d[1] = uni((unsigned)(b >> 32) & 0xffffu);
+  d[2] = uni(left > 0xffffffffll ? 0xffffffffu : (unsigned)left);
+  d[3] = 0x00020000u;
+  return d;
+}
+// 16 bytes a lane from descriptor + off + soff to LDS, lane after lane from `lds` on;
+// ONCE: read by nobody else, past the caches.
+template <bool ONCE>
+__device__ __forceinline__ void load(u32x4 from, unsigned off, int soff, int lds) {
+  if (ONCE)
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\t"
+                 "buffer_load_dwordx4 %0, %1, %2 offen nt lds"
+                 :: "v"(off), "s"(from), "s"(soff), "s"(lds) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\t"
+                 "buffer_load_dwordx4 %0, %1, %2 offen lds"
+                 :: "v"(off), "s"(from), "s"(soff), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void load_scales(const float* from, unsigned off, int lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+               "global_load_lds_dword %0, %1"
+               :: "v"(off), "s"(from), "s"(lds) : "memory", "m0");
 }
 
-// The same over contractions of X chunks a wave, for which x stays in registers: one
-// workgroup a CU that goes on from tile to tile, with all chunks of the next tile on
-// their way while this one's are multiplied and added up (sums and int8's scales
-// have two places in LDS, and a tile one barrier). Reading x again for each tile
-// takes the more of the time the more rows there are, and first loads and the last
-// round's end are a quarter of a workgroup's life that reads one tile. As many
-// workgroups as fill every round alike. us, few_rows_kernel / here, at 1, 8 and 16
-// rows: gate and up 14336, K 4096 bf16 44.0 / 40.9, 46.0 / 42.1, 51.1 / 43.9, int8 at 8
-// and 16 30.6 / 28.1, 35.4 / 29.7; 128256, K 4096 bf16 163 / 164, 186 / 174, 208 /
-// 181, int8 96 / 87, 112 / 92, 134 / 99; 9216, K 3072 bf16 14.3 / 12.8, 16.7 / 13.6, 18.2
-// (12 rows) / 14.2. Now 5.2 to 6.3 TB/s of W where it is large.
+// Each wave has a ring of its own in LDS, of D slots of 128 bytes of W's rows and what
+// belongs to them of x and of int8's scales; it goes on from tile to tile, so that the
+// ring is full while a tile's sums are added up, and waits for nobody before that.
 //
-// A workgroup's tiles are fixed at the launch and it takes a CU whole: where another
-// stream's kernel holds CUs and the workgroups are more than those left, some begin when
-// the first others end (us, few_rows_kernel / here, 8 rows, weights from memory, alone
-// and with 8 CUs held: 128256, K 4096 bf16 190 / 174 and 210 / 274, int8 128 / 97 and 132
-// / 152; 28672 bf16 51 / 42 and 54 / 65; but gate and up 14336, 224 workgroups, 45 / 42
-// and 46 / 41). Of the framework only ZeRO-3's gathers run beside such layers, and are
-// many times as long; a serving step's collectives wait for it and it for them. With
-// workgroups for 224 CUs nothing is lost where 8 are held, but alone 0 to 17% (int8
-// 32000, K 4096 28.4 / 32.3, 16384 16.6 / 19.5, bf16 12288 20.0 / 21.9, 128256 none).
-template <bool I8, int MODE, int FT, int X>
-__global__ __launch_bounds__(NW * 64, 2) void going_rows_kernel(const Args a,
-                                                                int tiles) {
-  constexpr int L = MODE == SWIGLU ? 2 : 1;   // weight streams a workgroup
-  constexpr int S = L * FT;                   // tiles of 16 features a wave
-  constexpr int C = X * NW, R = I8 ? (C * S * 16 + NW * 64 - 1) / (NW * 64) : 1;
-  __shared__ float sums[2][NW * S * 256];
-  __shared__ __attribute__((aligned(16)))
-  float scales[I8 ? 2 : 1][I8 ? C * S * 16 : 4];
+//   * Loads to LDS, not to registers: as operands of the products lanes next to each
+// other have different rows, and a load of 16 rows by 64 bytes takes the address unit
+// four times as long as one of 8 by 128 (out of L2 9.7 and 30 TB/s). W in that form is
+// a third of the unit's time at the memory's rate, x as much for every tile of 16
+// features and twice that for int8: with either straight in registers, several chunks
+// ahead, 8 rows took (us, K 4096 unless said, before / now): gate and up 14336 bf16
+// 41.5 / 35.0, int8 28.2 / 21.7; q, k, v 4096 + 2 x 1024 13.2 / 10.2 and 10.3 / 7.9; N
+// 4096 9.6 / 7.3 and 7.9 / 5.9; N 4096, K 14336 26.3 / 19.5 and 18.5 / 13.5; N 128256 175
+// / 152 and 92.4 / 81.2; N 3584, K 18944 31.9 / 23.6 and 23.1 / 16.5; 2048, K 2048 6.0 /
+// 4.6 and 5.1 / 4.2. 1 row and 16: 4096 8.6 / 7.2 and 10.9 / 8.0, N 128256 162 / 149 and
+// 183 / 153; int8 24 rows 4096, K 14336 31.0 / 21.3. A read of as many bytes alone takes
+// 6.4 (4096), 9.0 (6144) and 35 (28672 of K 4096 bf16).
+//   * W, which nobody else reads, passes the caches by: 3 to 12%.
+//   * Rows past M and features past N lie past their descriptors or repeat the last.
+//
+// A workgroup's tiles are fixed at the launch: where another stream's kernel holds CUs
+// and the workgroups are more than those left, some begin when the first others end.
 
-  const int lane = threadIdx.x & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+// A stream's place in LDS: W, x, int8's scales of the rows of a slot.
+template <bool I8, int XR, int S, int MODE>
+struct Slot {
+  static constexpr int XROW = I8 ? 256 : 128;       // bytes of x a row
+  static constexpr int X = S * 2048, SC = X + XR * XROW;
+  static constexpr int SCL = !I8 ? 0 : MODE == SWIGLU ? 2 : 1;
+  static constexpr int BYTES = SC + SCL * 256;
+  static constexpr int XL = XR * XROW / 1024, LOADS = 2 * S + XL + SCL;
+};
+
+// XR: rows of x that are loaded, 8 or 16 MT; S: tiles of 16 features a wave, with
+// SWIGLU half of them of the gate; D: slots of a wave's ring.
+template <bool I8, int XR, int S, int NW, int D, int MODE>
+__global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
+                                                              const int tiles) {
+  using P = Slot<I8, XR, S, MODE>;
+  constexpr int MT = (XR + 15) / 16, L = MODE == SWIGLU ? 2 : 1, FT = S / L;
+  constexpr int IN = I8 ? 128 : 64;     // inputs a chunk, 128 bytes of W's rows
+  constexpr int RING = D * P::BYTES;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  float* const sums = (float*)(lds + NW * RING);
+
+  const int lane = threadIdx.x & 63, wid = uni(threadIdx.x >> 6);
   const int col = lane & 15, g = lane >> 4;
-  const int turn = !I8 || a.K % 4096 ? 0      // as above
-      : __builtin_amdgcn_readfirstlane(
-            (blockIdx.x / 8 * 13 + blockIdx.x % 8 * 7) % 32 * C / 32);
+  const int KB = a.K * (I8 ? 1 : 2), chunks = a.K / IN;
+  const int n = (chunks - wid + NW - 1) / NW;       // wid, wid + NW, ..
+  // Each workgroup begins elsewhere in its rows, over an XCD and over the XCDs: rows
+  // that are multiples of 4 KB apart lie in few memory channels.
+  const int turn = uni((blockIdx.x / 8 * 13 + blockIdx.x % 8 * 7) % 32 * chunks / 32);
   auto chunk = [&](int i) __attribute__((always_inline)) {
     const int c = wid + i * NW + turn;
-    return c < C ? c : c - C;
+    return uni(c < chunks ? c : c - chunks);
   };
   struct Place { int layer, n0; };
   auto locate = [&](int tile) __attribute__((always_inline)) {
@@ -420,173 +338,172 @@ __global__ __launch_bounds__(NW * 64, 2) void going_rows_kernel(const Args a,
       while (tile >= a.tile_end[l]) ++l;
       if (l) tile -= a.tile_end[l - 1];
     }
-    return Place{l, tile * 16 * FT};
+    return Place{uni(l), uni(tile * 16 * FT)};
   };
-  int tile = blockIdx.x;
-  Place at = locate(tile);
-  Weights<I8> w[X][S];
-  long long row[FT];
-  Place from = at;
-  auto rows_of = [&](Place p) __attribute__((always_inline)) {
-    from = p;
+
+  // ---- loads. 16-byte chunk c of a row lies at c ^ (row & 7), so that 16 rows are
+  // read without bank conflicts.
+  const unsigned w0 = (lane >> 3) * (unsigned)KB + (((lane & 7) ^ (lane >> 3)) << 4);
+  const unsigned w1 = w0 + 8 * (unsigned)KB;
+  unsigned x0[P::XL];
 #pragma unroll
-    for (int f = 0; f < FT; ++f)
-      row[f] = (long long)min(p.n0 + 16 * f + col, a.n[p.layer] - 1) * a.K;
+  for (int j = 0; j < P::XL; ++j) {
+    const int r = I8 ? 4 * j + (lane >> 4) : 8 * j + (lane >> 3);
+    x0[j] = r * (unsigned)a.K * 2 + ((I8 ? (lane & 15) ^ (r & 7)
+                                         : (lane & 7) ^ (r & 7)) << 4);
+  }
+  const u32x4 xfrom = descriptor(a.x, (long long)a.M * a.K * 2);
+  const int put = uni((int)(uintptr_t)(__attribute__((address_space(3))) char*)lds +
+                      wid * RING);
+  int next = blockIdx.x, next_i = 0, at = 0;    // tile and chunk that come next
+  bool more = n > 0;
+  Place to;
+  u32x4 wfrom[S];
+  auto aim = [&]() __attribute__((always_inline)) {
+    to = locate(next);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {   // a tile past the end is the last row's
+      const int l = MODE == SWIGLU ? s / FT : to.layer;
+      const int f = min(to.n0 + 16 * (s % FT), a.n[l] - 1);
+      wfrom[s] = descriptor((const char*)a.w[l] + (long long)f * KB,
+                            (long long)(a.n[l] - f) * KB);
+    }
   };
-  auto load = [&](int i) __attribute__((always_inline)) {
+  auto fill = [&]() __attribute__((always_inline)) {
+    if (next_i == 0) aim();
+    const int c = chunk(next_i), b = put + at;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      load<true>(wfrom[s], w0, c * 128, b + s * 2048);
+      load<true>(wfrom[s], w1, c * 128, b + s * 2048 + 1024);
+    }
+#pragma unroll
+    for (int j = 0; j < P::XL; ++j)
+      load<false>(xfrom, x0[j], c * P::XROW, b + P::X + j * 1024);
+    if constexpr (I8) {
+      // lane: row; the group of its chunk, both in 256s of inputs
+      const int f = min(to.n0 + (lane & (16 * FT - 1)), a.n[to.layer] - 1);
+      const unsigned i = ((unsigned)f * (unsigned)(a.K / 256) + c / 2) /
+          (unsigned)(a.group / 256);
+#pragma unroll
+      for (int l = 0; l < P::SCL; ++l)
+        load_scales(a.scales[MODE == SWIGLU ? l : to.layer], i * 4,
+                    b + P::SC + l * 256);
+    }
+    at = at + P::BYTES == RING ? 0 : at + P::BYTES;
+    if (++next_i == n) {
+      next_i = 0;
+      next += gridDim.x;
+      more = next < tiles;
+    }
+  };
+  int filled = 0;
+#pragma unroll 1      // short layers wait for the kernel's instructions
+  for (; more && filled < D; ++filled) fill();
+
+  const char* const get = lds + wid * RING;
+  const int o0 = (g ^ (col & 7)) << 4;
+  const int xr = XR == 8 ? col & 7 : col;
+  int from = 0;
+  for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    f32x4 acc[S][MT];
 #pragma unroll
     for (int s = 0; s < S; ++s)
-      w[i][s].load(a.w[from.layer + s / FT], row[s % FT] + chunk(i) * CH, g);
-  };
-  // int8's scales of a tile [chunks][S][16], by way of registers
-  float sc[R];
-  auto load_scales = [&](Place p) __attribute__((always_inline)) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int e = min((int)threadIdx.x + r * NW * 64, C * S * 16 - 1);
-      const int c = e / (S * 16), f = e % (S * 16);
-      const long long n = min(p.n0 + f % (16 * FT), a.n[p.layer] - 1);
-      sc[r] = a.scales[p.layer + f / (16 * FT)][(n * a.K + c * CH) / a.group];
-    }
-  };
-  auto put_scales = [&](int b) __attribute__((always_inline)) {
+      for (int m = 0; m < MT; ++m) acc[s][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < n; ++i) {
+      if (filled == D) wait_loads<(D - 1) * P::LOADS>();
+      else wait_loads<0>();
+      const char* const b = get + from;
+      // the lane's 16 inputs of an int8 row are two operands'
+      constexpr int Q = I8 ? 4 : 2;
+      u32x4 w[S][2];
+      s16x8 x[MT][Q];
+      f32x4 sc[S];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int e = threadIdx.x + r * NW * 64;
-      if (e < C * S * 16) scales[I8 ? b : 0][e] = sc[r];
-    }
-  };
-  if (I8) load_scales(at);
-  rows_of(at);
+      for (int s = 0; s < S; ++s)
 #pragma unroll
-  for (int i = 0; i < X; ++i) load(i);
-  s16x8 x[X][CH / 32];
-  const short* xp = a.x + (long long)min(col, a.M - 1) * a.K;
+        for (int h = 0; h < 2; ++h)
+          w[s][h] = *(const u32x4*)(b + s * 2048 + col * 128 + (o0 ^ (64 * h)));
 #pragma unroll
-  for (int i = 0; i < X; ++i)
+      for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int k = 0; k < CH / 32; ++k)
-      x[i][k] = *(const s16x8*)(xp + chunk(i) * CH + input_at<I8>(k, g));
-  if (I8) {
-    put_scales(0);
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  }
-  int b = 0;
-  while (true) {
-    const int then = tile + gridDim.x;
-    const bool more = then < tiles;
-    const Place next = more ? locate(then) : at;
-    if (I8 && more) load_scales(next);
-    f32x4 acc[S];
+        for (int q = 0; q < Q; ++q) {
+          const int c = I8 ? (2 * g + 8 * (q >> 1) + (q & 1)) ^ (col & 7) : 0;
+          x[m][q] = *(const s16x8*)(b + P::X + (16 * m + xr) * P::XROW +
+                                    (I8 ? c << 4 : o0 ^ (64 * q)));
+        }
+      if (I8)     // of the rows 4 g + r that the lane holds the sums of
 #pragma unroll
-    for (int s = 0; s < S; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < X; ++i) {
+        for (int s = 0; s < S; ++s)
+          sc[s] = *(const f32x4*)(b + P::SC + s / FT * 256 + s % FT * 64 + 16 * g);
+      // what was in the slot is in registers
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) fill();
+      else --filled;
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int s = 0; s < S; ++s) {
-        f32x4 part = I8 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[s];
+        f32x4 part[MT];
 #pragma unroll
-        for (int k = 0; k < CH / 32; ++k)
-          part = mfma(w[i][s].operand(k), x[i][k], part);
-        if (I8) {     // of the rows 4 g + r that the lane holds the sums of
-          const f32x4 v = *(const f32x4*)(
-              &scales[I8 ? b : 0][(chunk(i) * S + s) * 16 + 4 * g]);
+        for (int m = 0; m < MT; ++m)
+          part[m] = I8 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[s][m];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[s][r] += part[r] * v[r];
-        } else {
-          acc[s] = part;
+        for (int q = 0; q < Q; ++q) {
+          u32x4 o = w[s][I8 ? q >> 1 : q];
+          if constexpr (I8) {
+            const unsigned lo = o[2 * (q & 1)], hi = o[2 * (q & 1) + 1];
+            unsigned v[4];
+            widen<true>(lo, v[0], v[1]);
+            widen<true>(hi, v[2], v[3]);
+            o = u32x4{v[0], v[1], v[2], v[3]};
+          }
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            part[m] = mfma(__builtin_bit_cast(s16x8, o), x[m][q], part[m]);
         }
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          if (I8)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[s][m][r] += part[m][r] * sc[s][r];
+          else
+            acc[s][m] = part[m];
       }
-      if (i == 0) rows_of(next);
-      if (more) load(i);
-      __builtin_amdgcn_sched_barrier(0);
+      from = from + P::BYTES == RING ? 0 : from + P::BYTES;
     }
-    float* const sum = sums[b];
+
+    // ---- add the waves up; features 4 g + r of a column lie side by side
+    if (tile != blockIdx.x) barrier();      // the last tile's are read
 #pragma unroll
     for (int s = 0; s < S; ++s)
-      *(f32x4*)(sum + (wid * S + s) * 256 + col * 16 + 4 * g) = acc[s];
-    if (I8 && more) put_scales(b ^ 1);
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    const int N = a.n[at.layer];
-    for (int e = threadIdx.x; e < FT * 256; e += NW * 64) {
-      const int f = e >> 8, o_ = e & 255;
-      const int r = o_ >> 4, n = at.n0 + 16 * f + (o_ & 15);
-      if (r >= a.M || n >= N) continue;
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        *(f32x4*)(sums + ((wid * S + s) * MT + m) * 256 + col * 16 + 4 * g) =
+            acc[s][m];
+    barrier();
+    const Place p = locate(tile);
+    const int N = a.n[p.layer];
+    for (int e = threadIdx.x; e < FT * MT * 256; e += NW * 64) {
+      const int f = e / (MT * 256), o_ = e % (MT * 256);
+      const int r = o_ >> 4, c = p.n0 + 16 * f + (o_ & 15);
+      if (r >= a.M || c >= N) continue;
       float y[L];
 #pragma unroll
-      for (int s = 0; s < L; ++s) {
+      for (int l = 0; l < L; ++l) {
         float t = 0.f;
 #pragma unroll
         for (int w_ = 0; w_ < NW; ++w_)
-          t += sum[(w_ * S + s * FT + f) * 256 + o_];
-        if (a.bias[at.layer + s]) t += value(a.bias[at.layer + s][n]);
-        y[s] = t;
+          t += sums[(w_ * S + l * FT + f) * MT * 256 + o_];
+        if (a.bias[p.layer + l]) t += value(a.bias[p.layer + l][c]);
+        y[l] = t;
       }
       float o = y[0];
       if (MODE == SWIGLU) o = y[0] / (1.f + expf(-y[0])) * y[L - 1];
-      a.out[at.layer][(long long)r * N + n] = bits(o);
+      a.out[p.layer][(long long)r * N + c] = bits(o);
     }
-    if (!more) break;
-    tile = then;
-    at = next;
-    b ^= 1;
   }
-}
-
-template <bool I8, int MODE, int X>
-int launch_going(Args a, int layers, hipStream_t st) {
-  constexpr int FT = I8 && MODE == PLAIN ? 2 : 1, CUS = 256;
-  int tiles = 0;
-  for (int i = 0; i < (MODE == SWIGLU ? 1 : layers); ++i)
-    a.tile_end[i] = tiles += (a.n[i] + 16 * FT - 1) / (16 * FT);
-  const int rounds = (tiles + CUS - 1) / CUS;
-  hipLaunchKernelGGL((going_rows_kernel<I8, MODE, FT, X>),
-                     dim3((tiles + rounds - 1) / rounds), dim3(NW * 64), 0, st,
-                     a, tiles);
-  return (int)hipGetLastError();
-}
-
-// Where they go on, for tiles of 16 features (us, few_rows_kernel / going on, K 4096
-// unless said): not a single round (bf16 4096 of 1 row 8.8 / 8.9, int8 6.9 / 9.1). Gates
-// whose rounds are whole from 9 rows on only (8192 of 1 row 25.2 / 25.9, 12288 35.1 /
-// 36.0, of 16 rows 29.1 / 27.9; 8448 of 1 row 31.6 / 28.3), int8's from 5 on unless
-// they are short (14336, K 3072 of 1 row 20.6 / 21.8, of 8 24.2 / 22.7; K 2048 of 1
-// 15.7 / 14.8). bf16 of one or two rows up to 4096 tiles (50304 67.9 / 65.9, 128256 163
-// / 164, K 3072 123 / 125). int8 of up to four rows not where the last round, of
-// tiles of 32, is filled (13824, K 3072 11.9 / 12.2, 16384 15.2 / 16.0; 12288 14.6 /
-// 14.1, 16640 20.2 / 18.7).
-// K 2048 bf16, where a wave has two chunks on their way, stays (14336 x 2 of 1 row
-// 23.9 / 26.4, 32000 of 8 25.2 / 27.2), as do 5 and more chunks a wave, for which the
-// registers do not reach, and contractions that are not whole chunks of eight waves.
-template <bool I8>
-bool goes_on(const Args& a, int mode, int tiles) {
-  const int X = a.K % (CH * NW) ? 0 : a.K / (CH * NW), pairs = tiles / 2;
-  if (X < (I8 ? 2 : 3) || X > 4) return false;
-  if (mode == SWIGLU)
-    return pairs > 256 && (a.M > 8 || pairs % 256) &&
-           (!I8 || a.M > 4 || X == 2);
-  if (!I8) return tiles > 256 && (a.M > 2 || tiles < 4096);
-  return a.M > 4 ? tiles > 256 : pairs > 512 || (pairs > 256 && pairs <= 384);
-}
-
-// D of chunks ahead, and the waves a SIMD that its registers leave.
-template <bool I8, int MODE, int FT, int D, int OCC>
-int launch_few(Args a, int layers, hipStream_t st) {
-  int tiles = 0;
-  for (int i = 0; i < (MODE == SWIGLU ? 1 : layers); ++i)
-    a.tile_end[i] = tiles += (a.n[i] + 16 * FT - 1) / (16 * FT);
-  constexpr int S = (MODE == SWIGLU ? 2 : 1) * FT;
-  const int lds = NW * S * 1024 + (I8 ? a.K / CH * S * 64 : 0);
-  auto kernel = a.K / CH % (NW * D) == 0
-      ? few_rows_kernel<I8, MODE, FT, D, OCC, true>
-      : few_rows_kernel<I8, MODE, FT, D, OCC, false>;
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(
-        (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess) return (int)e;
-  }
-  hipLaunchKernelGGL(kernel, dim3(tiles), dim3(NW * 64), lds, st, a);
-  return (int)hipGetLastError();
 }
 
 template <bool I8, int MT, int MODE, int FT>
@@ -599,50 +516,115 @@ int launch(Args a, int layers, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// Tiles of features a wave, where workgroups have one tile. Every workgroup reads
-// all of x, which costs M rows
-// out of L2 for 16 FT features of W; half the workgroups leave CUs idle where the
-// layer is small. Up to 16 rows (us, FT 1 / 2): N 4096 bf16 9.6 / 13, int8 8.6 /
-// 10.4; N 6144 15.7 / 13.3 and 12.3 / 10.8; N 128256 8 rows 205 / 192 and 148 /
-// 121, 16 rows 250 / 209 and 178 / 139, but bf16 1 row 168 / 178; gate and up,
-// whose two streams share x, 45.8 / 50.7 and 32.8 / 34.1. With two tiles bf16
-// has four chunks ahead where these are a wave's whole parts (N 6144 13.3, two
-// 14.5; N 32000, K 1024 two 14.4, four 17.7), int8 two (10.8, four 11.5).
-// Two tiles take two rounds of the CUs' time: not where the rounds grow by it (8
-// rows, FT 1 / 2, bf16: N 9216, K 4096 20.7 / 25.0; 12288 22.8 / 26.2; 10240, K 8192
-// 46 / 51; int8 of long layers and few rows: 10240, K 8192 28.0 / 31.3, but 12288, K
-// 4096 17.8 / 17.0), nor, there, where it leaves a CU one workgroup (8192, K 8192, 1
-// row 16.5 / 20.9).
-// More rows, int8 (FT 1 / 2 / 4): M 32: N 4096 11 / 14 / 20, N 6144 23 / 16.3 /
-// 23, N 14336 40 / 29.7 / 24.0; M 64: N 4096 21.1 / 23.8 / 44, N 14336 74 / 46 /
-// 51; gate and up M 32 53.8 / 42.6, M 64 88 / 67.
+// ALL: a workgroup a tile; otherwise as many as the CUs hold at a time, evenly.
+template <bool I8, int XR, int S, int NW, int D, int MODE>
+int launch_stream(Args a, int layers, bool all, hipStream_t st) {
+  constexpr int MT = (XR + 15) / 16, FT = MODE == SWIGLU ? S / 2 : S;
+  constexpr int LDS = NW * (D * Slot<I8, XR, S, MODE>::BYTES + S * MT * 1024);
+  static_assert(LDS <= 160 * 1024 && (!I8 || 16 * FT <= 64), "");
+  constexpr int CUS = 256, HELD = CUS * (160 * 1024 / LDS);
+  int tiles = 0;
+  for (int i = 0; i < (MODE == SWIGLU ? 1 : layers); ++i)
+    a.tile_end[i] = tiles += (a.n[i] + 16 * FT - 1) / (16 * FT);
+  const int rounds = all ? 1 : (tiles + HELD - 1) / HELD;
+  auto kernel = stream_rows_kernel<I8, XR, S, NW, D, MODE>;
+  const hipError_t e = hipFuncSetAttribute(
+      (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL(kernel, dim3((tiles + rounds - 1) / rounds), dim3(NW * 64),
+                     LDS, st, a, tiles);
+  return (int)hipGetLastError();
+}
+
+// Tiles a wave and waves by the layer's tiles of 16 features. us at 1, 8 and 16 rows,
+// S x waves, bf16 unless said:
+//   * A round of the CUs: one tile, so that all of them have work (256 tiles, K 4096:
+// 1 x 8 7.2, 7.3, 8.0, 2 x 8 8.4, 9.2, 10.0). Two up to two rounds (384, K 4096: 9.9,
+// 10.2, 10.8 and one 10.3, 11.2, 12.8; 512, K 28672: 69.8, 70.6, 74.3 and 69.2, 72.9,
+// 84.8; int8 384: 7.5, 7.9, 8.8 and 7.9, 8.4; by four waves 8.1, 8.1, 8.5).
+//   * More: x, which is read for each tile, is a third and half of what arrives at one
+// tile a wave of up to 8 and 16 rows, a ninth and a fifth at four. But one tile, for
+// which two workgroups fit a CU, evens out (576 tiles, K 3072: 11.8, 12.4, 14.4, four
+// 12.7, 13.3, 14.1; 2004: 30.0, 30.4, 34 and 31.1, 30.9, 31.3; 8016, K 4096: 149, 152,
+// 158 and 151, 151, 153); short ones go on from tile to tile (2000, K 1024 12.0 and
+// 12.1, a workgroup a tile 13.2). int8 by four waves, whose tiles end half as often
+// (2 x 4 / 4 x 4: 8016 78.6, 82.9, 97 / 79.6, 81.2, 87.7; 2004, K 3072 18.3, 18.9, 21.8 /
+// 19.1, 19.2, 20.9; 2000, K 1024 8.9, 9.4, 10.3 / 10.0, 10.1, 10.9; one tile: 576 9.0, 9.7,
+// 12.2, four 9.5, 9.9, 10.8; 1024 13.6 and two 13.4).
+//   * Gate and up, one pair: 896 pairs, K 4096 2 x 4 35.2, 35.0, 36.7, 4 x 4 35.7, 35.8,
+// 35.8; 352, K 2048 9.3, 9.9, 10.9 and 9.4, 9.7, 10.2; int8 21.2, 22.4, 25.5 and 21.4,
+// 21.7, 23.6; 176, K 1024 2 x 8 4.3, 4.5, 4.7, 2 x 4 4.6, 4.7, 4.9.
+//   * 17 to 32 rows of int8: 256 tiles, K 4096 1 x 4 8.8, 2 x 4 10.6; 384 14.7 and 11.0.
+template <bool I8, int XR>
+int launch_streams(const Args& a, int layers, int mode, int tiles,
+                   hipStream_t st) {
+#define STREAM(S, NW, D, MODE, ALL) \
+  return launch_stream<I8, XR, S, NW, D, MODE>(a, layers, ALL, st)
+  const bool few = a.M <= (I8 ? 4 : 8);
+  if constexpr (XR == 32) {
+    if constexpr (I8) {
+      if (mode == SWIGLU) STREAM(2, 4, 2, SWIGLU, false);
+      if (tiles <= 256) STREAM(1, 4, 3, PLAIN, false);
+      STREAM(2, 4, 2, PLAIN, false);
+    } else {
+      if (mode == SWIGLU) STREAM(2, 8, 2, SWIGLU, false);
+      if (tiles <= 256) STREAM(1, 8, 2, PLAIN, false);
+      STREAM(2, 8, 2, PLAIN, false);
+    }
+  } else if (mode == SWIGLU) {
+    if constexpr (I8) {
+      if (few || tiles <= 512) STREAM(2, 4, 2, SWIGLU, false);
+    } else {
+      if (tiles <= 512) STREAM(2, 8, 2, SWIGLU, false);
+      if (few) STREAM(2, 4, 4, SWIGLU, false);
+    }
+    STREAM(4, 4, 2, SWIGLU, false);
+  } else {
+    if (tiles <= 256) STREAM(1, 8, 2, PLAIN, false);
+    if constexpr (I8) {
+      if (tiles <= 512) {
+        if (a.M <= 8) STREAM(2, 8, 2, PLAIN, false);
+        STREAM(2, 4, 2, PLAIN, false);
+      }
+      if (few && tiles < 1024 && a.K >= 3072) STREAM(1, 8, 2, PLAIN, true);
+      if (few || a.K < 2048) STREAM(2, 4, 2, PLAIN, false);
+    } else {
+      if (tiles <= 512) STREAM(2, 8, 2, PLAIN, false);
+      if (few) STREAM(1, 8, 2, PLAIN, a.K >= 3072);
+    }
+    STREAM(4, 4, 2, PLAIN, false);
+  }
+#undef STREAM
+}
+
+// What stream_rows_kernel takes: a lane's offsets in a tile and int8's places of scales
+// are 32 bits, and x, which each workgroup reads at another place, stays in an XCD's
+// L2. Of 17 to 32 rows int8 but for short gates (2 x 5632, K 2048 32 rows 12.8, by
+// rows_linear_kernel 12.2), bf16 as ds_rows_linear is given them.
+template <bool I8>
+bool streams(const Args& a, int layers, int mode, int tiles) {
+  if (a.M > 32 || a.K > 1 << 22) return false;
+  if (I8)
+    for (int i = 0; i < layers; ++i)
+      if ((long long)a.n[i] * a.K >= 1ll << 38) return false;
+  return a.M <= 16 || !I8 || mode == PLAIN || tiles <= 512 || a.K > 2048;
+}
+
+// Tiles of features a wave of rows_linear_kernel. Every workgroup reads all of x, which
+// costs M rows out of L2 for 16 FT features of W; half the workgroups leave CUs idle
+// where the layer is small (int8, us, FT 1 / 2 / 4): M 32: N 4096 11 / 14 / 20, N 6144
+// 23 / 16.3 / 23, N 14336 40 / 29.7 / 24.0; M 64: N 4096 21.1 / 23.8 / 44, N 14336 74 /
+// 46 / 51; gate and up M 32 53.8 / 42.6, M 64 88 / 67.
 template <bool I8>
 int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
   int tiles = 0;
   for (int i = 0; i < layers; ++i) tiles += (a.n[i] + 15) / 16;
+  if (streams<I8>(a, layers, mode, tiles)) {
+    if (a.M <= 8) return launch_streams<I8, 8>(a, layers, mode, tiles, st);
+    if (a.M <= 16) return launch_streams<I8, 16>(a, layers, mode, tiles, st);
+    return launch_streams<I8, 32>(a, layers, mode, tiles, st);
+  }
   const bool big = tiles >= 384, huge = tiles >= 896;
-  // int8's scales in LDS: beside the sums 64 bytes a chunk and stream
-  if (a.M <= 16 && goes_on<I8>(a, mode, tiles)) {
-#define GO(X)                                                             \
-  if (a.K == X * CH * NW)                                                 \
-    return mode == SWIGLU ? launch_going<I8, SWIGLU, X>(a, layers, st)    \
-                          : launch_going<I8, PLAIN, X>(a, layers, st);
-    GO(4)
-    GO(3)
-    if constexpr (I8) { GO(2) }
-#undef GO
-  }
-  if (a.M <= 16 && (!I8 || a.K <= 1 << 16)) {
-    if (mode == SWIGLU) return launch_few<I8, SWIGLU, 1, 2, 4>(a, layers, st);
-    const bool rounds = 2 * ((tiles + 511) / 512) <= (tiles + 255) / 256;
-    const bool full = tiles > 448 && tiles <= 512;
-    if (!big || (I8 ? a.M <= 8 && a.K > 4096 && (!rounds || full)
-                    : !rounds || (a.M <= 4 && tiles >= 2048)))
-      return launch_few<I8, PLAIN, 1, 2, 4>(a, layers, st);
-    if (!I8 && a.K / CH % (4 * NW) == 0)
-      return launch_few<I8, PLAIN, 2, 4, 2>(a, layers, st);
-    return launch_few<I8, PLAIN, 2, 2, 4>(a, layers, st);
-  }
   if (mode == SWIGLU) {
     if (a.M <= 32) return launch<I8, 2, SWIGLU, 2>(a, layers, st);
     return launch<true, 4, SWIGLU, 2>(a, layers, st);

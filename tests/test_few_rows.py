@@ -78,3 +78,26 @@ def test_small_layers_of_up_to_32_rows_gpu(ns, k, m):
     x = torch.randn(m, k, generator=g).bfloat16().cuda()
     for y, (_, want) in zip(rows_linear(x, [b[0] for b in both]), both):
         _close(y, want(x))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("k", [256, 1792, 2304, 4352])
+@pytest.mark.parametrize("m", [4, 8, 17, 24, 32])
+@torch.no_grad()
+def test_streams_gpu(int8, k, m):
+    """Every number of tiles and waves: rings that are not filled once, waves
+    without a chunk, tiles that end in part and several to a workgroup, with the
+    bias of each layer."""
+    g = torch.Generator().manual_seed(k + m)
+    x = torch.randn(m, k, generator=g).bfloat16().cuda()
+    for ns, mode in (((4096,), 0), ((4100, 1030, 20), 0), ((8190,), 0),
+                     ((16500, 36), 0), ((4100, 4100), SWIGLU),
+                     ((12300, 12300), SWIGLU)):
+        both = [_layer(n, k, True, int8, g) for n in ns]
+        got = rows_linear(x, [b[0] for b in both], mode)
+        want = [f(x) for _, f in both]
+        if mode == SWIGLU:
+            want = [torch.nn.functional.silu(want[0]) * want[1]]
+        for y, w in zip(got, want):
+            _close(y, w)
