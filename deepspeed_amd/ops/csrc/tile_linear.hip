@@ -101,13 +101,21 @@ __device__ __forceinline__ const char* uni(const char* p) {
 }
 
 // 16 bytes a lane from base + off to LDS, lane after lane from `lds` on. Not the
-// builtin: behind that the compiler waits for all loads before it reads LDS.
+// builtin: behind that the compiler waits for all loads before it reads LDS. ONCE:
+// read by nobody else, past the caches.
+template <bool ONCE>
 __device__ __forceinline__ void load_lds(const char* base, unsigned off,
                                          int lds) {
-  asm volatile("s_mov_b32 m0, %2\n\t"
-               "s_nop 0\n\t"
-               "global_load_lds_dwordx4 %0, %1"
-               :: "v"(off), "s"(uni(base)), "s"(uni(lds)) : "memory", "m0");
+  if (ONCE)
+    asm volatile("s_mov_b32 m0, %2\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dwordx4 %0, %1 nt"
+                 :: "v"(off), "s"(uni(base)), "s"(uni(lds)) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dwordx4 %0, %1"
+                 :: "v"(off), "s"(uni(base)), "s"(uni(lds)) : "memory", "m0");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads() {  // but for the N youngest
@@ -163,7 +171,8 @@ __device__ __forceinline__ void last_steps(F& step, int it, int buf) {
   if constexpr (R > 0) last_steps<R - 1>(step, it + 1, buf);
 }
 
-template <int BM, int BN, int WM, int WN, int NS, int MODE>
+// ONCE: each of W is one workgroup's.
+template <int BM, int BN, int WM, int WN, int NS, int MODE, bool ONCE>
 __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
     const Args a) {
   constexpr bool GLU = MODE == SWIGLU;
@@ -296,7 +305,8 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN / 4) void tile_linear_kernel(
       if (MODE == GRAD_X) o = o * ld * 2 + ((lc ^ lr) << 4);
       p += (long long)step * ROW;
     }
-    load_lds(p, o, lds0 + buf + at);
+    if (ONCE && j < PW) load_lds<true>(p, o, lds0 + buf + at);
+    else load_lds<false>(p, o, lds0 + buf + at);
   };
 
   f32x4 acc[FN][FM];
@@ -520,9 +530,14 @@ __device__ __forceinline__ u32x4 descriptor(const char* base, long long left) {
 __device__ __forceinline__ void load_to(int lds, int n) {
   asm volatile("s_add_u32 m0, %0, %1" :: "s"(lds), "i"(n) : "memory", "m0", "scc");
 }
+template <bool ONCE>
 __device__ __forceinline__ void load(u32x4 from, unsigned off, int soff) {
-  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds"
-               :: "v"(off), "s"(from), "s"(soff) : "memory");
+  if (ONCE)
+    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen nt lds"
+                 :: "v"(off), "s"(from), "s"(soff) : "memory");
+  else
+    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds"
+                 :: "v"(off), "s"(from), "s"(soff) : "memory");
 }
 // The sums of a wave that has all 256 accumulation registers: four from R on. They
 // are named, not variables: those the compiler moves to other registers and, as they
@@ -595,7 +610,7 @@ __device__ __forceinline__ unsigned packed2(float lo, float hi) {
 // K 4096: 28672 696 / 648, 6144 166 / 159, gate and up 14336 712 / 680; gate and up
 // 18944, K 3584, 2331 rows 536 / 503; dx of 14336, K 4096, 8192 rows 745 / 706; dW of
 // that 789 / 727 (its transposing reads are two an operand).
-template <int MODE, bool PARTS>
+template <int MODE, bool PARTS, bool ONCE>
 __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   constexpr bool GLU = MODE == SWIGLU;
   constexpr bool WT = MODE == GRAD_X || MODE == GRAD_W, XT = MODE == GRAD_W;
@@ -786,7 +801,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
     for (int j = 0; j < P; ++j) {
       load_to(wput, j * 4096);
       asm volatile("s_nop 0");
-      load(wfrom, woff[j], wsoff);
+      load<ONCE>(wfrom, woff[j], wsoff);
     }
     wput = next_w(wput, put);
     if (--wleft == 0) turn_w();
@@ -797,7 +812,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
     for (int j = 0; j < P; ++j) {
       load_to(xput, j * 4096);
       asm volatile("s_nop 0");
-      load(xfrom, xoff[j], xsoff);
+      load<false>(xfrom, xoff[j], xsoff);
     }
     xput = xput == put + XAT ? xput + SX : put + XAT;
     if (--xleft == 0) turn_x();
@@ -898,8 +913,8 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int q = 0; q < P; ++q) {
-        if (i == BARRIER + 2 + 6 * q) load(xfrom, xoff[q], xsoff);
-        if (i == BARRIER + 52 + 6 * q) load(wfrom, woff[q], wsoff);
+        if (i == BARRIER + 2 + 6 * q) load<false>(xfrom, xoff[q], xsoff);
+        if (i == BARRIER + 52 + 6 * q) load<ONCE>(wfrom, woff[q], wsoff);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -1097,6 +1112,19 @@ int merge_splits(const Args& a, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+// W past the caches, which are then x's: over one tile of rows (us, before / now, K 4096
+// unless said: 224 rows 128256 247 / 216, gate and up 14336 63 / 60; 128 rows 128256 197 /
+// 168, gate and up 50 / 47; 32 rows 128256 179 / 165, gate and up 43 / 38, 9216, K 3072
+// 16.8 / 15.5). Not where the contraction is split (128 rows 4096, K 14336 in eight 34.0 /
+// 36.4, 64 rows 4096 in four 12.7 / 13.4), nor over several tiles of rows, which share W
+// (300 rows 128256 343 / 345, 2331 rows 3584, K 14336 245 / 251). Over 800 layers of 33 to
+// 256 rows 0.95 of the time, 1.01 at most, from 16 MB on; smaller ones, 0.98 out of
+// memory, may be found in the chip's cache as a whole model's (8 MB 1.08).
+bool once(const Args& a) {
+  return a.mtiles == 1 && a.splits == 1 &&
+      (long long)a.n_end[a.layers - 1] * a.K >= 1 << 23;
+}
+
 template <int BM, int BN, int WM, int WN, int NS, int MODE>
 int launch(Args a, bool merge, hipStream_t st) {
   constexpr int LDS = NS * (BM + BN) * ROW;
@@ -1115,7 +1143,9 @@ int launch(Args a, bool merge, hipStream_t st) {
   // 1.02, to 4 1.07, to 6 1.15, more 1.22 (256 rows 32064, K 16384 255 / 459 us).
   a.turn = a.mtiles == 1 && a.splits == 1 && a.K * 2 % 4096 == 0 &&
       (long long)a.M * a.K <= 1 << 20;
-  auto kernel = tile_linear_kernel<BM, BN, WM, WN, NS, MODE>;
+  auto kernel = tile_linear_kernel<BM, BN, WM, WN, NS, MODE, false>;
+  if constexpr (MODE <= SWIGLU)
+    if (once(a)) kernel = tile_linear_kernel<BM, BN, WM, WN, NS, MODE, true>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (e != hipSuccess) return (int)e;
@@ -1129,8 +1159,10 @@ int launch_wide(Args a, bool merge, hipStream_t st) {
   constexpr int LDS = 160 * 1024;
   const int items = count<256, 256, MODE>(a);
   auto kernel = MODE != SWIGLU && a.splits > 1
-      ? wide_linear_kernel<MODE, MODE != SWIGLU>
-      : wide_linear_kernel<MODE, false>;
+      ? wide_linear_kernel<MODE, MODE != SWIGLU, false>
+      : wide_linear_kernel<MODE, false, false>;
+  if constexpr (MODE <= SWIGLU)
+    if (once(a)) kernel = wide_linear_kernel<MODE, false, true>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (e != hipSuccess) return (int)e;

@@ -228,6 +228,26 @@ def test_one_tile_of_rows_gpu(m, ns, k, mode, tile):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mode", [0, SWIGLU])
+@pytest.mark.parametrize("tile", [1, 2, 4, 5, 7, 8, 9, 10, 11])
+@torch.no_grad()
+def test_weights_past_the_caches_gpu(tile, mode):
+    """One tile of rows over 16 MB of W and a bit less: W's loads are another
+    kind. A last tile of 4 features, gate and up ends in the wave's half."""
+    from deepspeed_amd.ops import _C
+    m = {1: 64, 2: 127, 4: 128, 5: 191, 10: 190}.get(tile, 255)
+    if (tile == 8 and mode) or (tile == 11 and not mode):
+        return      # no such kernels
+    for k in (704, 640):
+        ns = (6148, 6148) if mode else (8196, 3844)
+        assert (sum(ns) * k >= 1 << 23) == (k == 704)
+        x, ws, bs = _inputs(m, ns, k, m)
+        for y, want in zip(_C.tile_linear(x, ws, bs, mode, tile, 1),
+                           _want(x, ws, bs, mode)):
+            _close(y, want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [-1, 0, 1, None])
 def test_square_tile_gpu(rows, monkeypatch):
     """192 x 192, as the tiles before it."""
