@@ -25,9 +25,9 @@
 //
 //   * Bound by the stream of K and V (decode): 16-byte loads, the next tile in
 //     flight while the softmax and the second product of this one run, three
-//     waves a SIMD. 55 us a layer at 32 requests of 2000 tokens and 8 key
-//     heads (4.8 TB/s), 98 us at 8 of 16000 (5.3 TB/s; a large copy reaches
-//     4.9). One position a wave at a time (2-byte loads, a six-step shuffle
+//     waves a SIMD. 48 us a layer at 32 requests of 2000 tokens and 8 key
+//     heads (5.4 TB/s), 91 us at 8 of 16000 (5.8 TB/s; a large copy reaches
+//     4.9, a read 6.4). One position a wave at a time (2-byte loads, a six-step shuffle
 //     chain each) took 240 and 459 us.
 //   * S^T = K Q^T on mfma_f32_16x16x32_bf16: K rows go from global memory
 //     straight into A fragments (64 contiguous bytes a row and instruction).
@@ -91,16 +91,20 @@ __device__ __forceinline__ float value(short x) {
   return __builtin_bit_cast(float, (unsigned)(unsigned short)x << 16);
 }
 
-// One tile of keys: ALIGNED blocks (BS a multiple of 32) hold it whole.
-template <bool ALIGNED>
+// One tile of keys: ALIGNED blocks (BS a multiple of 32) hold it whole, the block `id`.
+// ONCE, where no other columns read them: V, whole lines of it a load, passes the
+// caches by (8 requests of 16000 105 -> 95 us; but 24 of 1000 beside a run of 200 rows,
+// whose tiles share its keys, 40 -> 46); K's lines are four loads', which find them
+// there.
+template <bool ALIGNED, bool ONCE>
 struct Keys {
   s16x8 k[2][4], v[8];
 
-  __device__ __forceinline__ void load(const Args& a, const int* tab, int hkv,
-                                       int kb, int kv_len, int lane) {
+  __device__ __forceinline__ void load(const Args& a, const int* tab, int id,
+                                       int hkv, int kb, int kv_len, int lane) {
     const int row = lane & 15, g = lane >> 4;
     if (ALIGNED) {
-      const long long blk = tab[kb / a.BS];
+      const long long blk = id;
       const long long base = ((blk * a.Hkv + hkv) * a.BS + kb % a.BS) * D;
       const short* kp = a.kpool + base + row * D + 8 * g;
       const short* vp = a.vpool + base + g * D + 8 * row;
@@ -110,7 +114,10 @@ struct Keys {
         for (int kk = 0; kk < 4; ++kk)
           k[t][kk] = *(const s16x8*)(kp + t * 16 * D + kk * 32);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = *(const s16x8*)(vp + i * 4 * D);
+      for (int i = 0; i < 8; ++i) {
+        const s16x8* p = (const s16x8*)(vp + i * 4 * D);
+        v[i] = ONCE ? __builtin_nontemporal_load(p) : *p;
+      }
     } else {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -138,7 +145,8 @@ __global__ __launch_bounds__(NW * 64, NQ == 1 ? 3 : 2) void rows_kernel(const Ar
   __shared__ float lds_ml[NW][NQ * 16][2];
   static_assert(16 * OSTR * 4 >= KT * D * 2, "the V tile fits");
 
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, g = lane >> 4;
   const int hkv = blockIdx.y, G = a.H / a.Hkv;
 
@@ -196,9 +204,19 @@ __global__ __launch_bounds__(NW * 64, NQ == 1 ? 3 : 2) void rows_kernel(const Ar
   const int xr = 4 * g + (col >> 2);
   const int xc = (col & 3) >> 1, xe = (col & 1) * 4;
 
-  Keys<ALIGNED> x;
+  Keys<ALIGNED, NQ == 1> x;
   int kb = key0 + wid * KT;
-  if (kb < key1) x.load(a, tab, hkv, kb, kv_len, lane);
+  // Blocks are looked up a tile ahead of the loads from them: a wave has one tile in
+  // flight, and waited for the table's entry before each (8 requests of 16000 in 2 and
+  // 12 splits 204 / 142 and 95 / 92 us, 32 of 2000 whole 58 / 48).
+  auto find = [&](int k) __attribute__((always_inline)) {
+    return ALIGNED ? tab[min(k, key1 - 1) / a.BS] : 0;
+  };
+  int id = 0;
+  if (kb < key1) {
+    x.load(a, tab, find(kb), hkv, kb, kv_len, lane);
+    id = find(kb + NW * KT);
+  }
   for (; kb < key1; kb += NW * KT) {
     // V into LDS (own region of the wave: its LDS operations keep their order)
     if (kb + KT > kv_len) {   // rows past the end: whatever the pool holds
@@ -223,8 +241,10 @@ __global__ __launch_bounds__(NW * 64, NQ == 1 ? 3 : 2) void rows_kernel(const Ar
           s[n][t] = mfma(x.k[t][kk], qf[n][kk], s[n][t]);
       }
     // the next tile's loads run behind the rest of this one
-    if (kb + NW * KT < key1)
-      x.load(a, tab, hkv, kb + NW * KT, kv_len, lane);
+    if (kb + NW * KT < key1) {
+      x.load(a, tab, id, hkv, kb + NW * KT, kv_len, lane);
+      id = find(kb + 2 * NW * KT);
+    }
 
     const bool whole = kb + KT <= key1 && kb + KT - 1 <= low;
     s16x8 hi[NQ], lo[NQ];

@@ -27,11 +27,18 @@ struct Blocks { int64_t at, count; };     // of a slot
 struct Run { int64_t row0, rows, keys, blocks; };
 struct Tile { int64_t run, tile, end, splits; };
 
+int64_t most_keys(const std::vector<Tile>& tiles) {
+  int64_t most = 0;
+  for (auto& t : tiles) most = std::max(most, t.end);
+  return most;
+}
+
 }  // namespace
 
 // slots and pos: request slot and position of every row; tables[slot]: its blocks.
 // lines: ROUND of one and of two tiles, FEWER, KEYS, MIN_SPLIT, BLOCK, BLOCK_WORK,
-// CUS, WORKGROUPS, LONG. -> (int32 values on the host: items, runs, merges, blocks,
+// CUS, WORKGROUPS, LONG, STEP of one and of two tiles, HELD of these, BYTES, MERGE,
+// MERGED, ROOMS. -> (int32 values on the host: items, runs, merges, blocks,
 // places of the rows; items, runs, merges, whether any history is split, nq, index of
 // the places).
 std::tuple<at::Tensor, int64_t, int64_t, int64_t, bool, int64_t, int64_t>
@@ -43,7 +50,7 @@ step_plan(const pybind11::sequence& slots,
   namespace py = pybind11;
   const int64_t T = py::len(slots), G = kv_heads > 0 ? heads / kv_heads : 0;
   if (T < 1 || pos.ndim() != 1 || pos.size() != T || block_size < 1 || G < 1 ||
-      lines.size() != 10)
+      lines.size() < 19)
     throw py::value_error("step_plan: a step of rows, each with its position");
   const int64_t* at = pos.data();
   const int64_t min_split = lines[4];
@@ -132,6 +139,45 @@ step_plan(const pybind11::sequence& slots,
     int64_t per = std::max(min_split,
                            total / std::max<int64_t>(1, room - n / 2));
     while (splits(per) > std::max(room, n)) per += per / 16;
+    const bool few = n * kv_heads <= fewer && (nq == 1 || runs.size() > 1);
+    if (few) {
+      // ns that the tiles take in these parts
+      const int64_t held = lines[13 + nq], slots_ = held * lines[7];
+      auto cost = [&] {
+        int64_t count = 0, longest = 0;
+        bool any = false;
+        for (auto& t : tiles) {
+          const int64_t step = ceil_div(ceil_div(t.end, t.splits), grain) * grain;
+          count += ceil_div(t.end, step);
+          longest = std::max(longest, std::min(step, t.end));
+          any |= t.end > step;
+        }
+        count *= kv_heads;
+        longest = ceil_div(longest, 128);
+        const int64_t keys = total * kv_heads;
+        const int64_t each = lines[8 + 2 * nq] +
+            lines[9 + 2 * nq] * std::min(held, ceil_div(count, lines[7]));
+        int64_t ns = std::max(longest * each, keys * 512 / lines[16]);
+        if (count > slots_)     // behind one another
+          ns = std::max(ns, (keys + 64 * count) / 128 * each / slots_ +
+                                5 * longest * each / 8);
+        return ns + (any ? lines[17] + lines[18] * count : 0);
+      };
+      int64_t best = most_keys(tiles);
+      splits(best);
+      int64_t least = cost();
+      for (size_t i = 19; i < lines.size(); ++i) {
+        if (lines[i] > full) continue;
+        const int64_t cut = std::max(min_split, ceil_div(total * kv_heads, lines[i]));
+        if (splits(cut) > room) continue;
+        const int64_t ns = cost();
+        if (ns < least) {
+          least = ns;
+          best = cut;
+        }
+      }
+      splits(best);
+    }
     // keys of the longest part, and rounds of two tiles' workgroups
     auto rounds = [&] {
       int64_t longest = 0, count = 0;
@@ -141,7 +187,7 @@ step_plan(const pybind11::sequence& slots,
       }
       return std::make_pair(longest, ceil_div(count * kv_heads, fewer));
     };
-    if (nq == 2) {
+    if (nq == 2 && !few) {
       const auto [longest, k] = rounds();
       if (k > 1 && longest > lines[9] &&
           10 * total * kv_heads < 7 * k * fewer * longest) {

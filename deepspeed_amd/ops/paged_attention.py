@@ -38,6 +38,18 @@ ROUND, FEWER, KEYS = {1: 768, 2: 1024}, 512, 384
 LONG = 2048
 # Keys of the shortest split: one tile of 32 for each of a workgroup's waves.
 MIN_SPLIT = 128
+# Up to FEWER workgroups of whole histories are cut by what the parts would take
+# (``_cost``, ns): for workgroups of ROOMS in all, up to the rounds above, or not at
+# all, since a merge costs as much as reading 500 keys (us, 8 key heads, before / now:
+# 32 of 2000 in 512 / whole 53.3 / 48.4; 24 of 150 17.0 / 11.3; 3 of 125 10.7 / 6.9; 8
+# of 16000 in 768 / 512 92.4 / 91.2). STEP: a workgroup's 128 keys by tiles of columns,
+# and for each workgroup a CU holds beside it, of HELD; BYTES a ns. Fitted to 8000 steps
+# of 1 to 64 requests, half of them beside a run of up to 256 rows, 1 to 32 key heads:
+# 0.90 of the time of the rounds alone, 1.01 of the fastest cut. A run of several rows
+# alone keeps the rounds (its attention is 1 to 2% of such a step).
+ROOMS = 64, 128, 192, 256, 384, 512, 768
+STEP, HELD, BYTES, MERGE, MERGED = {1: (300, 1100), 2: (100, 1500)}, {1: 3, 2: 2}, \
+    7500, 4400, 5
 # Items of 128 columns (rows times heads a key head), eight waves of them a CU,
 # take steps of runs of BLOCK columns and more each that have BLOCK_WORK columns
 # times keys times key heads. us, 32 on 8 heads, tiles of 32 columns and of 128:
@@ -51,7 +63,8 @@ BLOCK, BLOCK_WORK, CUS = 64, 1 << 21, 256
 def _lines() -> List[int]:
     """As csrc/step_plan.cpp reads them."""
     return [ROUND[1], ROUND[2], FEWER, KEYS, MIN_SPLIT, BLOCK, BLOCK_WORK, CUS,
-            WORKGROUPS, LONG]
+            WORKGROUPS, LONG, *STEP[1], *STEP[2], HELD[1], HELD[2], BYTES, MERGE,
+            MERGED, *ROOMS]
 
 
 def paged_decode_available(q: torch.Tensor, kpool: torch.Tensor) -> bool:
@@ -143,6 +156,26 @@ def _rounds(end, n, kv_heads: int):
     return int((-(-end // n)).max()), -(-int(n.sum()) * kv_heads // FEWER)
 
 
+def _parts(end, n, grain: int):
+    """Parts of each tile in whole steps, and keys of a part."""
+    step = -(-(-(-end // n)) // grain) * grain
+    return -(-end // step), step
+
+
+def _cost(end, n, kv_heads: int, nq: int) -> int:
+    """ns that the tiles take in n parts each."""
+    n, step = _parts(end, n, 32)
+    count, total = int(n.sum()) * kv_heads, int(end.sum()) * kv_heads
+    longest = -(-int(np.minimum(step, end).max()) // 128)
+    room = HELD[nq] * CUS
+    each = STEP[nq][0] + STEP[nq][1] * min(HELD[nq], -(-count // CUS))
+    ns = max(longest * each, total * 512 // BYTES)
+    if count > room:    # behind one another
+        ns = max(ns, (total + 64 * count) // 128 * each // room
+                 + 5 * longest * each // 8)
+    return ns + (MERGE + MERGED * count if (n > 1).any() else 0)
+
+
 def _planned(slots, pos, tables, block_size: int, heads: int, kv_heads: int):
     """``step_plan`` of csrc/step_plan.cpp, for a host without the extension."""
     T = len(slots)
@@ -194,15 +227,25 @@ def _planned(slots, pos, tables, block_size: int, heads: int, kv_heads: int):
         while n.sum() > max(room, len(end)):
             per += per // 16
             n = -(-end // per)
-        if nq == 2:
+        if len(end) * kv_heads <= FEWER and (nq == 1 or len(m) > 1):
+            n = np.ones_like(end)
+            least = _cost(end, n, kv_heads, nq)
+            for r in ROOMS:
+                per = max(MIN_SPLIT, -(-total * kv_heads // r))
+                other = -(-end // per)
+                if r > full or int(other.sum()) > room:
+                    continue
+                ns = _cost(end, other, kv_heads, nq)
+                if ns < least:
+                    least, n = ns, other
+        elif nq == 2:
             longest, rounds = _rounds(end, n, kv_heads)
             if rounds > 1 and longest > LONG and \
                     10 * total * kv_heads < 7 * rounds * FEWER * longest:
                 other = -(-end // max(MIN_SPLIT, total * kv_heads // WORKGROUPS))
                 if math.prod(_rounds(end, other, kv_heads)) < rounds * longest:
                     n = other
-    step = -(-(-(-end // n)) // grain) * grain
-    n = -(-end // step)
+    n, step = _parts(end, n, grain)
     of = np.repeat(np.arange(len(end)), n)
     first = np.cumsum(n) - n
     part = np.arange(len(of)) - first[of]

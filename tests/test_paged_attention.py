@@ -75,6 +75,24 @@ def test_many_tiles_and_even_ones(lens, rows, heads, split):
         assert plan.items == 2 * plan.merges
 
 
+@pytest.mark.parametrize("lens,heads,parts", [
+    # whole, since a merge takes longer, and cut
+    ([125] * 3, (32, 8), 1), ([150] * 24, (32, 8), 1), ([2000] * 32, (32, 8), 1),
+    ([500], (32, 8), 1), ([16000] * 8, (32, 8), 3), ([11000], (16, 1), 86),
+    # a tile of columns of 64 requests: as many as the first line takes, one more
+    ([4000] * 64, (32, 8), 1), ([9000] * 65, (32, 8), 1)])
+def test_cuts_by_what_they_take(lens, heads, parts):
+    tables = {s: list(range(300)) for s in range(len(lens))}
+    plan = StepPlan.build(list(range(len(lens))), np.array(lens), tables, 64,
+                          *heads, "cpu")
+    assert plan.any_merge == (plan.items > plan.merges)
+    if len(lens) * heads[1] <= plans.FEWER:
+        assert plan.items == parts * len(lens)
+        end, n = np.array(lens) + 1, np.full(len(lens), parts)
+        whole = plans._cost(end, np.ones_like(n), heads[1], plan.nq)
+        assert plans._cost(end, n, heads[1], plan.nq) <= whole
+
+
 @pytest.mark.parametrize("heads", [(8, 8), (14, 2), (32, 8), (16, 1)])
 def test_step_plan_equals_numpys(heads):
     """Single rows and runs of every length, slots that come again, tables of any
