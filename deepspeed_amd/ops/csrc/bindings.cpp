@@ -113,6 +113,13 @@ extern "C" int ds_rows_linear(const void* x, int layers, const void* const* w,
                               const void* const* bias, void* const* out,
                               const int* n, int M, int K, int group, int mode,
                               void* stream);
+extern "C" int ds_rows_append(const void* x, const void* const* w,
+                              const float* const* scales,
+                              const void* const* bias, void* q, const int* n,
+                              int M, int K, int group, void* kpool,
+                              void* vpool, const int* dst, const float* cs,
+                              const float* sn, const int* positions, int S,
+                              int BS, void* stream);
 extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
                                    int mode, int* splits);
 extern "C" int ds_tile_linear_stages(int tile, int mode);
@@ -453,22 +460,19 @@ at::Tensor paged_rows(at::Tensor q, at::Tensor kpool, at::Tensor vpool,
   return o;
 }
 
-// What both forms below share; q of T rows and H heads: its values, or what it
-// is like.
-at::Tensor append_rows(const at::Tensor& q, const void* k, const void* v,
-                       const void* q_or_bias, const float* part, int splits,
-                       at::Tensor kpool, at::Tensor vpool, at::Tensor dst,
-                       c10::optional<at::Tensor> cos_table,
-                       c10::optional<at::Tensor> sin_table,
-                       c10::optional<at::Tensor> positions, int64_t S,
-                       at::Tensor out) {
-  const int T = q.size(0), H = q.size(1), Hkv = kpool.size(1);
-  TORCH_CHECK(dst.scalar_type() == at::kInt && dst.is_cuda() &&
-              dst.is_contiguous() && dst.numel() == T, "paged_append: dst");
-  TORCH_CHECK(S >= 1 && T % S == 0, "paged_append: S");
+// Angles of a step's T rows, and that these have each a row of the pool.
+struct Turn {
   const float *cs = nullptr, *sn = nullptr;
   const int* pos = nullptr;
-  if (cos_table.has_value()) {
+
+  Turn(int64_t T, const at::Tensor& dst,
+       const c10::optional<at::Tensor>& cos_table,
+       const c10::optional<at::Tensor>& sin_table,
+       const c10::optional<at::Tensor>& positions, int64_t S) {
+    TORCH_CHECK(dst.scalar_type() == at::kInt && dst.is_cuda() &&
+                dst.is_contiguous() && dst.numel() == T, "paged_append: dst");
+    TORCH_CHECK(S >= 1 && T % S == 0, "paged_append: S");
+    if (!cos_table.has_value()) return;
     for (auto& t : {*cos_table, *sin_table})
       TORCH_CHECK(t.scalar_type() == at::kFloat && t.is_cuda() &&
                   t.is_contiguous() && t.dim() == 2 && t.size(1) == 64,
@@ -484,10 +488,24 @@ at::Tensor append_rows(const at::Tensor& q, const void* k, const void* v,
       TORCH_CHECK(cos_table->size(0) >= S, "table shorter than sequence");
     }
   }
+};
+
+// What both forms below share; q of T rows and H heads: its values, or what it
+// is like.
+at::Tensor append_rows(const at::Tensor& q, const void* k, const void* v,
+                       const void* q_or_bias, const float* part, int splits,
+                       at::Tensor kpool, at::Tensor vpool, at::Tensor dst,
+                       c10::optional<at::Tensor> cos_table,
+                       c10::optional<at::Tensor> sin_table,
+                       c10::optional<at::Tensor> positions, int64_t S,
+                       at::Tensor out) {
+  const int T = q.size(0), H = q.size(1), Hkv = kpool.size(1);
+  const Turn turn(T, dst, cos_table, sin_table, positions, S);
   if (T == 0) return out;
   ds_paged_append(q_or_bias, k, v, part, splits, out.data_ptr(),
-                  kpool.data_ptr(), vpool.data_ptr(), dst.data_ptr<int>(), cs,
-                  sn, pos, T, (int)S, H, Hkv, (int)kpool.size(2),
+                  kpool.data_ptr(), vpool.data_ptr(), dst.data_ptr<int>(),
+                  turn.cs, turn.sn, turn.pos, T, (int)S, H, Hkv,
+                  (int)kpool.size(2),
                   cur_stream());
   return out;
 }
@@ -529,6 +547,7 @@ bool few_rows(int64_t M, int64_t all, int64_t K, int64_t mode) {
 // one each, or with mode 1 silu(layer 0) * layer 1.
 struct Layers {
   const void *w[3], *b[3];
+  const float* sc[3];
   void* o[3];
   int n[3];
   int count = 0;
@@ -537,7 +556,7 @@ struct Layers {
 
   void add(const char* what, const at::Tensor& x, const at::Tensor& weight,
            const c10::optional<at::Tensor>& bias, at::ScalarType type,
-           int64_t mode) {
+           int64_t mode, bool output = true) {
     const int64_t M = x.size(0), K = x.size(1);
     const int i = count++;
     TORCH_CHECK(weight.is_cuda() && weight.is_contiguous() &&
@@ -554,9 +573,20 @@ struct Layers {
                   bias->numel() == n[i], what, ": bias");
       b[i] = bias->data_ptr();
     }
-    if (mode == 0 || i == 0) out.push_back(at::empty({M, n[i]}, x.options()));
-    o[i] = out.back().data_ptr();
+    if (output && (mode == 0 || i == 0))
+      out.push_back(at::empty({M, n[i]}, x.options()));
+    o[i] = output ? out.back().data_ptr() : nullptr;
     TORCH_CHECK(mode == 0 || n[0] == n[i], what, ": gate and up");
+  }
+  // The last one's scales.
+  void scaled(const char* what, const at::Tensor& weight,
+              const at::Tensor& scales, int64_t group) {
+    TORCH_CHECK(scales.is_cuda() && scales.is_contiguous() &&
+                scales.scalar_type() == at::kFloat && group > 0 &&
+                group % 256 == 0 &&
+                scales.numel() == (weight.numel() + group - 1) / group,
+                what, ": scales");
+    sc[count - 1] = scales.data_ptr<float>();
   }
   // Whether tile_linear.hip takes them; does it if so. A tile and a number of
   // splits may be asked for. With `parts`, sums in parts [splits, M, all] are left
@@ -610,23 +640,14 @@ std::vector<at::Tensor> rows_linear(
               (int)biases.size() == L, "rows_linear: shape");
   TORCH_CHECK(((uintptr_t)x.data_ptr() & 15) == 0, "rows_linear: alignment");
   const bool i8 = !scales.empty();
-  const float* sc[3];
   Layers y;
   for (int i = 0; i < L; ++i) {
     y.add("rows_linear", x, weights[i], biases[i],
           i8 ? at::kChar : at::kBFloat16, mode);
-    if (i8) {
-      TORCH_CHECK(scales[i].is_cuda() && scales[i].is_contiguous() &&
-                  scales[i].scalar_type() == at::kFloat && group > 0 &&
-                  group % 256 == 0 &&
-                  scales[i].numel() ==
-                      (weights[i].numel() + group - 1) / group,
-                  "rows_linear: scales");
-      sc[i] = scales[i].data_ptr<float>();
-    }
+    if (i8) y.scaled("rows_linear", weights[i], scales[i], group);
   }
   if (!i8 && !few_rows(M, y.all, K, mode) && y.tiled(x, mode)) return y.out;
-  const int e = ds_rows_linear(x.data_ptr(), L, y.w, i8 ? sc : nullptr, y.b,
+  const int e = ds_rows_linear(x.data_ptr(), L, y.w, i8 ? y.sc : nullptr, y.b,
                                y.o, y.n, (int)M, (int)K, (int)group, (int)mode,
                                cur_stream());
   TORCH_CHECK(e == 0, "rows_linear: launch failed with error ", e);
@@ -956,7 +977,7 @@ bool own_forward(int64_t M, const std::vector<int64_t>& ns, int64_t K,
 // stream x [.., H] that still lacks the last layer's output delta, to the same:
 // norm, q k v, rotation and append, attention, output, norm, gated MLP. What the
 // modules of models/llama.py call one by one, without their host time between
-// the launches (a layer of nine 180 us there, 45 here). norms: two weights.
+// the launches (a layer of nine 180 us there, 40 here). norms: two weights.
 // weights: q, k, v, o, gate, up, down; int8 with scales. meta.. nq: StepPlan.
 // Products whose contraction is split leave their sums in parts to what reads
 // them next: the append, the norms, and with `parts` the next layer's, whose
@@ -1052,13 +1073,47 @@ std::tuple<at::Tensor, at::Tensor> paged_decoder_layer(
     add_norm(*delta, norms[0], eps0);
   else
     h = std::get<0>(norm_fwd(stream, norms[0], c10::nullopt, eps0, false));
-  at::Tensor q;
-  auto [qkv, qkv_part] = sums(h, 0, 3);
-  for (auto& t : qkv) t = t.view({M, -1, 128});
-  check_pool(qkv[0], kpool, vpool, "paged_decoder_layer");
-  TORCH_CHECK(qkv[1].size(1) == kpool.size(1) &&
-              qkv[2].size(1) == kpool.size(1), "paged_decoder_layer: heads");
-  if (qkv_part.defined()) {
+  // q turned, k and v in the pool, by the product of few rows itself
+  auto few_append = [&]() -> at::Tensor {
+    const bool i8 = !scales.empty();
+    const int64_t all =
+        (weights[0].numel() + weights[1].numel() + weights[2].numel()) / H;
+    if (M > 32 || H % 256 || !(i8 || few_rows(M, all, H, 0)))
+      return at::Tensor();
+    Layers y;
+    for (int i = 0; i < 3; ++i) {
+      y.add("paged_decoder_layer", h, weights[i], biases[i],
+            i8 ? at::kChar : at::kBFloat16, 0, i == 0);
+      if (i8)
+        y.scaled("paged_decoder_layer", weights[i], scales[i], group);
+      if (y.n[i] % 128) return at::Tensor();
+    }
+    auto out = y.out[0].view({M, -1, 128});
+    check_pool(out, kpool, vpool, "paged_decoder_layer");
+    TORCH_CHECK(y.n[1] == kpool.size(1) * 128 && y.n[2] == y.n[1],
+                "paged_decoder_layer: heads");
+    const Turn turn(M, dst, cos_table, sin_table, positions, S);
+    const int e = ds_rows_append(
+        h.data_ptr(), y.w, i8 ? y.sc : nullptr, y.b, y.o[0], y.n, (int)M,
+        (int)H, (int)group, kpool.data_ptr(), vpool.data_ptr(),
+        dst.data_ptr<int>(), turn.cs, turn.sn, turn.pos, (int)S,
+        (int)kpool.size(2), cur_stream());
+    if (e < 0) return at::Tensor();
+    TORCH_CHECK(e == 0, "paged_decoder_layer: launch failed with error ", e);
+    return out;
+  };
+  auto q = few_append();
+  std::vector<at::Tensor> qkv;
+  at::Tensor qkv_part;
+  if (!q.defined()) {
+    std::tie(qkv, qkv_part) = sums(h, 0, 3);
+    for (auto& t : qkv) t = t.view({M, -1, 128});
+    check_pool(qkv[0], kpool, vpool, "paged_decoder_layer");
+    TORCH_CHECK(qkv[1].size(1) == kpool.size(1) &&
+                qkv[2].size(1) == kpool.size(1), "paged_decoder_layer: heads");
+  }
+  if (q.defined()) {
+  } else if (qkv_part.defined()) {
     const void* b[3];
     for (int i = 0; i < 3; ++i)
       b[i] = biases[i].has_value() ? biases[i]->data_ptr() : nullptr;

@@ -42,6 +42,15 @@ __device__ __forceinline__ float from_f32<float>(float x) {
   return x;
 }
 
+// Rotary embedding of the features d (a) and d + half (b), rounded alike wherever it
+// is taken.
+struct Turned {
+  float lo, hi;
+};
+__device__ __forceinline__ Turned turn(float a, float b, float c, float s) {
+  return {__builtin_fmaf(a, c, -(b * s)), __builtin_fmaf(b, c, a * s)};
+}
+
 // Full-wave (64-lane) reductions via xor shuffles.
 __device__ __forceinline__ float wave_reduce_sum(float x) {
 #pragma unroll

@@ -757,8 +757,9 @@ __global__ __launch_bounds__(256) void append_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float a = value(x1[e]), b = value(x2[e]);
-      x1[e] = bits(a * cp[e] - b * sp[e]);
-      x2[e] = bits(b * cp[e] + a * sp[e]);
+      const ds::Turned t = ds::turn(a, b, cp[e], sp[e]);
+      x1[e] = bits(t.lo);
+      x2[e] = bits(t.hi);
     }
   }
   *(s16x8*)(to + j) = x1;

@@ -38,7 +38,18 @@ constexpr int NW = 8;       // waves a workgroup, there
 constexpr int MAXL = 3;     // layers a launch
 constexpr int CH = 128;     // inputs a chunk of rows_linear_kernel
 
-enum { PLAIN = 0, SWIGLU = 1 };
+// QKV: three layers of heads of 128 features
+enum { PLAIN = 0, SWIGLU = 1, QKV = 2 };
+
+// With `dst`, where q, k and v go: q turned to out[0], k turned and v to rows dst of the
+// paged pool [blocks, heads, BS, 128].
+struct Append {
+  const float *cs, *sn;     // [positions, 64]
+  const int* positions;     // [M], or null: row % S
+  const int* dst;
+  short *kpool, *vpool;
+  int S, heads, BS;
+};
 
 struct Args {
   const void* w[MAXL];
@@ -48,6 +59,7 @@ struct Args {
   int n[MAXL], tile_end[MAXL];
   const short* x;
   int M, K, group;
+  Append to;
 };
 
 __device__ __forceinline__ f32x4 mfma(s16x8 a, s16x8 b, f32x4 c) {
@@ -303,18 +315,25 @@ template <bool I8, int XR, int S, int MODE>
 struct Slot {
   static constexpr int XROW = I8 ? 256 : 128;       // bytes of x a row
   static constexpr int X = S * 2048, SC = X + XR * XROW;
-  static constexpr int SCL = !I8 ? 0 : MODE == SWIGLU ? 2 : 1;
+  static constexpr int SCL = !I8 ? 0 : MODE == PLAIN ? 1 : 2;
   static constexpr int BYTES = SC + SCL * 256;
   static constexpr int XL = XR * XROW / 1024, LOADS = 2 * S + XL + SCL;
 };
 
 // XR: rows of x that are loaded, 8 or 16 MT; S: tiles of 16 features a wave, with
 // SWIGLU half of them of the gate; D: slots of a wave's ring.
+//
+// QKV: half of the tiles lie 64 features behind the others, so that the threads that add
+// a pair up turn it and write it where attention reads it. What that asks for (positions,
+// rows of the pool, angles) is fetched before the weights are waited for. q, k and v that
+// are only wanted as they are have the same tiles, and the same sums. A launch and 3 us a
+// layer less: steps of four layers, one request of 500 532 -> 525 us, 8 of 16000 873 ->
+// 857, int8 8 of 1000, where the host is as long, 402 -> 381.
 template <bool I8, int XR, int S, int NW, int D, int MODE>
 __global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
                                                               const int tiles) {
   using P = Slot<I8, XR, S, MODE>;
-  constexpr int MT = (XR + 15) / 16, L = MODE == SWIGLU ? 2 : 1, FT = S / L;
+  constexpr int MT = (XR + 15) / 16, L = MODE == PLAIN ? 1 : 2, FT = S / L;
   constexpr int IN = I8 ? 128 : 64;     // inputs a chunk, 128 bytes of W's rows
   constexpr int RING = D * P::BYTES;
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -334,11 +353,15 @@ __global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
   struct Place { int layer, n0; };
   auto locate = [&](int tile) __attribute__((always_inline)) {
     int l = 0;
-    if (MODE == PLAIN) {
+    if (MODE != SWIGLU) {
       while (tile >= a.tile_end[l]) ++l;
       if (l) tile -= a.tile_end[l - 1];
     }
     return Place{uni(l), uni(tile * 16 * FT)};
+  };
+  // QKV: n0 counts in the halves of heads
+  auto feature = [&](int n) __attribute__((always_inline)) {
+    return MODE == QKV ? (n >> 6) * 128 + (n & 63) : n;
   };
 
   // ---- loads. 16-byte chunk c of a row lies at c ^ (row & 7), so that 16 rows are
@@ -364,7 +387,8 @@ __global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
 #pragma unroll
     for (int s = 0; s < S; ++s) {   // a tile past the end is the last row's
       const int l = MODE == SWIGLU ? s / FT : to.layer;
-      const int f = min(to.n0 + 16 * (s % FT), a.n[l] - 1);
+      const int f = min(feature(to.n0 + 16 * (s % FT)) +
+                        (MODE == QKV ? s / FT * 64 : 0), a.n[l] - 1);
       wfrom[s] = descriptor((const char*)a.w[l] + (long long)f * KB,
                             (long long)(a.n[l] - f) * KB);
     }
@@ -382,13 +406,15 @@ __global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
       load<false>(xfrom, x0[j], c * P::XROW, b + P::X + j * 1024);
     if constexpr (I8) {
       // lane: row; the group of its chunk, both in 256s of inputs
-      const int f = min(to.n0 + (lane & (16 * FT - 1)), a.n[to.layer] - 1);
-      const unsigned i = ((unsigned)f * (unsigned)(a.K / 256) + c / 2) /
-          (unsigned)(a.group / 256);
+      const int f = feature(to.n0 + (lane & (16 * FT - 1)));
 #pragma unroll
-      for (int l = 0; l < P::SCL; ++l)
+      for (int l = 0; l < P::SCL; ++l) {
+        const int r = min(f + (MODE == QKV ? 64 * l : 0), a.n[to.layer] - 1);
+        const unsigned i = ((unsigned)r * (unsigned)(a.K / 256) + c / 2) /
+            (unsigned)(a.group / 256);
         load_scales(a.scales[MODE == SWIGLU ? l : to.layer], i * 4,
                     b + P::SC + l * 256);
+      }
     }
     at = at + P::BYTES == RING ? 0 : at + P::BYTES;
     if (++next_i == n) {
@@ -397,6 +423,20 @@ __global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
       more = next < tiles;
     }
   };
+  // A thread adds up elements threadIdx.x + k NW 64 of a tile, of one row or MT.
+  constexpr int E = (FT * MT * 256 + NW * 64 - 1) / (NW * 64);
+  auto row_of = [&](int k) __attribute__((always_inline)) {
+    return min((int)((threadIdx.x + k * NW * 64) % (MT * 256)) >> 4, a.M - 1);
+  };
+  const bool turned = MODE == QKV && a.to.dst != nullptr;
+  int position[MT], row[MT];
+  if (turned)
+#pragma unroll
+    for (int k = 0; k < MT && k < E; ++k) {
+      const int r = row_of(k);
+      position[k] = a.to.positions ? a.to.positions[r] : r % a.to.S;
+      row[k] = a.to.dst[r];
+    }
   int filled = 0;
 #pragma unroll 1      // short layers wait for the kernel's instructions
   for (; more && filled < D; ++filled) fill();
@@ -406,6 +446,19 @@ __global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
   const int xr = XR == 8 ? col & 7 : col;
   int from = 0;
   for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    float angle[E][2];
+    if (turned) {
+      const Place p = locate(tile);
+      if (p.layer < 2)
+#pragma unroll
+        for (int k = 0; k < E; ++k) {
+          const int e = threadIdx.x + k * NW * 64;
+          const int j = (p.n0 + e / (MT * 256) * 16 + (e & 15)) & 63;
+          const long long at = (long long)position[k % MT] * 64 + j;
+          angle[k][0] = a.to.cs[at];
+          angle[k][1] = a.to.sn[at];
+        }
+    }
     f32x4 acc[S][MT];
 #pragma unroll
     for (int s = 0; s < S; ++s)
@@ -485,10 +538,12 @@ __global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
     barrier();
     const Place p = locate(tile);
     const int N = a.n[p.layer];
-    for (int e = threadIdx.x; e < FT * MT * 256; e += NW * 64) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      const int e = threadIdx.x + k * NW * 64;
       const int f = e / (MT * 256), o_ = e % (MT * 256);
-      const int r = o_ >> 4, c = p.n0 + 16 * f + (o_ & 15);
-      if (r >= a.M || c >= N) continue;
+      const int r = o_ >> 4, c = feature(p.n0 + 16 * f + (o_ & 15));
+      if (e >= FT * MT * 256 || r >= a.M || c >= N) continue;
       float y[L];
 #pragma unroll
       for (int l = 0; l < L; ++l) {
@@ -496,12 +551,35 @@ __global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
 #pragma unroll
         for (int w_ = 0; w_ < NW; ++w_)
           t += sums[(w_ * S + l * FT + f) * MT * 256 + o_];
-        if (a.bias[p.layer + l]) t += value(a.bias[p.layer + l][c]);
+        if (MODE == QKV) {
+          if (a.bias[p.layer]) t += value(a.bias[p.layer][c + 64 * l]);
+        } else if (a.bias[p.layer + l]) {
+          t += value(a.bias[p.layer + l][c]);
+        }
         y[l] = t;
       }
-      float o = y[0];
-      if (MODE == SWIGLU) o = y[0] / (1.f + expf(-y[0])) * y[L - 1];
-      a.out[p.layer][(long long)r * N + c] = bits(o);
+      if constexpr (MODE == QKV) {
+        short* to = a.out[p.layer] + (long long)r * N + c;
+        short lo = bits(y[0]), hi = bits(y[1]);
+        if (turned && p.layer < 2) {
+          const ds::Turned t =
+              ds::turn(value(lo), value(hi), angle[k][0], angle[k][1]);
+          lo = bits(t.lo);
+          hi = bits(t.hi);
+        }
+        if (turned && p.layer) {
+          const int at = row[k % MT];
+          to = (p.layer == 1 ? a.to.kpool : a.to.vpool) + c % 128 +
+              (((long long)(at / a.to.BS) * a.to.heads + c / 128) * a.to.BS +
+               at % a.to.BS) * 128;
+        }
+        to[0] = lo;
+        to[64] = hi;
+      } else {
+        float o = y[0];
+        if (MODE == SWIGLU) o = y[0] / (1.f + expf(-y[0])) * y[L - 1];
+        a.out[p.layer][(long long)r * N + c] = bits(o);
+      }
     }
   }
 }
@@ -519,13 +597,14 @@ int launch(Args a, int layers, hipStream_t st) {
 // ALL: a workgroup a tile; otherwise as many as the CUs hold at a time, evenly.
 template <bool I8, int XR, int S, int NW, int D, int MODE>
 int launch_stream(Args a, int layers, bool all, hipStream_t st) {
-  constexpr int MT = (XR + 15) / 16, FT = MODE == SWIGLU ? S / 2 : S;
+  constexpr int MT = (XR + 15) / 16, FT = MODE == PLAIN ? S : S / 2;
   constexpr int LDS = NW * (D * Slot<I8, XR, S, MODE>::BYTES + S * MT * 1024);
   static_assert(LDS <= 160 * 1024 && (!I8 || 16 * FT <= 64), "");
   constexpr int CUS = 256, HELD = CUS * (160 * 1024 / LDS);
   int tiles = 0;
   for (int i = 0; i < (MODE == SWIGLU ? 1 : layers); ++i)
-    a.tile_end[i] = tiles += (a.n[i] + 16 * FT - 1) / (16 * FT);
+    a.tile_end[i] = tiles +=
+        (a.n[i] / (MODE == QKV ? 2 : 1) + 16 * FT - 1) / (16 * FT);
   const int rounds = all ? 1 : (tiles + HELD - 1) / HELD;
   auto kernel = stream_rows_kernel<I8, XR, S, NW, D, MODE>;
   const hipError_t e = hipFuncSetAttribute(
@@ -564,10 +643,12 @@ int launch_streams(const Args& a, int layers, int mode, int tiles,
   if constexpr (XR == 32) {
     if constexpr (I8) {
       if (mode == SWIGLU) STREAM(2, 4, 2, SWIGLU, false);
+      if (mode == QKV) STREAM(2, 4, 2, QKV, false);
       if (tiles <= 256) STREAM(1, 4, 3, PLAIN, false);
       STREAM(2, 4, 2, PLAIN, false);
     } else {
       if (mode == SWIGLU) STREAM(2, 8, 2, SWIGLU, false);
+      if (mode == QKV) STREAM(2, 8, 2, QKV, false);
       if (tiles <= 256) STREAM(1, 8, 2, PLAIN, false);
       STREAM(2, 8, 2, PLAIN, false);
     }
@@ -579,6 +660,11 @@ int launch_streams(const Args& a, int layers, int mode, int tiles,
       if (few) STREAM(2, 4, 4, SWIGLU, false);
     }
     STREAM(4, 4, 2, SWIGLU, false);
+  } else if (mode == QKV) {
+    if (I8 ? tiles <= 512 && a.M <= 8 : tiles <= 512 || few)
+      STREAM(2, 8, 2, QKV, false);
+    if (I8 && (tiles <= 512 || few)) STREAM(2, 4, 2, QKV, false);
+    STREAM(4, 4, 2, QKV, false);
   } else {
     if (tiles <= 256) STREAM(1, 8, 2, PLAIN, false);
     if constexpr (I8) {
@@ -610,6 +696,12 @@ bool streams(const Args& a, int layers, int mode, int tiles) {
   return a.M <= 16 || !I8 || mode == PLAIN || tiles <= 512 || a.K > 2048;
 }
 
+// Queries, keys and values, or what has their form.
+bool in_heads(const Args& a, int layers) {
+  return layers == 3 && a.n[0] % 128 == 0 && a.n[1] % 128 == 0 &&
+      a.n[2] % 128 == 0;
+}
+
 // Tiles of features a wave of rows_linear_kernel. Every workgroup reads all of x, which
 // costs M rows out of L2 for 16 FT features of W; half the workgroups leave CUs idle
 // where the layer is small (int8, us, FT 1 / 2 / 4): M 32: N 4096 11 / 14 / 20, N 6144
@@ -620,6 +712,7 @@ int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
   int tiles = 0;
   for (int i = 0; i < layers; ++i) tiles += (a.n[i] + 15) / 16;
   if (streams<I8>(a, layers, mode, tiles)) {
+    if (mode == PLAIN && in_heads(a, layers)) mode = QKV;
     if (a.M <= 8) return launch_streams<I8, 8>(a, layers, mode, tiles, st);
     if (a.M <= 16) return launch_streams<I8, 16>(a, layers, mode, tiles, st);
     return launch_streams<I8, 32>(a, layers, mode, tiles, st);
@@ -638,16 +731,9 @@ int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
   return launch<true, 4, PLAIN, 1>(a, layers, st);
 }
 
-}  // namespace
-
-// layers: 1..3 weights on one input; mode 1: silu(layer 0) * layer 1. K and,
-// int8, the group are multiples of 256: a chunk of a feature has one scale.
-// M up to 32, int8 64. Returns a hipError_t.
-extern "C" int ds_rows_linear(const void* x, int layers, const void* const* w,
-                              const float* const* scales,
-                              const void* const* bias, void* const* out,
-                              const int* n, int M, int K, int group, int mode,
-                              void* stream) {
+Args arguments(const void* x, int layers, const void* const* w,
+               const float* const* scales, const void* const* bias,
+               void* const* out, const int* n, int M, int K, int group) {
   Args a = {};
   for (int i = 0; i < layers; ++i) {
     a.w[i] = w[i];
@@ -658,7 +744,43 @@ extern "C" int ds_rows_linear(const void* x, int layers, const void* const* w,
   }
   a.x = (const short*)x;
   a.M = M; a.K = K; a.group = group;
+  return a;
+}
+
+}  // namespace
+
+// layers: 1..3 weights on one input; mode 1: silu(layer 0) * layer 1. K and,
+// int8, the group are multiples of 256: a chunk of a feature has one scale.
+// M up to 32, int8 64. Returns a hipError_t.
+extern "C" int ds_rows_linear(const void* x, int layers, const void* const* w,
+                              const float* const* scales,
+                              const void* const* bias, void* const* out,
+                              const int* n, int M, int K, int group, int mode,
+                              void* stream) {
+  const Args a = arguments(x, layers, w, scales, bias, out, n, M, K, group);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   return scales ? launch_rows<true>(a, layers, mode, st)
                 : launch_rows<false>(a, layers, mode, st);
+}
+
+// q [M, H, 128] turned and k and v into the paged pool, as the layers and then
+// ds_paged_append would have it bit by bit: one launch for two. -1: not these.
+extern "C" int ds_rows_append(const void* x, const void* const* w,
+                              const float* const* scales,
+                              const void* const* bias, void* q, const int* n,
+                              int M, int K, int group, void* kpool,
+                              void* vpool, const int* dst, const float* cs,
+                              const float* sn, const int* positions, int S,
+                              int BS, void* stream) {
+  void* const out[] = {q, nullptr, nullptr};
+  Args a = arguments(x, 3, w, scales, bias, out, n, M, K, group);
+  const int tiles = (n[0] + n[1] + n[2]) / 16;
+  if (!in_heads(a, 3) || !(scales ? streams<true>(a, 3, PLAIN, tiles)
+                                  : streams<false>(a, 3, PLAIN, tiles)))
+    return -1;
+  a.to = {cs, sn, positions, dst, (short*)kpool, (short*)vpool, S, n[1] / 128,
+          BS};
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  return scales ? launch_rows<true>(a, 3, PLAIN, st)
+                : launch_rows<false>(a, 3, PLAIN, st);
 }

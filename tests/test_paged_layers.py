@@ -167,6 +167,70 @@ def test_same_as_modules_gpu(kind, positions, monkeypatch):
         assert torch.equal(a, b)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv_heads", [(2, 1), (32, 8), (36, 18),
+                                            (56, 8)])
+@pytest.mark.parametrize("rows", [1, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("int8", [False, True])
+@torch.no_grad()
+def test_append_with_the_products_gpu(heads, kv_heads, rows, int8, monkeypatch):
+    """q, k and v turned and written by their products, bit by bit as behind
+    them: one and two pairs of tiles a wave, a tile and several a workgroup; and
+    these near fp32."""
+    torch.manual_seed(rows)
+    cfg = llama.LlamaConfig(vocab_size=64, hidden_size=heads * 128,
+                            intermediate_size=256, num_layers=1,
+                            num_heads=heads, num_kv_heads=kv_heads,
+                            max_seq_len=256, attention_bias=True)
+    model = llama.LlamaForCausalLM(cfg).to("cuda", torch.bfloat16).eval()
+    attn = model.model.layers[0].self_attn
+    for lin in (attn.q_proj, attn.k_proj, attn.v_proj):
+        lin.bias.data.normal_()
+    refs = [(lin.weight.float(), lin.bias.float())
+            for lin in (attn.q_proj, attn.k_proj, attn.v_proj)]
+    if int8:
+        for m in (attn, model.model.layers[0].mlp):
+            for name, lin in list(m.named_children()):
+                setattr(m, name, WOQLinear(lin, QuantizationConfig()))
+    ids = torch.randint(0, 64, (rows, 1), device="cuda")
+    pos = torch.arange(rows, device="cuda", dtype=torch.int32)[:, None] + 3
+    calls, native = [], llama.get_ext().paged_decoder_layer
+    monkeypatch.setattr(llama.get_ext(), "paged_decoder_layer",
+                        lambda *a: calls.append(1) or native(*a))
+    out = []
+    for own in (True, False):
+        if not own:
+            monkeypatch.setattr(llama.LlamaModel, "_paged_plan",
+                                lambda *a: None)
+        cache = PagedKVCache(1, rows, kv_heads, 256, 128,
+                             dtype=torch.bfloat16, device="cuda")
+        for s in range(rows):
+            cache.begin_step([s], 3 + s)
+            cache.end_step()
+        cache.begin_step(list(range(rows)), 1)
+        got = model(ids, positions=pos, kv_cache=cache)
+        cache.end_step()
+        out.append((got, cache.k[0], cache.v[0]))
+    assert len(calls) == 1
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+    # the pool's rows against fp32 products
+    norm = model.model.layers[0].input_layernorm
+    h = norm(model.model.embed_tokens(ids))[:, 0].float()
+    k, v = ((h @ w.t() + b).view(rows, kv_heads, 128) for w, b in refs[1:])
+    inv = cfg.rope_theta ** (-torch.arange(64, device="cuda") / 64.0)
+    c, s = (f(pos * inv)[:, None] for f in (torch.cos, torch.sin))
+    k1, k2 = k[..., :64], k[..., 64:]
+    k = torch.cat([k1 * c - k2 * s, k2 * c + k1 * s], -1)
+    for pool, want in ((out[0][1], k), (out[0][2], v)):
+        rows_of = torch.stack([
+            pool[cache.block_table[r][(3 + r) // cache.block_size], :,
+                 (3 + r) % cache.block_size].float() for r in range(rows)])
+        # bf16 outputs, and int8 weights within half a step of max / 127
+        bound = 0.02 if int8 else 0.006
+        assert (rows_of - want).norm() <= bound * want.norm()
+
+
 class _Strided(llama.LlamaDecoderLayer):
     """Hands on a stream that lies across."""
 
