@@ -633,6 +633,11 @@ int launch_stream(Args a, int layers, bool all, hipStream_t st) {
 //   * Gate and up, one pair: 896 pairs, K 4096 2 x 4 35.2, 35.0, 36.7, 4 x 4 35.7, 35.8,
 // 35.8; 352, K 2048 9.3, 9.9, 10.9 and 9.4, 9.7, 10.2; int8 21.2, 22.4, 25.5 and 21.4,
 // 21.7, 23.6; 176, K 1024 2 x 8 4.3, 4.5, 4.7, 2 x 4 4.6, 4.7, 4.9.
+//   * q, k and v, two or four: 384 tiles, K 4096 2 x 8 10.9, 10.8, 11.4, 4 x 4 14.7, 15.3,
+// 16.2, int8 8.7, 8.8, 9.4 and 13.1, 13.4, 14.7; 640, K 8192 29.0, 30.9, 33.4 and 28.2,
+// 28.6, 30.0; 768, K 4096 18.1, 18.9, 20.1 and 19.3, 19.5, 19.8; int8 of 640 2 x 8 / 2 x 4
+// / 4 x 4 20.4, 22.7, 26.1 / 20.5, 22.2, 25.7 / 21.3, 22.0, 23.6, of 576, K 3072 11.1,
+// 11.7, 13.1 / 10.8, 11.1, 12.3 / 11.7, 12.0, 12.9.
 //   * 17 to 32 rows of int8: 256 tiles, K 4096 1 x 4 8.8, 2 x 4 10.6; 384 14.7 and 11.0.
 template <bool I8, int XR>
 int launch_streams(const Args& a, int layers, int mode, int tiles,
@@ -661,9 +666,8 @@ int launch_streams(const Args& a, int layers, int mode, int tiles,
     }
     STREAM(4, 4, 2, SWIGLU, false);
   } else if (mode == QKV) {
-    if (I8 ? tiles <= 512 && a.M <= 8 : tiles <= 512 || few)
-      STREAM(2, 8, 2, QKV, false);
-    if (I8 && (tiles <= 512 || few)) STREAM(2, 4, 2, QKV, false);
+    if (tiles <= 512 || (!I8 && a.M <= 4)) STREAM(2, 8, 2, QKV, false);
+    if (I8 && a.M <= 8) STREAM(2, 4, 2, QKV, false);
     STREAM(4, 4, 2, QKV, false);
   } else {
     if (tiles <= 256) STREAM(1, 8, 2, PLAIN, false);
