@@ -480,7 +480,7 @@ def chunked_cross_entropy(hidden, lm_head, labels, chunk_tokens=8192):
     the per-chunk softmax+nll runs as the fused bf16 HIP kernel and no
     fp32 logits are materialized at all."""
     from ..ops.cross_entropy import (fused_cross_entropy_mean,
-                                     fused_cross_entropy_sum)
+                                     fused_cross_entropy_sum, head_loss_fits)
     B, S, H = hidden.shape
     hidden = hidden.reshape(-1, H)
     labels = labels.reshape(-1)
@@ -489,6 +489,11 @@ def chunked_cross_entropy(hidden, lm_head, labels, chunk_tokens=8192):
         if labels.shape[0] > n:
             labels = labels[:n]
         return fused_cross_entropy_mean(call(lm_head, hidden), labels)
+    if n and labels.shape[0] >= n and labels.dtype is torch.long and \
+            head_loss_fits(lm_head, hidden):
+        total, count = lm_head(hidden, loss=(labels[:n].contiguous(),
+                                             chunk_tokens))
+        return total / count.clamp(min=1)
     total = hidden.new_zeros((), dtype=torch.float32)
     count = hidden.new_zeros((), dtype=torch.float32)
     for s in range(0, n, chunk_tokens):

@@ -10,6 +10,7 @@ import os
 
 import torch
 
+from . import linear
 from ._loader import get_ext
 
 
@@ -34,6 +35,83 @@ class _FusedCE(torch.autograd.Function):
         d = get_ext().ce_bwd(logits, labels, lse, g.contiguous().float(),
                              ctx.ignore_index, count)
         return d, None, None, None
+
+
+class _HeadLoss(torch.autograd.Function):
+    """(sum of the rows' losses, labels that count) of the logits x W^T, in chunks
+    of rows. As one node: the chunks' gradients of W are added up by the products,
+    those of x are made in their places and W is transposed once, where slices and
+    calls of a head each clear, fill and add up gradients of all rows and of W
+    (32768 rows of 4096, 128256 features in four chunks: 3.4 of 162 ms)."""
+
+    @staticmethod
+    def forward(ctx, x, weight, labels, rows, ignore_index):
+        ctx.slot = linear.uses(weight)
+        ctx.rows, ctx.ignore_index = rows, ignore_index
+        total, count, kept = None, None, []
+        for xs, ys in zip(x.split(rows), labels.split(rows)):
+            logits = linear._forward(xs, [weight], [None])[0]
+            t, c, _, lse = get_ext().ce_loss(logits, ys, ignore_index)
+            total = t if total is None else total + t
+            count = c if count is None else count + c
+            kept += logits, lse
+        ctx.save_for_backward(x, weight, labels, *kept)
+        ctx.mark_non_differentiable(count)
+        return total, count
+
+    @staticmethod
+    def backward(ctx, g, _gcount):
+        x, w, labels, *kept = ctx.saved_tensors
+        rows, (need_x, need_w) = ctx.rows, ctx.needs_input_grad[:2]
+        g = g.contiguous().float()
+        parts = list(zip(x.split(rows), labels.split(rows), kept[::2],
+                         kept[1::2]))
+
+        def gradient(part):
+            return get_ext().ce_bwd(part[2], part[1], part[3], g,
+                                    ctx.ignore_index, None)
+        if torch.is_grad_enabled():     # differentiated themselves
+            ds = [gradient(p) for p in parts]
+            dx = torch.cat([d @ w for d in ds]) if need_x else None
+            dw = sum(d.t() @ p[0] for d, p in zip(ds, parts)) \
+                if need_w else None
+            return dx, dw, None, None, None
+        dx = torch.empty_like(x) if need_x else None
+        dw = turned = None
+        for i, part in enumerate(parts):
+            d = gradient(part)
+            n = d.shape[0]
+            if need_x:
+                to = dx[i * rows:i * rows + n]
+                if linear.own_dx(n, w.shape[:1], w.shape[1]) and \
+                        linear._aligned(d, w):
+                    to.copy_(linear._dx([d], [w], True))
+                elif linear.backward_plan(n, *w.shape)[0]:
+                    if turned is None:
+                        turned = linear._transposed(w)
+                    torch.mm(d, turned.t(), out=to)
+                else:
+                    torch.mm(d, w, out=to)
+            if need_w and i:
+                linear.add_dw(dw, part[0], d)
+            elif need_w:
+                dw = linear._dw(part[0], [d], True, [need_x and ctx.slot])[0]
+        return dx, dw, None, None, None
+
+
+def head_loss(x, weight, labels, rows, ignore_index=-100):
+    return _HeadLoss.apply(x, weight, labels, rows, ignore_index)
+
+
+def head_loss_fits(head, x) -> bool:
+    """A head without bias of the framework's own, watched by its own hooks at
+    most, and rows with gradients: one that takes ``loss``."""
+    return (type(head) is linear.Linear and head.bias is None
+            and linear.unhooked(head, internal_ok=True)
+            and x.is_contiguous() and linear._differentiable(x, ())
+            and type(head.weight) is torch.nn.Parameter
+            and head.weight.dtype is torch.bfloat16
+            and fused_ce_available(x))
 
 
 def fused_ce_available(logits) -> bool:

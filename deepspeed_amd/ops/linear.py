@@ -219,11 +219,11 @@ def _dx(dys, weights, own: bool):
         return get_ext().tile_linear_dx(dys, weights)
     dx = None
     for dy, w in zip(dys, weights):
-        if own and backward_plan(T, *w.shape)[0]:
-            part = nn.functional.linear(dy, _transposed(w))
-        else:
-            part = dy @ w
-        dx = part if dx is None else dx + part
+        b = _transposed(w).t() if own and backward_plan(T, *w.shape)[0] else w
+        if dx is None:
+            dx = dy @ b
+        else:       # by the product itself: two reads and a write less
+            dx = dx.addmm_(dy, b) if own else dx + dy @ b
     return dx
 
 
@@ -303,13 +303,24 @@ def _dw(x, dys, own: bool, slots):
                 for dy, out in zip(dys, into)]
     dws = []
     for dy, out in zip(dys, into):
-        dy_t = x_t = False
-        if own:
-            _, dy_t, x_t = backward_plan(T, dy.shape[1], K)
-        a = _transposed(dy) if dy_t else dy.t()
-        b = _transposed(x).t() if x_t else x
+        a, b = _across(x, dy) if own else (dy.t(), x)
         dws.append(a @ b if out is None else torch.mm(a, b, out=out))
     return dws
+
+
+def _across(x, dy):
+    """Operands of the library's dy^T x, laid out as ``backward_plan`` says."""
+    _, dy_t, x_t = backward_plan(x.shape[0], dy.shape[1], x.shape[1])
+    return (_transposed(dy) if dy_t else dy.t(),
+            _transposed(x).t() if x_t else x)
+
+
+def add_dw(dw, x, dy):
+    """dw += dy^T x."""
+    if own_dw(x.shape[0], *dw.shape) and _aligned(x, dy):
+        dw += get_ext().tile_linear_dw(x, [dy], into=[None])[0]
+    else:
+        dw.addmm_(*_across(x, dy))
 
 
 class _Linears(torch.autograd.Function):
@@ -437,10 +448,14 @@ def _differentiable(x, weights) -> bool:
 @movable
 class Linear(nn.Linear):
     """nn.Linear with the backward of ``_Linears`` on a GPU, and with ``own`` its
-    forward."""
+    forward. ``loss``, labels and rows a chunk: ``head_loss`` in the place of
+    outputs."""
 
-    def forward(self, x, own: bool = False):
+    def forward(self, x, own: bool = False, loss=None):
         w = self.weight
+        if loss is not None:
+            from .cross_entropy import head_loss
+            return head_loss(x, w, *loss)
         if _differentiable(x, (w,)):
             T = x.numel() // w.shape[1]
             if any(own_products(T, *w.shape)) or \

@@ -1,0 +1,79 @@
+"""The head's loss over chunks of rows as one node (ops/cross_entropy.py)."""
+
+import pytest
+import torch
+
+from deepspeed_amd.models.llama import chunked_cross_entropy
+from deepspeed_amd.ops import cross_entropy, linear
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,rows", [(300, 128), (512, 256), (257, 256),
+                                    (6400, 3200), (6144, 3200), (9000, 8192)])
+@pytest.mark.parametrize("v", [1000, 1088])
+@pytest.mark.parametrize("frozen", [None, "x", "w"])
+def test_against_fp32_gpu(n, rows, v, frozen):
+    """Whole and ragged chunks; products of the library and of the kernels, with
+    and without transposed copies; one of the gradients not asked for."""
+    g = torch.Generator(device="cuda").manual_seed(n + v)
+    h = 1024 if rows > 3000 else 256
+    x = torch.randn(1, n, h, device="cuda", generator=g).bfloat16()
+    head = linear.Linear(h, v, bias=False).to("cuda", torch.bfloat16)
+    head.weight.data.normal_(0.0, 0.05, generator=g)
+    labels = torch.randint(0, v, (n,), device="cuda", generator=g)
+    labels[::7] = -100
+    x.requires_grad_(frozen != "x")
+    head.weight.requires_grad_(frozen != "w")
+    assert cross_entropy.head_loss_fits(head, x.view(n, h))
+    loss = chunked_cross_entropy(x, head, labels, rows)
+    loss.backward()
+    xr, wr = (t.detach().float().requires_grad_() for t in (x, head.weight))
+    # logits, as they are kept, are rounded to bf16
+    logits = xr[0] @ wr.t()
+    logits = logits + (logits.detach().bfloat16().float() - logits.detach())
+    want = torch.nn.functional.cross_entropy(logits, labels)
+    want.backward()
+    # fp32 sums over bf16 logits, some of which the order of a product's sums
+    # rounds the other way; gradients through bf16 ones: 2^-9 a rounding
+    assert abs(loss.item() - want.item()) <= 1e-4 * want.item()
+    for t, r in ((x, xr), (head.weight, wr)):
+        if not t.requires_grad:
+            assert t.grad is None
+            continue
+        err = (t.grad.float() - r.grad).norm() / r.grad.norm()
+        assert err < 2 ** -7
+
+
+@pytest.mark.gpu
+def test_same_as_chunk_by_chunk_gpu(monkeypatch):
+    """Loss bit by bit, gradients but for their roundings; a hooked head and one of
+    another class are called."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn(2, 300, 256, device="cuda", generator=g).bfloat16()
+    head = linear.Linear(256, 640, bias=False).to("cuda", torch.bfloat16)
+    labels = torch.randint(0, 640, (600,), device="cuda", generator=g)
+    out = []
+    for own in (True, False):
+        if not own:
+            monkeypatch.setattr(cross_entropy, "head_loss_fits",
+                                lambda *a: False)
+        leaf = x.detach().clone().requires_grad_()
+        head.weight.grad = None
+        loss = chunked_cross_entropy(leaf, head, labels, 256)
+        loss.backward()
+        out.append((loss.detach(), leaf.grad, head.weight.grad))
+    assert torch.equal(out[0][0], out[1][0])
+    for a, b in zip(out[0][1:], out[1][1:]):
+        assert (a.float() - b.float()).norm() <= 2 ** -7 * b.float().norm()
+    monkeypatch.undo()
+    flat = x.view(600, 256).requires_grad_()
+    seen = []
+    hook = head.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    assert not cross_entropy.head_loss_fits(head, flat)
+    chunked_cross_entropy(flat[None], head, labels, 256)
+    assert seen == [(256, 640), (256, 640), (88, 640)]
+    hook.remove()
+    other = torch.nn.Linear(256, 640, bias=False).to("cuda", torch.bfloat16)
+    assert not cross_entropy.head_loss_fits(other, flat)
+    with torch.no_grad():
+        assert not cross_entropy.head_loss_fits(head, flat)
