@@ -581,10 +581,11 @@ __device__ __forceinline__ unsigned packed2(float lo, float hi) {
                             __builtin_convertvector((f32x2{lo, hi}), b16x2));
 }
 
-// The largest tiles, 256 x 256, by four waves of 128 x 128, one a SIMD: a wave's
-// 256 sums are the accumulation registers, and LDS is read for 64 products of a
-// half stage by 16 operands (eight waves of 128 x 64: 12 for 32). The chip's power
-// bounds these products, so reads that are not made become clock.
+// The largest tiles, 256 x 256, by four waves of 128 x 128, one a SIMD (FW: tiles of 16
+// columns a wave; with six of them 256 x 192): a wave's 256 sums are the accumulation
+// registers, and LDS is read for 64 products of a half stage by 16 operands (eight
+// waves of 128 x 64: 12 for 32). The chip's power bounds these products, so reads that
+// are not made become clock.
 //
 //   * A tile a workgroup. One that goes on from tile to tile, its ring filled across
 // the border, gains up to 1.3% alone on the chip (2.5 at K 2048, 4.5 at 1024), but
@@ -610,12 +611,15 @@ __device__ __forceinline__ unsigned packed2(float lo, float hi) {
 // K 4096: 28672 696 / 648, 6144 166 / 159, gate and up 14336 712 / 680; gate and up
 // 18944, K 3584, 2331 rows 536 / 503; dx of 14336, K 4096, 8192 rows 745 / 706; dW of
 // that 789 / 727 (its transposing reads are two an operand).
-template <int MODE, bool PARTS, bool ONCE>
+template <int MODE, bool PARTS, bool ONCE, int FW = 8>
 __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   constexpr bool GLU = MODE == SWIGLU;
   constexpr bool WT = MODE == GRAD_X || MODE == GRAD_W, XT = MODE == GRAD_W;
-  constexpr int BM = 256, BN = 256, F = 8;      // tiles of 16 a wave, either way
-  constexpr int P = 8;                          // loads of 1 KB a wave, each
+  constexpr int F = 8;      // tiles of 16 a wave: of rows, FW of columns
+  constexpr int BM = 256, BN = 32 * FW;
+  constexpr int P = F, PW = FW;     // loads of 1 KB a wave: of x, of W
+  static_assert(FW == 8 || (FW == 6 && !PARTS && (MODE == PLAIN || MODE == GRAD_X)),
+                "");
   constexpr int SW = BN * ROW, SX = BM * ROW, XAT = 3 * SW;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int lane = threadIdx.x & 63;
@@ -670,9 +674,10 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       return (unsigned)(piece % 8 * 8 + lr) * K * 2 +
           2 * (piece / 8 * 64 +
                8 * (lc ^ (2 * ((lr >> 1) & 1) + 4 * (wid & 1))));
-    // tile f of a wave: features F c + f, or gate and up of 4 c + f / 2
-    const int half = piece / 16, f = piece / 2 % 8, c = piece % 2 * 8 + lr;
-    const int r = GLU ? half * 64 + F / 2 * c + (f >> 1) : half * 128 + F * c + f;
+    // tile f of a wave: features FW c + f, or gate and up of 4 c + f / 2
+    const int half = piece / (2 * FW), f = piece / 2 % FW, c = piece % 2 * 8 + lr;
+    const int r = GLU ? half * 64 + FW / 2 * c + (f >> 1)
+                      : half * 16 * FW + FW * c + f;
     return (unsigned)r * K * 2 + ((lc ^ lr) << 4);
   };
   auto place_x = [&](int j, int ld) INLINE {
@@ -683,12 +688,11 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
                8 * (lc ^ (2 * ((lr >> 1) & 1) + 4 * (wid & 1))));
     return (unsigned)(piece * 8 + lr) * ld * 2 + ((lc ^ lr) << 4);
   };
-  unsigned woff[P], xoff[P];
+  unsigned woff[PW], xoff[P];
 #pragma unroll
-  for (int j = 0; j < P; ++j) {
-    woff[j] = place_w(j);
-    xoff[j] = place_x(j, K);
-  }
+  for (int j = 0; j < PW; ++j) woff[j] = place_w(j);
+#pragma unroll
+  for (int j = 0; j < P; ++j) xoff[j] = place_x(j, K);
   // From contraction step `step` of a tile on: descriptor, bytes to its end (the
   // operands that lie across move it), stages that follow one another there.
   u32x4 wfrom, xfrom;
@@ -798,7 +802,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   };
   auto fill_w = [&]() INLINE {
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
+    for (int j = 0; j < PW; ++j) {
       load_to(wput, j * 4096);
       asm volatile("s_nop 0");
       load<ONCE>(wfrom, woff[j], wsoff);
@@ -820,7 +824,8 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   };
 
   // ---- operands: 16 rows (or columns) by inputs 32 h + 8 g + j, at the lane's
-  // addresses and constants. Across, tiles of 16 columns have four of them.
+  // addresses and constants. Across, tiles of 16 columns have four of them, or where
+  // a wave does not begin with a block of 64 one each.
   const int tr = (8 * g + (col >> 2)) * 128 + (col & 3) * 8 +
       32 * ((col >> 3) & 1) + 64 * (g & 1);
   const int o0 = (g ^ (col & 7)) << 4;
@@ -828,12 +833,15 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
                     : lds_at + (wn * (BN / 2) + col) * ROW + o0;
   const int x0 = XAT + (XT ? lds_at + wm * 16384 + tr
                            : lds_at + (wm * (BM / 2) + col) * ROW + o0);
-  int wat[WT ? 4 : 1], xat[XT ? 4 : 1];
+  constexpr int WA = !WT ? 1 : FW == 8 ? 4 : FW;
+  int wat[WA], xat[XT ? 4 : 1];
   auto aim = [&](int h) INLINE {    // at a half of the stage
     if (!WT || h == 0)
 #pragma unroll
-      for (int c = 0; c < (WT ? 4 : 1); ++c) {
-        wat[c] = (w0 ^ (WT ? 32 * c : 64 * h)) + wget;
+      for (int c = 0; c < WA; ++c) {
+        const int t = wn * FW + c;
+        if (WT && FW < 8) wat[c] = lds_at + t / 4 * 8192 + (tr ^ t % 4 * 32) + wget;
+        else wat[c] = (w0 ^ (WT ? 32 * c : 64 * h)) + wget;
         asm volatile("" : "+v"(wat[c]));
       }
     if (!XT || h == 0)
@@ -843,19 +851,19 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
         asm volatile("" : "+v"(xat[c]));
       }
   };
-  s16x8 wa[2][F], xa[2][F];
+  s16x8 wa[2][FW], xa[2][F];
   auto across = [&](int at, int i, int h) INLINE {
     const s16x4 lo = lds_tr_read(at + i / 4 * 8192 + h * 4096);
     const s16x4 hi = lds_tr_read(at + i / 4 * 8192 + h * 4096 + 512);
     return s16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
   };
   auto get = [&](int q, int h) INLINE {
-    if (q < F)
-      wa[h][q] = WT ? across(wat[WT ? q % 4 : 0], q, h)
+    if (q < FW)
+      wa[h][q] = WT ? across(wat[q % WA], FW == 8 ? q : 0, h)
                     : lds_read(wat[0] + q * 16 * ROW);
     else
-      xa[h][q - F] = XT ? across(xat[XT ? q % 4 : 0], q - F, h)
-                        : lds_read(xat[0] + (q - F) * 16 * ROW);
+      xa[h][q - FW] = XT ? across(xat[XT ? q % 4 : 0], q - FW, h)
+                         : lds_read(xat[0] + (q - FW) * 16 * ROW);
   };
   // sums of a tile of W and one of x
 #define acc(f, m) (((f) * F + (m)) * 4)
@@ -868,26 +876,28 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   fill_w();
   fill_x();
   fill_w();
-  wait_loads<3 * P>();
+  wait_loads<2 * PW + P>();
   barrier();
   aim(0);
 #pragma unroll
-  for (int q = 0; q < 2 * F; ++q) get(q, 0);
+  for (int q = 0; q < FW + F; ++q) get(q, 0);
 
-  // A stage's 128 products. Reads of its second half lie between the first ones,
+  // A stage's 16 FW products. Reads of its second half lie between the first ones,
   // those of the next stage's first half behind the middle; x two stages ahead and
   // W three are loaded behind the barrier.
-  constexpr int N2 = 2 * F * F, BARRIER = 30;
+  constexpr int N1 = F * FW, N2 = 2 * N1, BARRIER = FW == 8 ? 30 : 24;
+  constexpr int X1 = BARRIER + 2, XN = FW == 8 ? 6 : 4;     // loads of x and of W: the
+  constexpr int W1 = FW == 8 ? BARRIER + 52 : 58, WN = 6;   // first one's product, a step
   auto stage = [&](auto first) INLINE {
     constexpr bool FIRST = decltype(first)::value;
     __builtin_amdgcn_sched_barrier(0);
     wait_reads();
     aim(1);
     auto product = [&](auto at) INLINE {
-      constexpr int i = decltype(at)::value, h = i / (F * F), m = i / F % F;
-      constexpr int f = m % 2 ? F - 1 - i % F : i % F;
+      constexpr int i = decltype(at)::value, h = i / N1, m = i / FW % F;
+      constexpr int f = m % 2 ? FW - 1 - i % FW : i % FW;
       if constexpr (i == BARRIER) {
-        wait_loads<P>();
+        wait_loads<PW>();
         wait_reads();
         __builtin_amdgcn_s_barrier();
         wget = next_w(wget, 0);
@@ -897,14 +907,14 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       }
 #pragma unroll
       for (int q = 0; q < P; ++q) {
-        if (i == BARRIER + 2 + 6 * q) load_to(xput, q * 4096);
-        if (i == BARRIER + 52 + 6 * q) load_to(wput, q * 4096);
+        if (i == X1 + XN * q) load_to(xput, q * 4096);
+        if (q < PW && i == W1 + WN * q) load_to(wput, q * 4096);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int q = 0; q < 2 * F; ++q) {
+      for (int q = 0; q < FW + F; ++q) {
         if (i == q * 3 / 2) get(q, 1);
-        if (i == 66 + 3 * q) get(q, 0);
+        if (i == N1 + 2 + 3 * q) get(q, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
       const s16x8 u = WT ? wa[h][f] : xa[h][m], v = WT ? xa[h][m] : wa[h][f];
@@ -913,8 +923,8 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int q = 0; q < P; ++q) {
-        if (i == BARRIER + 2 + 6 * q) load<false>(xfrom, xoff[q], xsoff);
-        if (i == BARRIER + 52 + 6 * q) load<ONCE>(wfrom, woff[q], wsoff);
+        if (i == X1 + XN * q) load<false>(xfrom, xoff[q], xsoff);
+        if (q < PW && i == W1 + WN * q) load<ONCE>(wfrom, woff[q % PW], wsoff);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -998,10 +1008,11 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
             u32x4{lo[0], hi[0], lo[1], hi[1]}, to,
             n < N ? (unsigned)((16 * m + col) * N + n) * 2 : NOWHERE, 0, STREAM);
       };
-      each(std::make_integer_sequence<int, F / 2 * F>{}, store);
+      each(std::make_integer_sequence<int, FW / 2 * F>{}, store);
     } else {
-      constexpr int W = GLU ? F / 2 : F;      // features a lane
+      constexpr int W = GLU ? FW / 2 : FW;    // features a lane
       const int n = at.n0 + wn * (GLU ? BN / 4 : BN / 2) + W * col;
+      const bool at_edge = at.n0 + BN > N;
       float b[GLU ? 2 : 1][W];
       const bool biased = a.bias[GLU ? 0 : at.layer] || (GLU && a.bias[1]);
       if (biased)
@@ -1033,9 +1044,22 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
         };
         const u32x2 v = {packed2(one(Int<0>{}), one(Int<1>{})),
                          packed2(one(Int<2>{}), one(Int<3>{}))};
-        if constexpr (GLU)
+        if constexpr (GLU) {
           __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, STREAM);
-        else {
+        } else if constexpr (FW == 6) {
+          typedef unsigned u32x3 __attribute__((ext_vector_type(3)));
+          const unsigned u = packed2(one(Int<4>{}), one(Int<5>{}));
+          if (at_edge) {      // N is a multiple of four, six features may pass it
+            __builtin_amdgcn_raw_buffer_store_b32(v[0], to, o, 0, STREAM);
+            __builtin_amdgcn_raw_buffer_store_b32(
+                v[1], to, n + 2 < N ? o + 4 : NOWHERE, 0, STREAM);
+            __builtin_amdgcn_raw_buffer_store_b32(
+                u, to, n + 4 < N ? o + 8 : NOWHERE, 0, STREAM);
+          } else {
+            __builtin_amdgcn_raw_buffer_store_b96(u32x3{v[0], v[1], u}, to, o, 0,
+                                                  STREAM);
+          }
+        } else {
           const u32x2 u = {packed2(one(Int<4>{}), one(Int<5>{})),
                            packed2(one(Int<6>{}), one(Int<7>{}))};
           if (N % 8 == 0) {
@@ -1171,6 +1195,19 @@ int launch_wide(Args a, bool merge, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+// 256 x 192 by four waves, too.
+template <int MODE>
+int launch_wide192(Args a, hipStream_t st) {
+  constexpr int LDS = (3 * 192 + 2 * 256) * ROW;
+  const int items = count<256, 192, MODE>(a);
+  auto kernel = wide_linear_kernel<MODE, false, false, 6>;
+  const hipError_t e = hipFuncSetAttribute(
+      (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL(kernel, dim3(items), dim3(256), LDS, st, a);
+  return (int)hipGetLastError();
+}
+
 // What the largest tile does not take: outputs are stored at 32-bit offsets in 128
 // rows of ``columns`` sums, and the rows that GRAD_X reads lie behind a descriptor of
 // less than 2^32 bytes, which 256 rows of 2^23 features fill.
@@ -1193,6 +1230,15 @@ bool past_wide(int mode, double columns, int most) {
   X(6, 192, 256, 4, 2, 2, 1.047f, 6.3f)    \
   X(7, 256, 128, 4, 2, 3, 0.754f, 5.2f)    \
   X(8, 256, 192, 2, 4, 2, 1.023f, 6.3f)
+// 256 x 192 is wide_linear_kernel's as well, of several tiles of rows and whole
+// contractions, forward and the input's gradient (us by eight waves of 128 x 48, which
+// LDS bounds, and four of 128 x 96: 4000 rows 9216, K 3072 179.0 / 168.6, 3072, K 8192
+// 148.6 / 141.1, 4096 rows 3072, K 3072 67.1 / 61.0; input's gradient of 9216, K 3072
+// 211 / 188, of 32064 670 / 631).
+constexpr int NARROW = 8;
+bool narrow_by_four(int M, int splits, int mode) {
+  return splits == 1 && M > 256 && (mode == PLAIN || mode == GRAD_X);
+}
 constexpr int WIDE = 9;
 // 192 x 192, for what lies between the rounds of the others (us, the choice without it /
 // this; over 500 layers that it is chosen for 0.94 of one's or several layers' forward,
@@ -1309,6 +1355,7 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
       if (steps / s < t.stages) break;
       float us = estimate(t, tiles, steps, rows, columns, bytes, s, mode);
       if (i == SQUARE && mode == GRAD_X) us *= 1.04f;
+      if (i == NARROW && narrow_by_four(M, s, mode)) us *= 0.95f;
       if (best < 0 || us < least) {
         best = i;
         least = us;
@@ -1358,6 +1405,10 @@ extern "C" int ds_tile_linear(const void* const* x, int layers,
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (tile == WIDE && past_wide(mode, mode >= GRAD_X ? K : total, most))
     return (int)hipErrorInvalidValue;
+  if (tile == NARROW && narrow_by_four(M, splits, mode) &&
+      !past_wide(mode, mode >= GRAD_X ? K : total, most))
+    return mode == GRAD_X ? launch_wide192<GRAD_X>(a, st)
+                          : launch_wide192<PLAIN>(a, st);
   switch (tile) {
 #define X(I, BM, BN, WM, WN, NS, U, F)                                    \
   case I:                                                                 \

@@ -212,6 +212,30 @@ def test_widest_tile_in_rounds_gpu(steps):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("steps", [2, 3, 4, 5, 9])
+@torch.no_grad()
+def test_narrow_tile_by_four_waves_gpu(steps):
+    """256 x 192 of several tiles of rows: features that end anywhere in a lane's six
+    and in a tile, layers that end in one, columns of the input's gradient."""
+    from deepspeed_amd.ops import _C
+    tile, k = TILES.index((256, 192, 2)), 64 * steps
+    for m, ns in ((257, (196,)), (513, (580, 4, 188)), (700, (1000, 392)),
+                  (2600, (3076,))):
+        x, ws, bs = _inputs(m, ns, k, steps)
+        for biases in (bs, [None] * len(ns)):
+            for y, want in zip(_C.tile_linear(x, ws, biases, 0, tile, 1),
+                               _want(x, ws, biases, 0)):
+                _close(y, want)
+    for m, ns, k in ((257, (64 * steps,), 200), (700, (64 * (steps - 1), 64), 376),
+                     (2600, (64, 64 * steps, 128), 3080)):
+        _, ws, _ = _inputs(1, ns, k, steps)
+        dys = [_inputs(m, (), n, n)[0] for n in ns]
+        want = sum(d.double() @ w.double() for d, w in zip(dys, ws))
+        err = (_C.tile_linear_dx(dys, ws, tile, 1).double() - want).abs()
+        assert (err <= _limit(want, sum(ns))).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m,ns,k,mode,tile", [
     (40, (20000,), 2048, 0, 0), (33, (9000, 9000), 4096, SWIGLU, 1),
     (100, (8200, 4100), 2048, 0, 3), (190, (16396,), 4096, 0, 6),
