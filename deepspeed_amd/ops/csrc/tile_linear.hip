@@ -581,8 +581,8 @@ __device__ __forceinline__ unsigned packed2(float lo, float hi) {
                             __builtin_convertvector((f32x2{lo, hi}), b16x2));
 }
 
-// The largest tiles, 256 x 256, by four waves of 128 x 128, one a SIMD (FW: tiles of 16
-// columns a wave; with six of them 256 x 192): a wave's 256 sums are the accumulation
+// The largest tiles, 256 x 256, by four waves of 128 x 128, one a SIMD (FX, FW: tiles of
+// 16 rows and columns a wave; with six of either 192): a wave's sums are its accumulation
 // registers, and LDS is read for 64 products of a half stage by 16 operands (eight
 // waves of 128 x 64: 12 for 32). The chip's power bounds these products, so reads that
 // are not made become clock.
@@ -611,15 +611,15 @@ __device__ __forceinline__ unsigned packed2(float lo, float hi) {
 // K 4096: 28672 696 / 648, 6144 166 / 159, gate and up 14336 712 / 680; gate and up
 // 18944, K 3584, 2331 rows 536 / 503; dx of 14336, K 4096, 8192 rows 745 / 706; dW of
 // that 789 / 727 (its transposing reads are two an operand).
-template <int MODE, bool PARTS, bool ONCE, int FW = 8>
+template <int MODE, bool PARTS, bool ONCE, int FX = 8, int FW = 8>
 __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   constexpr bool GLU = MODE == SWIGLU;
   constexpr bool WT = MODE == GRAD_X || MODE == GRAD_W, XT = MODE == GRAD_W;
-  constexpr int F = 8;      // tiles of 16 a wave: of rows, FW of columns
-  constexpr int BM = 256, BN = 32 * FW;
-  constexpr int P = F, PW = FW;     // loads of 1 KB a wave: of x, of W
-  static_assert(FW == 8 || (FW == 6 && !PARTS && (MODE == PLAIN || MODE == GRAD_X)),
-                "");
+  constexpr int BM = 32 * FX, BN = 32 * FW;
+  constexpr int P = FX, PW = FW;    // loads of 1 KB a wave: of x, of W
+  static_assert((FX == 8 && FW == 8) ||
+                ((FX == 8 || FX == 6) && (FW == 8 || FW == 6) && !PARTS && !ONCE &&
+                 (FW == 8 || !GLU)), "");
   constexpr int SW = BN * ROW, SX = BM * ROW, XAT = 3 * SW;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int lane = threadIdx.x & 63;
@@ -833,8 +833,8 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
                     : lds_at + (wn * (BN / 2) + col) * ROW + o0;
   const int x0 = XAT + (XT ? lds_at + wm * 16384 + tr
                            : lds_at + (wm * (BM / 2) + col) * ROW + o0);
-  constexpr int WA = !WT ? 1 : FW == 8 ? 4 : FW;
-  int wat[WA], xat[XT ? 4 : 1];
+  constexpr int WA = !WT ? 1 : FW == 8 ? 4 : FW, XA = !XT ? 1 : FX == 8 ? 4 : FX;
+  int wat[WA], xat[XA];
   auto aim = [&](int h) INLINE {    // at a half of the stage
     if (!WT || h == 0)
 #pragma unroll
@@ -846,12 +846,15 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       }
     if (!XT || h == 0)
 #pragma unroll
-      for (int c = 0; c < (XT ? 4 : 1); ++c) {
-        xat[c] = (x0 ^ (XT ? 32 * c : 64 * h)) + xget;
+      for (int c = 0; c < XA; ++c) {
+        const int t = wm * FX + c;
+        if (XT && FX < 8)
+          xat[c] = lds_at + XAT + t / 4 * 8192 + (tr ^ t % 4 * 32) + xget;
+        else xat[c] = (x0 ^ (XT ? 32 * c : 64 * h)) + xget;
         asm volatile("" : "+v"(xat[c]));
       }
   };
-  s16x8 wa[2][FW], xa[2][F];
+  s16x8 wa[2][FW], xa[2][FX];
   auto across = [&](int at, int i, int h) INLINE {
     const s16x4 lo = lds_tr_read(at + i / 4 * 8192 + h * 4096);
     const s16x4 hi = lds_tr_read(at + i / 4 * 8192 + h * 4096 + 512);
@@ -862,11 +865,11 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       wa[h][q] = WT ? across(wat[q % WA], FW == 8 ? q : 0, h)
                     : lds_read(wat[0] + q * 16 * ROW);
     else
-      xa[h][q - FW] = XT ? across(xat[XT ? q % 4 : 0], q - FW, h)
+      xa[h][q - FW] = XT ? across(xat[(q - FW) % XA], FX == 8 ? q - FW : 0, h)
                          : lds_read(xat[0] + (q - FW) * 16 * ROW);
   };
   // sums of a tile of W and one of x
-#define acc(f, m) (((f) * F + (m)) * 4)
+#define acc(f, m) (((f) * FX + (m)) * 4)
   take_sums();
 
   seek_w(at.n0, at.layer, at.s0, at.s0 + at.n_it);
@@ -880,21 +883,26 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   barrier();
   aim(0);
 #pragma unroll
-  for (int q = 0; q < FW + F; ++q) get(q, 0);
+  for (int q = 0; q < FW + FX; ++q) get(q, 0);
 
-  // A stage's 16 FW products. Reads of its second half lie between the first ones,
+  // A stage's 2 FX FW products. Reads of its second half lie between the first ones,
   // those of the next stage's first half behind the middle; x two stages ahead and
   // W three are loaded behind the barrier.
-  constexpr int N1 = F * FW, N2 = 2 * N1, BARRIER = FW == 8 ? 30 : 24;
-  constexpr int X1 = BARRIER + 2, XN = FW == 8 ? 6 : 4;     // loads of x and of W: the
-  constexpr int W1 = FW == 8 ? BARRIER + 52 : 58, WN = 6;   // first one's product, a step
+  constexpr int N1 = FX * FW, N2 = 2 * N1;
+  constexpr int BARRIER = N1 == 64 ? 30 : N1 == 48 ? 24 : 20;
+  // loads of x and of W: the first one's product, a step
+  constexpr int X1 = BARRIER + 2, XN = N1 == 64 ? 6 : FX == 6 && FW == 8 ? 5 : 4;
+  constexpr int W1 = N1 == 64 ? 82 : N1 == 36 ? 46 : FW == 8 ? 54 : 58;
+  constexpr int WN = N1 == 64 ? 6 : N1 == 36 ? 4 : FW == 8 ? 5 : 6;
+  static_assert((FW + FX - 1) * 3 / 2 < BARRIER && X1 + XN * (P - 1) < W1 &&
+                W1 + WN * (PW - 1) < N2 && N1 + 2 + 3 * (FW + FX - 1) < N2, "");
   auto stage = [&](auto first) INLINE {
     constexpr bool FIRST = decltype(first)::value;
     __builtin_amdgcn_sched_barrier(0);
     wait_reads();
     aim(1);
     auto product = [&](auto at) INLINE {
-      constexpr int i = decltype(at)::value, h = i / N1, m = i / FW % F;
+      constexpr int i = decltype(at)::value, h = i / N1, m = i / FW % FX;
       constexpr int f = m % 2 ? FW - 1 - i % FW : i % FW;
       if constexpr (i == BARRIER) {
         wait_loads<PW>();
@@ -906,13 +914,13 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int q = 0; q < P; ++q) {
-        if (i == X1 + XN * q) load_to(xput, q * 4096);
+      for (int q = 0; q < 8; ++q) {
+        if (q < P && i == X1 + XN * q) load_to(xput, q * 4096);
         if (q < PW && i == W1 + WN * q) load_to(wput, q * 4096);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int q = 0; q < FW + F; ++q) {
+      for (int q = 0; q < FW + FX; ++q) {
         if (i == q * 3 / 2) get(q, 1);
         if (i == N1 + 2 + 3 * q) get(q, 0);
         __builtin_amdgcn_sched_barrier(0);
@@ -922,8 +930,8 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       else add_product<acc(f, m)>(u, v);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int q = 0; q < P; ++q) {
-        if (i == X1 + XN * q) load<false>(xfrom, xoff[q], xsoff);
+      for (int q = 0; q < 8; ++q) {
+        if (q < P && i == X1 + XN * q) load<false>(xfrom, xoff[q % P], xsoff);
         if (q < PW && i == W1 + WN * q) load<ONCE>(wfrom, woff[q % PW], wsoff);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -964,10 +972,10 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
                 (MODE == PLAIN ? before : 0)),
         (short)0, (int)((unsigned)have * all * 4), 0x00020000);
     // gradients: row col, columns 4 g ..; otherwise rows 4 g + r, half of eight
-    const int n1 = at.n0 + wn * (BN / 2) + (WT ? 4 * g : F * col);
+    const int n1 = at.n0 + wn * (BN / 2) + (WT ? 4 * g : FX * col);
     const int r1 = WT ? col : 4 * g;
     auto store = [&](auto at) INLINE {
-      constexpr int m = decltype(at)::value / F, i = decltype(at)::value % F;
+      constexpr int m = decltype(at)::value / FX, i = decltype(at)::value % FX;
       constexpr int f = 4 * (i & 1), r = i >> 1;
       f32x4 v;
       if constexpr (WT)
@@ -982,7 +990,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
           __builtin_bit_cast(u32x4, v), to,
           n < N && row < have ? (unsigned)(row * all + n) * 4 : NOWHERE, 0, 0);
     };
-    each(std::make_integer_sequence<int, F * F>{}, store);
+    each(std::make_integer_sequence<int, FX * FX>{}, store);
   } else {
     // outputs pass the caches by, which hold what other tiles still read
     constexpr int STREAM = 2;
@@ -995,7 +1003,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       // change places with even ones of the second
       const int n1 = at.n0 + wn * (BN / 2) + (g & 1) * 16 + (g >> 1) * 8;
       auto store = [&](auto at) INLINE {
-        constexpr int f = decltype(at)::value / F * 2, m = decltype(at)::value % F;
+        constexpr int f = decltype(at)::value / FX * 2, m = decltype(at)::value % FX;
         constexpr int A = acc(f, m), B = acc(f + 1, m);
         const unsigned y0 = packed2(sum<A>(), sum<A + 1>());
         const unsigned y1 = packed2(sum<A + 2>(), sum<A + 3>());
@@ -1008,7 +1016,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
             u32x4{lo[0], hi[0], lo[1], hi[1]}, to,
             n < N ? (unsigned)((16 * m + col) * N + n) * 2 : NOWHERE, 0, STREAM);
       };
-      each(std::make_integer_sequence<int, FW / 2 * F>{}, store);
+      each(std::make_integer_sequence<int, FW / 2 * FX>{}, store);
     } else {
       constexpr int W = GLU ? FW / 2 : FW;    // features a lane
       const int n = at.n0 + wn * (GLU ? BN / 4 : BN / 2) + W * col;
@@ -1074,8 +1082,8 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       };
       auto with = [&](auto at) INLINE { store(Int<1>{}, at); };
       auto without = [&](auto at) INLINE { store(Int<0>{}, at); };
-      if (biased) each(std::make_integer_sequence<int, 4 * F>{}, with);
-      else each(std::make_integer_sequence<int, 4 * F>{}, without);
+      if (biased) each(std::make_integer_sequence<int, 4 * FX>{}, with);
+      else each(std::make_integer_sequence<int, 4 * FX>{}, without);
     }
   }
   wait_loads<0>();
@@ -1195,12 +1203,12 @@ int launch_wide(Args a, bool merge, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// 256 x 192 by four waves, too.
-template <int MODE>
-int launch_wide192(Args a, hipStream_t st) {
-  constexpr int LDS = (3 * 192 + 2 * 256) * ROW;
-  const int items = count<256, 192, MODE>(a);
-  auto kernel = wide_linear_kernel<MODE, false, false, 6>;
+// The next smaller tiles by four waves.
+template <int BM, int BN, int MODE>
+int launch_four(Args a, hipStream_t st) {
+  constexpr int LDS = (3 * BN + 2 * BM) * ROW;
+  const int items = count<BM, BN, MODE>(a);
+  auto kernel = wide_linear_kernel<MODE, false, false, BM / 32, BN / 32>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (e != hipSuccess) return (int)e;
@@ -1230,15 +1238,15 @@ bool past_wide(int mode, double columns, int most) {
   X(6, 192, 256, 4, 2, 2, 1.047f, 6.3f)    \
   X(7, 256, 128, 4, 2, 3, 0.754f, 5.2f)    \
   X(8, 256, 192, 2, 4, 2, 1.023f, 6.3f)
-// 256 x 192 is wide_linear_kernel's as well, of several tiles of rows and whole
-// contractions, forward and the input's gradient (us by eight waves of 128 x 48, which
-// LDS bounds, and four of 128 x 96: 4000 rows 9216, K 3072 179.0 / 168.6, 3072, K 8192
-// 148.6 / 141.1, 4096 rows 3072, K 3072 67.1 / 61.0; input's gradient of 9216, K 3072
-// 211 / 188, of 32064 670 / 631).
-constexpr int NARROW = 8;
-bool narrow_by_four(int M, int splits, int mode) {
-  return splits == 1 && M > 256 && (mode == PLAIN || mode == GRAD_X);
-}
+// 192 x 256, 256 x 192 and (SQUARE) 192 x 192 are wide_linear_kernel's as well: by eight
+// waves LDS bounds them (256 x 192: 1850 cycles of it for 1536 of products), by four of
+// 128 x 96 it does not. Whole contractions of several tiles of rows; one tile of rows and
+// splits, which memory bounds, keep the deeper ring. us by eight waves and four, forward
+// 4000 rows 9216, K 3072 179 / 160, 171 / 159, 178 / 165, 2331 rows 3584, K 18944 290 /
+// 259, 277 / 264, 256 / 239; gate and up 14336, K 4096, 4096 rows 766 / 710; the input's
+// gradient of 4000 rows 9216, K 3072 185 / 159, 177 / 161, 284 / 235; the weights' 230 /
+// 204, 220 / 204, 196 / 179.
+constexpr int LOW = 6, NARROW = 8;
 constexpr int WIDE = 9;
 // 192 x 192, for what lies between the rounds of the others (us, the choice without it /
 // this; over 500 layers that it is chosen for 0.94 of one's or several layers' forward,
@@ -1252,6 +1260,18 @@ constexpr int WIDE = 9;
 // 3072 in three splits of 256 x 256 508, in this 549).
 constexpr int SQUARE = 10;
 #define BETWEEN(X) X(SQUARE, 192, 192, 4, 2, 3, 0.804f, 6.3f)
+bool by_four(int tile, int M, int splits, int mode) {
+  if (splits > 1) return false;
+  if (tile == LOW) return mode == GRAD_W || M > 192;
+  if (tile != NARROW && tile != SQUARE) return false;
+  return mode == GRAD_W || (mode != SWIGLU && M > (tile == NARROW ? 256 : 192));
+}
+// Of the time by eight waves, which the table's terms are fitted to: by mode.
+float four_takes(int tile, int mode) {
+  static const float of[3][4] = {
+      {0.91f, 0.94f, 0.88f, 0.92f}, {0.95f, 1, 0.91f, 0.94f}, {0.935f, 1, 0.87f, 0.90f}};
+  return of[tile == LOW ? 0 : tile == NARROW ? 1 : 2][mode];
+}
 // The largest tile by eight waves, two a SIMD: a short contraction is as much its first
 // loads and its stores, which the waves make beside each other's products. In place of
 // WIDE up to so many stages. Over 7000 layers, of the four waves' time: gate and up
@@ -1354,8 +1374,8 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
       if (s > 1 && (mode == SWIGLU || tiles * s > 520)) break;
       if (steps / s < t.stages) break;
       float us = estimate(t, tiles, steps, rows, columns, bytes, s, mode);
-      if (i == SQUARE && mode == GRAD_X) us *= 1.04f;
-      if (i == NARROW && narrow_by_four(M, s, mode)) us *= 0.95f;
+      if (by_four(i, M, s, mode)) us *= four_takes(i, mode);
+      else if (i == SQUARE && mode == GRAD_X) us *= 1.04f;
       if (best < 0 || us < least) {
         best = i;
         least = us;
@@ -1405,10 +1425,18 @@ extern "C" int ds_tile_linear(const void* const* x, int layers,
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (tile == WIDE && past_wide(mode, mode >= GRAD_X ? K : total, most))
     return (int)hipErrorInvalidValue;
-  if (tile == NARROW && narrow_by_four(M, splits, mode) &&
-      !past_wide(mode, mode >= GRAD_X ? K : total, most))
-    return mode == GRAD_X ? launch_wide192<GRAD_X>(a, st)
-                          : launch_wide192<PLAIN>(a, st);
+  if (by_four(tile, M, splits, mode) &&
+      !past_wide(mode, mode >= GRAD_X ? K : total, most)) {
+#define FOUR(BM, BN)                                                    \
+  mode == GRAD_X ? launch_four<BM, BN, GRAD_X>(a, st)                   \
+      : mode == GRAD_W ? launch_four<BM, BN, GRAD_W>(a, st)             \
+      : launch_four<BM, BN, PLAIN>(a, st)
+    if (tile == SQUARE) return FOUR(192, 192);
+    if (tile == NARROW) return FOUR(256, 192);
+    if (mode == SWIGLU) return launch_four<192, 256, SWIGLU>(a, st);
+    return FOUR(192, 256);
+#undef FOUR
+  }
   switch (tile) {
 #define X(I, BM, BN, WM, WN, NS, U, F)                                    \
   case I:                                                                 \

@@ -23,7 +23,7 @@ DEVICE_FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950",
                 "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # The source whose kernels name accumulation registers, and how many these are: the
 # build ends where the compiler's assembly does not go with it.
-NAMING, KERNELS = os.path.join(CSRC, "tile_linear.hip"), 11
+NAMING, KERNELS = os.path.join(CSRC, "tile_linear.hip"), 19
 
 
 def _named_registers():

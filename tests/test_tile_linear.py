@@ -212,27 +212,44 @@ def test_widest_tile_in_rounds_gpu(steps):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("steps", [2, 3, 4, 5, 9])
+@pytest.mark.parametrize("tile,bm,bn,least", [
+    (6, 192, 256, 2), (8, 256, 192, 2), (10, 192, 192, 3)])
+@pytest.mark.parametrize("more", [0, 1, 2, 3, 7])
 @torch.no_grad()
-def test_narrow_tile_by_four_waves_gpu(steps):
-    """256 x 192 of several tiles of rows: features that end anywhere in a lane's six
-    and in a tile, layers that end in one, columns of the input's gradient."""
+def test_tiles_by_four_waves_gpu(tile, bm, bn, least, more):
+    """Several tiles of rows: features that end anywhere in a lane's eight or six and
+    in a tile, layers that end in one, gates, both gradients."""
     from deepspeed_amd.ops import _C
-    tile, k = TILES.index((256, 192, 2)), 64 * steps
-    for m, ns in ((257, (196,)), (513, (580, 4, 188)), (700, (1000, 392)),
-                  (2600, (3076,))):
+    steps = least + more
+    k = 64 * steps
+    for m, ns in ((bm + 1, (bn + 4,)), (2 * bm + 1, (3 * bn + 4, 4, bn - 4)),
+                  (700, (1000, 2 * bn + 8)), (2600, (3076,))):
         x, ws, bs = _inputs(m, ns, k, steps)
         for biases in (bs, [None] * len(ns)):
             for y, want in zip(_C.tile_linear(x, ws, biases, 0, tile, 1),
                                _want(x, ws, biases, 0)):
                 _close(y, want)
-    for m, ns, k in ((257, (64 * steps,), 200), (700, (64 * (steps - 1), 64), 376),
+    if bn == 256:
+        for m, n in ((bm + 1, 132), (700, 1004), (2600, 2056)):
+            x, ws, bs = _inputs(m, (n, n), k, steps)
+            _close(_C.tile_linear(x, ws, bs, SWIGLU, tile, 1)[0],
+                   _want(x, ws, bs, SWIGLU)[0])
+    for m, ns, k in ((bm + 1, (64 * steps,), bn + 8),
+                     (700, (64 * (steps - 1), 64), 2 * bn - 8),
                      (2600, (64, 64 * steps, 128), 3080)):
         _, ws, _ = _inputs(1, ns, k, steps)
         dys = [_inputs(m, (), n, n)[0] for n in ns]
         want = sum(d.double() @ w.double() for d, w in zip(dys, ws))
         err = (_C.tile_linear_dx(dys, ws, tile, 1).double() - want).abs()
         assert (err <= _limit(want, sum(ns))).all()
+    for end, ns, k in ((-63, (bm,), bn), (-31, (bm - 8, 8, 2 * bm + 8), bn + 8),
+                       (-8, (1000,), 2 * bn - 8), (0, (3080, 264), 3080)):
+        m = 64 * steps + end
+        x, _, _ = _inputs(m, (), k, steps)
+        dys = [_inputs(m, (), n, n)[0] for n in ns]
+        for got, d in zip(_C.tile_linear_dw(x, dys, tile, 1), dys):
+            want = d.double().t() @ x.double()
+            assert ((got.double() - want).abs() <= _limit(want, m)).all()
 
 
 @pytest.mark.gpu
