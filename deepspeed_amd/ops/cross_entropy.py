@@ -46,10 +46,10 @@ class _HeadLoss(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight, labels, rows, ignore_index):
-        ctx.slot = linear.uses(weight)
         ctx.rows, ctx.ignore_index = rows, ignore_index
         total, count, kept = None, None, []
         for xs, ys in zip(x.split(rows), labels.split(rows)):
+            linear.uses(weight)     # a use each: W's place is not for their sum
             logits = linear._forward(xs, [weight], [None])[0]
             t, c, _, lse = get_ext().ce_loss(logits, ys, ignore_index)
             total = t if total is None else total + t
@@ -95,7 +95,7 @@ class _HeadLoss(torch.autograd.Function):
             if need_w and i:
                 linear.add_dw(dw, part[0], d)
             elif need_w:
-                dw = linear._dw(part[0], [d], True, [need_x and ctx.slot])[0]
+                dw = linear._dw(part[0], [d], True, [None])[0]
         return dx, dw, None, None, None
 
 
