@@ -12,6 +12,8 @@
 //            for the whole step: 3.4 us a layer at 32 requests, 7.5 us for a
 //            portion of 1024 tokens. As two strided copies a token it took 159
 //            us a layer (64 launches) and 5.2 ms (2051 launches).
+//            Of a few rows the products of q, k and v write them themselves
+//            (rows_linear.hip).
 //   rows     the split-KV attention described below; for steps of long runs
 //            block_kernel.
 //   merge    log-sum-exp merge of the splits, only where there is more than

@@ -231,7 +231,7 @@ def test_tiles_by_four_waves_gpu(tile, bm, bn, least, more):
                 _close(y, want)
     if bn == 256:
         for m, n in ((bm + 1, 132), (700, 1004), (2600, 2056)):
-            x, ws, bs = _inputs(m, (n, n), k, steps)
+            x, ws, bs = _inputs(m, (n, n), 64 * (23 + steps), steps)
             _close(_C.tile_linear(x, ws, bs, SWIGLU, tile, 1)[0],
                    _want(x, ws, bs, SWIGLU)[0])
     for m, ns, k in ((bm + 1, (64 * steps,), bn + 8),
