@@ -100,7 +100,17 @@ class _HeadLoss(torch.autograd.Function):
 
 
 def head_loss(x, weight, labels, rows, ignore_index=-100):
-    return _HeadLoss.apply(x, weight, labels, rows, ignore_index)
+    """(sum of the rows' losses, labels that count). The weight is looked at here,
+    behind the hooks that may have filled it in: one of another form or number of
+    inputs is torch's, which takes or refuses it, a chunk at a time."""
+    if linear._differentiable(x, (weight,)):
+        return _HeadLoss.apply(x, weight, labels, rows, ignore_index)
+    total = count = 0
+    for xs, ys in zip(x.split(rows), labels.split(rows)):
+        t, c = fused_cross_entropy_sum(torch.nn.functional.linear(xs, weight),
+                                       ys, ignore_index)
+        total, count = total + t, count + c
+    return total, count
 
 
 def head_loss_fits(head, x) -> bool:

@@ -561,6 +561,8 @@ struct Layers {
     const int i = count++;
     TORCH_CHECK(weight.is_cuda() && weight.is_contiguous() &&
                 weight.scalar_type() == type && weight.numel() % K == 0 &&
+                (type == at::kChar ||
+                 (weight.dim() == 2 && weight.size(1) == K)) &&
                 weight.numel() > 0 && weight.numel() / K < (1 << 30) &&
                 ((uintptr_t)weight.data_ptr() & 15) == 0, what, ": weight");
     n[i] = weight.numel() / K;

@@ -77,3 +77,35 @@ def test_same_as_chunk_by_chunk_gpu(monkeypatch):
     assert not cross_entropy.head_loss_fits(other, flat)
     with torch.no_grad():
         assert not cross_entropy.head_loss_fits(head, flat)
+
+
+@pytest.mark.gpu
+def test_weights_of_other_forms_gpu():
+    """A weight of another number of inputs is refused, by several chunks as by one
+    and by the kernels themselves; one that is not contiguous is taken."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(1, 600, 256, device="cuda", generator=g).bfloat16()
+    labels = torch.randint(0, 640, (600,), device="cuda", generator=g)
+    head = linear.Linear(512, 640, bias=False).to("cuda", torch.bfloat16)
+    for rows in (256, 600):
+        with pytest.raises(RuntimeError):
+            chunked_cross_entropy(x, head, labels, rows)
+    for w in (head.weight, head.weight.view(-1)):
+        for op in (cross_entropy.get_ext().tile_linear,
+                   lambda x, w, b, m: cross_entropy.get_ext().rows_linear(
+                       x[:8], w, [], b, 0, m)):
+            with pytest.raises(RuntimeError, match="weight"):
+                op(x[0], [w.detach()], [None], 0)
+    head = linear.Linear(256, 640, bias=False).to("cuda", torch.bfloat16)
+    out = []
+    for w in (head.weight.detach(), head.weight.detach().t().contiguous().t()):
+        head.weight = torch.nn.Parameter(w)
+        leaf = x.clone().requires_grad_()
+        loss = chunked_cross_entropy(leaf, head, labels, 256)
+        loss.backward()
+        out.append((loss.detach(), leaf.grad, head.weight.grad))
+    assert not w.is_contiguous()
+    # sums in another order round some bf16 logits and gradients the other way
+    assert abs(out[0][0] - out[1][0]) <= 1e-4 * out[0][0]
+    for a, b in zip(out[0][1:], out[1][1:]):
+        assert (a.float() - b.float()).norm() <= 2 ** -7 * a.float().norm()
