@@ -14,6 +14,20 @@ from . import linear
 from ._loader import get_ext
 
 
+def _dlogits(logits, labels, lse, g, ignore_index, count=None):
+    """Gradient of the logits of a sum of losses, or with ``count`` of their mean;
+    by torch's own operations where it is differentiated itself."""
+    if not torch.is_grad_enabled():
+        return get_ext().ce_bwd(logits, labels, lse, g.contiguous().float(),
+                                ignore_index, count)
+    live = (labels != ignore_index)[:, None]
+    p = torch.softmax(logits.float(), -1)
+    d = p.scatter_add(1, torch.where(live, labels[:, None], 0),
+                      p.new_full((len(p), 1), -1.0))
+    g = g.float() if count is None else g.float() / count.clamp(min=1)
+    return torch.where(live, d * g, 0).to(logits.dtype)
+
+
 class _FusedCE(torch.autograd.Function):
     """(sum of the rows' losses, labels that count), or with ``mean`` their
     quotient; what torch makes of it takes ten launches more."""
@@ -32,8 +46,7 @@ class _FusedCE(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g, _gcount=None):
         logits, labels, lse, count = ctx.saved_tensors
-        d = get_ext().ce_bwd(logits, labels, lse, g.contiguous().float(),
-                             ctx.ignore_index, count)
+        d = _dlogits(logits, labels, lse, g, ctx.ignore_index, count)
         return d, None, None, None
 
 
@@ -42,34 +55,40 @@ class _HeadLoss(torch.autograd.Function):
     of rows. As one node: the chunks' gradients of W are added up by the products,
     those of x are made in their places and W is transposed once, where slices and
     calls of a head each clear, fill and add up gradients of all rows and of W
-    (32768 rows of 4096, 128256 features in four chunks: 3.4 of 162 ms)."""
+    (32768 rows of 4096, 128256 features in four chunks: 3.4 of 162 ms). The logits
+    are outputs too: where the gradients are differentiated themselves, what they
+    owe to the logits comes back here."""
 
     @staticmethod
     def forward(ctx, x, weight, labels, rows, ignore_index):
         ctx.rows, ctx.ignore_index = rows, ignore_index
-        total, count, kept = None, None, []
+        ctx.set_materialize_grads(False)
+        total, count, lses, outputs = None, None, [], []
         for xs, ys in zip(x.split(rows), labels.split(rows)):
             linear.uses(weight)     # a use each: W's place is not for their sum
             logits = linear._forward(xs, [weight], [None])[0]
             t, c, _, lse = get_ext().ce_loss(logits, ys, ignore_index)
             total = t if total is None else total + t
             count = c if count is None else count + c
-            kept += logits, lse
-        ctx.save_for_backward(x, weight, labels, *kept)
+            lses.append(lse)
+            outputs.append(logits)
+        ctx.save_for_backward(x, weight, labels, *lses, *outputs)
         ctx.mark_non_differentiable(count)
-        return total, count
+        return (total, count, *outputs)
 
     @staticmethod
-    def backward(ctx, g, _gcount):
+    def backward(ctx, g, _gcount, *more):
         x, w, labels, *kept = ctx.saved_tensors
         rows, (need_x, need_w) = ctx.rows, ctx.needs_input_grad[:2]
-        g = g.contiguous().float()
-        parts = list(zip(x.split(rows), labels.split(rows), kept[::2],
-                         kept[1::2]))
+        parts = list(zip(x.split(rows), labels.split(rows), kept[:len(more)],
+                         kept[len(more):], more))
 
         def gradient(part):
-            return get_ext().ce_bwd(part[2], part[1], part[3], g,
-                                    ctx.ignore_index, None)
+            _, ys, lse, logits, d = part
+            if g is None:
+                return torch.zeros_like(logits) if d is None else d
+            own = _dlogits(logits, ys, lse, g, ctx.ignore_index)
+            return own if d is None else own + d
         if torch.is_grad_enabled():     # differentiated themselves
             ds = [gradient(p) for p in parts]
             dx = torch.cat([d @ w for d in ds]) if need_x else None
@@ -79,7 +98,7 @@ class _HeadLoss(torch.autograd.Function):
         dx = torch.empty_like(x) if need_x else None
         dw = turned = None
         for i, part in enumerate(parts):
-            d = gradient(part)
+            d = gradient(part).contiguous()
             n = d.shape[0]
             if need_x:
                 to = dx[i * rows:i * rows + n]
@@ -104,7 +123,7 @@ def head_loss(x, weight, labels, rows, ignore_index=-100):
     behind the hooks that may have filled it in: one of another form or number of
     inputs is torch's, which takes or refuses it, a chunk at a time."""
     if linear._differentiable(x, (weight,)):
-        return _HeadLoss.apply(x, weight, labels, rows, ignore_index)
+        return _HeadLoss.apply(x, weight, labels, rows, ignore_index)[:2]
     total = count = 0
     for xs, ys in zip(x.split(rows), labels.split(rows)):
         t, c = fused_cross_entropy_sum(torch.nn.functional.linear(xs, weight),

@@ -109,3 +109,36 @@ def test_weights_of_other_forms_gpu():
     assert abs(out[0][0] - out[1][0]) <= 1e-4 * out[0][0]
     for a, b in zip(out[0][1:], out[1][1:]):
         assert (a.float() - b.float()).norm() <= 2 ** -7 * a.float().norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [128, 300])
+@pytest.mark.parametrize("frozen", [None, "x", "w"])
+def test_second_derivatives_gpu(rows, frozen):
+    """Products of the Hessian and a vector, by several chunks and by one."""
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.randn(1, 300, 256, device="cuda", generator=g).bfloat16()
+    head = linear.Linear(256, 640, bias=False).to("cuda", torch.bfloat16)
+    head.weight.data.normal_(0.0, 0.05, generator=g)
+    labels = torch.randint(0, 640, (300,), device="cuda", generator=g)
+    labels[::7] = -100
+    x.requires_grad_(frozen != "x")
+    head.weight.requires_grad_(frozen != "w")
+    leaves = [t for t in (x, head.weight) if t.requires_grad]
+    ways = [torch.randn(t.shape, device="cuda", generator=g).bfloat16()
+            for t in leaves]
+
+    def products(loss, leaves, ways):
+        first = torch.autograd.grad(loss, leaves, create_graph=True)
+        return torch.autograd.grad(
+            sum((f.float() * v.float()).sum() for f, v in zip(first, ways)),
+            leaves)
+    got = products(chunked_cross_entropy(x, head, labels, rows), leaves, ways)
+    xr, wr = (t.detach().float().requires_grad_(t.requires_grad)
+              for t in (x, head.weight))
+    want = products(torch.nn.functional.cross_entropy(xr[0] @ wr.t(), labels),
+                    [t for t in (xr, wr) if t.requires_grad], ways)
+    # logits, two gradients of theirs, a product each: four roundings of 2^-9,
+    # of which the chunks' sums take another
+    for a, b in zip(got, want):
+        assert (a.float() - b).norm() <= 2 ** -6 * b.norm()
