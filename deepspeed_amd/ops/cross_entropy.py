@@ -89,7 +89,9 @@ class _HeadLoss(torch.autograd.Function):
                 return torch.zeros_like(logits) if d is None else d
             own = _dlogits(logits, ys, lse, g, ctx.ignore_index)
             return own if d is None else own + d
-        if torch.is_grad_enabled():     # differentiated themselves
+        # differentiable products where the gradient itself is differentiated,
+        # torch's own where something watches them
+        if torch.is_grad_enabled() or not linear.untransformed():
             ds = [gradient(p) for p in parts]
             dx = torch.cat([d @ w for d in ds]) if need_x else None
             dw = sum(d.t() @ p[0] for d, p in zip(ds, parts)) \

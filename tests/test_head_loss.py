@@ -2,6 +2,7 @@
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from deepspeed_amd.models.llama import chunked_cross_entropy
 from deepspeed_amd.ops import cross_entropy, linear
@@ -142,3 +143,29 @@ def test_second_derivatives_gpu(rows, frozen):
     # of which the chunks' sums take another
     for a, b in zip(got, want):
         assert (a.float() - b).norm() <= 2 ** -6 * b.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [128, 300])
+def test_watched_backward_gpu(rows):
+    """A mode about the backward alone sees the products."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(1, 300, 256, device="cuda", generator=g).bfloat16()
+    x.requires_grad_()
+    head = linear.Linear(256, 640, bias=False).to("cuda", torch.bfloat16)
+    labels = torch.randint(0, 640, (300,), device="cuda", generator=g)
+    loss = chunked_cross_entropy(x, head, labels, rows)
+    leaves = [x, head.weight]
+    want = torch.autograd.grad(loss, leaves, retain_graph=True)
+    seen = []
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.overloadpacket)
+            return func(*args, **(kwargs or {}))
+    with Watch():
+        got = torch.autograd.grad(loss, leaves)
+    assert seen.count(torch.ops.aten.mm) == 2 * -(-300 // rows)
+    # gradients rounded in other places and added up in bf16
+    for a, w in zip(got, want):
+        assert (a.float() - w.float()).norm() <= 2 ** -7 * w.float().norm()
