@@ -91,7 +91,8 @@ class _HeadLoss(torch.autograd.Function):
             return own if d is None else own + d
         # differentiable products where the gradient itself is differentiated,
         # torch's own where something watches them
-        if torch.is_grad_enabled() or not linear.untransformed():
+        if torch.is_grad_enabled() or not linear.untransformed() or any(
+                d is not None and linear._batched(d) for d in more):
             ds = [gradient(p) for p in parts]
             dx = torch.cat([d @ w for d in ds]) if need_x else None
             dw = sum(d.t() @ p[0] for d, p in zip(ds, parts)) \

@@ -134,6 +134,10 @@ def test_second_derivatives_gpu(rows, frozen):
         return torch.autograd.grad(
             sum((f.float() * v.float()).sum() for f, v in zip(first, ways)),
             leaves)
+    first = torch.autograd.grad(chunked_cross_entropy(x, head, labels, rows),
+                                leaves, create_graph=True)
+    both = torch.autograd.grad(first, leaves, [torch.stack([v, -v]) for v in ways],
+                               is_grads_batched=True)
     got = products(chunked_cross_entropy(x, head, labels, rows), leaves, ways)
     xr, wr = (t.detach().float().requires_grad_(t.requires_grad)
               for t in (x, head.weight))
@@ -141,8 +145,9 @@ def test_second_derivatives_gpu(rows, frozen):
                     [t for t in (xr, wr) if t.requires_grad], ways)
     # logits, two gradients of theirs, a product each: four roundings of 2^-9,
     # of which the chunks' sums take another
-    for a, b in zip(got, want):
-        assert (a.float() - b).norm() <= 2 ** -6 * b.norm()
+    for a, b, t in zip(got, want, both):
+        for a in (a, t[0], -t[1]):
+            assert (a.float() - b).norm() <= 2 ** -6 * b.norm()
 
 
 @pytest.mark.gpu
