@@ -14,6 +14,9 @@ from . import linear
 from ._loader import get_ext
 
 
+_saved_hooks = torch._C._autograd._top_saved_tensors_default_hooks
+
+
 def _dlogits(logits, labels, lse, g, ignore_index, count=None):
     """Gradient of the logits of a sum of losses, or with ``count`` of their mean;
     by torch's own operations where it is differentiated itself."""
@@ -57,7 +60,9 @@ class _HeadLoss(torch.autograd.Function):
     calls of a head each clear, fill and add up gradients of all rows and of W
     (32768 rows of 4096, 128256 features in four chunks: 3.4 of 162 ms). The logits
     are outputs too: where the gradients are differentiated themselves, what they
-    owe to the logits comes back here."""
+    owe to the logits comes back here. Kept is what a chunk's calls would keep, and
+    let go as early: a frozen head holds no input, and each chunk's logits go when
+    their gradient, one chunk's at a time, is made."""
 
     @staticmethod
     def forward(ctx, x, weight, labels, rows, ignore_index):
@@ -72,7 +77,9 @@ class _HeadLoss(torch.autograd.Function):
             count = c if count is None else count + c
             lses.append(lse)
             outputs.append(logits)
-        ctx.save_for_backward(x, weight, labels, *lses, *outputs)
+        need_x, need_w = ctx.needs_input_grad[:2]
+        ctx.save_for_backward(x if need_w else None, weight if need_x else None,
+                              labels, *lses, *outputs)
         ctx.mark_non_differentiable(count)
         return (total, count, *outputs)
 
@@ -80,57 +87,71 @@ class _HeadLoss(torch.autograd.Function):
     def backward(ctx, g, _gcount, *more):
         x, w, labels, *kept = ctx.saved_tensors
         rows, (need_x, need_w) = ctx.rows, ctx.needs_input_grad[:2]
-        parts = list(zip(x.split(rows), labels.split(rows), kept[:len(more)],
-                         kept[len(more):], more))
+        n = len(more)
+        lses, outputs = kept[:n], kept[n:]
+        del kept
+        ys = labels.split(rows)
+        xs = x.split(rows) if need_w else [None] * n
 
-        def gradient(part):
-            _, ys, lse, logits, d = part
+        def gradient(i):
+            logits, outputs[i], d = outputs[i], None, more[i]
             if g is None:
                 return torch.zeros_like(logits) if d is None else d
-            own = _dlogits(logits, ys, lse, g, ctx.ignore_index)
+            own = _dlogits(logits, ys[i], lses[i], g, ctx.ignore_index)
             return own if d is None else own + d
         # differentiable products where the gradient itself is differentiated,
         # torch's own where something watches them
         if torch.is_grad_enabled() or not linear.untransformed() or any(
                 d is not None and linear._batched(d) for d in more):
-            ds = [gradient(p) for p in parts]
+            ds = [gradient(i) for i in range(n)]
             dx = torch.cat([d @ w for d in ds]) if need_x else None
-            dw = sum(d.t() @ p[0] for d, p in zip(ds, parts)) \
-                if need_w else None
+            dw = sum(d.t() @ p for d, p in zip(ds, xs)) if need_w else None
             return dx, dw, None, None, None
-        dx = torch.empty_like(x) if need_x else None
-        dw = turned = None
-        for i, part in enumerate(parts):
-            d = gradient(part).contiguous()
-            n = d.shape[0]
+        ctx.maybe_clear_saved_tensors()     # unless the graph is to stay
+        dx = dw = turned = d = None
+        for i in range(n):
+            d = None
+            d = gradient(i).contiguous()
+            T = len(d)
             if need_x:
-                to = dx[i * rows:i * rows + n]
-                if linear.own_dx(n, w.shape[:1], w.shape[1]) and \
+                # all rows' from the second chunk on, when the first's logits are gone
+                to = None if dx is None else dx[i * rows:i * rows + T]
+                if linear.own_dx(T, w.shape[:1], w.shape[1]) and \
                         linear._aligned(d, w):
-                    to.copy_(linear._dx([d], [w], True))
-                elif linear.backward_plan(n, *w.shape)[0]:
+                    part = linear._dx([d], [w], True)
+                elif linear.backward_plan(T, *w.shape)[0]:
                     if turned is None:
                         turned = linear._transposed(w)
-                    torch.mm(d, turned.t(), out=to)
+                    part = torch.mm(d, turned.t(), out=to)
                 else:
-                    torch.mm(d, w, out=to)
+                    part = torch.mm(d, w, out=to)
+                if dx is None:
+                    dx = w.new_empty(len(labels), w.shape[1])
+                if part is not to:
+                    dx[i * rows:i * rows + T] = part
+                del part
             if need_w and i:
-                linear.add_dw(dw, part[0], d)
+                linear.add_dw(dw, xs[i], d)
             elif need_w:
-                dw = linear._dw(part[0], [d], True, [None])[0]
+                dw = linear._dw(xs[i], [d], True, [None])[0]
         return dx, dw, None, None, None
 
 
-def head_loss(x, weight, labels, rows, ignore_index=-100):
-    """(sum of the rows' losses, labels that count). The weight is looked at here,
-    behind the hooks that may have filled it in: one of another form or number of
-    inputs is torch's, which takes or refuses it, a chunk at a time."""
-    if linear._differentiable(x, (weight,)):
-        return _HeadLoss.apply(x, weight, labels, rows, ignore_index)[:2]
+def head_loss(head, x, labels, rows, ignore_index=-100):
+    """(sum of the rows' losses, labels that count) of ``head``, a ``linear.Linear``
+    that is being called. Its weight is looked at here, behind the hooks that may
+    have filled it in. What the node is not for goes a chunk at a time: weights of
+    another form or number of inputs, which torch's product takes or refuses,
+    nothing to differentiate, and hooks on what is saved, which then get a chunk's
+    logits back when these are needed."""
+    w = head.weight
+    if linear._differentiable(x, (w,)) and head.bias is None and \
+            (x.requires_grad or w.requires_grad) and _saved_hooks(False) is None:
+        return _HeadLoss.apply(x, w, labels, rows, ignore_index)[:2]
     total = count = 0
     for xs, ys in zip(x.split(rows), labels.split(rows)):
-        t, c = fused_cross_entropy_sum(torch.nn.functional.linear(xs, weight),
-                                       ys, ignore_index)
+        t, c = fused_cross_entropy_sum(linear.Linear.forward(head, xs, True), ys,
+                                       ignore_index)
         total, count = total + t, count + c
     return total, count
 

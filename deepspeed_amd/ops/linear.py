@@ -452,10 +452,10 @@ class Linear(nn.Linear):
     outputs."""
 
     def forward(self, x, own: bool = False, loss=None):
-        w = self.weight
         if loss is not None:
             from .cross_entropy import head_loss
-            return head_loss(x, w, *loss)
+            return head_loss(self, x, *loss)
+        w = self.weight
         if _differentiable(x, (w,)):
             T = x.numel() // w.shape[1]
             if any(own_products(T, *w.shape)) or \

@@ -174,3 +174,47 @@ def test_watched_backward_gpu(rows):
     # gradients rounded in other places and added up in bf16
     for a, w in zip(got, want):
         assert (a.float() - w.float()).norm() <= 2 ** -7 * w.float().norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("frozen", [None, "x", "w", "both"])
+def test_memory_gpu(monkeypatch, frozen):
+    """No more of it than by calls of the head, at the most and between forward and
+    backward; hooks on what is saved are given no more at a time."""
+    n, h, v, rows = 4096, 1024, 16000, 1024
+    x = torch.randn(1, n, h, device="cuda").bfloat16()
+    head = linear.Linear(h, v, bias=False).to("cuda", torch.bfloat16)
+    labels = torch.randint(0, v, (n,), device="cuda")
+    x.requires_grad_(frozen not in ("x", "both"))
+    head.weight.requires_grad_(frozen not in ("w", "both"))
+
+    def step():
+        # hidden states whose owner lets them go, as a norm's output
+        y = x * 1
+        return chunked_cross_entropy(y, head, labels, rows)
+
+    def memory(offloaded):
+        x.grad = head.weight.grad = None
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        if offloaded:
+            with torch.autograd.graph.save_on_cpu():
+                loss = step()
+        else:
+            loss = step()
+        most = [torch.cuda.max_memory_allocated() - before]
+        held = torch.cuda.memory_allocated() - before
+        torch.cuda.reset_peak_memory_stats()
+        if loss.requires_grad:
+            loss.backward()
+        most.append(torch.cuda.max_memory_allocated() - before)
+        return (held, *most)
+    got = []
+    for fits in (cross_entropy.head_loss_fits, lambda *a: False):
+        monkeypatch.setattr(cross_entropy, "head_loss_fits", fits)
+        memory(False)       # the library's workspace
+        got.append([memory(False), memory(True)])
+    # gradients of x are made in their places, those of calls piece by piece
+    for a, b in zip(sum(got[0], ()), sum(got[1], ())):
+        assert a <= b + 2 * h * rows + (1 << 16), got
