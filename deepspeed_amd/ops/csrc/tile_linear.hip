@@ -1260,18 +1260,33 @@ constexpr int WIDE = 9;
 // 3072 in three splits of 256 x 256 508, in this 549).
 constexpr int SQUARE = 10;
 #define BETWEEN(X) X(SQUARE, 192, 192, 4, 2, 3, 0.804f, 6.3f)
-// Gates of up to 24 stages, as much first loads and stores, stay as below.
-bool by_four(int tile, int M, int K, int splits, int mode) {
-  if (splits > 1 || (mode == SWIGLU && K <= 24 * BK)) return false;
-  if (tile == LOW) return mode == GRAD_W || M > 192;
-  if (tile != NARROW && tile != SQUARE) return false;
-  return mode == GRAD_W || (mode != SWIGLU && M > (tile == NARROW ? 256 : 192));
+// Short contractions, as much first loads and stores, which eight waves make beside each
+// other's products, stay as below. Of the time by eight waves, over 1200 weights and rows
+// (192 x 256, 256 x 192, 192 x 192): the input's gradient 1.04, 1.07 and 0.99 at 4 stages,
+// 0.98, 1.02 and 0.94 at 8, 0.95, 0.99 and 0.90 at 12 (4000 rows 256 features, K 14336 in
+// 256 x 192 45 by eight / 56 us, 512, K 11008 57 / 62, 1024, K 3072 26.1 / 24.4); the
+// weights' of more than 12288 columns that are no power of two up to 1.07 and 1.13 at 4,
+// 0.99 and 1.06 at 8 and 0.89 at 4 for 192 x 192 (4608 x 18432, 256 rows in 256 x 192 74 /
+// 82), of others 0.89, 0.93 and 0.84 at 4 already (3072 x 8192, 300 rows 29.3 / 23.8).
+bool by_four(int tile, int M, int K, int steps, int splits, int mode) {
+  if (tile != LOW && tile != NARROW && tile != SQUARE) return false;
+  if (tile != LOW && mode == SWIGLU) return false;
+  if (mode != GRAD_W && M <= (tile == NARROW ? 256 : 192)) return false;
+  const bool across = K > 12288 && (K & (K - 1));
+  const int few = mode == SWIGLU ? 24 : mode == GRAD_X ? (tile == SQUARE ? 4 : 8)
+      : mode == GRAD_W && across ? (tile == LOW ? 5 : tile == NARROW ? 8 : 0) : 0;
+  return splits == 1 && steps > few;
 }
-// Of the time by eight waves, which the table's terms are fitted to: by mode.
-float four_takes(int tile, int mode) {
+// Of the time by eight waves, which the table's terms are fitted to: by mode. Less is
+// gained over few stages.
+float four_takes(int tile, int steps, int mode) {
   static const float of[3][4] = {
       {0.91f, 0.94f, 0.88f, 0.92f}, {0.95f, 1, 0.91f, 0.94f}, {0.935f, 1, 0.84f, 0.90f}};
-  return of[tile == LOW ? 0 : tile == NARROW ? 1 : 2][mode];
+  static const float most[3] = {0.853f, 0.905f, 0.815f};    // of the input's gradient
+  const int i = tile == LOW ? 0 : tile == NARROW ? 1 : 2;
+  if (mode == GRAD_X) return fmaxf(of[i][mode], most[i] + 1.f / steps);
+  if (mode == GRAD_W && steps <= 8 && tile != SQUARE) return 0.96f;
+  return of[i][mode];
 }
 // The largest tile by eight waves, two a SIMD: a short contraction is as much its first
 // loads and its stores, which the waves make beside each other's products. In place of
@@ -1381,14 +1396,17 @@ extern "C" int ds_tile_linear_plan(const int* n, int layers, int M, int K,
       if (i == SQUARE && mode == GRAD_X) us *= 1.04f;
       const bool least_by_eight = old.tile < 0 || us < old.eight;
       if (least_by_eight) old = {i, s, us, us};
-      if (by_four(i, M, K, s, mode)) us *= four_takes(i, mode);
+      if (by_four(i, M, K, steps, s, mode)) us *= four_takes(i, steps, mode);
       if (least_by_eight) old.us = us;
       if (best.tile < 0 || us < best.us) best = {i, s, us, us};
     }
   }
   // The terms are off by a tenth: another tile for a lead only (3369 rows 32000, K 1024
-  // 256 x 256 185, 192 x 256, which these terms have ahead by a little, 190).
-  if (best.us > 0.96f * old.us) best = old;
+  // 256 x 256 185, 192 x 256, which these terms have ahead by a little, 190). Short
+  // gradients of the largest tile are EIGHT's.
+  const bool eight = old.tile == WIDE && mode >= GRAD_X &&
+      short_contraction(mode, steps / old.splits, K);
+  if (best.us > (eight ? 0.9f : 0.96f) * old.us) best = old;
   *splits = best.splits;
   if (best.tile == WIDE && short_contraction(mode, steps / *splits, K)) return EIGHT;
   return best.tile;
@@ -1432,7 +1450,9 @@ extern "C" int ds_tile_linear(const void* const* x, int layers,
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (tile == WIDE && past_wide(mode, mode >= GRAD_X ? K : total, most))
     return (int)hipErrorInvalidValue;
-  if (by_four(tile, M, K, splits, mode) &&
+  const int steps = mode == GRAD_X ? total / BK
+      : mode == GRAD_W ? (M + BK - 1) / BK : K / BK;
+  if (by_four(tile, M, K, steps, splits, mode) &&
       !past_wide(mode, mode >= GRAD_X ? K : total, most)) {
 #define FOUR(BM, BN)                                                    \
   mode == GRAD_X ? launch_four<BM, BN, GRAD_X>(a, st)                   \

@@ -252,6 +252,48 @@ def test_tiles_by_four_waves_gpu(tile, bm, bn, least, more):
             assert ((got.double() - want).abs() <= _limit(want, m)).all()
 
 
+def test_short_gradients():
+    """Those of few stages are the largest tile's by eight waves, where what was
+    measured of the tiles by four has them behind."""
+    ext = get_ext()
+    if ext is None:
+        pytest.skip("the plan is the extension's")
+    plan, eight = ext.tile_linear_plan, len(TILES) + 1
+    for m, n, k in ((4000, 512, 11008), (4000, 768, 14336), (6000, 512, 28672)):
+        assert plan([n], m, k, 2)[0] == eight
+    assert plan([1024], 4000, 3072, 2)[0] in (6, 8)
+    for n, k in ((32064, 3072), (3072, 18944)):
+        assert plan([n], 512, k, 3)[0] == eight
+    assert plan([128256], 256, 4096, 3)[0] == WIDE
+    for m in (200, 512):
+        assert plan([3072], m, 8192, 3) == (6, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,bm,bn,x,w", [
+    (6, 192, 256, 8, 5), (8, 256, 192, 8, 8), (10, 192, 192, 4, 3)])
+@torch.no_grad()
+def test_short_gradients_gpu(tile, bm, bn, x, w):
+    """Stages around those up to which eight waves take a tile, and one more for
+    each state of the four waves' rings."""
+    from deepspeed_amd.ops import _C
+    for steps in (x, *range(x + 1, x + 7)):
+        for m, n, k in ((bm + 1, 64 * steps, bn + 8), (700, 64 * steps, 2 * bn)):
+            _, ws, _ = _inputs(1, (n,), k, steps)
+            dys = [_inputs(m, (), n, n)[0]]
+            want = dys[0].double() @ ws[0].double()
+            err = (_C.tile_linear_dx(dys, ws, tile, 1).double() - want).abs()
+            assert (err <= _limit(want, n)).all()
+    for steps in (w, *range(w + 1, w + 4)):
+        for k in (12288, 12296, 16384):
+            m = 64 * steps - 3
+            i, _, _ = _inputs(m, (), k, steps)
+            d = _inputs(m, (), bm + 8, steps)[0]
+            want = d.double().t() @ i.double()
+            err = (_C.tile_linear_dw(i, [d], tile, 1)[0].double() - want).abs()
+            assert (err <= _limit(want, m)).all()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,ns,k,mode,tile", [
     (40, (20000,), 2048, 0, 0), (33, (9000, 9000), 4096, SWIGLU, 1),
