@@ -14,8 +14,8 @@
 // stream_rows_kernel, in which every load goes to LDS, 128 bytes of 8 rows an
 // instruction. Bound by the stream of W from memory, 6 to 7 TB/s where it is large,
 // by launch and first loads where it is small.
-//   * More rows of int8, rows_linear_kernel: W and x straight into registers, bound by
-// x out of L2. bf16 layers of more rows are tile_linear.hip's.
+//   * More rows of int8, and more than 2^22 inputs, rows_linear_kernel: W and x straight
+// into registers, bound by x out of L2. bf16 layers of more rows are tile_linear.hip's.
 //   * int8: a lane's 16 bytes are 16 inputs, split over two products; the order
 //     of the inputs inside a product is free, x is read in the same order. The
 //     bytes become bf16 exactly (8 bits), are summed in fp32 and multiplied by
@@ -708,9 +708,9 @@ bool in_heads(const Args& a, int layers) {
 
 // Tiles of features a wave of rows_linear_kernel. Every workgroup reads all of x, which
 // costs M rows out of L2 for 16 FT features of W; half the workgroups leave CUs idle
-// where the layer is small (int8, us, FT 1 / 2 / 4): M 32: N 4096 11 / 14 / 20, N 6144
-// 23 / 16.3 / 23, N 14336 40 / 29.7 / 24.0; M 64: N 4096 21.1 / 23.8 / 44, N 14336 74 /
-// 46 / 51; gate and up M 32 53.8 / 42.6, M 64 88 / 67.
+// where the layer is small (int8 of 64 rows, us, FT 1 / 2: N 4096 21.1 / 23.8, N 14336 74
+// / 46; gate and up 88 / 67, 32 rows 53.8 / 42.6). Up to 32 rows only what the streams
+// do not take comes here: gates of few inputs, and more than 2^22 of them.
 template <bool I8>
 int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
   int tiles = 0;
@@ -721,17 +721,12 @@ int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
     if (a.M <= 16) return launch_streams<I8, 16>(a, layers, mode, tiles, st);
     return launch_streams<I8, 32>(a, layers, mode, tiles, st);
   }
-  const bool big = tiles >= 384, huge = tiles >= 896;
   if (mode == SWIGLU) {
     if (a.M <= 32) return launch<I8, 2, SWIGLU, 2>(a, layers, st);
     return launch<true, 4, SWIGLU, 2>(a, layers, st);
   }
-  if (a.M <= 32) {
-    if (huge) return launch<I8, 2, PLAIN, 4>(a, layers, st);
-    if (big) return launch<I8, 2, PLAIN, 2>(a, layers, st);
-    return launch<I8, 2, PLAIN, 1>(a, layers, st);
-  }
-  if (big) return launch<true, 4, PLAIN, 2>(a, layers, st);
+  if (a.M <= 32) return launch<I8, 2, PLAIN, 1>(a, layers, st);
+  if (tiles >= 384) return launch<true, 4, PLAIN, 2>(a, layers, st);
   return launch<true, 4, PLAIN, 1>(a, layers, st);
 }
 

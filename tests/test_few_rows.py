@@ -101,3 +101,25 @@ def test_streams_gpu(int8, k, m):
             want = [torch.nn.functional.silu(want[0]) * want[1]]
         for y, w in zip(got, want):
             _close(y, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("m", [3, 20])
+@torch.no_grad()
+def test_past_the_streams_gpu(int8, m):
+    """More inputs than a lane's offsets are for: the kernel that takes its operands
+    straight to registers."""
+    k = (1 << 22) + 256
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, k, generator=g).bfloat16().cuda()
+    for ns, mode in (((20, 4), 0), ((17, 17), SWIGLU)):
+        both = [_layer(n, k, i == 0, int8, g) for i, n in enumerate(ns)]
+        got = rows_linear(x, [b[0] for b in both], mode)
+        want = [f(x) for _, f in both]
+        if mode == SWIGLU:
+            want = [torch.nn.functional.silu(want[0]) * want[1]]
+        for y, w in zip(got, want):
+            # fp32 sums of k / 8 terms a wave, two roundings with the gate
+            lim = 2.0 ** (-7 if mode else -8) * w.abs() + 2.0 ** -12 * w.abs().max()
+            assert ((y.double() - w).abs() <= lim).all()
