@@ -289,8 +289,10 @@ __device__ __forceinline__ void load_scales(const float* from, unsigned off, int
 }
 
 // Each wave has a ring of its own in LDS, of D slots of 128 bytes of W's rows and what
-// belongs to them of x and of int8's scales; it goes on from tile to tile, so that the
-// ring is full while a tile's sums are added up, and waits for nobody before that.
+// belongs to them of x and of int8's scales; it goes on from tile to tile, and waits for
+// nobody before a tile's sums are added up. The ring is full meanwhile; but loads come
+// back in their order, so threads that then fetch a bias or, with several tiles of q and
+// k a workgroup, angles wait for what is in it.
 //
 //   * Loads to LDS, not to registers: as operands of the products lanes next to each
 // other have different rows, and a load of 16 rows by 64 bytes takes the address unit

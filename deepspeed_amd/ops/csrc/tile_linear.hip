@@ -1151,7 +1151,10 @@ int merge_splits(const Args& a, hipStream_t st) {
 // 36.4, 64 rows 4096 in four 12.7 / 13.4), nor over several tiles of rows, which share W
 // (300 rows 128256 343 / 345, 2331 rows 3584, K 14336 245 / 251). Over 800 layers of 33 to
 // 256 rows 0.95 of the time, 1.01 at most, from 16 MB on; smaller ones, 0.98 out of
-// memory, may be found in the chip's cache as a whole model's (8 MB 1.08).
+// memory, may be found in the chip's cache of 256 MB as a whole model's (8 MB 1.08). So
+// may larger ones of a small model: layers of 1024 and a head of 32000 in turn, 40 to 250
+// rows, 1.01 of the time at 111 and 156 MB in all; but 0.98 at 246 MB, and layers of 2048,
+// 672 MB, 0.97. A line at 64 MB would have these at 1.00 all four.
 bool once(const Args& a) {
   return a.mtiles == 1 && a.splits == 1 &&
       (long long)a.n_end[a.layers - 1] * a.K >= 1 << 23;
