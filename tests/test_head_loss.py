@@ -218,3 +218,63 @@ def test_memory_gpu(monkeypatch, frozen):
     # gradients of x are made in their places, those of calls piece by piece
     for a, b in zip(sum(got[0], ()), sum(got[1], ())):
         assert a <= b + 2 * h * rows + (1 << 16), got
+
+
+def _moments(stage, gas):
+    """First moments of two steps of an engine over a model whose head's loss takes
+    several chunks, and the calls of ``head_loss``."""
+    import deepspeed_amd
+    from deepspeed_amd.models import llama
+    torch.manual_seed(0)
+    cfg = llama.LlamaConfig(vocab_size=512, hidden_size=256,
+                            intermediate_size=512, num_layers=2, num_heads=2,
+                            num_kv_heads=1, max_seq_len=4096)
+    model = llama.LlamaForCausalLM(cfg).cuda()
+    engine, opt, _, _ = deepspeed_amd.initialize(model=model, config={
+        "train_micro_batch_size_per_gpu": 3,
+        "gradient_accumulation_steps": gas, "bf16": {"enabled": True},
+        "zero_optimization": {"stage": stage},
+        "optimizer": {"type": "AdamW", "params": {"lr": 1e-3}}})
+    g = torch.Generator().manual_seed(1)
+    out, seen = [], []
+    own = cross_entropy.head_loss
+
+    def spy(head, x, labels, rows):
+        seen.append(tuple(head.weight.shape))   # filled in by then
+        return own(head, x, labels, rows)
+    cross_entropy.head_loss = spy
+    try:
+        for _ in range(2 * gas):
+            ids = torch.randint(0, 512, (3, 3000), generator=g).cuda()
+            loss = engine(ids, labels=ids)
+            engine.backward(loss)
+            engine.step()
+            out.append(loss.detach().view(1))
+    finally:
+        cross_entropy.head_loss = own
+    for part in opt.layout_manifest():
+        flat = opt.param_groups[part["group_idx"]]["params"][0]
+        first = opt.state[flat]["exp_avg"]
+        for _, at, n, _ in part["params"]:
+            at += part["master_offset"]
+            out.append(first[at:at + n].clone())
+    engine.destroy()
+    return out, seen
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stage,gas", [(2, 1), (2, 2), (3, 1), (3, 2)])
+def test_engine_with_several_chunks_gpu(stage, gas, monkeypatch):
+    """Losses and gradients as by calls of the head: its place in the flat buffer
+    closed, and with the hooks of partitioned weights about it."""
+    monkeypatch.setenv("MASTER_ADDR", "127.0.0.1")
+    monkeypatch.setenv("MASTER_PORT", "29549")
+    got, seen = _moments(stage, gas)
+    assert seen == [(512, 256)] * 2 * gas
+    monkeypatch.setattr(cross_entropy, "head_loss_fits", lambda *a: False)
+    want, seen = _moments(stage, gas)
+    assert not seen and len(got) == len(want)
+    # the second step's weights and losses follow from gradients rounded otherwise
+    assert torch.equal(got[0], want[0])
+    for a, b in zip(got[1:], want[1:]):
+        assert (a.float() - b.float()).norm() <= 2.0 ** -6 * b.float().norm()
