@@ -55,10 +55,11 @@ class _FusedCE(torch.autograd.Function):
 
 class _HeadLoss(torch.autograd.Function):
     """(sum of the rows' losses, labels that count) of the logits x W^T, in chunks
-    of rows. As one node: the chunks' gradients of W are added up by the products,
-    those of x are made in their places and W is transposed once, where slices and
-    calls of a head each clear, fill and add up gradients of all rows and of W
-    (32768 rows of 4096, 128256 features in four chunks: 3.4 of 162 ms). The logits
+    of rows. As one node: gradients of x are made in their places, W is transposed
+    once or twice and the library's products add the chunks' gradients of W up
+    (those of the kernels, ``own_dw``, are added in bf16), where slices and calls of
+    a head each clear, fill and add up gradients of all rows and of W (32768 rows of
+    4096, 128256 features in four chunks: 3.4 of 162 ms). The logits
     are outputs too: where the gradients are differentiated themselves, what they
     owe to the logits comes back here. Kept is what a chunk's calls would keep, and
     let go as early: a frozen head holds no input, and each chunk's logits go when
@@ -108,16 +109,13 @@ class _HeadLoss(torch.autograd.Function):
             dw = sum(d.t() @ p for d, p in zip(ds, xs)) if need_w else None
             return dx, dw, None, None, None
         ctx.maybe_clear_saved_tensors()     # unless the graph is to stay
-        dx = dw = turned = d = None
+        dx = dw = turned = None
         for i in range(n):
-            d = None
             d = gradient(i).contiguous()
-            T = len(d)
+            T, at = len(d), slice(i * rows, (i + 1) * rows)
             if need_x:
-                # all rows' from the second chunk on, when the first's logits are gone
-                to = None if dx is None else dx[i * rows:i * rows + T]
-                if linear.own_dx(T, w.shape[:1], w.shape[1]) and \
-                        linear._aligned(d, w):
+                to, K = None if dx is None else dx[at], w.shape[1]
+                if linear.own_dx(T, w.shape[:1], K) and linear._aligned(d, w):
                     part = linear._dx([d], [w], True)
                 elif linear.backward_plan(T, *w.shape)[0]:
                     if turned is None:
@@ -125,15 +123,20 @@ class _HeadLoss(torch.autograd.Function):
                     part = torch.mm(d, turned.t(), out=to)
                 else:
                     part = torch.mm(d, w, out=to)
-                if dx is None:
-                    dx = w.new_empty(len(labels), w.shape[1])
-                if part is not to:
-                    dx[i * rows:i * rows + T] = part
-                del part
+                # kept where the logits that are gone have left room for it
+                if 2 * w.numel() + len(labels) * K > (i + 1) * rows * len(w):
+                    turned = None
             if need_w and i:
                 linear.add_dw(dw, xs[i], d)
             elif need_w:
                 dw = linear._dw(xs[i], [d], True, [None])[0]
+            del d
+            if need_x:
+                if dx is None:      # not beside all of the logits
+                    dx = w.new_empty(len(labels), K)
+                if part is not to:
+                    dx[at] = part
+                del part
         return dx, dw, None, None, None
 
 

@@ -177,11 +177,12 @@ def test_watched_backward_gpu(rows):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,h,v,rows", [(4096, 1024, 16000, 1024),
+                                        (16384, 2048, 16064, 4096)])
 @pytest.mark.parametrize("frozen", [None, "x", "w", "both"])
-def test_memory_gpu(monkeypatch, frozen):
+def test_memory_gpu(monkeypatch, frozen, n, h, v, rows):
     """No more of it than by calls of the head, at the most and between forward and
     backward; hooks on what is saved are given no more at a time."""
-    n, h, v, rows = 4096, 1024, 16000, 1024
     x = torch.randn(1, n, h, device="cuda").bfloat16()
     head = linear.Linear(h, v, bias=False).to("cuda", torch.bfloat16)
     labels = torch.randint(0, v, (n,), device="cuda")
