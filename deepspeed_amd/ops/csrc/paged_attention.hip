@@ -28,9 +28,9 @@
 //   * Bound by the stream of K and V (decode): 16-byte loads, the next tile in
 //     flight while the softmax and the second product of this one run, three
 //     waves a SIMD. 48 us a layer at 32 requests of 2000 tokens and 8 key
-//     heads (5.4 TB/s), 91 us at 8 of 16000 (5.8 TB/s; a large copy reaches
-//     4.9, a read 6.4). One position a wave at a time (2-byte loads, a six-step shuffle
-//     chain each) took 240 and 459 us.
+//     heads (5.5 TB/s), 83 to 91 us at 8 of 16000 (5.8 to 6.3 TB/s; a large
+//     read reaches 6.3, past the caches 7.0). One position a wave at a time
+//     (2-byte loads, a six-step shuffle chain each) took 240 and 459 us.
 //   * S^T = K Q^T on mfma_f32_16x16x32_bf16: K rows go from global memory
 //     straight into A fragments (64 contiguous bytes a row and instruction).
 //     Lane (g = lane >> 4) then holds the scores of keys 16 t + 4 g + r of
