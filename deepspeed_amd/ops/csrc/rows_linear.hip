@@ -689,12 +689,31 @@ int launch_streams(const Args& a, int layers, int mode, int tiles,
 #undef STREAM
 }
 
+// Queries, keys and values, or what has their form.
+bool in_heads(const Args& a, int layers) {
+  return layers == 3 && a.n[0] % 128 == 0 && a.n[1] % 128 == 0 &&
+      a.n[2] % 128 == 0;
+}
+
+// Layers of less than a round of tiles whose contraction is a load or two a wave, to
+// rows_linear_kernel: straight to registers is a hop less, and less code to fetch. us of
+// the stream / so: bf16 K 256, N 2048 8 and 16 rows 3.16 / 2.89, 3.19 / 2.95, but 24 rows
+// of N 1024 2.96 / 3.28, and K 512, N 256 2.82 / 3.13; int8 K 256 2.75 to 3.40 / 2.83 to
+// 3.00, K 512, N 1024 1, 16 and 24 rows 3.39 / 3.04, 3.54 / 3.15, 3.77 / 3.71, but 32 rows
+// 3.77 / 3.89, a whole round of tiles at 16 3.67 / 3.88, and K 768, N 2048 3.59 / 3.77.
+template <bool I8>
+bool brief(const Args& a, int layers, int mode, int tiles) {
+  if (mode != PLAIN || tiles >= 256 || in_heads(a, layers)) return false;
+  return I8 ? a.K <= (a.M <= 24 ? 512 : 256) : a.M <= 16 && a.K <= 256;
+}
+
 // What stream_rows_kernel takes: a lane's offsets in a tile and int8's places of scales
 // are 32 bits, and x, which each workgroup reads at another place, stays in an XCD's
 // L2. Of 17 to 32 rows int8 but for short gates (2 x 5632, K 2048 32 rows 12.8, by
 // rows_linear_kernel 12.2), bf16 as ds_rows_linear is given them.
 template <bool I8>
 bool streams(const Args& a, int layers, int mode, int tiles) {
+  if (brief<I8>(a, layers, mode, tiles)) return false;
   if (a.M > 32 || a.K > 1 << 22) return false;
   if (I8)
     for (int i = 0; i < layers; ++i)
@@ -702,17 +721,11 @@ bool streams(const Args& a, int layers, int mode, int tiles) {
   return a.M <= 16 || !I8 || mode == PLAIN || tiles <= 512 || a.K > 2048;
 }
 
-// Queries, keys and values, or what has their form.
-bool in_heads(const Args& a, int layers) {
-  return layers == 3 && a.n[0] % 128 == 0 && a.n[1] % 128 == 0 &&
-      a.n[2] % 128 == 0;
-}
-
 // Tiles of features a wave of rows_linear_kernel. Every workgroup reads all of x, which
 // costs M rows out of L2 for 16 FT features of W; half the workgroups leave CUs idle
 // where the layer is small (int8 of 64 rows, us, FT 1 / 2: N 4096 21.1 / 23.8, N 14336 74
 // / 46; gate and up 88 / 67, 32 rows 53.8 / 42.6). Up to 32 rows only what the streams
-// do not take comes here: gates of few inputs, and more than 2^22 of them.
+// do not take comes here: brief layers, gates of few inputs, more than 2^22 of them.
 template <bool I8>
 int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
   int tiles = 0;
@@ -727,6 +740,7 @@ int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
     if (a.M <= 32) return launch<I8, 2, SWIGLU, 2>(a, layers, st);
     return launch<true, 4, SWIGLU, 2>(a, layers, st);
   }
+  if (a.M <= 16) return launch<I8, 1, PLAIN, 1>(a, layers, st);
   if (a.M <= 32) return launch<I8, 2, PLAIN, 1>(a, layers, st);
   if (tiles >= 384) return launch<true, 4, PLAIN, 2>(a, layers, st);
   return launch<true, 4, PLAIN, 1>(a, layers, st);

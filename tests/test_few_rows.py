@@ -123,3 +123,19 @@ def test_past_the_streams_gpu(int8, m):
             # fp32 sums of k / 8 terms a wave, two roundings with the gate
             lim = 2.0 ** (-7 if mode else -8) * w.abs() + 2.0 ** -12 * w.abs().max()
             assert ((y.double() - w).abs() <= lim).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("k", [256, 512, 768])
+@pytest.mark.parametrize("m", [1, 16, 17, 24, 25, 32])
+@torch.no_grad()
+def test_brief_layers_gpu(int8, k, m):
+    """A tile less than a round and a whole one, either side of the rows and inputs up
+    to which they go straight to registers; several layers, and of heads."""
+    g = torch.Generator().manual_seed(k + m)
+    x = torch.randn(m, k, generator=g).bfloat16().cuda()
+    for ns in ((4068,), (4084,), (2000, 36, 4), (256, 128, 128)):
+        both = [_layer(n, k, i == 0, int8, g) for i, n in enumerate(ns)]
+        for y, (_, want) in zip(rows_linear(x, [b[0] for b in both]), both):
+            _close(y, want(x))
