@@ -59,6 +59,7 @@ struct Args {
   int n[MAXL], tile_end[MAXL];
   const short* x;
   int M, K, group;
+  bool heads;               // PLAIN: workgroups begin as QKV's with their tiles do
   Append to;
 };
 
@@ -327,10 +328,11 @@ struct Slot {
 //
 // QKV: half of the tiles lie 64 features behind the others, so that the threads that add
 // a pair up turn it and write it where attention reads it. What that asks for (positions,
-// rows of the pool, angles) is fetched before the weights are waited for. q, k and v that
-// are only wanted as they are have the same tiles, and the same sums. A launch and 3 us a
-// layer less: steps of four layers, one request of 500 532 -> 525 us, 8 of 16000 873 ->
-// 857, int8 8 of 1000, where the host is as long, 402 -> 381.
+// rows of the pool, angles) is fetched before the weights are waited for. A launch and 3
+// us a layer less: steps of four layers, one request of 500 532 -> 525 us, 8 of 16000 873
+// -> 857, int8 8 of 1000, where the host is as long, 402 -> 381. q, k and v that are only
+// wanted as they are have the same sums: by the same tiles or, where these leave half of
+// the CUs idle, by PLAIN's of 16 features, whose workgroups begin alike (`heads`).
 template <bool I8, int XR, int S, int NW, int D, int MODE>
 __global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
                                                               const int tiles) {
@@ -347,7 +349,9 @@ __global__ __launch_bounds__(NW * 64) void stream_rows_kernel(const Args a,
   const int n = (chunks - wid + NW - 1) / NW;       // wid, wid + NW, ..
   // Each workgroup begins elsewhere in its rows, over an XCD and over the XCDs: rows
   // that are multiples of 4 KB apart lie in few memory channels.
-  const int turn = uni((blockIdx.x / 8 * 13 + blockIdx.x % 8 * 7) % 32 * chunks / 32);
+  const unsigned begin = MODE == PLAIN && a.heads ? blockIdx.x / 8 * 4 + blockIdx.x % 4
+                                                  : blockIdx.x;
+  const int turn = uni((begin / 8 * 13 + begin % 8 * 7) % 32 * chunks / 32);
   auto chunk = [&](int i) __attribute__((always_inline)) {
     const int c = wid + i * NW + turn;
     return uni(c < chunks ? c : c - chunks);
@@ -727,11 +731,18 @@ bool streams(const Args& a, int layers, int mode, int tiles) {
 // / 46; gate and up 88 / 67, 32 rows 53.8 / 42.6). Up to 32 rows only what the streams
 // do not take comes here: brief layers, gates of few inputs, more than 2^22 of them.
 template <bool I8>
-int launch_rows(const Args& a, int layers, int mode, hipStream_t st) {
+int launch_rows(Args a, int layers, int mode, hipStream_t st) {
   int tiles = 0;
   for (int i = 0; i < layers; ++i) tiles += (a.n[i] + 15) / 16;
   if (streams<I8>(a, layers, mode, tiles)) {
-    if (mode == PLAIN && in_heads(a, layers)) mode = QKV;
+    // Up to 256 tiles a workgroup has one, by either. us by pairs of tiles, and one:
+    // bf16 1664 + 2 x 1024, K 5120, 2 rows 13.2 / 8.8, 3 x 896, K 3584, 12 rows 9.5 / 7.9,
+    // 768 + 2 x 128, K 256, 2 rows 3.6 / 3.2; int8 640 + 2 x 1408, K 8192, 2 rows 12.4 /
+    // 8.7, 128 + 2 x 640, K 6656, 32 rows 16.3 / 12.0; 0.83 over 35 layers.
+    if (mode == PLAIN && in_heads(a, layers)) {
+      if (a.to.dst || tiles > 256) mode = QKV;
+      else a.heads = true;
+    }
     if (a.M <= 8) return launch_streams<I8, 8>(a, layers, mode, tiles, st);
     if (a.M <= 16) return launch_streams<I8, 16>(a, layers, mode, tiles, st);
     return launch_streams<I8, 32>(a, layers, mode, tiles, st);

@@ -316,3 +316,13 @@ def test_sums_in_parts_gpu(kind, monkeypatch):
 
     monkeypatch.setattr(llama, "LlamaConfig", Wide)
     test_same_as_modules_gpu(kind, True, monkeypatch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv_heads", [(8, 4), (16, 8), (18, 6), (24, 6)])
+@pytest.mark.parametrize("rows", [1, 9, 32])
+@pytest.mark.parametrize("int8", [False, True])
+def test_append_up_to_a_round_gpu(heads, kv_heads, rows, int8, monkeypatch):
+    """Bit by bit also where the products alone have a tile of 16 features a
+    workgroup and those that append pairs of them: up to 256 tiles, and more."""
+    test_append_with_the_products_gpu(heads, kv_heads, rows, int8, monkeypatch)
