@@ -1002,7 +1002,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       // columns 4 g .. of two tiles to 8 of one: odd rows of lanes of the first
       // change places with even ones of the second
       const int n1 = at.n0 + wn * (BN / 2) + (g & 1) * 16 + (g >> 1) * 8;
-      auto store = [&](auto at) INLINE {
+      auto store = [&](auto by, auto at) INLINE {
         constexpr int f = decltype(at)::value / FX * 2, m = decltype(at)::value % FX;
         constexpr int A = acc(f, m), B = acc(f + 1, m);
         const unsigned y0 = packed2(sum<A>(), sum<A + 1>());
@@ -1014,9 +1014,17 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
         const int n = n1 + 16 * f;
         __builtin_amdgcn_raw_buffer_store_b128(
             u32x4{lo[0], hi[0], lo[1], hi[1]}, to,
-            n < N ? (unsigned)((16 * m + col) * N + n) * 2 : NOWHERE, 0, STREAM);
+            n < N ? (unsigned)((16 * m + col) * N + n) * 2 : NOWHERE, 0,
+            decltype(by)::value);
       };
-      each(std::make_integer_sequence<int, FW / 2 * FX>{}, store);
+      auto past = [&](auto at) INLINE { store(Int<STREAM>{}, at); };
+      auto through = [&](auto at) INLINE { store(Int<0>{}, at); };
+      // A store is 64 bytes of each of 16 rows. Where these are parts of two lines they
+      // have to meet in a cache (us, past the caches / through them: the input's gradient
+      // of 576 features, K 2968, 6126 rows 48.6 / 31.7, the weights' of 23936 x 2408, 244
+      // rows 108 / 57; over 220 of the largest tile 0.87).
+      if (N % 32 == 0) each(std::make_integer_sequence<int, FW / 2 * FX>{}, past);
+      else each(std::make_integer_sequence<int, FW / 2 * FX>{}, through);
     } else {
       constexpr int W = GLU ? FW / 2 : FW;    // features a lane
       const int n = at.n0 + wn * (GLU ? BN / 4 : BN / 2) + W * col;
@@ -1271,13 +1279,18 @@ constexpr int SQUARE = 10;
 // weights' of more than 12288 columns that are no power of two up to 1.07 and 1.13 at 4,
 // 0.99 and 1.06 at 8 and 0.89 at 4 for 192 x 192 (4608 x 18432, 256 rows in 256 x 192 74 /
 // 82), of others 0.89, 0.93 and 0.84 at 4 already (3072 x 8192, 300 rows 29.3 / 23.8).
+// Gradients of columns that are no whole 64 bytes, over 190: 256 x 192 1.03 up to 10
+// stages (3072 x 3832, 216 rows 14.3 / 16.2; the input's of 576 features, K 4880, 4492
+// rows 33.4 / 35.3), 0.97 from 12 on, the others 0.91 as all.
 bool by_four(int tile, int M, int K, int steps, int splits, int mode) {
   if (tile != LOW && tile != NARROW && tile != SQUARE) return false;
   if (tile != LOW && mode == SWIGLU) return false;
   if (mode != GRAD_W && M <= (tile == NARROW ? 256 : 192)) return false;
-  const bool across = K > 12288 && (K & (K - 1));
-  const int few = mode == SWIGLU ? 24 : mode == GRAD_X ? (tile == SQUARE ? 4 : 8)
-      : mode == GRAD_W && across ? (tile == LOW ? 5 : tile == NARROW ? 8 : 0) : 0;
+  const bool across = K > 12288 && (K & (K - 1)), ragged = K % 32 != 0;
+  int few = mode == SWIGLU ? 24 : 0;
+  if (mode == GRAD_X) few = tile == SQUARE ? 4 : 8;
+  if (mode == GRAD_W && across) few = tile == LOW ? 5 : tile == NARROW ? 8 : 0;
+  if (mode >= GRAD_X && ragged && tile == NARROW) few = 12;
   return splits == 1 && steps > few;
 }
 // Of the time by eight waves, which the table's terms are fitted to: by mode. Less is

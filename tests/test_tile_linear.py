@@ -684,3 +684,26 @@ def test_largest_layers_gpu(n):
                      lambda: _C.tile_linear_dw(x.detach(), [dy])):
             with pytest.raises(RuntimeError, match="operands"):
                 call()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,bm,bn", [(6, 192, 256), (8, 256, 192),
+                                        (10, 192, 192), (9, 256, 256)])
+@torch.no_grad()
+def test_rows_of_parts_of_lines_gpu(tile, bm, bn):
+    """Gradients whose rows are whole 64 bytes or not, to the last column, either
+    side of the stages up to which eight waves take these."""
+    from deepspeed_amd.ops import _C
+    for steps in (12, 13, 14):
+        for k in (bn + 8, bn + 32, 2 * bn - 8, 2 * bn):
+            n, m = 64 * steps, 64 * steps - 3
+            _, ws, _ = _inputs(1, (n,), k, steps)
+            dys = [_inputs(bm + 1, (), n, n)[0]]
+            want = dys[0].double() @ ws[0].double()
+            err = (_C.tile_linear_dx(dys, ws, tile, 1).double() - want).abs()
+            assert (err <= _limit(want, n)).all()
+            i, _, _ = _inputs(m, (), k, steps)
+            d = _inputs(m, (), bm + 8, steps)[0]
+            want = d.double().t() @ i.double()
+            err = (_C.tile_linear_dw(i, [d], tile, 1)[0].double() - want).abs()
+            assert (err <= _limit(want, m)).all()
