@@ -994,6 +994,16 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
   } else {
     // outputs pass the caches by, which hold what other tiles still read
     constexpr int STREAM = 2;
+    // Not where rows are no whole 64 bytes: a store of 64 (gradients) or 192 and 256 bytes
+    // of a row is then parts of lines, which have to meet in a cache (us, past the caches /
+    // through them: the input's gradient of 576 features, K 2968, 6126 rows 48.6 / 31.7,
+    // the weights' of 23936 x 2408, 244 rows 108 / 57; over 220 of the largest tile 0.87;
+    // forward 9416, K 192, 6622 rows 57.4 / 42.5, 11608, K 192, 8682 rows 88.0 / 76.0; over
+    // 100 of the largest tile 0.95). But forward outputs that no cache holds go past, and
+    // gates, 128 bytes of a row and longer in the making, are even (32336, K 640, 8271 rows
+    // 353 / 391).
+    const bool whole = N % 32 == 0 || GLU ||
+        (!WT && (long long)rows * N > 1ll << 27);
     short* out = a.out[MODE == GRAD_X || GLU ? 0 : at.layer];
     const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(out + (long long)m_of * N), (short)0,
@@ -1019,11 +1029,7 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
       };
       auto past = [&](auto at) INLINE { store(Int<STREAM>{}, at); };
       auto through = [&](auto at) INLINE { store(Int<0>{}, at); };
-      // A store is 64 bytes of each of 16 rows. Where these are parts of two lines they
-      // have to meet in a cache (us, past the caches / through them: the input's gradient
-      // of 576 features, K 2968, 6126 rows 48.6 / 31.7, the weights' of 23936 x 2408, 244
-      // rows 108 / 57; over 220 of the largest tile 0.87).
-      if (N % 32 == 0) each(std::make_integer_sequence<int, FW / 2 * FX>{}, past);
+      if (whole) each(std::make_integer_sequence<int, FW / 2 * FX>{}, past);
       else each(std::make_integer_sequence<int, FW / 2 * FX>{}, through);
     } else {
       constexpr int W = GLU ? FW / 2 : FW;    // features a lane
@@ -1043,8 +1049,9 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
               from, (n + e) * 2, 0, 0));
       }
       typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-      auto store = [&](auto bias, auto at) INLINE {
+      auto store = [&](auto bias, auto by, auto at) INLINE {
         constexpr bool B = decltype(bias)::value;
+        constexpr int S = decltype(by)::value;
         constexpr int m = decltype(at)::value / 4, r = decltype(at)::value % 4;
         const unsigned o =
             n < N ? (unsigned)((4 * g + 16 * m + r) * N + n) * 2 : NOWHERE;
@@ -1061,37 +1068,41 @@ __global__ __launch_bounds__(256, 1) void wide_linear_kernel(const Args a) {
         const u32x2 v = {packed2(one(Int<0>{}), one(Int<1>{})),
                          packed2(one(Int<2>{}), one(Int<3>{}))};
         if constexpr (GLU) {
-          __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, STREAM);
+          __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, S);
         } else if constexpr (FW == 6) {
           typedef unsigned u32x3 __attribute__((ext_vector_type(3)));
           const unsigned u = packed2(one(Int<4>{}), one(Int<5>{}));
           if (at_edge) {      // N is a multiple of four, six features may pass it
-            __builtin_amdgcn_raw_buffer_store_b32(v[0], to, o, 0, STREAM);
+            __builtin_amdgcn_raw_buffer_store_b32(v[0], to, o, 0, S);
             __builtin_amdgcn_raw_buffer_store_b32(
-                v[1], to, n + 2 < N ? o + 4 : NOWHERE, 0, STREAM);
+                v[1], to, n + 2 < N ? o + 4 : NOWHERE, 0, S);
             __builtin_amdgcn_raw_buffer_store_b32(
-                u, to, n + 4 < N ? o + 8 : NOWHERE, 0, STREAM);
+                u, to, n + 4 < N ? o + 8 : NOWHERE, 0, S);
           } else {
             __builtin_amdgcn_raw_buffer_store_b96(u32x3{v[0], v[1], u}, to, o, 0,
-                                                  STREAM);
+                                                  S);
           }
         } else {
           const u32x2 u = {packed2(one(Int<4>{}), one(Int<5>{})),
                            packed2(one(Int<6>{}), one(Int<7>{}))};
           if (N % 8 == 0) {
             __builtin_amdgcn_raw_buffer_store_b128(u32x4{v[0], v[1], u[0], u[1]},
-                                                   to, o, 0, STREAM);
+                                                   to, o, 0, S);
           } else {
-            __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, STREAM);
+            __builtin_amdgcn_raw_buffer_store_b64(v, to, o, 0, S);
             __builtin_amdgcn_raw_buffer_store_b64(
-                u, to, n + 4 < N ? o + 8 : NOWHERE, 0, STREAM);
+                u, to, n + 4 < N ? o + 8 : NOWHERE, 0, S);
           }
         }
       };
-      auto with = [&](auto at) INLINE { store(Int<1>{}, at); };
-      auto without = [&](auto at) INLINE { store(Int<0>{}, at); };
-      if (biased) each(std::make_integer_sequence<int, 4 * FX>{}, with);
-      else each(std::make_integer_sequence<int, 4 * FX>{}, without);
+      auto all = [&](auto bias, auto by) INLINE {
+        auto one = [&](auto at) INLINE { store(bias, by, at); };
+        each(std::make_integer_sequence<int, 4 * FX>{}, one);
+      };
+      if (biased && whole) all(Int<1>{}, Int<STREAM>{});
+      else if (biased) all(Int<1>{}, Int<0>{});
+      else if (whole) all(Int<0>{}, Int<STREAM>{});
+      else all(Int<0>{}, Int<0>{});
     }
   }
   wait_loads<0>();

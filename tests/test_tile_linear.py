@@ -707,3 +707,21 @@ def test_rows_of_parts_of_lines_gpu(tile, bm, bn):
             want = d.double().t() @ i.double()
             err = (_C.tile_linear_dw(i, [d], tile, 1)[0].double() - want).abs()
             assert (err <= _limit(want, m)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,bm,bn", [(6, 192, 256), (8, 256, 192),
+                                        (10, 192, 192), (9, 256, 256)])
+@pytest.mark.parametrize("biased", [False, True])
+@torch.no_grad()
+def test_outputs_of_parts_of_lines_gpu(tile, bm, bn, biased):
+    """Forward rows that are whole 64 bytes or not, to the last feature, and outputs
+    that no cache holds."""
+    from deepspeed_amd.ops import _C
+    for m, n, k in ((bm + 1, bn + 4, 192), (2 * bm, 2 * bn - 8, 256),
+                    (bm + 70, bn + 32, 320), (8300, 16200, 192)):
+        x, ws, bs = _inputs(m, (n,), k, n)
+        bs = bs if biased else [None]
+        got = _C.tile_linear(x, ws, bs, 0, tile, 1)[0]
+        rows = torch.cat([torch.arange(64), torch.arange(m - 64, m)]).cuda()
+        _close(got[rows], _want(x[rows], ws, bs, 0)[0])
