@@ -139,7 +139,8 @@ step_plan(const pybind11::sequence& slots,
     int64_t per = std::max(min_split,
                            total / std::max<int64_t>(1, room - n / 2));
     while (splits(per) > std::max(room, n)) per += per / 16;
-    const bool few = n * kv_heads <= fewer && (nq == 1 || runs.size() > 1);
+    const bool few = block_size % 32 == 0 && n * kv_heads <= fewer &&
+        (nq == 1 || runs.size() > 1);
     if (few) {
       // ns that the tiles take in these parts
       const int64_t held = lines[13 + nq], slots_ = held * lines[7];

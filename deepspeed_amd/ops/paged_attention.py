@@ -46,7 +46,10 @@ MIN_SPLIT = 128
 # and for each workgroup a CU holds beside it, of HELD; BYTES a ns. Fitted to 8000 steps
 # of 1 to 64 requests, half of them beside a run of up to 256 rows, 1 to 32 key heads:
 # 0.90 of the time of the rounds alone, 1.01 of the fastest cut. A run of several rows
-# alone keeps the rounds (its attention is 1 to 2% of such a step).
+# alone keeps the rounds (its attention is 1 to 2% of such a step). So do blocks that
+# hold no whole tile, for which a wave asks key by key: fewer parts are as much longer (16
+# keys a block, by the rounds / by these: 31 of 1880, 8 key heads 54 / 69 us, 2 of 4541, 32
+# key heads 36 / 45).
 ROOMS = 64, 128, 192, 256, 384, 512, 768
 STEP, HELD, BYTES, MERGE, MERGED = {1: (300, 1100), 2: (100, 1500)}, {1: 3, 2: 2}, \
     7500, 4400, 5
@@ -227,7 +230,8 @@ def _planned(slots, pos, tables, block_size: int, heads: int, kv_heads: int):
         while n.sum() > max(room, len(end)):
             per += per // 16
             n = -(-end // per)
-        if len(end) * kv_heads <= FEWER and (nq == 1 or len(m) > 1):
+        if block_size % 32 == 0 and len(end) * kv_heads <= FEWER and (
+                nq == 1 or len(m) > 1):
             n = np.ones_like(end)
             least = _cost(end, n, kv_heads, nq)
             for r in ROOMS:

@@ -93,6 +93,16 @@ def test_cuts_by_what_they_take(lens, heads, parts):
         assert plans._cost(end, n, heads[1], plan.nq) <= whole
 
 
+@pytest.mark.parametrize("bs,parts", [(16, 3), (24, 3), (32, 1), (64, 1)])
+def test_cuts_by_blocks(bs, parts):
+    """Cuts by what the parts take are for blocks that hold a whole tile of keys."""
+    need = -(-1881 // bs)
+    tables = {s: list(range(s * need, (s + 1) * need)) for s in range(31)}
+    args = (list(range(31)), np.full(31, 1880, np.int64), tables, bs, 32, 8)
+    for items in (StepPlan.build(*args, "cpu").items, plans._planned(*args)[1]):
+        assert items == 31 * parts
+
+
 @pytest.mark.parametrize("heads", [(8, 8), (14, 2), (32, 8), (16, 1)])
 def test_step_plan_equals_numpys(heads):
     """Single rows and runs of every length, slots that come again, tables of any
