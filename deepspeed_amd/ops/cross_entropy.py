@@ -110,9 +110,12 @@ class _HeadLoss(torch.autograd.Function):
             return dx, dw, None, None, None
         ctx.maybe_clear_saved_tensors()     # unless the graph is to stay
         dx = dw = turned = None
-        for i in range(n):
+        gone = 0
+        # a shorter chunk first: its gradient is beside all of the logits
+        for i in range(n) if len(ys[-1]) == rows else (n - 1, *range(n - 1)):
             d = gradient(i).contiguous()
             T, at = len(d), slice(i * rows, (i + 1) * rows)
+            gone += T
             if need_x:
                 to, K = None if dx is None else dx[at], w.shape[1]
                 if linear.own_dx(T, w.shape[:1], K) and linear._aligned(d, w):
@@ -124,9 +127,9 @@ class _HeadLoss(torch.autograd.Function):
                 else:
                     part = torch.mm(d, w, out=to)
                 # kept where the logits that are gone have left room for it
-                if 2 * w.numel() + len(labels) * K > (i + 1) * rows * len(w):
+                if 2 * w.numel() + len(labels) * K > gone * len(w):
                     turned = None
-            if need_w and i:
+            if dw is not None:
                 linear.add_dw(dw, xs[i], d)
             elif need_w:
                 dw = linear._dw(xs[i], [d], True, [None])[0]

@@ -279,3 +279,11 @@ def test_engine_with_several_chunks_gpu(stage, gas, monkeypatch):
     assert torch.equal(got[0], want[0])
     for a, b in zip(got[1:], want[1:]):
         assert (a.float() - b.float()).norm() <= 2.0 ** -6 * b.float().norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("frozen", [None, "x", "w"])
+@pytest.mark.parametrize("n", [5600, 11000])
+def test_memory_of_uneven_chunks_gpu(monkeypatch, frozen, n):
+    """A last chunk that is shorter is the first to go."""
+    test_memory_gpu(monkeypatch, frozen, n, 1000, 32064, 4096)
