@@ -705,6 +705,7 @@ bool in_heads(const Args& a, int layers) {
 // of N 1024 2.96 / 3.28, and K 512, N 256 2.82 / 3.13; int8 K 256 2.75 to 3.40 / 2.83 to
 // 3.00, K 512, N 1024 1, 16 and 24 rows 3.39 / 3.04, 3.54 / 3.15, 3.77 / 3.71, but 32 rows
 // 3.77 / 3.89, a whole round of tiles at 16 3.67 / 3.88, and K 768, N 2048 3.59 / 3.77.
+// Not what has the form of q, k and v: its sums are those of the products that append.
 template <bool I8>
 bool brief(const Args& a, int layers, int mode, int tiles) {
   if (mode != PLAIN || tiles >= 256 || in_heads(a, layers)) return false;
